@@ -576,6 +576,17 @@ int mi355_top_k_top_p_min_p_sample(int32_t* ids, const float* probs, const int32
                                    const float* top_ps, const float* min_ps, const float* uniform,
                                    int64_t rows, int64_t vocab, int64_t row_stride, void* stream);
 
+/* The two above with every row cut into chunks handled by separate workgroups (a few rows are a few workgroups
+ * otherwise), in two launches each.  Same kept set and the same rule for the draw; sums are taken in another order.
+ * workspace: mi355_sampling_workspace_bytes(rows, vocab) bytes, 8-byte aligned, contents arbitrary; calls that may
+ * overlap on one GPU need workspaces of their own.  NULL, or a row too short to cut, runs the entry point above. */
+int64_t mi355_sampling_workspace_bytes(int64_t rows, int64_t vocab);
+int mi355_softmax_temperature_split(float* logits, const float* temperatures, int64_t rows, int64_t vocab, int64_t row_stride,
+                                    void* workspace, int64_t workspace_bytes, void* stream);
+int mi355_top_k_top_p_min_p_sample_split(int32_t* ids, const float* probs, const int32_t* top_ks, const float* top_ps,
+                                         const float* min_ps, const float* uniform, int64_t rows, int64_t vocab,
+                                         int64_t row_stride, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* fp8_scaled_mm for M <= 64 on a weight packed by mi355_pack_weight (pass the fp8 bytes as an
  * [N, K/2] 16-bit matrix: the packed layout is defined on 16-byte fragments): the bf16 decode GEMM's
  * single-launch weight-streaming kernel with fp8 MFMA and the scale epilogue.  K % 512 == 0,

@@ -1,7 +1,8 @@
 // Sampling tail of the step: greedy arg-max, temperature softmax, and sort-free joint
-// top-k / top-p / min-p sampling over fp32 [rows, vocab] logits.  One workgroup of 1024
-// threads per row; rows are 0.5 MB at vocab 128256, so every pass after the first is served
-// from L2 / Infinity Cache.
+// top-k / top-p / min-p sampling over fp32 [rows, vocab] logits.  Rows are 0.5 MB at vocab 128256, so
+// every pass after the first is served from L2 / Infinity Cache.  What reads every entry is cut into
+// chunks of a row, one workgroup each (row_chunks); without a workspace, and for short rows, one
+// workgroup of 1024 threads does a whole row.
 #include "common.cuh"
 #include <math.h>
 #include <algorithm>
@@ -173,30 +174,149 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_temperature_kernel(
   for (int64_t i = threadIdx.x; i < vocab; i += SAMP_THREADS) row[i] = expf(row[i] / t - mx) / sum;
 }
 
+// The same over chunks of a row, in two launches: every chunk leaves its maximum and its sum of exponentials, then
+// every chunk normalises itself with what all of them left.  One workgroup per row reads its 0.5 MB three times with 4
+// bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
+// 18 + 16 us (33 MB read twice, the second time from L2, then read and written), bound by the precise division and
+// exponential of every entry in both.
+struct ChunkSpan {
+  int64_t v0, v1;   // first and one past the last of its groups of four elements
+  bool tail;        // whether the row's last vocab % 4 elements belong to it
+};
+__device__ __forceinline__ ChunkSpan chunk_span(int64_t vocab, int c, int chunks) {
+  const int64_t nv = vocab / 4, per = (nv + chunks - 1) / chunks;
+  ChunkSpan s;
+  s.v0 = min((int64_t)c * per, nv);
+  s.v1 = min(s.v0 + per, nv);
+  s.tail = c == chunks - 1;
+  return s;
+}
+// f(value) of every element of the span; vec: rows start at 16-byte boundaries
+template <typename F>
+__device__ __forceinline__ void span_each(const float* __restrict__ row, int64_t vocab, const ChunkSpan& sp, bool vec, F&& f) {
+  constexpr int U = 4;
+  int64_t i = sp.v0 + threadIdx.x;
+  for (; i + (U - 1) * SAMP_THREADS < sp.v1; i += U * SAMP_THREADS) {
+    Vec<float, 4> v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float* p = row + (i + u * SAMP_THREADS) * 4;
+      if (vec) v[u] = ldvec<float, 4>(p);
+      else
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[u].v[j] = p[j];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f(v[u].v[j]);
+  }
+  for (; i < sp.v1; i += SAMP_THREADS)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f(row[i * 4 + j]);
+  if (sp.tail) {
+    const int64_t k = vocab / 4 * 4 + threadIdx.x;
+    if (k < vocab) f(row[k]);
+  }
+}
+
+__global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
+    float2* __restrict__ partials, const float* __restrict__ logits, const float* __restrict__ temperatures, int64_t vocab,
+    int64_t row_stride) {
+  __shared__ float red[SAMP_THREADS / 64];
+  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
+  const float* row = logits + (int64_t)r * row_stride;
+  const bool vec = (row_stride % 4 == 0) && aligned16(logits);
+  const ChunkSpan sp = chunk_span(vocab, c, chunks);
+  const float t = temperatures[r];
+  float mx = -INFINITY;
+  span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, x / t); });
+  mx = block_reduce_max(mx, red);
+  float sum = 0.f;
+  span_each(row, vocab, sp, vec, [&](float x) { sum += expf(x / t - mx); });
+  sum = block_sum(sum, red);
+  if (threadIdx.x == 0) partials[(int64_t)r * chunks + c] = float2{mx, sum};
+}
+
+__global__ __launch_bounds__(SAMP_THREADS) void softmax_normalise_kernel(
+    float* __restrict__ logits, const float2* __restrict__ partials, const float* __restrict__ temperatures, int64_t vocab,
+    int64_t row_stride) {
+  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
+  float* row = logits + (int64_t)r * row_stride;
+  const bool vec = (row_stride % 4 == 0) && aligned16(logits);
+  const float t = temperatures[r];
+  float mx = -INFINITY, sum = 0.f;
+  for (int i = 0; i < chunks; ++i) mx = fmaxf(mx, partials[(int64_t)r * chunks + i].x);
+  for (int i = 0; i < chunks; ++i) {
+    const float2 p = partials[(int64_t)r * chunks + i];
+    // a chunk of nothing but -inf has no exponentials of its own (its sum is NaN) unless the whole row is like that
+    if (p.x != -INFINITY || mx == -INFINITY) sum += p.y * expf(p.x - mx);
+  }
+  const ChunkSpan sp = chunk_span(vocab, c, chunks);
+  for (int64_t i = sp.v0 + threadIdx.x; i < sp.v1; i += SAMP_THREADS) {
+    if (vec) {
+      Vec<float, 4> v = ldvec<float, 4>(row + i * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v.v[j] = expf(v.v[j] / t - mx) / sum;
+      stvec<float, 4>(row + i * 4, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) row[i * 4 + j] = expf(row[i * 4 + j] / t - mx) / sum;
+    }
+  }
+  if (sp.tail) {
+    const int64_t k = vocab / 4 * 4 + threadIdx.x;
+    if (k < vocab) row[k] = expf(row[k] / t - mx) / sum;
+  }
+}
+
 // ---- joint top-k / top-p / min-p filter + inverse-CDF draw --------------------------------
 // The kept set is {p >= tau}: tau is the smallest probability value v such that fewer than k
 // entries are strictly larger than v and the mass strictly above v is <= top_p.  It is found
 // by a 4-level radix select on the float bit pattern (non-negative floats order like their
 // bits) with 256-bin count/mass histograms in LDS, i.e. 4 passes over the row instead of a
 // sort.  min_p raises tau to min_p * pmax.  The draw walks the kept entries in index order.
-__global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
-    int32_t* __restrict__ ids, const float* __restrict__ probs, const int32_t* __restrict__ top_ks,
-    const float* __restrict__ top_ps, const float* __restrict__ min_ps,
-    const float* __restrict__ uniform, int64_t vocab, int64_t row_stride) {
-  __shared__ unsigned int hcount[256];
-  __shared__ float hmass[256];
-  __shared__ float red[SAMP_THREADS / 64];
-  __shared__ unsigned int s_prefix;   // bits fixed so far (high bits of tau)
-  __shared__ unsigned int s_count;    // entries strictly above the current bin range
-  __shared__ float s_mass;            // mass strictly above the current bin range
-  __shared__ float s_scan[SAMP_THREADS];
-  __shared__ int s_pick;
+struct SampleRow {
+  const float* row;
+  int64_t k;
+  float top_p, min_p, uniform;
+};
+__device__ __forceinline__ SampleRow sample_row(const float* probs, const int32_t* top_ks, const float* top_ps,
+                                                const float* min_ps, const float* uniform, int64_t row_stride) {
+  SampleRow r;
+  r.row = probs + (int64_t)blockIdx.x * row_stride;
+  r.k = top_ks ? (int64_t)top_ks[blockIdx.x] : (int64_t)1 << 30;
+  r.top_p = top_ps ? top_ps[blockIdx.x] : 1.0f;
+  if (r.top_p >= 1.0f) r.top_p = INFINITY;  // disabled: no rounding artefacts at the tail
+  r.min_p = min_ps ? min_ps[blockIdx.x] : 0.0f;
+  r.uniform = uniform[blockIdx.x];
+  return r;
+}
 
-  const float* row = probs + (int64_t)blockIdx.x * row_stride;
-  const int64_t k = top_ks ? (int64_t)top_ks[blockIdx.x] : (int64_t)1 << 30;
-  float top_p = top_ps ? top_ps[blockIdx.x] : 1.0f;
-  if (top_p >= 1.0f) top_p = INFINITY;  // disabled: no rounding artefacts at the tail
-  const float min_p = min_ps ? min_ps[blockIdx.x] : 0.0f;
+// LDS of the routine below, so that a kernel that has other uses for it can lend its own.
+struct SampleScratch {
+  unsigned int hcount[256];
+  float hmass[256];
+  float red[SAMP_THREADS / 64];
+  unsigned int prefix;   // bits fixed so far (high bits of tau)
+  unsigned int count;    // entries strictly above the current bin range
+  float mass;            // mass strictly above the current bin range
+  float scan[SAMP_THREADS];
+  int pick;
+};
+
+__device__ void sample_whole_row(int32_t* __restrict__ ids, const SampleRow& sr, int64_t vocab, SampleScratch& sm) {
+  unsigned int(&hcount)[256] = sm.hcount;
+  float(&hmass)[256] = sm.hmass;
+  float* red = sm.red;
+  unsigned int& s_prefix = sm.prefix;
+  unsigned int& s_count = sm.count;
+  float& s_mass = sm.mass;
+  float(&s_scan)[SAMP_THREADS] = sm.scan;
+  int& s_pick = sm.pick;
+  const float* row = sr.row;
+  const int64_t k = sr.k;
+  const float top_p = sr.top_p, min_p = sr.min_p;
 
   if (threadIdx.x == 0) {
     s_prefix = 0;
@@ -277,7 +397,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
   }
   __syncthreads();
   const float total = red[0];
-  const float target = uniform[blockIdx.x] * total;
+  const float target = sr.uniform * total;
   // the chunk containing the target: exclusive prefix <= target < prefix + part
   const float before = s_scan[threadIdx.x];
   if (part > 0.f && before <= target && (target < before + part)) {
@@ -309,9 +429,386 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
   }
 }
 
+__global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
+    int32_t* __restrict__ ids, const float* __restrict__ probs, const int32_t* __restrict__ top_ks,
+    const float* __restrict__ top_ps, const float* __restrict__ min_ps,
+    const float* __restrict__ uniform, int64_t vocab, int64_t row_stride) {
+  __shared__ SampleScratch sm;
+  sample_whole_row(ids, sample_row(probs, top_ks, top_ps, min_ps, uniform, row_stride), vocab, sm);
+}
+
+// ---- the same draw over chunks of a row -------------------------------------------------------
+// Launch 1, a workgroup per chunk: the chunk's positive entries in 2048 bins of 1/16 binade (the upper 13 bits of the
+// pattern), and its maximum.  Entries of a bin share exponent and upper mantissa, so their count (upper 24 bits) and the sum
+// of their 19 lower bits (lower 40) in one integer are their mass exactly, for one LDS atomic each; a count and a float
+// atomic took 47 us where this takes 10.  Launch 2, a workgroup per row: the first bin from the top that is not
+// kept whole holds tau; its entries -- hundreds where a vocabulary's probabilities spread over binades -- are collected in
+// LDS by one pass over the row and searched there bit by bit.  If they and the larger ones are few (a small top_k), all of
+// them are collected with their indices and the draw is made among them; otherwise a second pass sums what is kept per
+// tile of 256 entries, and the tile the draw falls into is walked.  A row whose tau lies above 1.9 (no probability does),
+// or with more entries in that bin than the list holds (an almost flat row), takes sample_whole_row.
+// The one-workgroup routine meets each of its four levels' 128256 entries in 256 bins of two binades, a handful of which
+// take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics; this
+// takes 10 + 28 us (58 when thousands are kept), the first bound by its LDS atomics too, the second by one CU's pass over 0.5 MB.
+constexpr int SB_BINS = 2048, SB_SHIFT = 19, SB_LIST = 8192, SB_SHORT = 512, SB_TILE = 256, SB_MAX_TILES = 4096;
+constexpr int SB_SUM_BITS = 40;
+constexpr int64_t SB_MAX_VOCAB = (int64_t)SB_TILE * SB_MAX_TILES;   // 2^20: counts fit 24 bits, sums of 19 bits fit 40
+typedef unsigned long long u64_t;
+
+__device__ __forceinline__ float bin_mass(int bin, u64_t x) {
+  const unsigned e = (unsigned)bin >> 4;                                          // exponent field
+  const double base = (double)((((unsigned)bin & 15u) << SB_SHIFT) + (e ? 1u << 23 : 0u));   // an entry's mantissa without its lower bits
+  return (float)ldexp((double)(x >> SB_SUM_BITS) * base + (double)(x & (((u64_t)1 << SB_SUM_BITS) - 1)), (int)(e ? e : 1u) - 150);
+}
+
+__global__ __launch_bounds__(SAMP_THREADS) void sample_bins_kernel(u64_t* __restrict__ bins, float* __restrict__ maxima,
+                                                                  const float* __restrict__ probs, int64_t vocab,
+                                                                  int64_t row_stride) {
+  __shared__ u64_t hist[SB_BINS];
+  __shared__ float red[SAMP_THREADS / 64];
+  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
+  const float* row = probs + (int64_t)r * row_stride;
+  const bool vec = (row_stride % 4 == 0) && aligned16(probs);
+  for (int i = threadIdx.x; i < SB_BINS; i += SAMP_THREADS) hist[i] = 0;
+  __syncthreads();
+  float mx = 0.f;
+  span_each(row, vocab, chunk_span(vocab, c, chunks), vec, [&](float v) {
+    if (v > 0.f) {
+      mx = fmaxf(mx, v);
+      const unsigned bits = __float_as_uint(v), b = min(bits >> SB_SHIFT, (unsigned)(SB_BINS - 1));
+      atomicAdd(&hist[b], ((u64_t)1 << SB_SUM_BITS) + (bits & ((1u << SB_SHIFT) - 1)));
+    }
+  });
+  mx = block_reduce_max(mx, red);
+  u64_t* out = bins + ((int64_t)r * chunks + c) * SB_BINS;
+  for (int i = threadIdx.x; i < SB_BINS; i += SAMP_THREADS) out[i] = hist[i];
+  if (threadIdx.x == 0) maxima[(int64_t)r * chunks + c] = mx;
+}
+
+// Of N bins (counts and masses in LDS), going down from the top: the first bin that is not kept whole, with the count and
+// mass above it; bin -1 if there is none.  Counts and masses grow on the way down, so from that bin on none is.  Empty
+// bins are passed over.  Every thread returns the same; begins and ends with a barrier.
+struct BinCut {
+  int bin;
+  unsigned count;
+  float mass;
+};
+struct CutScratch {
+  unsigned wc[SAMP_THREADS / 64];
+  float wm[SAMP_THREADS / 64];
+  BinCut cut;
+};
+template <int N>
+__device__ __forceinline__ BinCut cut_bins(const unsigned* hcount, const float* hmass, int64_t k, float top_p, unsigned count0,
+                                           float mass0, CutScratch& sm) {
+  constexpr int PER = (N + SAMP_THREADS - 1) / SAMP_THREADS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int top = N - 1 - (int)threadIdx.x * PER;     // this thread's bins: top, top - 1, .. (PER of them)
+  __syncthreads();
+  unsigned c[PER], ci = 0;
+  float m[PER], mi = 0.f;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    c[j] = top - j >= 0 ? hcount[top - j] : 0u;
+    m[j] = top - j >= 0 ? hmass[top - j] : 0.f;
+    ci += c[j];
+    mi += m[j];
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned oc = __shfl_up(ci, o, 64);
+    const float om = __shfl_up(mi, o, 64);
+    if (lane >= o) {
+      ci += oc;
+      mi += om;
+    }
+  }
+  if (lane == 63) {
+    sm.wc[wave] = ci;
+    sm.wm[wave] = mi;
+  }
+  if (threadIdx.x == 0) sm.cut = BinCut{-1, 0u, 0.f};
+  const unsigned cx = __shfl_up(ci, 1, 64);            // what the lanes before this one have
+  const float mx = __shfl_up(mi, 1, 64);
+  __syncthreads();
+  unsigned above = count0;
+  float mass = mass0;
+  for (int w = 0; w < wave; ++w) {
+    above += sm.wc[w];
+    mass += sm.wm[w];
+  }
+  if (lane > 0) {
+    above += cx;
+    mass += mx;
+  }
+  BinCut mine{-1, 0u, 0.f};
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if (mine.bin < 0 && c[j] != 0) {
+      if ((int64_t)above + c[j] <= k && mass + m[j] <= top_p) {
+        above += c[j];
+        mass += m[j];
+      } else {
+        mine = BinCut{top - j, above, mass};
+      }
+    }
+  }
+  if (mine.bin >= 0) atomicMax(&sm.cut.bin, mine.bin);
+  __syncthreads();
+  if (mine.bin >= 0 && mine.bin == sm.cut.bin) {
+    sm.cut.count = mine.count;
+    sm.cut.mass = mine.mass;
+  }
+  __syncthreads();
+  return sm.cut;
+}
+
+// Four elements of a row from group i on (groups of 4; vec: one 16-byte load), zeros past the end.
+__device__ __forceinline__ Vec<float, 4> row4(const float* __restrict__ row, int64_t vocab, int64_t i, bool vec) {
+  Vec<float, 4> v;
+  if (vec && i * 4 + 4 <= vocab) return ldvec<float, 4>(row + i * 4);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v.v[j] = i * 4 + j < vocab ? row[i * 4 + j] : 0.f;
+  return v;
+}
+
+__global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
+    int32_t* __restrict__ ids, const u64_t* __restrict__ bins, const float* __restrict__ maxima, int chunks,
+    const float* __restrict__ probs, const int32_t* __restrict__ top_ks, const float* __restrict__ top_ps,
+    const float* __restrict__ min_ps, const float* __restrict__ uniform, int64_t vocab, int64_t row_stride) {
+  __shared__ unsigned hcount[SB_BINS];
+  __shared__ float hmass[SB_BINS];
+  __shared__ union {
+    unsigned list[SB_LIST];        // the cut bin's entries, until tau is known
+    float tile[SB_MAX_TILES];      // kept mass per tile of 256 entries, afterwards
+    SampleScratch whole;
+  } sm;
+  __shared__ CutScratch cs;
+  __shared__ unsigned n_list;
+  __shared__ int s_tile, s_last, s_pick;
+  __shared__ float s_before;
+  const SampleRow sr = sample_row(probs, top_ks, top_ps, min_ps, uniform, row_stride);
+  const float* row = sr.row;
+  const bool vec = (row_stride % 4 == 0) && aligned16(probs);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const u64_t* rb = bins + (int64_t)blockIdx.x * chunks * SB_BINS;
+  float pmax = 0.f;
+  for (int c = 0; c < chunks; ++c) pmax = fmaxf(pmax, maxima[(int64_t)blockIdx.x * chunks + c]);
+  for (int i = threadIdx.x; i < SB_BINS; i += SAMP_THREADS) {
+    u64_t x = 0;
+    for (int c = 0; c < chunks; ++c) x += rb[(int64_t)c * SB_BINS + i];
+    hcount[i] = (unsigned)(x >> SB_SUM_BITS);
+    hmass[i] = bin_mass(i, x);
+  }
+  if (threadIdx.x == 0) {
+    n_list = 0;
+    s_tile = SB_MAX_TILES;
+    s_last = -1;
+    s_pick = 0x7fffffff;
+  }
+  BinCut cut = cut_bins<SB_BINS>(hcount, hmass, sr.k, sr.top_p, 0u, 0.f, cs);
+  float tau = 0.f;
+  bool few = false;
+  if (cut.bin >= 0) {
+    unsigned size = hcount[cut.bin];
+    if (cut.bin == SB_BINS - 1 || size > (unsigned)SB_LIST) {
+      __syncthreads();
+      sample_whole_row(ids, sr, vocab, sm.whole);
+      return;
+    }
+    few = cut.count + size <= (unsigned)SB_SHORT;
+    // the cut bin's entries; with the larger ones and everybody's index if they are few
+    const unsigned lowest = (unsigned)cut.bin << SB_SHIFT, bound = few ? 0x7f800000u : lowest + (1u << SB_SHIFT);
+    constexpr int U = 8;
+    const int64_t groups = (vocab + 3) / 4;
+    for (int64_t i0 = threadIdx.x; i0 < groups; i0 += U * SAMP_THREADS) {
+      Vec<float, 4> v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = i0 + u * SAMP_THREADS;
+        if (i < groups) v[u] = row4(row, vocab, i, vec);
+        else v[u] = Vec<float, 4>{{0.f, 0.f, 0.f, 0.f}};
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const unsigned bits = __float_as_uint(v[u].v[j]);
+          if (v[u].v[j] > 0.f && bits >= lowest && bits < bound) {
+            const unsigned at = atomicAdd(&n_list, 1u);
+            if (at < (unsigned)SB_LIST) sm.list[at] = bits;
+            if (few && at < (unsigned)SB_SHORT) sm.list[SB_SHORT + at] = (unsigned)((i0 + u * SAMP_THREADS) * 4 + j);
+          }
+        }
+    }
+    if (few) size += cut.count;
+    // its 19 lower bits, ten and then nine of them
+    unsigned prefix = (unsigned)cut.bin;
+    unsigned himask = ~0u << SB_SHIFT;
+    const int shifts[2] = {9, 0};
+#pragma unroll
+    for (int level = 0; level < 2; ++level) {
+      const int nb = level == 0 ? 1024 : 512, shift = shifts[level];
+      __syncthreads();
+      for (int i = threadIdx.x; i < 1024; i += SAMP_THREADS) {
+        hcount[i] = 0;
+        hmass[i] = 0.f;
+      }
+      __syncthreads();
+      const unsigned want = prefix << (level == 0 ? SB_SHIFT : 9);
+      for (unsigned i = threadIdx.x; i < size; i += SAMP_THREADS) {
+        const unsigned bits = sm.list[i];
+        if ((bits & himask) == want) {
+          const unsigned b = (bits >> shift) & (unsigned)(nb - 1);
+          atomicAdd(&hcount[b], 1u);
+          unsafeAtomicAdd(&hmass[b], __uint_as_float(bits));
+        }
+      }
+      const BinCut next = cut_bins<1024>(hcount, hmass, sr.k, sr.top_p, cut.count, cut.mass, cs);
+      // the coarser bin was not kept whole, but its parts' rounded masses may add up to less: then its lowest part is taken
+      cut = next.bin >= 0 ? next : BinCut{0, cut.count, cut.mass};
+      prefix = (prefix << (level == 0 ? 10 : 9)) | (unsigned)cut.bin;
+      himask = ~0u << shift;
+    }
+    // entries above the pattern number cut.count with mass cut.mass; those equal to it are kept iff the rule still holds
+    const bool keep = (int64_t)cut.count < sr.k && cut.mass <= sr.top_p;
+    tau = __uint_as_float(keep ? prefix : prefix + 1u);
+  }
+  tau = fmaxf(tau, sr.min_p * pmax);
+  if (!(tau > 0.f)) tau = __uint_as_float(1u);   // never keep zero-probability entries
+  if (few) {
+    // the draw among the listed entries, in index order; sums in double, so that the list's order leaves no trace
+    __syncthreads();
+    const int n = (int)min(n_list, (unsigned)SB_SHORT), me = (int)threadIdx.x;
+    const bool in = me < n && __uint_as_float(sm.list[me]) >= tau;
+    const unsigned own = in ? sm.list[SB_SHORT + me] : 0u;
+    double upto = 0.0, total = 0.0;
+    if (wave * 64 < n)
+      for (int j = 0; j < n; ++j) {
+        const float p = __uint_as_float(sm.list[j]);
+        const double q = p >= tau ? (double)p : 0.0;
+        total += q;
+        upto += sm.list[SB_SHORT + j] <= own ? q : 0.0;
+      }
+    if (in) {
+      atomicMax(&s_last, (int)own);
+      if (upto > (double)sr.uniform * total) atomicMin(&s_pick, (int)own);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) ids[blockIdx.x] = s_pick != 0x7fffffff ? s_pick : max(s_last, 0);
+    return;
+  }
+  __syncthreads();
+
+  // kept mass per tile of 256 entries (one wave's load)
+  const int tiles = (int)((vocab + SB_TILE - 1) / SB_TILE);
+  for (int t0 = wave; t0 < tiles; t0 += 8 * (SAMP_THREADS / 64)) {
+    Vec<float, 4> v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int t = t0 + u * (SAMP_THREADS / 64);
+      if (t < tiles) v[u] = row4(row, vocab, (int64_t)t * 64 + lane, vec);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int t = t0 + u * (SAMP_THREADS / 64);
+      if (t < tiles) {
+        float part = 0.f;
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          any |= v[u].v[j] >= tau;
+          part += v[u].v[j] >= tau ? v[u].v[j] : 0.f;
+        }
+        if (__any(any)) part = wave_sum(part);
+        if (lane == 0) sm.tile[t] = part;
+      }
+    }
+  }
+  __syncthreads();
+  // exclusive sums over tiles, four tiles a thread
+  float part[4], before[4], run = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int t = (int)threadIdx.x * 4 + j;
+    part[j] = t < tiles ? sm.tile[t] : 0.f;
+    before[j] = run;
+    run += part[j];
+  }
+  float incl = run;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float up = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += up;
+  }
+  if (lane == 63) cs.wm[wave] = incl;
+  const float left = __shfl_up(incl, 1, 64);
+  __syncthreads();
+  float base = 0.f, total = 0.f;
+  for (int w = 0; w < SAMP_THREADS / 64; ++w) {
+    if (w < wave) base += cs.wm[w];
+    total += cs.wm[w];
+  }
+  if (lane > 0) base += left;
+  const float target = sr.uniform * total;
+  // the first tile whose running mass passes the target, and the last one with anything in it
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int t = (int)threadIdx.x * 4 + j;
+    if (part[j] > 0.f) {
+      atomicMax(&s_last, t);
+      if (base + before[j] + part[j] > target) atomicMin(&s_tile, t);
+    }
+  }
+  __syncthreads();
+  const int hit = s_tile < SB_MAX_TILES ? s_tile : s_last;   // rounding at the very end of the CDF: the last kept entry
+  if (hit >= 0 && (int)threadIdx.x == hit / 4) s_before = base + before[hit % 4];
+  __syncthreads();
+  if (wave != 0) return;
+  if (hit < 0) {
+    if (lane == 0) ids[blockIdx.x] = 0;
+    return;
+  }
+  const Vec<float, 4> v = row4(row, vocab, (int64_t)hit * 64 + lane, vec);
+  float own = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) own += v.v[j] >= tau ? v.v[j] : 0.f;
+  float sum = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float up = __shfl_up(sum, o, 64);
+    if (lane >= o) sum += up;
+  }
+  const float upto = __shfl_up(sum, 1, 64);
+  float at = s_before + (lane > 0 ? upto : 0.f);
+  int pick = 0x7fffffff, kept = -1;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (v.v[j] >= tau) {
+      at += v.v[j];
+      kept = hit * SB_TILE + lane * 4 + j;
+      if (pick == 0x7fffffff && at > target) pick = kept;
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    pick = min(pick, __shfl_xor(pick, o, 64));
+    kept = max(kept, __shfl_xor(kept, o, 64));
+  }
+  if (lane == 0) ids[blockIdx.x] = pick != 0x7fffffff ? pick : kept;
+}
+
+// Chunks of a row for `rows` rows: enough workgroups for every CU, at least 8 K entries each (below that a launch is all
+// latency), at most 16.
+static int row_chunks(int64_t rows, int64_t vocab) {
+  const int64_t want = (256 + rows - 1) / rows;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 16), vocab / 8192));
+}
+
 }  // namespace mi355
 
 using namespace mi355;
+
+
 
 extern "C" {
 
@@ -367,6 +864,29 @@ int mi355_softmax_temperature(float* logits, const float* temperatures, int64_t 
   return MI355_OK;
 }
 
+int64_t mi355_sampling_workspace_bytes(int64_t rows, int64_t vocab) {
+  if (rows <= 0 || vocab <= 0) return 0;
+  return rows * row_chunks(rows, vocab) * (SB_BINS * (int64_t)sizeof(u64_t) + (int64_t)sizeof(float2));
+}
+
+int mi355_softmax_temperature_split(float* logits, const float* temperatures, int64_t rows, int64_t vocab, int64_t row_stride,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  MI355_REQUIRE(logits && temperatures, MI355_ERR_INVALID, "softmax_temperature_split: null pointer");
+  MI355_REQUIRE(rows >= 0 && vocab > 0 && row_stride >= vocab, MI355_ERR_INVALID, "softmax_temperature_split: bad shape");
+  const int chunks = rows > 0 ? row_chunks(rows, vocab) : 1;
+  if (chunks <= 1 || !workspace) return mi355_softmax_temperature(logits, temperatures, rows, vocab, row_stride, stream);
+  MI355_REQUIRE(workspace_bytes >= rows * chunks * (int64_t)sizeof(float2) && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0,
+                MI355_ERR_INVALID, "softmax_temperature_split: workspace of %lld bytes (8-byte aligned) required",
+                (long long)mi355_sampling_workspace_bytes(rows, vocab));
+  float2* partials = static_cast<float2*>(workspace);
+  hipLaunchKernelGGL(softmax_partials_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, partials,
+                     logits, temperatures, vocab, row_stride);
+  hipLaunchKernelGGL(softmax_normalise_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, logits,
+                     partials, temperatures, vocab, row_stride);
+  MI355_CHECK_LAUNCH("softmax_temperature_split");
+  return MI355_OK;
+}
+
 int mi355_top_k_top_p_min_p_sample(int32_t* ids, const float* probs, const int32_t* top_ks,
                                    const float* top_ps, const float* min_ps, const float* uniform,
                                    int64_t rows, int64_t vocab, int64_t row_stride, void* stream) {
@@ -378,6 +898,28 @@ int mi355_top_k_top_p_min_p_sample(int32_t* ids, const float* probs, const int32
                      (hipStream_t)stream, ids, probs, top_ks, top_ps, min_ps, uniform, vocab,
                      row_stride);
   MI355_CHECK_LAUNCH("top_k_top_p_min_p_sample");
+  return MI355_OK;
+}
+
+int mi355_top_k_top_p_min_p_sample_split(int32_t* ids, const float* probs, const int32_t* top_ks, const float* top_ps,
+                                         const float* min_ps, const float* uniform, int64_t rows, int64_t vocab,
+                                         int64_t row_stride, void* workspace, int64_t workspace_bytes, void* stream) {
+  // a short row is two launches' latency for nothing; a vocabulary past the tiles' table does not exist
+  if (!workspace || rows <= 0 || vocab < 4096 || vocab > SB_MAX_VOCAB)
+    return mi355_top_k_top_p_min_p_sample(ids, probs, top_ks, top_ps, min_ps, uniform, rows, vocab, row_stride, stream);
+  MI355_REQUIRE(ids && probs && uniform, MI355_ERR_INVALID, "top_k_top_p_min_p_sample_split: null pointer");
+  MI355_REQUIRE(row_stride >= vocab, MI355_ERR_INVALID, "top_k_top_p_min_p_sample_split: bad shape");
+  const int64_t need = mi355_sampling_workspace_bytes(rows, vocab);
+  MI355_REQUIRE(workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0, MI355_ERR_INVALID,
+                "top_k_top_p_min_p_sample_split: workspace of %lld bytes (8-byte aligned) required", (long long)need);
+  const int chunks = row_chunks(rows, vocab);
+  u64_t* bins = static_cast<u64_t*>(workspace);
+  float* maxima = reinterpret_cast<float*>(bins + rows * chunks * SB_BINS);
+  hipLaunchKernelGGL(sample_bins_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, bins, maxima,
+                     probs, vocab, row_stride);
+  hipLaunchKernelGGL(sample_pick_kernel, dim3((unsigned)rows), dim3(SAMP_THREADS), 0, (hipStream_t)stream, ids, bins, maxima,
+                     chunks, probs, top_ks, top_ps, min_ps, uniform, vocab, row_stride);
+  MI355_CHECK_LAUNCH("top_k_top_p_min_p_sample_split");
   return MI355_OK;
 }
 

@@ -1065,14 +1065,20 @@ def argmax(logits: torch.Tensor) -> torch.Tensor:
     return ids
 
 
+def _sampling_workspace(x: torch.Tensor) -> torch.Tensor:
+    """Scratch of the chunked sampling launches: the caching allocator's, so on the stream of the call."""
+    return torch.empty(max(8, int(_lib_().mi355_sampling_workspace_bytes(x.shape[0], x.shape[1]))), dtype=torch.uint8, device=x.device)
+
+
 def softmax_temperature_(logits: torch.Tensor, temperatures: torch.Tensor) -> torch.Tensor:
     """In place logits.div_(temperatures); logits[:] = softmax(logits) (layers/sampler.py:79-81)."""
     _gpu(logits, temperatures)
     assert logits.dim() == 2 and logits.dtype == torch.float32 and logits.stride(1) == 1
     assert temperatures.dtype == torch.float32 and temperatures.numel() == logits.shape[0]
-    check(_lib_().mi355_softmax_temperature(logits.data_ptr(), temperatures.data_ptr(),
-                                            logits.shape[0], logits.shape[1], logits.stride(0),
-                                            _stream(logits)), "softmax_temperature")
+    ws = _sampling_workspace(logits)
+    check(_lib_().mi355_softmax_temperature_split(logits.data_ptr(), temperatures.data_ptr(), logits.shape[0], logits.shape[1],
+                                                  logits.stride(0), ws.data_ptr(), ws.numel(), _stream(logits)),
+          "softmax_temperature")
     return logits
 
 
@@ -1088,10 +1094,10 @@ def top_k_top_p_min_p_sample(probs: torch.Tensor, top_ks: Optional[torch.Tensor]
     assert top_ps is None or (top_ps.dtype == torch.float32 and top_ps.numel() == B)
     assert min_ps is None or (min_ps.dtype == torch.float32 and min_ps.numel() == B)
     ids = torch.empty(B, dtype=torch.int32, device=probs.device)
-    check(_lib_().mi355_top_k_top_p_min_p_sample(ids.data_ptr(), probs.data_ptr(), _p(top_ks),
-                                                 _p(top_ps), _p(min_ps), uniform.data_ptr(), B,
-                                                 probs.shape[1], probs.stride(0), _stream(probs)),
-          "top_k_top_p_min_p_sample")
+    ws = _sampling_workspace(probs)
+    check(_lib_().mi355_top_k_top_p_min_p_sample_split(ids.data_ptr(), probs.data_ptr(), _p(top_ks), _p(top_ps), _p(min_ps),
+                                                       uniform.data_ptr(), B, probs.shape[1], probs.stride(0), ws.data_ptr(),
+                                                       ws.numel(), _stream(probs)), "top_k_top_p_min_p_sample")
     return ids
 
 

@@ -1235,3 +1235,54 @@ def test_extend_attention_matrix_core_tile_192_wide_keys(ops, dtn):
                                          vc[slots[b]].transpose(0, 1), Dq ** -0.5, pre[b]).transpose(0, 1)
             assert maxdiff(o[p: p + ext[b]], ref) <= ATTN_TOL[dtn], (H, b)
             p += ext[b]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,vocab,pad", [(1, 128256, 0), (3, 4096, 0), (2, 8191, 0), (5, 32769, 3), (64, 16384, 0), (300, 4099, 1), (1, 300001, 0)])
+def test_chunked_softmax_and_sampler_edges(ops, rows, vocab, pad):
+    """Rows cut into chunks: vocabularies around the cut's limits, rows whose stride breaks the 16-byte alignment, -inf entries,
+    a row of nothing but -inf but one, flat and two-valued rows (the cut bin overflows its list), unnormalised rows.  Softmax
+    against float64: 2e-6 relative covers a 3e5-term fp32 sum (terms <= 1, pairwise over >= 1024 partial sums: < 8 levels of 2^-24
+    per lane sum of <= 300 terms) beside the exponential's own 2 ulp.  The draw: index-order inverse CDF over the kept set in
+    float64, the target within 1e-5 of the entry's own interval."""
+    g = torch.Generator().manual_seed(rows * 7 + vocab)
+    logits = 2.5 * torch.randn((rows, vocab), generator=g)
+    logits[0, vocab // 2:] = float("-inf")
+    logits[-1] = float("-inf")
+    logits[-1, vocab - 1] = 1.0
+    temps = torch.rand((rows,), generator=g) + 0.5
+    buf = torch.zeros((rows, vocab + pad), device=DEV)
+    got = buf[:, :vocab]
+    got.copy_(logits)
+    ops.softmax_temperature_(got, temps.to(DEV))
+    ref = torch.softmax(logits.double() / temps.double()[:, None], -1)
+    assert (got.cpu().double() - ref).norm() <= 2e-6 * ref.norm() and ((got.cpu() > 0) == (ref.float() > 0)).float().mean() > 0.999
+    kinds = [torch.softmax(2.5 * torch.randn(vocab, generator=g), -1), torch.full((vocab,), 1.0 / vocab), torch.softmax((torch.arange(vocab) % 2).float(), -1),
+             torch.softmax(0.01 * torch.randn(vocab, generator=g), -1), 3.0 * torch.rand(vocab, generator=g) ** 4,
+             torch.nn.functional.one_hot(torch.tensor(vocab - 1), vocab).float()]
+    for kind, p in enumerate(kinds):
+        if rows > 8 and kind not in (0, 5):
+            continue
+        probs = torch.zeros((rows, vocab + pad))[:, :vocab]
+        probs.copy_(p[None].expand(rows, vocab))
+        dev = torch.zeros((rows, vocab + pad), device=DEV)[:, :vocab]
+        dev.copy_(probs)
+        for k, tp, mp in ((1, 1.0, 0.0), (50, 0.9, 0.0), (1 << 30, 0.7, 0.0), (1 << 30, 1.0, 0.0), (700, 0.95, 0.02)):
+            u = torch.rand((rows,), generator=g)
+            ids = ops.top_k_top_p_min_p_sample(dev, torch.full((rows,), k, dtype=torch.int32, device=DEV), torch.full((rows,), tp, device=DEV),
+                                               torch.full((rows,), mp, device=DEV), u.to(DEV)).cpu().long()
+            # an entry is kept iff fewer than k are larger and at most top_p lies above it; mass compared in float64, entries
+            # within 1e-5 of the bound may go either way
+            vals, order = p.double().sort(descending=True, stable=True)
+            above = torch.searchsorted(-vals, -vals, right=False)
+            mass = torch.cat([torch.zeros(1, dtype=torch.float64), vals.cumsum(0)])[above]
+            lim = tp if tp < 1.0 else float("inf")
+            for slack in (-1e-5, 0.0, 1e-5):
+                keep = torch.zeros(vocab, dtype=torch.bool)
+                keep[order] = (above < k) & (mass <= lim + slack) & (vals > 0) & (vals >= mp * vals[0])
+                cdf = torch.where(keep, p.double(), torch.zeros(())).cumsum(0)
+                t = u.double() * cdf[-1]
+                ok = keep[ids] & (cdf[ids] >= t - 2e-5 * cdf[-1]) & (cdf[ids] - p.double()[ids] <= t + 2e-5 * cdf[-1])
+                if ok.all():
+                    break
+            assert ok.all(), (kind, k, tp, mp, ids[~ok][:4].tolist())

@@ -781,12 +781,13 @@ int mi355_sigmoid_attention(void* out, const void* q, const void* k_cache, const
  *   (mi355_moe_block_rows(0), or mi355_moe_block_rows(1) for prefill-sized steps of 16-bit models) of one expert each: src_row[p] = token of sorted row p or -1 (padding), rows[pair] = p, tile_expert[block] = its expert,
  *   *n_tiles = blocks in use.  `padded` (a multiple of the block) must be at least pairs + min(experts, pairs) * (block - 1).
  * mi355_moe_grouped_linear: out[p][.] = act(weight[tile_expert[p / block]] . in[gather ? src_row[p] : p]) for every sorted
- *   row p of a block in use (0 for padding rows); weight [experts, n, k]; act: 0 nothing, 1 erf-GELU, 2 the square of relu. */
+ *   row p of a block in use (0 for padding rows, which blocks of 256 rows leave unwritten); weight [experts, n, k]; act: 0 nothing, 1 erf-GELU, 2 the square of relu. */
 int mi355_moe_route_grouped(int32_t* ids, float* weights, const float* logits, const float* correction, int64_t tokens,
                             int num_experts, int top, int n_groups, int keep_groups, float scale, void* stream);
 int mi355_moe_block_rows(int wide);
 /* The grouped GEMM over 256-row blocks on the prefill projection kernel (mi355_linear_tiled's): every 256-row tile of the
- * sorted rows multiplies weight[tile_expert[tile]]; row_map (null: identity) gathers the rows of x; tiles at or past
+ * sorted rows multiplies weight[tile_expert[tile]]; row_map (null: identity) gathers the rows of x, negative entries (padding
+ * behind a tile's rows) are not computed; tiles at or past
  * *tiles_used are skipped; act 1 = erf-GELU.  Same shape conditions as mi355_linear_tiled, rows a multiple of 256. */
 int mi355_moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const void* w, const int32_t* row_map,
                                    const int32_t* tile_expert, const int32_t* tiles_used, int act, int64_t rows, int64_t n,

@@ -779,6 +779,111 @@ static void launch_skinny(const T* x, const T* w, const T* bias, OUT* y, void* w
 #undef SK
 }
 
+// fp32 products with few columns (router, gate and step-size logits): out[t][n] = x[t] . w[n] with T operands, as summed or
+// (ROUND, mi355_linear's contract) rounded to T once.  (A product of two 16-bit numbers is exact in fp32; fp32 operands take the fp32 matrix instruction, one rounding per
+// product and sum.)  A workgroup takes 16 rows x 16 NT columns; its eight waves walk every eighth step of 32 (fp32:
+// 16) of K on the matrix cores and meet in LDS, in a fixed order whatever the number of rows.
+// The 64 x 64 vector-ALU tiles of gemm_tiled_kernel leave most of a tile empty at such widths and are a handful of
+// workgroups each walking all of K: 3000 fp32 rows x 32 columns x 2048 took 250 us, 7400 bf16 rows x 32 x 2048 took 187 us;
+// here 14 and 14 us, bound by reading x (25 and 30 MB).
+constexpr int PJ_WAVES = 8;
+template <typename T> struct PjMma {
+  static constexpr int STEP = 32, PER = 8;      // K per step, elements per lane
+  using frag = typename Mfma<T>::frag;
+  static __device__ __forceinline__ f32x4 run(frag a, frag b, f32x4 c) { return Mfma<T>::run(a, b, c); }
+};
+template <> struct PjMma<float> {
+  static constexpr int STEP = 16, PER = 4;
+  using frag = f32x4;                            // lane group lg holds k = 4 lg .. 4 lg + 3, one of them per instruction
+  static __device__ __forceinline__ f32x4 run(frag a, frag b, f32x4 c) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+    return c;
+  }
+};
+template <typename T, int NT, bool ROUND>
+__global__ __launch_bounds__(64 * PJ_WAVES) void project_f32_mfma_kernel(float* __restrict__ out, const T* __restrict__ x, int64_t x_stride,
+                                                                        const T* __restrict__ w, int64_t rows, int N, int K) {
+  using M = PjMma<T>;
+  using Frag = typename M::frag;
+  __shared__ __attribute__((aligned(16))) f32x4 part[PJ_WAVES][NT][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  const int64_t t = (int64_t)blockIdx.x * 16 + li;
+  // rows past either end read row 0; their results are not stored
+  const T* xr = x + (t < rows ? t : 0) * x_stride;
+  const T* wr[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) {
+    const int n = (blockIdx.y * NT + y) * 16 + li;
+    wr[y] = w + (int64_t)(n < N ? n : 0) * K;
+  }
+  const Frag zero = {};
+  f32x4 acc[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) acc[y] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k0 = M::STEP * wv; k0 < K; k0 += M::STEP * PJ_WAVES) {
+    const bool in_k = k0 + M::PER * lg < K;
+    const int k = in_k ? k0 + M::PER * lg : 0;
+    const Frag av = *reinterpret_cast<const Frag*>(xr + k);
+    Frag bv[NT];
+#pragma unroll
+    for (int y = 0; y < NT; ++y) bv[y] = *reinterpret_cast<const Frag*>(wr[y] + k);
+#pragma unroll
+    for (int y = 0; y < NT; ++y) acc[y] = M::run(in_k ? av : zero, in_k ? bv[y] : zero, acc[y]);
+  }
+#pragma unroll
+  for (int y = 0; y < NT; ++y) part[wv][y][lane] = acc[y];
+  __syncthreads();
+  if (wv >= NT) return;
+  f32x4 sum = part[0][wv][lane];
+#pragma unroll
+  for (int o = 1; o < PJ_WAVES; ++o) sum += part[o][wv][lane];
+  const int n = (blockIdx.y * NT + wv) * 16 + li;
+  if (n >= N) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t row = (int64_t)blockIdx.x * 16 + 4 * lg + r;
+    if (row < rows) out[row * N + n] = ROUND ? round_to<T>(sum[r]) : sum[r];
+  }
+}
+
+// The same for widths that are no multiple of 8: one wave per result.
+template <typename T>
+__global__ __launch_bounds__(256) void project_f32_kernel(float* __restrict__ out, const T* __restrict__ x, int64_t x_stride,
+                                                          const T* __restrict__ w, int64_t rows, int N, int K) {
+  const int lane = threadIdx.x & 63;
+  const int64_t idx = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (idx >= rows * N) return;
+  const int64_t t = idx / N;
+  const int n = (int)(idx - t * N);
+  float acc = 0.f;
+  for (int k = lane; k < K; k += 64) acc = fmaf(to_f32(x[t * x_stride + k]), to_f32(w[(int64_t)n * K + k]), acc);
+  acc = wave_sum(acc);
+  if (lane == 0) out[idx] = acc;
+}
+
+template <typename T>
+bool project_mfma_ok(const void* x, int64_t x_stride, const void* w, int64_t k) {
+  return k % PjMma<T>::PER == 0 && x_stride % PjMma<T>::PER == 0 && aligned16(x) && aligned16(w);
+}
+template <typename T, bool ROUND>
+void launch_project_mfma(float* out, const void* x, int64_t x_stride, const void* w, int64_t rows, int n, int k, hipStream_t st) {
+  const unsigned gx = (unsigned)cdiv(rows, 16);
+#define MI355_PJ(NT)                                                                                                              \
+  hipLaunchKernelGGL((project_f32_mfma_kernel<T, NT, ROUND>), dim3(gx, (unsigned)cdiv(n, 16 * NT)), dim3(64 * PJ_WAVES), 0, st, out,     \
+                     (const T*)x, x_stride, (const T*)w, rows, n, k)
+  if (n <= 16) MI355_PJ(1);
+  else if (n <= 32) MI355_PJ(2);
+  else MI355_PJ(4);
+#undef MI355_PJ
+}
+
+// Columns up to which mi355_linear takes the kernel above for fp32 results without a bias (more rows than the skinny
+// kernels serve).  Every 64 columns read x again, from L2: 7400 rows x K 2048 in us, this / the 64 x 64 tiles: bf16 32 columns
+// 14 / 165, 256: 72 / 238, 512: 131 / 320; fp32 32: 25 / 239, 256: 147 / 289, 512: 270 / 350, where the lines are about to meet.
+constexpr int64_t PROJECT_MAX_N = 512;
+
 template <typename T, typename OUT>
 static void launch_linear_t(void* y, const void* x, const void* w, const void* bias, int64_t m,
                             int64_t n, int64_t k, int64_t x_stride, void* ws, bool skinny,
@@ -787,6 +892,12 @@ static void launch_linear_t(void* y, const void* x, const void* w, const void* b
     if (skinny) {
       launch_skinny<T, OUT>((const T*)x, (const T*)w, (const T*)bias, (OUT*)y, ws, (int)m, (int)n,
                             (int)k, x_stride, st);
+      return;
+    }
+  }
+  if constexpr (std::is_same<OUT, float>::value) {
+    if (bias == nullptr && n <= PROJECT_MAX_N && project_mfma_ok<T>(x, x_stride, w, k)) {
+      launch_project_mfma<T, true>((float*)y, x, x_stride, w, m, (int)n, (int)k, st);
       return;
     }
   }
@@ -999,6 +1110,29 @@ int mi355_linear(void* y, const void* x, const void* w, const void* bias, int64_
                        launch_linear<T>(y, x, w, bias, m, n, k, x_stride, workspace, skinny,
                                         out_f32, (hipStream_t)stream));
   MI355_CHECK_LAUNCH("linear");
+  return MI355_OK;
+}
+
+int mi355_project_f32(float* out, const void* x, int64_t x_stride, const void* weight, int64_t rows, int n, int k, int dtype, void* stream) {
+  MI355_REQUIRE(out && x && weight, MI355_ERR_INVALID, "project_f32: null pointer");
+  MI355_REQUIRE(rows >= 0 && rows < (1ll << 31) && n > 0 && n <= 65536 && k > 0 && x_stride >= k, MI355_ERR_INVALID, "project_f32: bad shape");
+  MI355_REQUIRE(dtype == MI355_BF16 || dtype == MI355_F16, MI355_ERR_UNSUPPORTED, "project_f32: 16-bit operands");
+  if (rows == 0) return MI355_OK;
+  const bool mfma = project_mfma_ok<bf16_t>(x, x_stride, weight, k);
+  const int64_t waves = rows * n;
+  MI355_REQUIRE(mfma || waves / 4 < (1ll << 31) - 1, MI355_ERR_UNSUPPORTED, "project_f32: too many results");
+#define MI355_PJ(T)                                                                                                             \
+  do {                                                                                                                          \
+    if (mfma)                                                                                                                   \
+      launch_project_mfma<T, false>(out, x, x_stride, weight, rows, n, k, (hipStream_t)stream);                                        \
+    else                                                                                                                        \
+      hipLaunchKernelGGL((project_f32_kernel<T>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream, out,    \
+                         (const T*)x, x_stride, (const T*)weight, rows, n, k);                                                  \
+  } while (0)
+  if (dtype == MI355_BF16) MI355_PJ(bf16_t);
+  else MI355_PJ(f16_t);
+#undef MI355_PJ
+  MI355_CHECK_LAUNCH("project_f32");
   return MI355_OK;
 }
 

@@ -8,7 +8,6 @@
 //     16-bit dtypes with K a multiple of 8 run on the matrix cores, reading both operands' fragments straight from
 //     global memory (a weight row and an input row are both contiguous along K, which is the fragment's direction);
 //     everything else (fp32: exact) on the vector ALU through LDS tiles,
-//   * mi355_project_f32: unrounded fp32 products of 16-bit rows with a small 16-bit table (router and gate logits),
 //   * mi355_clamped_glu: the clamped gated unit between an expert's two GEMMs, with the token's weight on the expert's INPUT.
 #include "common.cuh"
 
@@ -16,6 +15,10 @@
 #include <type_traits>
 
 namespace mi355 {
+int moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const void* w, const int32_t* row_map, int gather,
+                             const int32_t* tile_expert, const int32_t* tiles_used, int act, int64_t rows, int64_t n, int64_t k,
+                             int dtype, void* stream);   // gemm_tiled.hip
+
 namespace {
 
 constexpr int MOE_BLOCK = 64;
@@ -123,43 +126,74 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(int32_t* __restr
   }
 }
 
-// One workgroup.  src_row must hold `padded` entries, tile_expert padded / block.
+// One workgroup.  src_row must hold `padded` entries, tile_expert padded / block.  The pair that finds its expert's count at r is
+// that expert's row r: kept in registers, it is all the second pass needs (a thread's pairs past ALIGN_KEEP are counted again).
+// Bound by latency: one load of the ids, one LDS atomic, a scan by the first wave, the scattered stores.  12000 pairs of
+// 32 experts: 16.2 us with a serial scan and the ids read and counted twice, 9.2 us so; 256 pairs: 3.9 us.
+constexpr int ALIGN_KEEP = 16;
 __global__ __launch_bounds__(1024) void moe_align_kernel(int32_t* __restrict__ src_row, int32_t* __restrict__ rows,
                                                          int32_t* __restrict__ tile_expert, int32_t* __restrict__ n_tiles,
                                                          const int32_t* __restrict__ ids, int64_t pairs, int top, int E, int block,
                                                          int64_t padded) {
   extern __shared__ int smi[];
   int* count = smi;            // [E]
-  int* start = smi + E;        // [E + 1]
-  for (int e = threadIdx.x; e < E; e += blockDim.x) count[e] = 0;
-  for (int64_t p = threadIdx.x; p < padded; p += blockDim.x) src_row[p] = -1;
+  int* start = smi + E;        // [E]
+  int id[ALIGN_KEEP], rank[ALIGN_KEEP];
+#pragma unroll
+  for (int u = 0; u < ALIGN_KEEP; ++u) {
+    const int64_t i = threadIdx.x + (int64_t)u * 1024;
+    id[u] = i < pairs ? ids[i] : -1;
+  }
+  for (int e = threadIdx.x; e < E; e += 1024) count[e] = 0;
+  for (int64_t p = threadIdx.x; p < padded; p += 1024) src_row[p] = -1;
   __syncthreads();
-  for (int64_t i = threadIdx.x; i < pairs; i += blockDim.x) {
-    const int e = ids[i];
-    if (e >= 0 && e < E) atomicAdd(&count[e], 1);
+#pragma unroll
+  for (int u = 0; u < ALIGN_KEEP; ++u) rank[u] = id[u] >= 0 && id[u] < E ? atomicAdd(&count[id[u]], 1) : 0;
+  if (pairs > (int64_t)ALIGN_KEEP * 1024) {
+    __syncthreads();             // the kept pairs of an expert have its first rows
+    for (int64_t i = threadIdx.x + (int64_t)ALIGN_KEEP * 1024; i < pairs; i += 1024) {
+      const int e = ids[i];
+      if (e >= 0 && e < E) atomicAdd(&count[e], 1);
+    }
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0;
-    for (int e = 0; e < E; ++e) {
-      start[e] = at;
+  if (threadIdx.x < 64) {
+    // lane l has experts [l per, (l + 1) per): whole blocks of each, then where each starts
+    const int per = (E + 63) / 64, e0 = (int)threadIdx.x * per, e1 = min(e0 + per, E);
+    int blocks = 0;
+    for (int e = e0; e < e1; ++e) blocks += (count[e] + block - 1) / block;
+    int upto = blocks;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(upto, o, 64);
+      if ((int)threadIdx.x >= o) upto += up;
+    }
+    int at = upto - blocks;
+    for (int e = e0; e < e1; ++e) {
+      start[e] = at * block;
       const int nb = (count[e] + block - 1) / block;
-      for (int b = 0; b < nb; ++b) tile_expert[at / block + b] = e;
-      at += nb * block;
-      count[e] = 0;              // becomes the cursor
+      for (int j = 0; j < nb; ++j) tile_expert[at + j] = e;
+      at += nb;
     }
-    start[E] = at;
-    *n_tiles = at / block;
+    if (threadIdx.x == 63) *n_tiles = upto;
   }
   __syncthreads();
-  for (int64_t i = threadIdx.x; i < pairs; i += blockDim.x) {
+#pragma unroll
+  for (int u = 0; u < ALIGN_KEEP; ++u) {
+    const int64_t i = threadIdx.x + (int64_t)u * 1024;
+    if (i >= pairs) break;
+    const bool ok = id[u] >= 0 && id[u] < E;
+    const int p = ok ? start[id[u]] + rank[u] : 0;
+    if (ok) src_row[p] = (int)(i / top);
+    rows[i] = p;
+  }
+  if (pairs <= (int64_t)ALIGN_KEEP * 1024) return;
+  // the pairs that were not kept take an expert's rows from the last one down
+  for (int64_t i = threadIdx.x + (int64_t)ALIGN_KEEP * 1024; i < pairs; i += 1024) {
     const int e = ids[i];
-    if (e < 0 || e >= E) {
-      rows[i] = 0;
-      continue;
-    }
-    const int p = start[e] + atomicAdd(&count[e], 1);
-    src_row[p] = (int)(i / top);
+    const bool ok = e >= 0 && e < E;
+    const int p = ok ? start[e] + atomicSub(&count[e], 1) - 1 : 0;
+    if (ok) src_row[p] = (int)(i / top);
     rows[i] = p;
   }
 }
@@ -448,58 +482,6 @@ __global__ __launch_bounds__(256) void moe_router_logits_kernel(float* __restric
   }
 }
 
-// Unrounded fp32 products of few table rows: out[t][n] = x[t] . w[n] with T operands (a product of two 16-bit numbers is exact
-// in fp32).  A workgroup takes a 16 x 16 tile of the result; its eight waves walk every eighth 32-wide step of K on the matrix
-// cores and meet in LDS, in a fixed order whatever the number of rows.
-constexpr int PJ_WAVES = 8;
-template <typename T>
-__global__ __launch_bounds__(64 * PJ_WAVES) void project_f32_mfma_kernel(float* __restrict__ out, const T* __restrict__ x, int64_t x_stride,
-                                                                        const T* __restrict__ w, int64_t rows, int N, int K) {
-  using Frag = typename Mfma<T>::frag;
-  __shared__ __attribute__((aligned(16))) f32x4 part[PJ_WAVES][64];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
-  const int64_t t = (int64_t)blockIdx.x * 16 + li;
-  const int n = blockIdx.y * 16 + li;
-  // rows past either end read row 0; their results are not stored
-  const T* xr = x + (t < rows ? t : 0) * x_stride;
-  const T* wr = w + (int64_t)(n < N ? n : 0) * K;
-  const Frag zero = {};
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 32 * wv; k0 < K; k0 += 32 * PJ_WAVES) {
-    const bool in_k = k0 + 8 * lg < K;
-    const int k = in_k ? k0 + 8 * lg : 0;
-    const Frag av = *reinterpret_cast<const Frag*>(xr + k);
-    const Frag bv = *reinterpret_cast<const Frag*>(wr + k);
-    acc = Mfma<T>::run(in_k ? av : zero, bv, acc);
-  }
-  part[wv][lane] = acc;
-  __syncthreads();
-  if (wv != 0) return;
-#pragma unroll
-  for (int o = 1; o < PJ_WAVES; ++o) acc += part[o][lane];
-  if (n >= N) return;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int64_t row = (int64_t)blockIdx.x * 16 + 4 * lg + r;
-    if (row < rows) out[row * N + n] = acc[r];
-  }
-}
-
-// The same for widths that are no multiple of 8: one wave per result.
-template <typename T>
-__global__ __launch_bounds__(256) void project_f32_kernel(float* __restrict__ out, const T* __restrict__ x, int64_t x_stride,
-                                                          const T* __restrict__ w, int64_t rows, int N, int K) {
-  const int lane = threadIdx.x & 63;
-  const int64_t idx = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (idx >= rows * N) return;
-  const int64_t t = idx / N;
-  const int n = (int)(idx - t * N);
-  float acc = 0.f;
-  for (int k = lane; k < K; k += 64) acc = fmaf(to_f32(x[t * x_stride + k]), to_f32(w[(int64_t)n * K + k]), acc);
-  acc = wave_sum(acc);
-  if (lane == 0) out[idx] = acc;
-}
-
 // out[p][i] = g sigmoid(alpha g) (u + 1) with g = min(c a[p][i], limit), u = clamp(c a[p][ff + i], -limit, limit): a gated unit on
 // [gate | up] rows.  The rows are p = rows[j] (a token's sorted expert rows) for j < pairs, or j itself; c = coef[j], or 1: the
 // factor belongs on the layer's input, which it commutes with as the projections have no bias.
@@ -606,7 +588,7 @@ int mi355_moe_align(int32_t* src_row, int32_t* rows, int32_t* tile_expert, int32
   MI355_REQUIRE(padded % block == 0 && padded >= tokens * top + (int64_t)std::min<int64_t>(num_experts, tokens * top) * (block - 1),
                 MI355_ERR_INVALID, "moe_align: %lld padded rows cannot hold %lld pairs of %d experts", (long long)padded,
                 (long long)(tokens * top), num_experts);
-  const size_t lds = (size_t)(2 * num_experts + 1) * sizeof(int);
+  const size_t lds = (size_t)2 * num_experts * sizeof(int);
   hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), lds, (hipStream_t)stream, src_row, rows, tile_expert, n_tiles, ids,
                      tokens * top, top, num_experts, block, padded);
   MI355_CHECK_LAUNCH("moe_align");
@@ -619,8 +601,7 @@ int mi355_moe_grouped_linear(void* out, const void* in, int64_t in_stride, const
   MI355_REQUIRE(out && in && weight && src_row && tile_expert && n_tiles, MI355_ERR_INVALID, "moe_grouped_linear: null pointer");
   MI355_REQUIRE(act >= 0 && act <= 2, MI355_ERR_INVALID, "moe_grouped_linear: activation %d", act);
   if (block == MOE_TILED)
-    return mi355_moe_grouped_linear_tiled(out, in, in_stride, weight, gather ? src_row : nullptr, tile_expert, n_tiles, act,
-                                          padded, n, k, dtype, stream);
+    return moe_grouped_linear_tiled(out, in, in_stride, weight, src_row, gather, tile_expert, n_tiles, act, padded, n, k, dtype, stream);
   MI355_REQUIRE(block == MOE_BLOCK || block == MOE_WIDE, MI355_ERR_INVALID, "moe_grouped_linear: blocks of %d or %d rows", MOE_BLOCK,
                 MOE_WIDE);
   MI355_REQUIRE(padded >= 0 && padded % block == 0 && n > 0 && k > 0 && in_stride >= k && padded / block <= 65535,
@@ -636,31 +617,6 @@ int mi355_moe_grouped_linear(void* out, const void* in, int64_t in_stride, const
   });
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("moe_grouped_linear");
-  return MI355_OK;
-}
-
-int mi355_project_f32(float* out, const void* x, int64_t x_stride, const void* weight, int64_t rows, int n, int k, int dtype, void* stream) {
-  MI355_REQUIRE(out && x && weight, MI355_ERR_INVALID, "project_f32: null pointer");
-  MI355_REQUIRE(rows >= 0 && rows < (1ll << 31) && n > 0 && n <= 65536 && k > 0 && x_stride >= k, MI355_ERR_INVALID, "project_f32: bad shape");
-  MI355_REQUIRE(dtype == MI355_BF16 || dtype == MI355_F16, MI355_ERR_UNSUPPORTED, "project_f32: 16-bit operands");
-  if (rows == 0) return MI355_OK;
-  const bool mfma = k % 8 == 0 && x_stride % 8 == 0 && aligned16(x) && aligned16(weight);
-  const dim3 grid((unsigned)cdiv(rows, 16), (unsigned)cdiv(n, 16));
-  const int64_t waves = rows * n;
-  MI355_REQUIRE(mfma || waves / 4 < (1ll << 31) - 1, MI355_ERR_UNSUPPORTED, "project_f32: too many results");
-#define MI355_PJ(T)                                                                                                                   \
-  do {                                                                                                                                \
-    if (mfma)                                                                                                                         \
-      hipLaunchKernelGGL((project_f32_mfma_kernel<T>), grid, dim3(64 * PJ_WAVES), 0, (hipStream_t)stream, out, (const T*)x, x_stride, \
-                         (const T*)weight, rows, n, k);                                                                               \
-    else                                                                                                                              \
-      hipLaunchKernelGGL((project_f32_kernel<T>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream, out,          \
-                         (const T*)x, x_stride, (const T*)weight, rows, n, k);                                                        \
-  } while (0)
-  if (dtype == MI355_BF16) MI355_PJ(bf16_t);
-  else MI355_PJ(f16_t);
-#undef MI355_PJ
-  MI355_CHECK_LAUNCH("project_f32");
   return MI355_OK;
 }
 

@@ -76,7 +76,7 @@ class GroupedExperts(nn.Module):
         ops = get_ops()
         sixteen = h.dtype != torch.float32
         plan = ops.moe_align(expert_ids, self.num_experts, wide_ok=sixteen and self.hidden % 8 == 0 and self.ff % 8 == 0,
-                             tiled_ok=sixteen and h.shape[0] > 64 and h.stride(0) % 8 == 0
+                             tiled_ok=sixteen and h.stride(0) % 8 == 0
                              and ops.linear_tiled_supported(256, self.w_up.shape[1], self.hidden, h.dtype)
                              and ops.linear_tiled_supported(256, self.hidden, self.ff, h.dtype))
         if self.activation == "clamped_glu":

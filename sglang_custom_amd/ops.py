@@ -1527,8 +1527,8 @@ ROUTER_SKINNY_MAX_ROWS = 256
 
 
 def moe_router_logits(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """fp32 x [T, D] against the fp32 router table [E, D] -> exact fp32 logits [T, E].  Few rows go to a wave-per-row kernel
-    (a tiled GEMM with E columns would occupy a handful of CUs), many to the exact tiled GEMM."""
+    """fp32 x [T, D] against the fp32 router table [E, D] -> exact fp32 logits [T, E].  Few rows go to a wave-per-row kernel,
+    many to mi355_linear, which serves such narrow products with the fp32 matrix instructions."""
     _gpu(x, weight)
     assert x.dtype == torch.float32 and weight.dtype == torch.float32 and x.is_contiguous() and weight.is_contiguous()
     T, K = x.shape
@@ -1542,12 +1542,15 @@ def moe_router_logits(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 def moe_align(expert_ids: torch.Tensor, num_experts: int, wide_ok: bool = False, tiled_ok: bool = False) -> MoePlan:
     """wide_ok: the grouped GEMMs that follow can take blocks of 128 rows (16-bit operands, 16-byte rows); tiled_ok: they
-    can run on the prefill projection kernel over blocks of 256 rows (linear_tiled_supported for both of them).  The
-    larger blocks are used when the experts have at least two of them worth of rows on average."""
+    can run on the prefill projection kernel over blocks of 256 rows (linear_tiled_supported for both of them), which does
+    no work for the rows a block does not have and wins from half a row per expert on (one
+    GEMM of 32 experts of 2048 x 2048, 4 per token, in us against blocks of 64: 1 token 44 / 29, 4 tokens 48 / 45, 16: 53 / 82,
+    64: 55 / 91, 1024: 72 / 306; 64 experts of 1536 x 4096, 8 per token: 4 tokens 89 / 120, 64: 205 / 280).  Blocks of 128 are used, where those cannot be,
+    when the experts have at least two of them worth of rows on average."""
     _gpu(expert_ids)
     T, top = expert_ids.shape
     assert expert_ids.dtype == torch.int32 and expert_ids.is_contiguous()
-    wide = 2 if (tiled_ok and T * top >= 512 * num_experts) else 1 if ((wide_ok or tiled_ok) and T * top >= 256 * num_experts) else 0
+    wide = 2 if (tiled_ok and 2 * T * top >= num_experts) else 1 if (wide_ok and T * top >= 256 * num_experts) else 0
     block = int(_lib_().mi355_moe_block_rows(wide))
     pairs = T * top
     padded = (pairs + min(num_experts, pairs) * (block - 1) + block - 1) // block * block

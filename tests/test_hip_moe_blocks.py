@@ -1,0 +1,80 @@
+"""GPU: the mixture's block sizes and plans at their edges -- 256-row blocks that do no work for padding rows, the sorted plan past
+its register-kept pairs, narrow fp32 products -- against plain float64 / integer restatements."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sglang_custom_amd import ops as o
+
+    return o
+
+
+@pytest.mark.parametrize("T,E,top,block", [(1, 5, 1, 64), (3, 2, 2, 256), (64, 32, 4, 256), (300, 200, 2, 128), (5000, 32, 4, 256),
+                                           (16384, 3, 1, 64), (16385, 7, 1, 256), (9000, 1500, 3, 64)])
+def test_align_sorts_every_pair_once(ops, T, E, top, block):
+    g = torch.Generator().manual_seed(T + E)
+    ids = torch.rand(T, E, generator=g).topk(top, -1).indices.int() if E * T < 10 ** 7 else torch.randint(0, E, (T, top), generator=g).int()
+    if E > 4:
+        ids[ids == 1] = 0                      # one expert without rows
+    lib = ops._lib_()
+    padded = (T * top + min(E, T * top) * (block - 1) + block - 1) // block * block
+    src, rows = torch.empty(padded, dtype=torch.int32, device=DEV), torch.empty((T, top), dtype=torch.int32, device=DEV)
+    te, nt = torch.full((padded // block,), -7, dtype=torch.int32, device=DEV), torch.empty(1, dtype=torch.int32, device=DEV)
+    d = ids.to(DEV).contiguous()
+    ops.check(lib.mi355_moe_align(src.data_ptr(), rows.data_ptr(), te.data_ptr(), nt.data_ptr(), d.data_ptr(), T, top, E, block, padded,
+                                  ops._stream(d)), "moe_align")
+    src, rows, te, nt = src.cpu(), rows.cpu().long(), te.cpu(), int(nt.item())
+    counts = torch.bincount(ids.flatten().long(), minlength=E)
+    assert nt == int(((counts + block - 1) // block).sum())
+    assert rows.flatten().unique().numel() == T * top and int(rows.max()) < nt * block
+    assert torch.equal(src[rows], torch.arange(T, dtype=torch.int32)[:, None].expand(T, top))
+    assert torch.equal(te[rows // block], ids)
+    live = (src[: nt * block] >= 0).view(nt, block)
+    assert int(live.sum()) == T * top and not (~live[:, :-1] & live[:, 1:]).any()        # a block's rows lie in front of its padding
+    assert (src[nt * block:] == -1).all()
+
+
+@pytest.mark.parametrize("sizes", [(0, 1, 8), (15, 16, 17), (127, 128, 129), (255, 256, 257), (500, 3, 300)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_blocks_of_256_rows_skip_padding(ops, sizes, dtype):
+    """An expert's last block at every edge of the 8-, 16- and 128-row pieces; both GEMMs.  One rounding of the float64 product
+    (2^-8 / 2^-11 relative) plus the fp32 sums' 1e-5 of the row's scale."""
+    g = torch.Generator().manual_seed(sum(sizes))
+    E, K, N = 3, 192, 320
+    T = sum(sizes)
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(sizes)])[torch.randperm(T, generator=g)][:, None].contiguous()
+    x = torch.randn(T, K, generator=g).to(dtype)
+    up, down = (torch.randn(E, N, K, generator=g) * K ** -0.5).to(dtype), (torch.randn(E, K, N, generator=g) * N ** -0.5).to(dtype)
+    plan = ops.moe_align(ids.to(DEV), E, tiled_ok=True)
+    assert plan.block == 256
+    a = ops.moe_grouped_linear(x.to(DEV), up.to(DEV), plan, gather=True, gelu=False, relu2=True)
+    rows = plan.rows.long().cpu()[:, 0]
+    e = ids[:, 0].long()
+    want = torch.einsum("tk,tnk->tn", x.double(), up.double()[e]).clamp_min(0) ** 2
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert ((a.cpu()[rows].double() - want).abs() <= ulp * want.abs() + 1e-5 * 16).all()
+    b = ops.moe_grouped_linear(a, down.to(DEV), plan, gather=False, gelu=False).cpu()[rows]
+    want = torch.einsum("tn,tkn->tk", a.cpu()[rows].double(), down.double()[e])
+    assert ((b.double() - want).abs() <= ulp * want.abs() + 1e-5 * 16).all()
+
+
+@pytest.mark.parametrize("T,N,K,off", [(65, 1, 8, 0), (100, 16, 2048, 0), (257, 33, 200, 0), (300, 512, 264, 8), (1000, 5, 4, 0), (70, 513, 64, 0), (90, 40, 37, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_narrow_products_in_fp32(ops, T, N, K, off, dtype):
+    """fp32 results of mi355_linear on both sides of the narrow kernel's conditions.  Each of K terms and partial sums rounds once in
+    fp32: 2 sqrt(K) 2^-24 times the root of the summed squares bounds what is seen; 4 x that is allowed, and for bf16 operands the one
+    rounding of the sum to bf16 (half an ulp: 2^-9 relative, 2^-8 where the sum's own error moves it over a rounding boundary)."""
+    g = torch.Generator().manual_seed(T * N + K)
+    x, w = torch.randn(T, K + off, generator=g).to(dtype), torch.randn(N, K, generator=g).to(dtype)
+    got = ops.linear(x.to(DEV)[:, off:], w.to(DEV), out_dtype=torch.float32).cpu().double()
+    xd, wd = x[:, off:].double(), w.double()
+    want = xd @ wd.T
+    ulp = 0.0 if dtype == torch.float32 else 2.0 ** -8
+    assert ((got - want).abs() <= ulp * want.abs() + 8 * K ** 0.5 * 2.0 ** -24 * ((xd ** 2) @ (wd ** 2).T).sqrt() + 1e-12).all()
+    if dtype != torch.float32:
+        assert torch.equal(got, got.bfloat16().double())

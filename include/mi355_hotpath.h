@@ -402,6 +402,17 @@ int mi355_mla_prefill_assemble(void* q, void* k, void* v, const void* kv, const 
                                int heads, int nope_dim, int rope_dim, int v_dim, int kv_lora_rank, int64_t q_stride,
                                int64_t num_slots, int dtype, void* stream);
 
+/* Causal attention of whole sequences (nothing cached) whose per-head keys and values were expanded from one latent per token:
+ * q [tokens, heads, nope + rope] through q_stride, its rope part unrotated; kv [tokens, heads, nope keys | v values] through
+ * kv_stride; k_rope [tokens, rope] rotated key part that the heads share, rows k_rope_stride apart; out [tokens, heads, v]
+ * contiguous.  Sequence b is tokens seg_start[b] .. + seg_len[b], at most max_len long.  The first rot_dims features of q's rope
+ * part turn by positions[t] * inv_freq[i] (pairs 2 i, 2 i + 1 if interleaved, else i, i + rot_dims / 2), cos and sin times rot_mag. */
+int mi355_latent_prefill_attention_supported(int nope_dim, int rope_dim, int v_dim, int rot_dims, int interleaved, int dtype);
+int mi355_latent_prefill_attention(void* out, const void* q, int64_t q_stride, const void* kv, int64_t kv_stride, const void* k_rope,
+                                   int64_t k_rope_stride, const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions,
+                                   const float* inv_freq, int rot_dims, int interleaved, float rot_mag, int64_t bs, int64_t max_len,
+                                   int heads, int nope_dim, int rope_dim, int v_dim, float scale, int dtype, void* stream);
+
 /* ---- K12/K13 dense projection y = x @ W^T ------------------------------------------------------
  * x [M, K] (row stride x_stride), W [N, K] contiguous (nn.Linear layout), y [M, N] contiguous.
  * M <= 64 uses the weight-streaming MFMA kernel (bf16/f16); fp32 uses an exact-fp32 tiled kernel

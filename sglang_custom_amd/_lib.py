@@ -91,6 +91,8 @@ _SIGNATURES = {
     "mi355_per_token_quant_fp8": (I, [P, P, P, L, L, L, L, I, P]),
     "mi355_fp8_workspace_bytes": (L, [L, L, L]),
     "mi355_fp8_scaled_mm": (I, [P, P, P, P, P, P, L, L, L, P, L, I, P]),
+    "mi355_latent_prefill_attention_supported": (I, [I, I, I, I, I, I]),
+    "mi355_latent_prefill_attention": (I, [P, P, L, P, L, P, L, P, P, P, P, I, I, F, L, L, I, I, I, I, F, I, P]),
     "mi355_argmax": (I, [P, P, L, L, L, P]),
     "mi355_argmax_workspace_bytes": (L, [L]),
     "mi355_argmax_chunked": (I, [P, P, L, L, L, P, L, P]),

@@ -50,7 +50,7 @@ FAMILY_SOURCES = {
     "Fudonex": ["elementwise.hip", "index_ops.hip", "gemm.hip", "gemm_tiled.hip", "postnorm_ops.hip", "recurrence.hip",
                 "conv_ops.hip", "attn_window.hip"],
     "Silatar": ["elementwise.hip", "index_ops.hip", "gemm.hip", "gemm_tiled.hip", "stream_ops.hip", "attn_latent.hip", "postnorm_ops.hip",
-                "recurrence.hip", "moe_ops.hip", "conv_ops.hip", "mla_proj.hip"],
+                "recurrence.hip", "moe_ops.hip", "conv_ops.hip", "mla_proj.hip", "attn_extend.hip"],
     "Lomazen": ["elementwise.hip", "index_ops.hip", "gemm.hip", "gemm_tiled.hip", "stream_ops.hip", "postnorm_ops.hip", "moe_ops.hip",
                 "attn_causal.hip"],
 }

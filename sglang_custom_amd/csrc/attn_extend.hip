@@ -29,6 +29,16 @@ struct ExtendParams {
   // the cache buffers: elements between consecutive slots / consecutive kv heads ([slots, hkv, d] or head-major)
   int64_t kb_slot, kb_head, vb_slot, vb_head;
   int kv8;   // the cache holds e4m3fn bytes behind the element pointers (strides count bytes); read by the VALU kernel
+  // latent form (extend_attn_latent_kernel): whole sequences, tokens seg_start[b] .. + seg_len[b]
+  const int32_t* seg_start;
+  const int32_t* seg_len;
+  const int64_t* positions;   // [tokens]
+  const float* inv_freq;      // [rot_dims / 2]
+  const void* k_rope;         // [tokens, 64] rotated key part that the heads share, rows k_rope_stride apart
+  int64_t k_rope_stride;
+  int kv_head;                // elements between consecutive heads of k / v
+  int rot_dims, interleaved;  // of the query's rope part: features 2 i with 2 i + 1, or (rot_dims 64) i with i + 32
+  float rot_mag;
 };
 
 // DP: padded head dim (>= D, Dv; multiple of 64). BN: keys per tile. VEC: 16-B global loads.
@@ -560,7 +570,10 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // DQ: query / key head dimension, 128 or 192 (the multi-head form of MLA prefill: 128 nope + 64 rope features
 // against 128-wide values).  Features 128 .. 191 of the K tile are a second 256-byte-row image (half of each row
 // used) with the same chunk XOR, so the fragment reads of score steps 8 .. 11 are as conflict-free as the others.
-template <typename T, bool KV8, int DQ>
+// LATENT: no cached prefix; the heads' keys (features 0 .. 127) and values come interleaved per token and head out of one
+// projection of the latent, the keys' features 128 .. 191 from one row per token that the heads share, and the queries'
+// features 128 .. 191 are rotated here, in fp32 and rounded to T, as the absorbed kernels do it.
+template <typename T, bool KV8, int DQ, bool LATENT = false>
 __device__ __forceinline__ void extend_attn_mfma32_body(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs) {
@@ -581,10 +594,10 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const int t_in_pair = slot % per_pair;
   const int qb = nqb - 1 - t_in_pair / G;          // long (late) blocks first
   const int b = pair / p.hkv, kvh = pair % p.hkv, h = kvh * G + t_in_pair % G;
-  const int q_start = p.qo_indptr[b];
-  const int ext = p.qo_indptr[b + 1] - q_start;
-  const int kv_start = p.kv_indptr[b];
-  const int prefix = p.kv_indptr[b + 1] - kv_start;
+  const int q_start = LATENT ? p.seg_start[b] : p.qo_indptr[b];
+  const int ext = LATENT ? p.seg_len[b] : p.qo_indptr[b + 1] - q_start;
+  const int kv_start = LATENT ? 0 : p.kv_indptr[b];
+  const int prefix = LATENT ? 0 : p.kv_indptr[b + 1] - kv_start;
   const int r0 = qb * 128;
   if (r0 >= ext) return;   // whole workgroup: EXEC stays full for the transposed reads below
 
@@ -601,19 +614,58 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
 #pragma unroll
     for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const frag*>(qp + 16 * s);
   }
+  if constexpr (LATENT) {
+    // lane's features 16 (s - 8) + 8 hh + 0 .. 7 of the rope part: pairs of neighbours lie in one fragment, pairs (i, i + 32)
+    // in fragments s and s + 2
+    const float pos = (float)p.positions[q_start + qrow_c];
+    auto turn = [&](int i, T& a, T& c) {
+      float sn, cs;
+      sincosf(pos * p.inv_freq[i], &sn, &cs);
+      sn *= p.rot_mag;
+      cs *= p.rot_mag;
+      const float u = to_f32(a), w = to_f32(c);
+      a = from_f32<T>(u * cs - w * sn);
+      c = from_f32<T>(w * cs + u * sn);
+    };
+    if (p.interleaved) {
+#pragma unroll
+      for (int s = 8; s < NS; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const int i = (16 * (s - 8) + 8 * hh + e) >> 1;
+          if (2 * i < p.rot_dims) {
+            T a = qf[s][e], c = qf[s][e + 1];
+            turn(i, a, c);
+            qf[s][e] = a;
+            qf[s][e + 1] = c;
+          }
+        }
+    } else if (p.rot_dims == 64) {
+#pragma unroll
+      for (int s = 8; s < 10; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          T a = qf[s][e], c = qf[s + 2][e];
+          turn(16 * (s - 8) + 8 * hh + e, a, c);
+          qf[s][e] = a;
+          qf[s + 2][e] = c;
+        }
+    }
+  }
 
   const int last_row = min(r0 + 127, ext - 1);
-  const int total = p.is_causal ? prefix + last_row + 1 : prefix + ext;
+  const int total = LATENT || p.is_causal ? prefix + last_row + 1 : prefix + ext;
   const int n_tiles = (total + 63) / 64;
-  const int my_limit = p.is_causal ? prefix + qrow_c : prefix + ext - 1;   // last visible key of this lane's query
-  const int wave_min_limit = p.is_causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
-  const int wave_max_limit = p.is_causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
+  const int my_limit = LATENT || p.is_causal ? prefix + qrow_c : prefix + ext - 1;   // last visible key of this lane's query
+  const int wave_min_limit = LATENT || p.is_causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
+  const int wave_max_limit = LATENT || p.is_causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
 
   // tile staging: thread -> rows (threadIdx.x >> 4) + 16 i, 16-B chunk (threadIdx.x & 15)
   const int srow = threadIdx.x >> 4, sch = threadIdx.x & 15;
   Vec<T, 8> kreg[4], vreg[4], kreg2[WIDE ? 4 : 1];   // kreg2: features 128 + 8 sch .. + 7 (threads with sch < 8)
-  const T* k_lin = k_ext + (int64_t)(q_start - prefix + srow) * p.k_stride + (int64_t)kvh * DQ + sch * 8;
-  const T* v_lin = v_ext + (int64_t)(q_start - prefix + srow) * p.v_stride + (int64_t)kvh * D + sch * 8;
+  const T* k_lin = k_ext + (int64_t)(q_start - prefix + srow) * p.k_stride + (int64_t)kvh * (LATENT ? p.kv_head : DQ) + sch * 8;
+  const T* v_lin = v_ext + (int64_t)(q_start - prefix + srow) * p.v_stride + (int64_t)kvh * (LATENT ? p.kv_head : D) + sch * 8;
+  const T* r_lin = LATENT ? (const T*)p.k_rope + (int64_t)(q_start + srow) * p.k_rope_stride + sch * 8 : nullptr;
   auto load_tile = [&](int kt) {
     if (kt * 64 >= prefix && kt * 64 + 63 < total) {   // whole tile in the extend part (workgroup-uniform)
 #pragma unroll
@@ -622,8 +674,18 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
         kreg[i] = ldvec<T, 8>(k_lin + key * p.k_stride);
         vreg[i] = ldvec<T, 8>(v_lin + key * p.v_stride);
         if constexpr (WIDE) {
-          if (sch < 8) kreg2[i] = ldvec<T, 8>(k_lin + key * p.k_stride + 128);
+          if (sch < 8) kreg2[i] = LATENT ? ldvec<T, 8>(r_lin + key * p.k_rope_stride) : ldvec<T, 8>(k_lin + key * p.k_stride + 128);
         }
+      }
+      return;
+    }
+    if constexpr (LATENT) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t key = min(kt * 64 + srow + 16 * i, total - 1) - srow;
+        kreg[i] = ldvec<T, 8>(k_lin + key * p.k_stride);
+        vreg[i] = ldvec<T, 8>(v_lin + key * p.v_stride);
+        if (sch < 8) kreg2[i] = ldvec<T, 8>(r_lin + key * p.k_rope_stride);
       }
       return;
     }
@@ -832,6 +894,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   extend_attn_mfma32_body<T, false, 192>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
 }
 
+// Whole prompts over a latent cache (rank 512 + 64) in expanded form: per visible pair and head 2 (128 + 64 + 128) flops
+// instead of the absorbed form's 2 (512 + 64 + 512), for one projection of every latent to its heads' keys and values (4 x 1900
+// tokens x 16 heads: 230 us, and about 70 for that projection; the absorbed launch with its two per-head products took 1570 us).
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void extend_attn_latent_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o, ExtendParams p, int nqb, int npairs) {
+  extend_attn_mfma32_body<T, false, 192, true>(q, k, v, o, nullptr, nullptr, p, nqb, npairs);
+}
+
 template <typename T, int DP, int BN>
 static int launch_extend_cfg(const void* q, const void* k, const void* v, void* o, const void* kb,
                              const void* vb, const ExtendParams& p, int64_t bs,
@@ -983,6 +1054,44 @@ int mi355_extend_attention(const void* q_extend, const void* k_extend, const voi
                                              v_buffer, p, bs, max_len_extend, kv8, (hipStream_t)stream));
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("extend_attention");
+  return MI355_OK;
+}
+
+int mi355_latent_prefill_attention_supported(int nope_dim, int rope_dim, int v_dim, int rot_dims, int interleaved, int dtype) {
+  return (dtype == MI355_BF16 || dtype == MI355_F16) && nope_dim == 128 && rope_dim == 64 && v_dim == 128 && rot_dims >= 0 &&
+         rot_dims <= 64 && rot_dims % 2 == 0 && (interleaved || rot_dims == 0 || rot_dims == 64);
+}
+
+int mi355_latent_prefill_attention(void* out, const void* q, int64_t q_stride, const void* kv, int64_t kv_stride, const void* k_rope,
+                                   int64_t k_rope_stride, const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions,
+                                   const float* inv_freq, int rot_dims, int interleaved, float rot_mag, int64_t bs, int64_t max_len,
+                                   int heads, int nope_dim, int rope_dim, int v_dim, float scale, int dtype, void* stream) {
+  MI355_REQUIRE(out && q && kv && k_rope && seg_start && seg_len && positions && (inv_freq || rot_dims == 0), MI355_ERR_INVALID,
+                "latent_prefill_attention: null pointer");
+  MI355_REQUIRE(mi355_latent_prefill_attention_supported(nope_dim, rope_dim, v_dim, rot_dims, interleaved, dtype), MI355_ERR_UNSUPPORTED,
+                "latent_prefill_attention: 16-bit heads of 128 + 64 key and 128 value features (nope=%d rope=%d v=%d rot=%d dtype=%d)",
+                nope_dim, rope_dim, v_dim, rot_dims, dtype);
+  MI355_REQUIRE(bs >= 0 && max_len >= 0 && heads > 0 && scale > 0.f, MI355_ERR_INVALID, "latent_prefill_attention: bad shape");
+  MI355_REQUIRE(q_stride >= (int64_t)heads * 192 && q_stride % 8 == 0 && kv_stride >= (int64_t)heads * 256 && kv_stride % 8 == 0 &&
+                    k_rope_stride >= 64 && k_rope_stride % 8 == 0 && aligned16(q) && aligned16(kv) && aligned16(k_rope) && aligned16(out),
+                MI355_ERR_INVALID, "latent_prefill_attention: rows must be 16-byte aligned and hold every head");
+  if (bs == 0 || max_len == 0) return MI355_OK;
+  ExtendParams p = {};
+  p.seg_start = seg_start; p.seg_len = seg_len; p.positions = positions; p.inv_freq = inv_freq;
+  p.rot_dims = rot_dims; p.interleaved = interleaved; p.rot_mag = rot_mag;
+  p.q_stride = q_stride; p.k_stride = p.v_stride = kv_stride; p.kv_head = 256;
+  p.k_rope = k_rope; p.k_rope_stride = k_rope_stride;
+  p.is_causal = 1; p.hq = p.hkv = heads; p.D = 192; p.Dv = 128; p.sm_scale = scale;
+  const int nqb = (int)((max_len + 127) / 128);
+  const int64_t npairs = bs * heads, wgs = 8 * ((npairs + 7) / 8) * nqb;
+  MI355_REQUIRE(wgs < (int64_t)1 << 31, MI355_ERR_UNSUPPORTED, "latent_prefill_attention: too many query blocks");
+#define MI355_LP(T)                                                                                                            \
+  hipLaunchKernelGGL((extend_attn_latent_kernel<T>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, (const T*)q,       \
+                     (const T*)kv, (const T*)kv + 128, (T*)out, p, nqb, (int)npairs)
+  if (dtype == MI355_BF16) MI355_LP(bf16_t);
+  else MI355_LP(f16_t);
+#undef MI355_LP
+  MI355_CHECK_LAUNCH("latent_prefill_attention");
   return MI355_OK;
 }
 

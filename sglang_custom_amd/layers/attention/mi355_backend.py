@@ -21,6 +21,7 @@ from typing import Optional
 import torch
 
 from ...ops_backend import get_ops
+from ..quantization.unquant import SKINNY_MAX_M
 from .base_attn_backend import AttentionBackend
 
 MAX_KV_SPLITS = 64
@@ -323,6 +324,25 @@ class Mi355AttnBackend(AttentionBackend):
             forward_batch.positions, layer.sink.data if layer.sink is not None else None, layer.inv_freq, layer.rot_dims, layer.window,
             layer.scaling, gate=gate, tok_req=forward_batch.token_req_index(), blocks=self._latent_blocks(forward_batch, bq),
             num_splits=splits, interleaved=layer.interleaved, rot_mag=layer.rot_mag)
+
+    def latent_prefill_ok(self, layer, forward_batch, nope: int, v: int, dtype) -> bool:
+        """Whether forward_latent_prefill serves the step: whole prompts (nothing cached), every earlier token, a plain softmax,
+        more tokens than the decode-sized kernels take."""
+        return (not forward_batch.forward_mode.is_decode_or_idle() and forward_batch.extend_prefix_lens_cpu is not None
+                and not any(forward_batch.extend_prefix_lens_cpu) and layer.window == 0 and layer.sink is None
+                and forward_batch.extend_num_tokens > SKINNY_MAX_M and str(self.device).startswith("cuda")
+                and get_ops().latent_prefill_attention_supported(nope, layer.rope_dim, v, layer.rot_dims, layer.interleaved, dtype))
+
+    def forward_latent_prefill(self, q, expand, layer, forward_batch, cache_layer=None):
+        """q [T, H, nope + rope] with its rope part unrotated; expand(c [T, rank]) -> [T, H, nope + v], every head's keys and
+        values from the latents -> [T, H, v].  The new tokens' rows are in the cache already."""
+        ops = get_ops()
+        rows = ops.embedding(forward_batch.out_cache_loc,
+                             forward_batch.token_to_kv_pool.get_key_buffer(layer.layer_id if cache_layer is None else cache_layer))
+        return ops.latent_prefill_attention(
+            q, expand(rows[:, : layer.kv_rank]), rows[:, layer.kv_rank:], forward_batch.extend_start_loc, forward_batch.extend_seq_lens,
+            forward_batch.positions, layer.inv_freq, layer.rot_dims, max(forward_batch.extend_seq_lens_cpu), layer.scaling,
+            interleaved=layer.interleaved, rot_mag=layer.rot_mag)
 
     # ---- causal attention with sigmoid weights (no softmax) over per-layer key / value buffers ----
     def forward_sigmoid(self, q, layer, forward_batch, out):

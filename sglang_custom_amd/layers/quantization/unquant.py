@@ -158,6 +158,14 @@ def decode_linear_deferred(layer, x, needs_all_reduce: bool = True):
     return None if part is None else SplitKPartials(part)
 
 
+def prefill_linear(x2: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """16-bit rows [M, K] (M > SKINNY_MAX_M) against a plain weight [N, K]."""
+    if (x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and weight.is_contiguous()
+            and _use_tiled(x2.shape[0], weight.shape[0], weight.shape[0], weight.shape[1], x2.dtype, False)):
+        return get_ops().linear_tiled(x2, weight, bias)
+    return F.linear(x2, weight, bias)
+
+
 class UnquantizedLinearMethod:
     def process_weights_after_loading(self, layer) -> None:
         pack_for_decode(layer)
@@ -166,10 +174,6 @@ class UnquantizedLinearMethod:
         x2 = x.view(-1, x.shape[-1])
         if x2.shape[0] <= SKINNY_MAX_M or x2.dtype == torch.float32 or not x2.is_cuda:
             y = decode_linear(layer, x2, bias)
-        elif (x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and layer.weight.is_contiguous()
-              and _use_tiled(x2.shape[0], layer.weight.shape[0], layer.weight.shape[0], layer.weight.shape[1],
-                             x2.dtype, False)):
-            y = get_ops().linear_tiled(x2, layer.weight, bias)
         else:
-            y = F.linear(x2, layer.weight, bias)
+            y = prefill_linear(x2, layer.weight, bias)
         return y.view(*x.shape[:-1], y.shape[-1])

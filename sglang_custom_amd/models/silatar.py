@@ -17,7 +17,8 @@ latent attention and the mixture.)
 Per layer run (T tokens, width D), besides the GEMMs' own launches:
 
   latent_attention   in_proj [q | kv latent | shared key part]; LatentWindowAttention.write_rows (latent norm, rotation, cache row);
-                     W_uk per head; LatentWindowAttention (rotation of q inside); W_uv per head; o
+                     W_uk per head; LatentWindowAttention (rotation of q inside); W_uv per head; o.  Whole prompts instead
+                     expand the latents to every head's keys and values (one projection) and attend over those
   mlstm              in_proj [q | k | v | g] and, in unrounded fp32, [i | f]; MatrixMemory; HeadNormGate; o
   LayerNormResidualAdd   x += L(y) in place, and the layer norm in front of the next sublayer              1 launch, fp32
   dense              up, gelu, down
@@ -42,6 +43,7 @@ from ..layers.linear_recurrence import HeadNormGate, MatrixMemory
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import LayerNormResidualAdd
+from ..layers.quantization.unquant import prefill_linear
 from ..layers.rotary_embedding import scaled_pair_inv_freq
 from ..layers.token_shift import ShiftedLayerNorm
 from ..layers.vocab_parallel_embedding import ParallelLMHead
@@ -58,6 +60,7 @@ class SilatarLatentAttention(nn.Module):
         self.kv_norm = nn.Parameter(torch.ones(rank, dtype=dtype, device=device), requires_grad=False)
         self.uk = PerHeadLinear(H, dn, rank, dtype, device)      # absorbed: q_nope -> latent (the transpose of the key expansion)
         self.uv = PerHeadLinear(H, rank, dv, dtype, device)
+        self.kv_expand = None      # [H (dn + dv), rank]: every head's keys and values of a latent, for whole prompts
         self.o_proj = ReplicatedLinear(H * dv, hidden, dtype, device)
         rot = mx.get("rot") or {}
         dims = int(rot.get("dims", 0))
@@ -70,10 +73,20 @@ class SilatarLatentAttention(nn.Module):
         p = self.in_proj(h)[0]
         self.attn.write_rows(p, self.q_width, self.kv_norm.data, self.eps, positions, forward_batch, cache_layer=run)
         q = p[:, : self.q_width].view(T, H, self.dn + self.dr)
+        if self.kv_expand is not None and forward_batch.attn_backend.latent_prefill_ok(self.attn, forward_batch, self.dn, self.dv, h.dtype):
+            # nothing cached: keys and values per head cost less than scores and sums in the latent space
+            expand = lambda c: prefill_linear(c, self.kv_expand).view(T, H, self.dn + self.dv)
+            o = forward_batch.attn_backend.forward_latent_prefill(q, expand, self.attn, forward_batch, cache_layer=run)
+            return self.o_proj(o.view(T, H * self.dv))[0]
         qa = self.uk(q[..., : self.dn])
         o_lat = torch.empty((H, T, self.rank), dtype=h.dtype, device=h.device).transpose(0, 1)
         self.attn(qa, q[..., self.dn:], None, forward_batch, o_lat, cache_layer=run)
         return self.o_proj(self.uv(o_lat).reshape(T, H * self.dv))[0]
+
+
+    def process_weights_after_loading(self) -> None:
+        w = torch.cat([self.uk.weight.data.transpose(1, 2), self.uv.weight.data], 1)
+        self.kv_expand = w.reshape(self.H * (self.dn + self.dv), self.rank).contiguous() if w.is_cuda and w.dtype != torch.float32 else None
 
 
 class SilatarMatrixMemory(nn.Module):
@@ -270,7 +283,7 @@ class SilatarForCausalLM(nn.Module):
         for module in self.modules():
             if isinstance(module, ReplicatedLinear):
                 module.quant_method.process_weights_after_loading(module)
-            elif isinstance(module, PerHeadLinear):
+            elif isinstance(module, (PerHeadLinear, SilatarLatentAttention)):
                 module.process_weights_after_loading()
 
     @torch.no_grad()

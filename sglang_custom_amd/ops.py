@@ -1282,6 +1282,32 @@ def latent_window_attention(qa: torch.Tensor, qr: torch.Tensor, cache: torch.Ten
     return out
 
 
+def latent_prefill_attention_supported(nope: int, rope: int, v: int, rot_dims: int, interleaved: bool, dtype: torch.dtype) -> bool:
+    return dtype in _DT and bool(_lib_().mi355_latent_prefill_attention_supported(nope, rope, v, rot_dims, int(bool(interleaved)), _DT[dtype]))
+
+
+def latent_prefill_attention(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Tensor, seg_start: torch.Tensor, seg_len: torch.Tensor,
+                             positions: torch.Tensor, inv_freq: torch.Tensor, rot_dims: int, max_len: int, scale: float,
+                             interleaved: bool = False, rot_mag: float = 1.0) -> torch.Tensor:
+    """Causal attention of whole sequences over expanded latents: q [T, H, nope + rope] (any row stride), rope part unrotated; kv
+    [T, H, nope + v]; k_rope [T, rope] (any row stride) rotated -> [T, H, v]."""
+    _gpu(q, kv, k_rope, seg_start, seg_len, positions, inv_freq)
+    T, H, d = q.shape
+    rope = k_rope.shape[1]
+    nope = d - rope
+    v = kv.shape[2] - nope
+    assert q.stride(2) == 1 and q.stride(1) == d and kv.stride(2) == 1 and kv.stride(1) == nope + v and k_rope.stride(1) == 1
+    assert kv.shape[:2] == (T, H) and k_rope.shape[0] == T and positions.numel() == T
+    assert q.dtype == kv.dtype == k_rope.dtype and seg_start.dtype == seg_len.dtype == torch.int32 and positions.dtype == torch.int64
+    assert inv_freq.dtype == torch.float32 and 2 * inv_freq.numel() >= rot_dims
+    out = torch.empty((T, H, v), dtype=q.dtype, device=q.device)
+    check(_lib_().mi355_latent_prefill_attention(out.data_ptr(), q.data_ptr(), q.stride(0), kv.data_ptr(), kv.stride(0), k_rope.data_ptr(),
+                                                 k_rope.stride(0), seg_start.data_ptr(), seg_len.data_ptr(), positions.data_ptr(),
+                                                 inv_freq.data_ptr(), rot_dims, int(bool(interleaved)), float(rot_mag), seg_len.numel(),
+                                                 int(max_len), H, nope, rope, v, float(scale), _dt(q), _stream(q)), "latent_prefill_attention")
+    return out
+
+
 # ------------------------------------------------------- post-norm fp32 stream, head norms and rotations
 def scaled_add_group_rmsnorm(x: torch.Tensor, branch: Optional[torch.Tensor], alpha: float, weight: torch.Tensor, groups: int,
                              eps: float, rows: Optional[torch.Tensor] = None, coef: Optional[torch.Tensor] = None,

@@ -132,12 +132,340 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
   }
 }
 
+// ---- the recurrences with one decay per head and token over a step's many tokens, 64 of them at a time ------------------
+// Inside a chunk the decays multiply out: with L_t the sum of their logarithms from the chunk's start to token t, the state at
+// its start S0 and w_s = 1 (or the step size dt_s),
+//     out_t = e^(L_t) S0^T q_t + sum_{s <= t} e^(L_t - L_s) (q_t . k_s) w_s u_s,     S <- e^(L_end) S0 + sum_s e^(L_end - L_s) w_s k_s u_s^T
+// where u_s = v_s for the state-space form, and for the delta rule the solution of the unit lower triangular system
+//     u_t + beta_t sum_{s < t} e^(L_t - L_s) (k_t . k_s) u_s = beta_t (v_t - e^(L_t) S0^T k_t).
+// All of it is matrix products: the weights q . k and k . k and the state's update on the double matrix instruction, rounded once
+// (their errors are the results' where decays are strong), everything else on the fp32 one; the triangular system is solved in
+// blocks of 16 tokens with their inverses.  L is summed in double and
+// kept as two floats, so that differences of long sums lose nothing.  Exponents are never positive.
+// One workgroup of 8 waves per (sequence, head, 32 value columns), chunk after chunk; the next chunk's rows are on their way
+// while one is multiplied.  A token by token launch is a chain of LDS reads, multiply-adds and lane exchanges of 1000 (plain) and
+// 1400 (delta) cycles a token, on one wave per SIMD: 4 x 1900 tokens, 16 heads of 64 x 128 took 800 and 1105 us; this takes
+// 214 and 342 (161 and 265 with every product in fp32, whose errors were 1.4 and 1.7 times the token by token form's at
+// strong decays; now they are 0.6 to 1.0 times), bound by the matrix instructions' issue and five to eight barriers a chunk.
+// What a later token of a chunk holds is multiplied by zero for an earlier one: an infinite or NaN input reaches the outputs of
+// its own sequence's chunk, not only those behind it.
+constexpr int CK = 64;               // tokens of a chunk, and key channels (padded)
+constexpr int CLD = CK + 4;          // LDS row: the 16 rows of a 16-byte fragment read fall into different banks
+constexpr int CK_THREADS = 512;
+
+__device__ __forceinline__ f32x4 f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ void mma4(f32x4& acc, const f32x4& a, const f32x4& b) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+}
+// sum_k A[i][k] B[j][k] over 64 of k; a, b: this lane's row li at k = 4 lg.  Four sums of 16 that meet in pairs: a chain of 64
+// roundings shows in results that are little more than one such product.
+__device__ __forceinline__ f32x4 tile_mma(const float* a, const float* b) {
+  f32x4 p[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) p[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      p[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4(a + 16 * k)[j], f4(b + 16 * k)[j], p[k], 0, 0, 0);
+  return (p[0] + p[1]) + (p[2] + p[3]);
+}
+
+// The same for weights, whose errors a strong decay leaves as the results': summed in double, rounded once.  The double instruction
+// hands row 4 r + lg of its 16 to register r, so row i of A is loaded from row 4 (i & 3) + (i >> 2) of the tile: lane lg then holds
+// rows 4 lg + r as in the fp32 layout.  a: the tile's first row, b: this lane's row, both at k = 0.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 tile_mma_exact(const float* a, const float* b, int li, int lg) {
+  const float* ar = a + (4 * (li & 3) + (li >> 2)) * CLD + 4 * lg;
+  const float* br = b + 4 * lg;
+  f64x4 p = f64x4{0., 0., 0., 0.}, o = p;
+#pragma unroll
+  for (int k = 0; k < 4; k += 2) {
+    const f32x4 a0 = f4(ar + 16 * k), b0 = f4(br + 16 * k), a1 = f4(ar + 16 * k + 16), b1 = f4(br + 16 * k + 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      p = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a0[j], (double)b0[j], p, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a1[j], (double)b1[j], o, 0, 0, 0);
+    }
+  }
+  p += o;
+  return f32x4{(float)p[0], (float)p[1], (float)p[2], (float)p[3]};
+}
+
+struct ChunkArgs {
+  float* out;
+  float* state;
+  const void* q;
+  const void* k;
+  const void* v;
+  const float* logits;        // [tokens][heads] step-size (plain) or decay (delta) logits
+  const float* bias;          // [heads]
+  const float* rate_log;      // [heads]
+  const float* skip;          // plain: [heads] or null
+  const void* beta_logits;    // delta: [tokens][heads]
+  const int32_t* req_to_state;
+  const int64_t* req_pool_indices;
+  const int32_t* seg_start;
+  const int32_t* seg_len;
+  const int64_t* positions;
+  int64_t q_stride, k_stride, v_stride, logit_stride, beta_stride;
+  int heads, qk_heads, dk, dv, beta_f32;
+  float q_scale;
+};
+
+template <typename QT, typename VT, bool DELTA>
+__global__ __launch_bounds__(CK_THREADS) void chunk_recurrence_kernel(ChunkArgs p) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* const Q = lds;                       // [t][d]
+  float* const K = Q + CK * CLD;              // [t][d]
+  float* const KT = K + CK * CLD;             // [d][t]
+  float* const M = KT + CK * CLD;             // [t][s] weights of u_s in out_t
+  float* const ST = M + CK * CLD;             // [c][d] state
+  float* const U = ST + RC_COLS * CLD;        // [c][t] v, then the right-hand side, then u
+  float* const L0 = U + RC_COLS * CLD;        // [t] L, upper part
+  float* const L1 = L0 + CK;                  // [t] lower part
+  float* const EL = L1 + CK;                  // [t] e^(L_t)
+  float* const WS = EL + CK;                  // [s] e^(L_end - L_s) w_s
+  float* const W = WS + CK;                   // [s] w_s (plain) or beta_t (delta)
+  float* const A = W + CK;                    // delta: [t][s] strictly lower part of the system
+  float* const INV = A + CK * CLD;            // delta: [4][16][20] inverses of its diagonal blocks
+  const int b = blockIdx.z, h = blockIdx.y, c0 = blockIdx.x * RC_COLS;
+  const int hq = h / (p.heads / p.qk_heads);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const int64_t t0 = p.seg_start[b];
+  const int n = p.seg_len[b];
+  if (n <= 0) return;
+  const int64_t slot = p.req_to_state[p.req_pool_indices[b]];
+  float* const sp = p.state + ((slot * p.heads + h) * (int64_t)p.dk) * p.dv;
+  const bool fresh = p.positions[t0] == 0;
+  const float rate = expf(p.rate_log[h]), bias = p.bias[h];
+  const float skip = !DELTA && p.skip != nullptr ? p.skip[h] : 0.f;
+  const QT* const qg = (const QT*)p.q;
+  const QT* const kg = (const QT*)p.k;
+  const VT* const vg = (const VT*)p.v;
+
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
+    ST[c * CLD + i] = (!fresh && i < p.dk && c0 + c < p.dv) ? sp[(int64_t)i * p.dv + c0 + c] : 0.f;
+  }
+  // this wave's tile of the state: d = 16 (wave >> 1) + 4 lg + r, column 16 (wave & 1) + li
+  const int sd = (wave >> 1) * 16, sc = (wave & 1) * 16;
+
+  // the next chunk's elements: 8 of q and of k (element tid + 512 u is token e >> 6, channel e & 63), 4 of v, one logit (or two)
+  QT qr[8], kr[8];
+  VT vr[4];
+  float zr = 0.f, br = 0.f;
+  auto request = [&](int base) {
+    const int m = n - base;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = tid + CK_THREADS * u, t = min(e >> 6, m - 1), i = min(e & 63, p.dk - 1);
+      qr[u] = qg[(t0 + base + t) * p.q_stride + (int64_t)hq * p.dk + i];
+      kr[u] = kg[(t0 + base + t) * p.k_stride + (int64_t)hq * p.dk + i];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + CK_THREADS * u, t = min(e >> 5, m - 1), c = min(c0 + (e & 31), p.dv - 1);
+      vr[u] = vg[(t0 + base + t) * p.v_stride + (int64_t)h * p.dv + c];
+    }
+    if (tid < 64) {
+      const int64_t t = t0 + base + min(tid, m - 1);
+      zr = p.logits[t * p.logit_stride + h];
+      if (DELTA)
+        br = p.beta_f32 ? static_cast<const float*>(p.beta_logits)[t * p.beta_stride + h]
+                        : to_f32(static_cast<const VT*>(p.beta_logits)[t * p.beta_stride + h]);
+    }
+  };
+  request(0);
+
+  for (int base = 0; base < n; base += CK) {
+    const int m = min(CK, n - base);
+    __syncthreads();                     // the last chunk is done with, the state is in LDS
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = tid + CK_THREADS * u, t = e >> 6, i = e & 63;
+      const bool in = t < m && i < p.dk;
+      const float kv = in ? to_f32(kr[u]) : 0.f;
+      Q[t * CLD + i] = in ? to_f32(qr[u]) * p.q_scale : 0.f;
+      K[t * CLD + i] = kv;
+      KT[i * CLD + t] = kv;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + CK_THREADS * u, t = e >> 5, c = e & 31;
+      U[c * CLD + t] = t < m && c0 + c < p.dv ? to_f32(vr[u]) : 0.f;
+    }
+    if (tid < 64) {
+      const float sp_ = softplus_f(zr + bias);
+      float la = -rate * sp_;
+      la = la < -1e4f ? -1e4f : la;      // e^-10000 is zero as well, and differences of sums stay finite
+      if (lane >= m) la = 0.f;
+      double sum = (double)la;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const double up = __shfl_up(sum, o, 64);
+        if (lane >= o) sum += up;
+      }
+      const double end = __shfl(sum, 63, 64);
+      const float hi = (float)sum;
+      L0[lane] = hi;
+      L1[lane] = (float)(sum - (double)hi);
+      EL[lane] = expf(hi);
+      const float w = DELTA ? 1.0f / (1.0f + expf(-br)) : sp_;
+      W[lane] = lane < m ? w : 0.f;
+      WS[lane] = expf((float)(end - sum)) * (DELTA ? 1.f : lane < m ? w : 0.f);
+    }
+    __syncthreads();
+    if (base + CK < n) request(base + CK);
+    const float el_end = EL[CK - 1];
+
+    // weights: tiles (s, t) on and under the diagonal; lane holds s = 16 ts + 4 lg + r of token t = 16 tt + li
+    for (int x = wave; x < 10; x += 8) {
+      const int tt = x < 1 ? 0 : x < 3 ? 1 : x < 6 ? 2 : 3, ts = x - tt * (tt + 1) / 2;
+      const int t = tt * 16 + li, s = ts * 16 + 4 * lg;
+      const f32x4 qk = tile_mma_exact(K + ts * 16 * CLD, Q + t * CLD, li, lg);
+      const f32x4 l0 = f4(L0 + s), l1 = f4(L1 + s), w = f4(W + s);
+      const float lt0 = L0[t], lt1 = L1[t];
+      f32x4 o, a;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        a[r] = expf(fminf((lt0 - l0[r]) + (lt1 - l1[r]), 0.f));
+        o[r] = s + r <= t ? qk[r] * a[r] * (DELTA ? 1.f : w[r]) : 0.f;
+      }
+      *reinterpret_cast<f32x4*>(M + t * CLD + s) = o;
+      if constexpr (DELTA) {
+        const f32x4 kk = tile_mma_exact(K + ts * 16 * CLD, K + t * CLD, li, lg);
+        const float beta = W[t];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = s + r < t ? kk[r] * a[r] * beta : 0.f;
+        *reinterpret_cast<f32x4*>(A + t * CLD + s) = o;
+      }
+    }
+    if constexpr (DELTA) {
+      // right-hand side: lane holds tokens t = 16 (wave >> 1) + 4 lg + r of column 16 (wave & 1) + li
+      const f32x4 y = tile_mma(K + (sd + li) * CLD + 4 * lg, ST + (sc + li) * CLD + 4 * lg);
+      float* const up = U + (sc + li) * CLD + sd + 4 * lg;
+      const f32x4 vv = f4(up), el = f4(EL + sd + 4 * lg), be = f4(W + sd + 4 * lg);
+      f32x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = be[r] * (vv[r] - el[r] * y[r]);
+      *reinterpret_cast<f32x4*>(up) = o;
+      __syncthreads();
+      // inverses of the four diagonal blocks: wave w, lane j < 16 has column j of block w
+      if (wave < 4 && lane < 16) {
+        float x[16];
+        const float* a = A + (wave * 16) * CLD + wave * 16;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+          float acc = lane == t ? 1.f : 0.f;
+#pragma unroll
+          for (int s4 = 0; s4 < t; s4 += 4) {
+            const f32x4 av = f4(a + t * CLD + s4);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (s4 + r < t) acc = fmaf(-av[r], x[s4 + r], acc);
+          }
+          x[t] = acc;
+          INV[(wave * 16 + t) * 20 + lane] = acc;
+        }
+      }
+      __syncthreads();
+      // two waves, 16 columns each: block by block, what the earlier blocks take off and the diagonal block's inverse
+      if (wave < 2) {
+        float* const uc = U + (wave * 16 + li) * CLD;
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) {
+          f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int s = 0; s < blk; ++s) mma4(acc, f4(A + (blk * 16 + li) * CLD + s * 16 + 4 * lg), f4(uc + s * 16 + 4 * lg));
+          f32x4 rhs = f4(uc + blk * 16 + 4 * lg) - acc;     // lane: tokens 16 blk + 4 lg + r of column li, which is also a B row's k
+          f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
+          mma4(x, f4(INV + (blk * 16 + li) * 20 + 4 * lg), rhs);
+          *reinterpret_cast<f32x4*>(uc + blk * 16 + 4 * lg) = x;
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+      }
+    }
+    __syncthreads();
+    // outputs: wave takes column tile wave & 1 of token tile wave >> 1; lane holds columns 4 lg + r of token li of the tile
+    {
+      const int t = sd + li;
+      f32x4 acc = tile_mma(ST + (sc + li) * CLD + 4 * lg, Q + t * CLD + 4 * lg) * EL[t];
+      for (int s = 0; s <= wave >> 1; ++s) {
+        f32x4 part = f32x4{0.f, 0.f, 0.f, 0.f};
+        mma4(part, f4(U + (sc + li) * CLD + s * 16 + 4 * lg), f4(M + t * CLD + s * 16 + 4 * lg));
+        acc += part;
+      }
+      if (t < m) {
+        float* const o = p.out + ((t0 + base + t) * p.heads + h) * (int64_t)p.dv + c0 + sc + 4 * lg;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!DELTA) acc[r] = fmaf(skip, U[(sc + 4 * lg + r) * CLD + t], acc[r]);
+        if (p.dv % 4 == 0 && c0 + sc + 4 * lg + 4 <= p.dv) {
+          *reinterpret_cast<f32x4*>(o) = acc;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (c0 + sc + 4 * lg + r < p.dv) o[r] = acc[r];
+        }
+      }
+    }
+    // state, in double like the weights: the sum over 64 tokens rounds once
+    f64x4 p64 = f64x4{0., 0., 0., 0.}, q64 = p64;
+    const float* const kt = KT + (sd + 4 * (li & 3) + (li >> 2)) * CLD + 4 * lg;
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) {
+      const f32x4 k0 = f4(kt + s * 16), k1 = f4(kt + s * 16 + 16);
+      const f32x4 u0 = f4(U + (sc + li) * CLD + s * 16 + 4 * lg), u1 = f4(U + (sc + li) * CLD + s * 16 + 16 + 4 * lg);
+      const f32x4 w0 = f4(WS + s * 16 + 4 * lg), w1 = f4(WS + s * 16 + 16 + 4 * lg);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        p64 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k0[j], (double)u0[j] * (double)w0[j], p64, 0, 0, 0);
+        q64 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k1[j], (double)u1[j] * (double)w1[j], q64, 0, 0, 0);
+      }
+    }
+    f32x4 S = f4(ST + (sc + li) * CLD + sd + 4 * lg);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = (float)((double)S[r] * (double)el_end + (p64[r] + q64[r]));
+    __syncthreads();                     // every wave has read the old state
+    *reinterpret_cast<f32x4*>(ST + (sc + li) * CLD + sd + 4 * lg) = S;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
+    if (i < p.dk && c0 + c < p.dv) sp[(int64_t)i * p.dv + c0 + c] = ST[c * CLD + i];
+  }
+}
+
+// Which launches take the chunks: one decay per head and token, at most 64 key channels (what the LDS tiles hold), and a step
+// whose sequences have segments, that is several tokens (a decode step is one token per sequence: the plain kernel's trip
+// through the matrix is all there is to it).
+inline bool chunks_serve(int dk, const int32_t* seg_len, const float* out, int dv) {
+  return dk <= CK && seg_len != nullptr && (dv % 4 != 0 || aligned16(out));
+}
+
+template <typename QT, typename VT, bool DELTA>
+int launch_chunks(const ChunkArgs& p, int64_t batch, hipStream_t st) {
+  constexpr size_t bytes = sizeof(float) * (4 * CK * CLD + 2 * RC_COLS * CLD + 5 * CK + (DELTA ? CK * CLD + 4 * 16 * 20 : 0));
+  auto kern = chunk_recurrence_kernel<QT, VT, DELTA>;
+  (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(p.dv, RC_COLS), (unsigned)p.heads, (unsigned)batch), dim3(CK_THREADS), bytes, st, p);
+  return MI355_OK;
+}
+
 template <typename QT, typename VT>
 int launch_recurrence(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
                       const void* gate_bias, const float* head_decay, const int32_t* req_to_state, const int64_t* req_pool_indices,
                       const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions, int64_t batch, int heads, int dk,
                       int dv, int64_t qs, int64_t ks, int64_t vs, int64_t gs, float q_scale, float tau, int qk_heads, const float* dt_logits,
                       int64_t dts, const float* dt_bias, const float* rate_log, const float* skip, hipStream_t stream) {
+  if (dt_logits != nullptr && chunks_serve(dk, seg_len, out, dv)) {
+    const ChunkArgs p{out, state, q, k, v, dt_logits, dt_bias, rate_log, skip, nullptr, req_to_state, req_pool_indices, seg_start, seg_len,
+                      positions, qs, ks, vs, dts, 0, heads, qk_heads, dk, dv, 0, q_scale};
+    return launch_chunks<QT, VT, false>(p, batch, stream);
+  }
   const dim3 grid((unsigned)cdiv(dv, RC_COLS), (unsigned)heads, (unsigned)batch);
 #define MI355_RC_LAUNCH(R)                                                                                                     \
   hipLaunchKernelGGL((linear_recurrence_kernel<QT, VT, R>), grid, dim3(256), 0, stream, out, state, (const QT*)q, (const QT*)k, \
@@ -271,6 +599,11 @@ int launch_delta(float* out, float* state, const void* q, const void* k, const v
                  const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions,
                  int64_t batch, int heads, int qk_heads, int dk, int dv, int64_t qs, int64_t ks, int64_t vs, int64_t bs, int64_t gs,
                  float q_scale, int gate_per_head, int beta_f32, hipStream_t stream) {
+  if (gate_per_head && chunks_serve(dk, seg_len, out, dv)) {
+    const ChunkArgs p{out, state, q, k, v, gate_logits, rate_bias, rate_log, nullptr, beta_logits, req_to_state, req_pool_indices, seg_start,
+                      seg_len, positions, qs, ks, vs, gs, bs, heads, qk_heads, dk, dv, beta_f32, q_scale};
+    return launch_chunks<QT, VT, true>(p, batch, stream);
+  }
   const dim3 grid((unsigned)cdiv(dv, RC_COLS), (unsigned)heads, (unsigned)batch);
 #define MI355_GD_LAUNCH(R)                                                                                                     \
   hipLaunchKernelGGL((gated_delta_rule_kernel<QT, VT, R>), grid, dim3(256), 0, stream, out, state, (const QT*)q, (const QT*)k,  \

@@ -233,6 +233,8 @@ int mi355_decode_attention(const void* q, const void* k_buffer, const void* v_bu
  * planner; never exceeds max_splits).
  * replaces: get_num_kv_splits_triton (layers/attention/triton_backend.py:875-924). */
 int mi355_decode_num_splits(int64_t bs, int hkv, int64_t max_seq_len, int max_splits);
+/* The same for a cache of e4m3fn rows, which fills the chip only at twice as many workgroups. */
+int mi355_decode_num_splits_fp8(int64_t bs, int hkv, int64_t max_seq_len, int max_splits);
 
 /* ---- K4 extend / prefill attention -----------------------------------------------------------
  * q_extend [T, Hq, D], k_extend/v_extend [T, Hkv, D|Dv] (row strides given), o_extend [T,Hq,Dv]

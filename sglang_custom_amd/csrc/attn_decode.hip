@@ -2703,6 +2703,11 @@ int mi355_decode_num_splits(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
   const int64_t wgs = bs * hkv;
   int64_t want = wgs >= 112 ? 1 : (160 + wgs - 1) / wgs;
   if (want > 1 && wgs * want < 192 && max_seq_len / ((256 + wgs - 1) / wgs) >= 1024) want = (256 + wgs - 1) / wgs;
+  // 112 to 128 workgroups draw the chip's rate only while every one of them runs: with 1 024 keys left per split half
+  // the CUs' worth more of them pays, and more again when the lengths differ and the longest row would run alone.
+  // 128 workgroups, head_dim 128, 1 -> 2 splits: 512 keys 11.1 -> 12.1 us, 1 024 17.7 -> 16.9, 2 048 28.3 -> 26.7,
+  // 4 096 57.4 -> 47.5, 1 638 to 4 096 52.8 -> 38.4; 144 workgroups (more than the CUs once doubled), 2 048: 29.2 -> 37.0.
+  if (wgs >= 112 && wgs <= 128 && max_seq_len >= 2048) want = 2;
   // A handful of workgroups (one sequence on a tensor-parallel rank): the launch is a latency chain, ~9.5 ns per key
   // of a split plus ~0.11 us per split merged, least at sqrt(keys / 12) splits.  One sequence x one kv head x 4104
   // keys: 22.3 / 17.6 / 16.2 / 16.2 / 16.6 / 17.5 / 21.7 us at 4 / 8 / 12 / 16 / 24 / 32 / 64 splits.
@@ -2713,6 +2718,28 @@ int mi355_decode_num_splits(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
   if (want > max_splits) want = max_splits;
   if (want < 1) want = 1;
   return (int)want;
+}
+
+int mi355_decode_num_splits_fp8(int64_t bs, int hkv, int64_t max_seq_len, int max_splits) {
+  const int64_t base = mi355_decode_num_splits(bs, hkv, max_seq_len, max_splits);
+  if (bs <= 0 || hkv <= 0 || max_splits <= 1) return (int)base;
+  // One-byte rows halve what a workgroup draws (~23 GB/s: its time per key is the chain of page read, row read and
+  // product, not the bytes), so the chip takes two workgroups per CU before it is full: 512 of them, at most 4 splits
+  // (a fifth is a second merge chain).  A split has to keep 512 keys, and 4 per workgroup of the unsplit launch, to pay
+  // for its partial: where the launch is already wide there is less left to fill.  head_dim 128, 8 kv heads, us at
+  // 1 / 2 / 3 / 4 splits (bracket: taken):
+  //   64 wgs, 4 096 keys  46.7 / 29.1 / 22.9 / [19.6];   128 wgs, 512 keys [10.3] / 10.2 / 12.9 / 11.7;
+  //  128 wgs, 1 024       16.2 / [13.3] / 15.6 / 14.0;   128 wgs, 2 048     26.5 / 18.9 / 21.8 / [19.0];
+  //  128 wgs, 4 096       47.8 / 30.5 / 32.8 / [28.7];   144 wgs, 1 024    [16.0] / 17.1 / 15.9 / 17.1;
+  //  160 wgs, 2 048       27.0 / 25.3 / [22.6] / 24.7;   160 wgs, 4 096     48.4 / 41.9 / [34.9] / 39.2;
+  //  224 wgs, 4 096       49.6 / [46.5] / 50.7 / 54.9;   256 wgs, 1 024    [16.8] / 18.6 / 21.4 / 25.9;
+  //  256 wgs, 4 096       51.0 / [49.2] / 51.8 / 59.7;   384 wgs, 4 096    [74.7] / 70.5 / 78.6 / 77.0.
+  const int64_t wgs = bs * hkv;
+  int64_t want = 512 / wgs < 4 ? 512 / wgs : 4;
+  const int64_t keep = 4 * wgs > 512 ? 4 * wgs : 512;
+  if (want > max_seq_len / keep) want = max_seq_len / keep;
+  if (want > max_splits) want = max_splits;
+  return (int)(want > base ? want : base);
 }
 
 int mi355_decode_attention(const void* q, const void* k_buffer, const void* v_buffer, void* o,

@@ -133,7 +133,8 @@ class Mi355AttnBackend(AttentionBackend):
             # 2 / 4 / 8 / 16 splits)
             wgs = max(1, bs * self.num_kv_head)
             return max(1, min(MAX_KV_SPLITS, (512 + wgs - 1) // wgs, max(1, max_seq_len // 256)))
-        return get_ops().decode_num_splits(bs, self.num_kv_head, max_seq_len, MAX_KV_SPLITS)
+        plan = get_ops().decode_num_splits_fp8 if self.kv_fp8 else get_ops().decode_num_splits
+        return plan(bs, self.num_kv_head, max_seq_len, MAX_KV_SPLITS)
 
     # ---- eager ----
     def init_forward_metadata(self, forward_batch):

@@ -360,6 +360,10 @@ def decode_num_splits(bs: int, hkv: int, max_seq_len: int, max_splits: int) -> i
     return _lib_().mi355_decode_num_splits(bs, hkv, max_seq_len, max_splits)
 
 
+def decode_num_splits_fp8(bs: int, hkv: int, max_seq_len: int, max_splits: int) -> int:
+    return _lib_().mi355_decode_num_splits_fp8(bs, hkv, max_seq_len, max_splits)
+
+
 def decode_attention_fwd(q, k_buffer, v_buffer, o, kv_indptr, kv_indices, attn_logits, attn_lse,
                          num_kv_splits: int, max_kv_splits: int, sm_scale: float,
                          logit_cap: float = 0.0, tickets=None, kv_chunk_keys=None) -> None:

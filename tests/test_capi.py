@@ -80,3 +80,14 @@ def test_planner_is_pure_host_logic(lib):
     assert lib.mi355_linear_workspace_bytes(64, 28672, 4096) == 0    # wide outputs are never split
     assert lib.mi355_linear_workspace_bytes(64, 128256, 4096) == 0
     assert lib.mi355_linear_workspace_bytes(65, 4096, 4096) == 0
+
+
+@pytest.mark.parametrize("bs,hkv,keys,most,bf16,fp8", [
+    (14, 8, 2047, 64, 1, 3), (14, 8, 2048, 64, 2, 4), (16, 8, 2048, 64, 2, 4), (17, 8, 4096, 64, 1, 3),   # edges of 112 and 128 workgroups
+    (16, 8, 1023, 64, 1, 1), (16, 8, 1024, 64, 1, 2), (16, 8, 2048, 2, 2, 2), (16, 8, 2048, 1, 1, 1),     # 512 keys a split, the caller's cap
+    (32, 8, 2047, 64, 1, 1), (32, 8, 2048, 64, 1, 2), (33, 8, 8192, 64, 1, 1),                            # 256 workgroups, one more
+    (1, 8, 1100, 64, 8, 8), (0, 8, 4096, 64, 1, 1),                                                       # never fewer than bf16 rows take
+])
+def test_split_plan_of_one_byte_rows(lib, bs, hkv, keys, most, bf16, fp8):
+    assert lib.mi355_decode_num_splits(bs, hkv, keys, most) == bf16
+    assert lib.mi355_decode_num_splits_fp8(bs, hkv, keys, most) == fp8

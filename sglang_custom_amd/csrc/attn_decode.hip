@@ -1458,7 +1458,8 @@ __global__ __launch_bounds__(256) void decode_attn_mla_mfma_kernel(const T* __re
 // A wave issues 5 loads per tile: rows 4 w .. 4 w + 3 (1 KiB each) and their rope parts (half a wave).
 // grid (ceil(hq / 16), num_splits, B), block 256.
 // ------------------------------------------------------------------------------------------
-// 0 = plan (two teams per workgroup when the grid allows), 1 = one team (ablation; development build, mi355_debug_set key 10)
+// 0 = plan (two teams per workgroup when the grid allows: two splits, or two head groups of one), 1 = one team, 2 = never two
+// head groups (ablation; development build, mi355_debug_set key 10)
 #ifdef MI355_DEV_BUILD
 int g_mla_teams = 0;
 #else
@@ -1471,6 +1472,12 @@ constexpr int MLR_TILE = MLR_TAIL + 16 * 128;        // 18944
 // NSB step buffers of two tiles each: 2 -> 75776 bytes (two workgroups per CU, one step in flight),
 // 4 -> 151552 bytes (one workgroup per CU, three steps = 111 KiB in flight)
 constexpr int mlr_lds_bytes(int nsb) { return 2 * nsb * MLR_TILE; }
+constexpr int MLR_XCH = 4 * 64 * 16;                 // a team's four partial score tiles
+constexpr int MLR_SLOTS = 32;                        // a wave's page-table entries of one step
+constexpr int mlr_lds_total(int rings, int nsb, int teams) {   // (teams that share a ring exchange two steps' scores)
+  return rings * mlr_lds_bytes(nsb) + teams * ((rings < teams ? 2 : 1) * MLR_XCH + 4 * MLR_SLOTS * nsb);
+}
+static_assert(mlr_lds_total(2, 2, 2) <= 160 * 1024 && 2 * mlr_lds_total(1, 2, 1) <= 160 * 1024 && mlr_lds_total(1, 3, 2) <= 160 * 1024, "");
 
 __device__ __forceinline__ unsigned lds_byte_address(const void* p) {
   return (unsigned)(uintptr_t)(const char __attribute__((address_space(3)))*)(p);
@@ -1514,6 +1521,23 @@ __device__ __forceinline__ void load_to_lds_16_s(uint64_t base, unsigned lane_of
         : "memory");
 }
 
+// max of a value over the lanes that differ in bit 16 or 32 of their number, in registers: swapping a register with its own
+// copy leaves one half's values in all lanes of the first result and the other half's in the second
+template <int X> __device__ __forceinline__ float max_xor(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+}
+
+// One 4-byte load per active lane to LDS at `lds_base` (wave-uniform) + 4 * lane.
+__device__ __forceinline__ void load_to_lds_4_v(const void* src, unsigned lds_base) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(src), "s"(lds_base)
+               : "memory");
+}
+
 // Inputs of the decode launch that also applies RoPE and writes the new token's latent row: q's rope part
 // and k_pe arrive UNROTATED, the new row [k_nope | rope(k_pe)] is not in the cache yet.
 struct MlaRope {
@@ -1531,6 +1555,29 @@ template <typename T> __device__ __forceinline__ float mla_cs_t(const MlaRope& r
                       : to_f32(static_cast<const T*>(rp.cos_sin)[pos * MLA_ROPE + idx]);
 }
 
+// Workgroup -> (head group, split, sequence) of the MLA ring kernels.  Consecutive workgroups are dealt to the eight XCDs
+// in turn, so the head groups of one key range, neighbours in the grid, would read the same rows into different L2s: the
+// launch then draws them from HBM once per head group.  Eight key ranges at a time, all first head groups go ahead of
+// all second ones, which puts the head groups of a range on the same XCD, eight workgroups apart.  (What is left when the
+// ranges are no multiple of eight follows the same pattern with fewer; it need not share an XCD.)
+struct MlaBlock { int group, split, seq; };
+__device__ __forceinline__ MlaBlock mla_block() {
+  const unsigned G = gridDim.x, S = gridDim.y;
+  const unsigned id = blockIdx.x + G * (blockIdx.y + S * blockIdx.z);
+  const unsigned units = S * gridDim.z, whole = units & ~7u;   // key ranges; those in full eights
+  unsigned group, unit;
+  if (id < whole * G) {
+    const unsigned eight = id / (8 * G), in = id - eight * 8 * G;
+    group = in >> 3;
+    unit = eight * 8 + (in & 7);
+  } else {
+    const unsigned in = id - whole * G, rest = units - whole;
+    group = in / rest;
+    unit = whole + in - group * rest;
+  }
+  return MlaBlock{(int)group, (int)(unit % S), (int)(unit / S)};
+}
+
 // ROPE: the launch rotates the query's rope part (in registers) and the new token's k_pe, writes the new
 // latent row to the cache (one workgroup per sequence) and -- in every workgroup whose key range ends at the
 // new token -- puts that row into the LDS tile over whatever the load unit fetched from the not yet written
@@ -1538,24 +1585,37 @@ template <typename T> __device__ __forceinline__ float mla_cs_t(const MlaRope& r
 // TEAMS = 2: two teams of four waves per workgroup, each with its own ring, on two consecutive KV splits of the
 // launch's plan; their results meet in LDS and ONE partial leaves the workgroup (see the fp8 ring kernel below:
 // what a launch pays for its splits is the merge of S partials of 16 heads x 512 features).  grid.y = num_splits / TEAMS.
-template <typename T, bool CAP, int NSB, bool ROPE = false, int TEAMS = 1>
+// PAIR: the two teams are two head groups over ONE ring, so the rows reach the CU once for 32 heads.  grid.x = pairs.
+// A team's waves share the scores: wave w multiplies tile w >> 1 over half w & 1 of the features, the partial tiles meet in
+// LDS.  What bounds it: the rows (64 x 4096 x 32 heads: 266 MB, 54 us at the card's copy rate, 66 taken); at few keys per
+// workgroup the chain of a step (reads, nine MFMAs, exchange, softmax, P.V: 1.3 us) and the merge.  Before -- all four waves
+// multiplied all scores, the head groups of a range ran on different XCDs and drew the rows from HBM each, the page-table
+// entries were waited for in every step -- 64 x 4096 keys took 117 us with 32 heads and 390 with 128.
+template <typename T, bool CAP, int NSB, bool ROPE = false, int TEAMS = 1, bool PAIR = false>
 __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
     const T* __restrict__ q, const T* __restrict__ kvbuf, T* __restrict__ o, DecodeParams p, MlaRope rp) {
-  constexpr int NS = MLA_D / 32;   // 18 score k-steps
+  constexpr int NH = MLA_D / 64;   // 9 of the 18 score k-steps per wave
   using frag = typename Mfma<T>::frag;
-  using frag4 = typename Mfma16<T>::frag;
+  constexpr int RINGS = PAIR ? 1 : TEAMS;
+  constexpr int XCH = PAIR ? 2 * MLR_XCH : MLR_XCH;
+  constexpr int LOADS = PAIR ? 6 : 11;   // a wave's requests per step: rows, rope parts and one of page-table entries
   constexpr int P = NSB - 1;   // steps requested ahead of the one being computed
-  static_assert(P >= 1 && P <= 3, "the wait below knows 0, 10 or 20 younger loads");
-  extern __shared__ __attribute__((aligned(16))) char sm_raw[];   // TEAMS * mlr_lds_bytes(NSB)
+  static_assert(P >= 1 && P <= 3, "the wait below knows 0, 1 or 2 younger steps");
+  extern __shared__ __attribute__((aligned(16))) char sm_raw[];   // mlr_lds_total(RINGS, NSB, TEAMS)
 
-  const int head0 = blockIdx.x * 16, b = blockIdx.z;
+  const MlaBlock blk = mla_block();
+  const int b = blk.seq;
   const int lane = threadIdx.x & 63;
   const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
   const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);   // within the team
   const int tid = threadIdx.x & 255;                                         // within the team
-  const int split = blockIdx.y * TEAMS + team;
-  char* sm_team = sm_raw + team * mlr_lds_bytes(NSB);
+  const int head0 = PAIR ? (blk.group * TEAMS + team) * 16 : blk.group * 16;
+  const int split = PAIR ? blk.split : blk.split * TEAMS + team;
+  char* sm_team = sm_raw + (PAIR ? 0 : team) * mlr_lds_bytes(NSB);
+  f32x4* xw = reinterpret_cast<f32x4*>(sm_raw + RINGS * mlr_lds_bytes(NSB) + team * XCH);
+  char* sm_slots = sm_raw + RINGS * mlr_lds_bytes(NSB) + TEAMS * XCH + (team * 4 + wave) * MLR_SLOTS * NSB;   // this wave's own
   const int r16 = lane & 15, c4 = lane >> 4;
+  const int tile_w = wave >> 1, half = wave & 1;   // this wave's part of the scores
 
   int64_t page_off, len;
   seq_range(p, b, page_off, len);
@@ -1569,7 +1629,7 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
   bool new_team[TEAMS];
 #pragma unroll
   for (int tt = 0; tt < TEAMS; ++tt) {
-    const int64_t a0 = (int64_t)(blockIdx.y * TEAMS + tt) * chunk;
+    const int64_t a0 = PAIR ? k0 : (int64_t)(blk.split * TEAMS + tt) * chunk;
     const int64_t a1 = a0 + chunk < len ? a0 + chunk : len;
     n_team[tt] = a1 > a0 ? (int)((a1 - a0 + 31) / 32) : 0;
     new_team[tt] = ROPE && a1 == len && len > a0;
@@ -1607,7 +1667,7 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
           }
         }
       }
-      if (blockIdx.x == 0) {   // one workgroup per sequence writes the row to the cache
+      if (blk.group == 0 && (!PAIR || team == 0)) {   // one workgroup per sequence writes the row to the cache
         T* dst = const_cast<T*>(kvbuf) + rp.out_loc[b] * p.k_slot_stride;
         if (tid < 64) stvec<T, 8>(dst + 8 * tid, new_a);
         else if (tid < 72 && !rp.is_neox) stvec<T, 8>(dst + MLA_RANK + 8 * (tid - 64), new_a);
@@ -1619,16 +1679,31 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
     }
   }
 
-  // page-table reads through the scalar unit (wave-uniform index, read-only data)
+  // the first steps' page-table reads go through the scalar unit (wave-uniform index, read-only data)
   const int32_t __attribute__((address_space(4)))* pt =
       (const int32_t __attribute__((address_space(4)))*)(p.page_table + page_off);
   const int64_t last_key = len - 1;
-  struct Slots { int32_t a0, a1, a2, a3, b0, b1, b2, b3; };   // rows 4 wave .. + 3 of a step's two tiles
+  struct Slots { int32_t a0, a1, a2, a3, b0, b1, b2, b3; };   // rows 4 wave .. + 3 of a step's two tiles (PAIR: of tile `team`)
   auto slot_of = [&](int64_t key) -> int32_t { return pt[key < last_key ? key : last_key]; };
   auto slots_of = [&](int step) -> Slots {
-    const int64_t key = k0 + (int64_t)step * 32 + 4 * wave;
+    const int64_t key = k0 + (int64_t)step * 32 + 4 * wave + (PAIR ? 16 * team : 0);
+    if constexpr (PAIR) return Slots{slot_of(key), slot_of(key + 1), slot_of(key + 2), slot_of(key + 3), 0, 0, 0, 0};
     return Slots{slot_of(key), slot_of(key + 1), slot_of(key + 2), slot_of(key + 3),
                  slot_of(key + 16), slot_of(key + 17), slot_of(key + 18), slot_of(key + 19)};
+  };
+  // The entries of later steps come the way of the rows, with the same counted wait: step j's requests include the slots
+  // of step j + P.  Scalar reads inside the loop would be waited for at its barriers (they share the LDS counter), a
+  // round trip to memory in every step: 128 steps of one workgroup took 190 us so, most of it that wait.
+  const unsigned slot_ring = lds_byte_address(sm_slots);
+  auto issue_slots = [&](int step, int buf) {
+    const int64_t key = k0 + (int64_t)step * 32 + 4 * wave + (lane & 3) + (PAIR ? 16 * team : 16 * (lane >> 2));
+    if (lane < (PAIR ? 4 : 8)) load_to_lds_4_v(p.page_table + page_off + (key < last_key ? key : last_key), slot_ring + (unsigned)(buf * MLR_SLOTS));
+  };
+  auto landed_slots = [&](int buf) -> Slots {
+    const int4* q4 = reinterpret_cast<const int4*>(sm_slots + buf * MLR_SLOTS);
+    const int4 a = q4[0], c = PAIR ? int4{0, 0, 0, 0} : q4[1];
+    auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    return Slots{uni(a.x), uni(a.y), uni(a.z), uni(a.w), uni(c.x), uni(c.y), uni(c.z), uni(c.w)};
   };
   const unsigned ring = lds_byte_address(sm_team);
   const uint64_t kv_base = (uint64_t)(uintptr_t)kvbuf;
@@ -1637,22 +1712,29 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
   const int trow = lane >> 3, tch = lane & 7;   // rope part: lane (row 4 wave + trow (lanes 0..31), chunk tch)
   const unsigned tsw = MLA_RANK * sizeof(T) + 16 * (tch ^ (((4 * wave + trow) >> 1) & 7));   // byte offset of the chunk this lane fetches
   const int tm0 = -(int)(trow == 0), tm1 = -(int)(trow == 1), tm2 = -(int)(trow == 2), tm3 = -(int)(trow == 3);
-  auto issue_tile = [&](int buf, int32_t s0, int32_t s1, int32_t s2, int32_t s3) {
+  auto issue_tile = [&](auto nt, int buf, int32_t s0, int32_t s1, int32_t s2, int32_t s3) {
+    constexpr bool NT = decltype(nt)::value;
     const unsigned base = ring + (unsigned)buf * MLR_TILE + (unsigned)(4 * wave) * MLR_ROWB;
-    load_to_lds_16_s<true>(kv_base + (uint64_t)(uint32_t)s0 * row_bytes, lane16, base);
-    load_to_lds_16_s<true>(kv_base + (uint64_t)(uint32_t)s1 * row_bytes, lane16, base + MLR_ROWB);
-    load_to_lds_16_s<true>(kv_base + (uint64_t)(uint32_t)s2 * row_bytes, lane16, base + 2 * MLR_ROWB);
-    load_to_lds_16_s<true>(kv_base + (uint64_t)(uint32_t)s3 * row_bytes, lane16, base + 3 * MLR_ROWB);
+    load_to_lds_16_s<NT>(kv_base + (uint64_t)(uint32_t)s0 * row_bytes, lane16, base);
+    load_to_lds_16_s<NT>(kv_base + (uint64_t)(uint32_t)s1 * row_bytes, lane16, base + MLR_ROWB);
+    load_to_lds_16_s<NT>(kv_base + (uint64_t)(uint32_t)s2 * row_bytes, lane16, base + 2 * MLR_ROWB);
+    load_to_lds_16_s<NT>(kv_base + (uint64_t)(uint32_t)s3 * row_bytes, lane16, base + 3 * MLR_ROWB);
     // row trow's slot by masks (a chain of selects would be turned into an indexed array in scratch memory)
     const uint32_t ts = (uint32_t)((s0 & tm0) | (s1 & tm1) | (s2 & tm2) | (s3 & tm3));
     if (lane < 32)
-      load_to_lds_16_v<true>(reinterpret_cast<const char*>(kvbuf) + (uint64_t)ts * row_bytes + tsw,
+      load_to_lds_16_v<NT>(reinterpret_cast<const char*>(kvbuf) + (uint64_t)ts * row_bytes + tsw,
                        ring + (unsigned)buf * MLR_TILE + MLR_TAIL + (unsigned)(4 * wave) * 128);
   };
   auto issue_step = [&](int step, const Slots& sl) {
     const int buf = 2 * (step % NSB);
-    issue_tile(buf, sl.a0, sl.a1, sl.a2, sl.a3);
-    issue_tile(buf + 1, sl.b0, sl.b1, sl.b2, sl.b3);
+    issue_slots(step + P, step % NSB);
+    if (gridDim.x == 1) {   // rows that no other head group reads
+      issue_tile(std::true_type{}, buf + (PAIR ? team : 0), sl.a0, sl.a1, sl.a2, sl.a3);
+      if constexpr (!PAIR) issue_tile(std::true_type{}, buf + 1, sl.b0, sl.b1, sl.b2, sl.b3);
+    } else {
+      issue_tile(std::false_type{}, buf + (PAIR ? team : 0), sl.a0, sl.a1, sl.a2, sl.a3);
+      if constexpr (!PAIR) issue_tile(std::false_type{}, buf + 1, sl.b0, sl.b1, sl.b2, sl.b3);
+    }
   };
 
   float m = -INFINITY, l = 0.f;
@@ -1661,33 +1743,34 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
   for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // read addresses inside a tile (bytes)
-  const int k_rd = MLR_ROWB * r16 + 16 * c4;                                          // + 64 s
-  const int kt_rd0 = MLR_TAIL + 128 * r16 + 16 * (c4 ^ ((r16 >> 1) & 7));             // rope k-step 16
-  const int kt_rd1 = MLR_TAIL + 128 * r16 + 16 * ((4 + c4) ^ ((r16 >> 1) & 7));       // rope k-step 17
+  const int k_rd = MLR_TILE * tile_w + MLR_ROWB * r16 + 16 * c4 + 64 * NH * half;      // + 64 s', the wave's steps 0 .. 6
+  const int kt_rd0 = half ? MLR_TILE * tile_w + MLR_TAIL + 128 * r16 + 16 * (c4 ^ ((r16 >> 1) & 7))         // step 7: rope k-step 16
+                          : k_rd + 64 * (NH - 2);
+  const int kt_rd1 = half ? MLR_TILE * tile_w + MLR_TAIL + 128 * r16 + 16 * ((4 + c4) ^ ((r16 >> 1) & 7))   // step 8: rope k-step 17
+                          : k_rd + 64 * (NH - 1);
   const int v_rd = MLR_ROWB * (4 * c4 + (r16 >> 2)) + 8 * (r16 & 3) + 256 * wave;    // + 32 dt
 
-  Slots s_nxt{};
   if (n_steps > 0) {   // (an empty sequence has no page-table entry to read)
+    Slots first[P];
 #pragma unroll
-    for (int i = 0; i < P; ++i) {
-      s_nxt = slots_of(i);   // clamped to the last key when past the end
-      if (i < n_steps) issue_step(i, s_nxt);
-    }
-    s_nxt = slots_of(P);
+    for (int i = 0; i < P; ++i) first[i] = slots_of(i);   // clamped to the last key when past the end
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+      if (i < n_steps) issue_step(i, first[i]);
   }
 
-  // B operand of the scores: this lane's head (r16), features 32 s + 8 c4 .. + 7.  Fetched AFTER the first
+  // B operand of this wave's score steps: this lane's head (r16), features 32 (9 half + s') + 8 c4 .. + 7.  Fetched AFTER the first
   // tiles were requested, and waited for here, before the loop: the compiler does not count the
   // loads-to-LDS, and a wait for these fragments placed inside the loop would drain the ring every step.
-  frag qf[NS];
+  frag qf[NH];
   {
     const int hq_c = head0 + r16 < p.hq ? head0 + r16 : p.hq - 1;   // rows of heads past hq are computed and dropped
-    const T* qp = q + (int64_t)b * p.q_stride + (int64_t)hq_c * MLA_D + 8 * c4;
+    const T* qp = q + (int64_t)b * p.q_stride + (int64_t)hq_c * MLA_D + 32 * NH * half + 8 * c4;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const frag*>(qp + 32 * s);
-    if constexpr (ROPE) {
-      // rope part = k-steps 16 and 17: the lane holds features 8 c4 .. + 7 and 32 + 8 c4 .. + 7 of its head
-      Vec<T, 8> a = __builtin_bit_cast(Vec<T, 8>, qf[16]), b2 = __builtin_bit_cast(Vec<T, 8>, qf[17]);
+    for (int s = 0; s < NH; ++s) qf[s] = *reinterpret_cast<const frag*>(qp + 32 * s);
+    if (ROPE && half == 1) {
+      // rope part = k-steps 16 and 17 = this wave's last two: the lane holds features 8 c4 .. + 7 and 32 + 8 c4 .. + 7 of its head
+      Vec<T, 8> a = __builtin_bit_cast(Vec<T, 8>, qf[NH - 2]), b2 = __builtin_bit_cast(Vec<T, 8>, qf[NH - 1]);
       if (!rp.is_neox) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1705,51 +1788,57 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
                        mla_cs_t<T>(rp, rope_pos, MLA_ROPE / 2 + i), a.v[j], b2.v[j]);
         }
       }
-      qf[16] = __builtin_bit_cast(frag, a);
-      qf[17] = __builtin_bit_cast(frag, b2);
+      qf[NH - 2] = __builtin_bit_cast(frag, a);
+      qf[NH - 1] = __builtin_bit_cast(frag, b2);
     }
 #pragma unroll
-    for (int s = 0; s < NS; ++s) asm volatile("" ::"v"(qf[s]));
+    for (int s = 0; s < NH; ++s) asm volatile("" ::"v"(qf[s]));
   }
 
-  // one step (32 keys = two tiles at `tile`): scores, online softmax, this wave's quarter of P.V
-  auto step_compute = [&](int t, const char* tile) {
-    f32x4 sa = f32x4{0.f, 0.f, 0.f, 0.f}, sb = f32x4{0.f, 0.f, 0.f, 0.f};
-    // key fragments are read MLR_AHEAD k-steps before the MFMAs that use them (a ring of registers; the
-    // fences keep the order): left alone the compiler puts each read next to its MFMA, and the score
-    // phase then runs at one LDS round trip per k-step instead of at the matrix rate
-    constexpr int MLR_AHEAD = 4;
-    auto k_off = [&](int s) { return s < 16 ? k_rd + 64 * s : (s == 16 ? kt_rd0 : kt_rd1); };
-    frag ka[MLR_AHEAD], kb[MLR_AHEAD];
+  // one step (32 keys = two tiles at `tile`).  First this wave's part of the scores -- 16 keys of tile `tile_w` x 16
+  // heads over its half of the feature steps -- put into the exchange; the value fragments of its quarter of P.V, which
+  // need no scores, are on their way meanwhile.
+  typename TrRead<T>::v4 va[8], vb[8];
+  frag kf[NH];
+  auto read_keys = [&](const char* tile) {
 #pragma unroll
-    for (int s = 0; s < MLR_AHEAD; ++s) {
-      ka[s] = *reinterpret_cast<const frag*>(tile + k_off(s));
-      kb[s] = *reinterpret_cast<const frag*>(tile + MLR_TILE + k_off(s));
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    for (int s = 0; s < NH; ++s)
+      kf[s] = *reinterpret_cast<const frag*>(tile + (s < NH - 2 ? k_rd + 64 * s : (s == NH - 2 ? kt_rd0 : kt_rd1)));
+  };
+  auto read_values = [&](const char* tile) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      sa = Mfma<T>::run(ka[s % MLR_AHEAD], qf[s], sa);
-      sb = Mfma<T>::run(kb[s % MLR_AHEAD], qf[s], sb);
-      __builtin_amdgcn_sched_barrier(0);
-      if (s + MLR_AHEAD < NS) {
-        ka[s % MLR_AHEAD] = *reinterpret_cast<const frag*>(tile + k_off(s + MLR_AHEAD));
-        kb[s % MLR_AHEAD] = *reinterpret_cast<const frag*>(tile + MLR_TILE + k_off(s + MLR_AHEAD));
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    for (int i = 0; i < 8; ++i) {
+      va[i] = TrRead<T>::run(reinterpret_cast<const T*>(tile + v_rd + 32 * i));
+      vb[i] = TrRead<T>::run(reinterpret_cast<const T*>(tile + MLR_TILE + v_rd + 32 * i));
     }
-
-    const int64_t kb0 = k0 + (int64_t)t * 32 + 4 * c4;
+  };
+  auto step_scores = [&](f32x4* to) {
+    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NH; s += 2) {
+      s0 = Mfma<T>::run(kf[s], qf[s], s0);
+      if (s + 1 < NH) s1 = Mfma<T>::run(kf[s + 1], qf[s + 1], s1);
+    }
+    to[wave * 64 + lane] = s0 + s1;
+  };
+  // then, with all four partial tiles in LDS: every wave adds the halves in the same order (the same softmax statistics in
+  // all of them), online softmax, this wave's quarter of P.V
+  struct Scores { f32x4 a, b; };
+  auto read_scores = [&](const f32x4* from) { return Scores{from[lane] + from[64 + lane], from[128 + lane] + from[192 + lane]}; };
+  const int n_keys = (int)(k1 - k0);   // (of this split; nothing is computed when it is not positive)
+  auto step_compute = [&](int t, const Scores& sc) {
+    const f32x4 sa = sc.a, sb = sc.b;
+    const int kb0 = 32 * t + 4 * c4;
     float x[8], mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       float v = (r < 4 ? sa[r & 3] : sb[r & 3]) * qmul;
       if (CAP) v = p.logit_cap * tanhf(v / p.logit_cap) * kLog2e;
-      x[r] = kb0 + (r & 3) + 16 * (r >> 2) < k1 ? v : -INFINITY;
+      x[r] = kb0 + (r & 3) + 16 * (r >> 2) < n_keys ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor<16>(mx);   // (over registers: a shuffle would queue behind the fragment reads in flight)
+    mx = max_xor<32>(mx);
     // lazy rescale, as in the register kernel: the reference point moves only when a step's maximum exceeds it by 2^8
     const bool need = mx > m + 8.f;
     if (__builtin_amdgcn_ballot_w64(need) != 0) {
@@ -1762,82 +1851,99 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
     }
     const float ms = safe_m(m);
     float psum = 0.f;
-    T pa4[4], pb4[4];
+    Vec<T, 8> p8;   // key slots 8 c4 + j of the P.V step: keys 4 c4 + j of the first tile (j < 4), 4 c4 + j - 4 of the second
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float pa = exp2f(x[r] - ms), pb = exp2f(x[4 + r] - ms);
-      psum += pa + pb;
-      pa4[r] = from_f32<T>(pa);
-      pb4[r] = from_f32<T>(pb);
+    for (int r = 0; r < 8; ++r) {
+      const float pe = exp2f(x[r] - ms);
+      psum += pe;
+      p8.v[r] = from_f32<T>(pe);
     }
     l += psum;
-    const frag4 pa = __builtin_bit_cast(frag4, pa4), pb = __builtin_bit_cast(frag4, pb4);
-    // transposed value reads in two batches of eight ahead of their MFMAs (see the score phase above)
+    const frag pf = __builtin_bit_cast(frag, p8);
+    struct Two { typename TrRead<T>::v4 a, b; };
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      typename TrRead<T>::v4 va[4], vb[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        va[i] = TrRead<T>::run(reinterpret_cast<const T*>(tile + v_rd + 32 * (4 * h + i)));
-        vb[i] = TrRead<T>::run(reinterpret_cast<const T*>(tile + MLR_TILE + v_rd + 32 * (4 * h + i)));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        acc[4 * h + i] = Mfma16<T>::run(__builtin_bit_cast(frag4, va[i]), pa, acc[4 * h + i]);
-        acc[4 * h + i] = Mfma16<T>::run(__builtin_bit_cast(frag4, vb[i]), pb, acc[4 * h + i]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int i = 0; i < 8; ++i) acc[i] = Mfma<T>::run(__builtin_bit_cast(frag, Two{va[i], vb[i]}), pf, acc[i]);
   };
 
-  {
+  // ROPE: when step t's tiles hold some team's new token, its row is put over what was fetched
+  auto patch_new_row = [&](int t) {
+    bool patch_any = false;   // (workgroup-uniform)
+#pragma unroll
+    for (int tt = 0; tt < TEAMS; ++tt) patch_any |= new_team[tt] && t == n_team[tt] - 1;
+    if (!patch_any) return;
+    if (has_new && t == n_steps - 1 && (!PAIR || team == 0)) {
+      // the new token is the last key of the last step: its row goes into the tile over what was fetched
+      // from the slot (every wave's loads of this step have landed: the barrier above)
+      const int kl = (int)(len - 1 - k0) - 32 * t;           // 0 .. 31 inside the step
+      char* row_tile = sm_team + (2 * (t % NSB) + (kl >> 4)) * MLR_TILE;
+      const int r = kl & 15;
+      if (tid < 64) {
+        *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_ROWB * r + 16 * tid) = new_a;
+      } else if (tid < 72 && !rp.is_neox) {
+        *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_TAIL + 128 * r + 16 * ((tid - 64) ^ ((r >> 1) & 7))) = new_a;
+      } else if (tid < 68) {
+        *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_TAIL + 128 * r + 16 * ((tid - 64) ^ ((r >> 1) & 7))) = new_a;
+        *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_TAIL + 128 * r + 16 * ((tid - 60) ^ ((r >> 1) & 7))) = new_b;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  };
+  // Step t's requests of this wave have landed and so has, past the barrier, the whole step; the requests of step t + P go out
+  // into the tiles that the barrier frees.
+  auto open_step = [&](int t) {
+    Slots s_nxt{};
+    if (t < n_steps) {
+      // landed: at most the loads (LOADS per step) of the younger steps are out
+      const int younger = min(P - 1, n_steps - 1 - t);
+      if (P >= 3 && younger >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+      else if (P >= 2 && younger >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (t + P < n_steps) s_nxt = landed_slots(t % NSB);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of step t - 1 have returned
+    __builtin_amdgcn_s_barrier();
+    if (t + P < n_steps) issue_step(t + P, s_nxt);
+    if constexpr (ROPE) patch_new_row(t);
+  };
+
+  if constexpr (PAIR) {
+    // one barrier a step: iteration t multiplies step t's scores and finishes step t - 1, whose partial scores the barrier
+    // has made visible, so that the reads and MFMAs of the one run beside the softmax of the other
+    for (int t = 0; t <= n_steps; ++t) {
+      open_step(t);
+      const char* tile = sm_team + 2 * (t % NSB) * MLR_TILE;
+      Scores sc{};
+      if (t > 0) sc = read_scores(xw + (~t & 1) * 256);
+      if (t < n_steps) read_keys(tile);
+      __builtin_amdgcn_sched_barrier(0);
+      if (t > 0) step_compute(t - 1, sc);
+      if (t < n_steps) {
+        __builtin_amdgcn_sched_barrier(0);
+        read_values(tile);
+        step_scores(xw + (t & 1) * 256);
+      }
+    }
+  } else {
     for (int t = 0; t < n_all; ++t) {
       const bool live = t < n_steps;   // (team-uniform; a team that has run out of steps keeps the barriers company)
+      open_step(t);
       if (live) {
-        // this wave's part of step t has landed when at most the loads (10 per step) of the younger steps are out
-        const int younger = min(P - 1, n_steps - 1 - t);
-        if (P >= 3 && younger >= 2) asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
-        else if (P >= 2 && younger == 1) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const char* tile = sm_team + 2 * (t % NSB) * MLR_TILE;
+        read_keys(tile);
+        read_values(tile);
+        __builtin_amdgcn_sched_barrier(0);   // (left alone the compiler puts each read next to its MFMA: one LDS round trip per k-step)
+        step_scores(xw);
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // and its reads of step t - 1 have returned
-      __builtin_amdgcn_s_barrier();                         // every wave's part of step t is in LDS; step t - 1's tiles are free
-      if (live) {
-        if (t + P < n_steps) issue_step(t + P, s_nxt);
-        s_nxt = slots_of(t + P + 1);
-      }
-      if constexpr (ROPE) {
-        bool patch_any = false;   // some team patches the new row into its tile in this iteration (workgroup-uniform)
-#pragma unroll
-        for (int tt = 0; tt < TEAMS; ++tt) patch_any |= new_team[tt] && t == n_team[tt] - 1;
-        if (patch_any) {
-          if (has_new && t == n_steps - 1) {
-            // the new token is the last key of the last step: its row goes into the tile over what was fetched
-            // from the slot (every wave's loads of this step have landed: the barrier above)
-            const int kl = (int)(len - 1 - k0) - 32 * t;           // 0 .. 31 inside the step
-            char* row_tile = sm_team + (2 * (t % NSB) + (kl >> 4)) * MLR_TILE;
-            const int r = kl & 15;
-            if (tid < 64) {
-              *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_ROWB * r + 16 * tid) = new_a;
-            } else if (tid < 72 && !rp.is_neox) {
-              *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_TAIL + 128 * r + 16 * ((tid - 64) ^ ((r >> 1) & 7))) = new_a;
-            } else if (tid < 68) {
-              *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_TAIL + 128 * r + 16 * ((tid - 64) ^ ((r >> 1) & 7))) = new_a;
-              *reinterpret_cast<Vec<T, 8>*>(row_tile + MLR_TAIL + 128 * r + 16 * ((tid - 60) ^ ((r >> 1) & 7))) = new_b;
-            }
-          }
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-          __builtin_amdgcn_s_barrier();
-        }
-      }
-      if (live) step_compute(t, sm_team + 2 * (t % NSB) * MLR_TILE);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();   // the four partial score tiles are in LDS (they are read before the next step's first barrier)
+      if (live) step_compute(t, read_scores(xw));
     }
   }
 
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  if constexpr (TEAMS > 1) {
+  if constexpr (TEAMS > 1 && !PAIR) {
     // the teams' (reference point, sum, 512-feature accumulators) meet in LDS; team 0 carries the result out
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();   // every team is done with its rings
@@ -1865,8 +1971,8 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
       }
     }
   }
-  const int s_out = p.num_splits / TEAMS;   // partials that leave the launch per (sequence, head)
-  if (team == 0 && head0 + r16 < p.hq) {
+  const int s_out = PAIR ? p.num_splits : p.num_splits / TEAMS;   // partials that leave the launch per (sequence, head)
+  if ((PAIR || team == 0) && head0 + r16 < p.hq) {
     const int head = head0 + r16;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     // lane (head r16, c4) holds features 128 wave + 16 dt + 4 c4 .. + 3
@@ -1883,7 +1989,7 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
       // write-through, so that the workgroup that merges the splits (below) sees them without a fence
       // (the resources start at the workgroup's first head: wave-uniform; the lane adds its head and features)
       const int64_t ph0 = ((int64_t)b * p.hq + head0) * s_out;
-      const int cell = r16 * s_out + (int)blockIdx.y;
+      const int cell = r16 * s_out + blk.split;
       const auto rs = wt_rsrc(p.part_o + ph0 * MLA_RANK, 16 * s_out * MLA_RANK * 4);
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt)
@@ -1895,10 +2001,11 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
     }
   }
   if (s_out > 1 && p.tickets) {
-    const int nheads = p.hq - head0 < 16 ? p.hq - head0 : 16;
+    const int first = PAIR ? blk.group * TEAMS * 16 : head0, most = PAIR ? TEAMS * 16 : 16;   // the workgroup's heads
+    const int nheads = p.hq - first < most ? p.hq - first : most;
     DecodeParams po = p;
     po.num_splits = s_out;
-    merge_splits_if_last<T, 4>(po, o, b, head0, nheads, MLA_RANK, b * (int)gridDim.x + (int)blockIdx.x, reinterpret_cast<float*>(sm_raw));
+    merge_splits_if_last<T, 4>(po, o, b, first, nheads, MLA_RANK, b * (int)gridDim.x + blk.group, reinterpret_cast<float*>(sm_raw));
   }
 }
 
@@ -3072,9 +3179,17 @@ static int decode_attention_mla_impl(const MlaRope* rope, const void* q, const v
       constexpr int NSB_ = 2;
       const bool deep = g_decode_variant == 5;
       // two KV splits per workgroup (two teams of four waves) when the halved grid still gives every CU a workgroup
-      const bool two = !deep && num_splits % 2 == 0 && (int64_t)grid.x * grid.y * grid.z >= 512 && g_mla_teams != 1;
+      // Two head groups per workgroup over one copy of the rows: where at least half the CUs get such a workgroup, in one
+      // round if an odd last group leaves a team idle, and at most four partials meet in the merge (32 heads of them are
+      // merged by one workgroup).  bf16, 32 / 128 heads, apart -> paired: 64 x 4096 keys 4 splits 84.7 -> 66.0 us, 1 split
+      // 203.8 -> 181.9; 16 x 4096 x 128 heads, 4 splits 71.7 -> 63.3; left apart: 32 x 2000 x 32 heads, 8 splits 29.8 (34.7),
+      // 8 x 4096 x 128 heads, 8 splits 43.5 (46.7), 48 x 1300 x 48 heads, 3 splits (288 workgroups) 37.8 (55.9).
+      const int64_t pair_wgs = (int64_t)((grid.x + 1) / 2) * grid.y * grid.z;
+      const bool pair = !deep && g_mla_teams == 0 && grid.x > 1 && num_splits <= 4 && pair_wgs >= 128 &&
+                        (grid.x % 2 == 0 || pair_wgs <= 256);
+      const bool two = !pair && !deep && num_splits % 2 == 0 && (int64_t)grid.x * grid.y * grid.z >= 512 && g_mla_teams != 1;
       const int s_out = two ? num_splits / 2 : num_splits;
-      const dim3 grid_t(grid.x, (unsigned)s_out, grid.z);
+      const dim3 grid_t(pair ? (grid.x + 1) / 2 : grid.x, (unsigned)s_out, grid.z);
       if (s_out > 1 && s_out <= MERGE_MAX_SPLITS && aligned16(o)) p.tickets = split_tickets;   // this kernel merges the splits itself
 #define MLR_GO(T_, KERN_, LDS_, THREADS_)                                                                      \
   do {                                                                                                         \
@@ -3085,11 +3200,13 @@ static int decode_attention_mla_impl(const MlaRope* rope, const void* q, const v
   } while (0)
 #define MLR_LAUNCH(T_, CAP_)                                                                                   \
   do {                                                                                                         \
-    if (two && rope) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_, true, 2>), 2 * mlr_lds_bytes(NSB_), 512); \
-    else if (two) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_, false, 2>), 2 * mlr_lds_bytes(NSB_), 512);   \
-    else if (rope) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_, true>), mlr_lds_bytes(NSB_), 256);  \
-    else if (deep) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, 4>), mlr_lds_bytes(4), 256);              \
-    else MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_>), mlr_lds_bytes(NSB_), 256);                  \
+    if (pair && rope) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, 3, true, 2, true>), mlr_lds_total(1, 3, 2), 512);            \
+    else if (pair) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, 3, false, 2, true>), mlr_lds_total(1, 3, 2), 512);              \
+    else if (two && rope) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_, true, 2>), mlr_lds_total(2, NSB_, 2), 512); \
+    else if (two) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_, false, 2>), mlr_lds_total(2, NSB_, 2), 512);        \
+    else if (rope) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_, true>), mlr_lds_total(1, NSB_, 1), 256);           \
+    else if (deep) MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, 4>), mlr_lds_total(1, 4, 1), 256);                       \
+    else MLR_GO(T_, (decode_attn_mla_ring_kernel<T_, CAP_, NSB_>), mlr_lds_total(1, NSB_, 1), 256);                           \
     if (s_out > 1 && !p.tickets)                                                                               \
       hipLaunchKernelGGL((decode_merge_kernel<T_>), dim3((unsigned)(bs * hq)), dim3(128), 0, st, p.part_o,     \
                          p.part_lse, (T_*)o, s_out, kv_lora_rank);                                             \

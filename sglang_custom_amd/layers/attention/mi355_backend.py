@@ -130,9 +130,10 @@ class Mi355AttnBackend(AttentionBackend):
             # 512 workgroups (64 sequences x 16 heads x 4096 keys: 190 / 107 / 75 / 68 us at 1 / 2 / 4 / 8 splits,
             # 91 at 10) with at least 256 keys per split (64 x 1024 keys: 31.6 us at 4 splits, 34.5 at 8)
             # (the ring over an e4m3fn latent cache has the same shape: 64 x 16 x 4096: 103 / 68 / 57 / 81 us at
-            # 2 / 4 / 8 / 16 splits)
+            # 2 / 4 / 8 / 16 splits); never past 512, which would be a second round of workgroups
+            # (24 x 48 heads x 2700 keys, 216 per split: 38.9 us at 7 splits, 60.7 at 8)
             wgs = max(1, bs * self.num_kv_head)
-            return max(1, min(MAX_KV_SPLITS, (512 + wgs - 1) // wgs, max(1, max_seq_len // 256)))
+            return max(1, min(MAX_KV_SPLITS, 512 // wgs, max_seq_len // 256))
         plan = get_ops().decode_num_splits_fp8 if self.kv_fp8 else get_ops().decode_num_splits
         return plan(bs, self.num_kv_head, max_seq_len, MAX_KV_SPLITS)
 

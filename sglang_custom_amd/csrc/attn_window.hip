@@ -7,9 +7,8 @@
 // A workgroup takes one run of consecutive tokens of one sequence, one kv head and the query heads that share it as rows of
 // one tile, walks the key tiles that any of its rows can see (from the window's lower edge of the run's first token to the
 // run's last token) and keeps the running (max, sum) pair per row, started at (sink, 1) -- or (-huge, 0) without a sink.
-//   * 16-bit dtypes, d a multiple of 32 and dv of 16: matrix cores, 64 rows per workgroup (S = Q K^T on 16x16x32 MFMA from
-//     LDS rows, the weights through LDS in the activation dtype, P V with V read by columns; a row's rescale factor travels
-//     through LDS from the wave that owns the row's scores to the waves that own its result columns),
+//   * 16-bit dtypes, d a multiple of 32 and dv of 16: matrix cores, 64 rows per workgroup (S^T = K Q^T and O^T = V^T P^T on
+//     16x16x32 MFMA, a wave per 16 rows, the weights in the activation dtype),
 //   * everything else (fp32, odd widths): vector ALU, 16 rows per workgroup, all fp32.
 // Prefill portions, decode steps and mixed batches are the same launch, told apart only by the list of runs.  A launch of
 // single tokens (a decode step) may cut each token's keys into num_splits ranges: every range leaves its unnormalised sum,
@@ -233,28 +232,33 @@ __global__ __launch_bounds__(256) void window_attention_merge_kernel(T* __restri
   }
 }
 
-// Matrix-core kernel for 16-bit dtypes, d % 32 == 0, dv % 16 == 0.  Four waves, 64 (token, head) rows.  Per key tile of 32:
-//   S: wave w computes its 16 rows x 32 keys with 2 * d / 32 MFMA 16x16x32 (A = Q rows, B = K rows from LDS), masks, updates
-//      its rows' running (max, sum), leaves P in LDS as T and each row's rescale factor in LDS as fp32;
-//   O: wave w owns CT 16-column tiles of the result for ALL row tiles: it rescales them by the rows' factors and adds P V,
-//      one MFMA 16x16x32 per (row tile, column tile), each V fragment read (transposed) once per workgroup.
-// The next tile's K and V rows are requested from global memory into registers before the current tile's products and
-// stored to LDS after them.
-// sm: Qs [64][d + 8] | Ks [32][d + 8] | Vs [32][dv + 8] | Ps [64][32 + 8]   (all T)
+// Matrix-core kernel for 16-bit dtypes, d % 32 == 0, dv % 16 == 0.  Four waves of 16 (token, head) rows.  Per key tile of 32 a
+// wave computes S^T = K Q^T for its rows with 2 * d / 32 MFMA 16x16x32 (A = K rows from LDS, B = Q rows, held in registers):
+// a lane then holds eight scores of ONE row, so that masks, maximum, sum and rescale factor are the lane's own but for two
+// exchanges over registers, and its weights are, rounded to T, the B operand of O^T += V^T P^T as they stand (one MFMA
+// 16x16x32 per 16 result columns, V read transposed).  Nothing travels between waves; the tiles of K and V take turns in two
+// LDS buffers, one barrier each, the next tile's rows on their way from memory meanwhile.
+// What bounds it: the vector ALU (about 90 operations per lane and tile beside 16 MFMAs at d = dv = 128).  7381 prefill tokens
+// of 16 heads over 4, d = 128, window 512 and averaged blocks of 64 (37 GFLOP): 116 us; 273 with S = Q K^T, where a row's
+// scores lay in 16 lanes, its weights and factor went through LDS and the waves shared the result columns (three barriers).
+// sm: 2 x (Ks [32][d + 8] | Vs [32][dv + 8])   (all T)
 constexpr int WAM_ROWS = 64;
-constexpr int WAM_MAXC = 4;      // 16-byte chunks of a K (V) tile per thread: d (dv) up to 256
+constexpr int WAM_MAX = 256;     // d and dv
 
-template <typename T, int CT>
+// max over the lanes that differ in bit 16 or 32 of their number, in registers: a register swapped with its own copy holds one
+// half's values in all lanes of the first result and the other half's in the second
+template <int X> __device__ __forceinline__ float wa_max_xor(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+}
+
+template <typename T, int CT, int CK>
 __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smraw[];
   const int d = a.d, dv = a.dv;
-  const int qld = d + 8, vld = dv + 8, pld = WA_KT + 8;
-  T* Qs = reinterpret_cast<T*>(smraw);
-  T* Ks = Qs + WAM_ROWS * qld;
-  T* Vs = Ks + WA_KT * qld;
-  T* Ps = Vs + WA_KT * vld;
-  __shared__ int row_pos[WAM_ROWS];
-  __shared__ float row_alpha[WAM_ROWS], row_l[WAM_ROWS], row_m[WAM_ROWS];
+  const int qld = d + 8, vld = dv + 8;
+  const int buf_elems = WA_KT * (qld + vld);     // one tile's keys and values; two tiles in turn
   const int rep = a.heads / a.kv_heads;
   const int HR = a.heads_per_tile;
   const int chunks = (rep + HR - 1) / HR;
@@ -268,24 +272,25 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
   const int nh = min(HR, rep - hc * HR);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  const T* q = (const T*)a.q;
   const int dch = d / 8, vch = dv / 8;           // 16-byte chunks per row
   const int live_rows = nt * HR;                 // rows at or past this hold no (token, head)
-  for (int e = tid; e < WAM_ROWS * dch; e += 256) {
-    const int r = e / dch, ch = e - r * dch;
-    const int tl = r / HR, hl = r - tl * HR;
-    Vec<T, 8> val;
-    if (tl < nt && hl < nh) {
-      val = ldvec<T, 8>(q + (t0 + tl) * a.q_token_stride + (int64_t)(h0 + hl) * a.q_head_stride + ch * 8);
-    } else {
+  using Frag = typename Mfma<T>::frag;
+  // this lane's row (the column of its score and result tiles): query li of the wave's sixteen, features 32 c + 8 lg .. + 7
+  const int row = 16 * wv + li;
+  const int tl = row / HR, hl = row - tl * HR;
+  const bool row_ok = tl < nt && hl < nh;
+  const int rp = row_ok ? (int)a.positions[t0 + tl] : -1;
+  Frag qf[2 * CK];
+  {
+    const T* q = (const T*)a.q + (t0 + (row_ok ? tl : 0)) * a.q_token_stride + (int64_t)(h0 + (row_ok ? hl : 0)) * a.q_head_stride + 8 * lg;
+#pragma unroll
+    for (int c = 0; c < 2 * CK; ++c) {
+      Vec<T, 8> val;
 #pragma unroll
       for (int x = 0; x < 8; ++x) val.v[x] = from_f32<T>(0.f);
+      if (32 * c < d && row_ok) val = ldvec<T, 8>(q + 32 * c);
+      qf[c] = __builtin_bit_cast(Frag, val);
     }
-    lds_store16(Qs + r * qld + ch * 8, val);
-  }
-  if (tid < WAM_ROWS) {
-    const int tl = tid / HR, hl = tid - tl * HR;
-    row_pos[tid] = (tl < nt && hl < nh) ? (int)a.positions[t0 + tl] : -1;
   }
   const int first = (int)a.positions[t0];
   const int last = first + nt - 1;
@@ -299,48 +304,39 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
   const int per = (ntiles + a.num_splits - 1) / a.num_splits;
   const int tile_lo = split * per, tile_hi = min(ntiles, tile_lo + per);
   const int nblk = dv / 16;
-  // this lane's four score rows: 16 wv + 4 lg + x
-  float run_m[4], run_l[4];
+  // running maximum of the row (the same in its four lanes) and this lane's share of the running sum
+  float run_m = WA_NEG, run_l = 0.f;
+  if (a.sink != nullptr && split == 0) { run_m = a.sink[h0 + min(hl, nh - 1)]; run_l = lg == 0 ? 1.f : 0.f; }
+  f32x4 acc[4 * CT];
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int r = 16 * wv + 4 * lg + x;
-    const int hl = r % HR;
-    if (a.sink != nullptr && split == 0) { run_m[x] = a.sink[h0 + min(hl, nh - 1)]; run_l[x] = 1.f; }
-    else { run_m[x] = WA_NEG; run_l[x] = 0.f; }
-  }
-  f32x4 acc[4][CT];
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[rt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < 4 * CT; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const T* kc = (const T*)a.k_cache;
   const T* vc = (const T*)a.v_cache;
-  using Frag = typename Mfma<T>::frag;
-  Vec<T, 8> kreg[WAM_MAXC], vreg[WAM_MAXC];
-  int64_t ksrc[WAM_MAXC], vsrc[WAM_MAXC];
-  // every load is unconditional: chunk numbers past the tile's last one are clamped (and never stored), keys outside
+  Vec<T, 8> kreg[CK], vreg[CT];
+  int64_t ksrc[CK], vsrc[CT];
+  int kkey[CK], kch[CK], vkey[CT], vchk[CT];     // (key, chunk) of this thread's pieces of a tile; past the last one: the last
+#pragma unroll
+  for (int u = 0; u < CK; ++u) { const int e = min(tid + 256 * u, WA_KT * dch - 1); kkey[u] = e / dch; kch[u] = 8 * (e - kkey[u] * dch); }
+#pragma unroll
+  for (int u = 0; u < CT; ++u) { const int e = min(tid + 256 * u, WA_KT * vch - 1); vkey[u] = e / vch; vchk[u] = 8 * (e - vkey[u] * vch); }
+  // every load is unconditional: a piece past the tile's last one is the last one again (and never stored), keys outside
   // [0, last] (pooled rows past the last one the run sees) are clamped to a valid row (and masked below)
   auto load_slots = [&](int tile) {
     const bool ptile = tile < ptiles;
     const int j0 = (ptile ? tile : all_lo + tile - ptiles) * WA_KT;
     kc = (const T*)(ptile ? a.pooled_k : a.k_cache);
     vc = (const T*)(ptile ? a.pooled_v : a.v_cache);
+    auto slot = [&](int j) -> int64_t { return ptile ? table[min(j, nb_run - 1) * a.pool + a.pool - 1] / a.pool_div : table[min(j, last)]; };
 #pragma unroll
-    for (int u = 0; u < WAM_MAXC; ++u) {
-      const int ek = min(tid + 256 * u, WA_KT * dch - 1), ev = min(tid + 256 * u, WA_KT * vch - 1);
-      const int kk = ek / dch, kv = ev / vch;
-      const int64_t rk = ptile ? table[min(j0 + kk, nb_run - 1) * a.pool + a.pool - 1] / a.pool_div : table[min(j0 + kk, last)];
-      const int64_t rv = ptile ? table[min(j0 + kv, nb_run - 1) * a.pool + a.pool - 1] / a.pool_div : table[min(j0 + kv, last)];
-      ksrc[u] = (rk * a.kv_heads + g) * d + (ek - kk * dch) * 8;
-      vsrc[u] = (rv * a.kv_heads + g) * dv + (ev - kv * vch) * 8;
-    }
+    for (int u = 0; u < CK; ++u) ksrc[u] = (slot(j0 + kkey[u]) * a.kv_heads + g) * d + kch[u];
+#pragma unroll
+    for (int u = 0; u < CT; ++u) vsrc[u] = (slot(j0 + vkey[u]) * a.kv_heads + g) * dv + vchk[u];
   };
   auto request = [&]() {
 #pragma unroll
-    for (int u = 0; u < WAM_MAXC; ++u) {
-      kreg[u] = ldvec<T, 8>(kc + ksrc[u]);
-      vreg[u] = ldvec<T, 8>(vc + vsrc[u]);
-    }
+    for (int u = 0; u < CK; ++u) kreg[u] = ldvec<T, 8>(kc + ksrc[u]);
+#pragma unroll
+    for (int u = 0; u < CT; ++u) vreg[u] = ldvec<T, 8>(vc + vsrc[u]);
   };
   if (tile_lo < tile_hi) {
     load_slots(tile_lo);
@@ -350,113 +346,95 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
   for (int tile = tile_lo; tile < tile_hi; ++tile) {
     const bool ptile = tile < ptiles;
     const int j0 = (ptile ? tile : all_lo + tile - ptiles) * WA_KT;
-    __syncthreads();                             // the last tile's readers are done (and, the first time, Qs is written)
+    T* Ks = reinterpret_cast<T*>(smraw) + (tile & 1) * buf_elems;   // (its readers, two tiles back, passed the last barrier)
+    T* Vs = Ks + WA_KT * qld;
 #pragma unroll
-    for (int u = 0; u < WAM_MAXC; ++u) {
-      const int e = tid + 256 * u;
-      if (e < WA_KT * dch) {
-        const int kk = e / dch, ch = e - kk * dch;
-        lds_store16(Ks + kk * qld + ch * 8, kreg[u]);
-      }
-      if (e < WA_KT * vch) {
-        const int kk = e / vch, ch = e - kk * vch;
-        lds_store16(Vs + kk * vld + ch * 8, vreg[u]);
-      }
-    }
+    for (int u = 0; u < CK; ++u)
+      if (tid + 256 * u < WA_KT * dch) lds_store16(Ks + kkey[u] * qld + kch[u], kreg[u]);
+#pragma unroll
+    for (int u = 0; u < CT; ++u)
+      if (tid + 256 * u < WA_KT * vch) lds_store16(Vs + vkey[u] * vld + vchk[u], vreg[u]);
     __syncthreads();
     if (tile + 1 < tile_hi) {                    // in flight during this tile's products
       request();
       load_slots(min(tile + 2, tile_hi - 1));
     }
-    if (16 * wv < live_rows) {
-      f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
-      for (int c = 0; c < d; c += 32) {
-        const Frag af = lds_load16<Frag>(Qs + (16 * wv + li) * qld + c + 8 * lg);
-        const Frag b0 = lds_load16<Frag>(Ks + li * qld + c + 8 * lg);
-        const Frag b1 = lds_load16<Frag>(Ks + (16 + li) * qld + c + 8 * lg);
-        s0 = Mfma<T>::run(af, b0, s0);
-        s1 = Mfma<T>::run(af, b1, s1);
-      }
-      // result lane: rows 16 wv + 4 lg + x, key columns li (s0) and 16 + li (s1); a row's 32 scores sit in 16 lanes
+    if (16 * wv >= live_rows) continue;
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int r = 16 * wv + 4 * lg + x;
-        const int rp = row_pos[r];
-        const int ja = j0 + li, jb = j0 + 16 + li;
-        const bool va = ptile ? (rp >= 0 && ja * a.pool + a.pool - 1 <= rp - a.window) : (ja <= rp && (a.window <= 0 || rp - ja < a.window));
-        const bool vb = ptile ? (rp >= 0 && jb * a.pool + a.pool - 1 <= rp - a.window) : (jb <= rp && (a.window <= 0 || rp - jb < a.window));
-        const float sa = va ? s0[x] * a.scale : WA_NEG, sb = vb ? s1[x] * a.scale : WA_NEG;
-        const float new_m = fmaxf(run_m[x], row16_max(fmaxf(sa, sb)));
-        const float alpha = __expf(run_m[x] - new_m);
-        const float pa = va ? __expf(sa - new_m) : 0.f, pb = vb ? __expf(sb - new_m) : 0.f;
-        run_l[x] = run_l[x] * alpha + row16_sum(pa + pb);
-        run_m[x] = new_m;
-        lds_store2(Ps + r * pld + li, from_f32<T>(pa));
-        lds_store2(Ps + r * pld + 16 + li, from_f32<T>(pb));
-        if (li == 0) row_alpha[r] = alpha;
+    for (int c = 0; c < 2 * CK; ++c) {
+      if (32 * c < d) {
+        s[0] = Mfma<T>::run(lds_load16<Frag>(Ks + li * qld + 32 * c + 8 * lg), qf[c], s[0]);
+        s[1] = Mfma<T>::run(lds_load16<Frag>(Ks + (16 + li) * qld + 32 * c + 8 * lg), qf[c], s[1]);
       }
-    } else if (lane < 16) {
-      row_alpha[16 * wv + lane] = 1.f;
     }
-    __syncthreads();
-    {
-      const T* vrow = Vs + (8 * lg + (li >> 2)) * vld + 4 * (li & 3) + 16 * CT * wv;
-      typename TrRead<T>::v4 lo[CT], hi[CT];
+    // the lane holds eight scores of its row: keys 4 lg + x of both halves of the tile
+    bool seen[8];
+    float x8[8], mx = run_m;
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        if (CT * wv + c < nblk) {
-          lo[c] = TrRead<T>::run(vrow + 16 * c);
-          hi[c] = TrRead<T>::run(vrow + 4 * vld + 16 * c);
-        }
-      }
+    for (int i = 0; i < 8; ++i) {
+      const int j = j0 + 16 * (i >> 2) + 4 * lg + (i & 3);
+      seen[i] = ptile ? (rp >= 0 && j * a.pool + a.pool - 1 <= rp - a.window) : (j <= rp && (a.window <= 0 || rp - j < a.window));
+      x8[i] = seen[i] ? s[i >> 2][i & 3] * a.scale : WA_NEG;
+      mx = fmaxf(mx, x8[i]);
+    }
+    mx = wa_max_xor<16>(mx);
+    mx = wa_max_xor<32>(mx);
+    const float alpha = __expf(run_m - mx);
+    run_m = mx;
+    Vec<T, 8> p8;      // key slots 8 lg + i of the product with V: the keys above, in that order
+    float sum = 0.f;
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        if (16 * rt < live_rows) {
-          const Frag pa = lds_load16<Frag>(Ps + (16 * rt + li) * pld + 8 * lg);
-          float al[4];
+    for (int i = 0; i < 8; ++i) {
+      const float pe = seen[i] ? __expf(x8[i] - mx) : 0.f;
+      sum += pe;
+      p8.v[i] = from_f32<T>(pe);
+    }
+    run_l = run_l * alpha + sum;
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
-          for (int x = 0; x < 4; ++x) al[x] = row_alpha[16 * rt + 4 * lg + x];
+      for (int c = 0; c < 4 * CT; ++c) acc[c] *= alpha;
+    }
+    const Frag pf = __builtin_bit_cast(Frag, p8);
+    const T* vrow = Vs + (4 * lg + (li >> 2)) * vld + 4 * (li & 3);
 #pragma unroll
-          for (int c = 0; c < CT; ++c) {
-            if (CT * wv + c < nblk) {
-#pragma unroll
-              for (int x = 0; x < 4; ++x) acc[rt][c][x] *= al[x];
-              typename TrRead<T>::v4 both[2] = {lo[c], hi[c]};
-              acc[rt][c] = Mfma<T>::run(pa, __builtin_bit_cast(Frag, both), acc[rt][c]);
-            }
-          }
-        }
+    for (int c = 0; c < 4 * CT; ++c) {
+      if (c < nblk) {
+        typename TrRead<T>::v4 both[2] = {TrRead<T>::run(vrow + 16 * c), TrRead<T>::run(vrow + 16 * vld + 16 * c)};
+        acc[c] = Mfma<T>::run(__builtin_bit_cast(Frag, both), pf, acc[c]);
       }
     }
   }
-  __syncthreads();
-  if (li == 0) {
+  run_l += __shfl_xor(run_l, 16, 64);
+  run_l += __shfl_xor(run_l, 32, 64);
+  if (!row_ok) return;
+  // the lane holds features 16 c + 4 lg + x of its row
+  if (a.num_splits > 1) {
+    float* part = a.partial + (((int64_t)split * a.tokens + t0 + tl) * a.heads + h0 + hl) * (dv + 2);
 #pragma unroll
-    for (int x = 0; x < 4; ++x) { row_l[16 * wv + 4 * lg + x] = run_l[x]; row_m[16 * wv + 4 * lg + x] = run_m[x]; }
+    for (int c = 0; c < 4 * CT; ++c)
+      if (c < nblk)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) part[16 * c + 4 * lg + x] = acc[c][x];
+    if (lg == 0) { part[dv] = run_m; part[dv + 1] = run_l; }
+    return;
   }
-  __syncthreads();
+  float mul = run_l > 0.f ? 1.f : 0.f;
+  const float den = run_l > 0.f ? run_l : 1.f;
+  if (a.gate != nullptr) mul *= wa_sigmoid(to_f32(((const T*)a.gate)[(t0 + tl) * a.gate_token_stride + h0 + hl]));
+  T* out = (T*)a.out + (t0 + tl) * a.out_token_stride + (int64_t)(h0 + hl) * a.out_head_stride + 4 * lg;
+  const bool four = (reinterpret_cast<uintptr_t>(a.out) & 7) == 0 && ((a.out_token_stride | a.out_head_stride) & 3) == 0;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
+  for (int c = 0; c < 4 * CT; ++c) {
+    if (c >= nblk) continue;
+    Vec<T, 4> w;
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
-      if (CT * wv + c >= nblk) continue;
-      const int col = 16 * (CT * wv + c) + li;
+    for (int x = 0; x < 4; ++x) w.v[x] = from_f32<T>(acc[c][x] / den * mul);
+    if (four) {
+      stvec<T, 4>(out + 16 * c, w);
+    } else {
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int r = 16 * rt + 4 * lg + x;
-        const int tl = r / HR, hl = r - tl * HR;
-        if (tl >= nt || hl >= nh) continue;
-        if (a.num_splits > 1) {
-          float* part = a.partial + (((int64_t)split * a.tokens + t0 + tl) * a.heads + h0 + hl) * (dv + 2);
-          part[col] = acc[rt][c][x];
-          if (col == 0) { part[dv] = row_m[r]; part[dv + 1] = row_l[r]; }
-          continue;
-        }
-        const float l = row_l[r];
-        float o = l > 0.f ? acc[rt][c][x] / l : 0.f;
-        if (a.gate != nullptr) o *= wa_sigmoid(to_f32(((const T*)a.gate)[(t0 + tl) * a.gate_token_stride + h0 + hl]));
-        ((T*)a.out)[(t0 + tl) * a.out_token_stride + (int64_t)(h0 + hl) * a.out_head_stride + col] = from_f32<T>(o);
-      }
+      for (int x = 0; x < 4; ++x) out[16 * c + x] = w.v[x];
     }
   }
 }
@@ -533,26 +511,32 @@ __global__ __launch_bounds__(256) void pool_kv_blocks_kernel(T* __restrict__ pk,
 }
 
 inline bool wa_mfma_shape(int dtype, int d, int dv) {
-  return dtype != MI355_F32 && d % 32 == 0 && dv % 16 == 0 && d <= 32 * WAM_MAXC * 2 && dv <= 32 * WAM_MAXC * 2;
+  return dtype != MI355_F32 && d % 32 == 0 && dv % 16 == 0 && d <= WAM_MAX && dv <= WAM_MAX;
 }
 
 template <typename T> int launch_window(const WaArgs& a, dim3 grid, bool mfma, hipStream_t stream) {
   if constexpr (!std::is_same<T, float>::value) {
     if (mfma) {
-      const size_t lds = ((size_t)(WAM_ROWS + WA_KT) * (a.d + 8) + (size_t)WA_KT * (a.dv + 8) + WAM_ROWS * (WA_KT + 8)) * sizeof(T);
-      const int nblk = a.dv / 16;
-#define MI355_WA_LAUNCH(CT)                                                                                                    \
+      const size_t lds = 2 * (size_t)WA_KT * (a.d + 8 + a.dv + 8) * sizeof(T);
+#define MI355_WA_LAUNCH(CT, CK)                                                                                                \
   do {                                                                                                                         \
     if (lds > 64 * 1024) {                                                                                                     \
-      hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel<T, CT>,                                     \
+      hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel<T, CT, CK>,                                 \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                                \
       MI355_REQUIRE(e == hipSuccess, MI355_ERR_LAUNCH, "window_attention: %zu bytes of LDS refused", lds);                     \
     }                                                                                                                          \
-    hipLaunchKernelGGL((window_attention_mfma_kernel<T, CT>), grid, dim3(256), lds, stream, a);                                \
+    hipLaunchKernelGGL((window_attention_mfma_kernel<T, CT, CK>), grid, dim3(256), lds, stream, a);                            \
   } while (0)
-      if (nblk <= 4) MI355_WA_LAUNCH(1);
-      else if (nblk <= 8) MI355_WA_LAUNCH(2);
-      else MI355_WA_LAUNCH(4);
+#define MI355_WA_KEYS(CT)                                                                                                      \
+  do {                                                                                                                         \
+    if (a.d <= 64) MI355_WA_LAUNCH(CT, 1);                                                                                     \
+    else if (a.d <= 128) MI355_WA_LAUNCH(CT, 2);                                                                               \
+    else MI355_WA_LAUNCH(CT, 4);                                                                                               \
+  } while (0)
+      if (a.dv <= 64) MI355_WA_KEYS(1);
+      else if (a.dv <= 128) MI355_WA_KEYS(2);
+      else MI355_WA_KEYS(4);
+#undef MI355_WA_KEYS
 #undef MI355_WA_LAUNCH
       return MI355_OK;
     }

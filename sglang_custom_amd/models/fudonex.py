@@ -53,6 +53,7 @@ from ..layers.linear_recurrence import (
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.post_norm import NormedResidualAdd
 from ..layers.pre_norm import OffsetRMSNorm
+from ..layers.quantization.unquant import gate_up_silu_mul, pack_gate_up_for_decode
 from ..layers.rotary_embedding import scaled_pair_inv_freq
 from ..layers.short_conv import ShortCausalConv
 from ..layers.vocab_parallel_embedding import ParallelLMHead
@@ -169,7 +170,7 @@ class FudonexMLP(nn.Module):
         self.down = ReplicatedLinear(ff, hidden, dtype, device)
 
     def forward(self, h):
-        return self.down(self.act(self.gate_up(h)[0]))[0]
+        return self.down(gate_up_silu_mul(self.gate_up, self.act, h))[0]
 
 
 _MIXERS = {"attention": FudonexAttention, "mamba2": FudonexStateSpace, "delta": FudonexDeltaRule}
@@ -322,6 +323,9 @@ class FudonexForCausalLM(nn.Module):
     def process_weights_after_loading(self) -> None:
         for lin in self._linears():
             lin.quant_method.process_weights_after_loading(lin)
+        for layer in self.model.layers:
+            if layer.mlp is not None:
+                pack_gate_up_for_decode(layer.mlp.gate_up)   # gate and up rows interleaved: silu * up in the decode GEMM's epilogue
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

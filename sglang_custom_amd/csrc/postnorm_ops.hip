@@ -161,6 +161,163 @@ __global__ __launch_bounds__(256) void rmsnorm_residual_add_kernel(float* __rest
   }
 }
 
+
+// Heads of 16-bit rows, eight features per lane: `lanes` lanes (a power of two, at least width / 8) hold one head's row, so the
+// row is one 16-byte load and store a lane and its sum of squares a few exchanges, and a workgroup takes ONE token's heads,
+// for which it computes the rotation's sines and cosines once.  A wave per head with 2-byte accesses and two sincosf per pair
+// spent its time on those: 7381 tokens x 32 heads of 64 -> fp32 70 us, 16 heads of 128 53 us, and 24 heads of 128 of which 20
+// rotate, norms and cache rows included, 76 us; so 18, 18 and 25 us (floor 18, 12 and 18 us of memory traffic).
+constexpr int PNV_MAX = 512;   // a head's features: 64 lanes
+
+// sines and cosines of a token's pairs, times `mag`, for all threads of the workgroup
+__device__ __forceinline__ void token_angles(float* cs, int64_t position, const float* __restrict__ inv_freq, int half, float mag) {
+  const float pos = (float)position;
+  for (int i = threadIdx.x; i < half; i += blockDim.x) {
+    float sn, c;
+    sincosf(pos * inv_freq[i], &sn, &c);
+    cs[i] = c * mag;
+    cs[half + i] = sn * mag;
+  }
+  __syncthreads();
+}
+
+// One head's row in `lanes` lanes, lane c holding features 8 c .. + 7 in x: RMS norm by w (null: none) and rotation of the
+// first rot features.  Every lane of the group calls it.
+template <typename T>
+__device__ __forceinline__ void norm_rotate_row(float (&x)[8], int c, int lanes, int width, const T* __restrict__ w, bool norm, int rot, int rot_any,
+                                                int interleaved, const float* cs, float eps) {
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q += x[j] * x[j];
+  for (int o = lanes >> 1; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+  if (norm) {
+    const float inv = 1.0f / sqrtf(q / (float)width + eps);
+    Vec<T, 8> wv;
+    if (w != nullptr && 8 * c < width) wv = ldvec<T, 8>(w + 8 * c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = x[j] * inv * (w != nullptr && 8 * c < width ? to_f32(wv.v[j]) : 1.0f);
+  }
+  if (rot_any == 0) return;
+  const int half = rot_any / 2;
+  if (interleaved) {
+    if (8 * c < rot) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float cc = cs[4 * c + j], sn = cs[half + 4 * c + j];
+        const float a = x[2 * j], b = x[2 * j + 1];
+        x[2 * j] = a * cc - b * sn;
+        x[2 * j + 1] = b * cc + a * sn;
+      }
+    }
+    return;
+  }
+  const bool second = 8 * c >= half;
+  const int lane = threadIdx.x & 63;
+  const int partner = 8 * c < rot_any ? (second ? lane - half / 8 : lane + half / 8) : lane;
+  const int pair = second ? 8 * c - half : 8 * c;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float y = __shfl(x[j], partner, 64);
+    if (8 * c < rot) {
+      const float cc = cs[pair + j], sn = cs[half + pair + j];
+      x[j] = second ? x[j] * cc + y * sn : x[j] * cc - y * sn;
+    }
+  }
+}
+
+template <typename T, typename OT>
+__global__ __launch_bounds__(256) void head_norm_rope_vec_kernel(
+    OT* __restrict__ out, const T* __restrict__ src, const T* __restrict__ w, const int64_t* __restrict__ positions,
+    const int64_t* __restrict__ loc, const float* __restrict__ inv_freq, int heads, int d, int lanes, int64_t src_token_stride,
+    int64_t src_head_stride, int64_t out_token_stride, int64_t out_head_stride, int rot_dims, int interleaved, float scale,
+    float eps, float rot_mag) {
+  __shared__ float cs[PNV_MAX];
+  const int64_t t = blockIdx.x;
+  const int c = threadIdx.x & (lanes - 1), first = threadIdx.x / lanes, step = blockDim.x / lanes;
+  const bool live = 8 * c < d;
+  if (rot_dims > 0) token_angles(cs, positions[t], inv_freq, rot_dims / 2, rot_mag);
+  const int64_t orow = loc != nullptr ? loc[t] : t;
+  for (int h = first; h < heads; h += step) {
+    float x[8] = {};
+    if (live) {
+      const Vec<T, 8> v = ldvec<T, 8>(src + t * src_token_stride + (int64_t)h * src_head_stride + 8 * c);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = to_f32(v.v[j]);
+    }
+    norm_rotate_row<T>(x, c, lanes, d, w, w != nullptr, rot_dims, rot_dims, interleaved, cs, eps);
+    if (!live) continue;
+    OT* o = out + orow * out_token_stride + (int64_t)h * out_head_stride + 8 * c;
+    if constexpr (sizeof(OT) == 4) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        Vec<OT, 4> r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r.v[j] = x[4 * p + j] * scale;
+        stvec<OT, 4>(o + 4 * p, r);
+      }
+    } else {
+      Vec<OT, 8> r;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) r.v[j] = from_f32<OT>(x[j] * scale);
+      stvec<OT, 8>(o, r);
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void qkv_norm_rope_write_vec_kernel(
+    T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache, const T* __restrict__ q, const T* __restrict__ k,
+    const T* __restrict__ v, int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, const T* __restrict__ wq,
+    const T* __restrict__ wk, const int64_t* __restrict__ positions, const int64_t* __restrict__ loc,
+    const float* __restrict__ inv_freq, int heads, int kv_heads, int d, int dv, int lanes, int rot_dims, int interleaved,
+    float eps, float rot_mag) {
+  __shared__ float cs[PNV_MAX];
+  const int64_t t = blockIdx.x;
+  const int c = threadIdx.x & (lanes - 1), first = threadIdx.x / lanes, step = blockDim.x / lanes;
+  if (rot_dims > 0) token_angles(cs, positions[t], inv_freq, rot_dims / 2, rot_mag);
+  const int64_t slot = loc[t] * kv_heads;
+  for (int u = first; u < heads + 2 * kv_heads; u += step) {
+    const T *s, *w;
+    T* o;
+    int width = d, rot = rot_dims;
+    if (u < heads) {
+      s = q + t * q_token_stride + (int64_t)u * d; w = wq;
+      o = q_out + (t * heads + u) * (int64_t)d;
+    } else if (u < heads + kv_heads) {
+      const int g = u - heads;
+      s = k + t * k_token_stride + (int64_t)g * d; w = wk;
+      o = k_cache + (slot + g) * (int64_t)d;
+    } else {
+      const int g = u - heads - kv_heads;
+      s = v + t * v_token_stride + (int64_t)g * dv; w = nullptr; width = dv; rot = 0;
+      o = v_cache + (slot + g) * (int64_t)dv;
+    }
+    const bool live = 8 * c < width;
+    float x[8] = {};
+    if (live) {
+      const Vec<T, 8> xv = ldvec<T, 8>(s + 8 * c);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = to_f32(xv.v[j]);
+    }
+    norm_rotate_row<T>(x, c, lanes, width, w, true, rot, rot_dims, interleaved, cs, eps);
+    if (!live) continue;
+    Vec<T, 8> r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r.v[j] = from_f32<T>(x[j]);
+    stvec<T, 8>(o + 8 * c, r);
+  }
+}
+
+// the lanes of a row, and the threads that one token's rows fill
+int pnv_lanes(int width) {
+  int lanes = 1;
+  while (8 * lanes < width) lanes *= 2;
+  return lanes;
+}
+unsigned pnv_threads(int units, int lanes) { return (unsigned)std::min(256, (units * lanes + 63) / 64 * 64); }
+bool pnv_rotation(int rot_dims, int interleaved) { return rot_dims % (interleaved ? 8 : 16) == 0; }
+bool pnv_aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 // One wave per (token, head); four per workgroup.  sm: 4 rows of d floats.
 template <typename T, typename OT>
 __global__ __launch_bounds__(256) void head_norm_rope_kernel(
@@ -371,6 +528,41 @@ __global__ __launch_bounds__(256) void qkv_rotate_write_kernel(
 // gate applied BEFORE the norm.  y fp32 [tokens, D] contiguous, gate T row-strided, w T [D].  A part of up to 2048 features
 // keeps its gated values in registers between the two passes.
 constexpr int GGN_KEEP = 8;
+// Groups of at most 512 features in 16-bit results: `lanes` lanes hold a group, eight features each.  7381 tokens x 4 groups
+// of 512: 50 -> 25 us (floor 24); a workgroup per group moved two features a thread.
+template <typename T>
+__global__ __launch_bounds__(256) void gated_group_rmsnorm_vec_kernel(T* __restrict__ out, const float* __restrict__ y, const T* __restrict__ gate,
+                                                                      int64_t gate_stride, const T* __restrict__ w, int64_t rows, int groups,
+                                                                      int n, int lanes, float eps) {
+  const int c = threadIdx.x & (lanes - 1);
+  const int64_t idx = (int64_t)blockIdx.x * (256 / lanes) + threadIdx.x / lanes;
+  const bool live = idx < rows && 8 * c < n;
+  const int64_t t = idx / groups;
+  const int at = (int)(idx - t * groups) * n + 8 * c;
+  float r[8] = {};
+  Vec<T, 8> wv;
+  if (live) {
+    const Vec<float, 4> a = ldvec<float, 4>(y + idx * n + 8 * c), b = ldvec<float, 4>(y + idx * n + 8 * c + 4);
+    const Vec<T, 8> g = ldvec<T, 8>(gate + t * gate_stride + at);
+    wv = ldvec<T, 8>(w + at);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float z = to_f32(g.v[j]);
+      r[j] = (j < 4 ? a.v[j & 3] : b.v[j & 3]) * (z * pn_sigmoid(z));
+    }
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q += r[j] * r[j];
+  for (int s = lanes >> 1; s > 0; s >>= 1) q += __shfl_xor(q, s, 64);
+  if (!live) return;
+  const float inv = 1.0f / sqrtf(q / (float)n + eps);
+  Vec<T, 8> res;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) res.v[j] = from_f32<T>(r[j] * inv * to_f32(wv.v[j]));
+  stvec<T, 8>(out + idx * n + 8 * c, res);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(T* __restrict__ out, const float* __restrict__ y,
                                                                   const T* __restrict__ gate, int64_t gate_stride,
@@ -414,6 +606,42 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(T* __restrict_
 
 // One wave per (token, head): out = o / rms(o) (* w) * silu(gate), or * sigmoid(gate) with gate_act 1; w [dv] shared by the heads,
 // or (w_per_head) [heads, dv]
+// the same for 16-bit results, eight features per lane and `lanes` lanes a row: the fp32 row and the gate come once, in 16-byte
+// pieces.  7381 tokens x 16 heads of 128: 53 -> 27 us (floor 24).
+template <typename T>
+__global__ __launch_bounds__(256) void head_rmsnorm_gate_vec_kernel(T* __restrict__ out, const float* __restrict__ o, const T* __restrict__ w,
+                                                                    const T* __restrict__ gate, int64_t gate_stride, int64_t rows, int heads,
+                                                                    int dv, int lanes, float eps, int gate_act, int w_per_head) {
+  const int c = threadIdx.x & (lanes - 1);
+  const int64_t idx = (int64_t)blockIdx.x * (256 / lanes) + threadIdx.x / lanes;
+  const bool live = idx < rows && 8 * c < dv;
+  const int64_t t = idx / heads;
+  const int h = (int)(idx - t * heads);
+  float r[8] = {};
+  Vec<T, 8> g, wv;
+  if (live) {
+    const Vec<float, 4> a = ldvec<float, 4>(o + idx * dv + 8 * c), b = ldvec<float, 4>(o + idx * dv + 8 * c + 4);
+    g = ldvec<T, 8>(gate + t * gate_stride + (int64_t)h * dv + 8 * c);
+    if (w != nullptr) wv = ldvec<T, 8>(w + (w_per_head ? (int64_t)h * dv : 0) + 8 * c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { r[j] = a.v[j]; r[4 + j] = b.v[j]; }
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q += r[j] * r[j];
+  for (int s = lanes >> 1; s > 0; s >>= 1) q += __shfl_xor(q, s, 64);
+  if (!live) return;
+  const float inv = 1.0f / sqrtf(q / (float)dv + eps);
+  Vec<T, 8> res;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float z = to_f32(g.v[j]);
+    const float n = r[j] * inv * (w != nullptr ? to_f32(wv.v[j]) : 1.0f);
+    res.v[j] = from_f32<T>(gate_act == 1 ? n * pn_sigmoid(z) : n * z * pn_sigmoid(z));
+  }
+  stvec<T, 8>(out + idx * dv + 8 * c, res);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void head_rmsnorm_gate_kernel(T* __restrict__ out, const float* __restrict__ o,
                                                                 const T* __restrict__ w, const T* __restrict__ gate,
@@ -661,7 +889,28 @@ int mi355_head_norm_rope_mag(void* out, const void* src, const void* weight, con
   if (tokens == 0) return MI355_OK;
   const size_t lds = (size_t)4 * head_dim * sizeof(float);
   const unsigned grid = (unsigned)((tokens * heads + 3) / 4);
+  // whole 16-byte pieces of every row, in and out (a wave per head where they are not)
+  const bool vec = dtype != MI355_F32 && head_dim % 8 == 0 && head_dim <= PNV_MAX && pnv_rotation(rot_dims, interleaved) &&
+                   pnv_aligned(out) && pnv_aligned(src) && pnv_aligned(weight) && tokens < ((int64_t)1 << 31) &&
+                   ((src_token_stride | src_head_stride) & 7) == 0 &&
+                   ((out_token_stride | out_head_stride) & (out_dtype == MI355_F32 ? 3 : 7)) == 0;
+  const int lanes = pnv_lanes(head_dim);
   MI355_DISPATCH_DTYPE(dtype, "head_norm_rope", {
+    if constexpr (sizeof(T) == 2) {
+      if (vec) {
+        const dim3 g2((unsigned)tokens), b2(pnv_threads(heads, lanes));
+        if (out_dtype == dtype)
+          hipLaunchKernelGGL((head_norm_rope_vec_kernel<T, T>), g2, b2, 0, (hipStream_t)stream, (T*)out, (const T*)src, (const T*)weight,
+                             positions, loc, inv_freq, heads, head_dim, lanes, src_token_stride, src_head_stride, out_token_stride,
+                             out_head_stride, rot_dims, interleaved, scale, eps, rot_mag);
+        else
+          hipLaunchKernelGGL((head_norm_rope_vec_kernel<T, float>), g2, b2, 0, (hipStream_t)stream, (float*)out, (const T*)src,
+                             (const T*)weight, positions, loc, inv_freq, heads, head_dim, lanes, src_token_stride, src_head_stride,
+                             out_token_stride, out_head_stride, rot_dims, interleaved, scale, eps, rot_mag);
+        MI355_CHECK_LAUNCH("head_norm_rope");
+        return MI355_OK;
+      }
+    }
     if (out_dtype == dtype) {
       hipLaunchKernelGGL((head_norm_rope_kernel<T, T>), dim3(grid), dim3(256), lds, (hipStream_t)stream, (T*)out, (const T*)src,
                          (const T*)weight, positions, loc, inv_freq, tokens, heads, head_dim, src_token_stride, src_head_stride,
@@ -694,7 +943,20 @@ int mi355_head_rmsnorm_gate_wide(void* out, const float* o, const void* weight, 
                 "head_rmsnorm_gate: bad shape");
   if (tokens == 0) return MI355_OK;
   const unsigned grid = (unsigned)((tokens * heads + 3) / 4);
+  const bool vec = dtype != MI355_F32 && value_dim % 8 == 0 && value_dim <= PNV_MAX && pnv_aligned(out) && pnv_aligned(o) &&
+                   pnv_aligned(weight) && pnv_aligned(gate) && (gate_stride & 7) == 0;
   MI355_DISPATCH_DTYPE(dtype, "head_rmsnorm_gate", {
+    if constexpr (sizeof(T) == 2) {
+      if (vec) {
+        const int lanes = pnv_lanes(value_dim);
+        const int64_t per = 256 / lanes;
+        hipLaunchKernelGGL((head_rmsnorm_gate_vec_kernel<T>), dim3((unsigned)((tokens * heads + per - 1) / per)), dim3(256), 0,
+                           (hipStream_t)stream, (T*)out, o, (const T*)weight, (const T*)gate, gate_stride, tokens * heads, heads, value_dim,
+                           lanes, eps, gate_act, weight_per_head);
+        MI355_CHECK_LAUNCH("head_rmsnorm_gate");
+        return MI355_OK;
+      }
+    }
     hipLaunchKernelGGL((head_rmsnorm_gate_kernel<T>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (T*)out, o, (const T*)weight,
                        (const T*)gate, gate_stride, tokens, heads, value_dim, eps, gate_act, weight_per_head);
   });
@@ -716,7 +978,22 @@ int mi355_qkv_norm_rope_write(void* q_out, void* k_cache, void* v_cache, const v
   if (tokens == 0) return MI355_OK;
   const size_t lds = (size_t)4 * std::max(head_dim, v_head_dim) * sizeof(float);
   const unsigned grid = (unsigned)((tokens * (heads + 2 * kv_heads) + 3) / 4);
+  const bool vec = dtype != MI355_F32 && head_dim % 8 == 0 && v_head_dim % 8 == 0 && std::max(head_dim, v_head_dim) <= PNV_MAX &&
+                   pnv_rotation(rot_dims, interleaved) && pnv_aligned(q_out) && pnv_aligned(k_cache) && pnv_aligned(v_cache) &&
+                   pnv_aligned(q) && pnv_aligned(k) && pnv_aligned(v) && pnv_aligned(wq) && pnv_aligned(wk) &&
+                   ((q_token_stride | k_token_stride | v_token_stride) & 7) == 0 && tokens < ((int64_t)1 << 31);
+  const int lanes = pnv_lanes(std::max(head_dim, v_head_dim));
   MI355_DISPATCH_DTYPE(dtype, "qkv_norm_rope_write", {
+    if constexpr (sizeof(T) == 2) {
+      if (vec) {
+        hipLaunchKernelGGL((qkv_norm_rope_write_vec_kernel<T>), dim3((unsigned)tokens), dim3(pnv_threads(heads + 2 * kv_heads, lanes)), 0,
+                           (hipStream_t)stream, (T*)q_out, (T*)k_cache, (T*)v_cache, (const T*)q, (const T*)k, (const T*)v, q_token_stride,
+                           k_token_stride, v_token_stride, (const T*)wq, (const T*)wk, positions, loc, inv_freq, heads, kv_heads, head_dim,
+                           v_head_dim, lanes, rot_dims, interleaved, eps, rot_mag);
+        MI355_CHECK_LAUNCH("qkv_norm_rope_write");
+        return MI355_OK;
+      }
+    }
     hipLaunchKernelGGL((qkv_norm_rope_write_kernel<T>), dim3(grid), dim3(256), lds, (hipStream_t)stream, (T*)q_out, (T*)k_cache,
                        (T*)v_cache, (const T*)q, (const T*)k, (const T*)v, q_token_stride, k_token_stride, v_token_stride, (const T*)wq,
                        (const T*)wk, positions, loc, inv_freq, tokens, heads, kv_heads, head_dim, v_head_dim, rot_dims, interleaved, eps,
@@ -759,7 +1036,21 @@ int mi355_gated_group_rmsnorm(void* out, const float* y, const void* gate, int64
   MI355_REQUIRE(tokens >= 0 && hidden > 0 && groups >= 1 && hidden % groups == 0 && gate_stride >= hidden &&
                     tokens * groups < ((int64_t)1 << 31), MI355_ERR_INVALID, "gated_group_rmsnorm: bad shape");
   if (tokens == 0) return MI355_OK;
+  const int64_t n = hidden / groups;
+  const bool vec = dtype != MI355_F32 && n % 8 == 0 && n <= PNV_MAX && pnv_aligned(out) && pnv_aligned(y) && pnv_aligned(gate) &&
+                   pnv_aligned(weight) && (gate_stride & 7) == 0;
   MI355_DISPATCH_DTYPE(dtype, "gated_group_rmsnorm", {
+    if constexpr (sizeof(T) == 2) {
+      if (vec) {
+        const int lanes = pnv_lanes((int)n);
+        const int64_t per = 256 / lanes;
+        hipLaunchKernelGGL((gated_group_rmsnorm_vec_kernel<T>), dim3((unsigned)((tokens * groups + per - 1) / per)), dim3(256), 0,
+                           (hipStream_t)stream, (T*)out, y, (const T*)gate, gate_stride, (const T*)weight, tokens * groups, groups, (int)n,
+                           lanes, eps);
+        MI355_CHECK_LAUNCH("gated_group_rmsnorm");
+        return MI355_OK;
+      }
+    }
     hipLaunchKernelGGL((gated_group_rmsnorm_kernel<T>), dim3((unsigned)(tokens * groups)), dim3(256), 0, (hipStream_t)stream, (T*)out, y,
                        (const T*)gate, gate_stride, (const T*)weight, hidden, groups, eps);
   });

@@ -229,11 +229,39 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
   const bool vec = (row_stride % 4 == 0) && aligned16(logits);
   const ChunkSpan sp = chunk_span(vocab, c, chunks);
   const float t = temperatures[r];
-  float mx = -INFINITY;
-  span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, x / t); });
-  mx = block_reduce_max(mx, red);
-  float sum = 0.f;
-  span_each(row, vocab, sp, vec, [&](float x) { sum += expf(x / t - mx); });
+  float mx = -INFINITY, sum = 0.f;
+  constexpr int KEEP = 8;   // 16-byte pieces a thread holds: chunks up to 32 K entries (every vocabulary up to 512 K at few rows)
+  if (vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS) {
+    // The chunk is read once, all of it requested before anything is used, and divided once: 64 rows x 128256 entries
+    // 14.1 us (floor 7); 17.8 with two passes of one piece at a time.
+    Vec<float, 4> v[KEEP];
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) {
+      const int64_t i = sp.v0 + threadIdx.x + u * SAMP_THREADS;
+      v[u] = ldvec<float, 4>(row + 4 * (i < sp.v1 ? i : sp.v1 - 1));
+    }
+    const int64_t k = vocab / 4 * 4 + threadIdx.x;
+    const bool one = sp.tail && k < vocab;
+    const float last = one ? row[k] / t : -INFINITY;
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[u].v[j] /= t;
+        mx = fmaxf(mx, v[u].v[j]);   // (a piece past the end repeats the last one: the maximum does not mind)
+      }
+    mx = block_reduce_max(fmaxf(mx, last), red);
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u)
+      if (sp.v0 + threadIdx.x + u * SAMP_THREADS < sp.v1)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum += expf(v[u].v[j] - mx);
+    if (one) sum += expf(last - mx);
+  } else {
+    span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, x / t); });
+    mx = block_reduce_max(mx, red);
+    span_each(row, vocab, sp, vec, [&](float x) { sum += expf(x / t - mx); });
+  }
   sum = block_sum(sum, red);
   if (threadIdx.x == 0) partials[(int64_t)r * chunks + c] = float2{mx, sum};
 }

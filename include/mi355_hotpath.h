@@ -389,6 +389,14 @@ int mi355_mla_absorb(void* out, const void* a, const void* w_t, int64_t m, int h
                      int64_t a_row_stride, int64_t a_head_stride, int64_t out_row_stride, int64_t out_head_stride,
                      int dtype, void* stream);
 
+/* mi355_mla_prefill_rotate: the same without k and v, for mi355_latent_prefill_attention, which reads kv_b_proj's output as it
+ * is: q's rope part rotated in place, rope(k_pe[t]) to the dense k_pe_out [tokens, rope], the latent row written.  rope_dim a
+ * multiple of 16; k_pe rows of any alignment. */
+int mi355_mla_prefill_rotate(void* q, void* k_pe_out, const void* k_pe, int64_t k_pe_stride, const void* c_kv, int64_t c_kv_stride,
+                             const int64_t* positions, const void* cos_sin_cache, int cache_dtype, int is_neox, void* kv_cache,
+                             const int64_t* out_cache_loc, int64_t tokens, int heads, int nope_dim, int rope_dim, int kv_lora_rank,
+                             int64_t q_stride, int64_t num_slots, int dtype, void* stream);
+
 /* mi355_mla_prefill_assemble: the glue of MLA's multi-head prefill in one launch.  In place: q [tokens, heads, nope +
  * rope] (row stride q_stride) gets its rope part rotated at positions[t].  Out: k [tokens, heads, nope + rope] =
  * [kv's nope part | rope(k_pe[t])] and v [tokens, heads, v_dim] (both dense) from kv [tokens, heads, nope + v_dim]

@@ -256,6 +256,68 @@ __global__ __launch_bounds__(256) void mla_prefill_assemble_kernel(
   }
 }
 
+// What is left of the assembly where the attention kernel takes keys and values as kv_b_proj leaves them and the rope part of
+// the keys once per token: rotate q's rope parts in place, the token's k_pe into `pe_out`, write the latent row.  In 16-byte
+// pieces, the token's angles once: 7373 tokens x 32 heads of 128 + 64 25 us (90 MB, floor 18); with k and v assembled 94.
+template <typename T>
+__global__ __launch_bounds__(256) void mla_prefill_rotate_kernel(
+    T* __restrict__ q, T* __restrict__ pe_out, const T* __restrict__ k_pe, int64_t k_pe_stride, const T* __restrict__ c_kv,
+    int64_t c_kv_stride, const int64_t* __restrict__ positions, const void* __restrict__ cos_sin, int cache_f32, int is_neox,
+    void* __restrict__ cache, const int64_t* __restrict__ out_loc, int cache_fp8, int H, int nope, int rope, int rank, int64_t q_stride) {
+  __shared__ __attribute__((aligned(16))) T s_pe[256];
+  __shared__ float s_cs[256];
+  const int64_t t = blockIdx.x;
+  const int64_t pos = positions[t];
+  const int half = rope / 2;
+  for (int i = threadIdx.x; i < rope; i += 256)
+    s_cs[i] = cache_f32 ? static_cast<const float*>(cos_sin)[pos * rope + i] : to_f32(static_cast<const T*>(cos_sin)[pos * rope + i]);
+  __syncthreads();
+  const int ia = is_neox ? 1 : 2, ib = is_neox ? half : 1;
+  const T* pe = k_pe + t * k_pe_stride;
+  for (int i = threadIdx.x; i < half; i += 256) {
+    T o1, o2;
+    rope_pair<T>(to_f32(pe[ia * i]), to_f32(pe[ia * i + ib]), s_cs[i], s_cs[half + i], o1, o2);
+    s_pe[ia * i] = o1;
+    s_pe[ia * i + ib] = o2;
+  }
+  T* qt = q + t * q_stride + nope;
+  if (is_neox) {   // a piece and its partner half a part on
+    const int n = half / 8;
+    for (int it = threadIdx.x; it < H * n; it += 256) {
+      const int h = it / n, c = it - h * n;
+      T* p1 = qt + (int64_t)h * (nope + rope) + 8 * c;
+      Vec<T, 8> x1 = ldvec<T, 8>(p1), x2 = ldvec<T, 8>(p1 + half);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        rope_pair<T>(to_f32(x1.v[j]), to_f32(x2.v[j]), s_cs[8 * c + j], s_cs[half + 8 * c + j], x1.v[j], x2.v[j]);
+      stvec<T, 8>(p1, x1);
+      stvec<T, 8>(p1 + half, x2);
+    }
+  } else {
+    const int n = rope / 8;
+    for (int it = threadIdx.x; it < H * n; it += 256) {
+      const int h = it / n, c = it - h * n;
+      T* p1 = qt + (int64_t)h * (nope + rope) + 8 * c;
+      Vec<T, 8> x = ldvec<T, 8>(p1);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        rope_pair<T>(to_f32(x.v[2 * j]), to_f32(x.v[2 * j + 1]), s_cs[4 * c + j], s_cs[half + 4 * c + j], x.v[2 * j], x.v[2 * j + 1]);
+      stvec<T, 8>(p1, x);
+    }
+  }
+  __syncthreads();
+  const int64_t slot = out_loc[t];
+  for (int c = threadIdx.x; c < (rank + rope) / 8; c += 256) {
+    const bool rot = c >= rank / 8;
+    const Vec<T, 8> x = rot ? *reinterpret_cast<const Vec<T, 8>*>(s_pe + 8 * (c - rank / 8)) : ldvec<T, 8>(c_kv + t * c_kv_stride + 8 * c);
+    if (rot) stvec<T, 8>(pe_out + t * rope + 8 * (c - rank / 8), x);
+    if (cache_fp8)
+      *reinterpret_cast<uint2*>(static_cast<uint8_t*>(cache) + slot * (rank + rope) + 8 * c) = quant8_fp8<T>(x, 1.0f);
+    else
+      stvec<T, 8>(static_cast<T*>(cache) + slot * (rank + rope) + 8 * c, x);
+  }
+}
+
 }  // namespace mi355
 
 using namespace mi355;
@@ -361,6 +423,39 @@ int mi355_mla_prefill_assemble(void* q, void* k, void* v, const void* kv, const 
   else LAUNCH(f16_t);
 #undef LAUNCH
   MI355_CHECK_LAUNCH("mla_prefill_assemble");
+  return MI355_OK;
+}
+
+int mi355_mla_prefill_rotate(void* q, void* k_pe_out, const void* k_pe, int64_t k_pe_stride, const void* c_kv, int64_t c_kv_stride,
+                             const int64_t* positions, const void* cos_sin_cache, int cache_dtype, int is_neox, void* kv_cache,
+                             const int64_t* out_cache_loc, int64_t tokens, int heads, int nope_dim, int rope_dim, int kv_lora_rank,
+                             int64_t q_stride, int64_t num_slots, int dtype, void* stream) {
+  MI355_REQUIRE(q && k_pe_out && k_pe && c_kv && positions && cos_sin_cache && kv_cache && out_cache_loc, MI355_ERR_INVALID,
+                "mla_prefill_rotate: null pointer");
+  const bool kv8 = (dtype & MI355_KV_FP8) != 0;
+  dtype &= 0xff;
+  MI355_REQUIRE(dtype == MI355_BF16 || dtype == MI355_F16, MI355_ERR_UNSUPPORTED, "mla_prefill_rotate: only 16-bit dtypes");
+  MI355_REQUIRE(cache_dtype == MI355_F32 || cache_dtype == dtype, MI355_ERR_UNSUPPORTED,
+                "mla_prefill_rotate: cos_sin_cache must be fp32 or the tensor dtype");
+  MI355_REQUIRE(tokens >= 0 && heads >= 1 && nope_dim > 0 && rope_dim > 0 && kv_lora_rank > 0 && num_slots > 0 && nope_dim % 8 == 0 &&
+                    rope_dim % 16 == 0 && rope_dim <= 256 && kv_lora_rank % 8 == 0,
+                MI355_ERR_UNSUPPORTED, "mla_prefill_rotate: widths in pieces of 8, rope_dim of 16 and at most 256 (nope=%d rope=%d rank=%d)",
+                nope_dim, rope_dim, kv_lora_rank);
+  MI355_REQUIRE(q_stride >= (int64_t)heads * (nope_dim + rope_dim) && q_stride % 8 == 0 && k_pe_stride >= rope_dim &&
+                    c_kv_stride >= kv_lora_rank && c_kv_stride % 8 == 0,
+                MI355_ERR_INVALID, "mla_prefill_rotate: row strides must cover the rows and be multiples of 8");
+  MI355_REQUIRE(aligned16(q) && aligned16(k_pe_out) && aligned16(c_kv) && (reinterpret_cast<uintptr_t>(kv_cache) & (kv8 ? 7 : 15)) == 0,
+                MI355_ERR_INVALID, "mla_prefill_rotate: misaligned pointer");
+  if (tokens == 0) return MI355_OK;
+#define LAUNCH(T)                                                                                                    \
+  hipLaunchKernelGGL((mla_prefill_rotate_kernel<T>), dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream,      \
+                     (T*)q, (T*)k_pe_out, (const T*)k_pe, k_pe_stride, (const T*)c_kv, c_kv_stride, positions,       \
+                     cos_sin_cache, cache_dtype == MI355_F32 ? 1 : 0, is_neox, kv_cache, out_cache_loc,              \
+                     kv8 ? 1 : 0, heads, nope_dim, rope_dim, kv_lora_rank, q_stride)
+  if (dtype == MI355_BF16) LAUNCH(bf16_t);
+  else LAUNCH(f16_t);
+#undef LAUNCH
+  MI355_CHECK_LAUNCH("mla_prefill_rotate");
   return MI355_OK;
 }
 

@@ -346,6 +346,19 @@ class Mi355AttnBackend(AttentionBackend):
             forward_batch.positions, layer.inv_freq, layer.rot_dims, max(forward_batch.extend_seq_lens_cpu), layer.scaling,
             interleaved=layer.interleaved, rot_mag=layer.rot_mag)
 
+    def mla_expanded_prefill_ok(self, layer, forward_batch, nope: int, rope: int, v: int, dtype) -> bool:
+        """Whether forward_mla_expanded serves a step of whole prompts (nothing cached) over expanded keys and values."""
+        return (forward_batch.extend_prefix_lens_cpu is not None and not any(forward_batch.extend_prefix_lens_cpu)
+                and forward_batch.extend_start_loc is not None and layer.logit_cap == 0
+                and self.sliding_window_size is None and str(self.device).startswith("cuda") and rope % 16 == 0
+                and get_ops().latent_prefill_attention_supported(nope, rope, v, 0, False, dtype))
+
+    def forward_mla_expanded(self, q, kv, k_pe, layer, forward_batch):
+        """q [T, H, nope + rope] and k_pe [T, rope] rotated, kv [T, H, nope + v] -> [T, H, v]."""
+        return get_ops().latent_prefill_attention(
+            q, kv, k_pe, forward_batch.extend_start_loc, forward_batch.extend_seq_lens, forward_batch.positions, None, 0,
+            max(forward_batch.extend_seq_lens_cpu), layer.scaling)
+
     # ---- causal attention with sigmoid weights (no softmax) over per-layer key / value buffers ----
     def forward_sigmoid(self, q, layer, forward_batch, out):
         """q [T, H, d] normed and rotated -> out [T, H, dv] = sum over visible keys of sigmoid(q.k * scale * temp_h + bias_h) v.

@@ -178,6 +178,14 @@ class DeepseekV2AttentionMLA(nn.Module):
                 and positions.dtype == torch.int64 and kv.is_contiguous() and q.is_contiguous()
                 and ops.mla_prefill_assemble_supported(self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim,
                                                        self.kv_lora_rank, q.dtype)):
+            be = forward_batch.attn_backend
+            if getattr(be, "mla_expanded_prefill_ok", None) is not None and be.mla_expanded_prefill_ok(
+                    self.attn_mha, forward_batch, self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, q.dtype):
+                # RoPE of q and k_pe and the write of the latent rows; the attention reads kv_b_proj's output as it is
+                k_pe = ops.mla_prefill_rotate(q, k_pe_raw, kv_a, positions.flatten(), rot.cos_sin_cache, rot.is_neox_style,
+                                              pool.get_key_buffer(self.attn_mha.layer_id), forward_batch.out_cache_loc)
+                attn_output = be.forward_mla_expanded(q, kv, k_pe, self.attn_mha, forward_batch)
+                return self.o_proj(attn_output.view(-1, self.num_local_heads * self.v_head_dim))[0]
             # RoPE of q and k_pe, the k / v assembly and the write of the latent rows in one launch
             k, v = ops.mla_prefill_assemble(
                 q, kv, k_pe_raw, kv_a, positions.flatten(), rot.cos_sin_cache, rot.is_neox_style,

@@ -622,6 +622,27 @@ def mla_prefill_assemble(q, kv, k_pe, c_kv, positions, cos_sin_cache, is_neox: b
     return k, v
 
 
+def mla_prefill_rotate(q, k_pe, c_kv, positions, cos_sin_cache, is_neox: bool, kv_cache, out_cache_loc) -> torch.Tensor:
+    """mla_prefill_assemble without k and v, for latent_prefill_attention: q [T, H, nope + rope] gets its rope part rotated in
+    place, the latent row [c_kv | rope(k_pe)] is written; returns rope(k_pe) [T, rope]."""
+    _gpu(q, k_pe, c_kv, positions, cos_sin_cache, kv_cache, out_cache_loc)
+    T, H, D = q.shape
+    rank, rope = c_kv.shape[1], k_pe.shape[1]
+    assert D > rope and q.stride(2) == 1 and q.stride(1) == D and k_pe.shape[0] == c_kv.shape[0] == T
+    assert k_pe.stride(1) == 1 and c_kv.stride(1) == 1 and k_pe.dtype == q.dtype and c_kv.dtype == q.dtype
+    assert positions.dtype == torch.int64 and positions.is_contiguous() and positions.numel() == T
+    assert out_cache_loc.dtype == torch.int64 and out_cache_loc.is_contiguous() and out_cache_loc.numel() == T
+    assert cos_sin_cache.is_contiguous() and cos_sin_cache.shape[1] == rope
+    assert kv_cache.is_contiguous() and kv_cache.shape[1] == 1 and kv_cache.shape[2] == rank + rope
+    assert kv_cache.dtype in (q.dtype, torch.float8_e4m3fn)
+    pe = torch.empty((T, rope), dtype=q.dtype, device=q.device)
+    check(_lib_().mi355_mla_prefill_rotate(
+        q.data_ptr(), pe.data_ptr(), k_pe.data_ptr(), k_pe.stride(0), c_kv.data_ptr(), c_kv.stride(0), positions.data_ptr(),
+        cos_sin_cache.data_ptr(), _dt(cos_sin_cache), 1 if is_neox else 0, kv_cache.data_ptr(), out_cache_loc.data_ptr(), T, H,
+        D - rope, rope, rank, q.stride(0), kv_cache.shape[0], _kvdt(q, kv_cache), _stream(q)), "mla_prefill_rotate")
+    return pe
+
+
 def extend_attention_mla_supported(hq: int, kv_lora_rank: int, rope_dim: int, dtype: torch.dtype) -> bool:
     """Whether extend_attention_mla serves the shape (latent row of 512 + 64 features, 16-bit)."""
     return dtype in (torch.bfloat16, torch.float16) and bool(
@@ -1291,10 +1312,10 @@ def latent_prefill_attention_supported(nope: int, rope: int, v: int, rot_dims: i
 
 
 def latent_prefill_attention(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Tensor, seg_start: torch.Tensor, seg_len: torch.Tensor,
-                             positions: torch.Tensor, inv_freq: torch.Tensor, rot_dims: int, max_len: int, scale: float,
+                             positions: torch.Tensor, inv_freq: Optional[torch.Tensor], rot_dims: int, max_len: int, scale: float,
                              interleaved: bool = False, rot_mag: float = 1.0) -> torch.Tensor:
-    """Causal attention of whole sequences over expanded latents: q [T, H, nope + rope] (any row stride), rope part unrotated; kv
-    [T, H, nope + v]; k_rope [T, rope] (any row stride) rotated -> [T, H, v]."""
+    """Causal attention of whole sequences over expanded latents: q [T, H, nope + rope] (any row stride), the first rot_dims features
+    of its rope part unrotated; kv [T, H, nope + v]; k_rope [T, rope] (any row stride) rotated -> [T, H, v]."""
     _gpu(q, kv, k_rope, seg_start, seg_len, positions, inv_freq)
     T, H, d = q.shape
     rope = k_rope.shape[1]
@@ -1303,11 +1324,11 @@ def latent_prefill_attention(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Te
     assert q.stride(2) == 1 and q.stride(1) == d and kv.stride(2) == 1 and kv.stride(1) == nope + v and k_rope.stride(1) == 1
     assert kv.shape[:2] == (T, H) and k_rope.shape[0] == T and positions.numel() == T
     assert q.dtype == kv.dtype == k_rope.dtype and seg_start.dtype == seg_len.dtype == torch.int32 and positions.dtype == torch.int64
-    assert inv_freq.dtype == torch.float32 and 2 * inv_freq.numel() >= rot_dims
+    assert rot_dims == 0 or (inv_freq.dtype == torch.float32 and 2 * inv_freq.numel() >= rot_dims)
     out = torch.empty((T, H, v), dtype=q.dtype, device=q.device)
     check(_lib_().mi355_latent_prefill_attention(out.data_ptr(), q.data_ptr(), q.stride(0), kv.data_ptr(), kv.stride(0), k_rope.data_ptr(),
                                                  k_rope.stride(0), seg_start.data_ptr(), seg_len.data_ptr(), positions.data_ptr(),
-                                                 inv_freq.data_ptr(), rot_dims, int(bool(interleaved)), float(rot_mag), seg_len.numel(),
+                                                 _p(inv_freq), rot_dims, int(bool(interleaved)), float(rot_mag), seg_len.numel(),
                                                  int(max_len), H, nope, rope, v, float(scale), _dt(q), _stream(q)), "latent_prefill_attention")
     return out
 

@@ -662,10 +662,13 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
 
   // tile staging: thread -> rows (threadIdx.x >> 4) + 16 i, 16-B chunk (threadIdx.x & 15)
   const int srow = threadIdx.x >> 4, sch = threadIdx.x & 15;
-  Vec<T, 8> kreg[4], vreg[4], kreg2[WIDE ? 4 : 1];   // kreg2: features 128 + 8 sch .. + 7 (threads with sch < 8)
+  Vec<T, 8> kreg[4], vreg[4], kreg2[WIDE ? 2 : 1];
+  const int srow2 = threadIdx.x >> 3, sch2 = threadIdx.x & 7;   // kreg2: rows srow2 + 32 i, features 128 + 8 sch2 .. + 7
   const T* k_lin = k_ext + (int64_t)(q_start - prefix + srow) * p.k_stride + (int64_t)kvh * (LATENT ? p.kv_head : DQ) + sch * 8;
   const T* v_lin = v_ext + (int64_t)(q_start - prefix + srow) * p.v_stride + (int64_t)kvh * (LATENT ? p.kv_head : D) + sch * 8;
-  const T* r_lin = LATENT ? (const T*)p.k_rope + (int64_t)(q_start + srow) * p.k_rope_stride + sch * 8 : nullptr;
+  const T* r_lin = LATENT ? (const T*)p.k_rope + (int64_t)(q_start + srow2) * p.k_rope_stride + sch2 * 8
+                          : k_ext + (int64_t)(q_start - prefix + srow2) * p.k_stride + (int64_t)kvh * DQ + 128 + sch2 * 8;
+  const int64_t r_stride = LATENT ? p.k_rope_stride : p.k_stride;
   auto load_tile = [&](int kt) {
     if (kt * 64 >= prefix && kt * 64 + 63 < total) {   // whole tile in the extend part (workgroup-uniform)
 #pragma unroll
@@ -673,9 +676,10 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
         const int64_t key = kt * 64 + 16 * i;
         kreg[i] = ldvec<T, 8>(k_lin + key * p.k_stride);
         vreg[i] = ldvec<T, 8>(v_lin + key * p.v_stride);
-        if constexpr (WIDE) {
-          if (sch < 8) kreg2[i] = LATENT ? ldvec<T, 8>(r_lin + key * p.k_rope_stride) : ldvec<T, 8>(k_lin + key * p.k_stride + 128);
-        }
+      }
+      if constexpr (WIDE) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) kreg2[i] = ldvec<T, 8>(r_lin + (int64_t)(kt * 64 + 32 * i) * r_stride);
       }
       return;
     }
@@ -685,8 +689,9 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
         const int64_t key = min(kt * 64 + srow + 16 * i, total - 1) - srow;
         kreg[i] = ldvec<T, 8>(k_lin + key * p.k_stride);
         vreg[i] = ldvec<T, 8>(v_lin + key * p.v_stride);
-        if (sch < 8) kreg2[i] = ldvec<T, 8>(r_lin + key * p.k_rope_stride);
       }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) kreg2[i] = ldvec<T, 8>(r_lin + (int64_t)(min(kt * 64 + srow2 + 32 * i, total - 1) - srow2) * r_stride);
       return;
     }
 #pragma unroll
@@ -713,8 +718,14 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
       }
       kreg[i] = ldvec<T, 8>(kp + sch * 8);
       vreg[i] = ldvec<T, 8>(vp + sch * 8);
-      if constexpr (WIDE) {
-        if (sch < 8) kreg2[i] = ldvec<T, 8>(kp + 128 + sch * 8);
+    }
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int key = min(kt * 64 + srow2 + 32 * i, total - 1);
+        const T* kp = key < prefix ? kbuf + p.kv_indices[kv_start + key] * p.kb_slot + kvh * p.kb_head
+                                   : k_ext + (int64_t)(q_start + key - prefix) * p.k_stride + (int64_t)kvh * DQ;
+        kreg2[i] = ldvec<T, 8>(kp + 128 + sch2 * 8);
       }
     }
   };
@@ -724,9 +735,10 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
       const int off = xor_image_off(srow + 16 * i, sch);
       *reinterpret_cast<Vec<T, 8>*>(ks + off) = kreg[i];
       *reinterpret_cast<Vec<T, 8>*>(vs + off) = vreg[i];
-      if constexpr (WIDE) {
-        if (sch < 8) *reinterpret_cast<Vec<T, 8>*>(ks2 + off) = kreg2[i];
-      }
+    }
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<Vec<T, 8>*>(ks2 + xor_image_off(srow2 + 32 * i, sch2)) = kreg2[i];
     }
   };
 
@@ -878,9 +890,10 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   }
 }
 
-// Two workgroups per CU (256 registers per lane) at head dimension 128; the 192-wide variant needs ~280 registers and
-// runs one workgroup per CU instead of spilling (measured at 4 x 4096 tokens x 16 heads: 470 TFLOP/s against 412 with
-// 24 spilled registers at two workgroups per CU; issuing the next tile's loads behind the score phase spills more).
+// Two workgroups per CU (256 registers per lane) at head dimension 128; the 192-wide variant over a paged prefix needs
+// ~270 registers and runs one workgroup per CU instead of spilling (measured at 4 x 4096 tokens x 16 heads: 470 TFLOP/s
+// against 412 with 24 spilled registers at two workgroups per CU; issuing the next tile's loads behind the score phase
+// spills more).
 template <typename T, bool KV8 = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_mfma32_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
@@ -896,9 +909,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 // Whole prompts over a latent cache (rank 512 + 64) in expanded form: per visible pair and head 2 (128 + 64 + 128) flops
 // instead of the absorbed form's 2 (512 + 64 + 512), for one projection of every latent to its heads' keys and values (4 x 1900
-// tokens x 16 heads: 230 us, and about 70 for that projection; the absorbed launch with its two per-head products took 1570 us).
+// tokens x 16 heads: 154 us, and about 70 for that projection; the absorbed launch with its two per-head products took 1570 us).
+// Without a prefix to address, and with the rope part's rows dealt to all threads (two pieces each instead of four to half of
+// them), the body fits 256 registers: two workgroups per CU, one's softmax beside the other's MFMAs.  At one per CU: 226 us; 32
+// heads 404 -> 238.
 template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void extend_attn_latent_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_latent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o, ExtendParams p, int nqb, int npairs) {
   extend_attn_mfma32_body<T, false, 192, true>(q, k, v, o, nullptr, nullptr, p, nqb, npairs);
 }

@@ -211,12 +211,27 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const int g = wave >> 2, wc = wave & 3;
 
   // ---- workgroup -> output tile ------------------------------------------------------------
+  // Consecutive workgroups go to the eight XCDs in turn.  EPI 3, whose tile count only the device knows: blocks of 8 x 4 tiles
+  // in turn.  Otherwise every XCD gets an equal run of the tiles in block order (bands of 8 rows, blocks of 4 columns inside):
+  // whole blocks in turn left some XCDs a round more than others where the last band is short -- 18 x 24 tiles: 72 on two
+  // XCDs and 40 on four, of 32 CUs each.  M = 4605, K = 4096: N = 6144 267 -> 190 us, N = 28672 846 -> 792; 7381 x 2048 -> 2 x 5632 302 -> 280.
   const int b = blockIdx.x, li = b >> 3;
-  const int st = (li >> 5) * 8 + (b & 7), within = li & 31;
-  if (st >= p.nsuper) return;
-  const int sup_m = st / p.snt, sup_n = st - sup_m * p.snt;
-  const int tm = sup_m * 8 + (within & 7), tn = sup_n * 4 + (within >> 3);
-  if (tm >= p.mt || tn >= p.nt) return;
+  int tm, tn;
+  if constexpr (EPI == 3) {
+    const int st = (li >> 5) * 8 + (b & 7), within = li & 31;
+    if (st >= p.nsuper) return;
+    const int sup_m = st / p.snt, sup_n = st - sup_m * p.snt;
+    tm = sup_m * 8 + (within & 7);
+    tn = sup_n * 4 + (within >> 3);
+    if (tm >= p.mt || tn >= p.nt) return;
+  } else {
+    const int at = (b & 7) * (int)(gridDim.x >> 3) + li;
+    if (at >= p.mt * p.nt) return;
+    const int band = at / (8 * p.nt), in = at - band * 8 * p.nt;
+    const int rows = min(8, p.mt - 8 * band), col = in / (4 * rows), r = in - col * 4 * rows;
+    tm = band * 8 + r % rows;
+    tn = col * 4 + r / rows;
+  }
   // EPI 3: rows of the tile that are no padding (they lie in front of it).  Padding rows are neither loaded, multiplied nor
   // stored, 8, 16 and 1 at a time: an expert's last tile is as long as its rows.  64 tokens x 4 of 32 experts (2048 x 2048):
   // 88 us with padding worked on, 55 without (268 MB of weights); 1024 tokens: 85 and 72; 3000 tokens: 148 and 145.
@@ -470,8 +485,9 @@ template <typename T, int EPI, bool FP8>
 int launch_gemm_tiled(const GemmTiledParams& p, hipStream_t st) {
   auto kern = gemm_tiled_kernel<T, EPI, FP8>;
   (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS);
-  const int groups = (p.nsuper + 7) / 8;   // every XCD label gets the same number of 8 x 4 blocks
-  hipLaunchKernelGGL(kern, dim3((unsigned)(groups * 8 * 32)), dim3(512), GT_LDS, st, p);
+  // 8 x 4 blocks, or tiles, in equal numbers for every XCD
+  const int per = EPI == 3 ? (p.nsuper + 7) / 8 * 32 : (int)cdiv((int64_t)p.mt * p.nt, 8);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(per * 8)), dim3(512), GT_LDS, st, p);
   MI355_CHECK_LAUNCH(EPI == 3 ? "mi355_moe_grouped_linear_tiled" : EPI == 2 ? "mi355_qkv_proj_rope_tiled"
                      : FP8 ? "mi355_fp8_scaled_mm_tiled" : "mi355_linear_tiled");
   return MI355_OK;

@@ -329,10 +329,11 @@ class Mi355AttnBackend(AttentionBackend):
 
     def latent_prefill_ok(self, layer, forward_batch, nope: int, v: int, dtype) -> bool:
         """Whether forward_latent_prefill serves the step: whole prompts (nothing cached), every earlier token, a plain softmax,
-        more tokens than the decode-sized kernels take."""
+        more tokens than the decode-sized kernels take.  The queries and the cache rows are read where they lie, in rows that
+        hold the latent too: its rank decides whether those start at 16-byte boundaries."""
         return (not forward_batch.forward_mode.is_decode_or_idle() and forward_batch.extend_prefix_lens_cpu is not None
                 and not any(forward_batch.extend_prefix_lens_cpu) and layer.window == 0 and layer.sink is None
-                and forward_batch.extend_num_tokens > SKINNY_MAX_M and str(self.device).startswith("cuda")
+                and forward_batch.extend_num_tokens > SKINNY_MAX_M and layer.kv_rank % 8 == 0 and str(self.device).startswith("cuda")
                 and get_ops().latent_prefill_attention_supported(nope, layer.rope_dim, v, layer.rot_dims, layer.interleaved, dtype))
 
     def forward_latent_prefill(self, q, expand, layer, forward_batch, cache_layer=None):

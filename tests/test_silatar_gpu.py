@@ -179,6 +179,18 @@ def test_long_decode(dtype, tol):
         assert su.pools_are_whole(mr)
 
 
+@pytest.mark.parametrize("rank", [35, 36, 40])
+def test_whole_prompts_over_any_latent_rank(rank):
+    """Heads of 128 + 64 key and 128 value features, which whole prompts attend over in expanded form where the rows that hold
+    the latent start at 16-byte boundaries (rank 40) and in absorbed form where they do not."""
+    cfg = su.make_config(layers=[(su.latent(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=rank, scale=0.1), su.dense(64))], loop=(0, 1, 1))
+    w = su.make_weights(cfg, seed=6)
+    prompts = su.random_prompts(cfg, [130, 1, 70], seed=2)
+    mr = su.build_runner(cfg, w, dtype="bfloat16", device=DEV)
+    su.replay_and_compare(mr, cfg, w, prompts, [[("r0", 130), ("r1", 1), ("r2", 70)]], 6e-2)
+    assert su.pools_are_whole(mr)
+
+
 @pytest.mark.parametrize("dtype,tol", CASES)
 def test_sizes_that_are_multiples_of_nothing(dtype, tol):
     """Width 100, vocabulary 77, heads of 21 / 13 / 37, ranks of 29 and 51, odd feed-forward widths, pages of 5: no 16-byte row

@@ -175,7 +175,8 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_temperature_kernel(
 }
 
 // The same over chunks of a row, in two launches: every chunk leaves its maximum and its sum of exponentials, then
-// every chunk normalises itself with what all of them left.  One workgroup per row reads its 0.5 MB three times with 4
+// every chunk normalises itself with what all of them left.  (A chunk without a number in it has no maximum to take off: its
+// -inf entries count zero and a NaN makes its sum NaN, and with it the row, as one pass over the row has it.)  One workgroup per row reads its 0.5 MB three times with 4
 // bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
 // 18 + 16 us (33 MB read twice, the second time from L2, then read and written), bound by the precise division and
 // exponential of every entry in both.
@@ -251,16 +252,18 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
         mx = fmaxf(mx, v[u].v[j]);   // (a piece past the end repeats the last one: the maximum does not mind)
       }
     mx = block_reduce_max(fmaxf(mx, last), red);
+    const float ref = mx == -INFINITY ? 0.f : mx;
 #pragma unroll
     for (int u = 0; u < KEEP; ++u)
       if (sp.v0 + threadIdx.x + u * SAMP_THREADS < sp.v1)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sum += expf(v[u].v[j] - mx);
-    if (one) sum += expf(last - mx);
+        for (int j = 0; j < 4; ++j) sum += expf(v[u].v[j] - ref);
+    if (one) sum += expf(last - ref);
   } else {
     span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, x / t); });
     mx = block_reduce_max(mx, red);
-    span_each(row, vocab, sp, vec, [&](float x) { sum += expf(x / t - mx); });
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    span_each(row, vocab, sp, vec, [&](float x) { sum += expf(x / t - ref); });
   }
   sum = block_sum(sum, red);
   if (threadIdx.x == 0) partials[(int64_t)r * chunks + c] = float2{mx, sum};
@@ -277,8 +280,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_normalise_kernel(
   for (int i = 0; i < chunks; ++i) mx = fmaxf(mx, partials[(int64_t)r * chunks + i].x);
   for (int i = 0; i < chunks; ++i) {
     const float2 p = partials[(int64_t)r * chunks + i];
-    // a chunk of nothing but -inf has no exponentials of its own (its sum is NaN) unless the whole row is like that
-    if (p.x != -INFINITY || mx == -INFINITY) sum += p.y * expf(p.x - mx);
+    sum += p.y * expf(p.x - mx);
   }
   const ChunkSpan sp = chunk_span(vocab, c, chunks);
   for (int64_t i = sp.v0 + threadIdx.x; i < sp.v1; i += SAMP_THREADS) {

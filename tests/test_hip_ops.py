@@ -1286,3 +1286,27 @@ def test_chunked_softmax_and_sampler_edges(ops, rows, vocab, pad):
                 if ok.all():
                     break
             assert ok.all(), (kind, k, tp, mp, ids[~ok][:4].tolist())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,vocab", [(2, 32768), (3, 128259), (90, 24576), (130, 131072)])
+def test_chunked_softmax_keeps_nan(ops, rows, vocab):
+    """A chunk without a number in it -- NaN and -inf entries alone -- beside chunks of numbers: one NaN makes the row NaN, -inf
+    entries alone are zeros.  (130 rows of 131072 are chunks of more than a workgroup holds in registers.)  Finite rows against
+    float64 with the bound of the test above."""
+    g = torch.Generator().manual_seed(rows + vocab)
+    x = torch.randn((rows, vocab), generator=g)
+    lo, hi = vocab // 2, vocab - vocab % 4     # the second half: whole chunks at 2, 4, 8 or 16 of them
+    x[0, lo + 4: hi] = float("-inf")
+    x[0, lo: lo + 4] = 0.5
+    x[-1, lo: hi] = float("nan")
+    x[-1, lo + 5] = float("-inf")
+    got = x.to(DEV)
+    ops.softmax_temperature_(got, torch.ones(rows, device=DEV))
+    ref = torch.softmax(x.double(), -1)
+    assert got[-1].isnan().all() and ref[-1].isnan().all()
+    assert (got[:-1].cpu().double() - ref[:-1]).norm() <= 2e-6 * ref[:-1].norm()
+    x[-1, lo: vocab] = float("-inf")
+    got = x.to(DEV)
+    ops.softmax_temperature_(got, torch.ones(rows, device=DEV))
+    assert (got[-1].cpu().double() - torch.softmax(x[-1].double(), -1)).norm() <= 2e-6 * torch.softmax(x[-1].double(), -1).norm()

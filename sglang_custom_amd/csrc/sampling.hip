@@ -648,7 +648,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
     }
     few = cut.count + size <= (unsigned)SB_SHORT;
     // the cut bin's entries; with the larger ones and everybody's index if they are few
-    const unsigned lowest = (unsigned)cut.bin << SB_SHIFT, bound = few ? 0x7f800000u : lowest + (1u << SB_SHIFT);
+    const unsigned lowest = (unsigned)cut.bin << SB_SHIFT, bound = few ? 0x7f800001u : lowest + (1u << SB_SHIFT);   // (few: up to infinity, which the bins have counted)
     constexpr int U = 8;
     const int64_t groups = (vocab + 3) / 4;
     for (int64_t i0 = threadIdx.x; i0 < groups; i0 += U * SAMP_THREADS) {

@@ -1310,3 +1310,28 @@ def test_chunked_softmax_keeps_nan(ops, rows, vocab):
     got = x.to(DEV)
     ops.softmax_temperature_(got, torch.ones(rows, device=DEV))
     assert (got[-1].cpu().double() - torch.softmax(x[-1].double(), -1)).norm() <= 2e-6 * torch.softmax(x[-1].double(), -1).norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab", [4096, 40000])
+def test_sampler_over_chunks_with_infinite_entries(ops, vocab):
+    """Unnormalised weights with infinities among them: the same pick as the launch that takes a whole row at once (the last kept
+    entry, as no running sum passes an infinite total), whatever the draw before it left in LDS."""
+    g = torch.Generator().manual_seed(vocab)
+    rows = 8
+    busy = torch.softmax(2.5 * torch.randn((rows, vocab), generator=g), -1).to(DEV)
+    p = torch.rand((rows, vocab), generator=g) * 1e-3
+    p[:, 100] = 0.5
+    p[:, 7] = float("inf")
+    p[1::2, vocab - 2] = float("inf")
+    p[2::4, 200] = 0.25
+    p = p.to(DEV)
+    lib = ops._lib_()
+    for k in (2, 3, 5):
+        ks, u = torch.full((rows,), k, dtype=torch.int32, device=DEV), torch.rand((rows,), generator=g).to(DEV)
+        want = torch.empty(rows, dtype=torch.int32, device=DEV)
+        assert lib.mi355_top_k_top_p_min_p_sample(want.data_ptr(), p.data_ptr(), ks.data_ptr(), None, None, u.data_ptr(), rows, vocab, vocab, None) == 0
+        ops.top_k_top_p_min_p_sample(busy, ks, None, None, u)
+        got = ops.top_k_top_p_min_p_sample(p, ks, None, None, u)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), k

@@ -473,8 +473,9 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
 // kept whole holds tau; its entries -- hundreds where a vocabulary's probabilities spread over binades -- are collected in
 // LDS by one pass over the row and searched there bit by bit.  If they and the larger ones are few (a small top_k), all of
 // them are collected with their indices and the draw is made among them; otherwise a second pass sums what is kept per
-// tile of 256 entries, and the tile the draw falls into is walked.  A row whose tau lies above 1.9 (no probability does),
-// or with more entries in that bin than the list holds (an almost flat row), takes sample_whole_row.
+// tile of 256 entries, and the tile the draw falls into is walked.  More entries in that bin than the list holds (an
+// almost flat row) are searched in the row itself, a pass per step.  A row whose tau lies above 1.9 (no probability does) takes
+// sample_whole_row.
 // The one-workgroup routine meets each of its four levels' 128256 entries in 256 bins of two binades, a handful of which
 // take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics; this
 // takes 10 + 28 us (58 when thousands are kept), the first bound by its LDS atomics too, the second by one CU's pass over 0.5 MB.
@@ -483,9 +484,10 @@ constexpr int SB_SUM_BITS = 40;
 constexpr int64_t SB_MAX_VOCAB = (int64_t)SB_TILE * SB_MAX_TILES;   // 2^20: counts fit 24 bits, sums of 19 bits fit 40
 typedef unsigned long long u64_t;
 
-__device__ __forceinline__ float bin_mass(int bin, u64_t x) {
-  const unsigned e = (unsigned)bin >> 4;                                          // exponent field
-  const double base = (double)((((unsigned)bin & 15u) << SB_SHIFT) + (e ? 1u << 23 : 0u));   // an entry's mantissa without its lower bits
+// The mass of x = (entries << SB_SUM_BITS) + the sum of their lower bits, where `bits` is the pattern they share above those.
+__device__ __forceinline__ float bin_mass(unsigned bits, u64_t x) {
+  const unsigned e = bits >> 23;                                                        // exponent field
+  const double base = (double)((bits & ((1u << 23) - 1)) + (e ? 1u << 23 : 0u));        // an entry's mantissa without its lower bits
   return (float)ldexp((double)(x >> SB_SUM_BITS) * base + (double)(x & (((u64_t)1 << SB_SUM_BITS) - 1)), (int)(e ? e : 1u) - 150);
 }
 
@@ -608,6 +610,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
   __shared__ float hmass[SB_BINS];
   __shared__ union {
     unsigned list[SB_LIST];        // the cut bin's entries, until tau is known
+    u64_t cells[1024];             // or, if they are too many, their parts' counts and sums
     float tile[SB_MAX_TILES];      // kept mass per tile of 256 entries, afterwards
     SampleScratch whole;
   } sm;
@@ -626,7 +629,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
     u64_t x = 0;
     for (int c = 0; c < chunks; ++c) x += rb[(int64_t)c * SB_BINS + i];
     hcount[i] = (unsigned)(x >> SB_SUM_BITS);
-    hmass[i] = bin_mass(i, x);
+    hmass[i] = bin_mass((unsigned)i << SB_SHIFT, x);
   }
   if (threadIdx.x == 0) {
     n_list = 0;
@@ -639,7 +642,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
   bool few = false;
   if (cut.bin >= 0) {
     unsigned size = hcount[cut.bin];
-    if (cut.bin == SB_BINS - 1 || size > (unsigned)SB_LIST) {
+    if (cut.bin == SB_BINS - 1) {
       __syncthreads();
       sample_whole_row(ids, sr, vocab, sm.whole.hcount, sm.whole.hmass, sm.whole.scan, sm.whole.red);
       return;
@@ -647,28 +650,34 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
     few = cut.count + size <= (unsigned)SB_SHORT;
     // the cut bin's entries; with the larger ones and everybody's index if they are few
     const unsigned lowest = (unsigned)cut.bin << SB_SHIFT, bound = few ? 0x7f800001u : lowest + (1u << SB_SHIFT);   // (few: up to infinity, which the bins have counted)
-    constexpr int U = 8;
-    const int64_t groups = (vocab + 3) / 4;
-    for (int64_t i0 = threadIdx.x; i0 < groups; i0 += U * SAMP_THREADS) {
-      Vec<float, 4> v[U];
+    const bool listed = few || size <= (unsigned)SB_LIST;
+    // f(bits, index) of every entry of the row in [lo, hi) patterns
+    auto row_each = [&](unsigned lo, unsigned hi, auto&& f) {
+      constexpr int U = 8;
+      const int64_t groups = (vocab + 3) / 4;
+      for (int64_t i0 = threadIdx.x; i0 < groups; i0 += U * SAMP_THREADS) {
+        Vec<float, 4> v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + u * SAMP_THREADS;
-        if (i < groups) v[u] = row4(row, vocab, i, vec);
-        else v[u] = Vec<float, 4>{{0.f, 0.f, 0.f, 0.f}};
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const unsigned bits = __float_as_uint(v[u].v[j]);
-          if (v[u].v[j] > 0.f && bits >= lowest && bits < bound) {
-            const unsigned at = atomicAdd(&n_list, 1u);
-            if (at < (unsigned)SB_LIST) sm.list[at] = bits;
-            if (few && at < (unsigned)SB_SHORT) sm.list[SB_SHORT + at] = (unsigned)((i0 + u * SAMP_THREADS) * 4 + j);
-          }
+        for (int u = 0; u < U; ++u) {
+          const int64_t i = i0 + u * SAMP_THREADS;
+          if (i < groups) v[u] = row4(row, vocab, i, vec);
+          else v[u] = Vec<float, 4>{{0.f, 0.f, 0.f, 0.f}};
         }
-    }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const unsigned bits = __float_as_uint(v[u].v[j]);
+            if (v[u].v[j] > 0.f && bits >= lo && bits < hi) f(bits, (unsigned)((i0 + u * SAMP_THREADS) * 4 + j));
+          }
+      }
+    };
+    if (listed)
+      row_each(lowest, bound, [&](unsigned bits, unsigned index) {
+        const unsigned at = atomicAdd(&n_list, 1u);
+        if (at < (unsigned)SB_LIST) sm.list[at] = bits;
+        if (few && at < (unsigned)SB_SHORT) sm.list[SB_SHORT + at] = index;
+      });
     if (few) size += cut.count;
     // its 19 lower bits, ten and then nine of them
     unsigned prefix = (unsigned)cut.bin;
@@ -677,19 +686,32 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
 #pragma unroll
     for (int level = 0; level < 2; ++level) {
       const int nb = level == 0 ? 1024 : 512, shift = shifts[level];
+      const unsigned want = prefix << (level == 0 ? SB_SHIFT : 9);
       __syncthreads();
       for (int i = threadIdx.x; i < 1024; i += SAMP_THREADS) {
         hcount[i] = 0;
         hmass[i] = 0.f;
+        if (!listed) sm.cells[i] = 0;
       }
       __syncthreads();
-      const unsigned want = prefix << (level == 0 ? SB_SHIFT : 9);
-      for (unsigned i = threadIdx.x; i < size; i += SAMP_THREADS) {
-        const unsigned bits = sm.list[i];
-        if ((bits & himask) == want) {
-          const unsigned b = (bits >> shift) & (unsigned)(nb - 1);
-          atomicAdd(&hcount[b], 1u);
-          unsafeAtomicAdd(&hmass[b], __uint_as_float(bits));
+      if (listed) {
+        for (unsigned i = threadIdx.x; i < size; i += SAMP_THREADS) {
+          const unsigned bits = sm.list[i];
+          if ((bits & himask) == want) {
+            const unsigned b = (bits >> shift) & (unsigned)(nb - 1);
+            atomicAdd(&hcount[b], 1u);
+            unsafeAtomicAdd(&hmass[b], __uint_as_float(bits));
+          }
+        }
+      } else {
+        row_each(want, want - himask, [&](unsigned bits, unsigned) {
+          atomicAdd(&sm.cells[(bits >> shift) & (unsigned)(nb - 1)], ((u64_t)1 << SB_SUM_BITS) + (bits & ((1u << shift) - 1)));
+        });
+        __syncthreads();
+        if ((int)threadIdx.x < nb) {
+          const u64_t x = sm.cells[threadIdx.x];
+          hcount[threadIdx.x] = (unsigned)(x >> SB_SUM_BITS);
+          hmass[threadIdx.x] = bin_mass(want + (threadIdx.x << shift), x);
         }
       }
       const BinCut next = cut_bins<1024>(hcount, hmass, sr.k, sr.top_p, cut.count, cut.mass, cs);

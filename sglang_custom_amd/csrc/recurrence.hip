@@ -147,8 +147,11 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
 // 1400 (delta) cycles a token, on one wave per SIMD: 4 x 1900 tokens, 16 heads of 64 x 128 took 800 and 1105 us; this takes
 // 214 and 342 (161 and 265 with every product in fp32, whose errors were 1.4 and 1.7 times the token by token form's at
 // strong decays; now they are 0.6 to 1.0 times), bound by the matrix instructions' issue and five to eight barriers a chunk.
-// What a later token of a chunk holds is multiplied by zero for an earlier one: an infinite or NaN input reaches the outputs of
-// its own sequence's chunk, not only those behind it.
+// What a later token of a chunk holds is multiplied by zero for an earlier one, which an infinity or a NaN survives.  They stay in
+// the state, to the end: a sequence that ends with one in its state is done again token by token, so that non-finite
+// inputs reach their own token's outputs and later ones only.  (The second run's code costs the delta rule's chunks 3 % through
+// the compiler's schedule, 4 x 1000 tokens 178 -> 184 us; told that two waves a SIMD are all there will be, it costs the plain
+// ones nothing.)
 constexpr int CK = 64;               // tokens of a chunk, and key channels (padded)
 constexpr int CLD = CK + 4;          // LDS row: the 16 rows of a 16-byte fragment read fall into different banks
 constexpr int CK_THREADS = 512;
@@ -214,8 +217,55 @@ struct ChunkArgs {
   float q_scale;
 };
 
+// A workgroup's sequence, head and columns token by token, 16 lanes a column, four channels each: for the rare sequences that the
+// chunks do not serve.
+typedef const ChunkArgs __attribute__((address_space(4))) ChunkArgsInMemory;
 template <typename QT, typename VT, bool DELTA>
-__global__ __launch_bounds__(CK_THREADS) void chunk_recurrence_kernel(ChunkArgs p) {
+__device__ __forceinline__ void token_recurrence(ChunkArgsInMemory& p) {
+  const int b = blockIdx.z, h = blockIdx.y, c = threadIdx.x >> 4, d0 = 4 * (threadIdx.x & 15), col = blockIdx.x * RC_COLS + c;
+  const int hq = h / (p.heads / p.qk_heads);
+  const int64_t t0 = p.seg_start[b], t1 = t0 + p.seg_len[b], slot = p.req_to_state[p.req_pool_indices[b]];
+  float* const sp = p.state + ((slot * p.heads + h) * (int64_t)p.dk + d0) * p.dv + col;
+  const float rate = expf(p.rate_log[h]), bias = p.bias[h], skip = !DELTA && p.skip != nullptr ? p.skip[h] : 0.f;
+  const bool fresh = p.positions[t0] == 0, in_v = col < p.dv;
+  float S[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) S[r] = !fresh && d0 + r < p.dk && in_v ? sp[(int64_t)r * p.dv] : 0.f;
+  for (int64_t t = t0; t < t1; ++t) {
+    const float v = in_v ? to_f32(((const VT*)p.v)[t * p.v_stride + (int64_t)h * p.dv + col]) : 0.f;
+    const float dt = softplus_f(p.logits[t * p.logit_stride + h] + bias), decay = expf(-rate * dt);
+    float k[4], y = 0.f, u = dt * v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      k[r] = d0 + r < p.dk ? to_f32(((const QT*)p.k)[t * p.k_stride + (int64_t)hq * p.dk + d0 + r]) : 0.f;
+      S[r] *= decay;
+      y = fmaf(k[r], S[r], y);
+    }
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o, 64);
+      const float z = p.beta_f32 ? static_cast<const float*>(p.beta_logits)[t * p.beta_stride + h]
+                                 : to_f32(static_cast<const VT*>(p.beta_logits)[t * p.beta_stride + h]);
+      u = (v - y) / (1.0f + expf(-z));
+    }
+    y = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (d0 + r < p.dk) {
+        S[r] = fmaf(k[r], u, S[r]);
+        y = fmaf(to_f32(((const QT*)p.q)[t * p.q_stride + (int64_t)hq * p.dk + d0 + r]) * p.q_scale, S[r], y);
+      }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o, 64);
+    if (d0 == 0 && in_v) p.out[(t * p.heads + h) * (int64_t)p.dv + col] = DELTA ? y : fmaf(skip, v, y);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (d0 + r < p.dk && in_v) sp[(int64_t)r * p.dv] = S[r];
+}
+
+template <typename QT, typename VT, bool DELTA>
+__global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_recurrence_kernel(ChunkArgs p) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float* const Q = lds;                       // [t][d]
   float* const K = Q + CK * CLD;              // [t][d]
@@ -230,6 +280,7 @@ __global__ __launch_bounds__(CK_THREADS) void chunk_recurrence_kernel(ChunkArgs 
   float* const W = WS + CK;                   // [s] w_s (plain) or beta_t (delta)
   float* const A = W + CK;                    // delta: [t][s] strictly lower part of the system
   float* const INV = A + CK * CLD;            // delta: [4][16][20] inverses of its diagonal blocks
+  __shared__ int not_finite;
   const int b = blockIdx.z, h = blockIdx.y, c0 = blockIdx.x * RC_COLS;
   const int hq = h / (p.heads / p.qk_heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
@@ -250,6 +301,7 @@ __global__ __launch_bounds__(CK_THREADS) void chunk_recurrence_kernel(ChunkArgs 
     const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
     ST[c * CLD + i] = (!fresh && i < p.dk && c0 + c < p.dv) ? sp[(int64_t)i * p.dv + c0 + c] : 0.f;
   }
+  if (tid == 0) not_finite = 0;
   // this wave's tile of the state: d = 16 (wave >> 1) + 4 lg + r, column 16 (wave & 1) + li
   const int sd = (wave >> 1) * 16, sc = (wave & 1) * 16;
 
@@ -432,11 +484,29 @@ __global__ __launch_bounds__(CK_THREADS) void chunk_recurrence_kernel(ChunkArgs 
     *reinterpret_cast<f32x4*>(ST + (sc + li) * CLD + sd + 4 * lg) = S;
   }
   __syncthreads();
+  float last[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
-    if (i < p.dk && c0 + c < p.dv) sp[(int64_t)i * p.dv + c0 + c] = ST[c * CLD + i];
+    last[u] = ST[c * CLD + i];
+    if (!isfinite(last[u])) not_finite = 1;
   }
+  __syncthreads();
+  if (!not_finite) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
+      if (i < p.dk && c0 + c < p.dv) sp[(int64_t)i * p.dv + c0 + c] = last[u];
+    }
+    return;
+  }
+  // (this workgroup's part of the state in memory is still the one that it began with.  The arguments are read afresh: kept in
+  // registers through the chunks they would make those slower)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every output above is written before the ones of the second run
+  __syncthreads();
+  ChunkArgsInMemory* args = (ChunkArgsInMemory*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm("" : "+s"(args));
+  token_recurrence<QT, VT, DELTA>(*args);
 }
 
 // Which launches take the chunks: one decay per head and token, at most 64 key channels (what the LDS tiles hold), and a step

@@ -100,3 +100,41 @@ def test_total_forgetting_stays_finite(delta):
     else:
         ops.linear_recurrence(q, k, d["v"], out, d["state"], *args, dt_logits=d["z"], dt_bias=d["bias"], rate_log=d["rate"], skip=d["skip"], **seg)
     assert (out.cpu().double() - want).norm() <= 1e-5 * want.norm()
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("what", ["v", "k", "q", "z", "beta", "state"])
+def test_non_finite_inputs_reach_no_earlier_token(what, delta):
+    """An infinity or a NaN in the middle of a chunk, and the tokens behind it: finite outputs are where the token-by-token form
+    has them, and right there (the bound of the tests above)."""
+    from sglang_custom_amd import ops
+
+    if what == "beta" and not delta:
+        pytest.skip("the plain form has no beta")
+    lens, H, G, dk, dv = (150, 130), 2, 1, 40, 33
+    c = _case(lens, H, G, dk, dv, torch.float32, torch.float32, 11, -1.0)
+    nan, inf = float("nan"), float("inf")
+    if what == "v":
+        c["v"][70, 1, 5], c["v"][150 + 127, 0, 32] = inf, nan
+    elif what in ("k", "q"):
+        c[what][21, 7], c[what][150 + 64, 39] = nan, inf
+    elif what in ("z", "beta"):
+        c[what][100, 0], c[what][150 + 3, 1] = nan, nan
+    else:
+        c["state"][c["slots"][1], 0, 3, 4], c["state"][c["slots"][1], 1, 39, 32] = nan, inf
+    want, states = _exact(c, lens, H, G, dk, dv, delta, 0.25)
+    d = {n: t.to(DEV) for n, t in c.items()}
+    T, B = sum(lens), len(lens)
+    out = torch.empty((T, H, dv), device=DEV)
+    seg = dict(tok_req=torch.repeat_interleave(torch.arange(B, dtype=torch.int32), torch.tensor(lens)).to(DEV), seg_start=d["start"],
+               seg_len=torch.tensor(lens, dtype=torch.int32, device=DEV))
+    args = (d["slots"].int(), torch.arange(B, device=DEV), d["pos"], 0.25)
+    q, k = d["q"][:, : G * dk].view(T, G, dk), d["k"].view(T, G, dk)
+    if delta:
+        ops.gated_delta_rule(q, k, d["v"], d["beta"], d["z"], d["bias"], d["rate"], out, d["state"], *args, **seg)
+    else:
+        ops.linear_recurrence(q, k, d["v"], out, d["state"], *args, dt_logits=d["z"], dt_bias=d["bias"], rate_log=d["rate"], skip=d["skip"], **seg)
+    for got, ref in ((out.cpu().double(), want), (d["state"].cpu().double()[c["slots"]], states)):
+        ok = ref.isfinite()
+        assert torch.equal(got.isfinite(), ok)
+        assert (got - ref)[ok].norm() <= 1e-5 * ref[ok].norm()

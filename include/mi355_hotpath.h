@@ -899,7 +899,11 @@ int mi355_window_attention(void* out, const void* q, const void* k_cache, const 
  *   a = exp(-exp(rate_log[h]) * dt) for every key channel, S = a S + dt k v^T, out = S^T (q * q_scale) + skip[h] v (skip null:
  *   none).  Exactly one of gate_logits, head_decay, dt_logits is given.
  * mi355_gated_delta_rule_ex: mi355_gated_delta_rule with gate_per_head (gate_logits [tokens][heads], rate_bias [heads]: one
- *   decay per head and token) and beta_f32 (beta_logits are fp32). */
+ *   decay per head and token) and beta_f32 (beta_logits are fp32).
+ * mi355_linear_recurrence_ssm_sized, mi355_gated_delta_rule_sized: the same for a caller that knows the step's tokens in all and its
+ *   longest segment (0, 0: it does not).  With one decay per head and token, segments and key_dim <= 64, a launch that
+ *   mi355_recurrence_takes_chunks says so for then takes 64 tokens at a time: other sums in the same precision, several times
+ *   faster on few long segments, slower on many short ones. */
 int mi355_rmsnorm_residual_add_scaled(float* x, void* h_out, const void* y, int64_t y_stride, const void* weight,
                                       const void* layer_scale, float offset, float mult, int64_t tokens, int64_t hidden, float eps,
                                       int dtype, void* stream);
@@ -937,6 +941,21 @@ int mi355_gated_delta_rule_ex(float* out, float* state, const void* q, const voi
                               int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
                               int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
                               void* stream);
+int mi355_linear_recurrence_ssm_sized(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
+                                const void* gate_bias, const float* head_decay, const float* dt_logits, int64_t dt_token_stride,
+                                const float* dt_bias, const float* rate_log, const float* skip, const int32_t* req_to_state,
+                                const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                                const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                                int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t gate_token_stride,
+                                float q_scale, float tau, int qk_dtype, int v_dtype, int64_t tokens, int64_t longest, void* stream);
+int mi355_gated_delta_rule_sized(float* out, float* state, const void* q, const void* k, const void* v, const void* beta_logits,
+                              const float* gate_logits, const float* rate_bias, const float* rate_log, const int32_t* req_to_state,
+                              const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                              const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                              int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
+                              int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
+                              int64_t tokens, int64_t longest, void* stream);
+int mi355_recurrence_takes_chunks(int delta, int64_t batch, int heads, int key_dim, int value_dim, int64_t tokens, int64_t longest);
 
 /* ---- window attention with averaged blocks before the window and a gate per head -------------------------
  * mi355_pool_kv_blocks: for every token t of the step whose position p ends a block of `pool` tokens ((p + 1) % pool == 0):

@@ -509,11 +509,29 @@ __global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
   token_recurrence<QT, VT, DELTA>(*args);
 }
 
-// Which launches take the chunks: one decay per head and token, at most 64 key channels (what the LDS tiles hold), and a step
-// whose sequences have segments, that is several tokens (a decode step is one token per sequence: the plain kernel's trip
-// through the matrix is all there is to it).
-inline bool chunks_serve(int dk, const int32_t* seg_len, const float* out, int dv) {
-  return dk <= CK && seg_len != nullptr && (dv % 4 != 0 || aligned16(out));
+// Which launches take the chunks: one decay per head and token, at most 64 key channels (what the LDS tiles hold), a step whose
+// sequences have segments, of known lengths (tokens in all, the longest one), and less time by the two forms' models, which fit what
+// was measured within 15 % (16 heads of 64 x 128, in us).  A token of the token-by-token form takes a chain of 0.40 (delta 0.55)
+// or, from some 1000 workgroups on, its share of the chip, 0.43 (0.60) per 1000 of them; a chunk takes its workgroup 6.7 (10.6), one
+// workgroup to a CU, and about 3 more before the first.  Measured, token by token / chunks:
+//   plain  1 x 16   9.8 / 10.4   1 x 64   27 / 11     8 x 65   32 / 35    16 x 64    42 / 42    64 x 4    27 / 149   64 x 500   813 / 905
+//   delta  1 x 16  12.4 / 14.9   1 x 64   38 / 16     8 x 65   43 / 51    16 x 64    54 / 58    64 x 4    27 / 213   64 x 500  1096 / 1409
+//   plain  4 x 2000   827 / 223   16 x 1000   464 / 440   16 x 2000   1010 / 865;   delta   1130 / 348   667 / 691   1369 / 1372
+inline bool chunks_pay(bool delta, int64_t batch, int heads, int dk, int dv, int64_t tokens, int64_t longest) {
+  if (dk > CK || tokens <= 0 || longest <= 0 || batch <= 0) return false;
+  const double blocks = (double)heads * cdiv(dv, RC_COLS);                  // workgroups of a sequence
+  const double narrow = dk <= 32 ? 0.8 : 1.0;                               // (a token's cost follows its channels, a chunk's does not)
+  const double chain = narrow * (delta ? 0.55 : 0.40), share = narrow * (delta ? 0.60e-3 : 0.43e-3), chunk = delta ? 10.6 : 6.7;
+  const double by_token = 5 + std::max(chain * longest, share * tokens * blocks);
+  const double most = (double)cdiv(longest, CK);
+  const double chunks = std::min(batch * most, tokens / (double)CK + batch);   // of one head's columns, over all sequences
+  const double rounds = std::ceil(batch * blocks / 256);
+  return 3 + std::max(chunk * most + 3, rounds * (chunk * chunks / batch + 3)) < 0.97 * by_token;
+}
+
+inline bool chunks_serve(bool delta, int64_t batch, int heads, int dk, int dv, int64_t tokens, int64_t longest, const int32_t* seg_len,
+                         const float* out) {
+  return seg_len != nullptr && (dv % 4 != 0 || aligned16(out)) && chunks_pay(delta, batch, heads, dk, dv, tokens, longest);
 }
 
 template <typename QT, typename VT, bool DELTA>
@@ -530,8 +548,9 @@ int launch_recurrence(float* out, float* state, const void* q, const void* k, co
                       const void* gate_bias, const float* head_decay, const int32_t* req_to_state, const int64_t* req_pool_indices,
                       const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions, int64_t batch, int heads, int dk,
                       int dv, int64_t qs, int64_t ks, int64_t vs, int64_t gs, float q_scale, float tau, int qk_heads, const float* dt_logits,
-                      int64_t dts, const float* dt_bias, const float* rate_log, const float* skip, hipStream_t stream) {
-  if (dt_logits != nullptr && chunks_serve(dk, seg_len, out, dv)) {
+                      int64_t dts, const float* dt_bias, const float* rate_log, const float* skip, int64_t tokens, int64_t longest,
+                      hipStream_t stream) {
+  if (dt_logits != nullptr && chunks_serve(false, batch, heads, dk, dv, tokens, longest, seg_len, out)) {
     const ChunkArgs p{out, state, q, k, v, dt_logits, dt_bias, rate_log, skip, nullptr, req_to_state, req_pool_indices, seg_start, seg_len,
                       positions, qs, ks, vs, dts, 0, heads, qk_heads, dk, dv, 0, q_scale};
     return launch_chunks<QT, VT, false>(p, batch, stream);
@@ -668,8 +687,8 @@ int launch_delta(float* out, float* state, const void* q, const void* k, const v
                  const float* gate_logits, const float* rate_bias, const float* rate_log, const int32_t* req_to_state,
                  const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions,
                  int64_t batch, int heads, int qk_heads, int dk, int dv, int64_t qs, int64_t ks, int64_t vs, int64_t bs, int64_t gs,
-                 float q_scale, int gate_per_head, int beta_f32, hipStream_t stream) {
-  if (gate_per_head && chunks_serve(dk, seg_len, out, dv)) {
+                 float q_scale, int gate_per_head, int beta_f32, int64_t tokens, int64_t longest, hipStream_t stream) {
+  if (gate_per_head && chunks_serve(true, batch, heads, dk, dv, tokens, longest, seg_len, out)) {
     const ChunkArgs p{out, state, q, k, v, gate_logits, rate_bias, rate_log, nullptr, beta_logits, req_to_state, req_pool_indices, seg_start,
                       seg_len, positions, qs, ks, vs, gs, bs, heads, qk_heads, dk, dv, beta_f32, q_scale};
     return launch_chunks<QT, VT, true>(p, batch, stream);
@@ -858,6 +877,10 @@ int launch_matrix_memory(float* out, float* state, float* norm_state, const void
 
 using namespace mi355;
 
+int mi355_recurrence_takes_chunks(int delta, int64_t batch, int heads, int key_dim, int value_dim, int64_t tokens, int64_t longest) {
+  return heads > 0 && key_dim > 0 && value_dim > 0 && chunks_pay(delta != 0, batch, heads, key_dim, value_dim, tokens, longest);
+}
+
 int mi355_linear_recurrence(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
                             const void* gate_bias, const float* head_decay, const int32_t* req_to_state,
                             const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
@@ -879,6 +902,19 @@ int mi355_linear_recurrence_ssm(float* out, float* state, const void* q, const v
                                 const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
                                 int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t gate_token_stride,
                                 float q_scale, float tau, int qk_dtype, int v_dtype, void* stream) {
+  return mi355_linear_recurrence_ssm_sized(out, state, q, k, v, gate_logits, gate_bias, head_decay, dt_logits, dt_token_stride, dt_bias,
+                                           rate_log, skip, req_to_state, req_pool_indices, seg_start, seg_len, positions, batch, heads,
+                                           qk_heads, key_dim, value_dim, q_token_stride, k_token_stride, v_token_stride,
+                                           gate_token_stride, q_scale, tau, qk_dtype, v_dtype, 0, 0, stream);
+}
+
+int mi355_linear_recurrence_ssm_sized(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
+                                const void* gate_bias, const float* head_decay, const float* dt_logits, int64_t dt_token_stride,
+                                const float* dt_bias, const float* rate_log, const float* skip, const int32_t* req_to_state,
+                                const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                                const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                                int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t gate_token_stride,
+                                float q_scale, float tau, int qk_dtype, int v_dtype, int64_t tokens, int64_t longest, void* stream) {
   MI355_REQUIRE(out && state && q && k && v && req_to_state && req_pool_indices && positions, MI355_ERR_INVALID,
                 "linear_recurrence: null pointer");
   MI355_REQUIRE((gate_logits != nullptr) + (head_decay != nullptr) + (dt_logits != nullptr) == 1, MI355_ERR_INVALID,
@@ -899,12 +935,12 @@ int mi355_linear_recurrence_ssm(float* out, float* state, const void* q, const v
       rc = launch_recurrence<T, T>(out, state, q, k, v, gate_logits, gate_bias, head_decay, req_to_state, req_pool_indices,
                                    seg_start, seg_len, positions, batch, heads, key_dim, value_dim, q_token_stride, k_token_stride,
                                    v_token_stride, gate_token_stride, q_scale, tau, qk_heads, dt_logits, dt_token_stride, dt_bias,
-                                   rate_log, skip, (hipStream_t)stream);
+                                   rate_log, skip, tokens, longest, (hipStream_t)stream);
     else
       rc = launch_recurrence<float, T>(out, state, q, k, v, gate_logits, gate_bias, head_decay, req_to_state, req_pool_indices,
                                        seg_start, seg_len, positions, batch, heads, key_dim, value_dim, q_token_stride,
                                        k_token_stride, v_token_stride, gate_token_stride, q_scale, tau, qk_heads, dt_logits,
-                                       dt_token_stride, dt_bias, rate_log, skip, (hipStream_t)stream);
+                                       dt_token_stride, dt_bias, rate_log, skip, tokens, longest, (hipStream_t)stream);
   });
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("linear_recurrence");
@@ -930,6 +966,19 @@ int mi355_gated_delta_rule_ex(float* out, float* state, const void* q, const voi
                               int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
                               int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
                               void* stream) {
+  return mi355_gated_delta_rule_sized(out, state, q, k, v, beta_logits, gate_logits, rate_bias, rate_log, req_to_state, req_pool_indices,
+                                      seg_start, seg_len, positions, batch, heads, qk_heads, key_dim, value_dim, q_token_stride,
+                                      k_token_stride, v_token_stride, beta_token_stride, gate_token_stride, q_scale, gate_per_head,
+                                      beta_f32, qk_dtype, v_dtype, 0, 0, stream);
+}
+
+int mi355_gated_delta_rule_sized(float* out, float* state, const void* q, const void* k, const void* v, const void* beta_logits,
+                              const float* gate_logits, const float* rate_bias, const float* rate_log, const int32_t* req_to_state,
+                              const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                              const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                              int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
+                              int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
+                              int64_t tokens, int64_t longest, void* stream) {
   MI355_REQUIRE(out && state && q && k && v && beta_logits && gate_logits && rate_bias && rate_log && req_to_state &&
                     req_pool_indices && positions, MI355_ERR_INVALID, "gated_delta_rule: null pointer");
   MI355_REQUIRE((seg_start == nullptr) == (seg_len == nullptr), MI355_ERR_INVALID,
@@ -946,12 +995,12 @@ int mi355_gated_delta_rule_ex(float* out, float* state, const void* q, const voi
       rc = launch_delta<T, T>(out, state, q, k, v, beta_logits, gate_logits, rate_bias, rate_log, req_to_state, req_pool_indices,
                               seg_start, seg_len, positions, batch, heads, qk_heads, key_dim, value_dim, q_token_stride,
                               k_token_stride, v_token_stride, beta_token_stride, gate_token_stride, q_scale, gate_per_head, beta_f32,
-                              (hipStream_t)stream);
+                              tokens, longest, (hipStream_t)stream);
     else
       rc = launch_delta<float, T>(out, state, q, k, v, beta_logits, gate_logits, rate_bias, rate_log, req_to_state,
                                   req_pool_indices, seg_start, seg_len, positions, batch, heads, qk_heads, key_dim, value_dim,
                                   q_token_stride, k_token_stride, v_token_stride, beta_token_stride, gate_token_stride, q_scale,
-                                  gate_per_head, beta_f32, (hipStream_t)stream);
+                                  gate_per_head, beta_f32, tokens, longest, (hipStream_t)stream);
   });
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("gated_delta_rule");

@@ -46,6 +46,12 @@ from ..ops_backend import get_ops
 from .rotary_embedding import pair_inv_freq
 
 
+def _longest(forward_batch) -> Optional[int]:
+    """Tokens of the step's longest segment (None in a decode step, which has no segments)."""
+    lens = None if forward_batch.forward_mode.is_decode_or_idle() else forward_batch.extend_seq_lens_cpu
+    return max(lens) if lens else None
+
+
 class LinearRecurrence(nn.Module):
     def __init__(self, num_heads: int, key_dim: int, value_dim: int, layer_id: int, device, q_scale: float = 1.0,
                  head_decay=None, tau: float = 1.0):
@@ -82,7 +88,7 @@ class StateSpaceRecurrence(nn.Module):
         out = torch.empty((x.shape[0], self.num_heads, self.value_dim), dtype=torch.float32, device=x.device)
         get_ops().linear_recurrence(c, b, x, out, st.pool.matrices[self.layer_id], st.req_to_state, st.req_pool_indices,
                                     forward_batch.positions, 1.0, dt_logits=dt_logits, dt_bias=self.dt_bias.data,
-                                    rate_log=self.rate_log.data, skip=self.skip.data, **st.segments())
+                                    rate_log=self.rate_log.data, skip=self.skip.data, longest=_longest(forward_batch), **st.segments())
         return out
 
 
@@ -118,7 +124,7 @@ class GatedDeltaRule(nn.Module):
         out = torch.empty((q.shape[0], self.num_heads, self.value_dim), dtype=torch.float32, device=q.device)
         get_ops().gated_delta_rule(q, k, v, beta_logits, gate_logits, self.rate_bias.data, self.rate_log.data, out,
                                    st.pool.matrices[self.layer_id], st.req_to_state, st.req_pool_indices, forward_batch.positions,
-                                   self.q_scale, **st.segments())
+                                   self.q_scale, longest=_longest(forward_batch), **st.segments())
         return out
 
 

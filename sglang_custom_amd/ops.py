@@ -1464,17 +1464,24 @@ def gelu_tanh_mul_rows(gate: torch.Tensor, table: torch.Tensor, ids: torch.Tenso
 
 
 # ------------------------------------------------------- linear recurrence over per-sequence matrices
+def _longest(longest: Optional[int], tokens: int, batch: int) -> int:
+    return int(longest) if longest is not None else -(-tokens // max(batch, 1))
+
+
 def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
                       req_to_state: torch.Tensor, req_pool_indices: torch.Tensor, positions: torch.Tensor, q_scale: float,
                       gate_logits: Optional[torch.Tensor] = None, gate_bias: Optional[torch.Tensor] = None, tau: float = 1.0,
                       head_decay: Optional[torch.Tensor] = None, tok_req=None, seg_start=None, seg_len=None,
                       dt_logits: Optional[torch.Tensor] = None, dt_bias: Optional[torch.Tensor] = None,
-                      rate_log: Optional[torch.Tensor] = None, skip: Optional[torch.Tensor] = None) -> torch.Tensor:
+                      rate_log: Optional[torch.Tensor] = None, skip: Optional[torch.Tensor] = None,
+                      longest: Optional[int] = None) -> torch.Tensor:
     """S = diag(a) S + k v^T, out = S^T (q * q_scale) per head over every sequence's tokens of the step, on
     state[slot] ([slots, H, dk, dv] fp32, read unless the sequence starts at position 0, written back).  q, k [T, H, dk]
     (fp32 or v's dtype), v [T, H, dv]; the decay from gate_logits fp32 [T, H * dk] (+ gate_bias, / tau) or head_decay fp32 [H],
     or (state-space form) from step sizes: dt = softplus(dt_logits [T, H] + dt_bias [H]), a = exp(-exp(rate_log [H]) dt),
-    S = a S + dt k v^T, out += skip [H] * v (all fp32).  q and k may have G < H heads (head h reads head h // (H / G))."""
+    S = a S + dt k v^T, out += skip [H] * v (all fp32).  q and k may have G < H heads (head h reads head h // (H / G)).
+    longest: tokens of the step's longest segment, which with their number decides how many tokens the state-space form takes at a
+    time (not given: the segments' mean)."""
     _gpu(q, k, v, out, state, req_to_state, req_pool_indices, positions, gate_logits, gate_bias, head_decay, dt_logits, dt_bias,
          rate_log, skip)
     T, G, dk = q.shape
@@ -1499,13 +1506,13 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: to
     _, ss, sl = _seg(tok_req, seg_start, seg_len)
     B = req_pool_indices.numel()
     assert seg_start is not None or B == T, "without segments every token is a sequence of its own"
-    check(_lib_().mi355_linear_recurrence_ssm(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+    check(_lib_().mi355_linear_recurrence_ssm_sized(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                               _p(gate_logits), _p(gate_bias), _p(head_decay), _p(dt_logits),
                                               dt_logits.stride(0) if dt_logits is not None else 0, _p(dt_bias), _p(rate_log), _p(skip),
                                               req_to_state.data_ptr(), req_pool_indices.data_ptr(), ss, sl, positions.data_ptr(), B,
                                               H, G, dk, dv, q.stride(0), k.stride(0), v.stride(0),
                                               gate_logits.stride(0) if gate_logits is not None else 0, float(q_scale), float(tau),
-                                              _dt(q), _dt(v), _stream(q)), "linear_recurrence")
+                                              _dt(q), _dt(v), T, _longest(longest, T, B), _stream(q)), "linear_recurrence")
     return out
 
 
@@ -1733,12 +1740,12 @@ def activation(x: torch.Tensor, act: str) -> torch.Tensor:
 def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta_logits: torch.Tensor, gate_logits: torch.Tensor,
                      rate_bias: torch.Tensor, rate_log: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
                      req_to_state: torch.Tensor, req_pool_indices: torch.Tensor, positions: torch.Tensor, q_scale: float,
-                     tok_req=None, seg_start=None, seg_len=None) -> torch.Tensor:
+                     tok_req=None, seg_start=None, seg_len=None, longest: Optional[int] = None) -> torch.Tensor:
     """Per head  S = diag(a) S;  u = beta (v - S^T k);  S += k u^T;  out = S^T (q * q_scale)  over every sequence's tokens of the
     step on state[slot] ([slots, H, dk, dv] fp32).  q, k [T, G, dk] (fp32 or v's dtype; head h reads head h // (H / G)), v
     [T, H, dv], beta_logits [T, H] (row-strided, v's dtype or fp32), gate_logits fp32 [T, H * dk], rate_bias fp32 [H * dk],
     rate_log fp32 [H]:  a = exp(-exp(rate_log) * softplus(gate_logits + rate_bias)),  beta = sigmoid(beta_logits).  With
-    gate_logits [T, H] and rate_bias [H] the decay is one number per head and token."""
+    gate_logits [T, H] and rate_bias [H] the decay is one number per head and token.  longest: see linear_recurrence."""
     _gpu(q, k, v, beta_logits, gate_logits, rate_bias, rate_log, out, state, req_to_state, req_pool_indices, positions)
     T, G, dk = q.shape
     H, dv = v.shape[1], v.shape[2]
@@ -1756,12 +1763,12 @@ def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta_log
     _, ss, sl = _seg(tok_req, seg_start, seg_len)
     B = req_pool_indices.numel()
     assert seg_start is not None or B == T, "without segments every token is a sequence of its own"
-    check(_lib_().mi355_gated_delta_rule_ex(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+    check(_lib_().mi355_gated_delta_rule_sized(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                             beta_logits.data_ptr(), gate_logits.data_ptr(), rate_bias.data_ptr(), rate_log.data_ptr(),
                                             req_to_state.data_ptr(), req_pool_indices.data_ptr(), ss, sl, positions.data_ptr(), B, H, G,
                                             dk, dv, q.stride(0), k.stride(0), v.stride(0), beta_logits.stride(0), gate_logits.stride(0),
                                             float(q_scale), int(per_head), int(beta_logits.dtype == torch.float32 and v.dtype != torch.float32),
-                                            _dt(q), _dt(v), _stream(q)), "gated_delta_rule")
+                                            _dt(q), _dt(v), T, _longest(longest, T, B), _stream(q)), "gated_delta_rule")
     return out
 
 

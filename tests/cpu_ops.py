@@ -421,7 +421,7 @@ def qkv_norm_rope_write(q, k, v, wq, wk, eps, positions, inv_freq, rot_dims, int
 
 def linear_recurrence(q, k, v, out, state, req_to_state, req_pool_indices, positions, q_scale, gate_logits=None, gate_bias=None,
                       tau=1.0, head_decay=None, tok_req=None, seg_start=None, seg_len=None, dt_logits=None, dt_bias=None,
-                      rate_log=None, skip=None):
+                      rate_log=None, skip=None, longest=None):
     T, G, dk = q.shape
     H = v.shape[1]
     rep = H // G
@@ -629,7 +629,7 @@ def activation(x, act):
 
 
 def gated_delta_rule(q, k, v, beta_logits, gate_logits, rate_bias, rate_log, out, state, req_to_state, req_pool_indices, positions,
-                     q_scale, tok_req=None, seg_start=None, seg_len=None):
+                     q_scale, tok_req=None, seg_start=None, seg_len=None, longest=None):
     T, G, dk = q.shape
     H = v.shape[1]
     rep = H // G

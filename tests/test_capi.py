@@ -91,3 +91,14 @@ def test_planner_is_pure_host_logic(lib):
 def test_split_plan_of_one_byte_rows(lib, bs, hkv, keys, most, bf16, fp8):
     assert lib.mi355_decode_num_splits(bs, hkv, keys, most) == bf16
     assert lib.mi355_decode_num_splits_fp8(bs, hkv, keys, most) == fp8
+
+
+@pytest.mark.parametrize("delta,batch,heads,dk,dv,tokens,longest,chunks", [
+    (0, 1, 16, 64, 128, 1, 1, 0), (0, 1, 16, 64, 128, 16, 16, 0), (0, 1, 16, 64, 128, 64, 64, 1), (1, 1, 16, 64, 128, 16, 16, 0),   # short segments
+    (1, 1, 16, 64, 128, 64, 64, 1), (0, 4, 16, 64, 128, 7400, 2048, 1), (1, 4, 16, 64, 128, 7400, 2048, 1),
+    (0, 64, 16, 64, 128, 256, 4, 0), (0, 64, 16, 64, 128, 64 * 64, 64, 0), (1, 64, 16, 64, 128, 64 * 500, 500, 0),                  # more workgroups than CUs
+    (0, 8, 16, 64, 128, 8 * 65, 65, 0), (0, 8, 16, 64, 128, 8 * 128, 128, 1), (1, 32, 16, 64, 128, 32 + 2000, 2000, 1),             # one long among many short
+    (0, 1, 16, 65, 128, 4000, 4000, 0), (0, 4, 16, 64, 128, 0, 0, 0), (0, 0, 16, 64, 128, 10, 10, 0),                                # not served, not known
+])
+def test_recurrence_chunk_rule(lib, delta, batch, heads, dk, dv, tokens, longest, chunks):
+    assert lib.mi355_recurrence_takes_chunks(delta, batch, heads, dk, dv, tokens, longest) == chunks

@@ -235,6 +235,11 @@ int mi355_decode_attention(const void* q, const void* k_buffer, const void* v_bu
 int mi355_decode_num_splits(int64_t bs, int hkv, int64_t max_seq_len, int max_splits);
 /* The same for a cache of e4m3fn rows, which fills the chip only at twice as many workgroups. */
 int mi355_decode_num_splits_fp8(int64_t bs, int hkv, int64_t max_seq_len, int max_splits);
+/* Either plan (kv_fp8) for a launch whose lengths are not known yet, a captured one, with max_seq_len the most they may be: returns
+ * the splits to launch.  For a batch whose longest sequence is `len`, kv_chunk_keys should then come from max(fewest, min(splits,
+ * len / split_keys)) of them (all, if split_keys is 0): splits further than `fewest` pay only with split_keys keys each.  The
+ * matrix-core kernel (head_dim 128, 16-bit q) passes over those that the chunk leaves empty; elsewhere they cost as much as full ones. */
+int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_splits, int kv_fp8, int* fewest, int64_t* split_keys);
 
 /* ---- K4 extend / prefill attention -----------------------------------------------------------
  * q_extend [T, Hq, D], k_extend/v_extend [T, Hkv, D|Dv] (row strides given), o_extend [T,Hq,Dv]

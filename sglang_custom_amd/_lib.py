@@ -35,6 +35,7 @@ _SIGNATURES = {
     "mi355_decode_attention": (I, [P, P, P, P, P, I, P, P, P, L, P, P, P, P, I, L, I, I, I, I, L, L, F, F, I, P]),
     "mi355_decode_num_splits": (I, [L, I, L, I]),
     "mi355_decode_num_splits_fp8": (I, [L, I, L, I]),
+    "mi355_decode_split_plan": (I, [L, I, L, I, I, P, P]),
     "mi355_extend_attention": (I, [P, P, P, P, P, P, P, P, P, P, P, I, I, L, L, I, I, I, I, L, L, L,
                                    L, F, F, I, I, P]),
     "mi355_linear_workspace_bytes": (L, [L, L, L]),

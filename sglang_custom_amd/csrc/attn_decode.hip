@@ -707,6 +707,11 @@ constexpr int DV_ROW = 128 + 16;   // V tile row in LDS (elements): 288 B -> con
 // required (G = all query heads of the kv head), so nobody else reads or writes that slot.
 // KV8: the cache holds e4m3fn bytes (kbuf / vbuf are byte buffers behind the T pointers): rows are
 // widened to T on load, the new token's rows are stored quantised and used at their stored value.
+// grid: (hkv * (gtotal / G), B, num_splits): every sequence's first split is ahead of all second ones, and so on, so that where
+// the batch's chunk leaves splits empty (the last ones) the full ones are dealt out evenly; and a sequence whose keys all fall to
+// its first split is finished there, without a partial and a merge.  A captured launch of 4 splits on a batch that needs one:
+// 128 workgroups, e4m3fn rows, 300 / 4096 keys 14.0 / 68.2 us with sequences outside splits and the merge, 9.1 / 47.7 so (unsplit
+// 8.8 / 47.9); 512 workgroups, 16-bit rows, 300 keys 47.0 -> 16.7 (15.5).
 template <typename T, int G, bool CAP, bool FUSED = false, bool KV8 = false, bool KROW = false>
 __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __restrict__ q,
                                                                   const T* kbuf, const T* vbuf,
@@ -735,13 +740,15 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   const int xrot = (blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x;
   const int kvh = xrot / groups_per_kv;
   const int head0 = kvh * gtotal + (xrot % groups_per_kv) * G;
-  const int split = blockIdx.y, b = blockIdx.z;
+  const int b = blockIdx.y, split = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r16 = lane & 15, c4 = lane >> 4;
 
   int64_t page_off, len;
   seq_range(p, b, page_off, len);
   const int64_t chunk = split_chunk(p, len);
+  const bool alone = p.num_splits == 1 || (p.tickets && chunk >= len);
+  if (alone && split > 0) return;
   const int64_t k0 = (int64_t)split * chunk;
   const int64_t k1 = k0 + chunk < len ? k0 + chunk : len;
   const float qmul = CAP ? p.sm_scale : p.sm_scale * kLog2e;
@@ -1127,7 +1134,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
     const float val = lt > 0.f ? at / lt : 0.f;
     const int head = head0 + g;
-    if (p.num_splits == 1) {
+    if (alone) {
       o[((int64_t)b * p.hq + head) * D + d] = from_f32<T>(val);
     } else {
       // write-through, so that the workgroup that merges the splits (below) sees them without a fence;
@@ -1142,7 +1149,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
   }
   // (one counter per sequence and head group: blockIdx.x is rotated, xrot names the group)
-  if (p.num_splits > 1 && p.tickets) merge_splits_if_last<T, 1>(p, o, b, head0, G, D, b * (int)gridDim.x + xrot, &sm_acc[0][0][0]);
+  if (!alone && p.tickets) merge_splits_if_last<T, 1>(p, o, b, head0, G, D, b * (int)gridDim.x + xrot, &sm_acc[0][0][0]);
 }
 
 // Any head_dim / v_head_dim (<= 1024): one wave per (head, split, sequence); lanes stride the
@@ -2655,34 +2662,34 @@ static void launch_decode_dc(const T* q, const T* kb, const T* vb, T* o, const D
                              int64_t bs, bool kv8, hipStream_t st) {   // kv8: the KV cache holds e4m3fn bytes
   const int gtotal = p.hq / p.hkv;
   const int G = gtotal % 8 == 0 ? 8 : gtotal % 4 == 0 ? 4 : gtotal % 2 == 0 ? 2 : 1;
-  const dim3 grid((unsigned)(p.hkv * (gtotal / G)), (unsigned)p.num_splits, (unsigned)bs);
+  const dim3 grid((unsigned)(p.hkv * (gtotal / G)), (unsigned)p.num_splits, (unsigned)bs), grid_pv(grid.x, grid.z, grid.y);
   const dim3 block(256);
   if constexpr (D == 128 && !std::is_same<T, float>::value) {
     if (kv8) {
       switch (G) {
-        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP, false, true, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP, false, true, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP, false, true, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP, false, true, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
       }
       return;
     }
     if (g_decode_variant == 0) {
       switch (G) {
-        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP, false, false, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP, false, false, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP, false, false, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP, false, false, true>), grid, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
       }
       return;
     }
 #ifdef MI355_DEV_BUILD
     if (g_decode_variant == 3) {   // ablation: K rows loaded straight into MFMA fragments (16 rows x 64 B per instruction)
       switch (G) {
-        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
-        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
-        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
-        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
+        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
       }
       return;
     }
@@ -2759,7 +2766,7 @@ static int launch_decode_fused(const T* kb, const T* vb, T* o, const DecodeParam
   DecodeParams p = p_in;
   if (p.num_splits <= 1 || p.num_splits > MERGE_MAX_SPLITS) p.tickets = nullptr;
   const int G = p.hq / p.hkv;
-  const dim3 grid((unsigned)p.hkv, (unsigned)p.num_splits, (unsigned)bs), block(256);
+  const dim3 grid((unsigned)p.hkv, (unsigned)bs, (unsigned)p.num_splits), block(256);
   if (kv8) {
     switch (G) {
       case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, false, true, true, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
@@ -2796,57 +2803,66 @@ using namespace mi355;
 
 extern "C" {
 
-int mi355_decode_num_splits(int64_t bs, int hkv, int64_t max_seq_len, int max_splits) {
-  if (bs <= 0 || hkv <= 0 || max_splits <= 1) return 1;
-  // Split only until the launch can saturate HBM, and no further: a workgroup of the MFMA kernel
-  // streams ~45 GB/s, so ~112 of them already draw what the chip delivers to this access pattern,
-  // and every extra split costs fp32 partial traffic plus ~1 us of the merge launch.  Measured at
-  // 1064 keys, head_dim 128 (microseconds, best in brackets): 8 workgroups unsplit 17.6 [6-8 splits:
-  // 11.6]; 64: 19.9 [3: 14.4; 8: 19.1]; 128: 20.5 [2: 19.7; 4: 22.3]; 256: 31.7 [1; 2: 34.4].
-  // Long contexts (>= 1024 keys per split left) with fewer than 192 workgroups are split until every CU has one.
-  // 64 sequences x one kv head x 4136 keys with the merge inside the launch: 34.9 / 27.7 / 29.5 / 36.1 / 33.4 /
-  // 46.1 us at 2 / 3 / 4 / 6 / 8 / 16 splits -- 192 workgroups of 1 379 keys beat 256 of 1 034 (every split pays its
-  // own address chain and one more partial), and the same bytes unsplit (256 sequences x 1 034 keys) take 25.6.
-  const int64_t wgs = bs * hkv;
-  int64_t want = wgs >= 112 ? 1 : (160 + wgs - 1) / wgs;
-  if (want > 1 && wgs * want < 192 && max_seq_len / ((256 + wgs - 1) / wgs) >= 1024) want = (256 + wgs - 1) / wgs;
-  // 112 to 128 workgroups draw the chip's rate only while every one of them runs: with 1 024 keys left per split half
-  // the CUs' worth more of them pays, and more again when the lengths differ and the longest row would run alone.
-  // 128 workgroups, head_dim 128, 1 -> 2 splits: 512 keys 11.1 -> 12.1 us, 1 024 17.7 -> 16.9, 2 048 28.3 -> 26.7,
-  // 4 096 57.4 -> 47.5, 1 638 to 4 096 52.8 -> 38.4; 144 workgroups (more than the CUs once doubled), 2 048: 29.2 -> 37.0.
-  if (wgs >= 112 && wgs <= 128 && max_seq_len >= 2048) want = 2;
-  // A handful of workgroups (one sequence on a tensor-parallel rank): the launch is a latency chain, ~9.5 ns per key
-  // of a split plus ~0.11 us per split merged, least at sqrt(keys / 12) splits.  One sequence x one kv head x 4104
-  // keys: 22.3 / 17.6 / 16.2 / 16.2 / 16.6 / 17.5 / 21.7 us at 4 / 8 / 12 / 16 / 24 / 32 / 64 splits.
-  int64_t by_len = max_seq_len / 128 > 0 ? max_seq_len / 128 : 1;
-  const int64_t by_merge = (int64_t)std::ceil(std::sqrt((double)max_seq_len / 12.0));
-  if (by_len > by_merge) by_len = by_merge > 1 ? by_merge : 1;
-  if (want > by_len) want = by_len;
-  if (want > max_splits) want = max_splits;
-  if (want < 1) want = 1;
+int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_splits, int kv_fp8, int* fewest, int64_t* split_keys) {
+  int few = 1;
+  int64_t want = 1, keep = 0;   // splits further than `few` hold at least `keep` keys each (0: there are none)
+  if (bs > 0 && hkv > 0 && max_splits > 1) {
+    // Split only until the launch can saturate HBM, and no further: a workgroup of the MFMA kernel
+    // streams ~45 GB/s, so ~112 of them already draw what the chip delivers to this access pattern,
+    // and every extra split costs fp32 partial traffic plus ~1 us of the merge launch.  Measured at
+    // 1064 keys, head_dim 128 (microseconds, best in brackets): 8 workgroups unsplit 17.6 [6-8 splits:
+    // 11.6]; 64: 19.9 [3: 14.4; 8: 19.1]; 128: 20.5 [2: 19.7; 4: 22.3]; 256: 31.7 [1; 2: 34.4].
+    // Long contexts (>= 1024 keys per split left) with fewer than 192 workgroups are split until every CU has one.
+    // 64 sequences x one kv head x 4136 keys with the merge inside the launch: 34.9 / 27.7 / 29.5 / 36.1 / 33.4 /
+    // 46.1 us at 2 / 3 / 4 / 6 / 8 / 16 splits -- 192 workgroups of 1 379 keys beat 256 of 1 034 (every split pays its
+    // own address chain and one more partial), and the same bytes unsplit (256 sequences x 1 034 keys) take 25.6.
+    const int64_t wgs = bs * hkv;
+    int64_t base = wgs >= 112 ? 1 : (160 + wgs - 1) / wgs;
+    if (base > 1 && wgs * base < 192 && max_seq_len / ((256 + wgs - 1) / wgs) >= 1024) base = (256 + wgs - 1) / wgs;
+    // A handful of workgroups (one sequence on a tensor-parallel rank): the launch is a latency chain, ~9.5 ns per key
+    // of a split plus ~0.11 us per split merged, least at sqrt(keys / 12) splits.  One sequence x one kv head x 4104
+    // keys: 22.3 / 17.6 / 16.2 / 16.2 / 16.6 / 17.5 / 21.7 us at 4 / 8 / 12 / 16 / 24 / 32 / 64 splits.
+    int64_t by_len = max_seq_len / 128 > 0 ? max_seq_len / 128 : 1;
+    const int64_t by_merge = (int64_t)std::ceil(std::sqrt((double)max_seq_len / 12.0));
+    if (by_len > by_merge) by_len = by_merge > 1 ? by_merge : 1;
+    base = std::max<int64_t>(1, std::min({base, by_len, (int64_t)max_splits}));
+    few = (int)base;
+    want = base;
+    // 112 to 128 workgroups draw the chip's rate only while every one of them runs: with 1 024 keys left per split half
+    // the CUs' worth more of them pays, and more again when the lengths differ and the longest row would run alone.
+    // 128 workgroups, head_dim 128, 1 -> 2 splits: 512 keys 11.1 -> 12.1 us, 1 024 17.7 -> 16.9, 2 048 28.3 -> 26.7,
+    // 4 096 57.4 -> 47.5, 1 638 to 4 096 52.8 -> 38.4; 144 workgroups (more than the CUs once doubled), 2 048: 29.2 -> 37.0.
+    // (head_dim 64, whose splits take a second launch to merge: 128 workgroups, 2 048 keys 26.2 -> 20.5, 4 096 45.7 -> 30.4.)
+    if (wgs >= 112 && wgs <= 128) keep = 1024;
+    int64_t most = 2;
+    // One-byte rows halve what a workgroup draws (~23 GB/s: its time per key is the chain of page read, row read and
+    // product, not the bytes), so the chip takes two workgroups per CU before it is full: 512 of them, at most 4 splits
+    // (a fifth is a second merge chain).  A split has to keep 512 keys, and 4 per workgroup of the unsplit launch, to pay
+    // for its partial: where the launch is already wide there is less left to fill.  head_dim 128, 8 kv heads, us at
+    // 1 / 2 / 3 / 4 splits (bracket: taken):
+    //   64 wgs, 4 096 keys  46.7 / 29.1 / 22.9 / [19.6];   128 wgs, 512 keys [10.3] / 10.2 / 12.9 / 11.7;
+    //  128 wgs, 1 024       16.2 / [13.3] / 15.6 / 14.0;   128 wgs, 2 048     26.5 / 18.9 / 21.8 / [19.0];
+    //  128 wgs, 4 096       47.8 / 30.5 / 32.8 / [28.7];   144 wgs, 1 024    [16.0] / 17.1 / 15.9 / 17.1;
+    //  160 wgs, 2 048       27.0 / 25.3 / [22.6] / 24.7;   160 wgs, 4 096     48.4 / 41.9 / [34.9] / 39.2;
+    //  224 wgs, 4 096       49.6 / [46.5] / 50.7 / 54.9;   256 wgs, 1 024    [16.8] / 18.6 / 21.4 / 25.9;
+    //  256 wgs, 4 096       51.0 / [49.2] / 51.8 / 59.7;   384 wgs, 4 096    [74.7] / 70.5 / 78.6 / 77.0.
+    if (kv_fp8) {
+      most = 512 / wgs < 4 ? 512 / wgs : 4;
+      keep = most > 1 ? (4 * wgs > 512 ? 4 * wgs : 512) : 0;
+    }
+    if (keep > 0) want = std::max(want, std::min({most, max_seq_len / keep, (int64_t)max_splits}));
+  }
+  if (fewest) *fewest = few;
+  if (split_keys) *split_keys = keep;
   return (int)want;
 }
 
+int mi355_decode_num_splits(int64_t bs, int hkv, int64_t max_seq_len, int max_splits) {
+  return mi355_decode_split_plan(bs, hkv, max_seq_len, max_splits, 0, nullptr, nullptr);
+}
+
 int mi355_decode_num_splits_fp8(int64_t bs, int hkv, int64_t max_seq_len, int max_splits) {
-  const int64_t base = mi355_decode_num_splits(bs, hkv, max_seq_len, max_splits);
-  if (bs <= 0 || hkv <= 0 || max_splits <= 1) return (int)base;
-  // One-byte rows halve what a workgroup draws (~23 GB/s: its time per key is the chain of page read, row read and
-  // product, not the bytes), so the chip takes two workgroups per CU before it is full: 512 of them, at most 4 splits
-  // (a fifth is a second merge chain).  A split has to keep 512 keys, and 4 per workgroup of the unsplit launch, to pay
-  // for its partial: where the launch is already wide there is less left to fill.  head_dim 128, 8 kv heads, us at
-  // 1 / 2 / 3 / 4 splits (bracket: taken):
-  //   64 wgs, 4 096 keys  46.7 / 29.1 / 22.9 / [19.6];   128 wgs, 512 keys [10.3] / 10.2 / 12.9 / 11.7;
-  //  128 wgs, 1 024       16.2 / [13.3] / 15.6 / 14.0;   128 wgs, 2 048     26.5 / 18.9 / 21.8 / [19.0];
-  //  128 wgs, 4 096       47.8 / 30.5 / 32.8 / [28.7];   144 wgs, 1 024    [16.0] / 17.1 / 15.9 / 17.1;
-  //  160 wgs, 2 048       27.0 / 25.3 / [22.6] / 24.7;   160 wgs, 4 096     48.4 / 41.9 / [34.9] / 39.2;
-  //  224 wgs, 4 096       49.6 / [46.5] / 50.7 / 54.9;   256 wgs, 1 024    [16.8] / 18.6 / 21.4 / 25.9;
-  //  256 wgs, 4 096       51.0 / [49.2] / 51.8 / 59.7;   384 wgs, 4 096    [74.7] / 70.5 / 78.6 / 77.0.
-  const int64_t wgs = bs * hkv;
-  int64_t want = 512 / wgs < 4 ? 512 / wgs : 4;
-  const int64_t keep = 4 * wgs > 512 ? 4 * wgs : 512;
-  if (want > max_seq_len / keep) want = max_seq_len / keep;
-  if (want > max_splits) want = max_splits;
-  return (int)(want > base ? want : base);
+  return mi355_decode_split_plan(bs, hkv, max_seq_len, max_splits, 1, nullptr, nullptr);
 }
 
 int mi355_decode_attention(const void* q, const void* k_buffer, const void* v_buffer, void* o,

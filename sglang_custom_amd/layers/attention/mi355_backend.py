@@ -68,6 +68,9 @@ class Mi355AttnBackend(AttentionBackend):
         # per-layer key / value shapes (LayeredMHATokenToKVPool): served by forward_sigmoid alone, with the same metadata
         self.is_layered = hasattr(model_runner.token_to_kv_pool, "layer_shapes")
         self.kv_fp8 = getattr(model_runner.token_to_kv_pool, "dtype", None) == torch.float8_e4m3fn
+        # the decode kernel of these shapes merges its splits in its own launch and passes over empty ones
+        self.merges_in_launch = (not (self.is_mla or self.is_latent_window or self.is_layered)
+                                 and getattr(cfg, "head_dim", None) == 128 and getattr(model_runner, "dtype", None) in (torch.bfloat16, torch.float16))
         if self.is_mla:
             # what the split plan counts is workgroups per sequence, one per 16 query heads
             self.num_kv_head = (self.num_head + 15) // 16
@@ -90,6 +93,7 @@ class Mi355AttnBackend(AttentionBackend):
         # (get_num_kv_splits_triton of the reference, triton_backend.py:875-924)
         self._chunk_keys = torch.ones(1, dtype=torch.int32, device=self.device)
         self.graph_num_splits = {}
+        self.graph_split_rule = {}    # by batch size: (fewest, split_keys) of the captured splits
         self.graph_window_indptr = None
         self.graph_window_indices = None
 
@@ -137,6 +141,19 @@ class Mi355AttnBackend(AttentionBackend):
         plan = get_ops().decode_num_splits_fp8 if self.kv_fp8 else get_ops().decode_num_splits
         return plan(bs, self.num_kv_head, max_seq_len, MAX_KV_SPLITS)
 
+    def _plan_captured(self, bs: int, max_seq_len: int):
+        """(splits, fewest, split_keys) of a captured step, whose lengths are not known yet (see ops.decode_split_plan)."""
+        if self.is_mla:
+            splits = self._plan_splits(bs, max_seq_len)
+            return splits, splits, 0
+        splits, fewest, keys = get_ops().decode_split_plan(bs, self.num_kv_head, max_seq_len, MAX_KV_SPLITS, self.kv_fp8)
+        if not self.merges_in_launch:
+            # a split that a short batch leaves empty costs as much as a full one here.  The kernel that reads e4m3fn rows at other
+            # head sizes is so slow a chain per split that they pay at any length (128 workgroups, head_dim 64, 300 keys:
+            # 287 / 163 / 117 / 92 us at 1 / 2 / 3 / 4); 16-bit ones do not below some 700 keys (300: 9.7 / 11.7 at 1 / 2).
+            splits, fewest, keys = (splits, splits, 0) if self.kv_fp8 else (fewest, fewest, 0)
+        return splits, fewest, keys
+
     # ---- eager ----
     def init_forward_metadata(self, forward_batch):
         ops = get_ops()
@@ -157,7 +174,8 @@ class Mi355AttnBackend(AttentionBackend):
                                  tickets=self._tickets if logits is not None else None,
                                  kv_chunk_keys=self._chunk_keys if splits > 1 else None)
             self._reset_tickets(max(splits, wsplits))
-            self._set_chunk_keys(splits, max_len)
+            if splits > 1:
+                self._set_chunk_keys(splits, max_len)
             if self.sliding_window_size:
                 cpu = forward_batch.seq_lens_cpu.tolist() if forward_batch.seq_lens_cpu is not None else None
                 md.window_kv_indptr, md.window_kv_indices = self._window(
@@ -202,14 +220,16 @@ class Mi355AttnBackend(AttentionBackend):
             self.forward_metadata.latent_blocks = {}
             return
         # one graph serves every step: split for the longest context the model can reach
-        splits = self._plan_splits(bs, self.max_context_len)
+        splits, fewest, keys = self._plan_captured(bs, self.max_context_len)
         self.graph_num_splits[bs] = splits
-        wsplits = self._plan_splits(bs, self.sliding_window_size + 1) if self.sliding_window_size else 1
+        self.graph_split_rule[bs] = (fewest, keys)
+        wsplits = self._plan_captured(bs, self.sliding_window_size + 1)[1] if self.sliding_window_size else 1
         logits, lse = self._scratch(bs, max(splits, wsplits)) if max(splits, wsplits) > 1 else (None, None)
         md = ForwardMetadata(num_kv_splits=splits, attn_logits=logits, attn_lse=lse, window_num_kv_splits=wsplits,
                              tickets=self._tickets if logits is not None else None,
                              kv_chunk_keys=self._chunk_keys if splits > 1 else None)
-        self._set_chunk_keys(splits, 1)   # the capture runs on fill-value lengths
+        if splits > 1:
+            self._set_chunk_keys(splits, 1)   # the capture runs on fill-value lengths
         if self.sliding_window_size:
             md.window_kv_indptr, md.window_kv_indices = self._window(
                 seq_lens[:bs], None, req_pool_indices[:bs], bs, self.graph_window_indptr, self.graph_window_indices)
@@ -227,15 +247,18 @@ class Mi355AttnBackend(AttentionBackend):
         self._reset_tickets(max(splits, 2 if self.sliding_window_size else 1))
         if splits > 1:
             # the graph was planned for the longest context the model can reach; the batch in front of us sets
-            # the chunk, so that its longest sequence uses every split and shorter ones proportionally fewer
+            # the chunk, so that its longest sequence uses as many splits as pay for it and shorter ones proportionally fewer
+            fewest, keys = self.graph_split_rule.get(bs, (splits, 0))
             if seq_lens_cpu is not None:
-                self._set_chunk_keys(splits, int(seq_lens_cpu.max()) if bs > 0 else 1)
+                longest = int(seq_lens_cpu.max()) if bs > 0 else 1
+                self._set_chunk_keys(max(fewest, min(splits, longest // keys)) if keys else splits, longest)
             else:
-                self._chunk_keys.copy_(((seq_lens[:bs].max() + (splits - 1)) // splits).clamp(min=1).to(torch.int32).view(1))
+                longest = seq_lens[:bs].max()
+                used = (longest // keys).clamp(fewest, splits) if keys else splits
+                self._chunk_keys.copy_(((longest + (used - 1)) // used).clamp(min=1).to(torch.int32).view(1))
 
     def _set_chunk_keys(self, splits: int, max_len: int):
-        if splits > 1:
-            self._chunk_keys.fill_(max(1, (max_len + splits - 1) // splits))
+        self._chunk_keys.fill_(max(1, (max_len + splits - 1) // splits))
 
     def _reset_tickets(self, splits: int):
         """The kernels hand the split-merge counters back zeroed; a launch that died half-way (a failed

@@ -6,6 +6,7 @@ pointers and the current torch stream to libmi355_hotpath.so.  Nothing here comp
 is used for memory and streams only.  Outputs are allocated by the caller or returned fresh,
 mirroring sgl-kernel/python/sgl_kernel/{elementwise,sampling}.py.
 """
+import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -362,6 +363,14 @@ def decode_num_splits(bs: int, hkv: int, max_seq_len: int, max_splits: int) -> i
 
 def decode_num_splits_fp8(bs: int, hkv: int, max_seq_len: int, max_splits: int) -> int:
     return _lib_().mi355_decode_num_splits_fp8(bs, hkv, max_seq_len, max_splits)
+
+
+def decode_split_plan(bs: int, hkv: int, max_seq_len: int, max_splits: int, kv_fp8: bool) -> Tuple[int, int, int]:
+    """(splits, fewest, split_keys) of a launch that is captured before its lengths are known, at most max_seq_len: a batch whose
+    longest sequence is n takes max(fewest, min(splits, n // split_keys)) of the splits (all, if split_keys is 0)."""
+    fewest, keys = ctypes.c_int(), ctypes.c_int64()
+    splits = _lib_().mi355_decode_split_plan(bs, hkv, max_seq_len, max_splits, int(kv_fp8), ctypes.byref(fewest), ctypes.byref(keys))
+    return splits, fewest.value, keys.value
 
 
 def decode_attention_fwd(q, k_buffer, v_buffer, o, kv_indptr, kv_indices, attn_logits, attn_lse,

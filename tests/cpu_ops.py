@@ -91,6 +91,10 @@ def decode_num_splits_fp8(bs, hkv, max_seq_len, max_splits):
     return 1
 
 
+def decode_split_plan(bs, hkv, max_seq_len, max_splits, kv_fp8):
+    return 1, 1, 0
+
+
 def decode_attention_paged(q, k_buffer, v_buffer, o, req_to_token, req_pool_indices, seq_lens,
                            attn_logits, attn_lse, num_kv_splits, sm_scale, logit_cap=0.0, tickets=None, kv_chunk_keys=None):
     assert logit_cap == 0.0

@@ -102,3 +102,17 @@ def test_split_plan_of_one_byte_rows(lib, bs, hkv, keys, most, bf16, fp8):
 ])
 def test_recurrence_chunk_rule(lib, delta, batch, heads, dk, dv, tokens, longest, chunks):
     assert lib.mi355_recurrence_takes_chunks(delta, batch, heads, dk, dv, tokens, longest) == chunks
+
+
+@pytest.mark.parametrize("bs,hkv,keys,most,fp8,splits,fewest,split_keys", [
+    (16, 8, 4096, 64, 0, 2, 1, 1024), (14, 8, 1500, 64, 0, 1, 1, 1024), (17, 8, 4096, 64, 0, 1, 1, 0), (8, 8, 4096, 64, 0, 3, 3, 0),
+    (16, 8, 4096, 64, 1, 4, 1, 512), (32, 8, 4096, 64, 1, 2, 1, 1024), (33, 8, 8192, 64, 1, 1, 1, 0), (8, 8, 1100, 64, 1, 3, 3, 512),
+    (16, 8, 4096, 1, 1, 1, 1, 0), (0, 8, 4096, 64, 1, 1, 1, 0),
+])
+def test_split_plan_of_captured_launches(lib, bs, hkv, keys, most, fp8, splits, fewest, split_keys):
+    import ctypes
+
+    f, k = ctypes.c_int(-1), ctypes.c_int64(-1)
+    assert lib.mi355_decode_split_plan(bs, hkv, keys, most, fp8, ctypes.byref(f), ctypes.byref(k)) == splits
+    assert (f.value, k.value) == (fewest, split_keys)
+    assert splits == (lib.mi355_decode_num_splits_fp8 if fp8 else lib.mi355_decode_num_splits)(bs, hkv, keys, most)

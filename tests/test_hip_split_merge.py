@@ -319,3 +319,33 @@ def test_per_sequence_split_plan_on_a_ragged_batch(ops, in_kernel_merge):
     assert torch.equal(_bits(out), _bits(got))
     if tickets is not None:
         assert int(tickets.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,splits", [(32, 8, 4), (4, 4, 2), (16, 2, 16)])
+def test_sequences_of_one_split_are_finished_without_a_merge(ops, kv8, Hq, Hkv, splits):
+    """kv_chunk_keys at least a sequence's length: its first split answers with the bits of an unsplit launch and touches neither
+    partials nor counters; longer sequences of the batch are merged as ever."""
+    dt, D, chunk, lens = torch.bfloat16, 128, 300, [300, 1, 299, 0, 301, 620, 64, 2]
+    q, kc, vc, r2t, pool, lt = (x.to(DEV) for x in _paged(61, dt, len(lens), Hq, Hkv, D, [max(n, 1) for n in lens]))
+    lt = torch.tensor(lens, dtype=torch.int64, device=DEV)
+    if kv8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    B = len(lens)
+    whole, want, got = (torch.full((B, Hq, D), float("nan"), dtype=dt, device=DEV) for _ in range(3))
+    ops.decode_attention_paged(q, kc, vc, whole, r2t, pool, lt, None, None, 1, D ** -0.5)
+    ck = torch.tensor([chunk], dtype=torch.int32, device=DEV)
+    al, ll = torch.empty(B * Hq * splits * D, device=DEV), torch.empty(B * Hq * splits, device=DEV)
+    ops.decode_attention_paged(q, kc, vc, want, r2t, pool, lt, al, ll, splits, D ** -0.5, kv_chunk_keys=ck)
+    tickets = torch.zeros(4096, dtype=torch.int32, device=DEV)
+    for _ in range(2):
+        al.fill_(float("nan"))
+        ll.fill_(float("nan"))
+        got.fill_(float("nan"))
+        ops.decode_attention_paged(q, kc, vc, got, r2t, pool, lt, al, ll, splits, D ** -0.5, tickets=tickets, kv_chunk_keys=ck)
+        torch.cuda.synchronize()
+        for b, n in enumerate(lens):
+            one = n <= max(chunk, -(-n // splits))
+            assert torch.equal(_bits(got[b]), _bits((whole if one else want)[b])), (b, n)
+            assert al.view(B, Hq, -1)[b].isnan().all() == one
+        assert int(tickets.sum()) == 0

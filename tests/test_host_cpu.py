@@ -780,3 +780,39 @@ def test_no_cyclic_garbage_is_freed_during_a_capture():
         assert not gc.isenabled()
     finally:
         gc.enable()
+
+
+@pytest.mark.parametrize("head_dim,dtype,kv8,splits,used", [
+    (128, torch.bfloat16, False, 4, {300: 1, 1023: 1, 1024: 2, 1536: 3, 4096: 4}),   # merged in the launch: as many as the keys pay for
+    (128, torch.bfloat16, True, 4, {300: 1, 2048: 4}),
+    (64, torch.bfloat16, False, 1, {300: 1, 4096: 1}),                               # a second launch merges: what pays at any length
+    (64, torch.bfloat16, True, 4, {300: 4, 4096: 4}),                                # slow rows: always all of them
+    (128, torch.float32, False, 1, {300: 1}),
+])
+def test_captured_decode_steps_use_the_splits_that_their_keys_pay_for(monkeypatch, head_dim, dtype, kv8, splits, used):
+    """A captured step is planned at the model's context length; the chunk that a replay sets follows the batch in front of it."""
+    from types import SimpleNamespace
+
+    import cpu_ops
+    from sglang_custom_amd import ops_backend
+    from sglang_custom_amd.layers.attention.mi355_backend import Mi355AttnBackend
+    from sglang_custom_amd.mem_cache.memory_pool import MHATokenToKVPool, ReqToTokenPool
+    from sglang_custom_amd.model_executor.forward_batch_info import ForwardMode
+
+    monkeypatch.setattr(cpu_ops, "decode_split_plan", lambda bs, hkv, keys, most, fp8: (4, 1, 512) if keys >= 512 else (1, 1, 512))
+    ops_backend.set_ops_backend(cpu_ops)
+    try:
+        pool = MHATokenToKVPool(16, 1, torch.float8_e4m3fn if kv8 else dtype, 8, head_dim, 1, "cpu")
+        cfg = SimpleNamespace(num_attention_heads=32, num_key_value_heads=8, context_len=4096, head_dim=head_dim, v_head_dim=head_dim)
+        be = Mi355AttnBackend(SimpleNamespace(device="cpu", tp_size=1, req_to_token_pool=ReqToTokenPool(4, 8, "cpu"), token_to_kv_pool=pool,
+                                              model_config=cfg, sliding_window_size=None, attn_backend=None, dtype=dtype))
+        rows, lens = torch.zeros(2, dtype=torch.int64), torch.ones(2, dtype=torch.int64)
+        be.init_forward_metadata_capture_cuda_graph(2, 2, rows, lens, None, ForwardMode.DECODE, None)
+        assert be.forward_metadata.num_kv_splits == splits and (be.forward_metadata.kv_chunk_keys is not None) == (splits > 1)
+        for longest, n in used.items():
+            for cpu in (torch.tensor([5, longest]), None):
+                be.init_forward_metadata_replay_cuda_graph(2, rows, torch.tensor([5, longest]), 0, None, ForwardMode.DECODE, None, cpu)
+                if splits > 1:
+                    assert int(be._chunk_keys) == -(-longest // n), (longest, cpu)
+    finally:
+        ops_backend.set_ops_backend(None)

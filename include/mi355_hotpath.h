@@ -91,6 +91,8 @@ int mi355_prefetch_next(const void* w_packed, int64_t m, int64_t n, int64_t k, i
  *           silu_and_mul (sgl-kernel/csrc/elementwise/activation.cu:22-50). */
 int mi355_silu_and_mul(void* out, const void* x, int64_t rows, int64_t d, int dtype,
                        void* stream);
+/* The same for the listed rows alone: out[r] from x[r] for r = row_list[0 .. rows) (null: 0 .. rows). */
+int mi355_silu_and_mul_rows(void* out, const void* x, const int32_t* row_list, int64_t rows, int64_t d, int dtype, void* stream);
 
 /* ---- K12 epilogue: final-logit soft cap ---------------------------------------------------
  * logits[i] <- cap * tanh(logits[i] / cap), in place on n contiguous fp32 values, cap > 0.

@@ -586,7 +586,7 @@ def gatarax_stream_kernels(s: dict, tokens: int, segments: int) -> dict:
     plan = ops.moe_align(ids, E, wide_ok=True, tiled_ok=tokens > 64)
     gu_w = (torch.randn(E, 2 * ff, D, device=dev, generator=g) * D ** -0.5).to(dt)
     up = gu_w[:, :ff].contiguous()
-    t1 = _timed(lambda: ops.silu_and_mul(ops.moe_grouped_linear(h, gu_w, plan, gather=True, gelu=False)), 5)
+    t1 = _timed(lambda: ops.silu_and_mul_rows(ops.moe_grouped_linear(h, gu_w, plan, gather=True, gelu=False), plan.rows), 5)
     t2 = _timed(lambda: ops.moe_grouped_linear(h, up, plan, gather=True, gelu=True), 5)
     fl = tokens * top * 2 * ff * D
     res["moe_block_rows"] = plan.block

@@ -82,7 +82,7 @@ class GroupedExperts(nn.Module):
         if self.activation == "clamped_glu":
             a = self.act(ops.moe_grouped_linear(h, self.w_up.data, plan, gather=True, gelu=False), plan.rows, input_weights)
         elif self.activation == "silu_gated":
-            a = ops.silu_and_mul(ops.moe_grouped_linear(h, self.w_up.data, plan, gather=True, gelu=False))
+            a = ops.silu_and_mul_rows(ops.moe_grouped_linear(h, self.w_up.data, plan, gather=True, gelu=False), plan.rows)
         else:
             a = ops.moe_grouped_linear(h, self.w_up.data, plan, gather=True, gelu=self.activation == "gelu_erf",
                                        **({"relu2": True} if self.activation == "relu2" else {}))

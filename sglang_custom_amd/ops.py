@@ -126,6 +126,18 @@ def silu_and_mul(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.T
     return out
 
 
+def silu_and_mul_rows(x: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
+    """silu_and_mul of the rows x[r], r in `rows` (int32), alone; the other rows of the result are left unwritten."""
+    _gpu(x, rows)
+    assert x.dim() == 2 and x.is_contiguous() and x.shape[1] % 2 == 0 and rows.dtype == torch.int32 and rows.is_contiguous()
+    d = x.shape[1] // 2
+    out = torch.empty((x.shape[0], d), dtype=x.dtype, device=x.device)
+    if rows.numel():
+        check(_lib_().mi355_silu_and_mul_rows(out.data_ptr(), x.data_ptr(), rows.data_ptr(), rows.numel(), d, _dt(x), _stream(x)),
+              "silu_and_mul_rows")
+    return out
+
+
 def softcap_inplace(logits: torch.Tensor, cap: float) -> torch.Tensor:
     """fused_softcap(full_logits, final_logit_softcapping) (logits_processor.py:607-618): in place,
     fp32, logits <- cap * tanh(logits / cap)."""

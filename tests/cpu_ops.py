@@ -32,6 +32,13 @@ def silu_and_mul(x, out=None):
     return out
 
 
+def silu_and_mul_rows(x, rows):
+    out = torch.full((x.shape[0], x.shape[1] // 2), float("nan"), dtype=x.dtype)     # a row that nobody lists must not be read
+    todo = rows.reshape(-1).long()
+    out[todo] = ops_ref.silu_and_mul(x[todo])
+    return out
+
+
 def softcap_inplace(logits, cap):
     logits.copy_(ops_ref.softcap(logits, cap))
     return logits

@@ -78,3 +78,21 @@ def test_narrow_products_in_fp32(ops, T, N, K, off, dtype):
     assert ((got - want).abs() <= ulp * want.abs() + 8 * K ** 0.5 * 2.0 ** -24 * ((xd ** 2) @ (wd ** 2).T).sqrt() + 1e-12).all()
     if dtype != torch.float32:
         assert torch.equal(got, got.bfloat16().double())
+
+
+@pytest.mark.parametrize("d", [8, 192, 20, 7])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gated_unit_of_listed_rows(ops, d, dtype):
+    """The listed rows get the bits that the launch over every row gives them, whatever the others hold; the rest stays unwritten."""
+    g = torch.Generator().manual_seed(d)
+    x = torch.randn(70, 2 * d, generator=g).to(dtype).to(DEV)
+    rows = torch.randperm(70, generator=g)[:24].reshape(8, 3).int()
+    others = torch.ones(70, dtype=torch.bool)
+    others[rows.flatten().long()] = False
+    want, listed = ops.silu_and_mul(x), rows.to(DEV)
+    x[others] = float("nan")
+    out = torch.full((70, d), 3.0, dtype=dtype, device=DEV)
+    ops.check(ops._lib_().mi355_silu_and_mul_rows(out.data_ptr(), x.data_ptr(), listed.data_ptr(), 24, d, ops._dt(x), ops._stream(x)), "rows")
+    got = ops.silu_and_mul_rows(x, listed)
+    torch.cuda.synchronize()
+    assert torch.equal(out[~others], want[~others]) and (out[others] == 3.0).all() and torch.equal(got[~others], want[~others])

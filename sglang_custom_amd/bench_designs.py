@@ -375,8 +375,8 @@ def verozen_ff_and_stream_kernels(s: dict, tokens: int) -> dict:
     ids, wts = ops.moe_route_grouped(logits, corr, top, s["groups"], s["keep"], 1.0)
     t = _timed(lambda: ops.moe_route_grouped(logits, corr, top, s["groups"], s["keep"], 1.0), 10)
     res["moe_route_grouped"] = dict(us=round(t * 1e6, 1))
-    plan = ops.moe_align(ids, E, wide_ok=True, tiled_ok=tokens > 64)
-    t = _timed(lambda: ops.moe_align(ids, E, wide_ok=True, tiled_ok=tokens > 64), 10)
+    plan = ops.moe_align(ids, E, wide_ok=True, tiled_ok=True, columns=(ff, D))
+    t = _timed(lambda: ops.moe_align(ids, E, wide_ok=True, tiled_ok=True, columns=(ff, D)), 10)
     res["moe_align"] = dict(us=round(t * 1e6, 1))
     a = ops.moe_grouped_linear(h, up, plan, gather=True, gelu=True)
     t1 = _timed(lambda: ops.moe_grouped_linear(h, up, plan, gather=True, gelu=True), 5)
@@ -583,7 +583,7 @@ def gatarax_stream_kernels(s: dict, tokens: int, segments: int) -> dict:
     t = _timed(lambda: ops.moe_route_scores(torch.zeros(tokens, E, device=dev), None, top, s["groups"], s["keep"], 1.0, score_fn="softmax",
                                             group_best=1, renorm=False), 10)
     res["moe_route_scores (softmax; with the fill of its input)"] = dict(us=round(t * 1e6, 1))
-    plan = ops.moe_align(ids, E, wide_ok=True, tiled_ok=tokens > 64)
+    plan = ops.moe_align(ids, E, wide_ok=True, tiled_ok=True, columns=(2 * ff, D))
     gu_w = (torch.randn(E, 2 * ff, D, device=dev, generator=g) * D ** -0.5).to(dt)
     up = gu_w[:, :ff].contiguous()
     t1 = _timed(lambda: ops.silu_and_mul_rows(ops.moe_grouped_linear(h, gu_w, plan, gather=True, gelu=False), plan.rows), 5)

@@ -78,7 +78,8 @@ class GroupedExperts(nn.Module):
         plan = ops.moe_align(expert_ids, self.num_experts, wide_ok=sixteen and self.hidden % 8 == 0 and self.ff % 8 == 0,
                              tiled_ok=sixteen and h.stride(0) % 8 == 0
                              and ops.linear_tiled_supported(256, self.w_up.shape[1], self.hidden, h.dtype)
-                             and ops.linear_tiled_supported(256, self.hidden, self.ff, h.dtype))
+                             and ops.linear_tiled_supported(256, self.hidden, self.ff, h.dtype),
+                             columns=(self.w_up.shape[1], self.hidden))
         if self.activation == "clamped_glu":
             a = self.act(ops.moe_grouped_linear(h, self.w_up.data, plan, gather=True, gelu=False), plan.rows, input_weights)
         elif self.activation == "silu_gated":

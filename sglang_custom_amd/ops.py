@@ -7,7 +7,7 @@ is used for memory and streams only.  Outputs are allocated by the caller or ret
 mirroring sgl-kernel/python/sgl_kernel/{elementwise,sampling}.py.
 """
 import ctypes
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -1619,17 +1619,33 @@ def moe_router_logits(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def moe_align(expert_ids: torch.Tensor, num_experts: int, wide_ok: bool = False, tiled_ok: bool = False) -> MoePlan:
+def moe_block_class(pairs: int, num_experts: int, wide_ok: bool, tiled_ok: bool, columns: Sequence[int] = ()) -> int:
+    """0, 1, 2: blocks of 64, 128, 256 sorted rows (mi355_moe_block_rows) for `pairs` (token, expert) pairs.
+
+    Blocks of 256 rows run on the prefill projection kernel, which does no work for the rows a block does not have but takes a whole
+    CU per 256 x 256 tile: they win where the layer's products (`columns`: their widths; empty: not asked) are 256 such tiles, one
+    round of the chip, or 96 of them when the experts have 64 rows each, a second block of the smaller kernel.  A layer of gated
+    experts, both products and the activation, us with blocks of 64 / of 256 (tiles; bracket: taken): 32 experts of 2048 x 2048, 4
+    per token, 4 tokens 134 / [112] (384), 8 tokens 194 / [175] (768), 64 tokens 306 / [232]; 8 of 2048 x 4096, 2 per token, 2 tokens
+    [98] / 106 (160), 4 tokens 164 / [145] (320); 16 of 1024 x 1024, 2 per token, 8 to 256 tokens [49..58] / 57..61 (192), 512 tokens
+    92 / [64]; 8 of 512 x 512, 2 per token, 512 tokens [41] / 50 (48).  Blocks of 128 are used, where those are not, from two of them
+    per expert on.  (Sorted rows, and with them the scratch between the products, are as many as the worst case may need: pairs and a
+    block less one for every expert.)"""
+    if tiled_ok and 2 * pairs >= num_experts:
+        tiles = max(min(num_experts, pairs), pairs // 256) * sum(-(-n // 256) for n in columns)
+        if not columns or tiles >= 256 or (tiles >= 96 and pairs >= 64 * num_experts) or pairs >= 512 * num_experts:
+            return 2
+    return 1 if (wide_ok or tiled_ok) and pairs >= 256 * num_experts else 0
+
+
+def moe_align(expert_ids: torch.Tensor, num_experts: int, wide_ok: bool = False, tiled_ok: bool = False, columns: Sequence[int] = ()) -> MoePlan:
     """wide_ok: the grouped GEMMs that follow can take blocks of 128 rows (16-bit operands, 16-byte rows); tiled_ok: they
-    can run on the prefill projection kernel over blocks of 256 rows (linear_tiled_supported for both of them), which does
-    no work for the rows a block does not have and wins from half a row per expert on (one
-    GEMM of 32 experts of 2048 x 2048, 4 per token, in us against blocks of 64: 1 token 44 / 29, 4 tokens 48 / 45, 16: 53 / 82,
-    64: 55 / 91, 1024: 72 / 306; 64 experts of 1536 x 4096, 8 per token: 4 tokens 89 / 120, 64: 205 / 280).  Blocks of 128 are used, where those cannot be,
-    when the experts have at least two of them worth of rows on average."""
+    can run on the prefill projection kernel over blocks of 256 rows (linear_tiled_supported for both of them); columns: the
+    widths of their results.  moe_block_class chooses."""
     _gpu(expert_ids)
     T, top = expert_ids.shape
     assert expert_ids.dtype == torch.int32 and expert_ids.is_contiguous()
-    wide = 2 if (tiled_ok and 2 * T * top >= num_experts) else 1 if (wide_ok and T * top >= 256 * num_experts) else 0
+    wide = moe_block_class(T * top, num_experts, wide_ok, tiled_ok, columns)
     block = int(_lib_().mi355_moe_block_rows(wide))
     pairs = T * top
     padded = (pairs + min(num_experts, pairs) * (block - 1) + block - 1) // block * block

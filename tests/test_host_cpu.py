@@ -816,3 +816,18 @@ def test_captured_decode_steps_use_the_splits_that_their_keys_pay_for(monkeypatc
                     assert int(be._chunk_keys) == -(-longest // n), (longest, cpu)
     finally:
         ops_backend.set_ops_backend(None)
+
+
+@pytest.mark.parametrize("pairs,experts,columns,block", [
+    (8, 32, (2048, 2048), 0), (16, 32, (2048, 2048), 2), (256, 32, (2048, 2048), 2),              # half a row an expert; 256 tiles
+    (4, 8, (8192, 2048), 0), (8, 8, (8192, 2048), 2), (8, 8, (4096, 2048), 0), (512, 8, (4096, 2048), 2),
+    (512, 16, (2048, 1024), 0), (1023, 16, (2048, 1024), 0), (1024, 16, (2048, 1024), 2),         # 192 tiles: from 64 rows an expert on
+    (1024, 8, (1024, 512), 0), (2048, 8, (1024, 512), 1), (4096, 8, (1024, 512), 2),              # narrow experts: as many rows as fill it
+    (16, 32, (), 2), (15, 32, (), 0),
+])
+def test_expert_block_class(pairs, experts, columns, block):
+    from sglang_custom_amd import ops
+
+    assert ops.moe_block_class(pairs, experts, True, True, columns) == block
+    assert ops.moe_block_class(pairs, experts, True, False, columns) == (1 if pairs >= 256 * experts else 0)
+    assert ops.moe_block_class(pairs, experts, False, False, columns) == 0

@@ -826,6 +826,11 @@ int mi355_moe_align(int32_t* src_row, int32_t* rows, int32_t* tile_expert, int32
 int mi355_moe_grouped_linear(void* out, const void* in, int64_t in_stride, const void* weight, const int32_t* src_row,
                              const int32_t* tile_expert, const int32_t* n_tiles, int gather, int act, int64_t padded, int block,
                              int n, int k, int dtype, void* stream);
+/* The same for a caller that knows how many pairs of how many experts the rows hold (0, 0: it does not): blocks of 256 rows are
+ * computed by a kernel for mostly full or for mostly empty ones, with the same results. */
+int mi355_moe_grouped_linear_sized(void* out, const void* in, int64_t in_stride, const void* weight, const int32_t* src_row,
+                                   const int32_t* tile_expert, const int32_t* n_tiles, int gather, int act, int64_t padded, int block,
+                                   int n, int k, int dtype, int64_t pairs, int num_experts, void* stream);
 
 /* mi355_moe_route_scores: the same selection with its choices spelled out: score_fn 0 = sigmoid, 1 = softmax over all
  *   experts; correction may be null; a group scores the sum of its group_best (1 or 2) largest selection scores;

@@ -126,6 +126,7 @@ _SIGNATURES = {
     "mi355_moe_router_logits": (I, [P, P, P, L, I, I, P]),
     "mi355_moe_align": (I, [P, P, P, P, P, L, I, I, I, L, P]),
     "mi355_moe_grouped_linear": (I, [P, P, L, P, P, P, P, I, I, L, I, I, I, I, P]),
+    "mi355_moe_grouped_linear_sized": (I, [P, P, L, P, P, P, P, I, I, L, I, I, I, I, L, I, P]),
     "mi355_moe_route_scores": (I, [P, P, P, P, L, I, I, I, I, F, I, I, I, P]),
     "mi355_offset_rmsnorm": (I, [P, P, P, L, L, F, F, I, P]),
     "mi355_branch_residual_add": (I, [P, P, L, P, P, L, P, F, P, L, P, P, I, L, L, F, I, P]),

@@ -201,7 +201,11 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x
   }
 }
 
-template <typename T, int EPI, bool FP8>
+// MIXED (EPI 3): tiles without padding are as likely as tiles with; a wave whose rows are all there then takes a loop without the
+// conditions that leave padding out.  Those cost a full tile 5 %, the second loop a mostly empty one 3 to 6 (32 experts of 2048 x
+// 2048, 4 per token, both products: 8192 tokens 663 -> 624 us with it, 3000 297 -> 288, 1024 193 -> 197; 256 of 2048 x 512, 8 per
+// token, 64 tokens 304 -> 322).
+template <typename T, int EPI, bool FP8, bool MIXED>
 __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   extern __shared__ __attribute__((aligned(16))) char sm[];
   using frag = typename Mfma<T>::frag;
@@ -336,12 +340,12 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const int nA = EPI == 3 && g == 1 ? min(max((live - 128 - wc * 32 + 7) >> 3, 0), 4) : 4;
   const int nB = EPI == 3 && g == 1 ? min(max((live - wc * 32 + 7) >> 3, 0), 4) : 4;
 // four 1-KiB pieces of one half-tile of tile `tl`; TAIL: nothing past the last tile
-#define GT_LOAD4(ptr, ldso, tl, TAIL, COUNT)                                                 \
+#define GT_LOAD4(ptr, ldso, tl, TAIL, PART, COUNT)                                           \
   do {                                                                                       \
     if (!(TAIL) || (tl) < T_) {                                                              \
       char* d_ = lds_w + (((tl) & 1) ? GT_STAGE : 0) + (ldso);                               \
       _Pragma("unroll") for (int i = 0; i < 4; ++i)                                          \
-          if (EPI != 3 || i < (COUNT)) glds16(ptr[i] + (int64_t)(tl) * 128, d_ + i * 1024);  \
+          if (!(PART) || i < (COUNT)) glds16(ptr[i] + (int64_t)(tl) * 128, d_ + i * 1024);   \
     }                                                                                        \
   } while (0)
 #define GT_SLOT_END()                                                                        \
@@ -350,12 +354,12 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     __builtin_amdgcn_s_barrier();                                                            \
     __builtin_amdgcn_sched_barrier(0);                                                       \
   } while (0)
-#define GT_TILE(t, TAIL)                                                                     \
+#define GT_TILE(t, TAIL, PART)                                                               \
   do {                                                                                       \
     const int cur_ = ((t) & 1) ? GT_STAGE : 0;                                               \
     /* READ slot: request the group's two half-tiles, read the fragments of the whole K tile t */ \
-    GT_LOAD4(ldA, ldA_l, (t) + 1, TAIL, nA);                                                 \
-    GT_LOAD4(ldB, ldB_l, (t) + ldB_d, TAIL, nB);                                             \
+    GT_LOAD4(ldA, ldA_l, (t) + 1, TAIL, PART, nA);                                           \
+    GT_LOAD4(ldB, ldB_l, (t) + ldB_d, TAIL, PART, nB);                                       \
     _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) {                                       \
       const int ro_ = rd0 ^ (FP8 ? (kk << 4) : (kk << 6));                                   \
       const char* ab_ = sm + cur_ + a_off + ro_;                                             \
@@ -363,7 +367,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
       _Pragma("unroll") for (int ni = 0; ni < 4; ++ni)                                       \
           bf[kk][ni] = *reinterpret_cast<const i32x4*>(bb_ + ni * 2048);                     \
       _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                       \
-          if (EPI != 3 || mi < live_mi) af[kk][mi] = *reinterpret_cast<const i32x4*>(ab_ + mi * 2048); \
+          if (!(PART) || mi < live_mi) af[kk][mi] = *reinterpret_cast<const i32x4*>(ab_ + mi * 2048); \
     }                                                                                        \
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                       \
     GT_SLOT_END();                                                                           \
@@ -380,7 +384,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     } else {                                                                                 \
       _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                       \
         _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                     \
-          if (EPI != 3 || mi < live_mi)                                                      \
+          if (!(PART) || mi < live_mi)                                                       \
           _Pragma("unroll") for (int ni = 0; ni < 4; ++ni)                                   \
               acc[mi][ni] = Mfma<T>::run(__builtin_bit_cast(frag, bf[kk][ni]),               \
                                          __builtin_bit_cast(frag, af[kk][mi]), acc[mi][ni]); \
@@ -394,8 +398,13 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   GT_SLOT_END();
   if (g == 1) GT_SLOT_END();   // the second group runs one slot behind the first
   int t = 0;
-  for (; t + 2 < T_; ++t) GT_TILE(t, false);   // every request exists: no conditions in the loop
-  for (; t < T_; ++t) GT_TILE(t, true);
+  if (EPI == 3 && (!MIXED || live_mi < 8 || nA < 4 || nB < 4)) {   // (per wave; the barriers are as many either way)
+    for (; t + 2 < T_; ++t) GT_TILE(t, false, true);
+    for (; t < T_; ++t) GT_TILE(t, true, true);
+  } else {
+    for (; t + 2 < T_; ++t) GT_TILE(t, false, false);   // every request exists: no conditions in the loop
+    for (; t < T_; ++t) GT_TILE(t, true, false);
+  }
   if (g == 0) __builtin_amdgcn_s_barrier();
 #undef GT_LOAD4
 #undef GT_SLOT_END
@@ -481,9 +490,9 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   }
 }
 
-template <typename T, int EPI, bool FP8>
+template <typename T, int EPI, bool FP8, bool MIXED = false>
 int launch_gemm_tiled(const GemmTiledParams& p, hipStream_t st) {
-  auto kern = gemm_tiled_kernel<T, EPI, FP8>;
+  auto kern = gemm_tiled_kernel<T, EPI, FP8, MIXED>;
   (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS);
   // 8 x 4 blocks, or tiles, in equal numbers for every XCD
   const int per = EPI == 3 ? (p.nsuper + 7) / 8 * 32 : (int)cdiv((int64_t)p.mt * p.nt, 8);
@@ -542,10 +551,10 @@ extern "C" int mi355_linear_tiled(void* y, const void* x, const void* w, const v
 }
 
 namespace mi355 {
-// row_map says which rows are padding, and where the others come from if `gather` is set
+// row_map says which rows are padding, and where the others come from if `gather` is set; `mixed`: see the kernel
 int moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const void* w, const int32_t* row_map, int gather,
                              const int32_t* tile_expert, const int32_t* tiles_used, int act, int64_t rows, int64_t n, int64_t k,
-                             int dtype, void* stream) {
+                             int dtype, bool mixed, void* stream) {
   MI355_REQUIRE(y && x && w && tile_expert && tiles_used, MI355_ERR_INVALID, "mi355_moe_grouped_linear_tiled: null pointer");
   MI355_REQUIRE(rows > 0 && rows % 256 == 0 && mi355_linear_tiled_supported(rows, n, k, dtype, 0), MI355_ERR_UNSUPPORTED,
                 "mi355_moe_grouped_linear_tiled: needs whole 256-row tiles, a 16-bit dtype, K %% 64 == 0, K >= 128, N %% 16 == 0 "
@@ -560,6 +569,7 @@ int moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const voi
   fill_tiles(p, rows, n, 0);
   p.row_map = row_map; p.gather = gather; p.tile_expert = tile_expert; p.tiles_used = tiles_used; p.w_expert_stride = n * k; p.act = act;
   hipStream_t st = (hipStream_t)stream;
+  if (mixed) return dtype == MI355_BF16 ? launch_gemm_tiled<bf16_t, 3, false, true>(p, st) : launch_gemm_tiled<f16_t, 3, false, true>(p, st);
   return dtype == MI355_BF16 ? launch_gemm_tiled<bf16_t, 3, false>(p, st) : launch_gemm_tiled<f16_t, 3, false>(p, st);
 }
 }  // namespace mi355
@@ -567,7 +577,8 @@ int moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const voi
 extern "C" int mi355_moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const void* w, const int32_t* row_map,
                                               const int32_t* tile_expert, const int32_t* tiles_used, int act, int64_t rows,
                                               int64_t n, int64_t k, int dtype, void* stream) {
-  return moe_grouped_linear_tiled(y, x, x_stride, w, row_map, row_map != nullptr, tile_expert, tiles_used, act, rows, n, k, dtype, stream);
+  return moe_grouped_linear_tiled(y, x, x_stride, w, row_map, row_map != nullptr, tile_expert, tiles_used, act, rows, n, k, dtype, true,
+                                  stream);
 }
 
 extern "C" int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out_dtype, int epilogue) {

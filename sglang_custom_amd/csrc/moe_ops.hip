@@ -17,7 +17,7 @@
 namespace mi355 {
 int moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const void* w, const int32_t* row_map, int gather,
                              const int32_t* tile_expert, const int32_t* tiles_used, int act, int64_t rows, int64_t n, int64_t k,
-                             int dtype, void* stream);   // gemm_tiled.hip
+                             int dtype, bool mixed, void* stream);   // gemm_tiled.hip
 
 namespace {
 
@@ -598,10 +598,19 @@ int mi355_moe_align(int32_t* src_row, int32_t* rows, int32_t* tile_expert, int32
 int mi355_moe_grouped_linear(void* out, const void* in, int64_t in_stride, const void* weight, const int32_t* src_row,
                              const int32_t* tile_expert, const int32_t* n_tiles, int gather, int act, int64_t padded, int block,
                              int n, int k, int dtype, void* stream) {
+  return mi355_moe_grouped_linear_sized(out, in, in_stride, weight, src_row, tile_expert, n_tiles, gather, act, padded, block, n, k, dtype,
+                                        0, 0, stream);
+}
+
+int mi355_moe_grouped_linear_sized(void* out, const void* in, int64_t in_stride, const void* weight, const int32_t* src_row,
+                             const int32_t* tile_expert, const int32_t* n_tiles, int gather, int act, int64_t padded, int block,
+                             int n, int k, int dtype, int64_t pairs, int num_experts, void* stream) {
   MI355_REQUIRE(out && in && weight && src_row && tile_expert && n_tiles, MI355_ERR_INVALID, "moe_grouped_linear: null pointer");
   MI355_REQUIRE(act >= 0 && act <= 2, MI355_ERR_INVALID, "moe_grouped_linear: activation %d", act);
   if (block == MOE_TILED)
-    return moe_grouped_linear_tiled(out, in, in_stride, weight, src_row, gather, tile_expert, n_tiles, act, padded, n, k, dtype, stream);
+    // half the blocks are full from 256 rows per expert on; where that is not known they may be
+    return moe_grouped_linear_tiled(out, in, in_stride, weight, src_row, gather, tile_expert, n_tiles, act, padded, n, k, dtype,
+                                    pairs >= 256 * (int64_t)num_experts, stream);
   MI355_REQUIRE(block == MOE_BLOCK || block == MOE_WIDE, MI355_ERR_INVALID, "moe_grouped_linear: blocks of %d or %d rows", MOE_BLOCK,
                 MOE_WIDE);
   MI355_REQUIRE(padded >= 0 && padded % block == 0 && n > 0 && k > 0 && in_stride >= k && padded / block <= 65535,

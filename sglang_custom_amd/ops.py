@@ -1668,9 +1668,9 @@ def moe_grouped_linear(x: torch.Tensor, w: torch.Tensor, plan: MoePlan, gather: 
     assert w.is_contiguous() and x.dim() == 2 and x.shape[1] == K and x.stride(1) == 1 and x.dtype == w.dtype
     assert gather or x.shape[0] == plan.padded
     out = torch.empty((plan.padded, N), dtype=x.dtype, device=x.device)
-    check(_lib_().mi355_moe_grouped_linear(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), plan.src_row.data_ptr(),
-                                           plan.tile_expert.data_ptr(), plan.n_tiles.data_ptr(), int(gather), 2 if relu2 else int(gelu),
-                                           plan.padded, plan.block, N, K, _dt(x), _stream(x)), "moe_grouped_linear")
+    check(_lib_().mi355_moe_grouped_linear_sized(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), plan.src_row.data_ptr(),
+                                                 plan.tile_expert.data_ptr(), plan.n_tiles.data_ptr(), int(gather), 2 if relu2 else int(gelu),
+                                                 plan.padded, plan.block, N, K, _dt(x), plan.rows.numel(), E, _stream(x)), "moe_grouped_linear")
     return out
 
 

@@ -39,7 +39,7 @@ def test_align_sorts_every_pair_once(ops, T, E, top, block):
     assert (src[nt * block:] == -1).all()
 
 
-@pytest.mark.parametrize("sizes", [(0, 1, 8), (15, 16, 17), (127, 128, 129), (255, 256, 257), (500, 3, 300)])
+@pytest.mark.parametrize("sizes", [(0, 1, 8), (15, 16, 17), (127, 128, 129), (255, 256, 257), (500, 3, 300), (512, 241, 120)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_blocks_of_256_rows_skip_padding(ops, sizes, dtype):
     """An expert's last block at every edge of the 8-, 16- and 128-row pieces; both GEMMs.  One rounding of the float64 product

@@ -814,8 +814,8 @@ int mi355_moe_route_grouped(int32_t* ids, float* weights, const float* logits, c
                             int num_experts, int top, int n_groups, int keep_groups, float scale, void* stream);
 int mi355_moe_block_rows(int wide);
 /* The grouped GEMM over 256-row blocks on the prefill projection kernel (mi355_linear_tiled's): every 256-row tile of the
- * sorted rows multiplies weight[tile_expert[tile]]; row_map (null: identity) gathers the rows of x, negative entries (padding
- * behind a tile's rows) are not computed; tiles at or past
+ * sorted rows multiplies weight[tile_expert[tile]]; row_map (null: identity) gathers the rows of x, negative entries are
+ * padding: what their rows of y hold is undefined, and those behind a tile's last other row are not computed; tiles at or past
  * *tiles_used are skipped; act 1 = erf-GELU.  Same shape conditions as mi355_linear_tiled, rows a multiple of 256. */
 int mi355_moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const void* w, const int32_t* row_map,
                                    const int32_t* tile_expert, const int32_t* tiles_used, int act, int64_t rows, int64_t n,

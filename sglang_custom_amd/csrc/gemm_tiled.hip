@@ -63,7 +63,7 @@ struct GemmTiledParams {
   const void* loc;            // [M] cache slot of each row, int64 or int32
   int loc_i32;
   // EPI 3 (grouped: every 256-row tile of x multiplies the weight matrix of the tile's own expert)
-  const int32_t* row_map;      // [M] source row of x for output row m; negative: a padding row, behind its tile's others.  Null: none is
+  const int32_t* row_map;      // [M] source row of x for output row m; negative: a padding row.  Null: none is
   int gather;                  // whether row m reads row row_map[m] of x, or row m itself
   const int32_t* tile_expert;  // [mt] which of the stacked weight matrices tile tm uses
   const int32_t* tiles_used;   // device scalar: tiles at or past it are not computed
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     tm = band * 8 + r % rows;
     tn = col * 4 + r / rows;
   }
-  // EPI 3: rows of the tile that are no padding (they lie in front of it).  Padding rows are neither loaded, multiplied nor
+  // EPI 3: rows of the tile up to the last one that is no padding (a plan's padding lies behind them; between them it reads row 0).  Padding rows are neither loaded, multiplied nor
   // stored, 8, 16 and 1 at a time: an expert's last tile is as long as its rows.  64 tokens x 4 of 32 experts (2048 x 2048):
   // 88 us with padding worked on, 55 without (268 MB of weights); 1024 tokens: 85 and 72; 3000 tokens: 148 and 145.
   int live = 256;
@@ -245,7 +245,10 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     if (p.row_map != nullptr) {
       live = 0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) live += __popcll(__ballot(p.row_map[tm * 256 + i * 64 + lane] >= 0));
+      for (int i = 0; i < 4; ++i) {
+        const unsigned long long there = __ballot(p.row_map[tm * 256 + i * 64 + lane] >= 0);
+        live = there != 0 ? 64 * i + 64 - __clzll(there) : live;
+      }
       live = __builtin_amdgcn_readfirstlane(live);
     }
   }

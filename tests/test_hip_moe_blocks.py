@@ -96,3 +96,26 @@ def test_gated_unit_of_listed_rows(ops, d, dtype):
     got = ops.silu_and_mul_rows(x, listed)
     torch.cuda.synchronize()
     assert torch.equal(out[~others], want[~others]) and (out[others] == 3.0).all() and torch.equal(got[~others], want[~others])
+
+
+@pytest.mark.parametrize("holes", [(0, 5), (0, 200, 255), (100, 101, 254), tuple(range(0, 256, 2)), tuple(range(1, 256))])
+def test_padding_anywhere_in_a_tile(ops, holes):
+    """A caller's own row map may leave rows out in front of others (a plan of this library never does): the others are all there.
+    Small integers, so sums are exact."""
+    g = torch.Generator().manual_seed(len(holes))
+    K, N = 128, 272
+    x = torch.randint(-2, 3, (50, K), generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randint(-2, 3, (2, N, K), generator=g).to(torch.bfloat16).to(DEV)
+    rows = torch.randint(0, 50, (512,), generator=g).int()
+    rows[list(holes)] = -1
+    rows[256:400] = -1
+    te, used, rd = torch.tensor([1, 0], dtype=torch.int32, device=DEV), torch.tensor([2], dtype=torch.int32, device=DEV), rows.to(DEV)
+    y = torch.full((512, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.check(ops._lib_().mi355_moe_grouped_linear_tiled(y.data_ptr(), x.data_ptr(), K, w.data_ptr(), rd.data_ptr(), te.data_ptr(), used.data_ptr(),
+                                                         0, 512, N, K, ops._dt(x), ops._stream(x)), "tiled")
+    torch.cuda.synchronize()
+    for tile, e in ((0, 1), (1, 0)):
+        r = rows[256 * tile: 256 * tile + 256]
+        keep = r >= 0
+        want = (x.float()[r[keep].long().to(DEV)] @ w[e].float().T).to(torch.bfloat16)
+        assert torch.equal(y[256 * tile: 256 * tile + 256][keep.to(DEV)], want)

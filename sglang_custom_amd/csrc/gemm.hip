@@ -867,14 +867,19 @@ template <typename T>
 bool project_mfma_ok(const void* x, int64_t x_stride, const void* w, int64_t k) {
   return k % PjMma<T>::PER == 0 && x_stride % PjMma<T>::PER == 0 && aligned16(x) && aligned16(w);
 }
+constexpr int64_t PROJECT_FEW = 256;
 template <typename T, bool ROUND>
 void launch_project_mfma(float* out, const void* x, int64_t x_stride, const void* w, int64_t rows, int n, int k, hipStream_t st) {
   const unsigned gx = (unsigned)cdiv(rows, 16);
+  // Wider groups of columns read x once for more of them, but are fewer workgroups, each with NT chains to walk: they pay where
+  // the rows alone fill the chip.  bf16 rows x 64 columns x 2048, us at 1 / 4 tiles of 16 columns a workgroup: 1 row 4.4 / 9.5, 64
+  // rows 5.8 / 11.1, 1000 rows 6.2 / 11.2; 32 columns at 1 / 2: 1000 rows 5.9 / 7.7.
+  const bool one = n <= 16 || (int64_t)gx * cdiv(n, 16) <= PROJECT_FEW, two = n <= 32 || (int64_t)gx * cdiv(n, 32) <= PROJECT_FEW;
 #define MI355_PJ(NT)                                                                                                              \
   hipLaunchKernelGGL((project_f32_mfma_kernel<T, NT, ROUND>), dim3(gx, (unsigned)cdiv(n, 16 * NT)), dim3(64 * PJ_WAVES), 0, st, out,     \
                      (const T*)x, x_stride, (const T*)w, rows, n, k)
-  if (n <= 16) MI355_PJ(1);
-  else if (n <= 32) MI355_PJ(2);
+  if (one) MI355_PJ(1);
+  else if (two) MI355_PJ(2);
   else MI355_PJ(4);
 #undef MI355_PJ
 }

@@ -784,7 +784,7 @@ static void launch_skinny(const T* x, const T* w, const T* bias, OUT* y, void* w
 // product and sum.)  A workgroup takes 16 rows x 16 NT columns; its eight waves walk every eighth step of 32 (fp32:
 // 16) of K on the matrix cores and meet in LDS, in a fixed order whatever the number of rows.
 // The 64 x 64 vector-ALU tiles of gemm_tiled_kernel leave most of a tile empty at such widths and are a handful of
-// workgroups each walking all of K: 3000 fp32 rows x 32 columns x 2048 took 250 us, 7400 bf16 rows x 32 x 2048 took 187 us;
+// workgroups each walking all of K: 3000 fp32 rows x 32 columns x 2048 took 250 us, 7400 bf16 rows x 32 x 2048 took 165 us;
 // here 14 and 14 us, bound by reading x (25 and 30 MB).
 constexpr int PJ_WAVES = 8;
 template <typename T> struct PjMma {
@@ -886,8 +886,9 @@ void launch_project_mfma(float* out, const void* x, int64_t x_stride, const void
 
 // Columns up to which mi355_linear takes the kernel above for fp32 results without a bias (more rows than the skinny
 // kernels serve).  Every 64 columns read x again, from L2: 7400 rows x K 2048 in us, this / the 64 x 64 tiles: bf16 32 columns
-// 14 / 165, 256: 72 / 238, 512: 131 / 320; fp32 32: 25 / 239, 256: 147 / 289, 512: 270 / 350, where the lines are about to meet.
-constexpr int64_t PROJECT_MAX_N = 512;
+// 14 / 165, 256: 72 / 238, 512: 131 / 320; fp32 32: 25 / 239, 256: 147 / 289, 512: 270 / 350.  fp32 rows that fill the chip with
+// tiles have met the line before: 16384 rows, 320 columns 359 / 379, 512: 571 / 534.
+constexpr int64_t PROJECT_MAX_N = 512, PROJECT_MAX_N_TALL = 320;
 
 template <typename T, typename OUT>
 static void launch_linear_t(void* y, const void* x, const void* w, const void* bias, int64_t m,
@@ -901,7 +902,7 @@ static void launch_linear_t(void* y, const void* x, const void* w, const void* b
     }
   }
   if constexpr (std::is_same<OUT, float>::value) {
-    if (bias == nullptr && n <= PROJECT_MAX_N && project_mfma_ok<T>(x, x_stride, w, k)) {
+    if (bias == nullptr && n <= (sizeof(T) == 4 && m > 8192 ? PROJECT_MAX_N_TALL : PROJECT_MAX_N) && project_mfma_ok<T>(x, x_stride, w, k)) {
       launch_project_mfma<T, true>((float*)y, x, x_stride, w, m, (int)n, (int)k, st);
       return;
     }

@@ -63,7 +63,8 @@ def test_blocks_of_256_rows_skip_padding(ops, sizes, dtype):
     assert ((b.double() - want).abs() <= ulp * want.abs() + 1e-5 * 16).all()
 
 
-@pytest.mark.parametrize("T,N,K,off", [(65, 1, 8, 0), (100, 16, 2048, 0), (257, 33, 200, 0), (300, 512, 264, 8), (1000, 5, 4, 0), (70, 513, 64, 0), (90, 40, 37, 0)])
+@pytest.mark.parametrize("T,N,K,off", [(65, 1, 8, 0), (100, 16, 2048, 0), (257, 33, 200, 0), (300, 512, 264, 8), (1000, 5, 4, 0), (70, 513, 64, 0), (90, 40, 37, 0),
+                                       (2100, 100, 64, 0), (4100, 24, 64, 0), (4100, 64, 64, 0), (8200, 320, 64, 0), (8200, 321, 64, 0)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_narrow_products_in_fp32(ops, T, N, K, off, dtype):
     """fp32 results of mi355_linear on both sides of the narrow kernel's conditions.  Each of K terms and partial sums rounds once in

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void head_norm_rope_vec_kernel(
     float eps, float rot_mag) {
   __shared__ float cs[PNV_MAX];
   const int64_t t = blockIdx.x;
-  const int c = threadIdx.x & (lanes - 1), first = threadIdx.x / lanes, step = blockDim.x / lanes;
+  const int per = blockDim.x / lanes, c = threadIdx.x & (lanes - 1), first = blockIdx.y * per + threadIdx.x / lanes, step = gridDim.y * per;
   const bool live = 8 * c < d;
   if (rot_dims > 0) token_angles(cs, positions[t], inv_freq, rot_dims / 2, rot_mag);
   const int64_t orow = loc != nullptr ? loc[t] : t;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void qkv_norm_rope_write_vec_kernel(
     float eps, float rot_mag) {
   __shared__ float cs[PNV_MAX];
   const int64_t t = blockIdx.x;
-  const int c = threadIdx.x & (lanes - 1), first = threadIdx.x / lanes, step = blockDim.x / lanes;
+  const int per = blockDim.x / lanes, c = threadIdx.x & (lanes - 1), first = blockIdx.y * per + threadIdx.x / lanes, step = gridDim.y * per;
   if (rot_dims > 0) token_angles(cs, positions[t], inv_freq, rot_dims / 2, rot_mag);
   const int64_t slot = loc[t] * kv_heads;
   for (int u = first; u < heads + 2 * kv_heads; u += step) {
@@ -315,6 +315,15 @@ int pnv_lanes(int width) {
   return lanes;
 }
 unsigned pnv_threads(int units, int lanes) { return (unsigned)std::min(256, (units * lanes + 63) / 64 * 64); }
+// Workgroups that share one token's rows.  One alone computes the angles once but goes through the rows in turn: 256 tokens x 24
+// heads of 128 with 12 key and value heads 6.6 us, in as many workgroups as the rows fill 4.5; 16 tokens 5.0 and 4.1; 768: 7.6 and
+// 6.9; 1024: even; 2048: 11.7 and 12.8.
+unsigned pnv_parts(int64_t tokens, int units, int lanes) { return tokens < 1024 ? (unsigned)std::min(64, (units * lanes + 255) / 256) : 1u; }
+// Few narrow rows take the form with a wave per row, whose angles, loads and sums wait for nothing but each other: 16 tokens x 4
+// heads of 64 3.6 us against 4.0, 256 x 4 3.7 and 4.0, 1024 x 4 4.3 and 4.0, 256 x 16 4.3 and 3.9.  So does a single head, which
+// fills few lanes here: 8192 tokens of 64 features 5.3 us and 6.2, of 128 5.8 and 6.4.  At 128 features and more the row in
+// lanes is no slower for a single token (8 heads of 128: a wave per row 4.1 us, here 3.7).
+bool pnv_pays(int64_t tokens, int units, int width) { return units * width > 128 && (width >= 128 || tokens * units * width >= 196608); }
 bool pnv_rotation(int rot_dims, int interleaved) { return rot_dims % (interleaved ? 8 : 16) == 0; }
 bool pnv_aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -893,12 +902,13 @@ int mi355_head_norm_rope_mag(void* out, const void* src, const void* weight, con
   const bool vec = dtype != MI355_F32 && head_dim % 8 == 0 && head_dim <= PNV_MAX && pnv_rotation(rot_dims, interleaved) &&
                    pnv_aligned(out) && pnv_aligned(src) && pnv_aligned(weight) && tokens < ((int64_t)1 << 31) &&
                    ((src_token_stride | src_head_stride) & 7) == 0 &&
-                   ((out_token_stride | out_head_stride) & (out_dtype == MI355_F32 ? 3 : 7)) == 0;
+                   ((out_token_stride | out_head_stride) & (out_dtype == MI355_F32 ? 3 : 7)) == 0 &&
+                   pnv_pays(tokens, heads, head_dim);
   const int lanes = pnv_lanes(head_dim);
   MI355_DISPATCH_DTYPE(dtype, "head_norm_rope", {
     if constexpr (sizeof(T) == 2) {
       if (vec) {
-        const dim3 g2((unsigned)tokens), b2(pnv_threads(heads, lanes));
+        const dim3 b2(pnv_threads(heads, lanes)), g2((unsigned)tokens, pnv_parts(tokens, heads, lanes));
         if (out_dtype == dtype)
           hipLaunchKernelGGL((head_norm_rope_vec_kernel<T, T>), g2, b2, 0, (hipStream_t)stream, (T*)out, (const T*)src, (const T*)weight,
                              positions, loc, inv_freq, heads, head_dim, lanes, src_token_stride, src_head_stride, out_token_stride,
@@ -943,8 +953,11 @@ int mi355_head_rmsnorm_gate_wide(void* out, const float* o, const void* weight, 
                 "head_rmsnorm_gate: bad shape");
   if (tokens == 0) return MI355_OK;
   const unsigned grid = (unsigned)((tokens * heads + 3) / 4);
+  // whole 16-byte pieces; few narrow rows are sooner done by a wave each, one feature a lane (64 tokens x 4 heads of 64 3.2 us
+  // against 3.5, 64 x 24 heads of 128 3.7 and 3.8; 512 x 16 heads of 64 4.5 and 3.7)
   const bool vec = dtype != MI355_F32 && value_dim % 8 == 0 && value_dim <= PNV_MAX && pnv_aligned(out) && pnv_aligned(o) &&
-                   pnv_aligned(weight) && pnv_aligned(gate) && (gate_stride & 7) == 0;
+                   pnv_aligned(weight) && pnv_aligned(gate) && (gate_stride & 7) == 0 &&
+                   (value_dim > 128 || tokens * heads * value_dim >= 262144);
   MI355_DISPATCH_DTYPE(dtype, "head_rmsnorm_gate", {
     if constexpr (sizeof(T) == 2) {
       if (vec) {
@@ -981,12 +994,13 @@ int mi355_qkv_norm_rope_write(void* q_out, void* k_cache, void* v_cache, const v
   const bool vec = dtype != MI355_F32 && head_dim % 8 == 0 && v_head_dim % 8 == 0 && std::max(head_dim, v_head_dim) <= PNV_MAX &&
                    pnv_rotation(rot_dims, interleaved) && pnv_aligned(q_out) && pnv_aligned(k_cache) && pnv_aligned(v_cache) &&
                    pnv_aligned(q) && pnv_aligned(k) && pnv_aligned(v) && pnv_aligned(wq) && pnv_aligned(wk) &&
-                   ((q_token_stride | k_token_stride | v_token_stride) & 7) == 0 && tokens < ((int64_t)1 << 31);
-  const int lanes = pnv_lanes(std::max(head_dim, v_head_dim));
+                   ((q_token_stride | k_token_stride | v_token_stride) & 7) == 0 && tokens < ((int64_t)1 << 31) &&
+                   pnv_pays(tokens, heads + 2 * kv_heads, std::max(head_dim, v_head_dim));
+  const int lanes = pnv_lanes(std::max(head_dim, v_head_dim)), units = heads + 2 * kv_heads;
   MI355_DISPATCH_DTYPE(dtype, "qkv_norm_rope_write", {
     if constexpr (sizeof(T) == 2) {
       if (vec) {
-        hipLaunchKernelGGL((qkv_norm_rope_write_vec_kernel<T>), dim3((unsigned)tokens), dim3(pnv_threads(heads + 2 * kv_heads, lanes)), 0,
+        hipLaunchKernelGGL((qkv_norm_rope_write_vec_kernel<T>), dim3((unsigned)tokens, pnv_parts(tokens, units, lanes)), dim3(pnv_threads(units, lanes)), 0,
                            (hipStream_t)stream, (T*)q_out, (T*)k_cache, (T*)v_cache, (const T*)q, (const T*)k, (const T*)v, q_token_stride,
                            k_token_stride, v_token_stride, (const T*)wq, (const T*)wk, positions, loc, inv_freq, heads, kv_heads, head_dim,
                            v_head_dim, lanes, rot_dims, interleaved, eps, rot_mag);

@@ -37,15 +37,17 @@ def _close(got, want, size, what):
 
 
 # (d, dv, rot, interleaved): one lane a row; idle lanes in a row (24, 96); the widest; one past it and a rotation that is no
-# multiple of a piece (the form for any width)
+# multiple of a piece (the form for any width); 37 tokens, and as many as lead rows narrower than 128 and more than one pass of a
+# token's rows through a workgroup there
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("d,dv,rot,interleaved", [(8, 8, 8, True), (24, 16, 16, False), (64, 128, 64, False), (96, 64, 48, False), (128, 96, 64, True),
-                                                  (512, 256, 512, False), (128, 128, 0, False), (520, 64, 16, False), (64, 64, 20, False), (60, 64, 16, True)])
-def test_norm_rotate_and_write(dt, d, dv, rot, interleaved):
+@pytest.mark.parametrize("T,d,dv,rot,interleaved", [(2300, 8, 8, 8, True), (600, 24, 16, 16, False), (300, 64, 64, 64, False), (200, 96, 64, 48, False),
+                                                    (1030, 128, 96, 64, True), (1030, 64, 512, 64, False)] + [(37, *c) for c in [(8, 8, 8, True), (24, 16, 16, False), (64, 128, 64, False), (96, 64, 48, False), (128, 96, 64, True),
+                                                  (512, 256, 512, False), (128, 128, 0, False), (520, 64, 16, False), (64, 64, 20, False), (60, 64, 16, True)]])
+def test_norm_rotate_and_write(dt, T, d, dv, rot, interleaved):
     from sglang_custom_amd import ops
 
     g = torch.Generator().manual_seed(d + dv + rot)
-    T, H, G, eps, mag = 37, 5, 3, 1e-5, 1.25
+    H, G, eps, mag = 5, 3, 1e-5, 1.25
     rows = torch.randn(T, (H + G) * d + G * dv, generator=g).to(dt).to(DEV)
     q, k, v = rows[:, : H * d].view(T, H, d), rows[:, H * d: (H + G) * d].view(T, G, d), rows[:, (H + G) * d:].view(T, G, dv)
     wq, wk = (torch.randn(2, d, generator=g) + 1).to(dt).to(DEV)
@@ -70,7 +72,7 @@ def test_norm_rotate_and_write(dt, d, dv, rot, interleaved):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T,H,dv,pad", [(37, 5, 8, 0), (37, 3, 96, 8), (5, 4, 128, 1), (9, 2, 512, 0), (9, 1, 520, 0), (7, 3, 36, 0)])
+@pytest.mark.parametrize("T,H,dv,pad", [(37, 5, 8, 0), (37, 3, 96, 8), (5, 4, 128, 1), (9, 2, 512, 0), (9, 1, 520, 0), (7, 3, 36, 0), (6600, 5, 8, 0), (1000, 3, 96, 8), (600, 4, 128, 1), (600, 4, 128, 8)])
 def test_norm_and_gate(dt, T, H, dv, pad):
     from sglang_custom_amd import ops
 

@@ -806,8 +806,12 @@ int mi355_sigmoid_attention(void* out, const void* q, const void* k_cache, const
  *   smaller index); weights[t][k] = s[chosen] / (sum of the chosen s + 1e-20) * scale.
  * mi355_moe_router_logits: out[t][j] = x[t] . weight[j] in exact fp32 for few rows (one workgroup per row; k <= 16384).
  * mi355_moe_align: sorts the tokens * top (token, choice) pairs by expert into blocks of `block` rows
- *   (mi355_moe_block_rows(0), or mi355_moe_block_rows(1) for prefill-sized steps of 16-bit models) of one expert each: src_row[p] = token of sorted row p or -1 (padding), rows[pair] = p, tile_expert[block] = its expert,
+ *   of one expert each: src_row[p] = token of sorted row p or -1 (padding), rows[pair] = p, tile_expert[block] = its expert,
  *   *n_tiles = blocks in use.  `padded` (a multiple of the block) must be at least pairs + min(experts, pairs) * (block - 1).
+ *   Blocks of mi355_moe_block_rows(0) = 64 rows serve every dtype and width; of (1) = 128 rows 16-bit operands whose rows are 16-byte
+ *   pieces, from about 256 pairs per expert on; of (2) = 256 rows 16-bit products that mi355_linear_tiled_supported takes.  These do
+ *   no work for padding rows but occupy a CU per 256 x 256 tile of the result: they pay where the products fill the chip with such
+ *   tiles, down to half a pair per expert.
  * mi355_moe_grouped_linear: out[p][.] = act(weight[tile_expert[p / block]] . in[gather ? src_row[p] : p]) for every sorted
  *   row p of a block in use (0 for padding rows, which blocks of 256 rows leave unwritten); weight [experts, n, k]; act: 0 nothing, 1 erf-GELU, 2 the square of relu. */
 int mi355_moe_route_grouped(int32_t* ids, float* weights, const float* logits, const float* correction, int64_t tokens,

@@ -1528,14 +1528,6 @@ __device__ __forceinline__ void load_to_lds_16_s(uint64_t base, unsigned lane_of
         : "memory");
 }
 
-// max of a value over the lanes that differ in bit 16 or 32 of their number, in registers: swapping a register with its own
-// copy leaves one half's values in all lanes of the first result and the other half's in the second
-template <int X> __device__ __forceinline__ float max_xor(float v) {
-  const unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
-}
-
 // One 4-byte load per active lane to LDS at `lds_base` (wave-uniform) + 4 * lane.
 __device__ __forceinline__ void load_to_lds_4_v(const void* src, unsigned lds_base) {
   unsigned keep;

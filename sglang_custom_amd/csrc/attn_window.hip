@@ -241,17 +241,11 @@ __global__ __launch_bounds__(256) void window_attention_merge_kernel(T* __restri
 // What bounds it: the vector ALU (about 90 operations per lane and tile beside 16 MFMAs at d = dv = 128).  7381 prefill tokens
 // of 16 heads over 4, d = 128, window 512 and averaged blocks of 64 (37 GFLOP): 116 us; 273 with S = Q K^T, where a row's
 // scores lay in 16 lanes, its weights and factor went through LDS and the waves shared the result columns (three barriers).
+// Single tokens of 4 heads a key head are one live wave, whose chain is shorter too: 1 / 64 / 256 tokens x 2000 keys, same heads and
+// window, 22 / 31 / 66 us against 31 / 41 / 131.
 // sm: 2 x (Ks [32][d + 8] | Vs [32][dv + 8])   (all T)
 constexpr int WAM_ROWS = 64;
 constexpr int WAM_MAX = 256;     // d and dv
-
-// max over the lanes that differ in bit 16 or 32 of their number, in registers: a register swapped with its own copy holds one
-// half's values in all lanes of the first result and the other half's in the second
-template <int X> __device__ __forceinline__ float wa_max_xor(float v) {
-  const unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
-}
 
 template <typename T, int CT, int CK>
 __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
@@ -378,8 +372,8 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
       x8[i] = seen[i] ? s[i >> 2][i & 3] * a.scale : WA_NEG;
       mx = fmaxf(mx, x8[i]);
     }
-    mx = wa_max_xor<16>(mx);
-    mx = wa_max_xor<32>(mx);
+    mx = max_xor<16>(mx);
+    mx = max_xor<32>(mx);
     const float alpha = __expf(run_m - mx);
     run_m = mx;
     Vec<T, 8> p8;      // key slots 8 lg + i of the product with V: the keys above, in that order

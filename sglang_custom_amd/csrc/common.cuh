@@ -74,6 +74,14 @@ template <typename V> __device__ __forceinline__ void lds_store2(void* p, const 
 // Elements per 16-byte access.
 template <typename T> struct V16 { static constexpr int n = 16 / sizeof(T); };
 
+// max of a value over the lanes that differ in bit 16 or 32 of their number, in registers: swapping a register with its own
+// copy leaves one half's values in all lanes of the first result and the other half's in the second
+template <int X> __device__ __forceinline__ float max_xor(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+}
+
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);

@@ -236,8 +236,8 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     tm = band * 8 + r % rows;
     tn = col * 4 + r / rows;
   }
-  // EPI 3: rows of the tile up to the last one that is no padding (a plan's padding lies behind them; between them it reads row 0).  Padding rows are neither loaded, multiplied nor
-  // stored, 8, 16 and 1 at a time: an expert's last tile is as long as its rows.  64 tokens x 4 of 32 experts (2048 x 2048):
+  // EPI 3: rows of the tile up to the last one that is no padding (a plan's padding lies behind them; between them it reads row 0).
+  // Padding rows are neither loaded, multiplied nor stored, 8, 16 and 1 at a time: an expert's last tile is as long as its rows.  64 tokens x 4 of 32 experts (2048 x 2048):
   // 88 us with padding worked on, 55 without (268 MB of weights); 1024 tokens: 85 and 72; 3000 tokens: 148 and 145.
   int live = 256;
   if constexpr (EPI == 3) {

@@ -533,10 +533,8 @@ __global__ __launch_bounds__(256) void qkv_rotate_write_kernel(
   }
 }
 
-// One workgroup per (token, part): out = N(y * silu(gate)) * w over one of `groups` equal consecutive parts of the row, the
-// gate applied BEFORE the norm.  y fp32 [tokens, D] contiguous, gate T row-strided, w T [D].  A part of up to 2048 features
-// keeps its gated values in registers between the two passes.
-constexpr int GGN_KEEP = 8;
+// out = N(y * silu(gate)) * w over one of `groups` equal consecutive parts of the row, the gate applied BEFORE the norm.  y fp32
+// [tokens, D] contiguous, gate T row-strided, w T [D].
 // Groups of at most 512 features in 16-bit results: `lanes` lanes hold a group, eight features each.  7381 tokens x 4 groups
 // of 512: 50 -> 25 us (floor 24); a workgroup per group moved two features a thread.
 template <typename T>
@@ -572,6 +570,8 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_vec_kernel(T* __restr
   stvec<T, 8>(out + idx * n + 8 * c, res);
 }
 
+// Any other part: one workgroup per (token, part), which keeps up to 2048 gated values in registers between the two passes.
+constexpr int GGN_KEEP = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(T* __restrict__ out, const float* __restrict__ y,
                                                                   const T* __restrict__ gate, int64_t gate_stride,
@@ -613,10 +613,9 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(T* __restrict_
   }
 }
 
-// One wave per (token, head): out = o / rms(o) (* w) * silu(gate), or * sigmoid(gate) with gate_act 1; w [dv] shared by the heads,
-// or (w_per_head) [heads, dv]
-// the same for 16-bit results, eight features per lane and `lanes` lanes a row: the fp32 row and the gate come once, in 16-byte
-// pieces.  7381 tokens x 16 heads of 128: 53 -> 27 us (floor 24).
+// out = o / rms(o) (* w) * silu(gate), or * sigmoid(gate) with gate_act 1; w [dv] shared by the heads,
+// or (w_per_head) [heads, dv].
+// For 16-bit results, eight features per lane and `lanes` lanes a row: the fp32 row and the gate come once, in 16-byte 7381 tokens x 16 heads of 128: 53 -> 27 us (floor 24).
 template <typename T>
 __global__ __launch_bounds__(256) void head_rmsnorm_gate_vec_kernel(T* __restrict__ out, const float* __restrict__ o, const T* __restrict__ w,
                                                                     const T* __restrict__ gate, int64_t gate_stride, int64_t rows, int heads,
@@ -651,6 +650,7 @@ __global__ __launch_bounds__(256) void head_rmsnorm_gate_vec_kernel(T* __restric
   stvec<T, 8>(out + idx * dv + 8 * c, res);
 }
 
+// Any other row, and few narrow ones: one wave per (token, head).
 template <typename T>
 __global__ __launch_bounds__(256) void head_rmsnorm_gate_kernel(T* __restrict__ out, const float* __restrict__ o,
                                                                 const T* __restrict__ w, const T* __restrict__ gate,

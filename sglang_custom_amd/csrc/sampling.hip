@@ -176,8 +176,8 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_temperature_kernel(
 
 // The same over chunks of a row, in two launches: every chunk leaves its maximum and its sum of exponentials, then
 // every chunk normalises itself with what all of them left.  (A chunk without a number in it has no maximum to take off: its
-// -inf entries count zero and a NaN makes its sum NaN, and with it the row, as one pass over the row has it.)  One workgroup per row reads its 0.5 MB three times with 4
-// bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
+// -inf entries count zero and a NaN makes its sum NaN, and with it the row, as one pass over the row has it.)  One workgroup per
+// row reads its 0.5 MB three times with 4 bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
 // 18 + 16 us (33 MB read twice, the second time from L2, then read and written), bound by the precise division and
 // exponential of every entry in both.
 struct ChunkSpan {
@@ -231,7 +231,10 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
   const ChunkSpan sp = chunk_span(vocab, c, chunks);
   const float t = temperatures[r];
   float mx = -INFINITY, sum = 0.f;
-  constexpr int KEEP = 8;   // 16-byte pieces a thread holds: chunks up to 32 K entries (every vocabulary up to 512 K at few rows)
+  // 16-byte pieces a thread holds: chunks up to 32 K entries, every vocabulary up to 512 K at few rows.  More rows have fewer and longer
+  // chunks (row_chunks), which go through span_each twice: both launches at 128256 entries, 64 rows (4 chunks) 41 us, 86 (3) 73, 200 (2)
+  // 116; a whole row a workgroup 157, 163, 182.
+  constexpr int KEEP = 8;
   if (vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS) {
     // The chunk is read once, all of it requested before anything is used, and divided once: 64 rows x 128256 entries
     // 14.1 us (floor 7); 17.8 with two passes of one piece at a time.

@@ -673,6 +673,15 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const T* r_lin = LATENT ? (const T*)p.k_rope + (int64_t)(q_start + srow2) * p.k_rope_stride + sch2 * 8
                           : k_ext + (int64_t)(q_start - prefix + srow2) * p.k_stride + (int64_t)kvh * DQ + 128 + sch2 * 8;
   const int64_t r_stride = LATENT ? p.k_rope_stride : p.k_stride;
+  // Cache slots of the thread's rows of the next tile, read a tile ahead: otherwise every wave stands at the head of its tile for the
+  // slots before it can request the rows behind them.  32 / 8 heads, us a launch: 4 x 490 tokens on 1750 cached 165 -> 131, 6 x 500
+  // on 2900 278 -> 209, 1 x 65 on 3000 106 -> 82; without a prefix as before.
+  int32_t next_slot[4];
+  auto load_slots = [&](int kt) {
+    if (kt * 64 >= prefix) return;   // (workgroup-uniform)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) next_slot[i] = p.kv_indices[kv_start + min(kt * 64 + srow + 16 * i, prefix - 1)];
+  };
   auto load_tile = [&](int kt) {
     if (kt * 64 >= prefix && kt * 64 + 63 < total) {   // whole tile in the extend part (workgroup-uniform)
 #pragma unroll
@@ -704,7 +713,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
       int key = kt * 64 + srow + 16 * i;
       key = key < total ? key : total - 1;
       if (KV8 && key < prefix) {
-        const int64_t slot_ = p.kv_indices[kv_start + key];
+        const int64_t slot_ = next_slot[i];
         const uint8_t* kp8 = reinterpret_cast<const uint8_t*>(kbuf) + slot_ * p.kb_slot + kvh * p.kb_head + sch * 8;
         const uint8_t* vp8 = reinterpret_cast<const uint8_t*>(vbuf) + slot_ * p.vb_slot + kvh * p.vb_head + sch * 8;
         kreg[i] = cvt8_from_fp8<T>(*reinterpret_cast<const uint2*>(kp8));
@@ -713,7 +722,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
       }
       const T *kp, *vp;
       if (key < prefix) {
-        const int64_t slot_ = p.kv_indices[kv_start + key];
+        const int64_t slot_ = next_slot[i];
         kp = kbuf + slot_ * p.kb_slot + kvh * p.kb_head;
         vp = vbuf + slot_ * p.vb_slot + kvh * p.vb_head;
       } else {
@@ -768,12 +777,15 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const int vch = 2 * dhalf + (tpp >> 1);                   // + 4 dt
   const char* v_rd = vs + 256 * vrow + 8 * (tpp & 1);
 
+  if (!LATENT) load_slots(0);
   load_tile(0);
+  if (!LATENT) load_slots(1);
   for (int kt = 0; kt < n_tiles; ++kt) {
     __syncthreads();            // previous tile fully consumed
     store_tile();
     __syncthreads();
     if (kt + 1 < n_tiles) load_tile(kt + 1);
+    if (!LATENT) load_slots(kt + 2);
     if (kt * 64 > wave_max_limit) continue;   // every key of the tile is masked for every query of this wave (wave-uniform)
 
     f32x16 st[2];

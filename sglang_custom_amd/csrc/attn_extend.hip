@@ -2,7 +2,7 @@
 // through kv_indices from the paged KV cache, and (2) the new tokens themselves (causal
 // triangle), with one online softmax across both phases.
 //
-// Structure: a workgroup (4 waves) owns a tile of 64 "rows" = TM query tokens x Gc query heads
+// Structure of the general kernel: a workgroup (4 waves) owns a tile of 64 "rows" = TM query tokens x Gc query heads
 // that share one kv head, so every K/V tile staged in LDS is reused by all heads of the group.
 // K/V tiles of BN keys are gathered with 16-byte loads into padded LDS rows (bank-conflict free
 // for the access patterns below).  Scores and P.V are register-blocked fp32 VALU FMAs (each lane
@@ -573,14 +573,20 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // LATENT: no cached prefix; the heads' keys (features 0 .. 127) and values come interleaved per token and head out of one
 // projection of the latent, the keys' features 128 .. 191 from one row per token that the heads share, and the queries'
 // features 128 .. 191 are rotated here, in fp32 and rounded to T, as the absorbed kernels do it.
-template <typename T, bool KV8, int DQ, bool LATENT = false>
+// D: value head dimension.  At 64 the rows of the tile images are half used (the XOR spreads their eight chunks over the whole
+// 256 bytes), and P.V takes the weights as the sum of two 16-bit numbers: the vector-ALU kernel that served this size multiplied
+// fp32 weights, and two terms leave an error of at most 2^-16 of a weight in bf16 (2^-22 in fp16), far below the output's own
+// rounding (against float64 1.6563e-3 of the norm in either kernel).
+template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128>
 __device__ __forceinline__ void extend_attn_mfma32_body(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs) {
-  constexpr int D = 128;          // value head dimension = width of one tile image
   constexpr int NS = DQ / 16;     // score k-steps
   constexpr bool WIDE = DQ > 128;
-  static_assert(DQ == 128 || (DQ == 192 && !KV8), "128, or 192 over a 16-bit cache");
+  constexpr bool PSPLIT = D == 64;
+  constexpr int CH = D / 8, SR = 256 / CH, NI = 64 / SR;   // 16-byte chunks of a row; rows staged at once, and how often
+  constexpr int ND = D / 32;      // 32-feature tiles of the output
+  static_assert((D == 128 && (DQ == 128 || (DQ == 192 && !KV8))) || (D == 64 && DQ == 64), "64, 128, or 192 + 128 over a 16-bit cache");
   using frag = typename Mfma32<T>::frag;
   __shared__ __attribute__((aligned(16))) char ks[64 * 256];
   __shared__ __attribute__((aligned(16))) char ks2[WIDE ? 64 * 256 : 16];
@@ -660,13 +666,13 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const int wave_min_limit = LATENT || p.is_causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
   const int wave_max_limit = LATENT || p.is_causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
 
-  // tile staging: thread -> rows (threadIdx.x >> 4) + 16 i, 16-B chunk (threadIdx.x & 15)
-  const int srow = threadIdx.x >> 4, sch = threadIdx.x & 15;
+  // tile staging: thread -> rows threadIdx.x / CH + SR i, 16-B chunk threadIdx.x % CH
+  const int srow = threadIdx.x / CH, sch = threadIdx.x % CH;
   // kreg2: chunk sch2 of features 128 and up of two of kreg's four rows, so that a paged row's slot is read once and every thread
   // has a part.  16 requests x 64 tokens on 2000 cached, 16 heads, 133 us, 2048 tokens on none 60; with rows of another deal,
   // whose slots are read again, 169 and 67; in the threads with sch < 8 alone 152 and 76.  LATENT, where these features are
   // rows of their own: eight neighbours a load (a whole step of Silatar 1 % less than in the first deal).
-  Vec<T, 8> kreg[4], vreg[4], kreg2[WIDE ? 2 : 1];
+  Vec<T, 8> kreg[NI], vreg[NI], kreg2[WIDE ? 2 : 1];
   const int odd2 = sch >> 3, sch2 = sch & 7, srow2 = LATENT ? threadIdx.x >> 3 : srow + 16 * odd2;   // rows srow2 + 32 j
   const T* k_lin = k_ext + (int64_t)(q_start - prefix + srow) * p.k_stride + (int64_t)kvh * (LATENT ? p.kv_head : DQ) + sch * 8;
   const T* v_lin = v_ext + (int64_t)(q_start - prefix + srow) * p.v_stride + (int64_t)kvh * (LATENT ? p.kv_head : D) + sch * 8;
@@ -676,17 +682,17 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   // Cache slots of the thread's rows of the next tile, read a tile ahead: otherwise every wave stands at the head of its tile for the
   // slots before it can request the rows behind them.  32 / 8 heads, us a launch: 4 x 490 tokens on 1750 cached 165 -> 131, 6 x 500
   // on 2900 278 -> 209, 1 x 65 on 3000 106 -> 82; without a prefix as before.
-  int32_t next_slot[4];
+  int32_t next_slot[NI];
   auto load_slots = [&](int kt) {
     if (kt * 64 >= prefix) return;   // (workgroup-uniform)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) next_slot[i] = p.kv_indices[kv_start + min(kt * 64 + srow + 16 * i, prefix - 1)];
+    for (int i = 0; i < NI; ++i) next_slot[i] = p.kv_indices[kv_start + min(kt * 64 + srow + SR * i, prefix - 1)];
   };
   auto load_tile = [&](int kt) {
     if (kt * 64 >= prefix && kt * 64 + 63 < total) {   // whole tile in the extend part (workgroup-uniform)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t key = kt * 64 + 16 * i;
+      for (int i = 0; i < NI; ++i) {
+        const int64_t key = kt * 64 + SR * i;
         kreg[i] = ldvec<T, 8>(k_lin + key * p.k_stride);
         vreg[i] = ldvec<T, 8>(v_lin + key * p.v_stride);
       }
@@ -709,8 +715,8 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     }
     const T* row2[WIDE ? 4 : 1];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int key = kt * 64 + srow + 16 * i;
+    for (int i = 0; i < NI; ++i) {
+      int key = kt * 64 + srow + SR * i;
       key = key < total ? key : total - 1;
       if (KV8 && key < prefix) {
         const int64_t slot_ = next_slot[i];
@@ -741,8 +747,8 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   };
   auto store_tile = [&]() {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int off = xor_image_off(srow + 16 * i, sch);
+    for (int i = 0; i < NI; ++i) {
+      const int off = xor_image_off(srow + SR * i, sch);
       *reinterpret_cast<Vec<T, 8>*>(ks + off) = kreg[i];
       *reinterpret_cast<Vec<T, 8>*>(vs + off) = vreg[i];
     }
@@ -752,9 +758,9 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     }
   };
 
-  f32x16 ot[4];
+  f32x16 ot[ND];
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
+  for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) ot[dt][i] = 0.f;
   float m = -INFINITY, lsum = 0.f;
@@ -805,7 +811,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     // the first V^T fragments too: the tile is already in LDS, and the softmax below covers their latency
     typename TrRead<T>::v4 vlo[4], vhi[4];   // ring of four (u, dt) fragments
     auto v_read = [&](int i, int slot_) {
-      const int u = i >> 2, dt = i & 3;
+      const int u = i / ND, dt = i % ND;
       const int ch = 4 * dt + vch;
       vlo[slot_] = TrRead<T>::run(reinterpret_cast<const T*>(v_rd + 256 * (16 * u) + 16 * (ch ^ vf_lo)));
       vhi[slot_] = TrRead<T>::run(reinterpret_cast<const T*>(v_rd + 256 * (16 * u + 8) + 16 * (ch ^ vf_hi)));
@@ -855,32 +861,35 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     const float alpha = raw_exp2(m - ms);
     m = mnew;
     float psum = 0.f;
-    frag pb[4];
+    frag pb[4], pl[PSPLIT ? 4 : 1];
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float pe = raw_exp2(__builtin_fmaf(st[hf][i], qmul, -ms));
         psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V
-        pb[2 * hf + (i >> 3)][i & 7] = (T)pe;
+        const T hi = (T)pe;
+        pb[2 * hf + (i >> 3)][i & 7] = hi;
+        if constexpr (PSPLIT) pl[2 * hf + (i >> 3)][i & 7] = (T)(pe - (float)hi);   // what the rounding left
       }
     lsum = lsum * alpha + psum;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt) ot[dt] *= alpha;
+      for (int dt = 0; dt < ND; ++dt) ot[dt] *= alpha;
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {   // (u, dt) = (i >> 2, i & 3); fragment i + 4 is requested right behind MFMA i
+    for (int i = 0; i < 4 * ND; ++i) {   // (u, dt) = (i / ND, i % ND); fragment i + 4 is requested right behind MFMA i
       frag va;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         va[e] = vlo[i & 3][e];
         va[4 + e] = vhi[i & 3][e];
       }
-      ot[i & 3] = Mfma32<T>::run(va, pb[i >> 2], ot[i & 3]);
+      ot[i % ND] = Mfma32<T>::run(va, pb[i / ND], ot[i % ND]);
+      if constexpr (PSPLIT) ot[i % ND] = Mfma32<T>::run(va, pl[i / ND], ot[i % ND]);
       __builtin_amdgcn_sched_barrier(0);
-      if (i + 4 < 16) {
+      if (i + 4 < 4 * ND) {
         v_read(i + 4, i & 3);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -892,7 +901,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     T* op = o_ext + ((int64_t)(q_start + qrow) * p.hq + h) * D + 4 * hh;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
         Vec<T, 4> w;
@@ -912,6 +921,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
   extend_attn_mfma32_body<T, KV8, 128>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
+}
+// Head dimension 64 needs 168 registers: three workgroups per CU.  Bound by the softmax's instructions (about ten per score beside
+// three quarters of an MFMA cycle).  32 / 8 heads in bf16, us a launch, vector-ALU kernel -> this one: 4 x 340 tokens on 1180 cached
+// 378 -> 57, 704 + 430 tokens on none 121 -> 21, 4000 on none 1493 -> 138, 65 on 3000 510 -> 74, 70 on none 24 -> 13; fp8 cache,
+// 3 x 197 on 1614 478 -> 69.  The heads of a group packed into the rows (less of the triangle's edge in vain) was no faster.
+template <typename T, bool KV8 = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void extend_attn_mfma32_d64_kernel(
+    const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
+    const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
+  extend_attn_mfma32_body<T, KV8, 64, false, 64>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
 }
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void extend_attn_mfma32_wide_kernel(
@@ -976,14 +995,23 @@ static int launch_extend(const void* q, const void* k, const void* v, void* o, c
                    p.k_stride % VE == 0 && p.v_stride % VE == 0 && aligned16(q) && aligned16(k) &&
                    aligned16(v) && aligned16(o) && aligned16(kb) && aligned16(vb);
   if constexpr (!std::is_same<T, float>::value) {
-    if (vec && (p.D == 128 || (p.D == 192 && !kv8)) && p.Dv == 128 && !p.custom_mask && p.sliding_window <= 0 &&
-        p.logit_cap <= 0.f && p.sm_scale > 0.f && g_extend_variant == 0) {   // the 32x32 kernel takes the maximum of unscaled scores
+    if (vec && ((p.D == 128 && p.Dv == 128) || (p.D == 192 && p.Dv == 128 && !kv8) || (p.D == 64 && p.Dv == 64)) && !p.custom_mask &&
+        p.sliding_window <= 0 && p.logit_cap <= 0.f && p.sm_scale > 0.f && g_extend_variant == 0) {   // the 32x32 kernel takes the maximum of unscaled scores
       // 128 query rows of one head per workgroup; (sequence, kv head) pairs dealt round-robin to the XCDs
       const int nqb = (int)((max_len_extend + 127) / 128);
       const int64_t npairs = bs * p.hkv;
       const int64_t wgs = 8 * ((npairs + 7) / 8) * (p.hq / p.hkv) * nqb;
       if (wgs < (int64_t)1 << 31) {
         const dim3 grid1((unsigned)wgs);
+        if (p.D == 64) {
+          if (kv8)
+            hipLaunchKernelGGL((extend_attn_mfma32_d64_kernel<T, true>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
+                               (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
+          else
+            hipLaunchKernelGGL((extend_attn_mfma32_d64_kernel<T, false>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
+                               (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
+          return MI355_OK;
+        }
         if (p.D == 192)
           hipLaunchKernelGGL((extend_attn_mfma32_wide_kernel<T>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
                              (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);

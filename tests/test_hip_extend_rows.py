@@ -15,7 +15,7 @@ def ops():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("kv8", [False, True], ids=["cache16", "cache_fp8"])
-@pytest.mark.parametrize("hq,hkv,d", [(6, 2, 128)])
+@pytest.mark.parametrize("hq,hkv,d", [(6, 2, 128), (6, 2, 64), (4, 4, 64)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_tile_edges_over_a_paged_prefix(ops, dtype, kv8, hq, hkv, d, causal):
     g = torch.Generator().manual_seed(hq * 100 + d)

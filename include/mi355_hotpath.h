@@ -517,6 +517,17 @@ int mi355_linear_tiled_supported(int64_t m, int64_t n, int64_t k, int dtype, int
 int mi355_linear_tiled(void* y, const void* x, const void* w, const void* bias, int64_t m, int64_t n,
                        int64_t k, int64_t x_stride, int dtype, int epilogue, void* stream);
 
+/* The tiled projections with scratch memory: output tiles beyond whole rounds of 256 may then be computed by several workgroups
+ * each, which share K and leave fp32 sums in the workspace; a second launch adds them in their order and finishes the tiles.
+ * mi355_tiled_tail_splits: into how many parts K is cut (0: not at all); mi355_tiled_tail_workspace_bytes: the memory that takes (0:
+ * none needed, and workspace may be NULL).  fp8 1: e4m3fn operands; epilogue as in the product (0 for the qkv projection, n its rows).
+ * A NULL workspace gives the product without splits.  Nothing of the workspace is read before it is written. */
+int mi355_tiled_tail_splits(int64_t m, int64_t n, int64_t k, int fp8, int epilogue);
+int64_t mi355_tiled_tail_workspace_bytes(int64_t m, int64_t n, int64_t k, int fp8, int epilogue);
+int mi355_linear_tiled_ws(void* y, const void* x, const void* w, const void* bias, int64_t m, int64_t n,
+                          int64_t k, int64_t x_stride, int dtype, int epilogue, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
 /* ---- K14 fp8 W8A8 ------------------------------------------------------------------------------
  * Per-token dynamic quantisation to OCP e4m3fn (max 448): s[r] = max(absmax(x[r,:]), 1e-10)/448,
  * q = clamp(x/s, +-448) -> fp8.  Row r of xq starts at byte r * q_stride (q_stride >= k); bytes k .. q_stride of
@@ -549,6 +560,9 @@ int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out
 int mi355_fp8_scaled_mm_tiled(void* y, const uint8_t* xq, const uint8_t* wq, const float* x_scale,
                               const float* w_scale, const void* bias, int64_t m, int64_t n, int64_t k,
                               int out_dtype, int epilogue, void* stream);
+int mi355_fp8_scaled_mm_tiled_ws(void* y, const uint8_t* xq, const uint8_t* wq, const float* x_scale,
+                                 const float* w_scale, const void* bias, int64_t m, int64_t n, int64_t k,
+                                 int out_dtype, int epilogue, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The qkv projection of a prefill batch with RoPE and the KV-cache write in the GEMM's epilogue:
  *   qkv = x @ w^T (w [(hq + 2 hkv) * 128, K], rows q | k | v), rounded to the dtype;
@@ -569,6 +583,12 @@ int mi355_qkv_proj_rope_tiled(void* qkv, const void* x, const void* w, const flo
                               int head_dim, const int64_t* positions, const void* cos_sin_cache,
                               int cache_dtype, int rotary_dim, int is_neox, void* k_buffer, void* v_buffer,
                               const void* loc, int loc_itype, int64_t num_slots, int dtype, void* stream);
+int mi355_qkv_proj_rope_tiled_ws(void* qkv, const void* x, const void* w, const float* x_scale,
+                              const float* w_scale, int64_t m, int64_t k, int64_t x_stride, int hq, int hkv,
+                              int head_dim, const int64_t* positions, const void* cos_sin_cache,
+                              int cache_dtype, int rotary_dim, int is_neox, void* k_buffer, void* v_buffer,
+                              const void* loc, int loc_itype, int64_t num_slots, int dtype, void* workspace, int64_t workspace_bytes,
+                                 void* stream);
 
 /* ---- K11 sampling --------------------------------------------------------------------------------
  * ids[b] = first index of max(logits[b,:])   (torch.argmax tie rule)

@@ -58,6 +58,11 @@ _SIGNATURES = {
     "mi355_linear_packed_silu_mul": (I, [P, P, P, L, L, L, L, P, L, I, P]),
     "mi355_linear_tiled_supported": (I, [L, L, L, I, I]),
     "mi355_linear_tiled": (I, [P, P, P, P, L, L, L, L, I, I, P]),
+    "mi355_linear_tiled_ws": (I, [P, P, P, P, L, L, L, L, I, I, P, L, P]),
+    "mi355_tiled_tail_splits": (I, [L, L, L, I, I]),
+    "mi355_tiled_tail_workspace_bytes": (L, [L, L, L, I, I]),
+    "mi355_fp8_scaled_mm_tiled_ws": (I, [P, P, P, P, P, P, L, L, L, I, I, P, L, P]),
+    "mi355_qkv_proj_rope_tiled_ws": (I, [P, P, P, P, P, L, L, L, I, I, I, P, P, I, I, I, P, P, P, I, L, I, P, L, P]),
     "mi355_fp8_scaled_mm_tiled_supported": (I, [L, L, L, I, I]),
     "mi355_fp8_scaled_mm_tiled": (I, [P, P, P, P, P, P, L, L, L, I, I, P]),
     "mi355_qkv_proj_rope_tiled_supported": (I, [L, L, I, I, I, I, I, I, I]),

@@ -30,7 +30,10 @@
 //     columns (or, for SiLU-and-mul, 8 gate columns and the 8 matching up columns): the epilogue
 //     writes whole 128-byte lines with 16-byte stores and needs no cross-lane traffic.
 //   * workgroup -> tile: consecutive workgroups round-robin over the 8 XCDs, so workgroups b and
-//     b + 8 share an L2; each XCD works through 8 x 4 blocks of tiles (32 CUs = one block).
+//     b + 8 share an L2; each XCD works through 8 x 4 blocks of tiles (32 CUs = one block);
+//   * tiles beyond whole rounds of 256 may be split over K, their sums added by a second launch that also runs the epilogue.
+// What bounds it: the card's power.  A K tile takes 2320 of the 2048 cycles that its MFMAs need (88 %), but with random operands the
+// clock falls to 1.7 GHz (4096 x 4096 x 4096: 98 us; with x = 0 2.17 GHz and 77).
 #include "common.cuh"
 
 namespace mi355 {
@@ -52,6 +55,9 @@ struct GemmTiledParams {
   int ldy;          // elements between rows of y
   int mt, nt;       // output tiles along M and N
   int snt, nsuper;  // 8 x 4 blocks of tiles: count along N, total
+  // tail tiles whose K is split over `splits` workgroups each (0: none): tiles at .. `full` - 1 in tile order are computed whole
+  int full, tail, splits;
+  float* part;      // [splits, tail, 8 waves, 8 row groups, 4 column groups, 64 lanes, 4] sums of the splits
   // EPI 2 (qkv projection + RoPE + KV-cache write)
   const int64_t* positions;   // [M]
   const void* cos_sin;        // [max_pos, 128]: cos | sin, fp32 or the tensor dtype
@@ -96,14 +102,13 @@ template <bool FP8> __device__ __forceinline__ int gt_swz(int r) {
 // partners d0 + 64 .. d0 + 71 (acc[mi][2..3]).  Every load (positions, cache slots, cos / sin rows) is
 // requested before the arithmetic of the rows it belongs to: nothing else runs on the CU during an epilogue,
 // so a chain of dependent loads per row would be paid in full.
-template <typename T, bool FP8, bool CSF32>
-__device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x4 (&acc)[8][4], const float (&sxm)[8],
-                                                  int tm, int tn, int g, int wc, int q4, int r16) {
+template <typename T, bool FP8, bool CSF32, int NM>
+__device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], const float (&sxm)[NM],
+                                                  int mbase, int tn, int wc, int q4) {
 #pragma clang fp contract(off)
   T* yg = (T*)p.y;
   const int head = 2 * tn + (wc >> 1), d0 = (wc & 1) * 32 + q4 * 8;
   const int col0 = head * 128 + d0;
-  const int mbase = tm * 256 + g * 128 + r16;
   const bool rot = head < p.hq + p.hkv;
   T* cache_dst = nullptr;
   if (head >= p.hq + p.hkv) cache_dst = (T*)p.v_buffer + (int64_t)(head - p.hq - p.hkv) * p.kv_head + d0;
@@ -114,9 +119,9 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x
     slo[j] = FP8 ? p.w_scale[col0 + j] : 1.f;
     shi[j] = FP8 ? p.w_scale[col0 + 64 + j] : 1.f;
   }
-  int posv[8], slotv[8];   // positions and slot numbers fit 31 bits (the host checks the slot count)
+  int posv[NM], slotv[NM];   // positions and slot numbers fit 31 bits (the host checks the slot count)
 #pragma unroll
-  for (int mi = 0; mi < 8; ++mi) {
+  for (int mi = 0; mi < NM; ++mi) {
     const int m = mbase + mi * 16;
     posv[mi] = (int)p.positions[m < p.M ? m : p.M - 1];
     slotv[mi] = 0;
@@ -124,21 +129,21 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x
   if (cache_dst != nullptr) {
     if (p.loc_i32) {
 #pragma unroll
-      for (int mi = 0; mi < 8; ++mi) {
+      for (int mi = 0; mi < NM; ++mi) {
         const int m = mbase + mi * 16;
         slotv[mi] = ((const int32_t*)p.loc)[m < p.M ? m : p.M - 1];
       }
     } else {
 #pragma unroll
-      for (int mi = 0; mi < 8; ++mi) {
+      for (int mi = 0; mi < NM; ++mi) {
         const int m = mbase + mi * 16;
         slotv[mi] = (int)((const int64_t*)p.loc)[m < p.M ? m : p.M - 1];
       }
     }
   }
-  constexpr int G = (CSF32 || FP8) ? 2 : 4;   // rows whose cos / sin are in flight together (register budget)
+  constexpr int G = NM < 4 ? NM : (CSF32 || FP8) ? 2 : 4;   // rows whose cos / sin are in flight together (register budget)
 #pragma unroll
-  for (int half = 0; half < 8 / G; ++half) {
+  for (int half = 0; half < NM / G; ++half) {
     // cos / sin of G rows (v heads read them too and ignore them: the branch below is wave-uniform)
     float c[G][8], sn[G][8];
 #pragma unroll
@@ -201,6 +206,99 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x
   }
 }
 
+// Tile number `at` of the tile order: bands of 8 rows of tiles, blocks of 4 columns inside.
+__device__ __forceinline__ void tile_of(const GemmTiledParams& p, int at, int& tm, int& tn) {
+  const int band = at / (8 * p.nt), in = at - band * 8 * p.nt;
+  const int rows = min(8, p.mt - 8 * band), col = in / (4 * rows), r = in - col * 4 * rows;
+  tm = band * 8 + r % rows;
+  tn = col * 4 + r / rows;
+}
+
+// The results of NM groups of 16 rows (row mbase + 16 mi + r16 is lane (q4, r16)'s in group mi; mbase: the first group's first row).
+// acc[mi][ni][r]: W slot 16 ni + 4 q4 + r of the wave's 64, which the load mapping made output column 16 q4 + 4 ni + r (plain) or
+// gate / up column 8 q4 + 4 (ni & 1) + r.  EPI 3: `live` rows of the tile are no padding.
+template <typename T, int EPI, bool FP8, int NM>
+__device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], int m0, int tm, int tn, int wc, int q4, int r16,
+                                              int live) {
+  const int ncols = EPI == 1 ? (p.N >> 1) : p.N;   // output columns
+  const int mbase = m0 + r16;
+  T* yg = (T*)p.y;
+  const T* bias = (const T*)p.bias;
+  float sxm[NM];
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi) {
+    const int m = mbase + mi * 16;
+    sxm[mi] = FP8 ? p.x_scale[m < p.M ? m : p.M - 1] : 1.f;
+  }
+  if constexpr (EPI == 2) {
+    if (p.cs_f32) qkv_rope_epilogue<T, FP8, true, NM>(p, acc, sxm, mbase, tn, wc, q4);
+    else qkv_rope_epilogue<T, FP8, false, NM>(p, acc, sxm, mbase, tn, wc, q4);
+  } else if (EPI == 1) {
+    const int j0 = tn * 128 + wc * 32 + q4 * 8;
+    if (j0 < ncols) {
+      float sg[8], su[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        sg[j] = FP8 ? p.w_scale[j0 + j] : 1.f;
+        su[j] = FP8 ? p.w_scale[ncols + j0 + j] : 1.f;
+      }
+#pragma unroll
+      for (int mi = 0; mi < NM; ++mi) {
+        const int m = mbase + mi * 16;
+        Vec<T, 8> o;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float gv = acc[mi][h][r], uv = acc[mi][2 + h][r];
+            if (FP8) { gv = (gv * sxm[mi]) * sg[h * 4 + r]; uv = (uv * sxm[mi]) * su[h * 4 + r]; }
+            o.v[h * 4 + r] = silu_mul_one<T>(from_f32<T>(gv), from_f32<T>(uv));
+          }
+        if (m < p.M) stvec<T, 8>(yg + (int64_t)m * p.ldy + j0, o);
+      }
+    }
+  } else {
+    const int n0 = tn * 256 + wc * 64 + q4 * 16;
+    if (n0 < p.N) {
+      float bv[16], sw[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) { bv[j] = 0.f; sw[j] = FP8 ? p.w_scale[n0 + j] : 1.f; }
+      if (bias != nullptr) {
+        const Vec<T, 8> b0 = ldvec<T, 8>(bias + n0), b1 = ldvec<T, 8>(bias + n0 + 8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { bv[j] = to_f32(b0.v[j]); bv[8 + j] = to_f32(b1.v[j]); }
+      }
+#pragma unroll
+      for (int mi = 0; mi < NM; ++mi) {
+        const int m = mbase + mi * 16;
+        Vec<T, 8> o0, o1;
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float v0 = acc[mi][ni][r], v1 = acc[mi][2 + ni][r];
+            if (FP8) { v0 = (v0 * sxm[mi]) * sw[ni * 4 + r]; v1 = (v1 * sxm[mi]) * sw[8 + ni * 4 + r]; }
+            if constexpr (EPI == 3) {
+              if (p.act == 1) {
+                v0 = 0.5f * v0 * (1.0f + erff(v0 * 0.7071067811865476f));
+                v1 = 0.5f * v1 * (1.0f + erff(v1 * 0.7071067811865476f));
+              } else if (p.act == 2) {
+                v0 = fmaxf(v0, 0.f); v0 *= v0;
+                v1 = fmaxf(v1, 0.f); v1 *= v1;
+              }
+            }
+            o0.v[ni * 4 + r] = from_f32<T>(v0 + bv[ni * 4 + r]);
+            o1.v[ni * 4 + r] = from_f32<T>(v1 + bv[8 + ni * 4 + r]);
+          }
+        if (EPI == 3 ? m - tm * 256 < live : m < p.M) {
+          stvec<T, 8>(yg + (int64_t)m * p.ldy + n0, o0);
+          stvec<T, 8>(yg + (int64_t)m * p.ldy + n0 + 8, o1);
+        }
+      }
+    }
+  }
+}
+
 // MIXED (EPI 3): tiles without padding are as likely as tiles with; a wave whose rows are all there then takes a loop without the
 // conditions that leave padding out.  Those cost a full tile 5 %, the second loop a mostly empty one 3 to 6 (32 experts of 2048 x
 // 2048, 4 per token, both products: 8192 tokens 663 -> 624 us with it, 3000 297 -> 288, 1024 193 -> 197; 256 of 2048 x 512, 8 per
@@ -220,7 +318,8 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   // whole blocks in turn left some XCDs a round more than others where the last band is short -- 18 x 24 tiles: 72 on two
   // XCDs and 40 on four, of 32 CUs each.  M = 4605, K = 4096: N = 6144 267 -> 190 us, N = 28672 846 -> 792; 7381 x 2048 -> 2 x 5632 302 -> 280.
   const int b = blockIdx.x, li = b >> 3;
-  int tm, tn;
+  int tm, tn, T_ = (p.K * ES) >> 7, t0 = 0;   // K tiles of 128 bytes per row, and the first one of a split
+  float* part = nullptr;
   if constexpr (EPI == 3) {
     const int st = (li >> 5) * 8 + (b & 7), within = li & 31;
     if (st >= p.nsuper) return;
@@ -228,13 +327,20 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     tm = sup_m * 8 + (within & 7);
     tn = sup_n * 4 + (within >> 3);
     if (tm >= p.mt || tn >= p.nt) return;
-  } else {
-    const int at = (b & 7) * (int)(gridDim.x >> 3) + li;
+  } else if (p.splits == 0 || b < p.full) {
+    const int at = (b & 7) * (p.splits == 0 ? (int)(gridDim.x >> 3) : p.full >> 3) + li;
     if (at >= p.mt * p.nt) return;
-    const int band = at / (8 * p.nt), in = at - band * 8 * p.nt;
-    const int rows = min(8, p.mt - 8 * band), col = in / (4 * rows), r = in - col * 4 * rows;
-    tm = band * 8 + r % rows;
-    tn = col * 4 + r / rows;
+    tile_of(p, at, tm, tn);
+  } else {
+    // a split of a tail tile; every XCD takes neighbouring splits, one stretch of K of all the tail's operands
+    const int u = b - p.full, at = (u & 7) * (int)((gridDim.x - p.full) >> 3) + (u >> 3);
+    if (at >= p.tail * p.splits) return;
+    const int k = at / p.tail, t = at - k * p.tail;
+    tile_of(p, p.full + t, tm, tn);
+    part = p.part + ((int64_t)k * p.tail + t) * 65536;
+    const int all = T_;
+    t0 = all * k / p.splits;
+    T_ = all * (k + 1) / p.splits - t0;
   }
   // EPI 3: rows of the tile up to the last one that is no padding (a plan's padding lies behind them; between them it reads row 0).
   // Padding rows are neither loaded, multiplied nor stored, 8, 16 and 1 at a time: an expert's last tile is as long as its rows.  64 tokens x 4 of 32 experts (2048 x 2048):
@@ -254,7 +360,6 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   }
   const int live_mi = EPI == 3 ? min(max((live - g * 128 + 15) >> 4, 0), 8) : 8;
 
-  const int T_ = (p.K * ES) >> 7;   // K tiles of 128 bytes per row
   const char* xg = (const char*)p.x;
   const char* wg = (const char*)p.w;
   if constexpr (EPI == 3) wg += (int64_t)p.tile_expert[tm] * p.w_expert_stride * ES;
@@ -304,8 +409,8 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
       }
       ws[h] = wg + ((int64_t)n * p.K) * ES + c * 16;
     }
-    ldA[i] = g == 0 ? ws[0] : xs[1];
-    ldB[i] = g == 0 ? ws[1] : xs[0];
+    ldA[i] = (g == 0 ? ws[0] : xs[1]) + (int64_t)t0 * 128;
+    ldB[i] = (g == 0 ? ws[1] : xs[0]) + (int64_t)t0 * 128;
   }
   // LDS image of a K tile: x rows 0..255 (two halves), then W rows 0..255 (two halves)
   constexpr int LX0 = 0, LX1 = GT_HALF, LW0 = 2 * GT_HALF, LW1 = 3 * GT_HALF;
@@ -414,83 +519,40 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
 #undef GT_TILE
 
   // ---- epilogue ---------------------------------------------------------------------------------
-  // acc[mi][ni][r]: row m = 16 mi + (lane & 15) of the wave's 128 rows; W slot 16 ni + 4 q4 + r, which
-  // the load mapping above made output column 16 q4 + 4 ni + r (plain) or gate/up column 8 q4 + 4 (ni & 1) + r.
-  T* yg = (T*)p.y;
-  const T* bias = (const T*)p.bias;
-  float sxm[8];
+  if constexpr (EPI != 3) {
+    if (part != nullptr) {   // a split of a tail tile: its sums as they lie in the registers
 #pragma unroll
-  for (int mi = 0; mi < 8; ++mi) {
-    const int m = tm * 256 + g * 128 + mi * 16 + r16;
-    sxm[mi] = FP8 ? p.x_scale[m < p.M ? m : p.M - 1] : 1.f;
-  }
-  if constexpr (EPI == 2) {
-    if (p.cs_f32) qkv_rope_epilogue<T, FP8, true>(p, acc, sxm, tm, tn, g, wc, q4, r16);
-    else qkv_rope_epilogue<T, FP8, false>(p, acc, sxm, tm, tn, g, wc, q4, r16);
-  } else if (EPI == 1) {
-    const int j0 = tn * 128 + wc * 32 + q4 * 8;
-    if (j0 < ncols) {
-      float sg[8], su[8];
+      for (int mi = 0; mi < 8; ++mi)
+        if (tm * 256 + g * 128 + mi * 16 < p.M)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        sg[j] = FP8 ? p.w_scale[j0 + j] : 1.f;
-        su[j] = FP8 ? p.w_scale[ncols + j0 + j] : 1.f;
-      }
-#pragma unroll
-      for (int mi = 0; mi < 8; ++mi) {
-        const int m = tm * 256 + g * 128 + mi * 16 + r16;
-        Vec<T, 8> o;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float gv = acc[mi][h][r], uv = acc[mi][2 + h][r];
-            if (FP8) { gv = (gv * sxm[mi]) * sg[h * 4 + r]; uv = (uv * sxm[mi]) * su[h * 4 + r]; }
-            o.v[h * 4 + r] = silu_mul_one<T>(from_f32<T>(gv), from_f32<T>(uv));
-          }
-        if (m < p.M) stvec<T, 8>(yg + (int64_t)m * p.ldy + j0, o);
-      }
-    }
-  } else {
-    const int n0 = tn * 256 + wc * 64 + q4 * 16;
-    if (n0 < p.N) {
-      float bv[16], sw[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) { bv[j] = 0.f; sw[j] = FP8 ? p.w_scale[n0 + j] : 1.f; }
-      if (bias != nullptr) {
-        const Vec<T, 8> b0 = ldvec<T, 8>(bias + n0), b1 = ldvec<T, 8>(bias + n0 + 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { bv[j] = to_f32(b0.v[j]); bv[8 + j] = to_f32(b1.v[j]); }
-      }
-#pragma unroll
-      for (int mi = 0; mi < 8; ++mi) {
-        const int m = tm * 256 + g * 128 + mi * 16 + r16;
-        Vec<T, 8> o0, o1;
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float v0 = acc[mi][ni][r], v1 = acc[mi][2 + ni][r];
-            if (FP8) { v0 = (v0 * sxm[mi]) * sw[ni * 4 + r]; v1 = (v1 * sxm[mi]) * sw[8 + ni * 4 + r]; }
-            if constexpr (EPI == 3) {
-              if (p.act == 1) {
-                v0 = 0.5f * v0 * (1.0f + erff(v0 * 0.7071067811865476f));
-                v1 = 0.5f * v1 * (1.0f + erff(v1 * 0.7071067811865476f));
-              } else if (p.act == 2) {
-                v0 = fmaxf(v0, 0.f); v0 *= v0;
-                v1 = fmaxf(v1, 0.f); v1 *= v1;
-              }
-            }
-            o0.v[ni * 4 + r] = from_f32<T>(v0 + bv[ni * 4 + r]);
-            o1.v[ni * 4 + r] = from_f32<T>(v1 + bv[8 + ni * 4 + r]);
-          }
-        if (EPI == 3 ? m - tm * 256 < live : m < p.M) {
-          stvec<T, 8>(yg + (int64_t)m * p.ldy + n0, o0);
-          stvec<T, 8>(yg + (int64_t)m * p.ldy + n0 + 8, o1);
-        }
-      }
+          for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(part + ((wave * 8 + mi) * 4 + ni) * 256 + lane * 4) = acc[mi][ni];
+      return;
     }
   }
+  tile_epilogue<T, EPI, FP8, 8>(p, acc, tm * 256 + g * 128, tm, tn, wc, q4, r16, live);
+}
+
+// Sums the splits of the tail tiles in their order and finishes the tiles: a wave takes one 16-row group of one of the tile's waves,
+// its lanes' values in the order in which they were left (whole 1-KiB lines).
+template <typename T, int EPI, bool FP8>
+__global__ __launch_bounds__(256) void gemm_tiled_tail_kernel(GemmTiledParams p) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
+  const int task = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int t = task >> 6, wave = (task >> 3) & 7, mi = task & 7, g = wave >> 2, wc = wave & 3;
+  int tm, tn;
+  tile_of(p, p.full + t, tm, tn);
+  const int m0 = tm * 256 + g * 128 + mi * 16;
+  if (m0 >= p.M) return;
+  f32x4 acc[1][4];
+#pragma unroll
+  for (int ni = 0; ni < 4; ++ni) acc[0][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* src = p.part + (int64_t)t * 65536 + ((wave * 8 + mi) * 4) * 256 + lane * 4;
+#pragma unroll 4
+  for (int k = 0; k < p.splits; ++k) {
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni) acc[0][ni] += *reinterpret_cast<const f32x4*>(src + (int64_t)k * p.tail * 65536 + ni * 256);
+  }
+  tile_epilogue<T, EPI, FP8, 1>(p, acc, m0, tm, tn, wc, q4, r16, 256);
 }
 
 template <typename T, int EPI, bool FP8, bool MIXED = false>
@@ -498,8 +560,12 @@ int launch_gemm_tiled(const GemmTiledParams& p, hipStream_t st) {
   auto kern = gemm_tiled_kernel<T, EPI, FP8, MIXED>;
   (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS);
   // 8 x 4 blocks, or tiles, in equal numbers for every XCD
-  const int per = EPI == 3 ? (p.nsuper + 7) / 8 * 32 : (int)cdiv((int64_t)p.mt * p.nt, 8);
+  const int per = EPI == 3 ? (p.nsuper + 7) / 8 * 32 : p.splits == 0 ? (int)cdiv((int64_t)p.mt * p.nt, 8)
+                                                     : p.full / 8 + (int)cdiv((int64_t)p.tail * p.splits, 8);
   hipLaunchKernelGGL(kern, dim3((unsigned)(per * 8)), dim3(512), GT_LDS, st, p);
+  if constexpr (EPI != 3) {
+    if (p.splits != 0) hipLaunchKernelGGL((gemm_tiled_tail_kernel<T, EPI, FP8>), dim3((unsigned)p.tail * 16), dim3(256), 0, st, p);
+  }
   MI355_CHECK_LAUNCH(EPI == 3 ? "mi355_moe_grouped_linear_tiled" : EPI == 2 ? "mi355_qkv_proj_rope_tiled"
                      : FP8 ? "mi355_fp8_scaled_mm_tiled" : "mi355_linear_tiled");
   return MI355_OK;
@@ -509,6 +575,7 @@ void fill_tiles(GemmTiledParams& p, int64_t m, int64_t n, int epilogue) {
   p.positions = nullptr; p.cos_sin = nullptr; p.cs_f32 = 0; p.hq = p.hkv = 0;
   p.k_buffer = p.v_buffer = nullptr; p.loc = nullptr; p.loc_i32 = 0; p.kv_slot = p.kv_head = 0;
   p.row_map = p.tile_expert = p.tiles_used = nullptr; p.gather = 0; p.w_expert_stride = 0; p.act = 0;
+  p.full = p.tail = p.splits = 0; p.part = nullptr;
   const int ncols = epilogue == 1 ? (int)(n / 2) : (int)n;
   p.ldy = ncols;
   p.mt = cdiv(m, 256);
@@ -517,10 +584,48 @@ void fill_tiles(GemmTiledParams& p, int64_t m, int64_t n, int epilogue) {
   p.nsuper = cdiv(p.mt, 8) * p.snt;
 }
 
+// One workgroup is one CU, so tiles beyond whole rounds of 256 keep few CUs busy for as long as a round takes: those are split over K
+// where that pays.  Measured costs, in us: a K tile 1.2, a split of a tile (256 KiB of sums, written and read again) 0.075, the launch
+// that sums them 3.  bf16, us, whole tiles -> split: 4605 x 4096 x K 4096 (32 tail tiles, 5 splits) 168 -> 126, K 14336 (8) 538 -> 380;
+// 2 x 14336 columns, K 4096, 520 rows (80, 3) 168 -> 147, 1134 (48, 4) 262 -> 236, 1962 (128, 2) 373 -> 366.  Past half a round
+// (1353 rows of the last: 160 tiles) there is nobody to share with; 128 tiles of K 2048 gain less than the sums cost (101 either way).
+int plan_tail(int64_t m, int64_t n, int64_t kbytes, int epilogue) {
+  const int64_t tiles = cdiv(m, 256) * (epilogue == 1 ? cdiv(n / 2, 128) : cdiv(n, 256));
+  const int64_t kt = kbytes >> 7, tail = tiles % 256;
+  if (tail == 0) return 0;
+  int best = 0;
+  float cost = 1.2f * kt;
+  for (int64_t s = 2; s <= 256 / tail && s <= kt / 4; ++s) {
+    const float c = 1.2f * cdiv(kt, s) + 0.075f * (tail * s) + 3.f;
+    if (c < cost) { cost = c; best = (int)s; }
+  }
+  return best;
+}
+
+// workspace null: no tile is split
+int set_tail(GemmTiledParams& p, int splits, void* workspace, int64_t workspace_bytes, const char* what) {
+  if (workspace == nullptr || splits == 0) return MI355_OK;
+  const int tail = p.mt * p.nt % 256;
+  MI355_REQUIRE(aligned16(workspace) && workspace_bytes >= (int64_t)tail * splits * 65536 * 4, MI355_ERR_INVALID,
+                "%s: workspace of %ld bytes for %d tiles x %d splits", what, (long)workspace_bytes, tail, splits);
+  p.tail = tail; p.full = p.mt * p.nt - tail; p.splits = splits; p.part = (float*)workspace;
+  return MI355_OK;
+}
+
 }  // namespace
 }  // namespace mi355
 
 using namespace mi355;
+
+extern "C" int mi355_tiled_tail_splits(int64_t m, int64_t n, int64_t k, int fp8, int epilogue) {
+  if (m < 1 || n < 1 || k < 1 || m > (1 << 24) || n > (1 << 24)) return 0;
+  return plan_tail(m, n, fp8 ? k : k * 2, epilogue);
+}
+
+extern "C" int64_t mi355_tiled_tail_workspace_bytes(int64_t m, int64_t n, int64_t k, int fp8, int epilogue) {
+  const int64_t tail = (cdiv(m, 256) * (epilogue == 1 ? cdiv(n / 2, 128) : cdiv(n, 256))) % 256;
+  return mi355_tiled_tail_splits(m, n, k, fp8, epilogue) * tail * 65536 * 4;
+}
 
 extern "C" int mi355_linear_tiled_supported(int64_t m, int64_t n, int64_t k, int dtype, int epilogue) {
   if (dtype != MI355_BF16 && dtype != MI355_F16) return 0;
@@ -531,6 +636,12 @@ extern "C" int mi355_linear_tiled_supported(int64_t m, int64_t n, int64_t k, int
 extern "C" int mi355_linear_tiled(void* y, const void* x, const void* w, const void* bias, int64_t m,
                                   int64_t n, int64_t k, int64_t x_stride, int dtype, int epilogue,
                                   void* stream) {
+  return mi355_linear_tiled_ws(y, x, w, bias, m, n, k, x_stride, dtype, epilogue, nullptr, 0, stream);
+}
+
+extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, const void* bias, int64_t m,
+                                     int64_t n, int64_t k, int64_t x_stride, int dtype, int epilogue,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
   MI355_REQUIRE(y && x && w, MI355_ERR_INVALID, "mi355_linear_tiled: null pointer");
   MI355_REQUIRE(mi355_linear_tiled_supported(m, n, k, dtype, epilogue), MI355_ERR_UNSUPPORTED,
                 "mi355_linear_tiled: needs a 16-bit dtype, K %% 64 == 0, K >= 128, N %% 16 == 0 (m=%ld n=%ld k=%ld "
@@ -547,6 +658,7 @@ extern "C" int mi355_linear_tiled(void* y, const void* x, const void* w, const v
   p.M = (int)m; p.N = (int)n; p.K = (int)k;
   p.ldx = x_stride;
   fill_tiles(p, m, n, epilogue);
+  if (const int rc = set_tail(p, plan_tail(m, n, k * 2, epilogue), workspace, workspace_bytes, "mi355_linear_tiled_ws")) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MI355_BF16)
     return epilogue == 1 ? launch_gemm_tiled<bf16_t, 1, false>(p, st) : launch_gemm_tiled<bf16_t, 0, false>(p, st);
@@ -593,6 +705,13 @@ extern "C" int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t
 extern "C" int mi355_fp8_scaled_mm_tiled(void* y, const uint8_t* xq, const uint8_t* wq, const float* x_scale,
                                          const float* w_scale, const void* bias, int64_t m, int64_t n,
                                          int64_t k, int out_dtype, int epilogue, void* stream) {
+  return mi355_fp8_scaled_mm_tiled_ws(y, xq, wq, x_scale, w_scale, bias, m, n, k, out_dtype, epilogue, nullptr, 0, stream);
+}
+
+extern "C" int mi355_fp8_scaled_mm_tiled_ws(void* y, const uint8_t* xq, const uint8_t* wq, const float* x_scale,
+                                            const float* w_scale, const void* bias, int64_t m, int64_t n,
+                                            int64_t k, int out_dtype, int epilogue, void* workspace,
+                                            int64_t workspace_bytes, void* stream) {
   MI355_REQUIRE(y && xq && wq && x_scale && w_scale, MI355_ERR_INVALID, "mi355_fp8_scaled_mm_tiled: null pointer");
   MI355_REQUIRE(mi355_fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, epilogue), MI355_ERR_UNSUPPORTED,
                 "mi355_fp8_scaled_mm_tiled: needs a 16-bit output dtype, K %% 128 == 0, K >= 256, N %% 16 == 0 "
@@ -607,6 +726,7 @@ extern "C" int mi355_fp8_scaled_mm_tiled(void* y, const uint8_t* xq, const uint8
   p.M = (int)m; p.N = (int)n; p.K = (int)k;
   p.ldx = k;
   fill_tiles(p, m, n, epilogue);
+  if (const int rc = set_tail(p, plan_tail(m, n, k, epilogue), workspace, workspace_bytes, "mi355_fp8_scaled_mm_tiled_ws")) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (out_dtype == MI355_BF16)
     return epilogue == 1 ? launch_gemm_tiled<bf16_t, 1, true>(p, st) : launch_gemm_tiled<bf16_t, 0, true>(p, st);
@@ -627,6 +747,18 @@ extern "C" int mi355_qkv_proj_rope_tiled(void* qkv, const void* x, const void* w
                                          const void* cos_sin_cache, int cache_dtype, int rotary_dim, int is_neox,
                                          void* k_buffer, void* v_buffer, const void* loc, int loc_itype,
                                          int64_t num_slots, int dtype, void* stream) {
+  return mi355_qkv_proj_rope_tiled_ws(qkv, x, w, x_scale, w_scale, m, k, x_stride, hq, hkv, head_dim, positions, cos_sin_cache,
+                                      cache_dtype, rotary_dim, is_neox, k_buffer, v_buffer, loc, loc_itype, num_slots, dtype, nullptr, 0,
+                                      stream);
+}
+
+extern "C" int mi355_qkv_proj_rope_tiled_ws(void* qkv, const void* x, const void* w, const float* x_scale,
+                                            const float* w_scale, int64_t m, int64_t k, int64_t x_stride,
+                                            int hq, int hkv, int head_dim, const int64_t* positions,
+                                            const void* cos_sin_cache, int cache_dtype, int rotary_dim, int is_neox,
+                                            void* k_buffer, void* v_buffer, const void* loc, int loc_itype,
+                                            int64_t num_slots, int dtype, void* workspace, int64_t workspace_bytes,
+                                            void* stream) {
   const bool fp8 = x_scale != nullptr;
   const int kv_flags = dtype;
   dtype &= ~(MI355_KV_HEAD_MAJOR | MI355_KV_INTERLEAVED);
@@ -658,6 +790,7 @@ extern "C" int mi355_qkv_proj_rope_tiled(void* qkv, const void* x, const void* w
   p.hq = hq; p.hkv = hkv; p.k_buffer = k_buffer; p.v_buffer = v_buffer; p.loc = loc;
   kv_strides(kv_flags, num_slots, hkv, 128, p.kv_slot, p.kv_head);
   p.loc_i32 = loc_itype == MI355_I32;
+  if (const int rc = set_tail(p, plan_tail(m, n, fp8 ? k : k * 2, 0), workspace, workspace_bytes, "mi355_qkv_proj_rope_tiled_ws")) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MI355_BF16)
     return fp8 ? launch_gemm_tiled<bf16_t, 2, true>(p, st) : launch_gemm_tiled<bf16_t, 2, false>(p, st);

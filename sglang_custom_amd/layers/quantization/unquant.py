@@ -5,7 +5,7 @@ Decode-sized inputs (M <= 64 rows) and every fp32 input go to the hand-written k
 mi355_linear (weight-streaming MFMA / exact-fp32 tiled).  Large-M bf16/f16 GEMMs (prefill) run on the
 hand-written 256 x 256-tile matrix-core kernel behind mi355_linear_tiled, which can apply SiLU-and-mul in
 its epilogue.  PREFILL_GEMM (env MI355_PREFILL_GEMM) picks: "tiled" (default) = that kernel for every
-shape it serves (at least TILED_MIN_TILES output tiles; smaller problems and shapes it does not take
+shape it serves (at least TILED_MIN_TILES output tiles; smaller problems, but for long reductions, and shapes it does not take
 fall back to the library GEMM, torch.nn.functional.linear -> hipBLASLt); "auto" = the faster of the two
 per projection as measured on MI355X (the hand-written kernel for gate_up with the fused activation,
 1.02x the library pair; the library for the plain projections, where it is 4-6 % faster); "library" =
@@ -26,13 +26,21 @@ DECODE_FUSION = True
 PREFILL_GEMM = os.environ.get("MI355_PREFILL_GEMM", "tiled")
 # below this many 256 x 256 output tiles the one-tile-per-workgroup kernel leaves most CUs idle
 TILED_MIN_TILES = 192
+# ... unless the tiles share long reductions: with K split over the idle CUs the kernel is ahead of the library from K = 8192 on, but
+# for the few rows whose sums cost as much as the product (us, library | split: 4096 x 14336 with 126 rows 52 | 40, 330 75 | 58, 646
+# 106 | 84, 1134 140 | 125; 4096 x 11264 with 80 rows 36 | 37, 128 61 | 39, 700 84 | 72; 2048 x 8192 with 128 rows 22 | 25, 200
+# 30 | 27, 1000 52 | 48, 1353 53 | 56, 2100 83 | 74; 2048 x 5632 with 400 rows 26 | 29, 1000 40 | 40, 1500 45 | 48)
+SPLIT_MIN_K = 8192
+SPLIT_MIN_MK = 1200000
 
 
 def _use_tiled(m: int, n_out_tiles_cols: int, n: int, k: int, dtype, silu_mul: bool) -> bool:
     if PREFILL_GEMM == "library" or (PREFILL_GEMM == "auto" and not silu_mul):
         return False
     tiles = ((m + 255) // 256) * ((n_out_tiles_cols + 255) // 256)
-    return tiles >= TILED_MIN_TILES and get_ops().linear_tiled_supported(m, n, k, dtype, silu_mul)
+    ops = get_ops()
+    return ((tiles >= TILED_MIN_TILES or (k >= SPLIT_MIN_K and m * k >= SPLIT_MIN_MK and ops.tiled_tail_splits(m, n, k, False, silu_mul) > 1))
+            and ops.linear_tiled_supported(m, n, k, dtype, silu_mul))
 
 
 def pack_for_decode(layer) -> None:
@@ -80,7 +88,7 @@ def gate_up_silu_mul(layer, act_fn, x: torch.Tensor) -> torch.Tensor:
     if (x2.is_cuda and isinstance(layer.quant_method, UnquantizedLinearMethod) and getattr(layer, "bias", None) is None
             and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
             and _use_tiled(x2.shape[0], w.shape[0], w.shape[0], w.shape[1], x2.dtype, True)):
-        y = get_ops().linear_tiled(x2, w, None, silu_mul=True)
+        y = get_ops().linear_tiled(x2, w, None, silu_mul=True, split_tail=True)
         return y.view(*x.shape[:-1], y.shape[-1])
     gate_up, _ = layer(x)
     return act_fn(gate_up)
@@ -162,7 +170,7 @@ def prefill_linear(x2: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
     """16-bit rows [M, K] (M > SKINNY_MAX_M) against a plain weight [N, K]."""
     if (x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and weight.is_contiguous()
             and _use_tiled(x2.shape[0], weight.shape[0], weight.shape[0], weight.shape[1], x2.dtype, False)):
-        return get_ops().linear_tiled(x2, weight, bias)
+        return get_ops().linear_tiled(x2, weight, bias, split_tail=True)
     return F.linear(x2, weight, bias)
 
 

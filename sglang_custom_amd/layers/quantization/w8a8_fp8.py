@@ -34,7 +34,13 @@ SKINNY_MAX_M = 64
 # (hipBLASLt) on the plain projections and 1.23x on gate_up, whose scales and SiLU-and-mul run in its
 # epilogue; "library" = torch._scaled_mm everywhere.
 PREFILL_GEMM = os.environ.get("MI355_PREFILL_FP8_GEMM", "auto")
-TILED_MIN_TILES = 192   # below this many 256 x 256 output tiles most CUs would idle
+# Below this many 256 x 256 output tiles too many CUs idle (us, library | tiled: 4096 x 4096 with 1600 rows, 112 tiles, 34 | 42, 6144 x 4096
+# with 1100, 120, 36 | 43; 4096 x 4096 with 2300 rows, 144, 57 | 44, 6144 x 4096 with 1600, 168, 57 | 45; 4096 x 14336 with 2300, 144,
+# 171 | 128) ...
+TILED_MIN_TILES = 144
+# ... unless they share long reductions (4096 x 14336 with 80 rows 26 | 31, 150 35 | 33, 300 49 | 39, 646 70 | 52, 1100 90 | 71)
+SPLIT_MIN_K = 8192
+SPLIT_MIN_MK = 1900000
 _SCALED_MM_OK = None   # None = untried; torch._scaled_mm (hipBLASLt) with row-wise scales
 
 
@@ -58,7 +64,9 @@ def _library_scaled_mm(xq, wq, xs, ws, out_dtype, bias):
 
 def _tiled_ok(m: int, n: int, k: int, out_dtype, silu_mul: bool) -> bool:
     tiles = ((m + 255) // 256) * ((n + 255) // 256)
-    return tiles >= TILED_MIN_TILES and get_ops().fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, silu_mul)
+    ops = get_ops()
+    return ((tiles >= TILED_MIN_TILES or (k >= SPLIT_MIN_K and m * k >= SPLIT_MIN_MK and ops.tiled_tail_splits(m, n, k, True, silu_mul) > 1))
+            and ops.fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, silu_mul))
 
 
 def gate_up_silu_mul_prefill(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
@@ -75,7 +83,7 @@ def gate_up_silu_mul_prefill(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
         return None
     ops = get_ops()
     xq, xs = ops.per_token_quant_fp8(x2)
-    y = ops.fp8_scaled_mm_tiled(xq, w, xs, layer.weight_scale.view(-1), x2.dtype, None, silu_mul=True)
+    y = ops.fp8_scaled_mm_tiled(xq, w, xs, layer.weight_scale.view(-1), x2.dtype, None, silu_mul=True, split_tail=True)
     return y.view(*x.shape[:-1], y.shape[-1])
 
 
@@ -125,7 +133,7 @@ class W8A8Fp8LinearMethod:
         y = None
         if (PREFILL_GEMM != "library" and x2.shape[0] > SKINNY_MAX_M and x2.is_cuda
                 and _tiled_ok(x2.shape[0], layer.weight.shape[0], x2.shape[1], x2.dtype, False)):
-            y = ops.fp8_scaled_mm_tiled(xq, layer.weight, xs, layer.weight_scale.view(-1), x.dtype, bias)
+            y = ops.fp8_scaled_mm_tiled(xq, layer.weight, xs, layer.weight_scale.view(-1), x.dtype, bias, split_tail=True)
         if (y is None and x2.shape[0] > SKINNY_MAX_M and x2.is_cuda and x2.shape[1] % 16 == 0
                 and layer.weight.shape[0] % 16 == 0):
             y = _library_scaled_mm(xq, layer.weight, xs, layer.weight_scale, x.dtype, bias)

@@ -154,7 +154,7 @@ class LlamaAttention(nn.Module):
             ws = self.qkv_proj.weight_scale.view(-1)
         return ops.qkv_proj_rope_tiled(x, w, self.num_heads, self.num_kv_heads, self.head_dim, positions.flatten(),
                                        rope.cos_sin_cache, rope.is_neox_style, kb, vb, forward_batch.out_cache_loc,
-                                       x_scale=xs, w_scale=ws, out_dtype=hidden_states.dtype)
+                                       x_scale=xs, w_scale=ws, out_dtype=hidden_states.dtype, split_tail=True)
 
     def forward(self, positions, hidden_states, forward_batch):
         attn_output = self._fused_decode(positions, hidden_states, forward_batch)

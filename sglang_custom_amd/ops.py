@@ -771,11 +771,23 @@ def linear_tiled_supported(m: int, n: int, k: int, dtype: torch.dtype, silu_mul:
         _lib_().mi355_linear_tiled_supported(m, n, k, _DT[dtype], 1 if silu_mul else 0))
 
 
+def tiled_tail_splits(m: int, n: int, k: int, fp8: bool = False, silu_mul: bool = False) -> int:
+    """Into how many parts of K the tiled projections cut the output tiles beyond whole rounds of the chip; 0: not at all."""
+    return _lib_().mi355_tiled_tail_splits(m, n, k, 1 if fp8 else 0, 1 if silu_mul else 0)
+
+
+def _tail_workspace(split_tail: bool, m: int, n: int, k: int, fp8: bool, silu_mul: bool, device):
+    """Scratch for the sums of split tiles, new for every call (the caller's stream orders its reuse); (None, 0) if none are."""
+    need = _lib_().mi355_tiled_tail_workspace_bytes(m, n, k, 1 if fp8 else 0, 1 if silu_mul else 0) if split_tail else 0
+    return (torch.empty(need, dtype=torch.uint8, device=device), need) if need else (None, 0)
+
+
 def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-                 silu_mul: bool = False) -> torch.Tensor:
+                 silu_mul: bool = False, split_tail: bool = False) -> torch.Tensor:
     """Prefill-sized F.linear(x, weight, bias) (layers/quantization/unquant.py:110-122) on the
     256 x 256-tile matrix-core kernel; silu_mul=True applies SiluAndMul (layers/activation.py:55-65)
-    to the [gate; up] output in the epilogue and returns [M, N / 2]."""
+    to the [gate; up] output in the epilogue and returns [M, N / 2].  split_tail: tiles beyond whole rounds of
+    the chip may share K (tiled_tail_splits); their sums are then added in another order than the others'."""
     _gpu(x, weight, bias)
     assert x.dim() == 2 and x.stride(1) == 1 and weight.is_contiguous() and weight.dtype == x.dtype
     M, K = x.shape
@@ -784,8 +796,9 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     y = torch.empty((M, N // 2 if silu_mul else N), dtype=x.dtype, device=x.device)
     if M == 0:
         return y
-    check(_lib_().mi355_linear_tiled(y.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(bias), M, N, K,
-                                     x.stride(0), _dt(x), 1 if silu_mul else 0, _stream(x)), "linear_tiled")
+    ws, nbytes = _tail_workspace(split_tail, M, N, K, False, silu_mul, x.device)
+    check(_lib_().mi355_linear_tiled_ws(y.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(bias), M, N, K, x.stride(0), _dt(x),
+                                        1 if silu_mul else 0, _p(ws), nbytes, _stream(x)), "linear_tiled")
     return y
 
 
@@ -800,7 +813,7 @@ def qkv_proj_rope_tiled(x: torch.Tensor, weight: torch.Tensor, hq: int, hkv: int
                         positions: torch.Tensor, cos_sin_cache: torch.Tensor, is_neox: bool,
                         k_buffer: torch.Tensor, v_buffer: torch.Tensor, loc: torch.Tensor,
                         x_scale: Optional[torch.Tensor] = None, w_scale: Optional[torch.Tensor] = None,
-                        out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                        out_dtype: Optional[torch.dtype] = None, split_tail: bool = False) -> torch.Tensor:
     """qkv_proj -> rotary_emb -> set_kv_buffer of a prefill batch (models/llama.py:187-199) as one
     kernel: the 256 x 256-tile projection with neox RoPE and the cache write in its epilogue.
     Returns qkv [M, (hq + 2 hkv) * head_dim] holding rotated q, rotated k and v.  With x_scale / w_scale
@@ -825,12 +838,13 @@ def qkv_proj_rope_tiled(x: torch.Tensor, weight: torch.Tensor, hq: int, hkv: int
     qkv = torch.empty((M, N), dtype=dtype, device=x.device)
     if M == 0:
         return qkv
-    check(_lib_().mi355_qkv_proj_rope_tiled(
+    ws, nbytes = _tail_workspace(split_tail, M, N, K, fp8, False, x.device)
+    check(_lib_().mi355_qkv_proj_rope_tiled_ws(
         qkv.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(x_scale), _p(w_scale), M, K, x.stride(0), hq, hkv,
         head_dim, positions.data_ptr(), cos_sin_cache.data_ptr(), _dt(cos_sin_cache), cos_sin_cache.shape[1],
         1 if is_neox else 0, k_buffer.data_ptr(), v_buffer.data_ptr(), loc.data_ptr(), _IT[loc.dtype],
-        k_buffer.shape[0], _DT[dtype] | (_kvdt(qkv, k_buffer, v_buffer) & (KV_HEAD_MAJOR | KV_INTERLEAVED)), _stream(x)),
-        "qkv_proj_rope_tiled")
+        k_buffer.shape[0], _DT[dtype] | (_kvdt(qkv, k_buffer, v_buffer) & (KV_HEAD_MAJOR | KV_INTERLEAVED)), _p(ws), nbytes,
+        _stream(x)), "qkv_proj_rope_tiled")
     return qkv
 
 
@@ -1041,9 +1055,10 @@ def fp8_scaled_mm_tiled_supported(m: int, n: int, k: int, out_dtype: torch.dtype
 
 def fp8_scaled_mm_tiled(xq: torch.Tensor, wq: torch.Tensor, x_scale: torch.Tensor, w_scale: torch.Tensor,
                         out_dtype: torch.dtype, bias: Optional[torch.Tensor] = None,
-                        silu_mul: bool = False) -> torch.Tensor:
+                        silu_mul: bool = False, split_tail: bool = False) -> torch.Tensor:
     """fp8_scaled_mm at prefill sizes on the 256 x 256-tile matrix-core kernel (wq [N, K]);
-    silu_mul=True applies SiluAndMul to the [gate; up] output in the epilogue and returns [M, N / 2]."""
+    silu_mul=True applies SiluAndMul to the [gate; up] output in the epilogue and returns [M, N / 2];
+    split_tail as in linear_tiled."""
     _gpu(xq, wq, x_scale, w_scale, bias)
     assert xq.is_contiguous() and wq.is_contiguous()
     assert xq.dtype == torch.float8_e4m3fn and wq.dtype == torch.float8_e4m3fn
@@ -1056,9 +1071,10 @@ def fp8_scaled_mm_tiled(xq: torch.Tensor, wq: torch.Tensor, x_scale: torch.Tenso
     y = torch.empty((M, N // 2 if silu_mul else N), dtype=out_dtype, device=xq.device)
     if M == 0:
         return y
-    check(_lib_().mi355_fp8_scaled_mm_tiled(y.data_ptr(), xq.data_ptr(), wq.data_ptr(), x_scale.data_ptr(),
-                                            w_scale.data_ptr(), _p(bias), M, N, K, _DT[out_dtype],
-                                            1 if silu_mul else 0, _stream(xq)), "fp8_scaled_mm_tiled")
+    ws, nbytes = _tail_workspace(split_tail, M, N, K, True, silu_mul, xq.device)
+    check(_lib_().mi355_fp8_scaled_mm_tiled_ws(y.data_ptr(), xq.data_ptr(), wq.data_ptr(), x_scale.data_ptr(),
+                                               w_scale.data_ptr(), _p(bias), M, N, K, _DT[out_dtype],
+                                               1 if silu_mul else 0, _p(ws), nbytes, _stream(xq)), "fp8_scaled_mm_tiled")
     return y
 
 

@@ -33,7 +33,9 @@
 //     b + 8 share an L2; each XCD works through 8 x 4 blocks of tiles (32 CUs = one block);
 //   * tiles beyond whole rounds of 256 may be split over K, their sums added by a second launch that also runs the epilogue.
 // What bounds it: the card's power.  A K tile takes 2320 of the 2048 cycles that its MFMAs need (88 %), but with random operands the
-// clock falls to 1.7 GHz (4096 x 4096 x 4096: 98 us; with x = 0 2.17 GHz and 77).
+// clock falls to 1.7 GHz (4096 x 4096 x 4096: 98 us; with x = 0 2.17 GHz and 77).  So the order of a matrix slot's MFMAs counts: W fragments
+// go forth in one row of x fragments and back in the next, one operand of every MFMA the last one's (a loop of MFMAs alone 2045 ->
+// 2085 TFLOP/s, with the LDS reads 1797 -> 1829; 32 x 32 x 16 MFMAs 1795 and 1595).  4605 rows, a layer's four products 1408 -> 1381 us.
 #include "common.cuh"
 
 namespace mi355 {
@@ -483,7 +485,8 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     __builtin_amdgcn_s_setprio(1);                                                           \
     if constexpr (FP8) {                                                                     \
       _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                       \
-        _Pragma("unroll") for (int ni = 0; ni < 4; ++ni) {                                   \
+        _Pragma("unroll") for (int nj = 0; nj < 4; ++nj) {                                   \
+          const int ni = (mi & 1) ? 3 - nj : nj;                                             \
           const i32x8 a8_ = __builtin_shufflevector(bf[0][ni], bf[1][ni], 0, 1, 2, 3, 4, 5, 6, 7);\
           const i32x8 b8_ = __builtin_shufflevector(af[0][mi], af[1][mi], 0, 1, 2, 3, 4, 5, 6, 7);\
           acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(                    \
@@ -493,9 +496,11 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
       _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                       \
         _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                     \
           if (!(PART) || mi < live_mi)                                                       \
-          _Pragma("unroll") for (int ni = 0; ni < 4; ++ni)                                   \
+          _Pragma("unroll") for (int nj = 0; nj < 4; ++nj) {                                 \
+              const int ni = (mi & 1) ? 3 - nj : nj;                                         \
               acc[mi][ni] = Mfma<T>::run(__builtin_bit_cast(frag, bf[kk][ni]),               \
                                          __builtin_bit_cast(frag, af[kk][mi]), acc[mi][ni]); \
+          }                                                                                  \
     }                                                                                        \
     __builtin_amdgcn_s_setprio(0);                                                           \
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                         \

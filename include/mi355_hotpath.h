@@ -635,6 +635,12 @@ int mi355_top_k_top_p_min_p_sample_split(int32_t* ids, const float* probs, const
                                          const float* min_ps, const float* uniform, int64_t rows, int64_t vocab,
                                          int64_t row_stride, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Both in one call, the draw's first pass inside the softmax's last: logits become the probabilities that
+ * mi355_softmax_temperature_split leaves, ids what mi355_top_k_top_p_min_p_sample_split draws from those.  Same workspace. */
+int mi355_softmax_sample_split(int32_t* ids, float* logits, const float* temperatures, const int32_t* top_ks, const float* top_ps,
+                               const float* min_ps, const float* uniform, int64_t rows, int64_t vocab, int64_t row_stride, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
 /* fp8_scaled_mm for M <= 64 on a weight packed by mi355_pack_weight (pass the fp8 bytes as an
  * [N, K/2] 16-bit matrix: the packed layout is defined on 16-byte fragments): the bf16 decode GEMM's
  * single-launch weight-streaming kernel with fp8 MFMA and the scale epilogue.  K % 512 == 0,

@@ -110,6 +110,7 @@ _SIGNATURES = {
     "mi355_sampling_workspace_bytes": (L, [L, L]),
     "mi355_softmax_temperature_split": (I, [P, P, L, L, L, P, L, P]),
     "mi355_top_k_top_p_min_p_sample_split": (I, [P, P, P, P, P, P, L, L, L, P, L, P]),
+    "mi355_softmax_sample_split": (I, [P, P, P, P, P, P, P, L, L, L, P, L, P]),
     "mi355_bigram_embedding": (I, [P, P, P, P, P, P, P, P, P, P, P, L, L, L, F, L, L, L, I, P]),
     "mi355_layernorm_shift": (I, [P, P, P, P, P, P, P, P, P, P, P, P, P, L, L, F, I, P]),
     "mi355_commit_sequence_state": (I, [P, P, P, P, P, P, P, P, L, L, L, L, P]),

@@ -149,13 +149,27 @@ __global__ __launch_bounds__(SAMP_THREADS) void argmax_chunk_kernel(int64_t* __r
 }
 
 // ---- softmax(logits / temperature), in place ----------------------------------------------
+// Over the 16 waves of a workgroup: every lane takes one wave's value, four exchanges do the rest (sixteen LDS reads one behind
+// the other are 0.4 us).
 __device__ __forceinline__ float block_reduce_max(float x, float* red) {
+  static_assert(SAMP_THREADS == 1024, "16 waves");
   x = wave_max(x);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
   __syncthreads();
-  float t = -INFINITY;
-  for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t = fmaxf(t, red[i]);
+  float t = red[threadIdx.x & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) t = fmaxf(t, __shfl_xor(t, o, 64));
+  return t;
+}
+__device__ __forceinline__ float block_reduce_sum(float x, float* red) {
+  x = wave_sum(x);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  float t = red[threadIdx.x & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
   return t;
 }
 
@@ -178,8 +192,9 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_temperature_kernel(
 // every chunk normalises itself with what all of them left.  (A chunk without a number in it has no maximum to take off: its
 // -inf entries count zero and a NaN makes its sum NaN, and with it the row, as one pass over the row has it.)  One workgroup per
 // row reads its 0.5 MB three times with 4 bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
-// 18 + 16 us (33 MB read twice, the second time from L2, then read and written), bound by the precise division and
-// exponential of every entry in both.
+// 14 + 14 us (33 MB read twice, the second time from L2, then read and written; 16 + 16 with a precise division per entry in
+// both), bound by the exponentials and by the latency of a chunk's one round of loads.
+constexpr int MAX_CHUNKS = 16;
 struct ChunkSpan {
   int64_t v0, v1;   // first and one past the last of its groups of four elements
   bool tail;        // whether the row's last vocab % 4 elements belong to it
@@ -221,6 +236,28 @@ __device__ __forceinline__ void span_each(const float* __restrict__ row, int64_t
   }
 }
 
+// How a row's exponents are formed.  A temperature that is an ordinary positive number divides once: (x - max x) * (1 / t), where x / t
+// takes a precise division per entry in both launches, and no further from float64 (the difference is exact near the maximum, where the mass is).
+// Any other temperature (zero, negative, NaN, past 1e30 either way) keeps x / t - max(x / t).
+struct RowScale {
+  float t, inv;
+  bool plain;
+  __device__ __forceinline__ explicit RowScale(float t_) : t(t_), inv(1.0f / t_), plain(t_ >= 1e-30f && t_ <= 1e30f) {}
+  __device__ __forceinline__ float key(float x) const { return plain ? x : x / t; }                 // what the maximum is taken of
+  __device__ __forceinline__ float power(float k, float mx) const { return expf(plain ? (k - mx) * inv : k - mx); }
+};
+
+constexpr int KEEP = 8;   // 16-byte pieces of a chunk that a thread holds: chunks up to 32 K entries, every vocabulary up to 512 K at few rows
+
+// The thread's pieces of a chunk, all requested before anything is used (a piece past the end repeats the last one).
+__device__ __forceinline__ void chunk_load(Vec<float, 4> (&v)[KEEP], const float* __restrict__ row, const ChunkSpan& sp) {
+#pragma unroll
+  for (int u = 0; u < KEEP; ++u) {
+    const int64_t i = sp.v0 + threadIdx.x + u * SAMP_THREADS;
+    v[u] = ldvec<float, 4>(row + 4 * (i < sp.v1 ? i : sp.v1 - 1));
+  }
+}
+
 __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
     float2* __restrict__ partials, const float* __restrict__ logits, const float* __restrict__ temperatures, int64_t vocab,
     int64_t row_stride) {
@@ -229,29 +266,22 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
   const float* row = logits + (int64_t)r * row_stride;
   const bool vec = (row_stride % 4 == 0) && aligned16(logits);
   const ChunkSpan sp = chunk_span(vocab, c, chunks);
-  const float t = temperatures[r];
+  const RowScale rs(temperatures[r]);
   float mx = -INFINITY, sum = 0.f;
-  // 16-byte pieces a thread holds: chunks up to 32 K entries, every vocabulary up to 512 K at few rows.  More rows have fewer and longer
-  // chunks (row_chunks), which go through span_each twice: both launches at 128256 entries, 64 rows (4 chunks) 41 us, 86 (3) 73, 200 (2)
-  // 116; a whole row a workgroup 157, 163, 182.
-  constexpr int KEEP = 8;
-  if (vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS) {
-    // The chunk is read once, all of it requested before anything is used, and divided once: 64 rows x 128256 entries
-    // 14.1 us (floor 7); 17.8 with two passes of one piece at a time.
+  // More rows have fewer and longer chunks (row_chunks), which go through span_each twice: both launches at 128256 entries, 64 rows
+  // (4 chunks) 41 us, 86 (3) 73, 200 (2) 116; a whole row a workgroup 157, 163, 182.
+  if (vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS && sp.v0 < sp.v1) {
+    // The chunk is read once, into registers.
     Vec<float, 4> v[KEEP];
-#pragma unroll
-    for (int u = 0; u < KEEP; ++u) {
-      const int64_t i = sp.v0 + threadIdx.x + u * SAMP_THREADS;
-      v[u] = ldvec<float, 4>(row + 4 * (i < sp.v1 ? i : sp.v1 - 1));
-    }
+    chunk_load(v, row, sp);
     const int64_t k = vocab / 4 * 4 + threadIdx.x;
     const bool one = sp.tail && k < vocab;
-    const float last = one ? row[k] / t : -INFINITY;
+    const float last = one ? rs.key(row[k]) : -INFINITY;
 #pragma unroll
     for (int u = 0; u < KEEP; ++u)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        v[u].v[j] /= t;
+        v[u].v[j] = rs.key(v[u].v[j]);
         mx = fmaxf(mx, v[u].v[j]);   // (a piece past the end repeats the last one: the maximum does not mind)
       }
     mx = block_reduce_max(fmaxf(mx, last), red);
@@ -260,48 +290,39 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
     for (int u = 0; u < KEEP; ++u)
       if (sp.v0 + threadIdx.x + u * SAMP_THREADS < sp.v1)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sum += expf(v[u].v[j] - ref);
-    if (one) sum += expf(last - ref);
+        for (int j = 0; j < 4; ++j) sum += rs.power(v[u].v[j], ref);
+    if (one) sum += rs.power(last, ref);
   } else {
-    span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, x / t); });
+    span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, rs.key(x)); });
     mx = block_reduce_max(mx, red);
     const float ref = mx == -INFINITY ? 0.f : mx;
-    span_each(row, vocab, sp, vec, [&](float x) { sum += expf(x / t - ref); });
+    span_each(row, vocab, sp, vec, [&](float x) { sum += rs.power(rs.key(x), ref); });
   }
-  sum = block_sum(sum, red);
+  sum = block_reduce_sum(sum, red);
   if (threadIdx.x == 0) partials[(int64_t)r * chunks + c] = float2{mx, sum};
 }
 
-__global__ __launch_bounds__(SAMP_THREADS) void softmax_normalise_kernel(
-    float* __restrict__ logits, const float2* __restrict__ partials, const float* __restrict__ temperatures, int64_t vocab,
-    int64_t row_stride) {
-  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
-  float* row = logits + (int64_t)r * row_stride;
-  const bool vec = (row_stride % 4 == 0) && aligned16(logits);
-  const float t = temperatures[r];
-  float mx = -INFINITY, sum = 0.f;
-  for (int i = 0; i < chunks; ++i) mx = fmaxf(mx, partials[(int64_t)r * chunks + i].x);
-  for (int i = 0; i < chunks; ++i) {
-    const float2 p = partials[(int64_t)r * chunks + i];
-    sum += p.y * expf(p.x - mx);
-  }
-  const ChunkSpan sp = chunk_span(vocab, c, chunks);
-  for (int64_t i = sp.v0 + threadIdx.x; i < sp.v1; i += SAMP_THREADS) {
-    if (vec) {
-      Vec<float, 4> v = ldvec<float, 4>(row + i * 4);
+// The row's maximum and sum from what its chunks left, and the entries' probabilities.
+struct RowNorm {
+  RowScale rs;
+  float mx, sum, inv_sum;
+  __device__ __forceinline__ RowNorm(const float2* __restrict__ partials, int chunks, float t) : rs(t) {
+    const int i = threadIdx.x & (MAX_CHUNKS - 1);
+    const float2 p = i < chunks ? partials[i] : float2{-INFINITY, 0.f};     // a lane per chunk
+    mx = p.x;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v.v[j] = expf(v.v[j] / t - mx) / sum;
-      stvec<float, 4>(row + i * 4, v);
-    } else {
+    for (int o = MAX_CHUNKS / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    sum = i < chunks ? p.y * rs.power(p.x, mx) : 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) row[i * 4 + j] = expf(row[i * 4 + j] / t - mx) / sum;
-    }
+    for (int o = MAX_CHUNKS / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    inv_sum = 1.0f / sum;
   }
-  if (sp.tail) {
-    const int64_t k = vocab / 4 * 4 + threadIdx.x;
-    if (k < vocab) row[k] = expf(row[k] / t - mx) / sum;
+  // e / sum with sum in [1, vocab] (or NaN): the quotient by the reciprocal and one correction, in four operations
+  __device__ __forceinline__ float prob(float x) const {
+    const float e = rs.power(rs.key(x), mx), q = e * inv_sum;
+    return fmaf(fmaf(-q, sum, e), inv_sum, q);
   }
-}
+};
 
 // ---- joint top-k / top-p / min-p filter + inverse-CDF draw --------------------------------
 // The kept set is {p >= tau}: tau is the smallest probability value v such that fewer than k
@@ -470,18 +491,20 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
 
 // ---- the same draw over chunks of a row -------------------------------------------------------
 // Launch 1, a workgroup per chunk: the chunk's positive entries in 2048 bins of 1/16 binade (the upper 13 bits of the
-// pattern), and its maximum.  Entries of a bin share exponent and upper mantissa, so their count (upper 24 bits) and the sum
-// of their 19 lower bits (lower 40) in one integer are their mass exactly, for one LDS atomic each; a count and a float
-// atomic took 47 us where this takes 10.  Launch 2, a workgroup per row: the first bin from the top that is not
-// kept whole holds tau; its entries -- hundreds where a vocabulary's probabilities spread over binades -- are collected in
-// LDS by one pass over the row and searched there bit by bit.  If they and the larger ones are few (a small top_k), all of
-// them are collected with their indices and the draw is made among them; otherwise a second pass sums what is kept per
-// tile of 256 entries, and the tile the draw falls into is walked.  More entries in that bin than the list holds (an
-// almost flat row) are searched in the row itself, a pass per step.  A row whose tau lies above 1.9 (no probability does) takes
-// sample_whole_row.
+// pattern), its maximum, and the entries of its highest bins as a list.  Entries of a bin share exponent and upper mantissa, so their
+// count (upper 24 bits) and the sum of their 19 lower bits (lower 40) in one integer are their mass exactly, for one LDS atomic each; a
+// count and a float atomic took 47 us where this takes 10.  With the softmax in front the launch is that one's second (softmax_sample).
+// Launch 2, a workgroup per row: the first bin from the top that is not kept whole holds tau, and its entries are searched bit by bit.
+// Where the chunks' lists reach down to that bin -- top_k, top_p or min_p of common size -- they are all that is read: four entries a
+// thread, in registers, tau and the draw from them.  Otherwise (thousands kept, chunks that are not held in registers) the chunks' bins
+// give the cut, its entries are collected in LDS by one pass over the row, and the draw is made among them if they and the larger ones
+// are few, else a second pass sums what is kept per tile of 256 entries, and the tile the draw falls into is walked.  More entries in
+// that bin than the list holds (an almost flat row) are searched in the row itself, a pass per step.  A row whose tau lies above 1.9
+// (no probability does) takes sample_whole_row.
 // The one-workgroup routine meets each of its four levels' 128256 entries in 256 bins of two binades, a handful of which
-// take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics; this
-// takes 10 + 28 us (58 when thousands are kept), the first bound by its LDS atomics too, the second by one CU's pass over 0.5 MB.
+// take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics.  Launch 1 beside the
+// softmax takes 20 us for that (apart 16 + 10), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 14 from the
+// lists, a chain of some twenty barriers (28 from the row, one CU's pass over 0.5 MB; 58 when thousands are kept).
 constexpr int SB_BINS = 2048, SB_SHIFT = 19, SB_LIST = 8192, SB_SHORT = 512, SB_TILE = 256, SB_MAX_TILES = 4096;
 constexpr int SB_SUM_BITS = 40;
 constexpr int64_t SB_MAX_VOCAB = (int64_t)SB_TILE * SB_MAX_TILES;   // 2^20: counts fit 24 bits, sums of 19 bits fit 40
@@ -494,28 +517,197 @@ __device__ __forceinline__ float bin_mass(unsigned bits, u64_t x) {
   return (float)ldexp((double)(x >> SB_SUM_BITS) * base + (double)(x & (((u64_t)1 << SB_SUM_BITS) - 1)), (int)(e ? e : 1u) - 150);
 }
 
-__global__ __launch_bounds__(SAMP_THREADS) void sample_bins_kernel(u64_t* __restrict__ bins, float* __restrict__ maxima,
-                                                                  const float* __restrict__ probs, int64_t vocab,
-                                                                  int64_t row_stride) {
-  __shared__ u64_t hist[SB_BINS];
-  __shared__ float red[SAMP_THREADS / 64];
-  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y;
-  const float* row = probs + (int64_t)r * row_stride;
-  const bool vec = (row_stride % 4 == 0) && aligned16(probs);
-  for (int i = threadIdx.x; i < SB_BINS; i += SAMP_THREADS) hist[i] = 0;
+// What a chunk leaves beside its bins: the entries of its highest bins, in index order -- whole bins until there are more than top_k
+// entries (the row's cut cannot lie below the bin that has the chunk's own top_k-th), but at most 1 / chunks of SB_TOP.  Those are nearly
+// always all that a draw can take (top_p and min_p cut from below too), so that launch 2 reads them instead of the row.
+constexpr int SB_TOP = 4096;
+struct ChunkTop {
+  int count;      // entries listed; -1: none are (a chunk that its workgroup does not hold in registers)
+  int bin;        // the lowest bin listed
+  float mx;       // the chunk's maximum
+  int pad;
+};
+struct BinScratch {
+  u64_t hist[SB_BINS];
+  float red[SAMP_THREADS / 64];
+  int waves[SAMP_THREADS / 64];
+  int pieces[(KEEP + 1) * (SAMP_THREADS / 64)];
+  int passing, listed;
+};
+__device__ __forceinline__ unsigned sb_bin(float v) { return min(__float_as_uint(v) >> SB_SHIFT, (unsigned)(SB_BINS - 1)); }
+__device__ __forceinline__ void sb_count(u64_t* hist, float v) {
+  if (v > 0.f) atomicAdd(&hist[sb_bin(v)], ((u64_t)1 << SB_SUM_BITS) + (__float_as_uint(v) & ((1u << SB_SHIFT) - 1)));
+}
+
+// A chunk in registers (v as chunk_load lays it out, `last`: the thread's entry of the row's tail or 0): its list.  sm.hist is complete.
+__device__ __forceinline__ void chunk_list(const Vec<float, 4> (&v)[KEEP], float last, const ChunkSpan& sp, int64_t vocab, int most,
+                                           int want, BinScratch& sm, uint2* __restrict__ list, int& count, int& lowest) {
+  constexpr int W = SAMP_THREADS / 64;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // entries in this thread's two bins and all above
+  const int c1 = (int)(sm.hist[SB_BINS - 1 - 2 * tid] >> SB_SUM_BITS), c0 = (int)(sm.hist[SB_BINS - 2 - 2 * tid] >> SB_SUM_BITS);
+  int incl = c0 + c1;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += up;
+  }
+  if (lane == 63) sm.waves[wave] = incl;
+  if (tid == 0) sm.passing = sm.listed = 0;
   __syncthreads();
-  float mx = 0.f;
-  span_each(row, vocab, chunk_span(vocab, c, chunks), vec, [&](float v) {
-    if (v > 0.f) {
-      mx = fmaxf(mx, v);
-      const unsigned bits = __float_as_uint(v), b = min(bits >> SB_SHIFT, (unsigned)(SB_BINS - 1));
-      atomicAdd(&hist[b], ((u64_t)1 << SB_SUM_BITS) + (bits & ((1u << SB_SHIFT) - 1)));
+  int above = incl;
+#pragma unroll
+  for (int w = 0; w < W; ++w) above += w < wave ? sm.waves[w] : 0;
+  // A bin is listed if it and those above hold at most `most` entries, and those above it no more than `want` (counts grow on the way
+  // down: the bins that pass are the highest ones).
+  const int upper = above - c0, before_both = upper - c1;
+  const bool high = upper <= most && before_both <= want, low = above <= most && upper <= want;
+  const int pass = __popcll(__ballot(high)) + __popcll(__ballot(low));
+  int got = low ? above : high ? upper : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) got = max(got, __shfl_xor(got, o, 64));
+  if (lane == 0) {
+    atomicAdd(&sm.passing, pass);
+    atomicMax(&sm.listed, got);
+  }
+  __syncthreads();
+  lowest = SB_BINS - sm.passing;
+  count = sm.listed;
+  // the smallest value listed; nothing compares with NaN
+  const float from = lowest == SB_BINS ? NAN : __uint_as_float(max((unsigned)lowest << SB_SHIFT, 1u));
+  // places in index order: pieces, waves in a piece, lanes in a wave, four entries of a lane
+  int at[KEEP + 1];
+#pragma unroll
+  for (int u = 0; u <= KEEP; ++u) {
+    const bool there = u == KEEP || sp.v0 + tid + u * SAMP_THREADS < sp.v1;
+    const Vec<float, 4> x = u == KEEP ? Vec<float, 4>{{last, 0.f, 0.f, 0.f}} : v[u < KEEP ? u : 0];
+    int before = 0, total = 0, own = 0;
+    if (__any(there && (x.v[0] >= from || x.v[1] >= from || x.v[2] >= from || x.v[3] >= from)))
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool in = there && x.v[j] >= from;
+        const u64_t m = __ballot(in);
+        before += __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+        total += __popcll(m);
+        own |= in ? 1 << j : 0;
+      }
+    at[u] = own ? before << 4 | own : 0;
+    if (lane == 0) sm.pieces[u * W + wave] = total;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int run = 0;
+#pragma unroll
+    for (int i = 0; i < (KEEP + 1) * W; i += 64) {
+      const int n = i + lane < (KEEP + 1) * W ? sm.pieces[i + lane] : 0;
+      int x = n;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(x, o, 64);
+        if (lane >= o) x += up;
+      }
+      if (i + lane < (KEEP + 1) * W) sm.pieces[i + lane] = run + x - n;
+      run += __shfl(x, 63, 64);
     }
-  });
-  mx = block_reduce_max(mx, red);
-  u64_t* out = bins + ((int64_t)r * chunks + c) * SB_BINS;
-  for (int i = threadIdx.x; i < SB_BINS; i += SAMP_THREADS) out[i] = hist[i];
-  if (threadIdx.x == 0) maxima[(int64_t)r * chunks + c] = mx;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u <= KEEP; ++u)
+    if (at[u] != 0) {
+      int to = sm.pieces[u * W + wave] + (at[u] >> 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (u == KEEP && j > 0) break;
+        if (at[u] >> j & 1) {
+          const float x = u == KEEP ? last : v[u < KEEP ? u : 0].v[j];
+          const int64_t index = u == KEEP ? vocab / 4 * 4 + tid : (sp.v0 + tid + u * SAMP_THREADS) * 4 + j;
+          list[to++] = uint2{__float_as_uint(x), (unsigned)index};
+        }
+      }
+    }
+}
+
+// NORM: `data` holds logits, which become probabilities on the way (launch 2 of softmax_temperature); BINS: bins and lists of the
+// probabilities.  Both at once: 64 rows x 128256 20 us, apart 16 + 10.
+template <bool NORM, bool BINS>
+__global__ __launch_bounds__(SAMP_THREADS) void sample_chunk_kernel(float* __restrict__ data, const float2* __restrict__ partials,
+                                                                    const float* __restrict__ temperatures, const int32_t* __restrict__ top_ks,
+                                                                    u64_t* __restrict__ bins, uint2* __restrict__ lists, ChunkTop* __restrict__ tops, int64_t vocab,
+                                                                    int64_t row_stride) {
+  __shared__ BinScratch sm;
+  const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y, tid = (int)threadIdx.x;
+  float* row = data + (int64_t)r * row_stride;
+  const bool vec = (row_stride % 4 == 0) && aligned16(data);
+  const ChunkSpan sp = chunk_span(vocab, c, chunks);
+  const bool held = vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS && sp.v0 < sp.v1;
+  Vec<float, 4> v[KEEP];
+  if (held) chunk_load(v, row, sp);
+  const RowNorm norm(partials + (NORM ? (int64_t)r * chunks : 0), NORM ? chunks : 0, NORM ? temperatures[r] : 1.0f);
+  if constexpr (BINS) {
+    for (int i = tid; i < SB_BINS; i += SAMP_THREADS) sm.hist[i] = 0;
+    __syncthreads();
+  }
+  const int64_t k = vocab / 4 * 4 + tid;
+  const bool one = sp.tail && k < vocab;
+  float mx = 0.f, last = 0.f;
+  int count = -1, lowest = SB_BINS;
+  if (one) {
+    last = NORM ? norm.prob(row[k]) : row[k];
+    if (NORM) row[k] = last;
+    mx = fmaxf(mx, last);
+    if (BINS) sb_count(sm.hist, last);
+  }
+  if (held) {
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) {
+      const int64_t i = sp.v0 + tid + u * SAMP_THREADS;
+      if (i < sp.v1) {
+        if constexpr (NORM) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[u].v[j] = norm.prob(v[u].v[j]);
+          stvec<float, 4>(row + i * 4, v[u]);
+        }
+        if constexpr (BINS)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            mx = fmaxf(mx, v[u].v[j]);
+            sb_count(sm.hist, v[u].v[j]);
+          }
+      }
+    }
+    if constexpr (BINS) {
+      __syncthreads();
+      const int most = SB_TOP / chunks;
+      const int want = top_ks ? max(top_ks[r], 0) : 0x7fffffff;
+      chunk_list(v, last, sp, vocab, most, want, sm, lists + (int64_t)r * SB_TOP + c * most, count, lowest);
+    }
+  } else {
+    for (int64_t i = sp.v0 + tid; i < sp.v1; i += SAMP_THREADS) {
+      Vec<float, 4> v;
+      if (vec) v = ldvec<float, 4>(row + i * 4);
+      else
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v.v[j] = row[i * 4 + j];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (NORM) v.v[j] = norm.prob(v.v[j]);
+        mx = fmaxf(mx, v.v[j]);
+        if (BINS) sb_count(sm.hist, v.v[j]);
+      }
+      if (NORM) {
+        if (vec) stvec<float, 4>(row + i * 4, v);
+        else
+#pragma unroll
+          for (int j = 0; j < 4; ++j) row[i * 4 + j] = v.v[j];
+      }
+    }
+  }
+  if constexpr (BINS) {
+    mx = block_reduce_max(mx, sm.red);
+    u64_t* out = bins + ((int64_t)r * chunks + c) * SB_BINS;
+    for (int i = tid; i < SB_BINS; i += SAMP_THREADS) out[i] = sm.hist[i];
+    if (tid == 0) tops[(int64_t)r * chunks + c] = ChunkTop{count, lowest, mx, 0};
+  }
 }
 
 // Of N bins (counts and masses in LDS), going down from the top: the first bin that is not kept whole, with the count and
@@ -566,9 +758,12 @@ __device__ __forceinline__ BinCut cut_bins(const unsigned* hcount, const float* 
   __syncthreads();
   unsigned above = count0;
   float mass = mass0;
-  for (int w = 0; w < wave; ++w) {
-    above += sm.wc[w];
-    mass += sm.wm[w];
+#pragma unroll
+  for (int w = 0; w < SAMP_THREADS / 64; ++w) {
+    const unsigned wc = sm.wc[w];
+    const float wm = sm.wm[w];
+    above += w < wave ? wc : 0u;
+    mass += w < wave ? wm : 0.f;
   }
   if (lane > 0) {
     above += cx;
@@ -606,41 +801,92 @@ __device__ __forceinline__ Vec<float, 4> row4(const float* __restrict__ row, int
 }
 
 __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
-    int32_t* __restrict__ ids, const u64_t* __restrict__ bins, const float* __restrict__ maxima, int chunks,
+    int32_t* __restrict__ ids, const u64_t* __restrict__ bins, const uint2* __restrict__ lists, const ChunkTop* __restrict__ tops, int chunks,
     const float* __restrict__ probs, const int32_t* __restrict__ top_ks, const float* __restrict__ top_ps,
     const float* __restrict__ min_ps, const float* __restrict__ uniform, int64_t vocab, int64_t row_stride) {
-  __shared__ unsigned hcount[SB_BINS];
-  __shared__ float hmass[SB_BINS];
+  // 2048 bins as counts and masses, or as the integers that both come from
+  __shared__ alignas(16) u64_t hist[SB_BINS];
+  unsigned* const hcount = reinterpret_cast<unsigned*>(hist);
+  float* const hmass = reinterpret_cast<float*>(hist + SB_BINS / 2);
+  __shared__ alignas(16) u64_t cells[1024];      // counts and sums of the cut bin's parts
   __shared__ union {
-    unsigned list[SB_LIST];        // the cut bin's entries, until tau is known
-    u64_t cells[1024];             // or, if they are too many, their parts' counts and sums
+    unsigned list[SB_LIST];        // the cut bin's entries where the chunks' lists do not reach it, until tau is known
     float tile[SB_MAX_TILES];      // kept mass per tile of 256 entries, afterwards
     SampleScratch whole;
   } sm;
   __shared__ CutScratch cs;
+  __shared__ double sums[SAMP_THREADS / 64];
   __shared__ unsigned n_list;
   __shared__ int s_tile, s_last, s_pick;
   __shared__ float s_before;
   const SampleRow sr = sample_row(probs, top_ks, top_ps, min_ps, uniform, row_stride);
   const float* row = sr.row;
   const bool vec = (row_stride % 4 == 0) && aligned16(probs);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const u64_t* rb = bins + (int64_t)blockIdx.x * chunks * SB_BINS;
-  float pmax = 0.f;
-  for (int c = 0; c < chunks; ++c) pmax = fmaxf(pmax, maxima[(int64_t)blockIdx.x * chunks + c]);
-  for (int i = threadIdx.x; i < SB_BINS; i += SAMP_THREADS) {
-    u64_t x = 0;
-    for (int c = 0; c < chunks; ++c) x += rb[(int64_t)c * SB_BINS + i];
-    hcount[i] = (unsigned)(x >> SB_SUM_BITS);
-    hmass[i] = bin_mass((unsigned)i << SB_SHIFT, x);
-  }
-  if (threadIdx.x == 0) {
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const ChunkTop* top = tops + (int64_t)blockIdx.x * chunks;
+  const int most = SB_TOP / chunks;
+  if (tid == 0) {
     n_list = 0;
     s_tile = SB_MAX_TILES;
     s_last = -1;
     s_pick = 0x7fffffff;
   }
-  BinCut cut = cut_bins<SB_BINS>(hcount, hmass, sr.k, sr.top_p, 0u, 0.f, cs);
+  // The chunks' lists, four neighbouring slots a thread (an empty one is 0.0: not an entry); if all chunks have one they are complete
+  // from bin `floor` on.  A lane per chunk.
+  constexpr int SLOTS = SB_TOP / SAMP_THREADS;
+  uint2 slot[SLOTS];
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j) {
+    const int at = tid * SLOTS + j;
+    slot[j] = lists[(int64_t)blockIdx.x * SB_TOP + min(at, most * chunks - 1)];
+  }
+  const int ci = tid & (MAX_CHUNKS - 1);
+  const ChunkTop mine = top[min(ci, chunks - 1)];
+  float pmax = mine.mx;
+  int floor = mine.bin;
+  bool lists_hold = __ballot(mine.count < 0) == 0;
+#pragma unroll
+  for (int o = MAX_CHUNKS / 2; o > 0; o >>= 1) {
+    pmax = fmaxf(pmax, __shfl_xor(pmax, o, 64));
+    floor = max(floor, __shfl_xor(floor, o, 64));
+  }
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j) {
+    const int at = tid * SLOTS + j, c = min(at / most, chunks - 1);
+    const bool there = at - c * most < __shfl(mine.count, c, 64);
+    if (!there) slot[j].x = 0u;
+  }
+  auto split = [&](int i, u64_t v) {     // (between two barriers)
+    hcount[i] = (unsigned)(v >> SB_SUM_BITS);
+    hmass[i] = bin_mass((unsigned)i << SB_SHIFT, v);
+  };
+  BinCut cut{-1, 0u, 0.f};
+  if (lists_hold) {
+    hist[tid] = hist[tid + SAMP_THREADS] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j)
+      if ((int)sb_bin(__uint_as_float(slot[j].x)) >= floor) sb_count(hist, __uint_as_float(slot[j].x));
+    __syncthreads();
+    const u64_t lo = hist[tid], hi = hist[tid + SAMP_THREADS];
+    __syncthreads();
+    split(tid, lo);
+    split(tid + SAMP_THREADS, hi);
+    cut = cut_bins<SB_BINS>(hcount, hmass, sr.k, sr.top_p, 0u, 0.f, cs);
+    lists_hold = cut.bin >= 0 || floor == 0;     // (everything above zero is listed and kept, or the cut lies below)
+  }
+  if (!lists_hold) {
+    const u64_t* rb = bins + (int64_t)blockIdx.x * chunks * SB_BINS;
+    u64_t lo = 0, hi = 0;
+    for (int c = 0; c < chunks; ++c) {
+      lo += rb[(int64_t)c * SB_BINS + tid];
+      hi += rb[(int64_t)c * SB_BINS + tid + SAMP_THREADS];
+    }
+    __syncthreads();
+    split(tid, lo);
+    split(tid + SAMP_THREADS, hi);
+    cut = cut_bins<SB_BINS>(hcount, hmass, sr.k, sr.top_p, 0u, 0.f, cs);
+  }
   float tau = 0.f;
   bool few = false;
   if (cut.bin >= 0) {
@@ -650,7 +896,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
       sample_whole_row(ids, sr, vocab, sm.whole.hcount, sm.whole.hmass, sm.whole.scan, sm.whole.red);
       return;
     }
-    few = cut.count + size <= (unsigned)SB_SHORT;
+    few = !lists_hold && cut.count + size <= (unsigned)SB_SHORT;
     // the cut bin's entries; with the larger ones and everybody's index if they are few
     const unsigned lowest = (unsigned)cut.bin << SB_SHIFT, bound = few ? 0x7f800001u : lowest + (1u << SB_SHIFT);   // (few: up to infinity, which the bins have counted)
     const bool listed = few || size <= (unsigned)SB_LIST;
@@ -675,7 +921,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
           }
       }
     };
-    if (listed)
+    if (listed && !lists_hold)
       row_each(lowest, bound, [&](unsigned bits, unsigned index) {
         const unsigned at = atomicAdd(&n_list, 1u);
         if (at < (unsigned)SB_LIST) sm.list[at] = bits;
@@ -691,32 +937,24 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
       const int nb = level == 0 ? 1024 : 512, shift = shifts[level];
       const unsigned want = prefix << (level == 0 ? SB_SHIFT : 9);
       __syncthreads();
-      for (int i = threadIdx.x; i < 1024; i += SAMP_THREADS) {
-        hcount[i] = 0;
-        hmass[i] = 0.f;
-        if (!listed) sm.cells[i] = 0;
+      cells[tid] = 0;
+      __syncthreads();
+      auto part = [&](unsigned bits) {
+        atomicAdd(&cells[(bits >> shift) & (unsigned)(nb - 1)], ((u64_t)1 << SB_SUM_BITS) + (bits & ((1u << shift) - 1)));
+      };
+      if (lists_hold) {
+#pragma unroll
+        for (int j = 0; j < SLOTS; ++j)
+          if (slot[j].x != 0u && (slot[j].x & himask) == want) part(slot[j].x);
+      } else if (listed) {
+        for (unsigned i = threadIdx.x; i < size; i += SAMP_THREADS)
+          if ((sm.list[i] & himask) == want) part(sm.list[i]);
+      } else {
+        row_each(want, want - himask, [&](unsigned bits, unsigned) { part(bits); });
       }
       __syncthreads();
-      if (listed) {
-        for (unsigned i = threadIdx.x; i < size; i += SAMP_THREADS) {
-          const unsigned bits = sm.list[i];
-          if ((bits & himask) == want) {
-            const unsigned b = (bits >> shift) & (unsigned)(nb - 1);
-            atomicAdd(&hcount[b], 1u);
-            unsafeAtomicAdd(&hmass[b], __uint_as_float(bits));
-          }
-        }
-      } else {
-        row_each(want, want - himask, [&](unsigned bits, unsigned) {
-          atomicAdd(&sm.cells[(bits >> shift) & (unsigned)(nb - 1)], ((u64_t)1 << SB_SUM_BITS) + (bits & ((1u << shift) - 1)));
-        });
-        __syncthreads();
-        if ((int)threadIdx.x < nb) {
-          const u64_t x = sm.cells[threadIdx.x];
-          hcount[threadIdx.x] = (unsigned)(x >> SB_SUM_BITS);
-          hmass[threadIdx.x] = bin_mass(want + (threadIdx.x << shift), x);
-        }
-      }
+      hcount[tid] = (unsigned)(cells[tid] >> SB_SUM_BITS);
+      hmass[tid] = bin_mass(want + ((unsigned)tid << shift), cells[tid]);     // (parts past nb: none)
       const BinCut next = cut_bins<1024>(hcount, hmass, sr.k, sr.top_p, cut.count, cut.mass, cs);
       // the coarser bin was not kept whole, but its parts' rounded masses may add up to less: then its lowest part is taken
       cut = next.bin >= 0 ? next : BinCut{0, cut.count, cut.mass};
@@ -729,6 +967,44 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
   }
   tau = fmaxf(tau, sr.min_p * pmax);
   if (!(tau > 0.f)) tau = __uint_as_float(1u);   // never keep zero-probability entries
+  if (lists_hold) {
+    // the draw among the chunks' lists, four neighbouring entries a thread; sums in double
+    double upto[SLOTS], run = 0.0;
+    bool in[SLOTS];
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) {
+      const float p = __uint_as_float(slot[j].x);
+      in[j] = slot[j].x != 0u && p >= tau;
+      run += in[j] ? (double)p : 0.0;
+      upto[j] = run;
+    }
+    double incl = run;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double up = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += up;
+    }
+    if (lane == 63) sums[wave] = incl;
+    const double left = __shfl_up(incl, 1, 64);
+    __syncthreads();
+    double base = 0.0, total = 0.0;
+#pragma unroll
+    for (int w = 0; w < SAMP_THREADS / 64; ++w) {
+      const double x = sums[w];
+      base += w < wave ? x : 0.0;
+      total += x;
+    }
+    if (lane > 0) base += left;
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j)
+      if (in[j]) {
+        atomicMax(&s_last, (int)slot[j].y);
+        if (base + upto[j] > (double)sr.uniform * total) atomicMin(&s_pick, (int)slot[j].y);
+      }
+    __syncthreads();
+    if (tid == 0) ids[blockIdx.x] = s_pick != 0x7fffffff ? s_pick : max(s_last, 0);
+    return;
+  }
   if (few) {
     // the draw among the listed entries, in index order; sums in double, so that the list's order leaves no trace
     __syncthreads();
@@ -854,7 +1130,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
 // latency), at most 16.
 static int row_chunks(int64_t rows, int64_t vocab) {
   const int64_t want = (256 + rows - 1) / rows;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 16), vocab / 8192));
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, MAX_CHUNKS), vocab / 8192));
 }
 
 }  // namespace mi355
@@ -919,7 +1195,8 @@ int mi355_softmax_temperature(float* logits, const float* temperatures, int64_t 
 
 int64_t mi355_sampling_workspace_bytes(int64_t rows, int64_t vocab) {
   if (rows <= 0 || vocab <= 0) return 0;
-  return rows * row_chunks(rows, vocab) * (SB_BINS * (int64_t)sizeof(u64_t) + (int64_t)sizeof(float2));
+  return rows * row_chunks(rows, vocab) * (SB_BINS * (int64_t)sizeof(u64_t) + (int64_t)(sizeof(ChunkTop) + sizeof(float2))) +
+         rows * SB_TOP * (int64_t)sizeof(uint2);
 }
 
 int mi355_softmax_temperature_split(float* logits, const float* temperatures, int64_t rows, int64_t vocab, int64_t row_stride,
@@ -934,8 +1211,8 @@ int mi355_softmax_temperature_split(float* logits, const float* temperatures, in
   float2* partials = static_cast<float2*>(workspace);
   hipLaunchKernelGGL(softmax_partials_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, partials,
                      logits, temperatures, vocab, row_stride);
-  hipLaunchKernelGGL(softmax_normalise_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, logits,
-                     partials, temperatures, vocab, row_stride);
+  hipLaunchKernelGGL((sample_chunk_kernel<true, false>), dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, logits,
+                     partials, temperatures, (const int32_t*)nullptr, (u64_t*)nullptr, (uint2*)nullptr, (ChunkTop*)nullptr, vocab, row_stride);
   MI355_CHECK_LAUNCH("softmax_temperature_split");
   return MI355_OK;
 }
@@ -954,6 +1231,31 @@ int mi355_top_k_top_p_min_p_sample(int32_t* ids, const float* probs, const int32
   return MI355_OK;
 }
 
+// Launches 1 (unless `fused`: with softmax_temperature's second one) and 2 of the draw over chunks.
+static int sample_launches(int32_t* ids, float* data, const float* temperatures, const int32_t* top_ks, const float* top_ps, const float* min_ps,
+                           const float* uniform, int64_t rows, int64_t vocab, int64_t row_stride, bool fused, void* workspace,
+                           hipStream_t stream) {
+  const int chunks = row_chunks(rows, vocab);
+  const int64_t parts = rows * chunks;
+  u64_t* bins = static_cast<u64_t*>(workspace);
+  uint2* lists = reinterpret_cast<uint2*>(bins + parts * SB_BINS);
+  ChunkTop* tops = reinterpret_cast<ChunkTop*>(lists + rows * SB_TOP);
+  float2* partials = reinterpret_cast<float2*>(tops + parts);
+  const dim3 grid((unsigned)rows, chunks), block(SAMP_THREADS);
+  if (fused) {
+    hipLaunchKernelGGL(softmax_partials_kernel, grid, block, 0, stream, partials, data, temperatures, vocab, row_stride);
+    hipLaunchKernelGGL((sample_chunk_kernel<true, true>), grid, block, 0, stream, data, partials, temperatures, top_ks, bins, lists, tops, vocab,
+                       row_stride);
+  } else {
+    hipLaunchKernelGGL((sample_chunk_kernel<false, true>), grid, block, 0, stream, data, (const float2*)nullptr, (const float*)nullptr, top_ks,
+                       bins, lists, tops, vocab, row_stride);
+  }
+  hipLaunchKernelGGL(sample_pick_kernel, dim3((unsigned)rows), block, 0, stream, ids, bins, lists, tops, chunks, data, top_ks, top_ps, min_ps,
+                     uniform, vocab, row_stride);
+  MI355_CHECK_LAUNCH("top_k_top_p_min_p_sample_split");
+  return MI355_OK;
+}
+
 int mi355_top_k_top_p_min_p_sample_split(int32_t* ids, const float* probs, const int32_t* top_ks, const float* top_ps,
                                          const float* min_ps, const float* uniform, int64_t rows, int64_t vocab,
                                          int64_t row_stride, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -965,15 +1267,26 @@ int mi355_top_k_top_p_min_p_sample_split(int32_t* ids, const float* probs, const
   const int64_t need = mi355_sampling_workspace_bytes(rows, vocab);
   MI355_REQUIRE(workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0, MI355_ERR_INVALID,
                 "top_k_top_p_min_p_sample_split: workspace of %lld bytes (8-byte aligned) required", (long long)need);
-  const int chunks = row_chunks(rows, vocab);
-  u64_t* bins = static_cast<u64_t*>(workspace);
-  float* maxima = reinterpret_cast<float*>(bins + rows * chunks * SB_BINS);
-  hipLaunchKernelGGL(sample_bins_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, bins, maxima,
-                     probs, vocab, row_stride);
-  hipLaunchKernelGGL(sample_pick_kernel, dim3((unsigned)rows), dim3(SAMP_THREADS), 0, (hipStream_t)stream, ids, bins, maxima,
-                     chunks, probs, top_ks, top_ps, min_ps, uniform, vocab, row_stride);
-  MI355_CHECK_LAUNCH("top_k_top_p_min_p_sample_split");
-  return MI355_OK;
+  return sample_launches(ids, const_cast<float*>(probs), nullptr, top_ks, top_ps, min_ps, uniform, rows, vocab, row_stride, false, workspace,
+                         (hipStream_t)stream);
+}
+
+int mi355_softmax_sample_split(int32_t* ids, float* logits, const float* temperatures, const int32_t* top_ks, const float* top_ps,
+                               const float* min_ps, const float* uniform, int64_t rows, int64_t vocab, int64_t row_stride, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+  MI355_REQUIRE(ids && logits && temperatures && uniform, MI355_ERR_INVALID, "softmax_sample_split: null pointer");
+  MI355_REQUIRE(rows >= 0 && vocab > 0 && row_stride >= vocab, MI355_ERR_INVALID, "softmax_sample_split: bad shape");
+  if (!workspace || rows == 0 || vocab < 4096 || vocab > SB_MAX_VOCAB || row_chunks(rows, vocab) <= 1) {
+    const int rc = mi355_softmax_temperature_split(logits, temperatures, rows, vocab, row_stride, workspace, workspace_bytes, stream);
+    if (rc != MI355_OK) return rc;
+    return mi355_top_k_top_p_min_p_sample_split(ids, logits, top_ks, top_ps, min_ps, uniform, rows, vocab, row_stride, workspace,
+                                                workspace_bytes, stream);
+  }
+  const int64_t need = mi355_sampling_workspace_bytes(rows, vocab);
+  MI355_REQUIRE(workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0, MI355_ERR_INVALID,
+                "softmax_sample_split: workspace of %lld bytes (8-byte aligned) required", (long long)need);
+  return sample_launches(ids, logits, temperatures, top_ks, top_ps, min_ps, uniform, rows, vocab, row_stride, true, workspace,
+                         (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -35,11 +35,11 @@ class Sampler(nn.Module):
             if return_logprob:
                 logprobs = torch.nn.functional.log_softmax(logits, dim=-1)
         else:
-            probs = ops.softmax_temperature_(logits, sampling_info.temperatures.view(-1))
             u = torch.rand(logits.shape[0], dtype=torch.float32, device=logits.device,
                            generator=self.generator)
-            batch_next_token_ids = ops.top_k_top_p_min_p_sample(
-                probs, sampling_info.top_ks, sampling_info.top_ps,
+            probs = logits    # in place
+            batch_next_token_ids = ops.softmax_sample_(
+                logits, sampling_info.temperatures.view(-1), sampling_info.top_ks, sampling_info.top_ps,
                 sampling_info.min_ps if sampling_info.need_min_p_sampling else None, u)
             if return_logprob:
                 logprobs = torch.log(probs).clamp(min=torch.finfo(probs.dtype).min)

@@ -1167,6 +1167,26 @@ def top_k_top_p_min_p_sample(probs: torch.Tensor, top_ks: Optional[torch.Tensor]
     return ids
 
 
+def softmax_sample_(logits: torch.Tensor, temperatures: torch.Tensor, top_ks: Optional[torch.Tensor], top_ps: Optional[torch.Tensor],
+                    min_ps: Optional[torch.Tensor], uniform: torch.Tensor) -> torch.Tensor:
+    """softmax_temperature_ and top_k_top_p_min_p_sample of its result, in one launch less: logits become the probabilities, the ids
+    are returned."""
+    _gpu(logits, temperatures, top_ks, top_ps, min_ps, uniform)
+    assert logits.dim() == 2 and logits.dtype == torch.float32 and logits.stride(1) == 1
+    B = logits.shape[0]
+    assert temperatures.dtype == torch.float32 and temperatures.numel() == B
+    assert uniform.dtype == torch.float32 and uniform.numel() == B
+    assert top_ks is None or (top_ks.dtype == torch.int32 and top_ks.numel() == B)
+    assert top_ps is None or (top_ps.dtype == torch.float32 and top_ps.numel() == B)
+    assert min_ps is None or (min_ps.dtype == torch.float32 and min_ps.numel() == B)
+    ids = torch.empty(B, dtype=torch.int32, device=logits.device)
+    ws = _sampling_workspace(logits)
+    check(_lib_().mi355_softmax_sample_split(ids.data_ptr(), logits.data_ptr(), temperatures.data_ptr(), _p(top_ks), _p(top_ps), _p(min_ps),
+                                             uniform.data_ptr(), B, logits.shape[1], logits.stride(0), ws.data_ptr(), ws.numel(),
+                                             _stream(logits)), "softmax_sample")
+    return ids
+
+
 # ------------------------------------------------------- fp32 residual stream with per-sequence state
 def _seg(tok_req, seg_start, seg_len):
     assert (tok_req is None) == (seg_start is None) == (seg_len is None), "tok_req, seg_start and seg_len come together"

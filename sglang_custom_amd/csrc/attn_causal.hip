@@ -62,14 +62,10 @@ constexpr int CV_ROWS = 16;
 constexpr int CV_KT = 32;
 
 __device__ __forceinline__ float ca_row16_max(float x) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 16));
-  return x;
+  return row16_max(x);
 }
 __device__ __forceinline__ float ca_row16_sum(float x) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) x += __shfl_xor(x, o, 16);
-  return x;
+  return row16_sum(x);
 }
 
 template <typename T, int MAPS, int C>   // C: result columns per lane, dv <= 16 C
@@ -449,7 +445,7 @@ __device__ __forceinline__ void causal_attention_tile_body(const CaArgs& a, char
 #pragma unroll
         for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, st[hf][i]);
     }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = max_xor<32>(mloc);
     const float mnew = fmaxf(m, mloc * qmul);
     const float ms = mnew == -INFINITY ? 0.f : mnew;
     const float alpha = __builtin_amdgcn_exp2f(m - ms);
@@ -486,7 +482,7 @@ __device__ __forceinline__ void causal_attention_tile_body(const CaArgs& a, char
       }
     }
   }
-  lsum += __shfl_xor(lsum, 32, 64);
+  lsum = sum_xor<32>(lsum);
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   float mul = inv;
   if constexpr (MAPS == 2) {
@@ -522,7 +518,7 @@ __device__ __forceinline__ void causal_attention_tile_body(const CaArgs& a, char
           q2 += o * o;
         }
       }
-    q2 += __shfl_xor(q2, 32, 64);
+    q2 = sum_xor<32>(q2);
     mul = a.out_scale / sqrtf(q2 / (float)dv + a.eps);
   }
   if (!live) return;
@@ -675,8 +671,7 @@ __global__ __launch_bounds__(256) void causal_attention_token_kernel(CaArgs a) {
         st[hf][r] = x;
         mloc = fmaxf(mloc, x);
       }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = max_xor<32>(max_xor<16>(mloc));
     const float mnew = fmaxf(run_m, mloc * qmul);      // finite: a tile's first key is always visible
     const float alpha = __builtin_amdgcn_exp2f(run_m - mnew);
     run_m = mnew;
@@ -708,8 +703,7 @@ __global__ __launch_bounds__(256) void causal_attention_token_kernel(CaArgs a) {
     __builtin_amdgcn_wave_barrier();
   }
   // ---- the streams of a map: common maximum, sums, then rounds of adding through LDS; waves 0 (and 1: the second map) keep the result
-  run_l += __shfl_xor(run_l, 16, 64);
-  run_l += __shfl_xor(run_l, 32, 64);
+  run_l = sum_xor<32>(sum_xor<16>(run_l));
   if (lg == 0) { red_m[wave][li] = run_m; red_l[wave][li] = run_l; }
   __syncthreads();
   float M = -INFINITY, L = 0.f;
@@ -766,8 +760,7 @@ __global__ __launch_bounds__(256) void causal_attention_token_kernel(CaArgs a) {
     for (int c = 0; c < VC; ++c)
 #pragma unroll
       for (int r = 0; r < 4; ++r) q2 += 16 * c + 4 * lg < dv ? acc[c][r] * acc[c][r] : 0.f;
-    q2 += __shfl_xor(q2, 16, 64);
-    q2 += __shfl_xor(q2, 32, 64);
+    q2 = sum_xor<32>(sum_xor<16>(q2));
     mul = a.out_scale / sqrtf(q2 / (float)dv + a.eps);
   }
   if (wave != 0 || li >= nh) return;

@@ -205,21 +205,6 @@ __device__ __forceinline__ void merge_splits_if_last(const DecodeParams& p, T* _
   if (threadIdx.x == 0) *ticket = 0u;   // zero again for the next launch (published by the kernel boundary)
 }
 
-// Sum over the LPR consecutive lanes that hold one K row.  Up to 16 lanes the exchange is done
-// with DPP row operations (no LDS crossbar traffic); wider groups finish with xor-shuffles.
-template <int CTRL> __device__ __forceinline__ float dpp_add(float x) {
-  return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
-}
-template <int LPR> __device__ __forceinline__ float group_sum(float x) {
-  if (LPR >= 2) x = dpp_add<0xB1>(x);    // quad_perm [1,0,3,2]
-  if (LPR >= 4) x = dpp_add<0x4E>(x);    // quad_perm [2,3,0,1]
-  if (LPR >= 8) x = dpp_add<0x141>(x);   // row_half_mirror
-  if (LPR >= 16) x = dpp_add<0x140>(x);  // row_mirror
-  if (LPR >= 32) x += __shfl_xor(x, 16, 64);
-  if (LPR >= 64) x += __shfl_xor(x, 32, 64);
-  return x;
-}
-
 // q . k over one 16-byte vector pair, fp32 accumulate.  16-bit types use the packed dot
 // instructions (two MACs per lane-instruction, no widening of K).
 __device__ __forceinline__ float dot16(const Vec<bf16_t, 8>& a, const Vec<bf16_t, 8>& b) {
@@ -391,15 +376,18 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const T* __restrict__ 
   // merge the KPI row-groups of this wave
 #pragma unroll
   for (int off = LPR; off < 64; off <<= 1) {
+    auto other = [&](float x) {   // (off is a constant in each copy of the loop's body)
+      return off == 8 ? lane_xor<8>(x) : off == 16 ? lane_xor<16>(x) : off == 32 ? lane_xor<32>(x) : __shfl_xor(x, off, 64);
+    };
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      const float mo = __shfl_xor(m[g], off, 64), lo = __shfl_xor(l[g], off, 64);
+      const float mo = other(m[g]), lo = other(l[g]);
       const float mx = fmaxf(m[g], mo), ms = safe_m(mx);
       const float a = exp2f(m[g] - ms), bb = exp2f(mo - ms);
       l[g] = l[g] * a + lo * bb;
 #pragma unroll
       for (int j = 0; j < VE; ++j) {
-        const float ao = __shfl_xor(acc[g][j], off, 64);
+        const float ao = other(acc[g][j]);
         acc[g][j] = acc[g][j] * a + ao * bb;
       }
       m[g] = mx;
@@ -630,13 +618,13 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
   for (int off = 16; off < 64; off <<= 1) {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      const float mo = __shfl_xor(mg[g], off, 64), lo = __shfl_xor(lg[g], off, 64);
+      const float mo = off == 16 ? lane_xor<16>(mg[g]) : lane_xor<32>(mg[g]), lo = off == 16 ? lane_xor<16>(lg[g]) : lane_xor<32>(lg[g]);
       const float mx = fmaxf(mg[g], mo), ms = safe_m(mx);
       const float a = exp2f(mg[g] - ms), bb = exp2f(mo - ms);
       lg[g] = lg[g] * a + lo * bb;
 #pragma unroll
       for (int j = 0; j < VE; ++j) {
-        const float ao = __shfl_xor(acc[g][j], off, 64);
+        const float ao = off == 16 ? lane_xor<16>(acc[g][j]) : lane_xor<32>(acc[g][j]);
         acc[g][j] = acc[g][j] * a + ao * bb;
       }
       mg[g] = mx;
@@ -970,8 +958,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
       x[r] = kb0 + r < k1 ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor<32>(max_xor<16>(mx));
     mx = fmaxf(mx, m);
     const float ms = safe_m(mx);
     const float alpha = exp2f(m - ms);
@@ -1106,8 +1093,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
   }
 
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor<32>(sum_xor<16>(l));
   if (r16 < G) {
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
@@ -1338,8 +1324,7 @@ __global__ __launch_bounds__(256) void decode_attn_mla_mfma_kernel(const T* __re
       x[r] = kb0 + r < k1 ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor<32>(max_xor<16>(mx));
     // Lazy rescale: the reference point m moves only when a tile's maximum exceeds it by more than
     // 2^8 (probabilities then stay below 256 -- exact in fp32, same relative rounding in 16 bits),
     // so the 128 accumulator registers are rescaled a handful of times per sequence, not per tile.
@@ -1394,8 +1379,7 @@ __global__ __launch_bounds__(256) void decode_attn_mla_mfma_kernel(const T* __re
 
   // merge the four waves: common maximum per head, then the waves add their rescaled accumulators
   // into one fp32 tile in turn (fixed order: deterministic)
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor<32>(sum_xor<16>(l));
   if (c4 == 0) {
     sm_m[wave][r16] = m;
     sm_l[wave][r16] = l;
@@ -1940,8 +1924,7 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring_kernel(
     }
   }
 
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor<32>(sum_xor<16>(l));
   if constexpr (TEAMS > 1 && !PAIR) {
     // the teams' (reference point, sum, 512-feature accumulators) meet in LDS; team 0 carries the result out
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -2321,8 +2304,7 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring8_kernel(
       x[r] = kb0 + (r & 3) + 16 * (r >> 2) < k1 ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor<32>(max_xor<16>(mx));
     // lazy rescale: the reference point moves only when a step's maximum exceeds it by 2^8
     const bool need = mx > m + 8.f;
     if (__builtin_amdgcn_ballot_w64(need) != 0) {
@@ -2353,8 +2335,7 @@ __global__ __launch_bounds__(256 * TEAMS) void decode_attn_mla_ring8_kernel(
       acc[dt] = Mfma<T>::run(widen8<T>(uint2{(unsigned)vraw[dt][0], (unsigned)vraw[dt][1]}), pf, acc[dt]);
   }
 
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor<32>(sum_xor<16>(l));
   if constexpr (TEAMS > 1) {
     // the teams' (reference point, sum, 512-feature accumulators) meet in LDS; team 0 carries the result out
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -2551,8 +2532,7 @@ __global__ __launch_bounds__(256) void extend_attn_mla_tile_kernel(
       x[r] = kb0 + (r & 3) + 16 * (r >> 2) < len_w ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor<32>(max_xor<16>(mx));
     const bool need = mx > m + 8.f;
     if (__builtin_amdgcn_ballot_w64(need) != 0) {
       const float mnew = need ? mx : m;
@@ -2604,8 +2584,7 @@ __global__ __launch_bounds__(256) void extend_attn_mla_tile_kernel(
     if ((int64_t)t * 32 < len_w) step_compute(t, sm_raw + 2 * (t % NSB) * MLR_TILE);
   }
 
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor<32>(sum_xor<16>(l));
   if (valid && head0 + r16 < p.hq) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     // lane (head r16, c4) holds features 16 dt + 4 c4 .. + 3

@@ -240,8 +240,7 @@ __global__ __launch_bounds__(256, 2) void extend_attn_kernel(const T* __restrict
           s[i][j] = x;
           mx = fmaxf(mx, x);
         }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+        mx = row16_max(mx);
         const float mnew = fmaxf(m[i], mx);
         const float ms = mnew == -INFINITY ? 0.f : mnew;
         alpha[i] = exp2f(m[i] - ms);
@@ -301,8 +300,7 @@ __global__ __launch_bounds__(256, 2) void extend_attn_kernel(const T* __restrict
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float lt = l[i];
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) lt += __shfl_xor(lt, off, 64);
+    lt = row16_sum(lt);
     if (!row_ok[i]) continue;
     const float inv = lt > 0.f ? 1.0f / lt : 0.f;
     T* dst = o_ext + ((int64_t)(q_start + t0 + row_tok[i]) * p.hq + head0 + row_head[i]) * Dv +
@@ -486,8 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         st[t][r] = x;
         mloc = fmaxf(mloc, x);
       }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = max_xor<32>(max_xor<16>(mloc));
     const float mnew = fmaxf(m, mloc);
     const float ms = mnew == -INFINITY ? 0.f : mnew;
     const float alpha = raw_exp2(m - ms);
@@ -528,8 +525,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       }
   }
 
-  lsum += __shfl_xor(lsum, 16, 64);
-  lsum += __shfl_xor(lsum, 32, 64);
+  lsum = sum_xor<32>(sum_xor<16>(lsum));
   if (qrow < ext) {
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     T* op = o_ext + ((int64_t)(q_start + qrow) * p.hq + h) * D + 4 * c4;
@@ -855,7 +851,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
 #pragma unroll
         for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, st[hf][i]);
     }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = max_xor<32>(mloc);
     const float mnew = fmaxf(m, mloc * qmul);
     const float ms = mnew == -INFINITY ? 0.f : mnew;
     const float alpha = raw_exp2(m - ms);
@@ -896,7 +892,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     }
   }
 
-  lsum += __shfl_xor(lsum, 32, 64);
+  lsum = sum_xor<32>(lsum);
   if (qrow < ext) {
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     T* op = o_ext + ((int64_t)(q_start + qrow) * p.hq + h) * D + 4 * hh;

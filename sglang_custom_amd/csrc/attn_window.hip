@@ -399,8 +399,7 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
       }
     }
   }
-  run_l += __shfl_xor(run_l, 16, 64);
-  run_l += __shfl_xor(run_l, 32, 64);
+  run_l = sum_xor<32>(sum_xor<16>(run_l));
   if (!row_ok) return;
   // the lane holds features 16 c + 4 lg + x of its row
   if (a.num_splits > 1) {

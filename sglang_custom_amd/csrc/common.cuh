@@ -82,14 +82,48 @@ template <int X> __device__ __forceinline__ float max_xor(float v) {
   return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
+template <int X> __device__ __forceinline__ float sum_xor(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
+// A value moved between the lanes of a row of 16 (DPP), in registers.
+template <int CTRL> __device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ float dpp_add(float x) { return x + dpp<CTRL>(x); }
+// The value of the lane whose number differs in bit X (8, 16 or 32).
+template <int X> __device__ __forceinline__ float lane_xor(float v) {
+  if constexpr (X == 8) return dpp<0x128>(v);   // row_ror:8
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = X == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)((threadIdx.x & X) ? r[0] : r[1]));
+}
+
+// Over the 16 lanes of a row.  Rotations do what exchanges with the lanes 8, 4, 2 and 1 apart would: after each step the values
+// repeat with that period.
+__device__ __forceinline__ float row16_sum(float x) {
+  return dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(x))));
+}
+__device__ __forceinline__ float row16_max(float x) {
+  x = fmaxf(x, dpp<0x128>(x));
+  x = fmaxf(x, dpp<0x124>(x));
+  x = fmaxf(x, dpp<0x122>(x));
+  return fmaxf(x, dpp<0x121>(x));
+}
+// Over a wave, all 64 lanes at it.  In registers: six exchanges through the LDS crossbar, each waiting for the last, take 0.3 us, which
+// the kernels of a decode step have several times in a chain.  The sums are those of the exchanges, 32 apart first, to the bit.
+__device__ __forceinline__ float wave_sum(float x) { return row16_sum(sum_xor<16>(sum_xor<32>(x))); }
+__device__ __forceinline__ float wave_max(float x) { return row16_max(max_xor<16>(max_xor<32>(x))); }
+
+// Sum over the LPR consecutive lanes that hold one row.
+template <int LPR> __device__ __forceinline__ float group_sum(float x) {
+  if (LPR >= 2) x = dpp_add<0xB1>(x);    // quad_perm [1,0,3,2]
+  if (LPR >= 4) x = dpp_add<0x4E>(x);    // quad_perm [2,3,0,1]
+  if (LPR >= 8) x = dpp_add<0x141>(x);   // row_half_mirror
+  if (LPR >= 16) x = dpp_add<0x140>(x);  // row_mirror
+  if (LPR >= 32) x = sum_xor<16>(x);
+  if (LPR >= 64) x = sum_xor<32>(x);
   return x;
 }
 
@@ -101,7 +135,11 @@ __device__ __forceinline__ float block_sum(float x, float* red) {
   if (lane == 0) red[w] = x;
   __syncthreads();
   float t = 0.f;
-  for (int i = 0; i < nw; ++i) t += red[i];  // same order in every thread: identical result
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {   // (a loop over nw would read one value behind the other)
+    const float v = red[i];
+    t += i < nw ? v : 0.f;         // same order in every thread: identical result
+  }
   return t;
 }
 

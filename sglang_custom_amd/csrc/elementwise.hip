@@ -2,6 +2,7 @@
 // KV-cache scatter, embedding gather.  All use 16-byte vector accesses when the row length
 // and pointers allow it and fall back to scalar accesses otherwise.
 #include "common.cuh"
+#include <type_traits>
 #include <algorithm>
 
 namespace mi355 {
@@ -82,18 +83,35 @@ __global__ __launch_bounds__(BT) void rmsnorm_vec_kernel(T* __restrict__ out, T*
     // sum in split order and round once, exactly as that GEMM's own combine would have.
     const int64_t split_stride = (int64_t)(gridDim.x - pf_wgs) * hidden;
     const float* pr = part + row * hidden;
-#pragma unroll 4
-    for (int sp = 0; sp < nsplit; ++sp) {
+    // U splits' loads go out together (clamped addresses, masked values): one memory round trip for the eight splits of a
+    // long reduction too.
+    auto add_splits = [&](int sp0, auto batch) {
+      constexpr int U = decltype(batch)::value;
+      float4 f[U][CHUNKS][VE / 4];
 #pragma unroll
-      for (int c = 0; c < CHUNKS; ++c) {
-        const int vi = threadIdx.x + c * BT;
-        const int64_t vo = (int64_t)(vi < nvec ? vi : 0) * VE;
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int j4 = 0; j4 < VE; j4 += 4) {
-          const float4 f = *reinterpret_cast<const float4*>(pr + sp * split_stride + vo + j4);
-          sum[c][j4] += f.x; sum[c][j4 + 1] += f.y; sum[c][j4 + 2] += f.z; sum[c][j4 + 3] += f.w;
+        for (int c = 0; c < CHUNKS; ++c) {
+          const int vi = threadIdx.x + c * BT;
+          const float* at = pr + (int64_t)min(sp0 + u, nsplit - 1) * split_stride + (int64_t)(vi < nvec ? vi : 0) * VE;
+#pragma unroll
+          for (int j = 0; j < VE / 4; ++j) f[u][c][j] = *reinterpret_cast<const float4*>(at + 4 * j);
         }
-      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (sp0 + u < nsplit)
+#pragma unroll
+          for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+            for (int j = 0; j < VE / 4; ++j) {
+              sum[c][4 * j] += f[u][c][j].x; sum[c][4 * j + 1] += f[u][c][j].y;
+              sum[c][4 * j + 2] += f[u][c][j].z; sum[c][4 * j + 3] += f[u][c][j].w;
+            }
+    };
+    if (CHUNKS > 1 || nsplit <= 4) {
+      for (int sp = 0; sp < nsplit; sp += 4) add_splits(sp, std::integral_constant<int, 4>());
+    } else {
+      for (int sp = 0; sp < nsplit; sp += 8) add_splits(sp, std::integral_constant<int, 8>());
     }
     const float xs = part_xs ? part_xs[row] : 1.f;
 #pragma unroll

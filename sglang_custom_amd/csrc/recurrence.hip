@@ -119,9 +119,7 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
         acc = fmaf(S[r4 + 2], q4.z, acc);
         acc = fmaf(S[r4 + 3], q4.w, acc);
       }
-      acc += __shfl_xor(acc, 1, 64);
-      acc += __shfl_xor(acc, 2, 64);
-      acc += __shfl_xor(acc, 4, 64);
+      acc = group_sum<8>(acc);
       if (rg == 0 && col < dv) out[((t0 + base + tt) * heads + h) * (int64_t)dv + col] = fmaf(skip_h, vj, acc);
     }
   }
@@ -242,8 +240,7 @@ __device__ __forceinline__ void token_recurrence(ChunkArgsInMemory& p) {
       y = fmaf(k[r], S[r], y);
     }
     if constexpr (DELTA) {
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o, 64);
+      y = group_sum<16>(y);
       const float z = p.beta_f32 ? static_cast<const float*>(p.beta_logits)[t * p.beta_stride + h]
                                  : to_f32(static_cast<const VT*>(p.beta_logits)[t * p.beta_stride + h]);
       u = (v - y) / (1.0f + expf(-z));
@@ -255,8 +252,7 @@ __device__ __forceinline__ void token_recurrence(ChunkArgsInMemory& p) {
         S[r] = fmaf(k[r], u, S[r]);
         y = fmaf(to_f32(((const QT*)p.q)[t * p.q_stride + (int64_t)hq * p.dk + d0 + r]) * p.q_scale, S[r], y);
       }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o, 64);
+    y = group_sum<16>(y);
     if (d0 == 0 && in_v) p.out[(t * p.heads + h) * (int64_t)p.dv + col] = DELTA ? y : fmaf(skip, v, y);
   }
 #pragma unroll
@@ -651,9 +647,7 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
         dot = fmaf(S[r4 + 2], k4.z, dot);
         dot = fmaf(S[r4 + 3], k4.w, dot);
       }
-      dot += __shfl_xor(dot, 1, 64);
-      dot += __shfl_xor(dot, 2, 64);
-      dot += __shfl_xor(dot, 4, 64);
+      dot = group_sum<8>(dot);
       const float u = bs[tt] * (vs[tt][cl] - dot);
       float acc = 0.f;
 #pragma unroll
@@ -669,9 +663,7 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
         acc = fmaf(S[r4 + 2], q4.z, acc);
         acc = fmaf(S[r4 + 3], q4.w, acc);
       }
-      acc += __shfl_xor(acc, 1, 64);
-      acc += __shfl_xor(acc, 2, 64);
-      acc += __shfl_xor(acc, 4, 64);
+      acc = group_sum<8>(acc);
       if (rg == 0 && col < dv) out[((t0 + base + tt) * heads + h) * (int64_t)dv + col] = acc;
     }
   }
@@ -810,9 +802,7 @@ __global__ __launch_bounds__(MM_THREADS) void matrix_memory_kernel(
           acc = fmaf(S[r4 + 2], q4.z, acc);
           acc = fmaf(S[r4 + 3], q4.w, acc);
         }
-        acc += __shfl_xor(acc, 1, 64);
-        acc += __shfl_xor(acc, 2, 64);
-        acc += __shfl_xor(acc, 4, 64);
+        acc = group_sum<8>(acc);
         if (rg == 0) os[tt][cl] = acc;
       }
     } else {

@@ -573,7 +573,9 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // 256 bytes), and P.V takes the weights as the sum of two 16-bit numbers: the vector-ALU kernel that served this size multiplied
 // fp32 weights, and two terms leave an error of at most 2^-16 of a weight in bf16 (2^-22 in fp16), far below the output's own
 // rounding (against float64 1.6563e-3 of the norm in either kernel).
-template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128>
+// MASK: a custom mask instead of the causal rule (and of a prefix without conditions, unless skip_prefix_custom_mask): a row
+// [prefix + new tokens] of bytes per query.  The arithmetic is the causal launch's, so that a triangle for a mask gives its bits.
+template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128, bool MASK = false>
 __device__ __forceinline__ void extend_attn_mfma32_body(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs) {
@@ -656,11 +658,13 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   }
 
   const int last_row = min(r0 + 127, ext - 1);
-  const int total = LATENT || p.is_causal ? prefix + last_row + 1 : prefix + ext;
+  const bool causal = LATENT || (!MASK && p.is_causal);
+  const int total = causal ? prefix + last_row + 1 : prefix + ext;
   const int n_tiles = (total + 63) / 64;
-  const int my_limit = LATENT || p.is_causal ? prefix + qrow_c : prefix + ext - 1;   // last visible key of this lane's query
-  const int wave_min_limit = LATENT || p.is_causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
-  const int wave_max_limit = LATENT || p.is_causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
+  const int my_limit = causal ? prefix + qrow_c : prefix + ext - 1;   // last visible key of this lane's query
+  const int wave_min_limit = causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
+  const int wave_max_limit = causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
+  const uint8_t* mask_row = MASK ? p.custom_mask + p.mask_indptr[b] + (int64_t)qrow_c * (prefix + ext) : nullptr;
 
   // tile staging: thread -> rows threadIdx.x / CH + SR i, 16-B chunk threadIdx.x % CH
   const int srow = threadIdx.x / CH, sch = threadIdx.x % CH;
@@ -835,7 +839,18 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     // pay for masking (two instructions per score: the key offsets within a tile are compile-time
     // constants, the lane's limit is one subtraction per tile); the branch is wave-uniform.
     float mloc = -INFINITY;
-    if (kt * 64 + 63 > wave_min_limit) {
+    if constexpr (MASK) {
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = kt * 64 + 4 * hh + 32 * hf + 8 * (i >> 2) + (i & 3);
+          const bool seen = mask_row[min(key, my_limit)] != 0 || (key < prefix && p.skip_prefix_custom_mask);
+          const float x = key > my_limit || !seen ? -INFINITY : st[hf][i];
+          st[hf][i] = x;
+          mloc = fmaxf(mloc, x);
+        }
+    } else if (kt * 64 + 63 > wave_min_limit) {
       const int lim = my_limit - kt * 64 - 4 * hh;
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf)
@@ -922,11 +937,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // three quarters of an MFMA cycle).  32 / 8 heads in bf16, us a launch, vector-ALU kernel -> this one: 4 x 340 tokens on 1180 cached
 // 378 -> 57, 704 + 430 tokens on none 121 -> 21, 4000 on none 1493 -> 138, 65 on 3000 510 -> 74, 70 on none 24 -> 13; fp8 cache,
 // 3 x 197 on 1614 478 -> 69.  The heads of a group packed into the rows (less of the triangle's edge in vain) was no faster.
-template <typename T, bool KV8 = false>
+template <typename T, bool KV8, bool MASK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void extend_attn_mfma32_d64_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
-  extend_attn_mfma32_body<T, KV8, 64, false, 64>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
+  extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
 }
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void extend_attn_mfma32_wide_kernel(
@@ -991,8 +1006,8 @@ static int launch_extend(const void* q, const void* k, const void* v, void* o, c
                    p.k_stride % VE == 0 && p.v_stride % VE == 0 && aligned16(q) && aligned16(k) &&
                    aligned16(v) && aligned16(o) && aligned16(kb) && aligned16(vb);
   if constexpr (!std::is_same<T, float>::value) {
-    if (vec && ((p.D == 128 && p.Dv == 128) || (p.D == 192 && p.Dv == 128 && !kv8) || (p.D == 64 && p.Dv == 64)) && !p.custom_mask &&
-        p.sliding_window <= 0 && p.logit_cap <= 0.f && p.sm_scale > 0.f && g_extend_variant == 0) {   // the 32x32 kernel takes the maximum of unscaled scores
+    if (vec && ((p.D == 128 && p.Dv == 128) || (p.D == 192 && p.Dv == 128 && !kv8) || (p.D == 64 && p.Dv == 64)) &&
+        (!p.custom_mask || p.D == 64) && p.sliding_window <= 0 && p.logit_cap <= 0.f && p.sm_scale > 0.f && g_extend_variant == 0) {   // the 32x32 kernel takes the maximum of unscaled scores
       // 128 query rows of one head per workgroup; (sequence, kv head) pairs dealt round-robin to the XCDs
       const int nqb = (int)((max_len_extend + 127) / 128);
       const int64_t npairs = bs * p.hkv;
@@ -1000,12 +1015,10 @@ static int launch_extend(const void* q, const void* k, const void* v, void* o, c
       if (wgs < (int64_t)1 << 31) {
         const dim3 grid1((unsigned)wgs);
         if (p.D == 64) {
-          if (kv8)
-            hipLaunchKernelGGL((extend_attn_mfma32_d64_kernel<T, true>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
-                               (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
-          else
-            hipLaunchKernelGGL((extend_attn_mfma32_d64_kernel<T, false>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
-                               (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
+          const auto kernel = p.custom_mask ? (kv8 ? extend_attn_mfma32_d64_kernel<T, true, true> : extend_attn_mfma32_d64_kernel<T, false, true>)
+                                            : (kv8 ? extend_attn_mfma32_d64_kernel<T, true, false> : extend_attn_mfma32_d64_kernel<T, false, false>);
+          hipLaunchKernelGGL(kernel, grid1, dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb,
+                             (int)npairs);
           return MI355_OK;
         }
         if (p.D == 192)

@@ -50,3 +50,43 @@ def test_tile_edges_over_a_paged_prefix(ops, dtype, kv8, hq, hkv, d, causal):
         tol = u * ref.abs() + ((u if d == 128 else u * u) + 1e-5) * size
         assert bool(((o[at:at + n] - ref).abs() <= tol).all()), (n, pre)
         at, had = at + n, had + pre
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("skip_prefix", [False, True])
+@pytest.mark.parametrize("pre,ext", [([0, 70], [65, 3]), ([130, 63], [129, 64])])
+def test_custom_mask_at_head_dimension_64(ops, pre, ext, skip_prefix):
+    """A mask of its own per query -- holes, a row that sees its own key alone, keys behind the query -- over a prefix and new tokens around
+    tile edges, against float32 softmax; bound: weights and V exact to 2^-16, the output's rounding to bf16 (2^-8 of values up to 3)."""
+    torch.manual_seed(sum(pre) + sum(ext))
+    hq, hkv, d = 8, 2, 64
+    seq = [a + b for a, b in zip(pre, ext)]
+    slots = torch.randperm(sum(seq) + 5)[: sum(seq)].int()
+    kc, vc = torch.randn(sum(seq) + 5, hkv, d).bfloat16(), torch.randn(sum(seq) + 5, hkv, d).bfloat16()
+    T = sum(ext)
+    q, k, v = torch.randn(T, hq, d).bfloat16(), torch.randn(T, hkv, d).bfloat16(), torch.randn(T, hkv, d).bfloat16()
+    masks, indptr, want, at, was = [], [0], [], 0, 0
+    for a, b in zip(pre, ext):
+        m = torch.rand(b, a + b) < 0.5
+        m[torch.arange(b), a + torch.arange(b)] = True
+        m[0] = False
+        m[0, a] = True
+        masks.append(m.flatten())
+        indptr.append(indptr[-1] + m.numel())
+        seen = m.clone()
+        if skip_prefix:
+            seen[:, :a] = True
+        kk = torch.cat([kc[slots[was: was + a].long()], k[at: at + b]]).float().repeat_interleave(hq // hkv, 1)
+        vv = torch.cat([vc[slots[was: was + a].long()], v[at: at + b]]).float().repeat_interleave(hq // hkv, 1)
+        s = torch.matmul(q[at: at + b].float().transpose(0, 1), kk.permute(1, 2, 0)) * d ** -0.5
+        p = torch.softmax(s.masked_fill(~seen, float("-inf")), -1)
+        want.append(torch.matmul(p, vv.transpose(0, 1)).transpose(0, 1))
+        at, was = at + b, was + a
+    dev = lambda t: t.to("cuda")
+    o = torch.empty(T, hq, d, dtype=torch.bfloat16, device="cuda")
+    qo = torch.tensor([0] + ext, dtype=torch.int32).cumsum(0).int()
+    kvp = torch.tensor([0] + pre, dtype=torch.int32).cumsum(0).int()
+    ops.extend_attention_fwd(dev(q), dev(k), dev(v), o, dev(kc), dev(vc), dev(qo), dev(kvp), dev(slots), dev(torch.cat(masks)), True,
+                             dev(torch.tensor(indptr)), max(ext), d ** -0.5, skip_prefix_custom_mask=skip_prefix)
+    want = torch.cat(want)
+    assert (o.cpu().float() - want).abs().max() <= 3 * 2 ** -8 * 1.1

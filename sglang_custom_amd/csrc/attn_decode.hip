@@ -47,7 +47,7 @@ struct DecodeParams {
 // Keys per split of a sequence of `len` keys: the even cut into num_splits, or the batch's chunk when
 // that is larger (never smaller: num_splits chunks always cover the sequence).
 __device__ __forceinline__ int64_t split_chunk(const DecodeParams& p, int64_t len) {
-  int64_t chunk = (len + p.num_splits - 1) / p.num_splits;
+  int64_t chunk = ((unsigned)len + (unsigned)p.num_splits - 1) / (unsigned)p.num_splits;   // (a division of 64 bits is a hundred instructions)
   if (p.chunk_keys) {
     const int64_t c = *p.chunk_keys;
     chunk = c > chunk ? c : chunk;
@@ -81,6 +81,8 @@ __device__ __forceinline__ void seq_range(const DecodeParams& p, int b, int64_t&
 }
 
 __device__ __forceinline__ float safe_m(float m) { return m == -INFINITY ? 0.f : m; }
+// 2^x without the steps that keep results below 2^-126
+__device__ __forceinline__ float raw_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ---- stage 2 of split-KV decoding: o[b, h, :] = sum_s w_s part_o[b, h, s, :] / sum_s w_s with
 // w_s = exp(lse_s - max lse).  ONE statement of the arithmetic, shared by the merge launch and by the
@@ -867,13 +869,19 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int32_t* pt = p.page_table + page_off;
+  // (An empty sequence has no slot to read: it takes its length, or the first prefix sum, which are 0, for one.)
+  const int32_t* pt = len > 0 ? p.page_table + page_off : p.mode == 0 ? reinterpret_cast<const int32_t*>(p.seq_lens + b) : p.kv_indptr;
   const int64_t row_stride = p.k_slot_stride;
   const KVT* kbase = reinterpret_cast<const KVT*>(kbuf) + (int64_t)kvh * p.k_head_stride + 8 * (KROW ? r16 : c4);   // + slot * row_stride (+ 32 s)
   const KVT* vbase = reinterpret_cast<const KVT*>(vbuf) + (int64_t)kvh * p.v_head_stride + 8 * r16;    // + slot * row_stride
-  const int64_t wave_first = k0 + (int64_t)wave * 16;
-  const int n_iter = wave_first < k1 ? (int)((k1 - wave_first + 63) / 64) : 0;
-  const int64_t last_key = len - 1;
+  // Positions and a row's bytes in 32 bits (a sequence is shorter than 2^31 tokens and its slots are numbered from 0): a row's address is one
+  // multiply-add.  With one or two waves on a SIMD the instructions of a tile are its time.
+  const int wave_first = (int)k0 + wave * 16, end = (int)k1, last_key = max((int)len - 1, 0);
+  const int n_iter = wave_first < end ? (end - wave_first + 63) / 64 : 0;
+  const unsigned row_bytes = (unsigned)(row_stride * (int64_t)sizeof(KVT));
+  auto row_at = [&](const KVT* base, int32_t slot) {
+    return reinterpret_cast<const KVT*>(reinterpret_cast<const char*>(base) + (uint64_t)(unsigned)slot * row_bytes);
+  };
   T* v_wr = &sm_v[wave][(4 * c4) * DV_ROW + 8 * r16];                           // + u rows
   T* k_wr = &sm_k[KROW ? wave : 0][KROW ? (4 * c4) * DV_ROW + 8 * r16 : 0];     // + u rows
   const T* k_rd = &sm_k[KROW ? wave : 0][KROW ? r16 * DV_ROW + 8 * c4 : 0];     // + 32 s
@@ -895,38 +903,34 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   }
 
   auto load_slots = [&](int it, int32_t& sk, int32_t (&sv)[4]) {
-    const int64_t tb = wave_first + (int64_t)it * 64;
-    int64_t key = tb + r16;
-    sk = pt[key < last_key ? key : last_key];
+    const int tb = wave_first + it * 64;
+    sk = pt[(unsigned)min(tb + r16, last_key)];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      key = tb + 4 * c4 + u;
-      sv[u] = pt[key < last_key ? key : last_key];
-    }
+    for (int u = 0; u < 4; ++u) sv[u] = pt[(unsigned)min(tb + 4 * c4 + u, last_key)];
   };
 
   auto load_kv = [&](const int32_t& sk, const int32_t (&sv)[4], KRaw (&kf)[4], VRaw (&vv)[4]) {
-    const KVT* krow = kbase + (int64_t)sk * row_stride;
+    const KVT* krow = row_at(kbase, sk);
     if constexpr (KV8 && KROW) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) kf[u] = ld8_nt(kbase + (int64_t)sv[u] * row_stride);
+      for (int u = 0; u < 4; ++u) kf[u] = ld8_nt(row_at(kbase, sv[u]));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ld8_nt(vbase + (int64_t)sv[u] * row_stride);
+      for (int u = 0; u < 4; ++u) vv[u] = ld8_nt(row_at(vbase, sv[u]));
     } else if constexpr (KV8) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) kf[s] = *reinterpret_cast<const uint2*>(krow + 32 * s);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ld8_nt(vbase + (int64_t)sv[u] * row_stride);
+      for (int u = 0; u < 4; ++u) vv[u] = ld8_nt(row_at(vbase, sv[u]));
     } else if constexpr (KROW) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) kf[u] = ldvec_nt<T, VE>(kbase + (int64_t)sv[u] * row_stride);
+      for (int u = 0; u < 4; ++u) kf[u] = ldvec_nt<T, VE>(row_at(kbase, sv[u]));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ldvec_nt<T, VE>(vbase + (int64_t)sv[u] * row_stride);
+      for (int u = 0; u < 4; ++u) vv[u] = ldvec_nt<T, VE>(row_at(vbase, sv[u]));
     } else {
 #pragma unroll
       for (int s = 0; s < 4; ++s) kf[s] = *reinterpret_cast<const frag*>(krow + 32 * s);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ldvec<T, VE>(vbase + (int64_t)sv[u] * row_stride);
+      for (int u = 0; u < 4; ++u) vv[u] = ldvec<T, VE>(row_at(vbase, sv[u]));
     }
   };
   // One 16-key tile.  A tile past the end of the range is harmless: every key is masked, so the
@@ -949,23 +953,23 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 #pragma unroll
     for (int s = 0; s < 4; ++s) sc = Mfma<T>::run(kf[s], qf[s], sc);
 
-    const int64_t kb0 = wave_first + (int64_t)it * 64 + 4 * c4;
+    const int kb0 = wave_first + it * 64 + 4 * c4;
     float x[4], mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float v = sc[r] * qmul;
       if (CAP) v = p.logit_cap * tanhf(v / p.logit_cap) * kLog2e;
-      x[r] = kb0 + r < k1 ? v : -INFINITY;
+      x[r] = kb0 + r < end ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
     }
     mx = max_xor<32>(max_xor<16>(mx));
     mx = fmaxf(mx, m);
     const float ms = safe_m(mx);
-    const float alpha = exp2f(m - ms);
+    const float alpha = raw_exp2(m - ms);
     float pr[4], psum = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      pr[r] = exp2f(x[r] - ms);
+      pr[r] = raw_exp2(x[r] - ms);
       psum += pr[r];
     }
     l = l * alpha + psum;
@@ -1032,21 +1036,26 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   };
 
   // Two K/V register buffers: the loads of tile it+1 are in flight while tile it is computed, so a
-  // wave keeps 8-16 KiB outstanding at all times.  Addresses past the range are clamped (valid).
+  // wave keeps 8-16 KiB outstanding at all times.  Addresses past the range are clamped (valid).  (Four buffers for one-byte rows, or two
+  // tiles' chains side by side, took longer: a tile's own way through LDS, scores and softmax is what is left.)
   int32_t skA, svA[4], skB, svB[4];
   KRaw kfA[4], kfB[4];
   VRaw vvA[4], vvB[4];
-  if (n_iter > 0) {
-    load_slots(0, skA, svA);
-    load_slots(1, skB, svB);
-  }
+  load_slots(0, skA, svA);
+  load_slots(1, skB, svB);
+  const int64_t new_slot = FUSED ? fz.out_loc[b] : 0;   // (read here: behind the tiles' loads its wait would be for all of them)
   if constexpr (FUSED) reduce_qkv_to_lds();   // its loads share the page-table round trip
-  if (n_iter > 0) {   // the first two K/V tiles are in flight across the barrier below
-    load_kv(skA, svA, kfA, vvA);
-    load_kv(skB, svB, kfB, vvB);
-    load_slots(2, skA, svA);
-    load_slots(3, skB, svB);
-  }
+  // The first two K/V tiles are in flight across the barrier below.  Requested in the loop's order, fenced, and without a condition (a wave
+  // without keys reads its last row): the compiler counts what a wait may leave in flight for every way into the loop and the way round it
+  // together, and with another order, or a way past these loads, every tile's slots waited for the rows requested behind them.
+  load_kv(skA, svA, kfA, vvA);
+  __builtin_amdgcn_sched_barrier(0);
+  load_slots(2, skA, svA);
+  __builtin_amdgcn_sched_barrier(0);
+  load_kv(skB, svB, kfB, vvB);
+  __builtin_amdgcn_sched_barrier(0);
+  load_slots(3, skB, svB);
+  __builtin_amdgcn_sched_barrier(0);
   if constexpr (FUSED) {
     __syncthreads();
     frags_from_lds(r16 < G ? r16 : 0, qf);
@@ -1059,9 +1068,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     if (owner) {
       frags_from_lds(G, knew);
       vnew = ldvec<T, VE>(&sm_qkv[(G + 1) * D + 8 * r16]);
-      const int64_t slot = fz.out_loc[b];
-      KVT* kd = const_cast<KVT*>(reinterpret_cast<const KVT*>(kbuf)) + slot * row_stride + (int64_t)kvh * p.k_head_stride + 8 * c4;
-      KVT* vd = const_cast<KVT*>(reinterpret_cast<const KVT*>(vbuf)) + slot * row_stride + (int64_t)kvh * p.v_head_stride + 8 * r16;
+      KVT* kd = const_cast<KVT*>(reinterpret_cast<const KVT*>(kbuf)) + new_slot * row_stride + (int64_t)kvh * p.k_head_stride + 8 * c4;
+      KVT* vd = const_cast<KVT*>(reinterpret_cast<const KVT*>(vbuf)) + new_slot * row_stride + (int64_t)kvh * p.v_head_stride + 8 * r16;
       if constexpr (KV8) {
         // quantise once; the attention below sees exactly what a later step will read from the cache
 #pragma unroll
@@ -1084,12 +1092,17 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   }
   if (n_iter > 0) {
     for (int it = 0; it < n_iter; it += 2) {
+      // (Fenced: the rows' addresses would be formed at the head of a tile, behind a wait for slots that were requested last.)
       compute(kfA, vvA, it);
+      __builtin_amdgcn_sched_barrier(0);
       load_kv(skA, svA, kfA, vvA);      // tile it + 2
       load_slots(it + 4, skA, svA);
+      __builtin_amdgcn_sched_barrier(0);
       compute(kfB, vvB, it + 1);
+      __builtin_amdgcn_sched_barrier(0);
       load_kv(skB, svB, kfB, vvB);      // tile it + 3
       load_slots(it + 5, skB, svB);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -2806,17 +2819,17 @@ int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
     // (head_dim 64, whose splits take a second launch to merge: 128 workgroups, 2 048 keys 26.2 -> 20.5, 4 096 45.7 -> 30.4.)
     if (wgs >= 112 && wgs <= 128) keep = 1024;
     int64_t most = 2;
-    // One-byte rows halve what a workgroup draws (~23 GB/s: its time per key is the chain of page read, row read and
-    // product, not the bytes), so the chip takes two workgroups per CU before it is full: 512 of them, at most 4 splits
+    // One-byte rows halve what a workgroup draws (~27 GB/s: its time per key is the chain from row to product, not the
+    // bytes), so the chip takes two workgroups per CU before it is full: 512 of them, at most 4 splits
     // (a fifth is a second merge chain).  A split has to keep 512 keys, and 4 per workgroup of the unsplit launch, to pay
     // for its partial: where the launch is already wide there is less left to fill.  head_dim 128, 8 kv heads, us at
     // 1 / 2 / 3 / 4 splits (bracket: taken):
-    //   64 wgs, 4 096 keys  46.7 / 29.1 / 22.9 / [19.6];   128 wgs, 512 keys [10.3] / 10.2 / 12.9 / 11.7;
-    //  128 wgs, 1 024       16.2 / [13.3] / 15.6 / 14.0;   128 wgs, 2 048     26.5 / 18.9 / 21.8 / [19.0];
-    //  128 wgs, 4 096       47.8 / 30.5 / 32.8 / [28.7];   144 wgs, 1 024    [16.0] / 17.1 / 15.9 / 17.1;
-    //  160 wgs, 2 048       27.0 / 25.3 / [22.6] / 24.7;   160 wgs, 4 096     48.4 / 41.9 / [34.9] / 39.2;
-    //  224 wgs, 4 096       49.6 / [46.5] / 50.7 / 54.9;   256 wgs, 1 024    [16.8] / 18.6 / 21.4 / 25.9;
-    //  256 wgs, 4 096       51.0 / [49.2] / 51.8 / 59.7;   384 wgs, 4 096    [74.7] / 70.5 / 78.6 / 77.0.
+    //   64 wgs, 4 096 keys  40.0 / 25.0 / 19.7 / [16.9];   128 wgs, 512 keys [9.1] / 8.9 / 10.9 / 9.7;
+    //  128 wgs, 1 024       13.4 / [11.3] / 13.5 / 11.9;   128 wgs, 2 048     22.3 / 16.3 / 19.6 / [16.8];
+    //  128 wgs, 4 096       39.7 / 26.4 / 31.0 / [26.6];   144 wgs, 1 024    [13.5] / 14.8 / 13.8 / 14.8;
+    //  160 wgs, 2 048       22.4 / 23.2 / [20.6] / 22.2;   160 wgs, 4 096     40.3 / 40.0 / [33.4] / 37.4;
+    //  224 wgs, 4 096       41.4 / [43.5] / 48.9 / 48.4;   256 wgs, 1 024    [14.1] / 16.5 / 19.3 / 20.7;
+    //  256 wgs, 4 096       44.4 / [46.5] / 50.1 / 51.1;   384 wgs, 4 096    [72.4] / 67.0 / 76.4 / 74.2.
     if (kv_fp8) {
       most = 512 / wgs < 4 ? 512 / wgs : 4;
       keep = most > 1 ? (4 * wgs > 512 ? 4 * wgs : 512) : 0;

@@ -211,53 +211,59 @@ __global__ __launch_bounds__(256) void causal_attention_valu_kernel(CaArgs a) {
 }
 
 // Ranges of a token's keys, in order: a_m = sum_s acc_s e^(m_s - M) / sum_s l_s e^(m_s - M), M = max_s m_s; then the epilogue.
-// One wave per (token, head); a lane owns up to 8 columns lane, lane + 64, ... (dv <= 512).
+// One workgroup per (token, head), two columns a thread (dv <= 512); lane s of every wave has range s's weight (at most 64 of them).
+// 16 heads x 1 map of 128 columns, 32 ranges, 2 tokens: 22.5 us with one wave a head and a range's loads at a time, 5.9 so; 8 heads x 2 maps of
+// 256: 71.4 and 11.0; 64 tokens of 2 ranges 8.6 and 5.9.
 template <typename T, int MAPS>
 __global__ __launch_bounds__(256) void causal_attention_merge_kernel(CaArgs a) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t idx = (int64_t)blockIdx.x * 4 + wv;
-  if (idx >= a.num_runs * a.heads) return;
-  const int64_t run = idx / a.heads;
-  const int h = (int)(idx - run * a.heads);
+  __shared__ float red[16];
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int64_t run = blockIdx.x / a.heads;
+  const int h = (int)(blockIdx.x - run * a.heads);
   const int64_t t = a.runs != nullptr ? a.runs[2 * run] : run;
   const int dv = a.dv;
   const int64_t stride = a.tokens * a.heads * MAPS * (int64_t)(dv + 2);
-  float o[8];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) o[u] = 0.f;
+  const float* part = a.partial + (t * a.heads + h) * MAPS * (int64_t)(dv + 2);
+  const bool has = lane < a.num_splits;
+  float ms[MAPS], ls[MAPS];
 #pragma unroll
   for (int m = 0; m < MAPS; ++m) {
-    const float* p0 = a.partial + ((t * a.heads + h) * MAPS + m) * (int64_t)(dv + 2);
-    // lane s holds range s (at most 64 of them)
-    const bool has = lane < a.num_splits;
-    const float ms = has ? p0[lane * stride + dv] : CA_NEG, ls = has ? p0[lane * stride + dv + 1] : 0.f;
-    const float w = expf(ms - wave_max(ms));
-    const float L = wave_sum(ls * w);
-    const float wn = w * (m == 1 ? -a.lambda : 1.0f) * (L > 0.f ? 1.0f / L : 0.f);
-#pragma unroll 4
-    for (int s = 0; s < a.num_splits; ++s) {
-      const float f = __shfl(wn, s, 64);
+    const float* p = part + m * (dv + 2) + (int64_t)(has ? lane : 0) * stride + dv;
+    ms[m] = has ? p[0] : CA_NEG;
+    ls[m] = has ? p[1] : 0.f;
+  }
+  const int64_t col[2] = {min(tid, dv - 1), min(tid + 256, dv - 1)};
+  float o[2] = {0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (64 * u < dv && lane + 64 * u < dv) o[u] += p0[s * stride + lane + 64 * u] * f;
+  for (int m = 0; m < MAPS; ++m) {
+    const float w = expf(ms[m] - wave_max(ms[m]));
+    const float L = wave_sum(ls[m] * w);
+    const float wn = w * (m == 1 ? -a.lambda : 1.0f) * (L > 0.f ? 1.0f / L : 0.f);
+    auto weight = [&](int z) { return lane_value(wn, z); };
+    auto add = [](float f, float v, float x) { return x + v * f; };
+    if (dv <= 256) {
+      float o1[1] = {o[0]};
+      const int64_t col1[1] = {col[0]};
+      fold_splits(o1, part + m * (dv + 2), stride, a.num_splits, col1, weight, add);
+      o[0] = o1[0];
+    } else {
+      fold_splits(o, part + m * (dv + 2), stride, a.num_splits, col, weight, add);
     }
   }
   float mul = 1.f;
   if constexpr (MAPS == 2) {
-    float q2 = 0.f;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) q2 += o[u] * o[u];
-    mul = a.out_scale / sqrtf(wave_sum(q2) / (float)dv + a.eps);
+    const float q2 = (tid < dv ? o[0] * o[0] : 0.f) + (tid + 256 < dv ? o[1] * o[1] : 0.f);
+    mul = a.out_scale / sqrtf(block_sum(q2, red) / (float)dv + a.eps);
   }
   const T* gt = (const T*)a.gate + t * a.gate_token_stride;
   if (a.gate != nullptr && !a.gate_per_feature) mul *= ca_sigmoid(to_f32(gt[h]));
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int col = lane + 64 * u;
-    if (col >= dv) continue;
+  for (int u = 0; u < 2; ++u) {
+    const int c = tid + 256 * u;
+    if (c >= dv) continue;
     float y = o[u] * mul;
-    if (a.gate != nullptr && a.gate_per_feature) y *= ca_sigmoid(to_f32(gt[(int64_t)h * dv + col]));
-    ((T*)a.out)[t * a.out_token_stride + (int64_t)h * dv + col] = from_f32<T>(y);
+    if (a.gate != nullptr && a.gate_per_feature) y *= ca_sigmoid(to_f32(gt[(int64_t)h * dv + c]));
+    ((T*)a.out)[t * a.out_token_stride + (int64_t)h * dv + c] = from_f32<T>(y);
   }
 }
 
@@ -863,7 +869,7 @@ template <typename T, int MAPS> int launch_ca(const CaArgs& a, bool matrix, bool
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("causal_attention");
   if (a.num_splits > 1) {
-    hipLaunchKernelGGL((causal_attention_merge_kernel<T, MAPS>), dim3((unsigned)((a.num_runs * a.heads + 3) / 4)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((causal_attention_merge_kernel<T, MAPS>), dim3((unsigned)(a.num_runs * a.heads)), dim3(256), 0, st, a);
     MI355_CHECK_LAUNCH("causal_attention(merge)");
   }
   return MI355_OK;

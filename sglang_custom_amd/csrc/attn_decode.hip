@@ -2621,6 +2621,23 @@ __global__ __launch_bounds__(128) void decode_merge_kernel(const float* __restri
                                                            int Dv) {
   const int64_t bh = blockIdx.x;
   const float* lse = part_lse + bh * num_splits;
+  if (num_splits <= MERGE_MAX_SPLITS) {
+    // a lane per split; merge_weights' sum in its order (reading one log-sum-exp behind the other, three times over, was most of
+    // the launch: 32 heads x 1 token x 12 splits 6.8 -> 4.1 us)
+    const int lane = threadIdx.x & 63;
+    const float x = lane < num_splits ? lse[lane] : -INFINITY;
+    const float e = expf(x - safe_m(wave_max(x)));
+    float tot = 0.f;
+    for (int s = 0; s < num_splits; ++s) tot += lane_value(e, s);
+    for (int d0 = 0; d0 < Dv; d0 += 128) {
+      const int d = d0 + (int)threadIdx.x;
+      float a[1] = {0.f};
+      const int64_t col[1] = {min(d, Dv - 1)};
+      fold_splits(a, part_o + bh * num_splits * Dv, Dv, num_splits, col, [&](int s) { return lane_value(e, s); }, merge_step);
+      if (d < Dv) o[bh * Dv + d] = from_f32<T>(merge_finish(a[0], tot));
+    }
+    return;
+  }
   const float tot = merge_weights(lse, num_splits, nullptr);
   float mx = -INFINITY;
   for (int s = 0; s < num_splits; ++s) mx = fmaxf(mx, lse[s]);

@@ -611,19 +611,26 @@ __global__ __launch_bounds__(128) void latent_window_merge_kernel(const LatentAt
   if (p.rank % 4 == 0) {
     for (int c = 4 * threadIdx.x; c < p.rank; c += 4 * 128) {
       float4 o = float4{0.f, 0.f, 0.f, 0.f};
-      for (int z = 0; z < ns; ++z) {
-        const float4 v = *reinterpret_cast<const float4*>(p.part_o + z * zstride + cell0 + c);
-        const float w = wz[z];
-        o.x += v.x * w; o.y += v.y * w; o.z += v.z * w; o.w += v.w * w;
+      for (int z0 = 0; z0 < ns; z0 += 8) {      // eight splits' loads at a time
+        float4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float4*>(p.part_o + min(z0 + j, ns - 1) * zstride + cell0 + c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (z0 + j < ns) {
+            const float w = wz[z0 + j];
+            o.x += v[j].x * w; o.y += v[j].y * w; o.z += v[j].z * w; o.w += v[j].w * w;
+          }
       }
       out[c] = from_f32<T>(o.x * f); out[c + 1] = from_f32<T>(o.y * f);
       out[c + 2] = from_f32<T>(o.z * f); out[c + 3] = from_f32<T>(o.w * f);
     }
   } else {
     for (int c = threadIdx.x; c < p.rank; c += 128) {
-      float o = 0.f;
-      for (int z = 0; z < ns; ++z) o += p.part_o[z * zstride + cell0 + c] * wz[z];
-      out[c] = from_f32<T>(o * f);
+      float o[1] = {0.f};
+      const int64_t col[1] = {cell0 + c};
+      fold_splits(o, p.part_o, zstride, ns, col, [&](int z) { return wz[z]; }, [](float w, float v, float x) { return x + v * w; });
+      out[c] = from_f32<T>(o[0] * f);
     }
   }
 }

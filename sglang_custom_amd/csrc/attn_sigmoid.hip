@@ -144,8 +144,10 @@ __global__ __launch_bounds__(256) void sigmoid_attention_sum_kernel(T* __restric
                                                                     int64_t out_token_stride, int64_t out_head_stride) {
   const int64_t n = tokens * heads * dv;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int k = 0; k < num_splits; ++k) s += partial[(int64_t)k * n + idx];
+    float sum[1] = {0.f};
+    const int64_t col[1] = {idx};
+    fold_splits(sum, partial, n, num_splits, col, [](int) { return 1.f; }, [](float, float v, float x) { return x + v; });
+    const float s = sum[0];
     const int64_t t = idx / ((int64_t)heads * dv);
     const int64_t rem = idx - t * heads * dv;
     const int h = (int)(rem / dv), c = (int)(rem - (int64_t)h * dv);

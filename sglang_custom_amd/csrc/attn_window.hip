@@ -212,23 +212,22 @@ __global__ __launch_bounds__(256) void window_attention_merge_kernel(T* __restri
                                                                      int64_t tokens, int heads, int dv, int num_splits,
                                                                      int64_t out_token_stride, int64_t out_head_stride,
                                                                      const T* __restrict__ gate, int64_t gate_token_stride) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t idx = (int64_t)blockIdx.x * 4 + wv;
-  if (idx >= tokens * heads) return;
-  const int64_t t = idx / heads;
+  const int lane = threadIdx.x & 63;
+  const int64_t idx = blockIdx.x, t = idx / heads;
   const int h = (int)(idx - t * heads);
   const int64_t stride = tokens * heads * (int64_t)(dv + 2);
   const float* p0 = partial + idx * (dv + 2);
-  float M = WA_NEG;
-  for (int k = 0; k < num_splits; ++k) M = fmaxf(M, p0[k * stride + dv]);
-  float L = 0.f;
-  for (int k = 0; k < num_splits; ++k) L += p0[k * stride + dv + 1] * expf(p0[k * stride + dv] - M);
+  const bool has = lane < num_splits;      // lane k has split k's weight (at most 64 of them)
+  const float m = has ? p0[lane * stride + dv] : WA_NEG, l = has ? p0[lane * stride + dv + 1] : 0.f;
+  const float M = wave_max(m), w = has ? expf(m - M) : 0.f, L = wave_sum(l * w);   // (the lanes without a split have WA_NEG)
   float inv = L > 0.f ? 1.0f / L : 0.f;
   if (gate != nullptr) inv *= wa_sigmoid(to_f32(gate[t * gate_token_stride + h]));
-  for (int c = lane; c < dv; c += 64) {
-    float s = 0.f;
-    for (int k = 0; k < num_splits; ++k) s += p0[k * stride + c] * expf(p0[k * stride + dv] - M);
-    out[t * out_token_stride + (int64_t)h * out_head_stride + c] = from_f32<T>(s * inv);
+  for (int c0 = 0; c0 < dv; c0 += 256) {
+    const int c = c0 + (int)threadIdx.x;
+    float s[1] = {0.f};
+    const int64_t col[1] = {min(c, dv - 1)};
+    fold_splits(s, p0, stride, num_splits, col, [&](int k) { return lane_value(w, k); }, [](float f, float v, float x) { return x + v * f; });
+    if (c < dv) out[t * out_token_stride + (int64_t)h * out_head_stride + c] = from_f32<T>(s[0] * inv);
   }
 }
 
@@ -615,7 +614,7 @@ int mi355_window_attention_pooled(void* out, const void* q, const void* k_cache,
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("window_attention");
   if (num_splits > 1) {
-    const unsigned g2 = (unsigned)((tokens * heads + 3) / 4);
+    const unsigned g2 = (unsigned)(tokens * heads);
     MI355_DISPATCH_DTYPE(dtype, "window_attention", {
       hipLaunchKernelGGL((window_attention_merge_kernel<T>), dim3(g2), dim3(256), 0, (hipStream_t)stream, (T*)out, split_scratch, tokens,
                          heads, v_head_dim, num_splits, out_token_stride, out_head_stride, (const T*)head_gate, gate_token_stride);

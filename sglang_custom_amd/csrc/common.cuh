@@ -144,6 +144,31 @@ __device__ __forceinline__ float block_sum(float x, float* red) {
   return t;
 }
 
+// acc[u] <- f(weight(z), part[z * stride + col[u]], acc[u]) for z = 0 .. n - 1 in order: how the partial results of split launches are
+// folded.  Eight splits' loads go out together (clamped addresses, masked values): a loop that loads and folds one split at a time
+// is a memory round trip per split.
+template <int NU, typename W, typename F>
+__device__ __forceinline__ void fold_splits(float (&acc)[NU], const float* __restrict__ part, int64_t stride, int n, const int64_t (&col)[NU],
+                                            W&& weight, F&& f) {
+  for (int z0 = 0; z0 < n; z0 += 8) {
+    float v[8][NU];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int u = 0; u < NU; ++u) v[j][u] = part[(int64_t)min(z0 + j, n - 1) * stride + col[u]];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (z0 + j < n) {
+        const float w = weight(z0 + j);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) acc[u] = f(w, v[j][u], acc[u]);
+      }
+  }
+}
+// The value of lane z (the same z in all lanes), with all lanes of the wave at it: inside a branch that some have left, the compiler may
+// compute x there, for those that are in it alone.
+__device__ __forceinline__ float lane_value(float x, int z) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), z)); }
+
 // ---- host side -------------------------------------------------------------------------
 void set_error(const char* fmt, ...);
 

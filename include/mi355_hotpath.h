@@ -285,7 +285,7 @@ int mi355_decode_attention_static(const void* q, const void* k_buffer, const voi
                                   int dtype, void* stream);
 
 /* Decode attention fused with everything between the qkv GEMM and the attention kernel.
- * qkv_part: the fp32 split-K partials [nsplit][bs][(hq + 2 hkv) * 128] of the qkv projection
+ * qkv_part: the fp32 split-K partials [nsplit][bs][(hq + 2 hkv) * head_dim] of the qkv projection
  * (mi355_linear_packed_partials, or mi355_fp8_packed_partials together with that GEMM's per-token
  * and per-channel scales; both NULL otherwise).  The kernel sums them (split order, scales applied
  * as (sum * x_scale[b]) * w_scale[n], one rounding to the tensor dtype = the GEMM's own result), applies neox RoPE over the whole head to q and the new k with
@@ -293,7 +293,8 @@ int mi355_decode_attention_static(const void* q, const void* k_buffer, const voi
  * slot out_cache_loc[b] (which the page table must name for position seq_len - 1, except for padding
  * rows, whose writes go to the sink slot they name), and runs mi355_decode_attention.  Output and
  * cache contents are bit-identical to mi355_linear_packed -> mi355_rope_inplace (fused KV write) ->
- * mi355_decode_attention (split_tickets, kv_chunk_keys as there).  Needs head_dim 128, a 16-bit dtype, hq / hkv in {1, 2, 4, 8}, no logit cap.
+ * mi355_decode_attention (split_tickets, kv_chunk_keys as there).  Needs head_dim 128, or 64 over a 16-bit cache,
+ * a 16-bit dtype, hq / hkv in {1, 2, 4, 8}, no logit cap.
  * replaces: LlamaAttention.forward's rotary_emb + attn sequence (models/llama.py:180-191) on the
  *           decode path; the reference has no fused counterpart. */
 int mi355_decode_attention_fused_qkv(const float* qkv_part, int nsplit, const float* part_x_scale,

@@ -687,7 +687,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
 // every quarter-wave touch 16 rows x 16 bytes, i.e. sixteen cache-line look-ups for 256 bytes;
 // measured 58.8 -> 56.4 us at batch 64 x 1064 keys, 8 kv heads.
 // ------------------------------------------------------------------------------------------
-constexpr int DV_ROW = 128 + 16;   // V tile row in LDS (elements): 288 B -> conflict-free transposed reads
+template <int D> constexpr int dv_row() { return D + 16; }   // V tile row in LDS (elements): 288 or 160 B -> conflict-free transposed reads
 
 //
 // FUSED: q, k_new and v_new are summed from the qkv GEMM's split-K partials (split order, one
@@ -702,14 +702,22 @@ constexpr int DV_ROW = 128 + 16;   // V tile row in LDS (elements): 288 B -> con
 // its first split is finished there, without a partial and a merge.  A captured launch of 4 splits on a batch that needs one:
 // 128 workgroups, e4m3fn rows, 300 / 4096 keys 14.0 / 68.2 us with sequences outside splits and the merge, 9.1 / 47.7 so (unsplit
 // 8.8 / 47.9); 512 workgroups, 16-bit rows, 300 keys 47.0 -> 16.7 (15.5).
-template <typename T, int G, bool CAP, bool FUSED = false, bool KV8 = false, bool KROW = false>
+// D = 64: eight lanes a row, and the weights enter P.V as the sum of two 16-bit numbers: the vector-ALU kernel that served this size multiplied
+// fp32 weights, and two terms leave an error of at most 2^-16 of a weight in bf16 (2^-22 in fp16).  16 layers of 32 / 8 heads, a whole
+// step with the rotation, the sum of the projection's splits and the merge in this launch: 1 x 131 tokens 844 -> 769 us, 1 x 2000 936 -> 837,
+// 32 x 360 1043 -> 927, 33 x 1494 1442 -> 1201.
+template <typename T, int D, int G, bool CAP, bool FUSED = false, bool KV8 = false, bool KROW = false>
 __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __restrict__ q,
                                                                   const T* kbuf, const T* vbuf,
                                                                   T* __restrict__ o, DecodeParams p,
                                                                   FusedQkv fz = FusedQkv()) {
 #pragma clang fp contract(off)   // see the note in `compute`
   using KVT = typename std::conditional<KV8, uint8_t, T>::type;
-  constexpr int D = 128, VE = 8;
+  constexpr int VE = 8, DV_ROW = dv_row<D>();
+  constexpr int LPR = D / VE, NR = D / 32;    // lanes of a row; rows of a tile that a lane loads
+  constexpr int NS = D / 32, ND = D / 16;     // score k-steps; 16-feature tiles of the result
+  constexpr bool PSPLIT = D == 64;
+  static_assert((D == 128 || D == 64) && (D == 128 || KROW), "head dimensions 64 and 128");
   using frag = typename Mfma<T>::frag;
   using frag4 = typename Mfma16<T>::frag;
   // what the K/V register buffers hold between load and use: with an fp8 cache the raw 8 bytes
@@ -733,6 +741,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   const int b = blockIdx.y, split = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r16 = lane & 15, c4 = lane >> 4;
+  const int row0 = NR * (lane / LPR), ch8 = VE * (lane % LPR);    // a lane's rows row0 .. + NR - 1 of a tile, its features from ch8 on
 
   int64_t page_off, len;
   seq_range(p, b, page_off, len);
@@ -753,14 +762,14 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     // Every thread's items (one, or two at G = 8) and up to eight splits go out as ONE batch of loads -- clamped
     // addresses, masked values, never a condition on a load -- so a projection cut eleven ways (a tensor-parallel
     // rank's narrow qkv) costs two memory round trips here, not six.  The sum per element stays in split order.
-    constexpr int ITEMS = ((G + 2) * 32 + 255) / 256;
+    constexpr int F4 = D / 4, ITEMS = ((G + 2) * F4 + 255) / 256;   // float4s of a head
     float sums[ITEMS][4];
     {
       const float* srcs[ITEMS];
 #pragma unroll
       for (int it = 0; it < ITEMS; ++it) {
-        const int v = min((int)threadIdx.x + it * 256, (G + 2) * 32 - 1);
-        const int seg = v >> 5, f4 = v & 31;
+        const int v = min((int)threadIdx.x + it * 256, (G + 2) * F4 - 1);
+        const int seg = v / F4, f4 = v % F4;
         const int64_t head = seg < G ? head0 + seg : seg == G ? p.hq + kvh : p.hq + p.hkv + kvh;
         srcs[it] = fz.part + (int64_t)b * fz.row + head * D + 4 * f4;
 #pragma unroll
@@ -795,8 +804,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
       const int v = threadIdx.x + it * 256;
-      if (v >= (G + 2) * 32) break;   // (whole 32-lane slices drop out together)
-      const int seg = v >> 5, f4 = v & 31;
+      if (v >= (G + 2) * F4) break;   // (whole slices drop out together)
+      const int seg = v / F4, f4 = v % F4;
       const int64_t head = seg < G ? head0 + seg : seg == G ? p.hq + kvh : p.hq + p.hkv + kvh;
       const float (&sum)[4] = sums[it];
       Vec<T, 4> out;
@@ -812,29 +821,29 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
         for (int j = 0; j < 4; ++j) out.v[j] = from_f32<T>(sum[j] + 0.f);
       }
       // neox RoPE on the q heads and the new key, here, once per workgroup (each wave would otherwise rotate
-      // its own copy of all heads after the barrier): features i and i + 64 of a head sit in lanes 16 apart of
-      // this wave (f4 and f4 + 16).  Rounding points of the RoPE kernel; the value slice is left alone.
-      // (All 32 lanes of a slice are active together, and slices never straddle a wave: the exchange is safe.)
-      if (seg <= G) {   // (uniform over the 32 lanes of a slice)
+      // its own copy of all heads after the barrier): features i and i + D / 2 of a head sit in lanes D / 8 apart of
+      // this wave (f4 and f4 + D / 8).  Rounding points of the RoPE kernel; the value slice is left alone.
+      // (All lanes of a slice are active together, and slices never straddle a wave: the exchange is safe.)
+      if (seg <= G) {   // (uniform over the lanes of a slice)
 #pragma clang fp contract(off)
-        const int fl = f4 & 15;
+        const int fl = f4 & (F4 / 2 - 1);
         float c4v[4], s4v[4];
         if (fz.cache_f32) {
           const float4 cc = *reinterpret_cast<const float4*>(static_cast<const float*>(fz.cos_sin) + pos * D + 4 * fl);
-          const float4 ss = *reinterpret_cast<const float4*>(static_cast<const float*>(fz.cos_sin) + pos * D + 64 + 4 * fl);
+          const float4 ss = *reinterpret_cast<const float4*>(static_cast<const float*>(fz.cos_sin) + pos * D + D / 2 + 4 * fl);
           c4v[0] = cc.x; c4v[1] = cc.y; c4v[2] = cc.z; c4v[3] = cc.w;
           s4v[0] = ss.x; s4v[1] = ss.y; s4v[2] = ss.z; s4v[3] = ss.w;
         } else {
           const Vec<T, 4> cc = ldvec<T, 4>(static_cast<const T*>(fz.cos_sin) + pos * D + 4 * fl);
-          const Vec<T, 4> ss = ldvec<T, 4>(static_cast<const T*>(fz.cos_sin) + pos * D + 64 + 4 * fl);
+          const Vec<T, 4> ss = ldvec<T, 4>(static_cast<const T*>(fz.cos_sin) + pos * D + D / 2 + 4 * fl);
 #pragma unroll
           for (int j = 0; j < 4; ++j) { c4v[j] = to_f32(cc.v[j]); s4v[j] = to_f32(ss.v[j]); }
         }
-        const bool second = f4 >= 16;
+        const bool second = f4 >= F4 / 2;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float mine = to_f32(out.v[j]);
-          const float theirs = __shfl_xor(mine, 16, 64);
+          const float theirs = __shfl_xor(mine, F4 / 2, 64);
           const float c = round_to<T>(c4v[j]), sn = round_to<T>(s4v[j]);
           const float x1 = second ? theirs : mine, x2 = second ? mine : theirs;
           const float y = second ? round_to<T>(round_to<T>(x2 * c) + round_to<T>(x1 * sn))
@@ -845,15 +854,15 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
       stvec<T, 4>(&sm_qkv[seg * D + 4 * f4], out);
     }
   };
-  auto frags_from_lds = [&](int seg, frag (&y)[4]) {   // (rotated already)
+  auto frags_from_lds = [&](int seg, frag (&y)[NS]) {   // (rotated already)
 #pragma unroll
-    for (int s = 0; s < 4; ++s) y[s] = *reinterpret_cast<const frag*>(&sm_qkv[seg * D + 32 * s + 8 * c4]);
+    for (int s = 0; s < NS; ++s) y[s] = *reinterpret_cast<const frag*>(&sm_qkv[seg * D + 32 * s + 8 * c4]);
   };
 
-  frag qf[4];
+  frag qf[NS];
   if constexpr (!FUSED) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < NS; ++s) {
       if (r16 < G) {
         qf[s] = *reinterpret_cast<const frag*>(q + (int64_t)b * p.q_stride + (int64_t)(head0 + r16) * D + 32 * s + 8 * c4);
       } else {
@@ -865,15 +874,15 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 
   float m = -INFINITY;   // running maximum of head g = r16 (same in the four lanes c of a head)
   float l = 0.f;         // this lane's share of the denominator (its keys 4c..4c+3 of every tile)
-  f32x4 acc[8];
+  f32x4 acc[ND];
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < ND; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // (An empty sequence has no slot to read: it takes its length, or the first prefix sum, which are 0, for one.)
   const int32_t* pt = len > 0 ? p.page_table + page_off : p.mode == 0 ? reinterpret_cast<const int32_t*>(p.seq_lens + b) : p.kv_indptr;
   const int64_t row_stride = p.k_slot_stride;
-  const KVT* kbase = reinterpret_cast<const KVT*>(kbuf) + (int64_t)kvh * p.k_head_stride + 8 * (KROW ? r16 : c4);   // + slot * row_stride (+ 32 s)
-  const KVT* vbase = reinterpret_cast<const KVT*>(vbuf) + (int64_t)kvh * p.v_head_stride + 8 * r16;    // + slot * row_stride
+  const KVT* kbase = reinterpret_cast<const KVT*>(kbuf) + (int64_t)kvh * p.k_head_stride + (KROW ? ch8 : 8 * c4);   // + slot * row_stride (+ 32 s)
+  const KVT* vbase = reinterpret_cast<const KVT*>(vbuf) + (int64_t)kvh * p.v_head_stride + ch8;    // + slot * row_stride
   // Positions and a row's bytes in 32 bits (a sequence is shorter than 2^31 tokens and its slots are numbered from 0): a row's address is one
   // multiply-add.  With one or two waves on a SIMD the instructions of a tile are its time.
   const int wave_first = (int)k0 + wave * 16, end = (int)k1, last_key = max((int)len - 1, 0);
@@ -882,14 +891,14 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   auto row_at = [&](const KVT* base, int32_t slot) {
     return reinterpret_cast<const KVT*>(reinterpret_cast<const char*>(base) + (uint64_t)(unsigned)slot * row_bytes);
   };
-  T* v_wr = &sm_v[wave][(4 * c4) * DV_ROW + 8 * r16];                           // + u rows
-  T* k_wr = &sm_k[KROW ? wave : 0][KROW ? (4 * c4) * DV_ROW + 8 * r16 : 0];     // + u rows
+  T* v_wr = &sm_v[wave][row0 * DV_ROW + ch8];                           // + u rows
+  T* k_wr = &sm_k[KROW ? wave : 0][KROW ? row0 * DV_ROW + ch8 : 0];     // + u rows
   const T* k_rd = &sm_k[KROW ? wave : 0][KROW ? r16 * DV_ROW + 8 * c4 : 0];     // + 32 s
   const T* v_rd = &sm_v[wave][(4 * c4 + (r16 >> 2)) * DV_ROW + 4 * (r16 & 3)];  // + 16 dt
 
   // FUSED: the newest key (position len - 1) belongs to the last split; its 16-key tile is tile
   // `tl` of the split, walked by wave tl & 3 in iteration tl >> 2, row `rl` of the tile.
-  frag knew[4];
+  frag knew[NS];
   Vec<T, VE> vnew;
   bool owner = false;
   int it_new = -1, rl = 0;
@@ -902,56 +911,56 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
   }
 
-  auto load_slots = [&](int it, int32_t& sk, int32_t (&sv)[4]) {
+  auto load_slots = [&](int it, int32_t& sk, int32_t (&sv)[NR]) {
     const int tb = wave_first + it * 64;
     sk = pt[(unsigned)min(tb + r16, last_key)];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) sv[u] = pt[(unsigned)min(tb + 4 * c4 + u, last_key)];
+    for (int u = 0; u < NR; ++u) sv[u] = pt[(unsigned)min(tb + row0 + u, last_key)];
   };
 
-  auto load_kv = [&](const int32_t& sk, const int32_t (&sv)[4], KRaw (&kf)[4], VRaw (&vv)[4]) {
+  auto load_kv = [&](const int32_t& sk, const int32_t (&sv)[NR], KRaw (&kf)[NR], VRaw (&vv)[NR]) {
     const KVT* krow = row_at(kbase, sk);
     if constexpr (KV8 && KROW) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) kf[u] = ld8_nt(row_at(kbase, sv[u]));
+      for (int u = 0; u < NR; ++u) kf[u] = ld8_nt(row_at(kbase, sv[u]));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ld8_nt(row_at(vbase, sv[u]));
+      for (int u = 0; u < NR; ++u) vv[u] = ld8_nt(row_at(vbase, sv[u]));
     } else if constexpr (KV8) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[s] = *reinterpret_cast<const uint2*>(krow + 32 * s);
+      for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const uint2*>(krow + 32 * s);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ld8_nt(row_at(vbase, sv[u]));
+      for (int u = 0; u < NR; ++u) vv[u] = ld8_nt(row_at(vbase, sv[u]));
     } else if constexpr (KROW) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) kf[u] = ldvec_nt<T, VE>(row_at(kbase, sv[u]));
+      for (int u = 0; u < NR; ++u) kf[u] = ldvec_nt<T, VE>(row_at(kbase, sv[u]));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ldvec_nt<T, VE>(row_at(vbase, sv[u]));
+      for (int u = 0; u < NR; ++u) vv[u] = ldvec_nt<T, VE>(row_at(vbase, sv[u]));
     } else {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[s] = *reinterpret_cast<const frag*>(krow + 32 * s);
+      for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const frag*>(krow + 32 * s);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = ldvec<T, VE>(row_at(vbase, sv[u]));
+      for (int u = 0; u < NR; ++u) vv[u] = ldvec<T, VE>(row_at(vbase, sv[u]));
     }
   };
   // One 16-key tile.  A tile past the end of the range is harmless: every key is masked, so the
   // probabilities are zero and the rescale factor is one.
-  auto compute_tile = [&](frag (&kf)[4], Vec<T, VE> (&vv)[4], int it) {
+  auto compute_tile = [&](frag (&kf)[NS], Vec<T, VE> (&vv)[NR], int it) {
     // No multiply-add contraction in the softmax: the fused and the plain instantiation of this
     // kernel must round identically (the compiler otherwise contracts differently per instantiation).
 #pragma clang fp contract(off)
     if constexpr (FUSED) {
       if (owner && it == it_new) {   // this tile's row rl was loaded before the cache held it
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < NS; ++s)
           if (r16 == rl) kf[s] = knew[s];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (4 * c4 + u == rl) vv[u] = vnew;
+        for (int u = 0; u < NR; ++u)
+          if (row0 + u == rl) vv[u] = vnew;
       }
     }
     f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) sc = Mfma<T>::run(kf[s], qf[s], sc);
+    for (int s = 0; s < NS; ++s) sc = Mfma<T>::run(kf[s], qf[s], sc);
 
     const int kb0 = wave_first + it * 64 + 4 * c4;
     float x[4], mx = -INFINITY;
@@ -974,60 +983,67 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
     l = l * alpha + psum;
     m = mx;
-    T pt4[4];
+    T pt4[4], rest4[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pt4[r] = from_f32<T>(pr[r]);
-    const frag4 pb = __builtin_bit_cast(frag4, pt4);
+    for (int r = 0; r < 4; ++r) {
+      pt4[r] = from_f32<T>(pr[r]);
+      rest4[r] = from_f32<T>(PSPLIT ? pr[r] - to_f32(pt4[r]) : 0.f);
+    }
+    const frag4 pb = __builtin_bit_cast(frag4, pt4), pl = __builtin_bit_cast(frag4, rest4);
 
 #pragma unroll
-    for (int u = 0; u < 4; ++u) stvec<T, VE>(v_wr + u * DV_ROW, vv[u]);
+    for (int u = 0; u < NR; ++u) stvec<T, VE>(v_wr + u * DV_ROW, vv[u]);
     __builtin_amdgcn_wave_barrier();
     // the running maximum rarely moves after the first tiles: skip the rescale (a multiplication by
     // exactly 1, so skipping it changes no bit) unless some lane of the wave needs it
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) acc[dt] *= alpha;
+      for (int dt = 0; dt < ND; ++dt) acc[dt] *= alpha;
     }
-    // all eight transposed reads first, then the MFMAs: written read-MFMA-read-MFMA the reads stay in
+    // all transposed reads first, then the MFMAs: written read-MFMA-read-MFMA the reads stay in
     // that order and every MFMA waits one LDS round trip
-    typename TrRead<T>::v4 vt[8];
+    typename TrRead<T>::v4 vt[ND];
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) vt[dt] = TrRead<T>::run(v_rd + 16 * dt);
+    for (int dt = 0; dt < ND; ++dt) vt[dt] = TrRead<T>::run(v_rd + 16 * dt);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) acc[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pb, acc[dt]);
+    for (int dt = 0; dt < ND; ++dt) acc[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pb, acc[dt]);
+    if constexpr (PSPLIT) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) acc[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pl, acc[dt]);
+    }
     __builtin_amdgcn_wave_barrier();
   };
 
   // widen an fp8 tile on use; a 16-bit tile is computed in place
-  auto compute = [&](KRaw (&kraw)[4], VRaw (&vraw)[4], int it) {
+  auto compute = [&](KRaw (&kraw)[NR], VRaw (&vraw)[NR], int it) {
     if constexpr (KV8 && KROW) {
-      Vec<T, VE> vv[4];
+      Vec<T, VE> vv[NR];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) stvec<T, VE>(k_wr + u * DV_ROW, cvt8_from_fp8<T>(kraw[u]));
+      for (int u = 0; u < NR; ++u) stvec<T, VE>(k_wr + u * DV_ROW, cvt8_from_fp8<T>(kraw[u]));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = cvt8_from_fp8<T>(vraw[u]);
+      for (int u = 0; u < NR; ++u) vv[u] = cvt8_from_fp8<T>(vraw[u]);
       __builtin_amdgcn_wave_barrier();
-      frag kf[4];
+      frag kf[NS];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[s] = *reinterpret_cast<const frag*>(k_rd + 32 * s);
+      for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const frag*>(k_rd + 32 * s);
       __builtin_amdgcn_wave_barrier();
       compute_tile(kf, vv, it);
     } else if constexpr (KV8) {
-      frag kf[4];
-      Vec<T, VE> vv[4];
+      frag kf[NS];
+      Vec<T, VE> vv[NR];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[s] = __builtin_bit_cast(frag, cvt8_from_fp8<T>(kraw[s]));
+      for (int s = 0; s < NS; ++s) kf[s] = __builtin_bit_cast(frag, cvt8_from_fp8<T>(kraw[s]));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) vv[u] = cvt8_from_fp8<T>(vraw[u]);
+      for (int u = 0; u < NR; ++u) vv[u] = cvt8_from_fp8<T>(vraw[u]);
       compute_tile(kf, vv, it);
     } else if constexpr (KROW) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) stvec<T, VE>(k_wr + u * DV_ROW, kraw[u]);
+      for (int u = 0; u < NR; ++u) stvec<T, VE>(k_wr + u * DV_ROW, kraw[u]);
       __builtin_amdgcn_wave_barrier();
-      frag kf[4];
+      frag kf[NS];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[s] = *reinterpret_cast<const frag*>(k_rd + 32 * s);
+      for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const frag*>(k_rd + 32 * s);
       __builtin_amdgcn_wave_barrier();
       compute_tile(kf, vraw, it);
     } else {
@@ -1038,9 +1054,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   // Two K/V register buffers: the loads of tile it+1 are in flight while tile it is computed, so a
   // wave keeps 8-16 KiB outstanding at all times.  Addresses past the range are clamped (valid).  (Four buffers for one-byte rows, or two
   // tiles' chains side by side, took longer: a tile's own way through LDS, scores and softmax is what is left.)
-  int32_t skA, svA[4], skB, svB[4];
-  KRaw kfA[4], kfB[4];
-  VRaw vvA[4], vvB[4];
+  int32_t skA, svA[NR], skB, svB[NR];
+  KRaw kfA[NR], kfB[NR];
+  VRaw vvA[NR], vvB[NR];
   load_slots(0, skA, svA);
   load_slots(1, skB, svB);
   const int64_t new_slot = FUSED ? fz.out_loc[b] : 0;   // (read here: behind the tiles' loads its wait would be for all of them)
@@ -1061,32 +1077,32 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     frags_from_lds(r16 < G ? r16 : 0, qf);
     if (r16 >= G) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < NS; ++s)
 #pragma unroll
         for (int j = 0; j < 8; ++j) qf[s][j] = (T)0.f;
     }
     if (owner) {
       frags_from_lds(G, knew);
-      vnew = ldvec<T, VE>(&sm_qkv[(G + 1) * D + 8 * r16]);
+      vnew = ldvec<T, VE>(&sm_qkv[(G + 1) * D + ch8]);
       KVT* kd = const_cast<KVT*>(reinterpret_cast<const KVT*>(kbuf)) + new_slot * row_stride + (int64_t)kvh * p.k_head_stride + 8 * c4;
-      KVT* vd = const_cast<KVT*>(reinterpret_cast<const KVT*>(vbuf)) + new_slot * row_stride + (int64_t)kvh * p.v_head_stride + 8 * r16;
+      KVT* vd = const_cast<KVT*>(reinterpret_cast<const KVT*>(vbuf)) + new_slot * row_stride + (int64_t)kvh * p.v_head_stride + ch8;
       if constexpr (KV8) {
         // quantise once; the attention below sees exactly what a later step will read from the cache
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
+        for (int s = 0; s < NS; ++s) {
           const uint2 qv = quant8_fp8<T>(__builtin_bit_cast(Vec<T, 8>, knew[s]), 1.0f);
           if (r16 == 0) *reinterpret_cast<uint2*>(kd + 32 * s) = qv;
           knew[s] = __builtin_bit_cast(frag, cvt8_from_fp8<T>(qv));
         }
         const uint2 qv = quant8_fp8<T>(vnew, 1.0f);
-        if (c4 == 0) *reinterpret_cast<uint2*>(vd) = qv;
+        if (row0 == 0) *reinterpret_cast<uint2*>(vd) = qv;
         vnew = cvt8_from_fp8<T>(qv);
       } else {
         if (r16 == 0) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) *reinterpret_cast<frag*>(kd + 32 * s) = knew[s];
+          for (int s = 0; s < NS; ++s) *reinterpret_cast<frag*>(kd + 32 * s) = knew[s];
         }
-        if (c4 == 0) stvec<T, VE>(vd, vnew);
+        if (row0 == 0) stvec<T, VE>(vd, vnew);
       }
     }
   }
@@ -1109,7 +1125,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   l = sum_xor<32>(sum_xor<16>(l));
   if (r16 < G) {
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
+    for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) sm_acc[wave][r16][16 * dt + 4 * c4 + r] = acc[dt][r];
     if (c4 == 0) {
@@ -2668,29 +2684,29 @@ static void launch_decode_dc(const T* q, const T* kb, const T* vb, T* o, const D
   if constexpr (D == 128 && !std::is_same<T, float>::value) {
     if (kv8) {
       switch (G) {
-        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 8, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 4, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 2, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 1, CAP, false, true, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
       }
       return;
     }
     if (g_decode_variant == 0) {
       switch (G) {
-        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
-        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 8, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 4, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 2, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 1, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
       }
       return;
     }
 #ifdef MI355_DEV_BUILD
     if (g_decode_variant == 3) {   // ablation: K rows loaded straight into MFMA fragments (16 rows x 64 B per instruction)
       switch (G) {
-        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
-        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
-        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
-        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 8, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 4, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 2, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
+        default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 128, 1, CAP>), grid_pv, block, 0, st, q, kb, vb, o, p); break;
       }
       return;
     }
@@ -2704,11 +2720,20 @@ static void launch_decode_dc(const T* q, const T* kb, const T* vb, T* o, const D
 #endif
     return;
   }
-  switch (G) {
-    case 8: hipLaunchKernelGGL((decode_attn_kernel<T, D, 8, (U > 2 ? 2 : U), CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
-    case 4: hipLaunchKernelGGL((decode_attn_kernel<T, D, 4, U, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
-    case 2: hipLaunchKernelGGL((decode_attn_kernel<T, D, 2, U, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
-    default: hipLaunchKernelGGL((decode_attn_kernel<T, D, 1, U, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
+  if constexpr (D == 64 && !std::is_same<T, float>::value) {
+    switch (G) {
+      case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 64, 8, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+      case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 64, 4, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+      case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 64, 2, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+      default: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 64, 1, CAP, false, false, true>), grid_pv, block, 0, st, q, kb, vb, o, p, FusedQkv()); break;
+    }
+  } else {
+    switch (G) {
+      case 8: hipLaunchKernelGGL((decode_attn_kernel<T, D, 8, (U > 2 ? 2 : U), CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
+      case 4: hipLaunchKernelGGL((decode_attn_kernel<T, D, 4, U, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
+      case 2: hipLaunchKernelGGL((decode_attn_kernel<T, D, 2, U, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
+      default: hipLaunchKernelGGL((decode_attn_kernel<T, D, 1, U, CAP>), grid, block, 0, st, q, kb, vb, o, p); break;
+    }
   }
 }
 
@@ -2731,8 +2756,8 @@ static int launch_decode(const void* q_, const void* kb_, const void* vb_, void*
   const bool vec = D == Dv && aligned16(q) && aligned16(kb) && aligned16(vb) &&
                    p.q_stride % V16<T>::n == 0;
   constexpr int VE = V16<T>::n;
-  // only the matrix-core kernel (head_dim 128, 16-bit) merges the splits itself
-  if (!(vec && D == 128 && !std::is_same<T, float>::value && (kv8 || g_decode_variant == 0) &&
+  // only the matrix-core kernel (head_dim 128, or 64 over a 16-bit cache) merges the splits itself
+  if (!(vec && ((D == 128 && (kv8 || g_decode_variant == 0)) || (D == 64 && !kv8)) && !std::is_same<T, float>::value &&
         p.num_splits > 1 && p.num_splits <= MERGE_MAX_SPLITS))
     p.tickets = nullptr;
   // an fp8 cache outside the matrix-core kernel's shape (head_dim 128, 16-bit, aligned): the wave-per-head kernel
@@ -2761,40 +2786,24 @@ static int launch_decode(const void* q_, const void* kb_, const void* vb_, void*
   return MI355_OK;
 }
 
-template <typename T>
-static int launch_decode_fused(const T* kb, const T* vb, T* o, const DecodeParams& p_in, const FusedQkv& fz,
-                               int64_t bs, bool kv8, hipStream_t st) {
+template <typename T, int D, bool KV8>
+static int launch_decode_fused(const T* kb, const T* vb, T* o, const DecodeParams& p_in, const FusedQkv& fz, int64_t bs, hipStream_t st) {
   DecodeParams p = p_in;
   if (p.num_splits <= 1 || p.num_splits > MERGE_MAX_SPLITS) p.tickets = nullptr;
   const int G = p.hq / p.hkv;
   const dim3 grid((unsigned)p.hkv, (unsigned)bs, (unsigned)p.num_splits), block(256);
-  if (kv8) {
-    switch (G) {
-      case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, false, true, true, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-      case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, false, true, true, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-      case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, false, true, true, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-      case 1: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, false, true, true, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-      default:
-        set_error("decode_attention_fused_qkv: %d query heads per kv head (needs 1, 2, 4 or 8)", G);
-        return MI355_ERR_UNSUPPORTED;
-    }
-    if (p.num_splits > 1 && !p.tickets)
-      hipLaunchKernelGGL((decode_merge_kernel<T>), dim3((unsigned)(bs * p.hq)), dim3(128), 0, st,
-                         p.part_o, p.part_lse, o, p.num_splits, 128);
-    return MI355_OK;
-  }
   switch (G) {
-    case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 8, false, true, false, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-    case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 4, false, true, false, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-    case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 2, false, true, false, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
-    case 1: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, 1, false, true, false, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
+    case 8: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, D, 8, false, true, KV8, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
+    case 4: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, D, 4, false, true, KV8, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
+    case 2: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, D, 2, false, true, KV8, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
+    case 1: hipLaunchKernelGGL((decode_attn_mfma_pv_kernel<T, D, 1, false, true, KV8, true>), grid, block, 0, st, (const T*)nullptr, kb, vb, o, p, fz); break;
     default:
       set_error("decode_attention_fused_qkv: %d query heads per kv head (needs 1, 2, 4 or 8)", G);
       return MI355_ERR_UNSUPPORTED;
   }
   if (p.num_splits > 1 && !p.tickets)
     hipLaunchKernelGGL((decode_merge_kernel<T>), dim3((unsigned)(bs * p.hq)), dim3(128), 0, st,
-                       p.part_o, p.part_lse, o, p.num_splits, 128);
+                       p.part_o, p.part_lse, o, p.num_splits, D);
   return MI355_OK;
 }
 
@@ -2833,7 +2842,6 @@ int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
     // the CUs' worth more of them pays, and more again when the lengths differ and the longest row would run alone.
     // 128 workgroups, head_dim 128, 1 -> 2 splits: 512 keys 11.1 -> 12.1 us, 1 024 17.7 -> 16.9, 2 048 28.3 -> 26.7,
     // 4 096 57.4 -> 47.5, 1 638 to 4 096 52.8 -> 38.4; 144 workgroups (more than the CUs once doubled), 2 048: 29.2 -> 37.0.
-    // (head_dim 64, whose splits take a second launch to merge: 128 workgroups, 2 048 keys 26.2 -> 20.5, 4 096 45.7 -> 30.4.)
     if (wgs >= 112 && wgs <= 128) keep = 1024;
     int64_t most = 2;
     // One-byte rows halve what a workgroup draws (~27 GB/s: its time per key is the chain from row to product, not the
@@ -3029,8 +3037,8 @@ int mi355_decode_attention_fused_qkv(const float* qkv_part, int nsplit, const fl
   const bool kv8 = (dtype & MI355_KV_FP8) != 0;
   const int kv_flags = dtype;
   dtype &= 0xff;
-  MI355_REQUIRE(head_dim == 128 && (dtype == MI355_BF16 || dtype == MI355_F16), MI355_ERR_UNSUPPORTED,
-                "decode_attention_fused_qkv: needs head_dim 128 and a 16-bit dtype");
+  MI355_REQUIRE((head_dim == 128 || (head_dim == 64 && !kv8)) && (dtype == MI355_BF16 || dtype == MI355_F16), MI355_ERR_UNSUPPORTED,
+                "decode_attention_fused_qkv: needs head_dim 128, or 64 over a 16-bit cache, and a 16-bit dtype");
   MI355_REQUIRE(cache_dtype == MI355_F32 || cache_dtype == dtype, MI355_ERR_UNSUPPORTED,
                 "decode_attention_fused_qkv: cos_sin_cache must be fp32 or the tensor dtype");
   MI355_REQUIRE(num_splits >= 1 && num_splits <= MI355_MAX_KV_SPLITS && (num_splits == 1 || (attn_logits && attn_lse)),
@@ -3072,8 +3080,14 @@ int mi355_decode_attention_fused_qkv(const float* qkv_part, int nsplit, const fl
   fz.cache_f32 = cache_dtype == MI355_F32;
   hipStream_t st = (hipStream_t)stream;
   int rc;
-  if (dtype == MI355_BF16) rc = launch_decode_fused<bf16_t>((const bf16_t*)k_buffer, (const bf16_t*)v_buffer, (bf16_t*)o, p, fz, bs, kv8, st);
-  else rc = launch_decode_fused<f16_t>((const f16_t*)k_buffer, (const f16_t*)v_buffer, (f16_t*)o, p, fz, bs, kv8, st);
+  auto run = [&](auto t) {
+    using T = decltype(t);
+    const T* kb = (const T*)k_buffer;
+    const T* vb = (const T*)v_buffer;
+    if (head_dim == 64) return launch_decode_fused<T, 64, false>(kb, vb, (T*)o, p, fz, bs, st);
+    return kv8 ? launch_decode_fused<T, 128, true>(kb, vb, (T*)o, p, fz, bs, st) : launch_decode_fused<T, 128, false>(kb, vb, (T*)o, p, fz, bs, st);
+  };
+  rc = dtype == MI355_BF16 ? run(bf16_t()) : run(f16_t());
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("decode_attention_fused_qkv");
   return MI355_OK;

@@ -70,7 +70,7 @@ class Mi355AttnBackend(AttentionBackend):
         self.kv_fp8 = getattr(model_runner.token_to_kv_pool, "dtype", None) == torch.float8_e4m3fn
         # the decode kernel of these shapes merges its splits in its own launch and passes over empty ones
         self.merges_in_launch = (not (self.is_mla or self.is_latent_window or self.is_layered)
-                                 and getattr(cfg, "head_dim", None) == 128 and getattr(model_runner, "dtype", None) in (torch.bfloat16, torch.float16))
+                                 and getattr(cfg, "head_dim", None) in ((128,) if self.kv_fp8 else (64, 128)) and getattr(model_runner, "dtype", None) in (torch.bfloat16, torch.float16))
         if self.is_mla:
             # what the split plan counts is workgroups per sequence, one per 16 query heads
             self.num_kv_head = (self.num_head + 15) // 16
@@ -537,10 +537,10 @@ class Mi355AttnBackend(AttentionBackend):
     @staticmethod
     def supports_fused_qkv(layer, rotary_emb, dtype) -> bool:
         g = layer.tp_q_head_num // max(layer.tp_k_head_num, 1)
-        return (layer.qk_head_dim == 128 and layer.v_head_dim == 128 and dtype in (torch.bfloat16, torch.float16)
+        return (layer.qk_head_dim in (64, 128) and layer.v_head_dim == layer.qk_head_dim and dtype in (torch.bfloat16, torch.float16)
                 and layer.tp_q_head_num % layer.tp_k_head_num == 0 and g in (1, 2, 4, 8)
                 and not layer.logit_cap and layer.sliding_window_size in (None, -1)
-                and rotary_emb.is_neox_style and rotary_emb.rotary_dim == 128
+                and rotary_emb.is_neox_style and rotary_emb.rotary_dim == layer.qk_head_dim
                 and rotary_emb.cos_sin_cache.dtype in (torch.float32, dtype))
 
     def forward_extend(self, q, k, v, layer, forward_batch, save_kv_cache: bool = True):

@@ -115,6 +115,7 @@ class LlamaAttention(nn.Module):
         pool = forward_batch.token_to_kv_pool
         if (not forward_batch.forward_mode.is_decode()
                 or getattr(pool, "dtype", None) not in (hidden_states.dtype, torch.float8_e4m3fn)
+                or (pool.dtype != hidden_states.dtype and self.head_dim != 128)    # one-byte rows at other head sizes: a kernel of their own
                 or not backend.supports_fused_qkv(self.attn, self.rotary_emb, hidden_states.dtype)):
             return None
         part = decode_linear_deferred(self.qkv_proj, hidden_states, needs_all_reduce=False)

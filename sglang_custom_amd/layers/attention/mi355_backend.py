@@ -70,7 +70,7 @@ class Mi355AttnBackend(AttentionBackend):
         self.kv_fp8 = getattr(model_runner.token_to_kv_pool, "dtype", None) == torch.float8_e4m3fn
         # the decode kernel of these shapes merges its splits in its own launch and passes over empty ones
         self.merges_in_launch = (not (self.is_mla or self.is_latent_window or self.is_layered)
-                                 and getattr(cfg, "head_dim", None) in ((128,) if self.kv_fp8 else (64, 128)) and getattr(model_runner, "dtype", None) in (torch.bfloat16, torch.float16))
+                                 and getattr(cfg, "head_dim", None) == 128 and getattr(model_runner, "dtype", None) in (torch.bfloat16, torch.float16))
         if self.is_mla:
             # what the split plan counts is workgroups per sequence, one per 16 query heads
             self.num_kv_head = (self.num_head + 15) // 16

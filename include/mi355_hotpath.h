@@ -475,7 +475,8 @@ int mi355_linear_packed(void* y, const void* x, const void* w_packed, const void
  * rounds once.  mi355_rmsnorm_ex is the general row norm behind it: x or split-K partials (with
  * optional fp8 scales) in, optional fused add of `residual` (updated in place), normalised rows to
  * `out`, and optionally their per-token fp8 quantisation (q_out [rows, hidden] e4m3fn + q_scale
- * [rows]; identical to mi355_per_token_quant_fp8 applied to `out`) for the fp8 GEMM that follows.
+ * [rows]; identical to mi355_per_token_quant_fp8 applied to `out`) for the fp8 GEMM that follows; out may be
+ * null where x is given and the quantised rows are asked for.
  * mi355_silu_and_mul_quant_fp8 = mi355_silu_and_mul followed by mi355_per_token_quant_fp8 in one
  * launch (the 16-bit activation is never written); q_stride as in mi355_per_token_quant_fp8.
  * replaces: apply_fp8_linear's quantise-then-GEMM pairs (layers/quantization/fp8_utils.py:676-749)

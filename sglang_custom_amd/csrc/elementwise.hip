@@ -162,7 +162,7 @@ __global__ __launch_bounds__(BT) void rmsnorm_vec_kernel(T* __restrict__ out, T*
         ov[c].v[j] = from_f32<T>((vals[c][j] * inv) * to_f32(wv[c].v[j]));
         amax = fmaxf(amax, fabsf(to_f32(ov[c].v[j])));
       }
-      stvec<T, VE>(orow + (int64_t)vi * VE, ov[c]);
+      if (out != nullptr) stvec<T, VE>(orow + (int64_t)vi * VE, ov[c]);   // (null: the consumer takes the quantised row alone)
     }
   }
   if constexpr (VE == 8) {
@@ -658,7 +658,7 @@ int mi355_fused_add_rmsnorm_partials(void* x, void* residual, const void* weight
 int mi355_rmsnorm_ex(void* out, const void* x, void* residual, const void* weight, const float* part,
                      int nsplit, const float* part_x_scale, const float* part_w_scale, uint8_t* q_out,
                      float* q_scale, int64_t rows, int64_t hidden, float eps, int dtype, void* stream) {
-  MI355_REQUIRE(out && weight && (x || part), MI355_ERR_INVALID, "rmsnorm_ex: null pointer");
+  MI355_REQUIRE((out || (q_out && x)) && weight && (x || part), MI355_ERR_INVALID, "rmsnorm_ex: null pointer");
   MI355_REQUIRE(rows >= 0 && hidden > 0, MI355_ERR_INVALID, "rmsnorm_ex: bad shape");
   MI355_REQUIRE(!part || (nsplit >= 1 && nsplit <= 64 && aligned16(part)), MI355_ERR_INVALID,
                 "rmsnorm_ex: bad partials (nsplit=%d)", nsplit);

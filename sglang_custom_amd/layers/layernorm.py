@@ -20,11 +20,11 @@ class RMSNorm(CustomOp):
         self.variance_epsilon = eps
 
     def forward_hip(
-        self, x, residual: Optional[torch.Tensor] = None, quant_fp8: bool = False
+        self, x, residual: Optional[torch.Tensor] = None, quant_fp8: bool = False, dense: bool = True
     ) -> Union[torch.Tensor, Tuple[torch.Tensor, torch.Tensor]]:
         """x: a tensor, or the SplitKPartials of the GEMM that produced it (summed here).
         quant_fp8: also quantise the normalised rows per token for an fp8 GEMM -- the result is then
-        a QuantizedAct (decode-sized inputs only; callers check the ops backend supports it)."""
+        a QuantizedAct (callers check that the ops backend and the GEMM take it); dense=False: without the 16-bit rows."""
         ops = get_ops()
         if isinstance(x, PendingAllReduce):
             # partial sums of a row-parallel projection (layernorm.py:166-190 forward_with_allreduce_fusion)
@@ -38,13 +38,13 @@ class RMSNorm(CustomOp):
             assert part is None or residual is not None
             if part is not None and not quant_fp8 and part.x_scale is None:
                 return ops.fused_add_rmsnorm_partials(part.part, residual, self.weight.data, self.variance_epsilon), residual
-            dense = None if part is not None else (x if x.is_contiguous() else x.contiguous())
-            out, xq, xs = ops.rmsnorm_ex(self.weight.data, self.variance_epsilon, x=dense, residual=residual,
+            whole = None if part is not None else (x if x.is_contiguous() else x.contiguous())
+            out, xq, xs = ops.rmsnorm_ex(self.weight.data, self.variance_epsilon, x=whole, residual=residual,
                                          part=part.part if part is not None else None,
                                          part_x_scale=part.x_scale if part is not None else None,
                                          part_w_scale=part.w_scale if part is not None else None,
-                                         quant_fp8=quant_fp8)
-            y = QuantizedAct(xq, xs, out.dtype, out) if quant_fp8 else out
+                                         quant_fp8=quant_fp8, **({} if dense else {"dense": False}))
+            y = QuantizedAct(xq, xs, self.weight.dtype, out) if quant_fp8 else out
             return (y, residual) if residual is not None else y
         if not x.is_contiguous():
             x = x.contiguous()

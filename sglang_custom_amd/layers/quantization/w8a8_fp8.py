@@ -73,18 +73,26 @@ def gate_up_silu_mul_prefill(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
     """act_fn(gate_up_proj(x)) (models/llama.py:94-98) for a prefill-sized fp8 W8A8 gate_up
     projection: per-token quantisation, then ONE launch that multiplies, applies the scales and
     SiLU-and-mul.  None when the shape or the switch says to take the unfused path."""
-    if not isinstance(x, torch.Tensor):   # a QuantizedAct: the decode path, served by the packed kernels
-        return None
-    x2 = x.view(-1, x.shape[-1])
+    quantised = not isinstance(x, torch.Tensor)   # a QuantizedAct of the norm in front (decode: served by the packed kernels)
+    x2 = x.xq if quantised else x.view(-1, x.shape[-1])
     w = layer.weight
     if (PREFILL_GEMM == "library" or not x2.is_cuda or x2.shape[0] <= SKINNY_MAX_M
             or getattr(layer, "bias", None) is not None or w.dtype != FP8_DTYPE
-            or not _tiled_ok(x2.shape[0], w.shape[0], w.shape[1], x2.dtype, True)):
+            or not _tiled_ok(x2.shape[0], w.shape[0], w.shape[1], x.dtype, True)):
         return None
     ops = get_ops()
-    xq, xs = ops.per_token_quant_fp8(x2)
-    y = ops.fp8_scaled_mm_tiled(xq, w, xs, layer.weight_scale.view(-1), x2.dtype, None, silu_mul=True, split_tail=True)
+    xq, xs = (x.xq, x.x_scale) if quantised else ops.per_token_quant_fp8(x2)
+    y = ops.fp8_scaled_mm_tiled(xq, w, xs, layer.weight_scale.view(-1), x.dtype, None, silu_mul=True, split_tail=True)
     return y.view(*x.shape[:-1], y.shape[-1])
+
+
+def prefill_takes_quantised_rows(layer, m: int, dtype) -> bool:
+    """Whether a prefill-sized fp8 projection takes rows that the kernel in front of it (norm, SiLU-mul) has quantised itself: a launch and a
+    pass over the rows less than per_token_quant_fp8 behind it, for the same bits.  (What the limits are: 16-byte rows of 16-bit
+    input, at most 16384 of them held by that kernel.)"""
+    w = layer.weight
+    return (isinstance(layer.quant_method, W8A8Fp8LinearMethod) and m > SKINNY_MAX_M and w.is_cuda and w.dtype == FP8_DTYPE
+            and dtype in (torch.bfloat16, torch.float16) and w.shape[1] % 8 == 0 and w.shape[1] <= 16384)
 
 
 class W8A8Fp8LinearMethod:
@@ -122,7 +130,7 @@ class W8A8Fp8LinearMethod:
             if wp is not None and xq.shape[0] <= SKINNY_MAX_M and xq.shape[1] == layer.k_padded:
                 return ops.fp8_scaled_mm_packed(xq, wp, layer.weight.shape[0], xs, layer.weight_scale, out_dtype, bias)
             assert xq.shape[1] == layer.weight.shape[1], "a padded activation is for the packed decode GEMM only"
-            return ops.fp8_scaled_mm(xq, layer.weight, xs, layer.weight_scale, out_dtype, bias)
+            return self._many_rows(layer, xq, xs, out_dtype, bias)
         x2 = x.view(-1, x.shape[-1])
         wp = getattr(layer, "weight_packed", None)
         if wp is not None and x2.shape[0] <= SKINNY_MAX_M and x2.is_cuda:   # decode: the packed kernel (K padded if need be)
@@ -130,13 +138,19 @@ class W8A8Fp8LinearMethod:
             y = ops.fp8_scaled_mm_packed(xq, wp, layer.weight.shape[0], xs, layer.weight_scale, x.dtype, bias)
             return y.view(*x.shape[:-1], y.shape[-1])
         xq, xs = ops.per_token_quant_fp8(x2)
-        y = None
-        if (PREFILL_GEMM != "library" and x2.shape[0] > SKINNY_MAX_M and x2.is_cuda
-                and _tiled_ok(x2.shape[0], layer.weight.shape[0], x2.shape[1], x2.dtype, False)):
-            y = ops.fp8_scaled_mm_tiled(xq, layer.weight, xs, layer.weight_scale.view(-1), x.dtype, bias, split_tail=True)
-        if (y is None and x2.shape[0] > SKINNY_MAX_M and x2.is_cuda and x2.shape[1] % 16 == 0
-                and layer.weight.shape[0] % 16 == 0):
-            y = _library_scaled_mm(xq, layer.weight, xs, layer.weight_scale, x.dtype, bias)
-        if y is None:
-            y = ops.fp8_scaled_mm(xq, layer.weight, xs, layer.weight_scale, x.dtype, bias)
+        y = self._many_rows(layer, xq, xs, x.dtype, bias)
         return y.view(*x.shape[:-1], y.shape[-1])
+
+    @staticmethod
+    def _many_rows(layer, xq, xs, out_dtype, bias):
+        """Quantised rows [M, K] against the row-major weight: the tiled kernel, the library or the plain kernel."""
+        ops = get_ops()
+        m, k = xq.shape
+        y = None
+        if PREFILL_GEMM != "library" and m > SKINNY_MAX_M and xq.is_cuda and _tiled_ok(m, layer.weight.shape[0], k, out_dtype, False):
+            y = ops.fp8_scaled_mm_tiled(xq, layer.weight, xs, layer.weight_scale.view(-1), out_dtype, bias, split_tail=True)
+        if y is None and m > SKINNY_MAX_M and xq.is_cuda and k % 16 == 0 and layer.weight.shape[0] % 16 == 0:
+            y = _library_scaled_mm(xq, layer.weight, xs, layer.weight_scale, out_dtype, bias)
+        if y is None:
+            y = ops.fp8_scaled_mm(xq, layer.weight, xs, layer.weight_scale, out_dtype, bias)
+        return y

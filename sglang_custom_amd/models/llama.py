@@ -28,7 +28,7 @@ from ..layers.quantization.unquant import (
     pack_for_decode,
     pack_gate_up_for_decode,
 )
-from ..layers.quantization.w8a8_fp8 import W8A8Fp8LinearMethod
+from ..layers.quantization.w8a8_fp8 import W8A8Fp8LinearMethod, prefill_takes_quantised_rows
 from ..layers.quantization.w8a8_fp8 import gate_up_silu_mul_prefill as gate_up_silu_mul_prefill_fp8
 from ..layers.radix_attention import RadixAttention
 from ..ops_backend import get_ops
@@ -61,6 +61,8 @@ class LlamaMLP(nn.Module):
                 # SiLU-mul and the down projection's per-token quantisation in one launch
                 xq, xs = get_ops().silu_and_mul_quant_fp8(gate_up, pad_to=self.down_proj.k_padded)
                 x = QuantizedAct(xq, xs, gate_up.dtype)
+            elif gate_up.dim() == 2 and prefill_takes_quantised_rows(self.down_proj, gate_up.shape[0], gate_up.dtype):
+                x = QuantizedAct(*get_ops().silu_and_mul_quant_fp8(gate_up), gate_up.dtype)
             else:
                 x = self.act_fn(gate_up)
         deferred = decode_linear_deferred(self.down_proj, x)   # summed by the next layer's norm
@@ -129,15 +131,19 @@ class LlamaAttention(nn.Module):
         """Prefill fast path: ONE launch computes the qkv projection, rotates q and k and writes the new
         k / v rows into the KV cache (the rotation and the cache write run in the GEMM's epilogue).
         Returns the qkv tensor (q, k rotated) or None when it does not apply."""
-        if (PREFILL_QKV_ROPE == "off" or not isinstance(hidden_states, torch.Tensor) or not hidden_states.is_cuda
+        quantised = isinstance(hidden_states, QuantizedAct)     # by the norm in front
+        if (PREFILL_QKV_ROPE == "off" or not (quantised or isinstance(hidden_states, torch.Tensor))
                 or forward_batch.forward_mode.is_decode() or getattr(self.qkv_proj, "bias", None) is not None):
             return None
-        x = hidden_states.view(-1, hidden_states.shape[-1])
+        dtype = hidden_states.dtype
+        x = hidden_states.xq if quantised else hidden_states.view(-1, hidden_states.shape[-1])
+        if not x.is_cuda:
+            return None
         m, k = x.shape
         qm = self.qkv_proj.quant_method
         fp8 = isinstance(qm, W8A8Fp8LinearMethod)
         w = self.qkv_proj.weight
-        if not fp8 and (type(qm) is not UnquantizedLinearMethod or w.dtype != x.dtype):
+        if not fp8 and (type(qm) is not UnquantizedLinearMethod or w.dtype != dtype):
             return None
         if fp8 and w.dtype != torch.float8_e4m3fn:
             return None
@@ -145,17 +151,17 @@ class LlamaAttention(nn.Module):
         rope = self.rotary_emb
         ops = get_ops()
         n_tiles = ((m + 255) // 256) * (w.shape[0] // 256)
-        if (kb.dtype != x.dtype or n_tiles < PREFILL_QKV_MIN_TILES
+        if (kb.dtype != dtype or n_tiles < PREFILL_QKV_MIN_TILES
                 or not ops.qkv_proj_rope_tiled_supported(m, k, self.num_heads, self.num_kv_heads, self.head_dim,
-                                                         rope.cos_sin_cache.shape[1], rope.is_neox_style, x.dtype, fp8)):
+                                                         rope.cos_sin_cache.shape[1], rope.is_neox_style, dtype, fp8)):
             return None
         xs = ws = None
         if fp8:
-            x, xs = ops.per_token_quant_fp8(x)
+            x, xs = (x, hidden_states.x_scale) if quantised else ops.per_token_quant_fp8(x)
             ws = self.qkv_proj.weight_scale.view(-1)
         return ops.qkv_proj_rope_tiled(x, w, self.num_heads, self.num_kv_heads, self.head_dim, positions.flatten(),
                                        rope.cos_sin_cache, rope.is_neox_style, kb, vb, forward_batch.out_cache_loc,
-                                       x_scale=xs, w_scale=ws, out_dtype=hidden_states.dtype, split_tail=True)
+                                       x_scale=xs, w_scale=ws, out_dtype=dtype, split_tail=True)
 
     def forward(self, positions, hidden_states, forward_batch):
         attn_output = self._fused_decode(positions, hidden_states, forward_batch)
@@ -200,16 +206,23 @@ class LlamaDecoderLayer(nn.Module):
         m = hidden_states.shape[0]
         q_in = takes_fp8_rows_of_k(self.self_attn.qkv_proj, m)      # norm also quantises for the fp8 GEMM behind it
         q_mlp = takes_fp8_rows_of_k(self.mlp.gate_up_proj, m)
+        dense = True
+        if m > SKINNY_MAX_M and get_tensor_model_parallel_world_size() == 1:     # a prompt: the norms leave quantised rows alone
+            dtype = self.input_layernorm.weight.dtype
+            q_in = prefill_takes_quantised_rows(self.self_attn.qkv_proj, m, dtype)
+            q_mlp = prefill_takes_quantised_rows(self.mlp.gate_up_proj, m, dtype)
+            dense = False
         if residual is None:
             residual = hidden_states
-            hidden_states = self.input_layernorm(hidden_states, quant_fp8=True) if q_in else self.input_layernorm(hidden_states)
+            hidden_states = (self.input_layernorm(hidden_states, quant_fp8=True, dense=dense) if q_in
+                             else self.input_layernorm(hidden_states))
         elif q_in:
-            hidden_states, residual = self.input_layernorm(hidden_states, residual, quant_fp8=True)
+            hidden_states, residual = self.input_layernorm(hidden_states, residual, quant_fp8=True, dense=dense)
         else:
             hidden_states, residual = self.input_layernorm(hidden_states, residual)
         hidden_states = self.self_attn(positions, hidden_states, forward_batch)
         if q_mlp:
-            hidden_states, residual = self.post_attention_layernorm(hidden_states, residual, quant_fp8=True)
+            hidden_states, residual = self.post_attention_layernorm(hidden_states, residual, quant_fp8=True, dense=dense)
         else:
             hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
         hidden_states = self.mlp(hidden_states)

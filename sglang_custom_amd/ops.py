@@ -935,15 +935,17 @@ def fp8_packed_partials(xq: torch.Tensor, wq_packed: torch.Tensor, n: int) -> Op
 def rmsnorm_ex(weight: torch.Tensor, eps: float, x: Optional[torch.Tensor] = None,
                residual: Optional[torch.Tensor] = None, part: Optional[torch.Tensor] = None,
                part_x_scale: Optional[torch.Tensor] = None, part_w_scale: Optional[torch.Tensor] = None,
-               quant_fp8: bool = False):
-    """General decode row norm: input x or split-K partials [splits, M, hidden] (with the fp8 GEMM's
+               quant_fp8: bool = False, dense: bool = True):
+    """General row norm: input x or split-K partials [splits, M, hidden] (with the fp8 GEMM's
     scales when they come from one), optional fused add of residual (updated in place), and optionally
-    the per-token fp8 quantisation of the result.  Returns (out, xq or None, x_scale or None)."""
+    the per-token fp8 quantisation of the result; dense=False: that alone (of an input x).
+    Returns (out or None, xq or None, x_scale or None)."""
     src = part if part is not None else x
     _gpu(src, weight, residual)
     rows, hidden = (part.shape[1], part.shape[2]) if part is not None else x.shape
     dt = weight.dtype
-    out = torch.empty((rows, hidden), dtype=dt, device=weight.device)
+    assert dense or (quant_fp8 and part is None)
+    out = torch.empty((rows, hidden), dtype=dt, device=weight.device) if dense else None
     if part is not None:
         assert part.is_contiguous() and part.dtype == torch.float32
     else:
@@ -955,7 +957,7 @@ def rmsnorm_ex(weight: torch.Tensor, eps: float, x: Optional[torch.Tensor] = Non
         xq = torch.empty((rows, hidden), dtype=torch.float8_e4m3fn, device=weight.device)
         xs = torch.empty((rows, 1), dtype=torch.float32, device=weight.device)
     if rows:
-        check(_lib_().mi355_rmsnorm_ex(out.data_ptr(), _p(x), _p(residual), weight.data_ptr(), _p(part),
+        check(_lib_().mi355_rmsnorm_ex(_p(out), _p(x), _p(residual), weight.data_ptr(), _p(part),
                                        part.shape[0] if part is not None else 0, _p(part_x_scale), _p(part_w_scale),
                                        _p(xq), _p(xs), rows, hidden, float(eps), _dt(weight), _stream(weight)),
               "rmsnorm_ex")

@@ -192,7 +192,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_temperature_kernel(
 // every chunk normalises itself with what all of them left.  (A chunk without a number in it has no maximum to take off: its
 // -inf entries count zero and a NaN makes its sum NaN, and with it the row, as one pass over the row has it.)  One workgroup per
 // row reads its 0.5 MB three times with 4 bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
-// 14 + 14 us (33 MB read twice, the second time from L2, then read and written; 16 + 16 with a precise division per entry in
+// 13 + 14 us (33 MB read twice, the second time from L2, then read and written; 16 + 16 with a precise division per entry in
 // both), bound by the exponentials and by the latency of a chunk's one round of loads.
 constexpr int MAX_CHUNKS = 16;
 struct ChunkSpan {
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
 // (no probability does) takes sample_whole_row.
 // The one-workgroup routine meets each of its four levels' 128256 entries in 256 bins of two binades, a handful of which
 // take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics.  Launch 1 beside the
-// softmax takes 20 us for that (apart 16 + 10), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 14 from the
+// softmax takes 20 us for that (apart 14 + 13), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 14 from the
 // lists, a chain of some twenty barriers (28 from the row, one CU's pass over 0.5 MB; 58 when thousands are kept).
 constexpr int SB_BINS = 2048, SB_SHIFT = 19, SB_LIST = 8192, SB_SHORT = 512, SB_TILE = 256, SB_MAX_TILES = 4096;
 constexpr int SB_SUM_BITS = 40;
@@ -628,7 +628,7 @@ __device__ __forceinline__ void chunk_list(const Vec<float, 4> (&v)[KEEP], float
 }
 
 // NORM: `data` holds logits, which become probabilities on the way (launch 2 of softmax_temperature); BINS: bins and lists of the
-// probabilities.  Both at once: 64 rows x 128256 20 us, apart 16 + 10.
+// probabilities.  Both at once: 64 rows x 128256 20 us, apart 14 + 13.
 template <bool NORM, bool BINS>
 __global__ __launch_bounds__(SAMP_THREADS) void sample_chunk_kernel(float* __restrict__ data, const float2* __restrict__ partials,
                                                                     const float* __restrict__ temperatures, const int32_t* __restrict__ top_ks,

@@ -943,7 +943,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
   };
   // One 16-key tile.  A tile past the end of the range is harmless: every key is masked, so the
-  // probabilities are zero and the rescale factor is one.
+  // probabilities are zero, the value rows too, and the rescale factor is one.
   auto compute_tile = [&](frag (&kf)[NS], Vec<T, VE> (&vv)[NR], int it) {
     // No multiply-add contraction in the softmax: the fused and the plain instantiation of this
     // kernel must round identically (the compiler otherwise contracts differently per instantiation).
@@ -991,6 +991,16 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
     const frag4 pb = __builtin_bit_cast(frag4, pt4), pl = __builtin_bit_cast(frag4, rest4);
 
+    // Rows past the end of the range are other rows' contents (clamped addresses; FUSED: the newest token's slot as its last owner left
+    // it): their weights are zero, but zero times an infinity or a NaN is none.
+    const int live_rows = end - wave_first - it * 64;    // (wave-uniform)
+    if (live_rows < 16) {
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+        if (row0 + u >= live_rows)
+#pragma unroll
+          for (int j = 0; j < VE; ++j) vv[u].v[j] = from_f32<T>(0.f);
+    }
 #pragma unroll
     for (int u = 0; u < NR; ++u) stvec<T, VE>(v_wr + u * DV_ROW, vv[u]);
     __builtin_amdgcn_wave_barrier();

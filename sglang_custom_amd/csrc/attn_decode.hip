@@ -687,6 +687,36 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
 // every quarter-wave touch 16 rows x 16 bytes, i.e. sixteen cache-line look-ups for 256 bytes;
 // measured 58.8 -> 56.4 us at batch 64 x 1064 keys, 8 kv heads.
 // ------------------------------------------------------------------------------------------
+// Two weights 0 <= p <= 1 as 16-bit terms: p UP = hi + (mid + low) / MID, packed pairs.  In bf16 they hold all 24 bits of p; in fp16 too down
+// to 2^-25 (22 bits to 2^-28), below that to 2^-50.  hi is never zero (what it has too much is in mid).
+template <typename T> struct WeightTerms;
+template <> struct WeightTerms<bf16_t> {
+  static constexpr float UP = 1.f, MID = 1.f, TINY = 0x1p-126f;
+  static __device__ __forceinline__ unsigned pack(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, rt_bf16x2));
+  }
+  static __device__ __forceinline__ float first(unsigned u) { return __uint_as_float(u << 16); }
+  static __device__ __forceinline__ float second(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
+};
+template <> struct WeightTerms<f16_t> {
+  static constexpr float UP = 0x1p14f, MID = 0x1p11f, TINY = 0x1p-24f;
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  static __device__ __forceinline__ unsigned pack(float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, h2)); }
+  static __device__ __forceinline__ float first(unsigned u) { return (float)__builtin_bit_cast(h2, u)[0]; }
+  static __device__ __forceinline__ float second(unsigned u) { return (float)__builtin_bit_cast(h2, u)[1]; }
+};
+template <typename T> __device__ __forceinline__ void weight_terms(float a, float b, unsigned& hi, unsigned& mid, unsigned& low) {
+#pragma clang fp contract(off)
+  using W = WeightTerms<T>;
+  a *= W::UP;
+  b *= W::UP;
+  hi = W::pack(fmaxf(a, W::TINY), fmaxf(b, W::TINY));
+  a = (a - W::first(hi)) * W::MID;
+  b = (b - W::second(hi)) * W::MID;
+  mid = W::pack(a, b);
+  low = W::pack(a - W::first(mid), b - W::second(mid));
+}
+
 template <int D> constexpr int dv_row() { return D + 16; }   // V tile row in LDS (elements): 288 or 160 B -> conflict-free transposed reads
 
 //
@@ -702,10 +732,14 @@ template <int D> constexpr int dv_row() { return D + 16; }   // V tile row in LD
 // its first split is finished there, without a partial and a merge.  A captured launch of 4 splits on a batch that needs one:
 // 128 workgroups, e4m3fn rows, 300 / 4096 keys 14.0 / 68.2 us with sequences outside splits and the merge, 9.1 / 47.7 so (unsplit
 // 8.8 / 47.9); 512 workgroups, 16-bit rows, 300 keys 47.0 -> 16.7 (15.5).
-// D = 64: eight lanes a row, and the weights enter P.V as the sum of two 16-bit numbers: the vector-ALU kernel that served this size multiplied
-// fp32 weights, and two terms leave an error of at most 2^-16 of a weight in bf16 (2^-22 in fp16).  16 layers of 32 / 8 heads, a whole
-// step with the rotation, the sum of the projection's splits and the merge in this launch: 1 x 131 tokens 844 -> 769 us, 1 x 2000 936 -> 837,
-// 32 x 360 1043 -> 927, 33 x 1494 1442 -> 1201.
+// D = 64: eight lanes a row, and P.V multiplies fp32 weights, as the vector-ALU kernel does that serves other sizes: a weight is the sum of
+// three 16-bit terms (WeightTerms).  The matrix has columns to spare: every head's query is in two or four of them, so that all of
+// these have its scores, and each of a head's columns takes one term (G = 8, two columns a head: the third term in products of its own).  A
+// term's sums are its column's, so that fp16 terms can be scaled apart, and an infinite value row, which the first term (never
+// zero) makes infinite, is not lost to the second's sign.
+// 16 layers of 32 / 8 heads, a whole step with the rotation, the sum of the projection's splits and the merge in this launch, against the
+// vector-ALU kernel behind and in front of launches for those: 1 x 131 tokens 844 -> 768 us, 1 x 2000 936 -> 817, 32 x 360 1043 -> 925,
+// 33 x 1494 1442 -> 1193 (with two terms in one column's sum 757, 812, 912, 1185).
 template <typename T, int D, int G, bool CAP, bool FUSED = false, bool KV8 = false, bool KROW = false>
 __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __restrict__ q,
                                                                   const T* kbuf, const T* vbuf,
@@ -716,7 +750,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   constexpr int VE = 8, DV_ROW = dv_row<D>();
   constexpr int LPR = D / VE, NR = D / 32;    // lanes of a row; rows of a tile that a lane loads
   constexpr int NS = D / 32, ND = D / 16;     // score k-steps; 16-feature tiles of the result
-  constexpr bool PSPLIT = D == 64;
+  constexpr bool TERMS = D == 64;                           // weights as three 16-bit terms
+  constexpr int GC = !TERMS ? 16 : G > 4 ? 8 : 4;           // columns from one term of a head to its next
   static_assert((D == 128 || D == 64) && (D == 128 || KROW), "head dimensions 64 and 128");
   using frag = typename Mfma<T>::frag;
   using frag4 = typename Mfma16<T>::frag;
@@ -741,6 +776,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   const int b = blockIdx.y, split = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r16 = lane & 15, c4 = lane >> 4;
+  const int hcol = r16 % GC, term = r16 / GC;               // the lane's column: head head0 + hcol if that is below G
   const int row0 = NR * (lane / LPR), ch8 = VE * (lane % LPR);    // a lane's rows row0 .. + NR - 1 of a tile, its features from ch8 on
 
   int64_t page_off, len;
@@ -863,8 +899,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   if constexpr (!FUSED) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      if (r16 < G) {
-        qf[s] = *reinterpret_cast<const frag*>(q + (int64_t)b * p.q_stride + (int64_t)(head0 + r16) * D + 32 * s + 8 * c4);
+      if (hcol < G) {
+        qf[s] = *reinterpret_cast<const frag*>(q + (int64_t)b * p.q_stride + (int64_t)(head0 + hcol) * D + 32 * s + 8 * c4);
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) qf[s][j] = (T)0.f;
@@ -872,11 +908,15 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
   }
 
-  float m = -INFINITY;   // running maximum of head g = r16 (same in the four lanes c of a head)
+  float m = -INFINITY;   // running maximum of the column's head (same in the four lanes c of a column)
   float l = 0.f;         // this lane's share of the denominator (its keys 4c..4c+3 of every tile)
-  f32x4 acc[ND];
+  f32x4 acc[ND], acc_low[TERMS && GC == 8 ? ND : 1];
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (TERMS && GC == 8) {
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) acc_low[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // (An empty sequence has no slot to read: it takes its length, or the first prefix sum, which are 0, for one.)
   const int32_t* pt = len > 0 ? p.page_table + page_off : p.mode == 0 ? reinterpret_cast<const int32_t*>(p.seq_lens + b) : p.kv_indptr;
@@ -983,13 +1023,23 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     }
     l = l * alpha + psum;
     m = mx;
-    T pt4[4], rest4[4];
+    frag4 pb, pl;
+    if constexpr (TERMS) {
+      uint2 hi, mid, low;
+      weight_terms<T>(pr[0], pr[1], hi.x, mid.x, low.x);
+      weight_terms<T>(pr[2], pr[3], hi.y, mid.y, low.y);
+      if constexpr (GC == 8) {
+        pb = __builtin_bit_cast(frag4, term == 0 ? hi : mid);
+        pl = __builtin_bit_cast(frag4, low);
+      } else {
+        pb = __builtin_bit_cast(frag4, term == 0 ? hi : term == 2 ? low : mid);   // (mid on both sides of hi, all round)
+      }
+    } else {
+      T pt4[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      pt4[r] = from_f32<T>(pr[r]);
-      rest4[r] = from_f32<T>(PSPLIT ? pr[r] - to_f32(pt4[r]) : 0.f);
+      for (int r = 0; r < 4; ++r) pt4[r] = from_f32<T>(pr[r]);
+      pb = __builtin_bit_cast(frag4, pt4);
     }
-    const frag4 pb = __builtin_bit_cast(frag4, pt4), pl = __builtin_bit_cast(frag4, rest4);
 
     // Rows past the end of the range are other rows' contents (clamped addresses; FUSED: the newest token's slot as its last owner left
     // it): their weights are zero, but zero times an infinity or a NaN is none.
@@ -1008,7 +1058,10 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     // exactly 1, so skipping it changes no bit) unless some lane of the wave needs it
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
-      for (int dt = 0; dt < ND; ++dt) acc[dt] *= alpha;
+      for (int dt = 0; dt < ND; ++dt) {
+        acc[dt] *= alpha;
+        if constexpr (TERMS && GC == 8) acc_low[dt] *= alpha;
+      }
     }
     // all transposed reads first, then the MFMAs: written read-MFMA-read-MFMA the reads stay in
     // that order and every MFMA waits one LDS round trip
@@ -1018,9 +1071,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt) acc[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pb, acc[dt]);
-    if constexpr (PSPLIT) {
+    if constexpr (TERMS && GC == 8) {
 #pragma unroll
-      for (int dt = 0; dt < ND; ++dt) acc[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pl, acc[dt]);
+      for (int dt = 0; dt < ND; ++dt) acc_low[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pl, acc_low[dt]);
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -1084,8 +1137,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (FUSED) {
     __syncthreads();
-    frags_from_lds(r16 < G ? r16 : 0, qf);
-    if (r16 >= G) {
+    frags_from_lds(hcol < G ? hcol : 0, qf);
+    if (hcol >= G) {
 #pragma unroll
       for (int s = 0; s < NS; ++s)
 #pragma unroll
@@ -1133,6 +1186,16 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   }
 
   l = sum_xor<32>(sum_xor<16>(l));
+  if constexpr (TERMS) {
+    // (in columns 0 .. GC - 1) the terms' sums of a head, from the columns 4 (either way: mid) and 8 on
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float hi = acc[dt][r], rest = GC == 8 ? dpp<0x128>(hi) + acc_low[dt][r] : dpp<0x124>(hi) + dpp<0x128>(hi);
+        acc[dt][r] = (fabsf(hi) < INFINITY ? __builtin_fmaf(rest, 1.f / WeightTerms<T>::MID, hi) : hi) * (1.f / WeightTerms<T>::UP);
+      }
+  }
   if (r16 < G) {
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)

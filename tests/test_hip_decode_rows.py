@@ -54,3 +54,65 @@ def test_newest_slot_held_no_numbers(ops, D, dtype, fp8, hq, hkv):
                 assert not o.isnan().any(), (splits, tickets is not None, stale)
                 got.append(o)
             assert all(torch.equal(got[0], o) for o in got[1:])
+
+
+def _paged(ops, q, kb, vb, lens, r2t, rpi, splits, tickets=None, scale=1.0):
+    bs, hq, D = q.shape
+    o = torch.empty_like(q)
+    logits, lse = torch.empty(bs, hq, splits, D, device=DEV), torch.empty(bs, hq, splits, device=DEV)
+    ops.decode_attention_paged(q, kb, vb, o, r2t, rpi, lens, logits, lse, splits, scale, tickets=tickets)
+    return o
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (8, 1), (2, 2)])
+@pytest.mark.parametrize("D,dtype,fp8", KINDS[:4], ids=IDS[:4])
+def test_infinite_value_rows(ops, D, dtype, fp8, hq, hkv):
+    """An infinite value makes its feature infinite, whatever its key's weight (the largest included), and touches no other."""
+    lens = [1, 5, 16, 17, 64, 65, 90, 130]
+    r2t, rpi, _, slots = _batch(lens, 1)
+    g = torch.Generator().manual_seed(D + hq)
+    q = (torch.randn(len(lens), hq, D, generator=g) * 0.3).to(DEV, dtype)
+    kb, vb = (torch.randn(slots, hkv, D, generator=g).to(DEV, dtype) for _ in range(2))
+    lens_t = torch.tensor(lens, device=DEV)
+    for splits in (1, 3):
+        plain = _paged(ops, q, kb, vb, lens_t, r2t, rpi, splits, scale=D ** -0.5)
+        for key in (0, 4, 15, 16, 64, 89):      # (the sequences longer than that have it)
+            v2, has = vb.clone(), [b for b, n in enumerate(lens) if n > key]
+            rows = r2t[has, key].long()
+            v2[rows, :, 3], v2[rows, :, D - 1] = float("inf"), float("-inf")
+            got = _paged(ops, q, kb, v2, lens_t, r2t, rpi, splits, scale=D ** -0.5)
+            assert (got[has][..., 3] == float("inf")).all() and (got[has][..., D - 1] == float("-inf")).all(), (splits, key)
+            got[has, :, 3], got[has, :, D - 1] = plain[has, :, 3], plain[has, :, D - 1]
+            assert torch.equal(got, plain)
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (8, 1), (2, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_weights_of_fp32(ops, dtype, hq, hkv):
+    """Head dimension 64 multiplies values by fp32 weights.  The terms of every sum are alike in size (values grow as weights fall) and cancel, so
+    that the result is the sum's error: 0.5 to 0.8 times 2^-20 of the terms' root sum of squares in fp32, 5 with weights of 16 bits in
+    bf16 and 7.5 with two fp16 terms (each in torch on the CPU, the same values)."""
+    D, lens = 64, [200, 77, 129]
+    r2t, rpi, _, slots = _batch(lens, 2)
+    g = torch.Generator().manual_seed(3)
+    kb, vb = torch.zeros(slots, hkv, D, dtype=dtype), torch.zeros(slots, hkv, D, dtype=dtype)
+    ref, size = torch.zeros(len(lens), hkv, D, dtype=torch.float64), torch.zeros(len(lens), hkv, D, dtype=torch.float64)
+    for b, n in enumerate(lens):
+        s = r2t[b, :n].long().cpu()
+        for h in range(hkv):
+            t = -(6 * torch.rand(n, generator=g)).to(dtype).double()
+            t[n // 3] = 0
+            w = t.exp()
+            v = (torch.randn(n, D, generator=g, dtype=torch.float64) / w[:, None]).to(dtype).double()
+            for k in torch.argsort(w)[:5].flip(0):
+                v[k] = 0
+                v[k] = (-(w[:, None] * v).sum(0) / w[k]).to(dtype).double()
+            kb[s, h, 0], vb[s, h] = t.to(dtype), v.to(dtype)
+            ref[b, h] = (w[:, None] * v).sum(0) / w.sum()
+            size[b, h] = (w[:, None] * v).square().sum(0).sqrt() / w.sum()
+    q = torch.zeros(len(lens), hq, D, dtype=dtype)
+    q[..., 0] = 1
+    ref, size = (t.repeat_interleave(hq // hkv, 1) for t in (ref, size))
+    for splits in (1, 3):
+        got = _paged(ops, q.to(DEV), kb.to(DEV), vb.to(DEV), torch.tensor(lens, device=DEV), r2t, rpi, splits)
+        assert ((got.cpu().double() - ref).abs() / size).max() < 2 * 2 ** -20

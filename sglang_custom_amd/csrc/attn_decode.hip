@@ -81,7 +81,7 @@ __device__ __forceinline__ void seq_range(const DecodeParams& p, int b, int64_t&
 }
 
 __device__ __forceinline__ float safe_m(float m) { return m == -INFINITY ? 0.f : m; }
-// 2^x without the steps that keep results below 2^-126
+// 2^x, results below 2^-126 lost
 __device__ __forceinline__ float raw_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ---- stage 2 of split-KV decoding: o[b, h, :] = sum_s w_s part_o[b, h, s, :] / sum_s w_s with
@@ -687,11 +687,12 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
 // every quarter-wave touch 16 rows x 16 bytes, i.e. sixteen cache-line look-ups for 256 bytes;
 // measured 58.8 -> 56.4 us at batch 64 x 1064 keys, 8 kv heads.
 // ------------------------------------------------------------------------------------------
-// Two weights 0 <= p <= 1 as 16-bit terms: p UP = hi + (mid + low) / MID, packed pairs.  In bf16 they hold all 24 bits of p; in fp16 too down
-// to 2^-25 (22 bits to 2^-28), below that to 2^-50.  hi is never zero (what it has too much is in mid).
+// Two weights 0 <= p <= 1 as 16-bit terms: p UP = hi + (mid + low) / MID, packed pairs.  In bf16 they hold all 24 bits of p down to 2^-118 and
+// below that what lies above 2^-142, in fp16 all of them down to 2^-26 and then what lies above 2^-50.  hi is never zero (what it
+// has too much is in mid).  MID takes mid below half of hi, so that no product is larger than hi's.
 template <typename T> struct WeightTerms;
 template <> struct WeightTerms<bf16_t> {
-  static constexpr float UP = 1.f, MID = 1.f, TINY = 0x1p-126f;
+  static constexpr float UP = 1.f, MID = 0x1p8f, TINY = 0x1p-126f;
   static __device__ __forceinline__ unsigned pack(float a, float b) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, rt_bf16x2));
   }
@@ -1014,13 +1015,21 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     mx = max_xor<32>(max_xor<16>(mx));
     mx = fmaxf(mx, m);
     const float ms = safe_m(mx);
-    const float alpha = raw_exp2(m - ms);
-    float pr[4], psum = 0.f;
+    // (exp2f's steps for results below 2^-126 only in a tile that has one, the first and the masked among them: wave-uniform)
+    float alpha = m - ms, pr[4], psum = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      pr[r] = raw_exp2(x[r] - ms);
-      psum += pr[r];
+    for (int r = 0; r < 4; ++r) pr[r] = x[r] - ms;
+    if (__builtin_amdgcn_ballot_w64(fminf(fminf(fminf(pr[0], pr[1]), fminf(pr[2], pr[3])), alpha) < -126.f) != 0) {
+      alpha = exp2f(alpha);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pr[r] = exp2f(pr[r]);
+    } else {
+      alpha = raw_exp2(alpha);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pr[r] = raw_exp2(pr[r]);
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) psum += pr[r];
     l = l * alpha + psum;
     m = mx;
     frag4 pb, pl;

@@ -116,3 +116,22 @@ def test_weights_of_fp32(ops, dtype, hq, hkv):
     for splits in (1, 3):
         got = _paged(ops, q.to(DEV), kb.to(DEV), vb.to(DEV), torch.tensor(lens, device=DEV), r2t, rpi, splits)
         assert ((got.cpu().double() - ref).abs() / size).max() < 2 * 2 ** -20
+
+
+@pytest.mark.parametrize("first,second", [(3, 7), (7, 3), (3, 70), (70, 3), (5, 30)], ids=lambda x: str(x))
+@pytest.mark.parametrize("D", [64, 128])
+def test_weights_below_the_normal_range(ops, D, first, second):
+    """A value of 2^120 at a weight of 2^-129.8, beside a zero at weight 1, in the same tile and in others, in front and behind: 2^-9.8, up to
+    the bits that 16-bit weights have left there at head dimension 128 (multiples of 2^-133)."""
+    r2t, rpi, _, slots = _batch([80], 3)
+    kb, vb = torch.zeros(slots, 1, D), torch.zeros(slots, 1, D)
+    s = r2t[0, :80].long().cpu()
+    kb[s, :, 0] = -2000.0
+    kb[s[first], :, 0], vb[s[first]] = -90.0, 2.0 ** 120
+    kb[s[second], :, 0] = 0.0
+    q = torch.zeros(1, 4, D)
+    q[..., 0] = 1
+    for splits in (1, 2):
+        got = _paged(ops, *(t.to(DEV, torch.bfloat16) for t in (q, kb, vb)), torch.tensor([80], device=DEV), r2t, rpi, splits)
+        want = 2.0 ** 120 * torch.exp(torch.tensor(-90.0, dtype=torch.float64)).item()
+        assert (got.double() / want - 1).abs().max() < (2 ** -7 if D == 64 else 2 ** -4), got.flatten()[:2]

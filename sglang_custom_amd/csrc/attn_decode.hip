@@ -785,6 +785,18 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   const int64_t chunk = split_chunk(p, len);
   const bool alone = p.num_splits == 1 || (p.tickets && chunk >= len);
   if (alone && split > 0) return;
+  if (len <= 0) {   // (workgroup-uniform) no tokens, no slot to read: zeros, or a split without weight for the merge
+    for (int idx = threadIdx.x; idx < G * D; idx += 256) {
+      const int64_t row = (int64_t)b * p.hq + head0 + idx / D;
+      if (alone) {
+        o[row * D + idx % D] = from_f32<T>(0.f);
+      } else {
+        p.part_o[(row * p.num_splits + split) * D + idx % D] = 0.f;
+        if (idx % D == 0) p.part_lse[row * p.num_splits + split] = -INFINITY;
+      }
+    }
+    return;
+  }
   const int64_t k0 = (int64_t)split * chunk;
   const int64_t k1 = k0 + chunk < len ? k0 + chunk : len;
   const float qmul = CAP ? p.sm_scale : p.sm_scale * kLog2e;
@@ -919,14 +931,13 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     for (int dt = 0; dt < ND; ++dt) acc_low[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // (An empty sequence has no slot to read: it takes its length, or the first prefix sum, which are 0, for one.)
-  const int32_t* pt = len > 0 ? p.page_table + page_off : p.mode == 0 ? reinterpret_cast<const int32_t*>(p.seq_lens + b) : p.kv_indptr;
+  const int32_t* pt = p.page_table + page_off;
   const int64_t row_stride = p.k_slot_stride;
   const KVT* kbase = reinterpret_cast<const KVT*>(kbuf) + (int64_t)kvh * p.k_head_stride + (KROW ? ch8 : 8 * c4);   // + slot * row_stride (+ 32 s)
   const KVT* vbase = reinterpret_cast<const KVT*>(vbuf) + (int64_t)kvh * p.v_head_stride + ch8;    // + slot * row_stride
   // Positions and a row's bytes in 32 bits (a sequence is shorter than 2^31 tokens and its slots are numbered from 0): a row's address is one
   // multiply-add.  With one or two waves on a SIMD the instructions of a tile are its time.
-  const int wave_first = (int)k0 + wave * 16, end = (int)k1, last_key = max((int)len - 1, 0);
+  const int wave_first = (int)k0 + wave * 16, end = (int)k1, last_key = (int)len - 1;
   const int n_iter = wave_first < end ? (end - wave_first + 63) / 64 : 0;
   const unsigned row_bytes = (unsigned)(row_stride * (int64_t)sizeof(KVT));
   auto row_at = [&](const KVT* base, int32_t slot) {

@@ -135,3 +135,39 @@ def test_weights_below_the_normal_range(ops, D, first, second):
         got = _paged(ops, *(t.to(DEV, torch.bfloat16) for t in (q, kb, vb)), torch.tensor([80], device=DEV), r2t, rpi, splits)
         want = 2.0 ** 120 * torch.exp(torch.tensor(-90.0, dtype=torch.float64)).item()
         assert (got.double() / want - 1).abs().max() < (2 ** -7 if D == 64 else 2 ** -4), got.flatten()[:2]
+
+
+@pytest.mark.parametrize("D,dtype,fp8", KINDS, ids=IDS)
+@pytest.mark.parametrize("lens", [[0, 33, 0, 1, 0], [0, 0], [70, 0]], ids=lambda x: "-".join(map(str, x)))
+def test_no_tokens(ops, D, dtype, fp8, lens):
+    """Sequences of no tokens first, in the middle and last: zeros.  By index list (an index pointer cut from a longer one, whose first value
+    lies past the pool), by page table and in the fused launch, where they leave the cache as it is."""
+    hq, hkv, bs = 8, 2, len(lens)
+    r2t, rpi, _, slots = _batch([max(n, 1) for n in lens], 4)
+    lens_t, live = torch.tensor(lens, device=DEV), [b for b, n in enumerate(lens) if n]
+    g = torch.Generator().manual_seed(D)
+    q = torch.randn(bs, hq, D, generator=g).to(DEV, dtype)
+    kb, vb = (torch.randn(slots, hkv, D, generator=g).to(DEV, torch.float8_e4m3fn if fp8 else dtype) for _ in range(2))
+    first = slots + 1000
+    indptr = torch.tensor([0, first] + [first + sum(lens[: i + 1]) for i in range(bs)], dtype=torch.int32, device=DEV)[1:]
+    indices = torch.zeros(first + sum(lens) + 8, dtype=torch.int32)
+    indices[first: first + sum(lens)] = torch.cat([r2t[b, :n].cpu() for b, n in enumerate(lens)])
+    part = torch.randn(2, bs, (hq + 2 * hkv) * D, generator=g).to(DEV)
+    cache = torch.cat([torch.randn(96, D // 2, generator=g).cos(), torch.randn(96, D // 2, generator=g).sin()], 1).to(DEV)
+    loc = torch.tensor([int(r2t[b, max(n - 1, 0)]) for b, n in enumerate(lens)], device=DEV)
+    for splits in (1, 3):
+        logits, lse = torch.empty(bs, hq, splits, D, device=DEV), torch.empty(bs, hq, splits, device=DEV)
+        outs = [torch.full((bs, hq, D), 7.0, device=DEV, dtype=dtype) for _ in range(5)]
+        ops.decode_attention_fwd(q, kb, vb, outs[0], indptr, indices.to(DEV), logits, lse, splits, splits, D ** -0.5)
+        tickets = torch.zeros(bs * hq, dtype=torch.int32, device=DEV)
+        for o, tk in zip(outs[1:3], (None, tickets)):
+            ops.decode_attention_paged(q, kb, vb, o, r2t, rpi, lens_t, logits, lse, splits, D ** -0.5, tickets=tk)
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+        for o, tk in zip(outs[3:], (None, tickets)):
+            kb2, vb2 = kb.clone(), vb.clone()
+            ops.decode_attention_fused_qkv(part, (lens_t - 1).clamp(min=0), loc, cache, kb2, vb2, o, r2t, rpi, lens_t, logits, lse, splits, D ** -0.5, tickets=tk)
+            for b in set(range(bs)) - set(live):
+                assert torch.equal(kb2[loc[b]].view(torch.uint8), kb[loc[b]].view(torch.uint8)) and torch.equal(vb2[loc[b]].view(torch.uint8), vb[loc[b]].view(torch.uint8))
+        assert torch.equal(outs[3], outs[4]) and (tickets == 0).all()
+        for o in outs:
+            assert all((o[b] == 0).all() if b not in live else ((o[b].abs() < 6).all() and (o[b] != 0).any()) for b in range(bs))

@@ -691,20 +691,11 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
 // below that what lies above 2^-142, in fp16 all of them down to 2^-26 and then what lies above 2^-50.  hi is never zero (what it
 // has too much is in mid).  MID takes mid below half of hi, so that no product is larger than hi's.
 template <typename T> struct WeightTerms;
-template <> struct WeightTerms<bf16_t> {
+template <> struct WeightTerms<bf16_t> : Pair16<bf16_t> {
   static constexpr float UP = 1.f, MID = 0x1p8f, TINY = 0x1p-126f;
-  static __device__ __forceinline__ unsigned pack(float a, float b) {
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, rt_bf16x2));
-  }
-  static __device__ __forceinline__ float first(unsigned u) { return __uint_as_float(u << 16); }
-  static __device__ __forceinline__ float second(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
 };
-template <> struct WeightTerms<f16_t> {
+template <> struct WeightTerms<f16_t> : Pair16<f16_t> {
   static constexpr float UP = 0x1p14f, MID = 0x1p11f, TINY = 0x1p-24f;
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  static __device__ __forceinline__ unsigned pack(float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, h2)); }
-  static __device__ __forceinline__ float first(unsigned u) { return (float)__builtin_bit_cast(h2, u)[0]; }
-  static __device__ __forceinline__ float second(unsigned u) { return (float)__builtin_bit_cast(h2, u)[1]; }
 };
 template <typename T> __device__ __forceinline__ void weight_terms(float a, float b, unsigned& hi, unsigned& mid, unsigned& low) {
 #pragma clang fp contract(off)

@@ -570,18 +570,22 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // projection of the latent, the keys' features 128 .. 191 from one row per token that the heads share, and the queries'
 // features 128 .. 191 are rotated here, in fp32 and rounded to T, as the absorbed kernels do it.
 // D: value head dimension.  At 64 the rows of the tile images are half used (the XOR spreads their eight chunks over the whole
-// 256 bytes), and P.V takes the weights as the sum of two 16-bit numbers: the vector-ALU kernel that served this size multiplied
-// fp32 weights, and two terms leave an error of at most 2^-16 of a weight in bf16 (2^-22 in fp16), far below the output's own
-// rounding (against float64 1.6563e-3 of the norm in either kernel).
+// 256 bytes), and P.V takes each weight as the sum of three 16-bit numbers, for the vector-ALU kernel that serves other forms of this size
+// multiplies by fp32 weights: in bf16 they hold all 24 bits of a weight, in fp16, where the weights are scaled to 2^15 so that the terms of
+// small ones are no subnormals, all down to 2^-16 and what lies above 2^-40 further down.
 // MASK: a custom mask instead of the causal rule (and of a prefix without conditions, unless skip_prefix_custom_mask): a row
 // [prefix + new tokens] of bytes per query.  The arithmetic is the causal launch's, so that a triangle for a mask gives its bits.
+// careful (D = 64): value rows may hold infinities and NaN, which no product with a weight of zero may meet (keys that the query does not
+// see) nor with a weight's lower terms.  The images then hold the rows without them, and beside them, in the half that is free, the rows
+// as they are, from which they are added for the queries that see their key.  Returns (the same in all threads) whether a result is no number.
 template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128, bool MASK = false>
-__device__ __forceinline__ void extend_attn_mfma32_body(
+__device__ __forceinline__ bool extend_attn_mfma32_body(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
-    const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs) {
+    const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs, bool careful = false) {
   constexpr int NS = DQ / 16;     // score k-steps
   constexpr bool WIDE = DQ > 128;
-  constexpr bool PSPLIT = D == 64;
+  constexpr bool TERMS = D == 64;
+  constexpr float P_UP = TERMS && std::is_same<T, f16_t>::value ? 0x1p15f : 1.f;   // weights up to 2^15: terms of small ones stay normal
   constexpr int CH = D / 8, SR = 256 / CH, NI = 64 / SR;   // 16-byte chunks of a row; rows staged at once, and how often
   constexpr int ND = D / 32;      // 32-feature tiles of the output
   static_assert((D == 128 && (DQ == 128 || (DQ == 192 && !KV8))) || (D == 64 && DQ == 64), "64, 128, or 192 + 128 over a 16-bit cache");
@@ -590,11 +594,13 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   __shared__ __attribute__((aligned(16))) char ks2[WIDE ? 64 * 256 : 16];
   __shared__ __attribute__((aligned(16))) char vs[64 * 256];
 
+  int tid = (int)threadIdx.x;
+  if (careful) asm volatile("" : "+v"(tid));    // (addresses of its own: the first pass's would be kept for it in scratch memory)
   const int G = p.hq / p.hkv;
   const int per_pair = G * nqb;
   const int slot = blockIdx.x >> 3;
   const int pair = (blockIdx.x & 7) + 8 * (slot / per_pair);
-  if (pair >= npairs) return;
+  if (pair >= npairs) return false;
   const int t_in_pair = slot % per_pair;
   const int qb = nqb - 1 - t_in_pair / G;          // long (late) blocks first
   const int b = pair / p.hkv, kvh = pair % p.hkv, h = kvh * G + t_in_pair % G;
@@ -603,9 +609,9 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const int kv_start = LATENT ? 0 : p.kv_indptr[b];
   const int prefix = LATENT ? 0 : p.kv_indptr[b + 1] - kv_start;
   const int r0 = qb * 128;
-  if (r0 >= ext) return;   // whole workgroup: EXEC stays full for the transposed reads below
+  if (r0 >= ext) return false;   // whole workgroup: EXEC stays full for the transposed reads below
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = tid & 63, wave = tid >> 6;
   const int j32 = lane & 31, hh = lane >> 5;
   const int qrow = r0 + wave * 32 + j32;                  // this lane's query (row of the extend part)
   const int qrow_c = qrow < ext ? qrow : ext - 1;
@@ -666,14 +672,14 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const int wave_max_limit = causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
   const uint8_t* mask_row = MASK ? p.custom_mask + p.mask_indptr[b] + (int64_t)qrow_c * (prefix + ext) : nullptr;
 
-  // tile staging: thread -> rows threadIdx.x / CH + SR i, 16-B chunk threadIdx.x % CH
-  const int srow = threadIdx.x / CH, sch = threadIdx.x % CH;
+  // tile staging: thread -> rows tid / CH + SR i, 16-B chunk tid % CH
+  const int srow = tid / CH, sch = tid % CH;
   // kreg2: chunk sch2 of features 128 and up of two of kreg's four rows, so that a paged row's slot is read once and every thread
   // has a part.  16 requests x 64 tokens on 2000 cached, 16 heads, 133 us, 2048 tokens on none 60; with rows of another deal,
   // whose slots are read again, 169 and 67; in the threads with sch < 8 alone 152 and 76.  LATENT, where these features are
   // rows of their own: eight neighbours a load (a whole step of Silatar 1 % less than in the first deal).
   Vec<T, 8> kreg[NI], vreg[NI], kreg2[WIDE ? 2 : 1];
-  const int odd2 = sch >> 3, sch2 = sch & 7, srow2 = LATENT ? threadIdx.x >> 3 : srow + 16 * odd2;   // rows srow2 + 32 j
+  const int odd2 = sch >> 3, sch2 = sch & 7, srow2 = LATENT ? tid >> 3 : srow + 16 * odd2;   // rows srow2 + 32 j
   const T* k_lin = k_ext + (int64_t)(q_start - prefix + srow) * p.k_stride + (int64_t)kvh * (LATENT ? p.kv_head : DQ) + sch * 8;
   const T* v_lin = v_ext + (int64_t)(q_start - prefix + srow) * p.v_stride + (int64_t)kvh * (LATENT ? p.kv_head : D) + sch * 8;
   const T* r_lin = LATENT ? (const T*)p.k_rope + (int64_t)(q_start + srow2) * p.k_rope_stride + sch2 * 8
@@ -750,6 +756,12 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     for (int i = 0; i < NI; ++i) {
       const int off = xor_image_off(srow + SR * i, sch);
       *reinterpret_cast<Vec<T, 8>*>(ks + off) = kreg[i];
+      if (TERMS && careful) {
+        *reinterpret_cast<Vec<T, 8>*>(vs + xor_image_off(srow + SR * i, sch + 8)) = vreg[i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (!(fabsf(to_f32(vreg[i].v[j])) < INFINITY)) vreg[i].v[j] = from_f32<T>(0.f);
+      }
       *reinterpret_cast<Vec<T, 8>*>(vs + off) = vreg[i];
     }
     if constexpr (WIDE) {
@@ -783,15 +795,49 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
   const int vch = 2 * dhalf + (tpp >> 1);                   // + 4 dt
   const char* v_rd = vs + 256 * vrow + 8 * (tpp & 1);
 
-  if (!LATENT) load_slots(0);
-  load_tile(0);
-  if (!LATENT) load_slots(1);
+  // careful: the tile's values that are no numbers, for the queries that see their keys
+  auto add_odd_values = [&](int kt) {
+    bool odd = false;      // in row `lane` of the tile
+#pragma unroll
+    for (int ch = 8; ch < 16; ++ch) {
+      const Vec<T, 8> x = *reinterpret_cast<const Vec<T, 8>*>(vs + xor_image_off(lane, ch));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) odd |= !(fabsf(to_f32(x.v[j])) < INFINITY);
+    }
+    for (uint64_t rows = __builtin_amdgcn_ballot_w64(odd); rows != 0; rows &= rows - 1) {
+      const int row = __builtin_ctzll(rows), key = kt * 64 + row;
+      const bool seen = key <= my_limit && (!MASK || mask_row[min(key, my_limit)] != 0 || (key < prefix && p.skip_prefix_custom_mask));
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {      // the lane's features, as they are stored below
+          const Vec<T, 4> x = *reinterpret_cast<const Vec<T, 4>*>(vs + xor_image_off(row, 8 + 4 * dt + rq) + 8 * hh);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float v = to_f32(x.v[r]);
+            ot[dt][4 * rq + r] += seen && !(fabsf(v) < INFINITY) ? v : 0.f;
+          }
+        }
+    }
+  };
+
+  if (!careful) {
+    if (!LATENT) load_slots(0);
+    load_tile(0);
+    if (!LATENT) load_slots(1);
+  }
   for (int kt = 0; kt < n_tiles; ++kt) {
     __syncthreads();            // previous tile fully consumed
+    if (careful) {              // (nothing ahead: no registers spilled for a rare path)
+      load_slots(kt);
+      load_tile(kt);
+    }
     store_tile();
     __syncthreads();
-    if (kt + 1 < n_tiles) load_tile(kt + 1);
-    if (!LATENT) load_slots(kt + 2);
+    if (!careful) {
+      if (kt + 1 < n_tiles) load_tile(kt + 1);
+      if (!LATENT) load_slots(kt + 2);
+    }
     if (kt * 64 > wave_max_limit) continue;   // every key of the tile is masked for every query of this wave (wave-uniform)
 
     f32x16 st[2];
@@ -872,17 +918,31 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
     const float alpha = raw_exp2(m - ms);
     m = mnew;
     float psum = 0.f;
-    frag pb[4], pl[PSPLIT ? 4 : 1];
+    frag pb[TERMS ? 3 : 4];
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float pe = raw_exp2(__builtin_fmaf(st[hf][i], qmul, -ms));
-        psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V
-        const T hi = (T)pe;
-        pb[2 * hf + (i >> 3)][i & 7] = hi;
-        if constexpr (PSPLIT) pl[2 * hf + (i >> 3)][i & 7] = (T)(pe - (float)hi);   // what the rounding left
+        psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V, or three terms of them
+        if constexpr (TERMS) st[hf][i] = pe;
+        else pb[2 * hf + (i >> 3)][i & 7] = (T)pe;
       }
+    // the terms of the lane's eight weights of k-step u
+    auto terms = [&](int u) {
+      unsigned w[3][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float a = st[u >> 1][8 * (u & 1) + 2 * i] * P_UP, c = st[u >> 1][8 * (u & 1) + 2 * i + 1] * P_UP;
+        w[0][i] = Pair16<T>::pack(a, c);
+        a -= Pair16<T>::first(w[0][i]);
+        c -= Pair16<T>::second(w[0][i]);
+        w[1][i] = Pair16<T>::pack(a, c);
+        w[2][i] = Pair16<T>::pack(a - Pair16<T>::first(w[1][i]), c - Pair16<T>::second(w[1][i]));
+      }
+#pragma unroll
+      for (int t = 0; t < 3; ++t) pb[t] = __builtin_bit_cast(frag, w[t]);
+    };
     lsum = lsum * alpha + psum;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
@@ -897,19 +957,37 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
         va[e] = vlo[i & 3][e];
         va[4 + e] = vhi[i & 3][e];
       }
-      ot[i % ND] = Mfma32<T>::run(va, pb[i / ND], ot[i % ND]);
-      if constexpr (PSPLIT) ot[i % ND] = Mfma32<T>::run(va, pl[i / ND], ot[i % ND]);
+      if constexpr (TERMS) {
+        if (i % ND == 0) terms(i / ND);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) ot[i % ND] = Mfma32<T>::run(va, pb[t], ot[i % ND]);
+      } else {
+        ot[i % ND] = Mfma32<T>::run(va, pb[i / ND], ot[i % ND]);
+      }
       __builtin_amdgcn_sched_barrier(0);
       if (i + 4 < 4 * ND) {
         v_read(i + 4, i & 3);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if (TERMS && careful) add_odd_values(kt);
   }
 
   lsum = sum_xor<32>(lsum);
+  bool odd = false;
+  if (TERMS && !careful) {
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) odd |= !(fabsf(ot[dt][i]) < INFINITY);
+    int* flags = reinterpret_cast<int*>(ks2);      // (unused otherwise)
+    odd = __builtin_amdgcn_ballot_w64(odd) != 0;
+    if (lane == 0) flags[wave] = odd;
+    __syncthreads();
+    odd = (flags[0] | flags[1] | flags[2] | flags[3]) != 0;
+  }
   if (qrow < ext) {
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    const float inv = lsum > 0.f ? 1.f / (lsum * P_UP) : 0.f;
     T* op = o_ext + ((int64_t)(q_start + qrow) * p.hq + h) * D + 4 * hh;
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
@@ -921,6 +999,7 @@ __device__ __forceinline__ void extend_attn_mfma32_body(
         stvec<T, 4>(op + 32 * dt + 8 * rq, w);
       }
   }
+  return odd;
 }
 
 // Two workgroups per CU (256 registers per lane) at head dimension 128; the 192-wide variant over a paged prefix needs
@@ -941,7 +1020,10 @@ template <typename T, bool KV8, bool MASK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void extend_attn_mfma32_d64_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
-  extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
+  if (extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs)) {
+    __syncthreads();
+    extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs, true);
+  }
 }
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void extend_attn_mfma32_wide_kernel(

@@ -330,6 +330,22 @@ template <> __device__ __forceinline__ void round2_to<bf16_t>(float a, float b, 
   rb = __uint_as_float(u & 0xffff0000u);
 }
 
+// Two floats rounded to a 16-bit type in one register, and the two as floats again (through the integer view, as above).
+template <typename T> struct Pair16;
+template <> struct Pair16<bf16_t> {
+  static __device__ __forceinline__ unsigned pack(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, rt_bf16x2));
+  }
+  static __device__ __forceinline__ float first(unsigned u) { return __uint_as_float(u << 16); }
+  static __device__ __forceinline__ float second(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
+};
+template <> struct Pair16<f16_t> {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  static __device__ __forceinline__ unsigned pack(float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector(rt_f32x2{a, b}, h2)); }
+  static __device__ __forceinline__ float first(unsigned u) { return (float)__builtin_bit_cast(h2, u)[0]; }
+  static __device__ __forceinline__ float second(unsigned u) { return (float)__builtin_bit_cast(h2, u)[1]; }
+};
+
 // v_mfma_f32_16x16x32 on 16-bit operands.  Lane l holds A[i = l & 15][k = 8 * (l >> 4) + 0..7] and
 // B[k = 8 * (l >> 4) + 0..7][j = l & 15]; the result lane holds D[i = 4 * (l >> 4) + r][j = l & 15].
 typedef float f32x4 __attribute__((ext_vector_type(4)));

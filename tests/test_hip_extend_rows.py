@@ -90,3 +90,94 @@ def test_custom_mask_at_head_dimension_64(ops, pre, ext, skip_prefix):
                              dev(torch.tensor(indptr)), max(ext), d ** -0.5, skip_prefix_custom_mask=skip_prefix)
     want = torch.cat(want)
     assert (o.cpu().float() - want).abs().max() <= 3 * 2 ** -8 * 1.1
+
+
+def _extend(ops, q, k, v, kb, vb, slots, prefix, ext, causal=True, mask=None, scale=1.0):
+    """One call; mask: bytes per request [ext, prefix + ext], in a list."""
+    dev = lambda x: None if x is None else x.to(DEV)
+    qo, kv = ([0] + list(torch.tensor(x).cumsum(0)) for x in (ext, prefix))
+    mi = None if mask is None else torch.tensor([0] + [m.numel() for m in mask]).cumsum(0)
+    o = torch.full(q.shape, float("nan"), device=DEV, dtype=q.dtype)
+    ops.extend_attention_fwd(dev(q), dev(k), dev(v), o, dev(kb), dev(vb), dev(torch.tensor(qo, dtype=torch.int32)), dev(torch.tensor(kv, dtype=torch.int32)),
+                             dev(slots.to(torch.int32)), dev(torch.cat([m.flatten() for m in mask]).to(torch.uint8)) if mask else None, causal, dev(mi),
+                             max(ext), scale, skip_prefix_custom_mask=False)
+    return o
+
+
+@pytest.mark.parametrize("form", ["causal", "all", "mask", "cache_fp8"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_values_that_are_no_numbers(ops, dtype, form):
+    """Head dimension 64: infinities and NaN in value rows reach the queries that see their keys, in their own feature, and no other
+    number changes by more than fp32 sums in another order do."""
+    g = torch.Generator().manual_seed(5)
+    D, hq, hkv, prefix, ext = 64, 4, 2, [70, 0, 3], [130, 140, 40]
+    T, P = sum(ext), sum(prefix)
+    q, k, v = (torch.randn(T, h, D, generator=g).to(dtype) for h in (hq, hkv, hkv))
+    kb, vb = (torch.randn(P + 1, hkv, D, generator=g).to(dtype) for _ in range(2))
+    if form == "cache_fp8":
+        kb, vb = kb.to(torch.float8_e4m3fn), vb.to(torch.float8_e4m3fn)
+    slots = torch.randperm(P, generator=g) + 1
+    seen, mask = [], None
+    for n, pre in zip(ext, prefix):
+        m = torch.arange(pre + n) <= pre + torch.arange(n)[:, None] if form != "all" else torch.ones(n, pre + n, dtype=torch.bool)
+        if form == "mask":
+            m = m & ((torch.rand(n, pre + n, generator=g) < 0.6) | (torch.arange(pre + n) == pre + torch.arange(n)[:, None]))
+        seen.append(m)
+    if form == "mask":
+        mask = seen
+    call = lambda v_, vb_: _extend(ops, q, k, v_, kb, vb_, slots, prefix, ext, form != "all", mask, D ** -0.5)
+    plain = call(v, vb).cpu()
+    v2, vb2, expect = v.clone(), vb.clone(), plain.double()
+    # (request, key, feature, value); feature 9 of request 0 gets both infinities
+    for b, key, f, x in ((0, 0, 3, "inf"), (0, 69, 9, "nan" if form == "cache_fp8" else "-inf"), (0, 75, 9, "inf"), (0, 199, 63, "nan"), (0, 131, 40, "-inf"),
+                         (1, 0, 0, "inf"), (1, 64, 31, "nan"), (1, 130, 32, "inf"), (2, 2, 5, "nan"), (2, 42, 7, "-inf")):
+        pre, at, had = prefix[b], sum(ext[:b]), sum(prefix[:b])
+        if form == "cache_fp8" and key < pre:
+            x = "nan"      # (e4m3fn has no infinities)
+        if key < pre:
+            if form == "cache_fp8":
+                vb2.view(torch.uint8)[slots[had + key], :, f] = 0x7F
+            else:
+                vb2[slots[had + key], :, f] = float(x)
+        else:
+            v2[at + key - pre, :, f] = float(x)
+        rows = expect[at:at + ext[b]]
+        rows[seen[b][:, key], :, f] += float(x)
+    for _ in range(2):
+        got = call(v2, vb2).cpu().double()
+        assert torch.equal(got.isnan(), expect.isnan())
+        assert torch.equal(got.isinf(), expect.isinf()) and (got[got.isinf()] == expect[got.isinf()]).all()
+        ok = expect.isfinite()
+        assert (got[ok] - expect[ok]).abs().max() <= 2.0 ** (-7 if dtype == torch.bfloat16 else -10)     # a bit of values up to 4
+    assert torch.equal(call(v, vb).cpu(), plain)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_weights_of_fp32(ops, dtype):
+    """Head dimension 64 multiplies values by fp32 weights.  The terms of every sum are alike in size (values grow as weights fall) and cancel, so
+    that the result is the sum's error: 0.5 to 0.8 times 2^-20 of the terms' root sum of squares in fp32, 5 with weights of 16 bits in
+    bf16 and 7.5 with two fp16 terms (each in torch on the CPU, the same values)."""
+    g = torch.Generator().manual_seed(3)
+    D, prefix, ext = 64, [200, 70, 0], [1, 9, 160]
+    P, T = sum(prefix), sum(ext)
+    kb, vb, k, v = (torch.zeros(n, 1, D, dtype=dtype) for n in (P, P, T, T))
+    refs, sizes = [], []
+    for b, (pre, n) in enumerate(zip(prefix, ext)):
+        at, had, N = sum(ext[:b]), sum(prefix[:b]), pre + n
+        t = -(6 * torch.rand(N, generator=g)).to(dtype).double()
+        t[N // 3] = 0
+        w = t.exp()
+        x = (torch.randn(N, D, generator=g, dtype=torch.float64) / w[:, None]).to(dtype).double()
+        for i in torch.argsort(w)[:5].flip(0):
+            x[i] = 0
+            x[i] = (-(w[:, None] * x).sum(0) / w[i]).to(dtype).double()
+        kb[had:had + pre, 0, 0], k[at:at + n, 0, 0] = t[:pre].to(dtype), t[pre:].to(dtype)
+        vb[had:had + pre, 0], v[at:at + n, 0] = x[:pre].to(dtype), x[pre:].to(dtype)
+        refs.append((w[:, None] * x).sum(0) / w.sum())
+        sizes.append((w[:, None] * x).square().sum(0).sqrt() / w.sum())
+    q = torch.zeros(T, 2, D, dtype=dtype)
+    q[..., 0] = 1
+    got = _extend(ops, q, k, v, kb, vb, torch.arange(P), prefix, ext, causal=False).cpu().double()
+    for b, (ref, size) in enumerate(zip(refs, sizes)):
+        rows = got[sum(ext[:b]):sum(ext[:b + 1])]
+        assert ((rows - ref).abs() / size).max() < 2 * 2 ** -20, b

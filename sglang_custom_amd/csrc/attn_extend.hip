@@ -884,7 +884,13 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     // the maximum and folds into the exponent's multiply-add.  Only tiles that cross the wave's diagonal
     // pay for masking (two instructions per score: the key offsets within a tile are compile-time
     // constants, the lane's limit is one subtraction per tile); the branch is wave-uniform.
-    float mloc = -INFINITY;
+    float mloc = -INFINITY, least = INFINITY;
+    if constexpr (TERMS) {
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) least = fminf(least, st[hf][i]);
+    }
     if constexpr (MASK) {
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf)
@@ -915,25 +921,42 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     mloc = max_xor<32>(mloc);
     const float mnew = fmaxf(m, mloc * qmul);
     const float ms = mnew == -INFINITY ? 0.f : mnew;
-    const float alpha = raw_exp2(m - ms);
+    const float alpha = TERMS ? exp2f(m - ms) : raw_exp2(m - ms);
     m = mnew;
     float psum = 0.f;
     frag pb[TERMS ? 3 : 4];
+    if constexpr (!TERMS) {
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf)
+      for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pe = raw_exp2(__builtin_fmaf(st[hf][i], qmul, -ms));
-        psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V, or three terms of them
-        if constexpr (TERMS) st[hf][i] = pe;
-        else pb[2 * hf + (i >> 3)][i & 7] = (T)pe;
-      }
-    // the terms of the lane's eight weights of k-step u
+        for (int i = 0; i < 16; ++i) {
+          const float pe = raw_exp2(__builtin_fmaf(st[hf][i], qmul, -ms));
+          psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V
+          pb[2 * hf + (i >> 3)][i & 7] = (T)pe;
+        }
+    }
+    // TERMS: the lane's eight weights of k-step u.  Those below 2^-126 count: exp2f, in a tile that may have one (wave-uniform); the bare
+    // instruction makes them zero.
+    const bool deep = TERMS && __builtin_amdgcn_ballot_w64(__builtin_fmaf(least, qmul, -ms) < -126.f) != 0;
     auto terms = [&](int u) {
+      float pe[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pe[i] = __builtin_fmaf(st[u >> 1][8 * (u & 1) + i], qmul, -ms);
+      if (deep) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pe[i] = exp2f(pe[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pe[i] = raw_exp2(pe[i]);
+      }
       unsigned w[3][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float a = st[u >> 1][8 * (u & 1) + 2 * i] * P_UP, c = st[u >> 1][8 * (u & 1) + 2 * i + 1] * P_UP;
+        float a = pe[2 * i], c = pe[2 * i + 1];
+        psum += a;
+        psum += c;
+        a *= P_UP;
+        c *= P_UP;
         w[0][i] = Pair16<T>::pack(a, c);
         a -= Pair16<T>::first(w[0][i]);
         c -= Pair16<T>::second(w[0][i]);
@@ -943,7 +966,7 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
 #pragma unroll
       for (int t = 0; t < 3; ++t) pb[t] = __builtin_bit_cast(frag, w[t]);
     };
-    lsum = lsum * alpha + psum;
+    if constexpr (!TERMS) lsum = lsum * alpha + psum;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt) ot[dt] *= alpha;
@@ -970,7 +993,10 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (TERMS && careful) add_odd_values(kt);
+    if constexpr (TERMS) {
+      lsum = lsum * alpha + psum;
+      if (careful) add_odd_values(kt);
+    }
   }
 
   lsum = sum_xor<32>(lsum);
@@ -1012,12 +1038,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
   extend_attn_mfma32_body<T, KV8, 128>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
 }
-// Head dimension 64 needs 168 registers: three workgroups per CU.  Bound by the softmax's instructions (about ten per score beside
-// three quarters of an MFMA cycle).  32 / 8 heads in bf16, us a launch, vector-ALU kernel -> this one: 4 x 340 tokens on 1180 cached
-// 378 -> 57, 704 + 430 tokens on none 121 -> 21, 4000 on none 1493 -> 138, 65 on 3000 510 -> 74, 70 on none 24 -> 13; fp8 cache,
-// 3 x 197 on 1614 478 -> 69.  The heads of a group packed into the rows (less of the triangle's edge in vain) was no faster.
+// Head dimension 64 needs 190 registers: two workgroups per CU (three, with a few registers in scratch memory, took longer: 4 x 340 tokens on 1180
+// cached 80 us).  Bound by the softmax's instructions (about fifteen per score, five of them the weights' three terms, beside an MFMA
+// cycle).  32 / 8 heads in bf16, us a launch, vector-ALU kernel -> this one (two terms, no weight below 2^-126): 4 x 340 tokens on 1180
+// cached 378 -> 68 (54), 704 + 430 tokens on none 121 -> 24 (20), 4000 on none 1493 -> 170 (136), 65 on 3000 510 -> 84 (73), 70 on none 24 -> 9
+// (9); fp8 cache, 3 x 197 on 1614 478 -> 61 (53).  The heads of a group packed into the rows (less of the triangle's edge in vain) was
+// no faster.
 template <typename T, bool KV8, bool MASK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void extend_attn_mfma32_d64_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_mfma32_d64_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
   if (extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs)) {

@@ -181,3 +181,23 @@ def test_weights_of_fp32(ops, dtype):
     for b, (ref, size) in enumerate(zip(refs, sizes)):
         rows = got[sum(ext[:b]):sum(ext[:b + 1])]
         assert ((rows - ref).abs() / size).max() < 2 * 2 ** -20, b
+
+
+@pytest.mark.parametrize("first,second", [(3, 7), (7, 3), (3, 70), (70, 3), (140, 5)], ids=lambda x: str(x))
+def test_weights_below_the_normal_range(ops, first, second):
+    """Head dimension 64: a value of 2^120 at a weight of 2^-129.8, beside a zero at weight 1, in the same tile and in others, in front and behind: 2^-9.8,
+    up to the bits that bf16 terms have there (multiples of 2^-133)."""
+    D, N = 64, 150
+    kb, vb = torch.zeros(N, 1, D), torch.zeros(N, 1, D)
+    kb[:, :, 0] = -2000.0
+    kb[first, :, 0], vb[first] = -90.0, 2.0 ** 120
+    kb[second, :, 0] = 0.0
+    q = torch.zeros(2, 4, D)
+    q[..., 0] = 1
+    new = torch.zeros(2, 1, D)
+    new[..., 0] = -2000.0
+    q, new, kb, vb = (t.to(torch.bfloat16) for t in (q, new, kb, vb))
+    want = 2.0 ** 120 * torch.exp(torch.tensor(-90.0, dtype=torch.float64)).item()
+    for mask in (None, [torch.ones(2, N + 2, dtype=torch.bool)]):
+        got = _extend(ops, q, new, torch.zeros_like(new), kb, vb, torch.arange(N), [N], [2], mask=mask)
+        assert (got.double() / want - 1).abs().max() < 2 ** -4

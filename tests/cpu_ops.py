@@ -162,6 +162,10 @@ def top_k_top_p_min_p_sample(probs, top_ks, top_ps, min_ps, uniform):
     return (cdf < uniform.view(-1, 1) * cdf[:, -1:]).sum(-1).clamp(max=probs.shape[1] - 1).to(torch.int32)
 
 
+def softmax_sample_(logits, temperatures, top_ks, top_ps, min_ps, uniform):
+    return top_k_top_p_min_p_sample(softmax_temperature_(logits, temperatures), top_ks, top_ps, min_ps, uniform)
+
+
 def alloc_extend_pages(prefix_lens, seq_lens, last_loc, free_pages, page_size, extend_num_tokens):
     out, used = ops_ref.alloc_extend_pages(prefix_lens, seq_lens, last_loc, free_pages, page_size)
     assert out.numel() == extend_num_tokens
@@ -518,6 +522,10 @@ def moe_route_grouped(logits, correction, top, n_groups, keep_groups, scale):
 
 def moe_router_logits(x, weight):
     return F.linear(x, weight)
+
+
+def tiled_tail_splits(m, n, k, fp8=False, silu_mul=False):
+    return 0
 
 
 def linear_tiled_supported(m, n, k, dtype, silu_mul=False):

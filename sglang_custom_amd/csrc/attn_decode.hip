@@ -687,27 +687,55 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
 // every quarter-wave touch 16 rows x 16 bytes, i.e. sixteen cache-line look-ups for 256 bytes;
 // measured 58.8 -> 56.4 us at batch 64 x 1064 keys, 8 kv heads.
 // ------------------------------------------------------------------------------------------
-// Two weights 0 <= p <= 1 as 16-bit terms: p UP = hi + (mid + low) / MID, packed pairs.  In bf16 they hold all 24 bits of p down to 2^-118 and
-// below that what lies above 2^-142, in fp16 all of them down to 2^-26 and then what lies above 2^-50.  hi is never zero (what it
-// has too much is in mid).  MID takes mid below half of hi, so that no product is larger than hi's.
+// Weights 0 <= p <= 1 as 16-bit terms of whole products: p UP = hi + (mid + low) / MID.  MID takes mid below hi's size, so that no product is larger
+// than hi's.  The lanes of a column need one term each; a wave's time for a tile is the chain from its scores to its products.
+// bf16: the upper halves of p, of what that leaves and of what that leaves: all 24 bits down to 2^-117, and what lies above 2^-140 further down.
+// fp16: all bits down to 2^-26 and then what lies above 2^-50; hi is never zero (what it has too much is in mid), so that an infinite
+// value row makes infinity whatever its weight.
 template <typename T> struct WeightTerms;
-template <> struct WeightTerms<bf16_t> : Pair16<bf16_t> {
-  static constexpr float UP = 1.f, MID = 0x1p8f, TINY = 0x1p-126f;
-};
-template <> struct WeightTerms<f16_t> : Pair16<f16_t> {
-  static constexpr float UP = 0x1p14f, MID = 0x1p11f, TINY = 0x1p-24f;
-};
-template <typename T> __device__ __forceinline__ void weight_terms(float a, float b, unsigned& hi, unsigned& mid, unsigned& low) {
+template <> struct WeightTerms<bf16_t> {
+  static constexpr float UP = 1.f, MID = 0x1p6f;
+  static __device__ __forceinline__ unsigned upper(float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u); }
+  static __device__ __forceinline__ float without(float x, unsigned mask) { return x - __uint_as_float(__float_as_uint(x) & mask); }
+  // the lane's term of two weights
+  static __device__ __forceinline__ unsigned one(float a, float b, int term) {
 #pragma clang fp contract(off)
-  using W = WeightTerms<T>;
-  a *= W::UP;
-  b *= W::UP;
-  hi = W::pack(fmaxf(a, W::TINY), fmaxf(b, W::TINY));
-  a = (a - W::first(hi)) * W::MID;
-  b = (b - W::second(hi)) * W::MID;
-  mid = W::pack(a, b);
-  low = W::pack(a - W::first(mid), b - W::second(mid));
-}
+    const float s = term == 0 ? 1.f : MID;
+    const unsigned m1 = term == 0 ? 0u : 0xffff0000u, m2 = term == 2 ? 0xffff0000u : 0u;
+    return upper(without(without(a * s, m1), m2), without(without(b * s, m1), m2));
+  }
+  // hi (term 0) or mid, and low
+  static __device__ __forceinline__ void two(float a, float b, int term, unsigned& first, unsigned& low) {
+#pragma clang fp contract(off)
+    const float ra = without(a * MID, 0xffff0000u), rb = without(b * MID, 0xffff0000u);
+    first = term == 0 ? upper(a, b) : upper(ra, rb);
+    low = upper(without(ra, 0xffff0000u), without(rb, 0xffff0000u));
+  }
+};
+template <> struct WeightTerms<f16_t> {
+  static constexpr float UP = 0x1p14f, MID = 0x1p11f, TINY = 0x1p-24f;
+  static __device__ __forceinline__ void all(float a, float b, unsigned& hi, unsigned& mid, unsigned& low) {
+#pragma clang fp contract(off)
+    using P = Pair16<f16_t>;
+    a *= UP;
+    b *= UP;
+    hi = P::pack(fmaxf(a, TINY), fmaxf(b, TINY));
+    a = (a - P::first(hi)) * MID;
+    b = (b - P::second(hi)) * MID;
+    mid = P::pack(a, b);
+    low = P::pack(a - P::first(mid), b - P::second(mid));
+  }
+  static __device__ __forceinline__ unsigned one(float a, float b, int term) {
+    unsigned hi, mid, low;
+    all(a, b, hi, mid, low);
+    return term == 0 ? hi : term == 2 ? low : mid;
+  }
+  static __device__ __forceinline__ void two(float a, float b, int term, unsigned& first, unsigned& low) {
+    unsigned hi, mid;
+    all(a, b, hi, mid, low);
+    first = term == 0 ? hi : mid;
+  }
+};
 
 template <int D> constexpr int dv_row() { return D + 16; }   // V tile row in LDS (elements): 288 or 160 B -> conflict-free transposed reads
 
@@ -985,13 +1013,33 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
       for (int u = 0; u < NR; ++u) vv[u] = ldvec<T, VE>(row_at(vbase, sv[u]));
     }
   };
-  // One 16-key tile.  A tile past the end of the range is harmless: every key is masked, so the
-  // probabilities are zero, the value rows too, and the rescale factor is one.
-  auto compute_tile = [&](frag (&kf)[NS], Vec<T, VE> (&vv)[NR], int it) {
+  // the B operand of P.V for four weights (TERMS, GC = 8: and that of the third terms)
+  auto operand = [&](const float (&w)[4], frag4& pb, frag4& pl) {
+    if constexpr (TERMS) {
+      uint2 first, low;
+      if constexpr (GC == 8) {
+        WeightTerms<T>::two(w[0], w[1], term, first.x, low.x);
+        WeightTerms<T>::two(w[2], w[3], term, first.y, low.y);
+        pl = __builtin_bit_cast(frag4, low);
+      } else {
+        first.x = WeightTerms<T>::one(w[0], w[1], term);     // (mid on both sides of hi, all round)
+        first.y = WeightTerms<T>::one(w[2], w[3], term);
+      }
+      pb = __builtin_bit_cast(frag4, first);
+    } else {
+      T t4[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t4[r] = from_f32<T>(w[r]);
+      pb = __builtin_bit_cast(frag4, t4);
+    }
+  };
+  // One 16-key tile.  last: the wave's last one, which the end of the range may cross and which holds the newest key.
+  auto compute_tile = [&](frag (&kf)[NS], Vec<T, VE> (&vv)[NR], int it, auto last) {
     // No multiply-add contraction in the softmax: the fused and the plain instantiation of this
     // kernel must round identically (the compiler otherwise contracts differently per instantiation).
 #pragma clang fp contract(off)
-    if constexpr (FUSED) {
+    constexpr bool LAST = decltype(last)::value;
+    if constexpr (FUSED && LAST) {
       if (owner && it == it_new) {   // this tile's row rl was loaded before the cache held it
 #pragma unroll
         for (int s = 0; s < NS; ++s)
@@ -1006,72 +1054,49 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
     for (int s = 0; s < NS; ++s) sc = Mfma<T>::run(kf[s], qf[s], sc);
 
     const int kb0 = wave_first + it * 64 + 4 * c4;
-    float x[4], mx = -INFINITY;
+    float x[4], mx = -INFINITY, least = INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float v = sc[r] * qmul;
       if (CAP) v = p.logit_cap * tanhf(v / p.logit_cap) * kLog2e;
-      x[r] = kb0 + r < end ? v : -INFINITY;
+      x[r] = !LAST || kb0 + r < end ? v : -INFINITY;
       mx = fmaxf(mx, x[r]);
+      least = fminf(least, v);
     }
     mx = max_xor<32>(max_xor<16>(mx));
     mx = fmaxf(mx, m);
-    const float ms = safe_m(mx);
-    // (exp2f's steps for results below 2^-126 only in a tile that has one, the first and the masked among them: wave-uniform)
-    float alpha = m - ms, pr[4], psum = 0.f;
+    const float ms = safe_m(mx), down = m - ms;
+    const float alpha = raw_exp2(down);
+    float pr[4], psum = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pr[r] = x[r] - ms;
-    if (__builtin_amdgcn_ballot_w64(fminf(fminf(fminf(pr[0], pr[1]), fminf(pr[2], pr[3])), alpha) < -126.f) != 0) {
-      alpha = exp2f(alpha);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pr[r] = exp2f(pr[r]);
-    } else {
-      alpha = raw_exp2(alpha);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pr[r] = raw_exp2(pr[r]);
+    for (int r = 0; r < 4; ++r) {
+      x[r] -= ms;
+      pr[r] = raw_exp2(x[r]);
+      psum += pr[r];
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) psum += pr[r];
-    l = l * alpha + psum;
+    l = l * alpha + psum;      // (what lies below 2^-126 of the largest weight is no bit of the sum)
     m = mx;
     frag4 pb, pl;
-    if constexpr (TERMS) {
-      uint2 hi, mid, low;
-      weight_terms<T>(pr[0], pr[1], hi.x, mid.x, low.x);
-      weight_terms<T>(pr[2], pr[3], hi.y, mid.y, low.y);
-      if constexpr (GC == 8) {
-        pb = __builtin_bit_cast(frag4, term == 0 ? hi : mid);
-        pl = __builtin_bit_cast(frag4, low);
-      } else {
-        pb = __builtin_bit_cast(frag4, term == 0 ? hi : term == 2 ? low : mid);   // (mid on both sides of hi, all round)
-      }
-    } else {
-      T pt4[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pt4[r] = from_f32<T>(pr[r]);
-      pb = __builtin_bit_cast(frag4, pt4);
-    }
+    operand(pr, pb, pl);
 
-    // Rows past the end of the range are other rows' contents (clamped addresses; FUSED: the newest token's slot as its last owner left
-    // it): their weights are zero, but zero times an infinity or a NaN is none.
-    const int live_rows = end - wave_first - it * 64;    // (wave-uniform)
-    if (live_rows < 16) {
-#pragma unroll
-      for (int u = 0; u < NR; ++u)
-        if (row0 + u >= live_rows)
-#pragma unroll
-          for (int j = 0; j < VE; ++j) vv[u].v[j] = from_f32<T>(0.f);
-    }
 #pragma unroll
     for (int u = 0; u < NR; ++u) stvec<T, VE>(v_wr + u * DV_ROW, vv[u]);
+    // Rows past the end of the range are other rows' contents (clamped addresses; FUSED: the newest token's slot as its last owner left
+    // it): their weights are zero, but zero times an infinity or a NaN is none.
+    if constexpr (LAST) {
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+        if (wave_first + it * 64 + row0 + u >= end) stvec<T, VE>(v_wr + u * DV_ROW, Vec<T, VE>{});
+    }
     __builtin_amdgcn_wave_barrier();
     // the running maximum rarely moves after the first tiles: skip the rescale (a multiplication by
     // exactly 1, so skipping it changes no bit) unless some lane of the wave needs it
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+      const float f = exp2f(down);
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt) {
-        acc[dt] *= alpha;
-        if constexpr (TERMS && GC == 8) acc_low[dt] *= alpha;
+        acc[dt] *= f;
+        if constexpr (TERMS && GC == 8) acc_low[dt] *= f;
       }
     }
     // all transposed reads first, then the MFMAs: written read-MFMA-read-MFMA the reads stay in
@@ -1086,11 +1111,26 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt) acc_low[dt] = Mfma16<T>::run(__builtin_bit_cast(frag4, vt[dt]), pl, acc_low[dt]);
     }
+    // bf16 weights below 2^-126, which the bare exponential makes zero, scaled by 2^64: behind the others, where a condition (wave-uniform)
+    // holds up nothing.  (fp16 has no number for their products.)
+    if constexpr (std::is_same<T, bf16_t>::value) {
+      if (__builtin_amdgcn_ballot_w64(least - ms < -126.f) != 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pr[r] = x[r] < -126.f ? raw_exp2(x[r] + 64.f) : 0.f;
+        operand(pr, pb, pl);
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) {
+          const frag4 v = __builtin_bit_cast(frag4, vt[dt]);
+          acc[dt] += Mfma16<T>::run(v, pb, f32x4{0.f, 0.f, 0.f, 0.f}) * 0x1p-64f;
+          if constexpr (TERMS && GC == 8) acc_low[dt] += Mfma16<T>::run(v, pl, f32x4{0.f, 0.f, 0.f, 0.f}) * 0x1p-64f;
+        }
+      }
+    }
     __builtin_amdgcn_wave_barrier();
   };
 
   // widen an fp8 tile on use; a 16-bit tile is computed in place
-  auto compute = [&](KRaw (&kraw)[NR], VRaw (&vraw)[NR], int it) {
+  auto compute = [&](KRaw (&kraw)[NR], VRaw (&vraw)[NR], int it, auto last) {
     if constexpr (KV8 && KROW) {
       Vec<T, VE> vv[NR];
 #pragma unroll
@@ -1102,7 +1142,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 #pragma unroll
       for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const frag*>(k_rd + 32 * s);
       __builtin_amdgcn_wave_barrier();
-      compute_tile(kf, vv, it);
+      compute_tile(kf, vv, it, last);
     } else if constexpr (KV8) {
       frag kf[NS];
       Vec<T, VE> vv[NR];
@@ -1110,7 +1150,7 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
       for (int s = 0; s < NS; ++s) kf[s] = __builtin_bit_cast(frag, cvt8_from_fp8<T>(kraw[s]));
 #pragma unroll
       for (int u = 0; u < NR; ++u) vv[u] = cvt8_from_fp8<T>(vraw[u]);
-      compute_tile(kf, vv, it);
+      compute_tile(kf, vv, it, last);
     } else if constexpr (KROW) {
 #pragma unroll
       for (int u = 0; u < NR; ++u) stvec<T, VE>(k_wr + u * DV_ROW, kraw[u]);
@@ -1119,9 +1159,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
 #pragma unroll
       for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const frag*>(k_rd + 32 * s);
       __builtin_amdgcn_wave_barrier();
-      compute_tile(kf, vraw, it);
+      compute_tile(kf, vraw, it, last);
     } else {
-      compute_tile(kraw, vraw, it);
+      compute_tile(kraw, vraw, it, last);
     }
   };
 
@@ -1180,21 +1220,24 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
       }
     }
   }
-  if (n_iter > 0) {
-    for (int it = 0; it < n_iter; it += 2) {
-      // (Fenced: the rows' addresses would be formed at the head of a tile, behind a wait for slots that were requested last.)
-      compute(kfA, vvA, it);
-      __builtin_amdgcn_sched_barrier(0);
-      load_kv(skA, svA, kfA, vvA);      // tile it + 2
-      load_slots(it + 4, skA, svA);
-      __builtin_amdgcn_sched_barrier(0);
-      compute(kfB, vvB, it + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      load_kv(skB, svB, kfB, vvB);      // tile it + 3
-      load_slots(it + 5, skB, svB);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  constexpr std::false_type whole{};
+  constexpr std::true_type last{};
+  int it = 0;
+  for (; it + 2 < n_iter; it += 2) {
+    // (Fenced: the rows' addresses would be formed at the head of a tile, behind a wait for slots that were requested last.)
+    compute(kfA, vvA, it, whole);
+    __builtin_amdgcn_sched_barrier(0);
+    load_kv(skA, svA, kfA, vvA);      // tile it + 2
+    load_slots(it + 4, skA, svA);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(kfB, vvB, it + 1, whole);
+    __builtin_amdgcn_sched_barrier(0);
+    load_kv(skB, svB, kfB, vvB);      // tile it + 3
+    load_slots(it + 5, skB, svB);
+    __builtin_amdgcn_sched_barrier(0);
   }
+  if (it < n_iter) compute(kfA, vvA, it, last);
+  if (it + 1 < n_iter) compute(kfB, vvB, it + 1, last);
 
   l = sum_xor<32>(sum_xor<16>(l));
   if constexpr (TERMS) {

@@ -208,9 +208,10 @@ int mi355_prepare_decode(int32_t* req_to_token, const int64_t* req_pool_indices,
  * (unused when num_splits == 1; num_splits <= MI355_MAX_KV_SPLITS).  logit_cap > 0 applies cap*tanh(s/cap).
  * split_tickets (may be NULL): B * Hq uint32 arrival counters, ZERO when the call is made and zero
  * again when its kernels have finished (hipMemset them once, then hand the same array to every call on
- * one stream).  With them the head_dim-128 16-bit kernel merges the KV splits itself -- the last split
+ * one stream).  With them the matrix-core kernel (16-bit q; head_dim 128, or 64 over a 16-bit cache; 16-byte aligned) merges the KV
+ * splits itself -- the last split
  * workgroup of a (sequence, head group) to finish does it -- and no second launch follows; without them,
- * above 64 splits, and for every other shape, a merge kernel is launched behind the first.  Same bits
+ * above 64 splits, and for every other shape, which does not touch the counters, a merge kernel is launched behind the first.  Same bits
  * either way.  Calls that may overlap on the GPU need arrays of their own.
  * kv_chunk_keys (may be NULL): ONE int32 in device memory, read by the kernels when they run: the batch's
  * keys per split.  Sequence b is then cut into ceil(len(b) / *kv_chunk_keys) splits (at most num_splits; a
@@ -240,7 +241,8 @@ int mi355_decode_num_splits_fp8(int64_t bs, int hkv, int64_t max_seq_len, int ma
 /* Either plan (kv_fp8) for a launch whose lengths are not known yet, a captured one, with max_seq_len the most they may be: returns
  * the splits to launch.  For a batch whose longest sequence is `len`, kv_chunk_keys should then come from max(fewest, min(splits,
  * len / split_keys)) of them (all, if split_keys is 0): splits further than `fewest` pay only with split_keys keys each.  The
- * matrix-core kernel (head_dim 128, 16-bit q) passes over those that the chunk leaves empty; elsewhere they cost as much as full ones. */
+ * matrix-core kernel (16-bit q; head_dim 128, or 64 over a 16-bit cache) passes over those that the chunk leaves empty where it
+ * has split_tickets; elsewhere they cost as much as full ones.  The figures behind the plan are head_dim 128's. */
 int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_splits, int kv_fp8, int* fewest, int64_t* split_keys);
 
 /* ---- K4 extend / prefill attention -----------------------------------------------------------

@@ -61,13 +61,6 @@ __device__ __forceinline__ float ca_cap_fast(float s, float c, float k2) {
 constexpr int CV_ROWS = 16;
 constexpr int CV_KT = 32;
 
-__device__ __forceinline__ float ca_row16_max(float x) {
-  return row16_max(x);
-}
-__device__ __forceinline__ float ca_row16_sum(float x) {
-  return row16_sum(x);
-}
-
 template <typename T, int MAPS, int C>   // C: result columns per lane, dv <= 16 C
 __global__ __launch_bounds__(256) void causal_attention_valu_kernel(CaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -140,7 +133,7 @@ __global__ __launch_bounds__(256) void causal_attention_valu_kernel(CaArgs a) {
         sc[u] = j0 + kk <= rp ? s : CA_NEG;
         tmax = fmaxf(tmax, sc[u]);
       }
-      const float new_m = fmaxf(run_m[m], ca_row16_max(tmax));
+      const float new_m = fmaxf(run_m[m], row16_max(tmax));
       alpha[m] = expf(run_m[m] - new_m);              // 1 when nothing changed, also for rows that have seen nothing yet
       float psum = 0.f;
 #pragma unroll
@@ -149,7 +142,7 @@ __global__ __launch_bounds__(256) void causal_attention_valu_kernel(CaArgs a) {
         Ps[(m * CV_ROWS + r) * CV_KT + cx + 16 * u] = p;
         psum += p;
       }
-      run_l[m] = run_l[m] * alpha[m] + ca_row16_sum(psum);
+      run_l[m] = run_l[m] * alpha[m] + row16_sum(psum);
       run_m[m] = new_m;
     }
     __syncthreads();
@@ -196,7 +189,7 @@ __global__ __launch_bounds__(256) void causal_attention_valu_kernel(CaArgs a) {
     q2 += o[c] * o[c];
   }
   float mul = 1.f;
-  if constexpr (MAPS == 2) mul = a.out_scale / sqrtf(ca_row16_sum(q2) / (float)dv + a.eps);
+  if constexpr (MAPS == 2) mul = a.out_scale / sqrtf(row16_sum(q2) / (float)dv + a.eps);
   if (!live) return;
   const T* gt = (const T*)a.gate + t * a.gate_token_stride;
   if (a.gate != nullptr && !a.gate_per_feature) mul *= ca_sigmoid(to_f32(gt[h]));

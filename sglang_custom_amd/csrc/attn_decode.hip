@@ -58,14 +58,14 @@ __device__ __forceinline__ int64_t split_chunk(const DecodeParams& p, int64_t le
 // Inputs of the fused decode step: the qkv projection is still fp32 split-K partials, RoPE has
 // not been applied and the new token's K/V rows are not in the cache yet.
 struct FusedQkv {
-  const float* part;          // [nsplit][B][row] partials of the qkv GEMM, row = (hq + 2 hkv) * 128
+  const float* part;          // [nsplit][B][row] partials of the qkv GEMM, row = (hq + 2 hkv) * head_dim
   int nsplit;
   int64_t split_stride, row;  // elements
   const float* xs;            // fp8 qkv GEMM: per-token activation scales [B] and per-channel weight
   const float* ws;            //   scales [row]; both null for a 16-bit GEMM
   const int64_t* positions;   // [B]
   const int64_t* out_loc;     // [B] cache slot of the new token (padded rows of a captured batch name the sink slot)
-  const void* cos_sin;        // [max_pos][128]: cos (64) | sin (64), fp32 or the tensor dtype
+  const void* cos_sin;        // [max_pos][head_dim]: cos (head_dim / 2) | sin, fp32 or the tensor dtype
   int cache_f32;
 };
 
@@ -755,11 +755,11 @@ template <int D> constexpr int dv_row() { return D + 16; }   // V tile row in LD
 // D = 64: eight lanes a row, and P.V multiplies fp32 weights, as the vector-ALU kernel does that serves other sizes: a weight is the sum of
 // three 16-bit terms (WeightTerms).  The matrix has columns to spare: every head's query is in two or four of them, so that all of
 // these have its scores, and each of a head's columns takes one term (G = 8, two columns a head: the third term in products of its own).  A
-// term's sums are its column's, so that fp16 terms can be scaled apart, and an infinite value row, which the first term (never
-// zero) makes infinite, is not lost to the second's sign.
+// term's sums are its column's, so that terms can be scaled apart, and an infinite value row, which the first term makes infinite, is not
+// lost to the second's sign.
 // 16 layers of 32 / 8 heads, a whole step with the rotation, the sum of the projection's splits and the merge in this launch, against the
-// vector-ALU kernel behind and in front of launches for those: 1 x 131 tokens 844 -> 768 us, 1 x 2000 936 -> 817, 32 x 360 1043 -> 925,
-// 33 x 1494 1442 -> 1193 (with two terms in one column's sum 757, 812, 912, 1185).
+// vector-ALU kernel behind and in front of launches for those: 1 x 131 tokens 844 -> 750 us, 1 x 2000 936 -> 851, 32 x 360 1043 -> 938,
+// 33 x 1494 1442 -> 1219 (with two terms in one column's sum 744, 845, 926, 1202).
 template <typename T, int D, int G, bool CAP, bool FUSED = false, bool KV8 = false, bool KROW = false>
 __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __restrict__ q,
                                                                   const T* kbuf, const T* vbuf,
@@ -820,9 +820,9 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_pv_kernel(const T* __res
   const int64_t k1 = k0 + chunk < len ? k0 + chunk : len;
   const float qmul = CAP ? p.sm_scale : p.sm_scale * kLog2e;
 
-  // FUSED: the workgroup first reduces its (G + 2) x 128 slice of the qkv row (q heads, k, v) from
+  // FUSED: the workgroup first reduces its (G + 2) x D slice of the qkv row (q heads, k, v) from
   // the split-K partials into LDS -- one float4 per thread and split -- and applies neox RoPE to the q and
-  // k slices on the way (features i and i + 64 of a head exchange through a lane shuffle); the MFMA fragments
+  // k slices on the way (features i and i + D / 2 of a head exchange through a lane shuffle); the MFMA fragments
   // are then read from LDS as they are.
   __shared__ __attribute__((aligned(16))) T sm_qkv[FUSED ? (G + 2) * D : 8];
   auto reduce_qkv_to_lds = [&]() {
@@ -2946,9 +2946,10 @@ int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
   if (bs > 0 && hkv > 0 && max_splits > 1) {
     // Split only until the launch can saturate HBM, and no further: a workgroup of the MFMA kernel
     // streams ~45 GB/s, so ~112 of them already draw what the chip delivers to this access pattern,
-    // and every extra split costs fp32 partial traffic plus ~1 us of the merge launch.  Measured at
-    // 1064 keys, head_dim 128 (microseconds, best in brackets): 8 workgroups unsplit 17.6 [6-8 splits:
-    // 11.6]; 64: 19.9 [3: 14.4; 8: 19.1]; 128: 20.5 [2: 19.7; 4: 22.3]; 256: 31.7 [1; 2: 34.4].
+    // and every extra split costs fp32 partial traffic plus ~1 us of the merge.  Measured at
+    // 1064 keys, head_dim 128, merged in the launch (microseconds, best in brackets): 8 workgroups unsplit 12.8 [8 splits:
+    // 8.8]; 64: 13.6 [4: 10.4; 8: 11.3]; 128: 15.2 [2: 14.3; 4: 15.6]; 256: [22.1; 2: 26.2].  Head_dim 64: 10.0 [8: 7.8];
+    // 10.1 [4: 8.9; 8: 9.5]; 10.5 [2: 10.1; 4: 10.3]; [12.0; 2: 14.5].
     // Long contexts (>= 1024 keys per split left) with fewer than 192 workgroups are split until every CU has one.
     // 64 sequences x one kv head x 4136 keys with the merge inside the launch: 34.9 / 27.7 / 29.5 / 36.1 / 33.4 /
     // 46.1 us at 2 / 3 / 4 / 6 / 8 / 16 splits -- 192 workgroups of 1 379 keys beat 256 of 1 034 (every split pays its
@@ -2967,8 +2968,9 @@ int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
     want = base;
     // 112 to 128 workgroups draw the chip's rate only while every one of them runs: with 1 024 keys left per split half
     // the CUs' worth more of them pays, and more again when the lengths differ and the longest row would run alone.
-    // 128 workgroups, head_dim 128, 1 -> 2 splits: 512 keys 11.1 -> 12.1 us, 1 024 17.7 -> 16.9, 2 048 28.3 -> 26.7,
-    // 4 096 57.4 -> 47.5, 1 638 to 4 096 52.8 -> 38.4; 144 workgroups (more than the CUs once doubled), 2 048: 29.2 -> 37.0.
+    // 128 workgroups, head_dim 128, 1 -> 2 splits: 512 keys 9.3 -> 9.6 us, 1 024 14.5 -> 13.5, 2 048 25.7 -> 23.1,
+    // 4 096 47.7 -> 42.4, 1 638 to 4 096 45.8 -> 36.4; 144 workgroups (more than the CUs once doubled), 2 048: 27.3 -> 33.3.
+    // Head_dim 64: 512 keys 6.7 -> 7.8, 1 064 10.5 -> 10.1, 2 048 17.4 -> 14.2, 4 096 31.7 -> 23.1.
     if (wgs >= 112 && wgs <= 128) keep = 1024;
     int64_t most = 2;
     // One-byte rows halve what a workgroup draws (~27 GB/s: its time per key is the chain from row to product, not the
@@ -2976,12 +2978,14 @@ int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
     // (a fifth is a second merge chain).  A split has to keep 512 keys, and 4 per workgroup of the unsplit launch, to pay
     // for its partial: where the launch is already wide there is less left to fill.  head_dim 128, 8 kv heads, us at
     // 1 / 2 / 3 / 4 splits (bracket: taken):
-    //   64 wgs, 4 096 keys  40.0 / 25.0 / 19.7 / [16.9];   128 wgs, 512 keys [9.1] / 8.9 / 10.9 / 9.7;
-    //  128 wgs, 1 024       13.4 / [11.3] / 13.5 / 11.9;   128 wgs, 2 048     22.3 / 16.3 / 19.6 / [16.8];
-    //  128 wgs, 4 096       39.7 / 26.4 / 31.0 / [26.6];   144 wgs, 1 024    [13.5] / 14.8 / 13.8 / 14.8;
-    //  160 wgs, 2 048       22.4 / 23.2 / [20.6] / 22.2;   160 wgs, 4 096     40.3 / 40.0 / [33.4] / 37.4;
-    //  224 wgs, 4 096       41.4 / [43.5] / 48.9 / 48.4;   256 wgs, 1 024    [14.1] / 16.5 / 19.3 / 20.7;
-    //  256 wgs, 4 096       44.4 / [46.5] / 50.1 / 51.1;   384 wgs, 4 096    [72.4] / 67.0 / 76.4 / 74.2.
+    //   64 wgs, 4 096 keys  41.6 / 25.8 / 20.3 / [17.6];   128 wgs, 512 keys [9.6] / 9.5 / 10.3 / 9.8;
+    //  128 wgs, 1 024       14.3 / [12.1] / 13.6 / 12.1;   128 wgs, 2 048     23.2 / 17.1 / 18.5 / [16.8];
+    //  128 wgs, 4 096       41.1 / 27.0 / 30.5 / [26.6];   144 wgs, 1 024    [14.3] / 15.1 / 13.9 / 14.3;
+    //  160 wgs, 2 048       23.3 / 23.3 / [19.5] / 21.1;   160 wgs, 4 096     41.3 / 40.2 / [32.9] / 36.3;
+    //  224 wgs, 4 096       43.2 / [43.6] / 47.1 / 45.8;   256 wgs, 1 024    [14.7] / 16.4 / 17.6 / 18.9;
+    //  256 wgs, 4 096       44.8 / [46.3] / 47.8 / 48.1;   384 wgs, 4 096    [72.5] / 65.5 / 73.1 / 68.8.
+    // The line was drawn for a kernel whose chain per tile was a quarter longer; where two splits fill the chip in one round it is now up
+    // to 3 % on the wrong side (224 and 256 workgroups), and at 384, one and a half rounds, 10 %.
     if (kv_fp8) {
       most = 512 / wgs < 4 ? 512 / wgs : 4;
       keep = most > 1 ? (4 * wgs > 512 ? 4 * wgs : 512) : 0;

@@ -32,7 +32,7 @@
 //   * workgroup -> tile: consecutive workgroups round-robin over the 8 XCDs, so workgroups b and
 //     b + 8 share an L2; each XCD works through 8 x 4 blocks of tiles (32 CUs = one block);
 //   * tiles beyond whole rounds of 256 may be split over K, their sums added by a second launch that also runs the epilogue.
-// What bounds it: the card's power.  A K tile takes 2320 of the 2048 cycles that its MFMAs need (88 %), but with random operands the
+// What bounds it: the card's power.  The MFMAs of a K tile take 2048 of its 2320 cycles (88 %), but with random operands the
 // clock falls to 1.7 GHz (4096 x 4096 x 4096: 98 us; with x = 0 2.17 GHz and 77).  So the order of a matrix slot's MFMAs counts: W fragments
 // go forth in one row of x fragments and back in the next, one operand of every MFMA the last one's (a loop of MFMAs alone 2045 ->
 // 2085 TFLOP/s, with the LDS reads 1797 -> 1829; 32 x 32 x 16 MFMAs 1795 and 1595).  A Llama-3-8B

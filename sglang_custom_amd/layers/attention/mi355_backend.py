@@ -68,7 +68,8 @@ class Mi355AttnBackend(AttentionBackend):
         # per-layer key / value shapes (LayeredMHATokenToKVPool): served by forward_sigmoid alone, with the same metadata
         self.is_layered = hasattr(model_runner.token_to_kv_pool, "layer_shapes")
         self.kv_fp8 = getattr(model_runner.token_to_kv_pool, "dtype", None) == torch.float8_e4m3fn
-        # the decode kernel of these shapes merges its splits in its own launch and passes over empty ones
+        # captured steps of these shapes are planned with splits for any length: their decode kernel merges in its own launch and passes
+        # over empty splits
         self.merges_in_launch = (not (self.is_mla or self.is_latent_window or self.is_layered)
                                  and getattr(cfg, "head_dim", None) == 128 and getattr(model_runner, "dtype", None) in (torch.bfloat16, torch.float16))
         if self.is_mla:
@@ -148,9 +149,11 @@ class Mi355AttnBackend(AttentionBackend):
             return splits, splits, 0
         splits, fewest, keys = get_ops().decode_split_plan(bs, self.num_kv_head, max_seq_len, MAX_KV_SPLITS, self.kv_fp8)
         if not self.merges_in_launch:
-            # a split that a short batch leaves empty costs as much as a full one here.  The kernel that reads e4m3fn rows at other
-            # head sizes is so slow a chain per split that they pay at any length (128 workgroups, head_dim 64, 300 keys:
-            # 287 / 163 / 117 / 92 us at 1 / 2 / 3 / 4); 16-bit ones do not below some 700 keys (300: 9.7 / 11.7 at 1 / 2).
+            # Head sizes other than 128.  The kernel that reads e4m3fn rows there is so slow a chain per split that splits pay at any
+            # length, empty ones included (128 workgroups, head_dim 64, 300 keys: 287 / 163 / 117 / 92 us at 1 / 2 / 3 / 4).  Over 16-bit
+            # rows the fewest are captured: where a split that a short batch leaves empty costs as much as a full one, that is the plan
+            # for any length.  (At head_dim 64, whose kernel passes over empty splits, two of them captured for 128 workgroups
+            # would cost nothing at 300 keys and take 10.1 us for 10.5 at 1 064, 14.4 for 17.5 at 2 048.)
             splits, fewest, keys = (splits, splits, 0) if self.kv_fp8 else (fewest, fewest, 0)
         return splits, fewest, keys
 

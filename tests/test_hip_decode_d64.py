@@ -52,7 +52,7 @@ def test_fused_launch_and_float64(ops, dtype, cache_dtype, hq, hkv, bs, maxlen, 
             ops.decode_attention_fused_qkv(part, lens - 1, loc, cache, kb2, vb2, o, r2t, rpi, lens, logits, lse, splits, D ** -0.5, tickets=tickets)
             assert torch.equal(kb, kb2) and torch.equal(vb, vb2)
             assert torch.equal(o, want)
-    # rounding of the result (2^-9 of up to 3 in bf16), weights to 2^-16: the same bound as the prefill kernel's
+    # rounding of the result (2^-9 of up to 3 in bf16) and as much again: scores, exponentials and sums in fp32 are far below it
     for b in range(bs):
         s = r2t[rpi[b], : int(lens[b])].long()
         kk, vv = (t[s].double().repeat_interleave(hq // hkv, 1).cpu() for t in (kb, vb))
@@ -62,7 +62,7 @@ def test_fused_launch_and_float64(ops, dtype, cache_dtype, hq, hkv, bs, maxlen, 
 
 
 def test_empty_sequences(ops):
-    """A sequence of no tokens beside others: zeros, with one split and more, by table and by index list."""
+    """A sequence of no tokens beside others: zeros, with one split and more, by page table."""
     hq, hkv, D = 8, 2, 64
     q = torch.randn(3, hq, D, device=DEV).bfloat16()
     kb, vb = torch.randn(70, hkv, D, device=DEV).bfloat16(), torch.randn(70, hkv, D, device=DEV).bfloat16()

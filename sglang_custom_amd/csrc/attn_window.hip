@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void window_attention_valu_kernel(WaArgs a) {
   }
 }
 
-// out[t, h] = sum_s acc_s e^(m_s - M) / sum_s l_s e^(m_s - M), M = max_s m_s, over the key ranges in order.  One wave per
+// out[t, h] = sum_s acc_s e^(m_s - M) / sum_s l_s e^(m_s - M), M = max_s m_s, over the key ranges in order.  One workgroup per
 // (token, head).
 template <typename T>
 __global__ __launch_bounds__(256) void window_attention_merge_kernel(T* __restrict__ out, const float* __restrict__ partial,

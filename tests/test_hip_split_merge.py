@@ -3,7 +3,7 @@
 for bit, every counter zero again afterwards, back-to-back calls on one counter array, and against the
 CPU oracle.  Covers the matrix-core kernel (head_dim 128, 16-bit; GQA 1 / 2 / 4 / 8, both addressing
 modes, an fp8 cache), the launch fused with the qkv reduction / RoPE / cache write, the MLA kernel, and
-the shapes that keep the second launch (more than 64 splits, head_dim 64)."""
+the shapes that keep the second launch (more than 64 splits, head_dim 256)."""
 import pytest
 import torch
 
@@ -98,10 +98,10 @@ def test_in_kernel_merge_kv_indices_mode_and_fp8_cache(ops):
 
 
 def test_shapes_that_keep_the_merge_launch_ignore_the_counters(ops):
-    """More than 64 splits, and the head_dim-64 kernel: the counters are accepted and left alone."""
+    """More than 64 splits, and head_dim 256: the counters are accepted and left alone.  (At head_dim 64 they are zero again.)"""
     dt = torch.bfloat16
     tickets = torch.zeros(1024, dtype=torch.int32, device=DEV)
-    for (Hq, Hkv, D, lens, splits) in ((8, 2, 128, [9000, 130], 70), (8, 2, 64, [300, 40], 3)):
+    for (Hq, Hkv, D, lens, splits) in ((8, 2, 128, [9000, 130], 70), (8, 2, 256, [300, 40], 3), (8, 2, 64, [300, 40], 3)):
         B = len(lens)
         cpu = _paged(830 + D, dt, B, Hq, Hkv, D, lens)
         q, kc, vc, r2t, pool, lt = (x.to(DEV) for x in cpu)

@@ -503,7 +503,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
 // (no probability does) takes sample_whole_row.
 // The one-workgroup routine meets each of its four levels' 128256 entries in 256 bins of two binades, a handful of which
 // take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics.  Launch 1 beside the
-// softmax takes 20 us for that (apart 14 + 13), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 14 from the
+// softmax takes 20 us for that (apart 14 + 13), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 12 from the
 // lists, a chain of some twenty barriers (28 from the row, one CU's pass over 0.5 MB; 58 when thousands are kept).
 constexpr int SB_BINS = 2048, SB_SHIFT = 19, SB_LIST = 8192, SB_SHORT = 512, SB_TILE = 256, SB_MAX_TILES = 4096;
 constexpr int SB_SUM_BITS = 40;
@@ -632,14 +632,18 @@ __device__ __forceinline__ void chunk_list(const Vec<float, 4> (&v)[KEEP], float
 template <bool NORM, bool BINS>
 __global__ __launch_bounds__(SAMP_THREADS) void sample_chunk_kernel(float* __restrict__ data, const float2* __restrict__ partials,
                                                                     const float* __restrict__ temperatures, const int32_t* __restrict__ top_ks,
-                                                                    u64_t* __restrict__ bins, uint2* __restrict__ lists, ChunkTop* __restrict__ tops, int64_t vocab,
+                                                                    const float* __restrict__ top_ps, u64_t* __restrict__ bins, uint2* __restrict__ lists, ChunkTop* __restrict__ tops, int64_t vocab,
                                                                     int64_t row_stride) {
   __shared__ BinScratch sm;
   const int r = blockIdx.x, c = blockIdx.y, chunks = gridDim.y, tid = (int)threadIdx.x;
   float* row = data + (int64_t)r * row_stride;
   const bool vec = (row_stride % 4 == 0) && aligned16(data);
   const ChunkSpan sp = chunk_span(vocab, c, chunks);
-  const bool held = vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS && sp.v0 < sp.v1;
+  // A row that neither top_k nor top_p cuts short draws from entries that no list has, and without a list or a softmax nothing is gained by
+  // holding the chunk either (300 rows x 32768: 30 us with lists, 14 with the chunk held, 10.5 so).
+  const int want = BINS && top_ks != nullptr ? max(top_ks[r], 0) : 0x7fffffff;
+  const bool listed = BINS && (want <= SB_TOP || (top_ps != nullptr && top_ps[r] < 1.0f));
+  const bool held = (NORM || listed) && vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS && sp.v0 < sp.v1;
   Vec<float, 4> v[KEEP];
   if (held) chunk_load(v, row, sp);
   const RowNorm norm(partials + (NORM ? (int64_t)r * chunks : 0), NORM ? chunks : 0, NORM ? temperatures[r] : 1.0f);
@@ -678,29 +682,42 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_chunk_kernel(float* __res
     if constexpr (BINS) {
       __syncthreads();
       const int most = SB_TOP / chunks;
-      const int want = top_ks ? max(top_ks[r], 0) : 0x7fffffff;
-      chunk_list(v, last, sp, vocab, most, want, sm, lists + (int64_t)r * SB_TOP + c * most, count, lowest);
+      if (listed) chunk_list(v, last, sp, vocab, most, want, sm, lists + (int64_t)r * SB_TOP + c * most, count, lowest);
     }
   } else {
-    for (int64_t i = sp.v0 + tid; i < sp.v1; i += SAMP_THREADS) {
-      Vec<float, 4> v;
-      if (vec) v = ldvec<float, 4>(row + i * 4);
+    auto load = [&](int64_t i) {
+      Vec<float, 4> w;
+      if (vec) w = ldvec<float, 4>(row + i * 4);
       else
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v.v[j] = row[i * 4 + j];
+        for (int j = 0; j < 4; ++j) w.v[j] = row[i * 4 + j];
+      return w;
+    };
+    auto take = [&](Vec<float, 4> w, int64_t i) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        if (NORM) v.v[j] = norm.prob(v.v[j]);
-        mx = fmaxf(mx, v.v[j]);
-        if (BINS) sb_count(sm.hist, v.v[j]);
+        if (NORM) w.v[j] = norm.prob(w.v[j]);
+        mx = fmaxf(mx, w.v[j]);
+        if (BINS) sb_count(sm.hist, w.v[j]);
       }
       if (NORM) {
-        if (vec) stvec<float, 4>(row + i * 4, v);
+        if (vec) stvec<float, 4>(row + i * 4, w);
         else
 #pragma unroll
-          for (int j = 0; j < 4; ++j) row[i * 4 + j] = v.v[j];
+          for (int j = 0; j < 4; ++j) row[i * 4 + j] = w.v[j];
+      }
+    };
+    int64_t i = sp.v0 + tid;
+    if constexpr (!NORM) {     // four loads in flight (beside the exponentials they gain nothing: 200 rows x 128256 166 us the batch, 173 so)
+      for (; i + 3 * SAMP_THREADS < sp.v1; i += 4 * SAMP_THREADS) {
+        Vec<float, 4> w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = load(i + u * SAMP_THREADS);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) take(w[u], i + u * SAMP_THREADS);
       }
     }
+    for (; i < sp.v1; i += SAMP_THREADS) take(load(i), i);
   }
   if constexpr (BINS) {
     mx = block_reduce_max(mx, sm.red);
@@ -995,12 +1012,18 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_pick_kernel(
       total += x;
     }
     if (lane > 0) base += left;
+    // Slots are in index order: a wave's first entry past the draw and its last entry at all speak for it (an LDS atomic for every entry, on
+    // one address, took 3 us where thousands are kept).
+    int pick = -1, kept = -1;
 #pragma unroll
-    for (int j = 0; j < SLOTS; ++j)
+    for (int j = SLOTS - 1; j >= 0; --j)
       if (in[j]) {
-        atomicMax(&s_last, (int)slot[j].y);
-        if (base + upto[j] > (double)sr.uniform * total) atomicMin(&s_pick, (int)slot[j].y);
+        if (kept < 0) kept = (int)slot[j].y;
+        if (base + upto[j] > (double)sr.uniform * total) pick = (int)slot[j].y;
       }
+    const u64_t picks = __ballot(pick >= 0), keeps = __ballot(kept >= 0);
+    if (picks != 0 && lane == __ffsll((unsigned long long)picks) - 1) atomicMin(&s_pick, pick);
+    if (keeps != 0 && lane == 63 - __clzll((long long)keeps)) atomicMax(&s_last, kept);
     __syncthreads();
     if (tid == 0) ids[blockIdx.x] = s_pick != 0x7fffffff ? s_pick : max(s_last, 0);
     return;
@@ -1212,7 +1235,7 @@ int mi355_softmax_temperature_split(float* logits, const float* temperatures, in
   hipLaunchKernelGGL(softmax_partials_kernel, dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, partials,
                      logits, temperatures, vocab, row_stride);
   hipLaunchKernelGGL((sample_chunk_kernel<true, false>), dim3((unsigned)rows, chunks), dim3(SAMP_THREADS), 0, (hipStream_t)stream, logits,
-                     partials, temperatures, (const int32_t*)nullptr, (u64_t*)nullptr, (uint2*)nullptr, (ChunkTop*)nullptr, vocab, row_stride);
+                     partials, temperatures, (const int32_t*)nullptr, (const float*)nullptr, (u64_t*)nullptr, (uint2*)nullptr, (ChunkTop*)nullptr, vocab, row_stride);
   MI355_CHECK_LAUNCH("softmax_temperature_split");
   return MI355_OK;
 }
@@ -1244,10 +1267,10 @@ static int sample_launches(int32_t* ids, float* data, const float* temperatures,
   const dim3 grid((unsigned)rows, chunks), block(SAMP_THREADS);
   if (fused) {
     hipLaunchKernelGGL(softmax_partials_kernel, grid, block, 0, stream, partials, data, temperatures, vocab, row_stride);
-    hipLaunchKernelGGL((sample_chunk_kernel<true, true>), grid, block, 0, stream, data, partials, temperatures, top_ks, bins, lists, tops, vocab,
+    hipLaunchKernelGGL((sample_chunk_kernel<true, true>), grid, block, 0, stream, data, partials, temperatures, top_ks, top_ps, bins, lists, tops, vocab,
                        row_stride);
   } else {
-    hipLaunchKernelGGL((sample_chunk_kernel<false, true>), grid, block, 0, stream, data, (const float2*)nullptr, (const float*)nullptr, top_ks,
+    hipLaunchKernelGGL((sample_chunk_kernel<false, true>), grid, block, 0, stream, data, (const float2*)nullptr, (const float*)nullptr, top_ks, top_ps,
                        bins, lists, tops, vocab, row_stride);
   }
   hipLaunchKernelGGL(sample_pick_kernel, dim3((unsigned)rows), block, 0, stream, ids, bins, lists, tops, chunks, data, top_ks, top_ps, min_ps,

@@ -29,9 +29,14 @@ TILED_MIN_TILES = 192
 # ... unless the tiles share long reductions: with K split over the idle CUs the kernel is ahead of the library from K = 8192 on, but
 # for the few rows whose sums cost as much as the product (us, library | split: 4096 x 14336 with 126 rows 52 | 40, 330 75 | 58, 646
 # 106 | 84, 1134 140 | 125; 4096 x 11264 with 80 rows 36 | 37, 128 61 | 39, 700 84 | 72; 2048 x 8192 with 128 rows 22 | 25, 200
-# 30 | 27, 1000 52 | 48, 1353 53 | 56, 2100 83 | 74; 2048 x 5632 with 400 rows 26 | 29, 1000 40 | 40, 1500 45 | 48)
+# 30 | 27, 1000 52 | 48, 1353 53 | 56, 2100 83 | 74; 2048 x 5632 with 400 rows 26 | 29, 1000 40 | 40, 1500 45 | 48).  Products of less
+# than 2.1 billion multiply-adds are launches and sums more than anything else (library / split: 512 x 8192 with 300 rows 0.78, 128 x 16384 with
+# 256 0.64, 1024 x 14336 with 128 0.97, 150 1.23; 1280 x 8192 with 200 1.08), and columns of 16384 leave at most four workgroups a
+# tile (x 8192 with 150 to 300 rows 0.77 to 0.93, x 16384 0.85 to 1.25; 8192 x 8192 0.88 to 1.36, x 14336 1.01 to 1.77)
 SPLIT_MIN_K = 8192
 SPLIT_MIN_MK = 1200000
+SPLIT_MIN_MACS = 2.1e9
+SPLIT_MAX_N = 8192
 
 
 def _use_tiled(m: int, n_out_tiles_cols: int, n: int, k: int, dtype, silu_mul: bool) -> bool:
@@ -39,7 +44,8 @@ def _use_tiled(m: int, n_out_tiles_cols: int, n: int, k: int, dtype, silu_mul: b
         return False
     tiles = ((m + 255) // 256) * ((n_out_tiles_cols + 255) // 256)
     ops = get_ops()
-    return ((tiles >= TILED_MIN_TILES or (k >= SPLIT_MIN_K and m * k >= SPLIT_MIN_MK and ops.tiled_tail_splits(m, n, k, False, silu_mul) > 1))
+    return ((tiles >= TILED_MIN_TILES or (k >= SPLIT_MIN_K and m * k >= SPLIT_MIN_MK and m * n * k >= SPLIT_MIN_MACS and n <= SPLIT_MAX_N
+                                          and ops.tiled_tail_splits(m, n, k, False, silu_mul) > 1))
             and ops.linear_tiled_supported(m, n, k, dtype, silu_mul))
 
 

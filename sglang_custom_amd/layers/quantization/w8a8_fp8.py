@@ -38,9 +38,14 @@ PREFILL_GEMM = os.environ.get("MI355_PREFILL_FP8_GEMM", "auto")
 # with 1100, 120, 36 | 43; 4096 x 4096 with 2300 rows, 144, 57 | 44, 6144 x 4096 with 1600, 168, 57 | 45; 4096 x 14336 with 2300, 144,
 # 171 | 128) ...
 TILED_MIN_TILES = 144
-# ... unless they share long reductions (4096 x 14336 with 80 rows 26 | 31, 150 35 | 33, 300 49 | 39, 646 70 | 52, 1100 90 | 71)
+# ... unless they share long reductions (4096 x 14336 with 80 rows 26 | 31, 150 35 | 33, 300 49 | 39, 646 70 | 52, 1100 90 | 71), the shorter
+# the more rows and columns it takes (library / split: 2048 x 14336 with 256 rows 0.92, 300 1.07; 4096 x 11264 with 256 0.88, 300
+# 1.08; x 8192 with 300 0.90, 520 1.12; 2048 x 8192 with 800 0.83, 1100 1.17), and 128 rows (8192 x 14336 with 90 0.90, 128
+# 1.06) and at most 8192 columns (16384 x 8192 0.91, x 16384 0.7 to 0.95)
 SPLIT_MIN_K = 8192
-SPLIT_MIN_MK = 1900000
+SPLIT_MIN_M = 128
+SPLIT_MIN_MNKK = 1.2e14
+SPLIT_MAX_N = 8192
 _SCALED_MM_OK = None   # None = untried; torch._scaled_mm (hipBLASLt) with row-wise scales
 
 
@@ -65,7 +70,8 @@ def _library_scaled_mm(xq, wq, xs, ws, out_dtype, bias):
 def _tiled_ok(m: int, n: int, k: int, out_dtype, silu_mul: bool) -> bool:
     tiles = ((m + 255) // 256) * ((n + 255) // 256)
     ops = get_ops()
-    return ((tiles >= TILED_MIN_TILES or (k >= SPLIT_MIN_K and m * k >= SPLIT_MIN_MK and ops.tiled_tail_splits(m, n, k, True, silu_mul) > 1))
+    return ((tiles >= TILED_MIN_TILES or (k >= SPLIT_MIN_K and m >= SPLIT_MIN_M and m * n * k * k >= SPLIT_MIN_MNKK and n <= SPLIT_MAX_N
+                                          and ops.tiled_tail_splits(m, n, k, True, silu_mul) > 1))
             and ops.fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, silu_mul))
 
 

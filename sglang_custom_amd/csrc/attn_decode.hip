@@ -689,7 +689,8 @@ __global__ __launch_bounds__(256) void decode_attn_mfma_kernel(const T* __restri
 // ------------------------------------------------------------------------------------------
 // Weights 0 <= p <= 1 as 16-bit terms of whole products: p UP = hi + (mid + low) / MID.  MID takes mid below hi's size, so that no product is larger
 // than hi's.  The lanes of a column need one term each; a wave's time for a tile is the chain from its scores to its products.
-// bf16: the upper halves of p, of what that leaves and of what that leaves: all 24 bits down to 2^-117, and what lies above 2^-140 further down.
+// bf16: the upper halves of p, of what that leaves and of what that leaves: all 24 bits down to 2^-116, and what lies above 2^-139
+// down to 2^-126 (smaller weights come scaled).
 // fp16: all bits down to 2^-26 and then what lies above 2^-50; hi is never zero (what it has too much is in mid), so that an infinite
 // value row makes infinity whatever its weight.
 template <typename T> struct WeightTerms;

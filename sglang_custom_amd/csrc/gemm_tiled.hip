@@ -421,14 +421,22 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const int ldA_l = g == 0 ? LW0 : LX1, ldB_l = g == 0 ? LW1 : LX0;
   const int ldB_d = g == 0 ? 1 : 2;     // tile distance of the second request (the first is always t + 1)
 
+  // EPI 3: every expert's K is walked from another tile on and round the end.  Rows of operands lie 4 KB or more apart, so workgroups in
+  // step ask for the same 128-byte column of all the weights and with it for few memory channels.  A layer of 32 experts of 2048 x 2048, 4
+  // per token, us with K from its start -> staggered: 16 tokens 154 -> 131, 131 tokens 187 -> 144 (one product 75 -> 53: 268 MB at 5.1 TB/s),
+  // 1000 309 -> 279, 3000 325 -> 310; by column of tiles as well 147 at 131, by that alone 167.  A dense product's rows and columns have one order
+  // of K each, whichever tile they are in and whatever is fused behind it.
+  const int rot = EPI == 3 ? p.tile_expert[tm] % T_ : 0;
+#define GT_AT(tl) ((int64_t)(EPI == 3 && (tl) + rot >= T_ ? (tl) + rot - T_ : (tl) + rot) * 128)
+
   // ---- prologue: all of tile 0 and x rows 0..127 of tile 1 ------------------------------------
 #pragma unroll
-  for (int i = 0; i < 4; ++i) glds16(ldA[i], lds_w + ldA_l + i * 1024);            // W0(0) | x1(0)
+  for (int i = 0; i < 4; ++i) glds16(ldA[i] + GT_AT(0), lds_w + ldA_l + i * 1024);            // W0(0) | x1(0)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) glds16(ldB[i], lds_w + ldB_l + i * 1024);            // W1(0) | x0(0)
+  for (int i = 0; i < 4; ++i) glds16(ldB[i] + GT_AT(0), lds_w + ldB_l + i * 1024);            // W1(0) | x0(0)
   if (g == 1) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) glds16(ldB[i] + 128, lds_w + GT_STAGE + ldB_l + i * 1024);   // x0(1)
+    for (int i = 0; i < 4; ++i) glds16(ldB[i] + GT_AT(1), lds_w + GT_STAGE + ldB_l + i * 1024);   // x0(1)
   }
 
   // ---- fragment read addresses ----------------------------------------------------------------
@@ -456,7 +464,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     if (!(TAIL) || (tl) < T_) {                                                              \
       char* d_ = lds_w + (((tl) & 1) ? GT_STAGE : 0) + (ldso);                               \
       _Pragma("unroll") for (int i = 0; i < 4; ++i)                                          \
-          if (!(PART) || i < (COUNT)) glds16(ptr[i] + (int64_t)(tl) * 128, d_ + i * 1024);   \
+          if (!(PART) || i < (COUNT)) glds16(ptr[i] + GT_AT(tl), d_ + i * 1024);   \
     }                                                                                        \
   } while (0)
 #define GT_SLOT_END()                                                                        \
@@ -523,6 +531,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
 #undef GT_LOAD4
 #undef GT_SLOT_END
 #undef GT_TILE
+#undef GT_AT
 
   // ---- epilogue ---------------------------------------------------------------------------------
   if constexpr (EPI != 3) {

@@ -120,3 +120,21 @@ def test_padding_anywhere_in_a_tile(ops, holes):
         keep = r >= 0
         want = (x.float()[r[keep].long().to(DEV)] @ w[e].float().T).to(torch.bfloat16)
         assert torch.equal(y[256 * tile: 256 * tile + 256][keep.to(DEV)], want)
+
+
+@pytest.mark.parametrize("K", [128, 192, 448])
+def test_every_expert_walks_all_of_k(ops, K):
+    """Experts start K at different tiles of 64 and go round its end: two, three and seven of them for nine experts (more than there
+    are tiles to start from).  Small integers, so sums are exact; a tile skipped or taken twice shows."""
+    g = torch.Generator().manual_seed(K)
+    E, N, x = 9, 272, torch.randint(-2, 3, (40, K), generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randint(-2, 3, (E, N, K), generator=g).to(torch.bfloat16).to(DEV)
+    rows = torch.randint(0, 40, (E * 256,), generator=g).int().to(DEV)
+    te, used = torch.arange(E, dtype=torch.int32, device=DEV), torch.tensor([E], dtype=torch.int32, device=DEV)
+    y = torch.full((E * 256, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.check(ops._lib_().mi355_moe_grouped_linear_tiled(y.data_ptr(), x.data_ptr(), K, w.data_ptr(), rows.data_ptr(), te.data_ptr(),
+                                                         used.data_ptr(), 0, E * 256, N, K, ops._dt(x), ops._stream(x)), "tiled")
+    torch.cuda.synchronize()
+    for e in range(E):
+        part = slice(256 * e, 256 * e + 256)
+        assert torch.equal(y[part], (x.float()[rows[part].long()] @ w[e].float().T).to(torch.bfloat16)), e

@@ -264,6 +264,23 @@ int mi355_extend_attention(const void* q_extend, const void* k_extend, const voi
                            int v_head_dim, int64_t q_stride, int64_t k_stride, int64_t v_stride,
                            int64_t num_slots, float sm_scale, float logit_cap,
                            int sliding_window_size, int dtype, void* stream);
+/* The same with the keys of a block of queries shared by `splits` workgroups where the matrix-core kernel of head_dim 64 or 128 serves the
+ * call (elsewhere splits is ignored): rows = T, workspace of mi355_extend_attention_workspace_bytes (16-byte aligned, contents
+ * irrelevant).  mi355_extend_attention_splits: how many pay for T rows of bs sequences, the longest with max_len_extend of them, on
+ * prefix_tokens cached ones; 1: none. */
+int mi355_extend_attention_splits(int64_t rows, int64_t bs, int64_t max_len_extend, int64_t prefix_tokens, int has_mask, int hq, int head_dim,
+                                  int v_head_dim, float sm_scale, float logit_cap, int sliding_window_size, int dtype);
+int64_t mi355_extend_attention_workspace_bytes(int64_t rows, int hq, int v_head_dim, int splits);
+int mi355_extend_attention_ws(const void* q_extend, const void* k_extend, const void* v_extend,
+                              void* o_extend, const void* k_buffer, const void* v_buffer,
+                              const int32_t* qo_indptr, const int32_t* kv_indptr,
+                              const int32_t* kv_indices, const uint8_t* custom_mask,
+                              const int64_t* mask_indptr, int is_causal, int skip_prefix_custom_mask,
+                              int64_t bs, int64_t max_len_extend, int hq, int hkv, int head_dim,
+                              int v_head_dim, int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                              int64_t num_slots, float sm_scale, float logit_cap,
+                              int sliding_window_size, int dtype, int64_t rows, int splits, void* workspace,
+                              int64_t workspace_bytes, void* stream);
 
 /* mi355_decode_attention for callers that cannot allocate device memory or pass a workspace (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the split-KV

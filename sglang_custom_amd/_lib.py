@@ -39,6 +39,10 @@ _SIGNATURES = {
     "mi355_decode_split_plan": (I, [L, I, L, I, I, P, P]),
     "mi355_extend_attention": (I, [P, P, P, P, P, P, P, P, P, P, P, I, I, L, L, I, I, I, I, L, L, L,
                                    L, F, F, I, I, P]),
+    "mi355_extend_attention_ws": (I, [P, P, P, P, P, P, P, P, P, P, P, I, I, L, L, I, I, I, I, L, L, L,
+                                   L, F, F, I, I, L, I, P, L, P]),
+    "mi355_extend_attention_splits": (I, [L, L, L, L, I, I, I, I, F, F, I, I]),
+    "mi355_extend_attention_workspace_bytes": (L, [L, I, I, I]),
     "mi355_linear_workspace_bytes": (L, [L, L, L]),
     "mi355_linear": (I, [P, P, P, P, L, L, L, L, P, L, I, I, P]),
     "mi355_packed_weight_elems": (L, [L, L]),

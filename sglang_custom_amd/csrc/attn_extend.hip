@@ -10,6 +10,7 @@
 // every dtype -- this is also the fp32 parity path.  Row max uses xor-shuffles across the 16
 // lanes that share a row; the row sum is reduced once at the end.
 #include "common.cuh"
+#include <algorithm>
 #include <type_traits>
 #include <math.h>
 
@@ -39,6 +40,10 @@ struct ExtendParams {
   int kv_head;                // elements between consecutive heads of k / v
   int rot_dims, interleaved;  // of the query's rope part: features 2 i with 2 i + 1, or (rot_dims 64) i with i + 32
   float rot_mag;
+  // splits of the keys (grid y): unnormalised sums part [splits, rows, hq, Dv] and (maximum, weights' sum) part_ml [splits, rows, hq]
+  float* part;
+  float2* part_ml;
+  int64_t rows;
 };
 
 // DP: padded head dim (>= D, Dv; multiple of 64). BN: keys per tile. VEC: 16-B global loads.
@@ -578,7 +583,9 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // careful (D = 64): value rows may hold infinities and NaN, which no product with a weight of zero may meet (keys that the query does not
 // see) nor with a weight's lower terms.  The images then hold the rows without them, and beside them, in the half that is free, the rows
 // as they are, from which they are added for the queries that see their key.  Returns (the same in all threads) whether a result is no number.
-template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128, bool MASK = false>
+// SPLIT: gridDim.y workgroups share the block's key tiles, in runs of at least SPLIT_TILES; extend_split_merge_kernel adds their sums.
+constexpr int SPLIT_TILES = 4;
+template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128, bool MASK = false, bool SPLIT = false>
 __device__ __forceinline__ bool extend_attn_mfma32_body(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs, bool careful = false) {
@@ -666,7 +673,16 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
   const int last_row = min(r0 + 127, ext - 1);
   const bool causal = LATENT || (!MASK && p.is_causal);
   const int total = causal ? prefix + last_row + 1 : prefix + ext;
-  const int n_tiles = (total + 63) / 64;
+  int n_tiles = (total + 63) / 64, first_tile = 0;
+  if constexpr (SPLIT) {
+    const int run = max((n_tiles + (int)gridDim.y - 1) / (int)gridDim.y, SPLIT_TILES);
+    first_tile = run * (int)blockIdx.y;
+    if (first_tile >= n_tiles) {   // (workgroup-uniform) no weights: the merge reads no sums
+      if (hh == 0 && qrow < ext) p.part_ml[((int64_t)blockIdx.y * p.rows + q_start + qrow) * p.hq + h] = make_float2(-INFINITY, 0.f);
+      return false;
+    }
+    n_tiles = min(n_tiles, first_tile + run);
+  }
   const int my_limit = causal ? prefix + qrow_c : prefix + ext - 1;   // last visible key of this lane's query
   const int wave_min_limit = causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
   const int wave_max_limit = causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
@@ -822,11 +838,11 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
   };
 
   if (!careful) {
-    if (!LATENT) load_slots(0);
-    load_tile(0);
-    if (!LATENT) load_slots(1);
+    if (!LATENT) load_slots(first_tile);
+    load_tile(first_tile);
+    if (!LATENT) load_slots(first_tile + 1);
   }
-  for (int kt = 0; kt < n_tiles; ++kt) {
+  for (int kt = first_tile; kt < n_tiles; ++kt) {
     __syncthreads();            // previous tile fully consumed
     if (careful) {              // (nothing ahead: no registers spilled for a rare path)
       load_slots(kt);
@@ -1012,7 +1028,19 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     __syncthreads();
     odd = (flags[0] | flags[1] | flags[2] | flags[3]) != 0;
   }
-  if (qrow < ext) {
+  if (SPLIT) {
+    if (qrow < ext) {
+      const int64_t at = ((int64_t)blockIdx.y * p.rows + q_start + qrow) * p.hq + h;
+      if (hh == 0) p.part_ml[at] = make_float2(m, lsum * P_UP);
+      float* op = p.part + at * D + 4 * hh;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq)
+          *reinterpret_cast<float4*>(op + 32 * dt + 8 * rq) =
+              make_float4(ot[dt][4 * rq], ot[dt][4 * rq + 1], ot[dt][4 * rq + 2], ot[dt][4 * rq + 3]);
+    }
+  } else if (qrow < ext) {
     const float inv = lsum > 0.f ? 1.f / (lsum * P_UP) : 0.f;
     T* op = o_ext + ((int64_t)(q_start + qrow) * p.hq + h) * D + 4 * hh;
 #pragma unroll
@@ -1032,11 +1060,11 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
 // ~270 registers and runs one workgroup per CU instead of spilling (measured at 4 x 4096 tokens x 16 heads: 470 TFLOP/s
 // against 412 with 24 spilled registers at two workgroups per CU; issuing the next tile's loads behind the score phase
 // spills more).
-template <typename T, bool KV8 = false>
+template <typename T, bool KV8, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_mfma32_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
-  extend_attn_mfma32_body<T, KV8, 128>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
+  extend_attn_mfma32_body<T, KV8, 128, false, 128, false, SPLIT>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
 }
 // Head dimension 64 needs 190 registers: two workgroups per CU (three, with a few registers in scratch memory, took longer: 4 x 340 tokens on 1180
 // cached 80 us).  Bound by the softmax's instructions (about fifteen per score, five of them the weights' three terms, beside an MFMA
@@ -1044,15 +1072,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // cached 378 -> 68 (54), 704 + 430 tokens on none 121 -> 24 (20), 4000 on none 1493 -> 170 (136), 65 on 3000 510 -> 84 (73), 70 on none 24 -> 9
 // (9); fp8 cache, 3 x 197 on 1614 478 -> 61 (53).  The heads of a group packed into the rows (less of the triangle's edge in vain) was
 // no faster.
-template <typename T, bool KV8, bool MASK>
+template <typename T, bool KV8, bool MASK, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_mfma32_d64_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
-  if (extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs)) {
+  if (extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK, SPLIT>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs)) {
     __syncthreads();
-    extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs, true);
+    extend_attn_mfma32_body<T, KV8, 64, false, 64, MASK, SPLIT>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs, true);
   }
 }
+
+// Adds the splits' sums: D / 4 lanes a (row, head), the sums of four splits in flight.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void extend_split_merge_kernel(T* __restrict__ o, const float* __restrict__ part,
+                                                                 const float2* __restrict__ ml, const int32_t* __restrict__ qo_indptr, int64_t bs,
+                                                                 int64_t items, int hq, int splits) {
+  constexpr int L = D / 4;
+  const int64_t at = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+  if (at >= items || at < (int64_t)qo_indptr[0] * hq || at >= (int64_t)qo_indptr[bs] * hq) return;   // rows of no sequence stay as they are
+  const int c = 4 * (threadIdx.x % L);
+  float top = -INFINITY;
+  for (int s = 0; s < splits; ++s) top = fmaxf(top, ml[s * items + at].x);
+  const float ms = top == -INFINITY ? 0.f : top;
+  float l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < splits; s0 += 4) {
+    float4 v[4];
+    float w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int s = min(s0 + j, splits - 1);
+      const float2 a = ml[s * items + at];
+      const bool some = s0 + j < splits && a.y != 0.f;   // a split without weights has written no sums
+      w[j] = some ? exp2f(a.x - ms) : 0.f;
+      if (some) l = fmaf(a.y, w[j], l);
+      v[j] = some ? *reinterpret_cast<const float4*>(part + (s * items + at) * D + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      acc[0] = fmaf(v[j].x, w[j], acc[0]);
+      acc[1] = fmaf(v[j].y, w[j], acc[1]);
+      acc[2] = fmaf(v[j].z, w[j], acc[2]);
+      acc[3] = fmaf(v[j].w, w[j], acc[3]);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  Vec<T, 4> r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r.v[j] = from_f32<T>(acc[j] * inv);
+  stvec<T, 4>(o + at * D + c, r);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void extend_attn_mfma32_wide_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
@@ -1106,40 +1175,58 @@ int g_extend_variant = 0;
 static constexpr int g_extend_variant = 0;
 #endif
 
+// Which of the 32 x 32 kernels serves the call; the maximum is taken of unscaled scores.
+static bool mfma32_serves(int D, int Dv, bool kv8, bool mask, int sliding_window, float logit_cap, float sm_scale) {
+  return ((D == 128 && Dv == 128) || (D == 192 && Dv == 128 && !kv8) || (D == 64 && Dv == 64)) && (!mask || D == 64) && sliding_window <= 0 &&
+         logit_cap <= 0.f && sm_scale > 0.f && g_extend_variant == 0;
+}
+
+template <typename T, int D>
+static int launch_mfma32(const void* q, const void* k, const void* v, void* o, const void* kb, const void* vb, const ExtendParams& p,
+                         int64_t bs, int nqb, int64_t npairs, int64_t wgs, int splits, bool kv8, hipStream_t st) {
+  using Kernel = void (*)(const T*, const T*, const T*, T*, const T*, const T*, ExtendParams, int, int);
+  Kernel kernel;
+  if constexpr (D == 64) {
+    if (splits > 1)
+      kernel = p.custom_mask ? (kv8 ? extend_attn_mfma32_d64_kernel<T, true, true, true> : extend_attn_mfma32_d64_kernel<T, false, true, true>)
+                             : (kv8 ? extend_attn_mfma32_d64_kernel<T, true, false, true> : extend_attn_mfma32_d64_kernel<T, false, false, true>);
+    else
+      kernel = p.custom_mask ? (kv8 ? extend_attn_mfma32_d64_kernel<T, true, true, false> : extend_attn_mfma32_d64_kernel<T, false, true, false>)
+                             : (kv8 ? extend_attn_mfma32_d64_kernel<T, true, false, false> : extend_attn_mfma32_d64_kernel<T, false, false, false>);
+  } else {
+    if (splits > 1) kernel = kv8 ? extend_attn_mfma32_kernel<T, true, true> : extend_attn_mfma32_kernel<T, false, true>;
+    else kernel = kv8 ? extend_attn_mfma32_kernel<T, true, false> : extend_attn_mfma32_kernel<T, false, false>;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)wgs, (unsigned)splits), dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, (T*)o, (const T*)kb,
+                     (const T*)vb, p, nqb, (int)npairs);
+  if (splits > 1) {
+    const int64_t items = p.rows * p.hq;
+    hipLaunchKernelGGL((extend_split_merge_kernel<T, D>), dim3((unsigned)((items + 1024 / D - 1) / (1024 / D))), dim3(256), 0, st, (T*)o, p.part,
+                       p.part_ml, p.qo_indptr, bs, items, p.hq, splits);
+  }
+  return MI355_OK;
+}
+
 template <typename T>
 static int launch_extend(const void* q, const void* k, const void* v, void* o, const void* kb,
                          const void* vb, const ExtendParams& p, int64_t bs, int64_t max_len_extend,
-                         bool kv8, hipStream_t st) {   // kv8: the KV cache holds e4m3fn bytes
+                         bool kv8, int splits, hipStream_t st) {   // kv8: the KV cache holds e4m3fn bytes
   constexpr int VE = V16<T>::n;
   const int dmax = p.D > p.Dv ? p.D : p.Dv;
   const bool vec = p.D % VE == 0 && p.Dv % VE == 0 && p.q_stride % VE == 0 &&
                    p.k_stride % VE == 0 && p.v_stride % VE == 0 && aligned16(q) && aligned16(k) &&
                    aligned16(v) && aligned16(o) && aligned16(kb) && aligned16(vb);
   if constexpr (!std::is_same<T, float>::value) {
-    if (vec && ((p.D == 128 && p.Dv == 128) || (p.D == 192 && p.Dv == 128 && !kv8) || (p.D == 64 && p.Dv == 64)) &&
-        (!p.custom_mask || p.D == 64) && p.sliding_window <= 0 && p.logit_cap <= 0.f && p.sm_scale > 0.f && g_extend_variant == 0) {   // the 32x32 kernel takes the maximum of unscaled scores
+    if (vec && mfma32_serves(p.D, p.Dv, kv8, p.custom_mask != nullptr, p.sliding_window, p.logit_cap, p.sm_scale)) {
       // 128 query rows of one head per workgroup; (sequence, kv head) pairs dealt round-robin to the XCDs
       const int nqb = (int)((max_len_extend + 127) / 128);
       const int64_t npairs = bs * p.hkv;
       const int64_t wgs = 8 * ((npairs + 7) / 8) * (p.hq / p.hkv) * nqb;
       if (wgs < (int64_t)1 << 31) {
-        const dim3 grid1((unsigned)wgs);
-        if (p.D == 64) {
-          const auto kernel = p.custom_mask ? (kv8 ? extend_attn_mfma32_d64_kernel<T, true, true> : extend_attn_mfma32_d64_kernel<T, false, true>)
-                                            : (kv8 ? extend_attn_mfma32_d64_kernel<T, true, false> : extend_attn_mfma32_d64_kernel<T, false, false>);
-          hipLaunchKernelGGL(kernel, grid1, dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb,
-                             (int)npairs);
-          return MI355_OK;
-        }
-        if (p.D == 192)
-          hipLaunchKernelGGL((extend_attn_mfma32_wide_kernel<T>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
-                             (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
-        else if (kv8)
-          hipLaunchKernelGGL((extend_attn_mfma32_kernel<T, true>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
-                             (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
-        else
-          hipLaunchKernelGGL((extend_attn_mfma32_kernel<T, false>), grid1, dim3(256), 0, st, (const T*)q, (const T*)k,
-                             (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
+        if (p.D == 64) return launch_mfma32<T, 64>(q, k, v, o, kb, vb, p, bs, nqb, npairs, wgs, splits, kv8, st);
+        if (p.D == 128) return launch_mfma32<T, 128>(q, k, v, o, kb, vb, p, bs, nqb, npairs, wgs, splits, kv8, st);
+        hipLaunchKernelGGL((extend_attn_mfma32_wide_kernel<T>), dim3((unsigned)wgs), dim3(256), 0, st, (const T*)q, (const T*)k,
+                           (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
         return MI355_OK;
       }
     }
@@ -1171,6 +1258,27 @@ using namespace mi355;
 
 extern "C" {
 
+// The kernel holds two workgroups a CU, 512 in all; fewer leave CUs idle while each walks its keys alone.  Their number is estimated:
+// rows / 128 blocks of queries and half a block of each sequence, at most the longest's for all, times the heads.  `tiles` of 64 keys
+// a block on average, 4 or more a split.  us a launch out of cold caches, unsplit | split (32 / 8 heads): head_dim 128, fp8 cache 83 rows on 1933 cached
+// 111 | 29 (in a step), 97 x 6 on 2663 212 | 124 (2), 152 x 3 on 2411 189 | 75 (4), bf16 99 on 572 28 | 23 (2); head_dim 64, 3 x 121 on
+// 1513 50 | 35 (3), fp8 86 on 816 42 | 31 (2), 2 x 244 on 2141 97 | 49 (4).  Left whole: no cached tokens (1148 new ones, head_dim 64,
+// 37 | 42 in two; 3 x 993, 128, 51 | 80), 512 workgroups (4 x 490 on 1750 83 | 100), few tiles (400 new on 300, seven, 22 | 26).
+int mi355_extend_attention_splits(int64_t rows, int64_t bs, int64_t max_len_extend, int64_t prefix_tokens, int has_mask, int hq, int head_dim,
+                                  int v_head_dim, float sm_scale, float logit_cap, int sliding_window_size, int dtype) {
+  const bool kv8 = (dtype & MI355_KV_FP8) != 0;
+  if ((dtype & 0xff) == MI355_F32 || rows < 1 || bs < 1 || max_len_extend < 1 || hq < 1 || rows > (1 << 24) || hq > 4096 ||
+      !mfma32_serves(head_dim, v_head_dim, kv8, has_mask != 0, sliding_window_size, logit_cap, sm_scale) || head_dim > 128)
+    return 1;
+  const int64_t wgs = std::min(bs * ((max_len_extend + 127) / 128), rows / 128 + bs / 2 + 1) * hq;
+  const int64_t tiles = (prefix_tokens + rows / 2) / bs / 64;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({512 / wgs, (tiles - 2) / SPLIT_TILES, 8}));
+}
+
+int64_t mi355_extend_attention_workspace_bytes(int64_t rows, int hq, int v_head_dim, int splits) {
+  return splits > 1 ? (int64_t)splits * rows * hq * (v_head_dim + 2) * 4 : 0;
+}
+
 int mi355_extend_attention(const void* q_extend, const void* k_extend, const void* v_extend,
                            void* o_extend, const void* k_buffer, const void* v_buffer,
                            const int32_t* qo_indptr, const int32_t* kv_indptr,
@@ -1180,6 +1288,22 @@ int mi355_extend_attention(const void* q_extend, const void* k_extend, const voi
                            int v_head_dim, int64_t q_stride, int64_t k_stride, int64_t v_stride,
                            int64_t num_slots, float sm_scale, float logit_cap,
                            int sliding_window_size, int dtype, void* stream) {
+  return mi355_extend_attention_ws(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices, custom_mask,
+                                   mask_indptr, is_causal, skip_prefix_custom_mask, bs, max_len_extend, hq, hkv, head_dim, v_head_dim,
+                                   q_stride, k_stride, v_stride, num_slots, sm_scale, logit_cap, sliding_window_size, dtype, 0, 1, nullptr,
+                                   0, stream);
+}
+
+int mi355_extend_attention_ws(const void* q_extend, const void* k_extend, const void* v_extend,
+                              void* o_extend, const void* k_buffer, const void* v_buffer,
+                              const int32_t* qo_indptr, const int32_t* kv_indptr,
+                              const int32_t* kv_indices, const uint8_t* custom_mask,
+                              const int64_t* mask_indptr, int is_causal, int skip_prefix_custom_mask,
+                              int64_t bs, int64_t max_len_extend, int hq, int hkv, int head_dim,
+                              int v_head_dim, int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                              int64_t num_slots, float sm_scale, float logit_cap,
+                              int sliding_window_size, int dtype, int64_t rows, int splits, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
   MI355_REQUIRE(q_extend && k_extend && v_extend && o_extend && qo_indptr && kv_indptr,
                 MI355_ERR_INVALID, "extend_attention: null pointer");
   MI355_REQUIRE(k_buffer && v_buffer && kv_indices, MI355_ERR_INVALID,
@@ -1199,7 +1323,7 @@ int mi355_extend_attention(const void* q_extend, const void* k_extend, const voi
                 MI355_ERR_INVALID, "extend_attention: row strides smaller than rows");
   MI355_REQUIRE(bs <= 65535, MI355_ERR_UNSUPPORTED, "extend_attention: batch > 65535");
   if (bs == 0 || max_len_extend == 0) return MI355_OK;
-  ExtendParams p;
+  ExtendParams p = {};
   p.qo_indptr = qo_indptr;
   p.kv_indptr = kv_indptr;
   p.kv_indices = kv_indices;
@@ -1225,9 +1349,17 @@ int mi355_extend_attention(const void* q_extend, const void* k_extend, const voi
   const bool kv8 = (dtype & MI355_KV_FP8) != 0;
   p.kv8 = kv8 ? 1 : 0;
   dtype &= 0xff;
+  if (splits > 1) {
+    MI355_REQUIRE(splits <= 65535 && rows > 0 && workspace && aligned16(workspace) &&
+                      workspace_bytes >= mi355_extend_attention_workspace_bytes(rows, hq, v_head_dim, splits),
+                  MI355_ERR_INVALID, "extend_attention: workspace of %ld bytes for %ld rows x %d splits", (long)workspace_bytes, (long)rows, splits);
+    p.rows = rows;
+    p.part = (float*)workspace;
+    p.part_ml = (float2*)(p.part + (int64_t)splits * rows * hq * v_head_dim);
+  }
   MI355_DISPATCH_DTYPE(dtype, "extend_attention",
                        rc = launch_extend<T>(q_extend, k_extend, v_extend, o_extend, k_buffer,
-                                             v_buffer, p, bs, max_len_extend, kv8, (hipStream_t)stream));
+                                             v_buffer, p, bs, max_len_extend, kv8, splits > 1 ? splits : 1, (hipStream_t)stream));
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("extend_attention");
   return MI355_OK;

@@ -716,14 +716,20 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
             custom_mask = custom_mask.view(torch.uint8)
         assert custom_mask.dtype == torch.uint8
     bs = qo_indptr.numel() - 1
-    check(_lib_().mi355_extend_attention(
+    lib, dt = _lib_(), _kvdt(q_extend, k_buffer, v_buffer)
+    # few blocks of queries over many keys: workgroups share a block's keys (kv_indices holds the cached tokens' slots)
+    splits = lib.mi355_extend_attention_splits(T, bs, int(max_len_extend), kv_indices.numel(), 1 if custom_mask is not None else 0, Hq, D, Dv,
+                                               float(sm_scale), float(logit_cap), int(sliding_window_size), dt)
+    need = lib.mi355_extend_attention_workspace_bytes(T, Hq, Dv, splits) if splits > 1 else 0
+    ws = torch.empty(need, dtype=torch.uint8, device=q_extend.device) if need else None
+    check(lib.mi355_extend_attention_ws(
         q_extend.data_ptr(), k_extend.data_ptr(), v_extend.data_ptr(), o_extend.data_ptr(),
         k_buffer.data_ptr(), v_buffer.data_ptr(), qo_indptr.data_ptr(), kv_indptr.data_ptr(),
         kv_indices.data_ptr(), _p(custom_mask), _p(mask_indptr) if custom_mask is not None else None,
         1 if is_causal else 0, 1 if skip_prefix_custom_mask else 0, bs, int(max_len_extend), Hq,
         Hkv, D, Dv, q_extend.stride(0), k_extend.stride(0), v_extend.stride(0),
         k_buffer.shape[0], float(sm_scale), float(logit_cap), int(sliding_window_size),
-        _kvdt(q_extend, k_buffer, v_buffer), _stream(q_extend)), "extend_attention")
+        dt, T, splits, _p(ws), need, _stream(q_extend)), "extend_attention")
 
 
 # ---------------------------------------------------------------------------------- linear

@@ -1262,13 +1262,14 @@ extern "C" {
 // rows / 128 blocks of queries and half a block of each sequence, at most the longest's for all, times the heads.  `tiles` of 64 keys
 // a block on average, 4 or more a split.  us a launch out of cold caches, unsplit | split (32 / 8 heads): head_dim 128, fp8 cache 83 rows on 1933 cached
 // 111 | 29 (in a step), 97 x 6 on 2663 212 | 124 (2), 152 x 3 on 2411 189 | 75 (4), bf16 99 on 572 28 | 23 (2); head_dim 64, 3 x 121 on
-// 1513 50 | 35 (3), fp8 86 on 816 42 | 31 (2), 2 x 244 on 2141 97 | 49 (4).  Left whole: no cached tokens (1148 new ones, head_dim 64,
-// 37 | 42 in two; 3 x 993, 128, 51 | 80), 512 workgroups (4 x 490 on 1750 83 | 100), few tiles (400 new on 300, seven, 22 | 26).
+// 1513 50 | 35 (3), fp8 86 on 816 42 | 31 (2), 2 x 244 on 2141 97 | 49 (4).  Left whole: fewer than 512 cached tokens a sequence (1148 on
+// none, head_dim 64, 37 | 42 in two; 3 x 993, 128, 51 | 80; and a whole prompt's first rows are then a shorter one's, bit for bit), 512 workgroups (4 x 490 on 1750 83 | 100), few tiles (400 new on 300, seven, 22 | 26).
 int mi355_extend_attention_splits(int64_t rows, int64_t bs, int64_t max_len_extend, int64_t prefix_tokens, int has_mask, int hq, int head_dim,
                                   int v_head_dim, float sm_scale, float logit_cap, int sliding_window_size, int dtype) {
   const bool kv8 = (dtype & MI355_KV_FP8) != 0;
   if ((dtype & 0xff) == MI355_F32 || rows < 1 || bs < 1 || max_len_extend < 1 || hq < 1 || rows > (1 << 24) || hq > 4096 ||
-      !mfma32_serves(head_dim, v_head_dim, kv8, has_mask != 0, sliding_window_size, logit_cap, sm_scale) || head_dim > 128)
+      !mfma32_serves(head_dim, v_head_dim, kv8, has_mask != 0, sliding_window_size, logit_cap, sm_scale) || head_dim > 128 ||
+      prefix_tokens < 512 * bs)
     return 1;
   const int64_t wgs = std::min(bs * ((max_len_extend + 127) / 128), rows / 128 + bs / 2 + 1) * hq;
   const int64_t tiles = (prefix_tokens + rows / 2) / bs / 64;

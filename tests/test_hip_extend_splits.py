@@ -62,7 +62,8 @@ def test_splits_of_the_keys(ops, splits, ext, pre, d, kv8, dtype):
 
 @pytest.mark.parametrize("rows,bs,longest,prefix,hq,d,want", [
     (88, 1, 88, 1933, 32, 128, 7), (1730, 4, 490, 7000, 32, 128, 1), (591, 3, 197, 4842, 32, 64, 2), (1148, 1, 1148, 0, 32, 64, 1),
-    (400, 1, 400, 300, 32, 128, 1), (100, 1, 100, 30000, 8, 128, 8), (100, 1, 100, 30000, 8, 96, 1)])
+    (400, 1, 400, 300, 32, 128, 1), (100, 1, 100, 30000, 8, 128, 8), (100, 1, 100, 30000, 8, 96, 1),
+    (2048, 1, 2048, 1, 8, 128, 1), (4096, 1, 4096, 0, 8, 128, 1), (99, 1, 99, 511, 32, 128, 1), (99, 1, 99, 640, 32, 128, 2)])
 def test_rule(ops, rows, bs, longest, prefix, hq, d, want):
     f = ops._lib_().mi355_extend_attention_splits
     assert f(rows, bs, longest, prefix, 0, hq, d, d, 0.1, 0.0, -1, 1) == want

@@ -569,6 +569,14 @@ int mi355_fp8_scaled_mm(void* y, const uint8_t* xq, const uint8_t* wq, const flo
                         const float* w_scale, const void* bias, int64_t m, int64_t n, int64_t k,
                         void* workspace, int64_t workspace_bytes, int out_dtype, void* stream);
 
+/* The same products for few rows (65 to 256, fp8 operands with x_scale [M] and w_scale [N] to 512) and as many columns as one round of
+ * workgroups takes: smaller tiles, K walked by two groups of waves or split.  Epilogue, strides, bias and alignment as for
+ * mi355_linear_tiled; workspace as mi355_linear_few_workspace_bytes says (contents irrelevant). */
+int mi355_linear_few_supported(int64_t m, int64_t n, int64_t k, int fp8, int out_dtype, int epilogue);
+int64_t mi355_linear_few_workspace_bytes(int64_t m, int64_t n, int64_t k, int fp8);
+int mi355_linear_few(void* y, const void* x, const void* w, const float* x_scale, const float* w_scale, const void* bias, int64_t m,
+                     int64_t n, int64_t k, int64_t x_stride, int out_dtype, int epilogue, void* workspace, int64_t workspace_bytes,
+                     void* stream);
 /* mi355_fp8_scaled_mm at prefill sizes: the 256 x 256-tile kernel of mi355_linear_tiled on fp8 operands
  * (v_mfma_scale_f32_16x16x128_f8f6f4 with unit block scales: twice the 16-bit matrix rate), the
  * per-token / per-channel scales applied to the fp32 accumulator as (acc * x_scale[m]) * w_scale[n],

@@ -63,6 +63,9 @@ _SIGNATURES = {
     "mi355_linear_tiled_supported": (I, [L, L, L, I, I]),
     "mi355_linear_tiled": (I, [P, P, P, P, L, L, L, L, I, I, P]),
     "mi355_linear_tiled_ws": (I, [P, P, P, P, L, L, L, L, I, I, P, L, P]),
+    "mi355_linear_few_supported": (I, [L, L, L, I, I, I]),
+    "mi355_linear_few_workspace_bytes": (L, [L, L, L, I]),
+    "mi355_linear_few": (I, [P, P, P, P, P, P, L, L, L, L, I, I, P, L, P]),
     "mi355_tiled_tail_splits": (I, [L, L, L, I, I]),
     "mi355_tiled_tail_workspace_bytes": (L, [L, L, L, I, I]),
     "mi355_fp8_scaled_mm_tiled_ws": (I, [P, P, P, P, P, P, L, L, L, I, I, P, L, P]),

@@ -627,10 +627,223 @@ int set_tail(GemmTiledParams& p, int splits, void* workspace, int64_t workspace_
   return MI355_OK;
 }
 
+// ---- few rows -------------------------------------------------------------------------------------
+// A prompt or chunk of a few hundred rows is bound by the weights' way to the LDS: the 256 x 256 tile leaves most CUs without work.  Here a
+// workgroup has a ring of NS K tiles (128 bytes per row) in LDS, NS - 1 of them in flight, one barrier per tile, and (WM x WN waves)
+// tiles of 16 NM x 64 outputs a wave.  KS groups of waves take K tiles in turn, each with a ring of its own, and add their sums
+// through LDS: two groups are two times as many bytes in flight where there are fewer tiles than CUs.  Tiles may be split over K further,
+// with sums in `part` as they lie in the registers (gemm_few_tail_kernel adds them).  K starts at another tile in every
+// column of tiles and goes round the end (see gemm_tiled_kernel on why): a row's result depends on its own values alone.
+template <typename T, int EPI, bool FP8, int NM, int WM, int WN, int KS, int NS>
+__global__ __launch_bounds__(64 * WM * WN * KS) void gemm_few_kernel(GemmTiledParams p) {
+  extern __shared__ __attribute__((aligned(16))) char sm[];
+  using frag = typename Mfma<T>::frag;
+  constexpr int ES = FP8 ? 1 : 2, BM = 16 * NM * WM, BN = 64 * WN, NW = WM * WN;
+  constexpr int STAGE = (BM + BN) * 128, PP = (BM + BN) / 8 / NW;   // bytes of a K tile; 1-KiB pieces of it that a wave requests
+  static_assert((BM + BN) / 8 % NW == 0 && NS >= 3 && (NS - 2) * PP < 64, "whole pieces a wave, counted waits");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / NW, w = wave % NW, wm = w / WN, wn = w % WN;
+
+  // every XCD takes a run of tiles, rows fastest: the weights of a column of tiles come into one L2
+  const int splits = max(p.splits, 1), at = (blockIdx.x & 7) * (int)(gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (at >= p.mt * p.nt * splits) return;
+  const int tm = at % p.mt, tn = at / p.mt / splits, split = at / p.mt % splits;
+  const int all = (p.K * ES) >> 7, t0 = all * split / splits, T_ = all * (split + 1) / splits - t0;
+  const int its = (T_ + KS - 1) / KS, rot = tn % T_;
+  const int ncols = EPI == 1 ? (p.N >> 1) : p.N;
+
+  const char* src[PP];
+#pragma unroll
+  for (int i = 0; i < PP; ++i) {
+    const int row = (w * PP + i) * 8 + (lane >> 3), c = (lane & 7) ^ gt_swz<FP8>(row);
+    if (row < BM) {
+      const int m = min(tm * BM + row, p.M - 1);
+      src[i] = (const char*)p.x + (int64_t)m * p.ldx * ES + c * 16;
+    } else {
+      const int r = row - BM, G = tn * WN + (r >> 6), ni = (r & 63) >> 4, ii = r & 15;   // the wave's 64 columns, as tile_epilogue has them
+      int n;
+      if (EPI == 1) n = min(G * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3), ncols - 1) + (ni >> 1) * ncols;
+      else n = min(G * 64 + (ii >> 2) * 16 + ni * 4 + (ii & 3), p.N - 1);
+      src[i] = (const char*)p.w + (int64_t)n * p.K * ES + c * 16;
+    }
+    src[i] += (int64_t)t0 * 128;
+  }
+  char* const ring = sm + kg * NS * STAGE;
+  char* const dst = ring + w * PP * 1024;
+  auto request = [&](int it) {      // (a group without a tile in the last turn requests its last one again: the waits count requests)
+    int tl = min(it * KS + kg, T_ - 1) + rot;
+    tl = tl < T_ ? tl : tl - T_;
+    char* d = dst + it % NS * STAGE;
+#pragma unroll
+    for (int i = 0; i < PP; ++i) glds16(src[i] + (int64_t)tl * 128, d + i * 1024);
+  };
+  const int r16 = lane & 15, q4 = lane >> 4;
+  const int rd0 = r16 * 128 + (((FP8 ? 2 * q4 : q4) ^ gt_swz<FP8>(r16)) << 4);
+
+  f32x4 acc[NM][4];
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (i < its) request(i);
+  for (int it = 0; it < its; ++it) {
+    // this wave's part of tile `it` has landed; NS - 2 tiles behind it may be on their way
+    if (it + NS - 2 < its) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * PP) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();      // every wave's part has, and every wave is done with tile it - 1
+    __builtin_amdgcn_sched_barrier(0);
+    if (it + NS - 1 < its) request(it + NS - 1);
+    const char* stage = ring + it % NS * STAGE;
+    i32x4 af[2][NM], bf[2][4];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int ro = rd0 ^ (FP8 ? (kk << 4) : (kk << 6));
+      const char* ab = stage + wm * (NM * 2048) + ro;
+      const char* bb = stage + BM * 128 + wn * 8192 + ro;
+#pragma unroll
+      for (int ni = 0; ni < 4; ++ni) bf[kk][ni] = *reinterpret_cast<const i32x4*>(bb + ni * 2048);
+#pragma unroll
+      for (int mi = 0; mi < NM; ++mi) af[kk][mi] = *reinterpret_cast<const i32x4*>(ab + mi * 2048);
+    }
+    if (KS == 1 || it * KS + kg < T_) {
+      if constexpr (FP8) {
+#pragma unroll
+        for (int mi = 0; mi < NM; ++mi)
+#pragma unroll
+          for (int ni = 0; ni < 4; ++ni)
+            acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                __builtin_shufflevector(bf[0][ni], bf[1][ni], 0, 1, 2, 3, 4, 5, 6, 7),
+                __builtin_shufflevector(af[0][mi], af[1][mi], 0, 1, 2, 3, 4, 5, 6, 7), acc[mi][ni], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int mi = 0; mi < NM; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni)
+              acc[mi][ni] = Mfma<T>::run(__builtin_bit_cast(frag, bf[kk][ni]), __builtin_bit_cast(frag, af[kk][mi]), acc[mi][ni]);
+      }
+    }
+  }
+  if constexpr (KS > 1) {   // the groups' sums, in their order
+    constexpr int PART = NM * 4 * 1024;
+    static_assert((KS - 1) * NW * PART <= KS * NS * STAGE, "the sums lie where the rings were");
+    __syncthreads();
+    if (kg > 0) {
+#pragma unroll
+      for (int mi = 0; mi < NM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni)
+          *reinterpret_cast<f32x4*>(sm + ((kg - 1) * NW + w) * PART + (mi * 4 + ni) * 1024 + lane * 16) = acc[mi][ni];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 1; g < KS; ++g)
+#pragma unroll
+      for (int mi = 0; mi < NM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni)
+          acc[mi][ni] += *reinterpret_cast<const f32x4*>(sm + ((g - 1) * NW + w) * PART + (mi * 4 + ni) * 1024 + lane * 16);
+  }
+  const int G = tn * WN + wn, m0 = tm * BM + wm * 16 * NM;
+  if (p.splits > 1) {
+    // [split][64 columns][16 rows][4][64 lanes][4], whole 1-KiB lines
+    float* part = p.part + (((int64_t)split * p.nt * WN + G) * ((p.M + 15) >> 4) + (m0 >> 4)) * 1024 + lane * 4;
+#pragma unroll
+    for (int mi = 0; mi < NM; ++mi)
+      if (m0 + mi * 16 < p.M)
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(part + mi * 1024 + ni * 256) = acc[mi][ni];
+    return;
+  }
+  tile_epilogue<T, EPI, FP8, NM>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+}
+
+// A wave adds the splits' sums of 16 rows x 64 columns (W rows) in their order and finishes them.
+template <typename T, int EPI, bool FP8>
+__global__ __launch_bounds__(256) void gemm_few_tail_kernel(GemmTiledParams p, int groups) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4, rows16 = (p.M + 15) >> 4;
+  const int task = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int G = task / rows16, m0 = (task - G * rows16) * 16;
+  if (G >= groups) return;
+  f32x4 acc[1][4];
+#pragma unroll
+  for (int ni = 0; ni < 4; ++ni) acc[0][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* src = p.part + ((int64_t)G * rows16 + (m0 >> 4)) * 1024 + lane * 4;
+#pragma unroll 4
+  for (int k = 0; k < p.splits; ++k) {
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni) acc[0][ni] += *reinterpret_cast<const f32x4*>(src + (int64_t)k * groups * rows16 * 1024 + ni * 256);
+  }
+  tile_epilogue<T, EPI, FP8, 1>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+}
+
+template <typename T, int EPI, bool FP8, int NM, int WM, int WN, int KS, int NS>
+int launch_few_config(GemmTiledParams p, int splits, hipStream_t st) {
+  constexpr int BM = 16 * NM * WM, BN = 64 * WN, LDS = KS * NS * (BM + BN) * 128;
+  p.mt = cdiv(p.M, BM);
+  p.nt = cdiv(p.N, BN);      // (W rows: a group of 64 is 32 gate and 32 up columns with SiLU-and-mul)
+  p.splits = splits;
+  auto kern = gemm_few_kernel<T, EPI, FP8, NM, WM, WN, KS, NS>;
+  (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(cdiv((int64_t)p.mt * p.nt * splits, 8) * 8)), dim3(64 * WM * WN * KS), LDS, st, p);
+  if (splits > 1) {
+    const int groups = p.nt * WN;
+    hipLaunchKernelGGL((gemm_few_tail_kernel<T, EPI, FP8>), dim3((unsigned)cdiv((int64_t)groups * cdiv(p.M, 16), 4)), dim3(256), 0, st, p, groups);
+  }
+  MI355_CHECK_LAUNCH("mi355_linear_few");
+  return MI355_OK;
+}
+
+// The workgroups that the kernel comes in: tile, K tiles a turn, and us: fixed and for a turn, alone on a CU (c0's 0.535: 32 KB at 60 GB/s, a
+// load-to-LDS instruction of 1 KB every 35 cycles)
+struct FewShape { int bm, bn, ks; float fixed, turn; };
+constexpr FewShape FEW[] = {{128, 128, 1, 3.0f, 0.535f}, {64, 64, 2, 2.8f, 0.51f}, {128, 64, 2, 2.4f, 0.69f}};
+struct FewPlan { int shape, splits; };
+
+// The fastest of them in one round of workgroups (shape -1: none is), by what a launch was measured to take: the longer of its turns and
+// of the weights at 4.6 TB/s; splits: a second launch and their sums written and read.  From a second round on the 256 x 256 tile or a
+// library is ahead (2 x 14336 columns, K 4096, 207 rows: 448 tiles, 89 us, library 71), and from 256 rows in 16 bits, 512 in fp8.  us, library
+// (with the activation behind it) | here: bf16 3072 x 2048 70 rows 11.9 | 11.5, 207 12.9 | 11.7; 2 x 8192 x 2048 207 31 | 25; 2048 x
+// 8192 128 21 | 17, 207 28 | 21; 4096 x 4096 128 25 | 17, 207 22 | 20; 6144 x 4096 70 22 | 19, 207 26 | 27; 4096 x 14336 128 75 | 33 (256 x
+// 256 tiles 43), 2 x 14336 x 4096 70 56 | 50; fp8 6144 x 4096 330 25 | 21, 2 x 14336 x 4096 70 37 | 29, 4096 x 14336 207 34 | 27.
+FewPlan plan_few(int64_t m, int64_t n, int64_t k, bool fp8) {
+  const int64_t kt = (fp8 ? k : k * 2) >> 7;
+  FewPlan best = {-1, 1};
+  float cost = 1e30f;
+  if (m > (fp8 ? 512 : 256)) return best;
+  for (int c = 0; c < 3; ++c) {
+    const FewShape& f = FEW[c];
+    const int64_t tiles = (int64_t)cdiv(m, f.bm) * cdiv(n, f.bn);
+    for (int s = 1; s <= 8 && tiles * s <= 256; ++s) {
+      if (s > 1 && kt / s < 4 * f.ks) break;
+      const float turns = f.fixed + f.turn * cdiv(cdiv(kt, s), f.ks), stream = 2.f + 128e-6f / 4.6f * ((float)n * kt);
+      const float c1 = std::max(turns, stream) + (s > 1 ? 2.6f + 1.7e-6f * ((float)s * m * n) : 0.f);
+      if (c1 < cost) { cost = c1; best = {c, s}; }
+    }
+  }
+  return best;
+}
+
+template <typename T, int EPI, bool FP8>
+int launch_few(const GemmTiledParams& p, const FewPlan& plan, hipStream_t st) {
+  switch (plan.shape) {
+    case 0: return launch_few_config<T, EPI, FP8, 2, 4, 2, 1, 4>(p, plan.splits, st);
+    case 1: return launch_few_config<T, EPI, FP8, 2, 2, 1, 2, 4>(p, plan.splits, st);
+    default: return launch_few_config<T, EPI, FP8, 2, 4, 1, 2, 3>(p, plan.splits, st);
+  }
+}
+
 }  // namespace
 }  // namespace mi355
 
 using namespace mi355;
+
 
 extern "C" int mi355_tiled_tail_splits(int64_t m, int64_t n, int64_t k, int fp8, int epilogue) {
   if (m < 1 || n < 1 || k < 1 || m > (1 << 24) || n > (1 << 24)) return 0;
@@ -678,6 +891,51 @@ extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, cons
   if (dtype == MI355_BF16)
     return epilogue == 1 ? launch_gemm_tiled<bf16_t, 1, false>(p, st) : launch_gemm_tiled<bf16_t, 0, false>(p, st);
   return epilogue == 1 ? launch_gemm_tiled<f16_t, 1, false>(p, st) : launch_gemm_tiled<f16_t, 0, false>(p, st);
+}
+
+extern "C" int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out_dtype, int epilogue);
+
+extern "C" int mi355_linear_few_supported(int64_t m, int64_t n, int64_t k, int fp8, int out_dtype, int epilogue) {
+  if (!(fp8 ? mi355_fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, epilogue) : mi355_linear_tiled_supported(m, n, k, out_dtype, epilogue))) return 0;
+  return plan_few(m, n, k, fp8 != 0).shape >= 0 ? 1 : 0;
+}
+
+extern "C" int64_t mi355_linear_few_workspace_bytes(int64_t m, int64_t n, int64_t k, int fp8) {
+  const FewPlan plan = plan_few(m, n, k, fp8 != 0);
+  if (plan.shape < 0 || plan.splits == 1) return 0;
+  return (int64_t)plan.splits * cdiv(n, FEW[plan.shape].bn) * (FEW[plan.shape].bn / 64) * cdiv(m, 16) * 4096;
+}
+
+extern "C" int mi355_linear_few(void* y, const void* x, const void* w, const float* x_scale, const float* w_scale, const void* bias, int64_t m,
+                                int64_t n, int64_t k, int64_t x_stride, int out_dtype, int epilogue, void* workspace, int64_t workspace_bytes,
+                                void* stream) {
+  const bool fp8 = x_scale != nullptr;
+  MI355_REQUIRE(y && x && w && (!fp8 || w_scale), MI355_ERR_INVALID, "mi355_linear_few: null pointer");
+  MI355_REQUIRE(mi355_linear_few_supported(m, n, k, fp8, out_dtype, epilogue), MI355_ERR_UNSUPPORTED,
+                "mi355_linear_few: needs a 16-bit result, K %% 64 == 0, K >= 128 (fp8: %% 128, 256), N %% 16 == 0 and one round of workgroups (m=%ld n=%ld "
+                "k=%ld dtype=%d epilogue=%d)", (long)m, (long)n, (long)k, out_dtype, epilogue);
+  MI355_REQUIRE(fp8 ? x_stride == k : (x_stride >= k && x_stride % 8 == 0), MI355_ERR_INVALID, "mi355_linear_few: bad x_stride");
+  MI355_REQUIRE(aligned16(x) && aligned16(w) && aligned16(y) && (bias == nullptr || aligned16(bias)), MI355_ERR_INVALID,
+                "mi355_linear_few: pointers must be 16-byte aligned");
+  MI355_REQUIRE(epilogue == 0 || bias == nullptr, MI355_ERR_UNSUPPORTED, "mi355_linear_few: no bias with the SiLU-and-mul epilogue");
+  const int64_t need = mi355_linear_few_workspace_bytes(m, n, k, fp8);
+  MI355_REQUIRE(need == 0 || (workspace && aligned16(workspace) && workspace_bytes >= need), MI355_ERR_INVALID,
+                "mi355_linear_few: workspace of %ld bytes, %ld needed", (long)workspace_bytes, (long)need);
+  GemmTiledParams p;
+  p.x = x; p.w = w; p.bias = bias; p.y = y;
+  p.x_scale = x_scale; p.w_scale = w_scale;
+  p.M = (int)m; p.N = (int)n; p.K = (int)k;
+  p.ldx = x_stride;
+  fill_tiles(p, m, n, epilogue);
+  p.part = (float*)workspace;
+  const FewPlan plan = plan_few(m, n, k, fp8);
+  hipStream_t st = (hipStream_t)stream;
+  if (fp8) {
+    if (out_dtype == MI355_BF16) return epilogue == 1 ? launch_few<bf16_t, 1, true>(p, plan, st) : launch_few<bf16_t, 0, true>(p, plan, st);
+    return epilogue == 1 ? launch_few<f16_t, 1, true>(p, plan, st) : launch_few<f16_t, 0, true>(p, plan, st);
+  }
+  if (out_dtype == MI355_BF16) return epilogue == 1 ? launch_few<bf16_t, 1, false>(p, plan, st) : launch_few<bf16_t, 0, false>(p, plan, st);
+  return epilogue == 1 ? launch_few<f16_t, 1, false>(p, plan, st) : launch_few<f16_t, 0, false>(p, plan, st);
 }
 
 namespace mi355 {

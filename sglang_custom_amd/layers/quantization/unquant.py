@@ -4,9 +4,10 @@
 Decode-sized inputs (M <= 64 rows) and every fp32 input go to the hand-written kernels behind
 mi355_linear (weight-streaming MFMA / exact-fp32 tiled).  Large-M bf16/f16 GEMMs (prefill) run on the
 hand-written 256 x 256-tile matrix-core kernel behind mi355_linear_tiled, which can apply SiLU-and-mul in
-its epilogue.  PREFILL_GEMM (env MI355_PREFILL_GEMM) picks: "tiled" (default) = that kernel for every
-shape it serves (at least TILED_MIN_TILES output tiles; smaller problems, but for long reductions, and shapes it does not take
-fall back to the library GEMM, torch.nn.functional.linear -> hipBLASLt); "auto" = the faster of the two
+its epilogue, and few rows (to 256) on the smaller tiles behind mi355_linear_few, whose call also costs the host less than the
+library's (8 us for 20).  PREFILL_GEMM (env MI355_PREFILL_GEMM) picks: "tiled" (default) = that kernel for every
+shape it serves (at least TILED_MIN_TILES output tiles; smaller problems, but for few rows and for long reductions, and shapes it
+does not take fall back to the library GEMM, torch.nn.functional.linear -> hipBLASLt); "auto" = the faster of the two
 per projection as measured on MI355X (the hand-written kernel for gate_up with the fused activation,
 1.02x the library pair; the library for the plain projections, where it is 4-6 % faster); "library" =
 hipBLASLt everywhere."""
@@ -91,8 +92,12 @@ def gate_up_silu_mul(layer, act_fn, x: torch.Tensor) -> torch.Tensor:
         y = get_ops().linear_packed_silu_mul(x2, wp, layer.weight.shape[0])
         return y.view(*x.shape[:-1], y.shape[-1])
     w = layer.weight
-    if (x2.is_cuda and isinstance(layer.quant_method, UnquantizedLinearMethod) and getattr(layer, "bias", None) is None
-            and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
+    plain = x2.is_cuda and isinstance(layer.quant_method, UnquantizedLinearMethod) and getattr(layer, "bias", None) is None
+    if plain and x2.shape[0] > SKINNY_MAX_M and PREFILL_GEMM != "library":
+        y = get_ops().linear_few(x2, w, None, silu_mul=True)
+        if y is not None:
+            return y.view(*x.shape[:-1], y.shape[-1])
+    if (plain and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
             and _use_tiled(x2.shape[0], w.shape[0], w.shape[0], w.shape[1], x2.dtype, True)):
         y = get_ops().linear_tiled(x2, w, None, silu_mul=True, split_tail=True)
         return y.view(*x.shape[:-1], y.shape[-1])
@@ -174,6 +179,10 @@ def decode_linear_deferred(layer, x, needs_all_reduce: bool = True):
 
 def prefill_linear(x2: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """16-bit rows [M, K] (M > SKINNY_MAX_M) against a plain weight [N, K]."""
+    if x2.is_cuda and PREFILL_GEMM == "tiled":
+        y = get_ops().linear_few(x2, weight, bias)
+        if y is not None:
+            return y
     if (x2.stride(1) == 1 and x2.stride(0) % 8 == 0 and weight.is_contiguous()
             and _use_tiled(x2.shape[0], weight.shape[0], weight.shape[0], weight.shape[1], x2.dtype, False)):
         return get_ops().linear_tiled(x2, weight, bias, split_tail=True)

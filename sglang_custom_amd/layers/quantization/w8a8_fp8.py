@@ -32,7 +32,7 @@ SKINNY_MAX_M = 64
 # Large-M fp8 GEMMs: "auto" (default) and "tiled" = the hand-written 256 x 256-tile kernel
 # (mi355_fp8_scaled_mm_tiled) for every shape it serves -- on MI355X it is 1.00-1.10x torch._scaled_mm
 # (hipBLASLt) on the plain projections and 1.23x on gate_up, whose scales and SiLU-and-mul run in its
-# epilogue; "library" = torch._scaled_mm everywhere.
+# epilogue -- and few rows (to 512) on the smaller tiles of mi355_linear_few; "library" = torch._scaled_mm everywhere.
 PREFILL_GEMM = os.environ.get("MI355_PREFILL_FP8_GEMM", "auto")
 # Below this many 256 x 256 output tiles too many CUs idle (us, library | tiled: 4096 x 4096 with 1600 rows, 112 tiles, 34 | 42, 6144 x 4096
 # with 1100, 120, 36 | 43; 4096 x 4096 with 2300 rows, 144, 57 | 44, 6144 x 4096 with 1600, 168, 57 | 45; 4096 x 14336 with 2300, 144,
@@ -83,12 +83,18 @@ def gate_up_silu_mul_prefill(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
     x2 = x.xq if quantised else x.view(-1, x.shape[-1])
     w = layer.weight
     if (PREFILL_GEMM == "library" or not x2.is_cuda or x2.shape[0] <= SKINNY_MAX_M
-            or getattr(layer, "bias", None) is not None or w.dtype != FP8_DTYPE
-            or not _tiled_ok(x2.shape[0], w.shape[0], w.shape[1], x.dtype, True)):
+            or getattr(layer, "bias", None) is not None or w.dtype != FP8_DTYPE):
         return None
     ops = get_ops()
+    tiled = _tiled_ok(x2.shape[0], w.shape[0], w.shape[1], x.dtype, True)
+    if not tiled and not ops.linear_few_supported(x2.shape[0], w.shape[0], w.shape[1], x.dtype, True, fp8=True):
+        return None
     xq, xs = (x.xq, x.x_scale) if quantised else ops.per_token_quant_fp8(x2)
-    y = ops.fp8_scaled_mm_tiled(xq, w, xs, layer.weight_scale.view(-1), x.dtype, None, silu_mul=True, split_tail=True)
+    y = ops.linear_few(xq, w, None, True, xs, layer.weight_scale.view(-1), x.dtype)
+    if y is None and not tiled:
+        return None
+    if y is None:
+        y = ops.fp8_scaled_mm_tiled(xq, w, xs, layer.weight_scale.view(-1), x.dtype, None, silu_mul=True, split_tail=True)
     return y.view(*x.shape[:-1], y.shape[-1])
 
 
@@ -153,7 +159,9 @@ class W8A8Fp8LinearMethod:
         ops = get_ops()
         m, k = xq.shape
         y = None
-        if PREFILL_GEMM != "library" and m > SKINNY_MAX_M and xq.is_cuda and _tiled_ok(m, layer.weight.shape[0], k, out_dtype, False):
+        if PREFILL_GEMM != "library" and m > SKINNY_MAX_M and xq.is_cuda:
+            y = ops.linear_few(xq, layer.weight, bias, False, xs, layer.weight_scale.view(-1), out_dtype)
+        if y is None and PREFILL_GEMM != "library" and m > SKINNY_MAX_M and xq.is_cuda and _tiled_ok(m, layer.weight.shape[0], k, out_dtype, False):
             y = ops.fp8_scaled_mm_tiled(xq, layer.weight, xs, layer.weight_scale.view(-1), out_dtype, bias, split_tail=True)
         if y is None and m > SKINNY_MAX_M and xq.is_cuda and k % 16 == 0 and layer.weight.shape[0] % 16 == 0:
             y = _library_scaled_mm(xq, layer.weight, xs, layer.weight_scale, out_dtype, bias)

@@ -812,6 +812,42 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return y
 
 
+def linear_few_supported(m: int, n: int, k: int, out_dtype: torch.dtype, silu_mul: bool = False, fp8: bool = False) -> bool:
+    """Whether linear_few serves the shape."""
+    return out_dtype in (torch.bfloat16, torch.float16) and bool(
+        _lib_().mi355_linear_few_supported(m, n, k, 1 if fp8 else 0, _DT[out_dtype], 1 if silu_mul else 0))
+
+
+def linear_few(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, silu_mul: bool = False,
+               x_scale: Optional[torch.Tensor] = None, w_scale: Optional[torch.Tensor] = None,
+               out_dtype: Optional[torch.dtype] = None) -> Optional[torch.Tensor]:
+    """linear_tiled (with x_scale / w_scale fp8_scaled_mm_tiled, out_dtype naming the result) for a prompt of few rows, on tiles that
+    fill the chip with them; None where another kernel is ahead (more rows, more columns than one round of workgroups) or the operands are
+    none that it takes (16-byte rows)."""
+    m, k = x.shape
+    n = weight.shape[0]
+    fp8 = x_scale is not None
+    out_dtype = out_dtype or x.dtype
+    if (not 0 < m <= 512 or not x.is_cuda or out_dtype not in (torch.bfloat16, torch.float16) or (x.stride(0) != k if fp8 else x.stride(0) % 8 != 0)
+            or x.stride(1) != 1 or not weight.is_contiguous() or weight.dtype != x.dtype or weight.shape[1] != k
+            or (bias is not None and (silu_mul or bias.dtype != out_dtype or not bias.is_contiguous() or bias.data_ptr() % 16 != 0))
+            or x.data_ptr() % 16 != 0 or weight.data_ptr() % 16 != 0):
+        return None
+    lib, dt, epi = _lib_(), _DT[out_dtype], 1 if silu_mul else 0
+    if not lib.mi355_linear_few_supported(m, n, k, 1 if fp8 else 0, dt, epi):
+        return None
+    _gpu(weight, bias, x_scale, w_scale)
+    if fp8:
+        assert x.dtype == torch.float8_e4m3fn and x_scale.dtype == w_scale.dtype == torch.float32
+        assert x_scale.is_contiguous() and w_scale.is_contiguous() and x_scale.numel() == m and w_scale.numel() == n
+    y = torch.empty((m, n // 2 if silu_mul else n), dtype=out_dtype, device=x.device)
+    need = lib.mi355_linear_few_workspace_bytes(m, n, k, 1 if fp8 else 0)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib.mi355_linear_few(y.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(x_scale), _p(w_scale), _p(bias), m, n, k, x.stride(0), dt, epi,
+                               _p(ws), need, _stream(x)), "linear_few")
+    return y
+
+
 def qkv_proj_rope_tiled_supported(m: int, k: int, hq: int, hkv: int, head_dim: int, rotary_dim: int,
                                   is_neox: bool, dtype: torch.dtype, fp8: bool = False) -> bool:
     """Whether qkv_proj_rope_tiled serves the layer (head_dim = rotary_dim = 128, neox, 16-bit)."""

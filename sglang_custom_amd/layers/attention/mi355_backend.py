@@ -46,6 +46,7 @@ class ForwardMetadata:
     kv_indptr: Optional[torch.Tensor] = None
     kv_indices: Optional[torch.Tensor] = None
     max_extend_len: int = 0
+    longest: Optional[int] = None            # captured steps of walks_positions backends: the longest sequence that the graph must serve
     window_kv_indptr: Optional[torch.Tensor] = None
     window_kv_indices: Optional[torch.Tensor] = None
     window_num_kv_splits: int = 1
@@ -67,6 +68,8 @@ class Mi355AttnBackend(AttentionBackend):
         self.is_latent_window = hasattr(model_runner.token_to_kv_pool, "widths")
         # per-layer key / value shapes (LayeredMHATokenToKVPool): served by forward_sigmoid alone, with the same metadata
         self.is_layered = hasattr(model_runner.token_to_kv_pool, "layer_shapes")
+        # both read a step's lengths from its positions and no other metadata
+        self.walks_positions = self.is_latent_window or self.is_layered
         self.kv_fp8 = getattr(model_runner.token_to_kv_pool, "dtype", None) == torch.float8_e4m3fn
         # captured steps of these shapes are planned with splits for any length: their decode kernel merges in its own launch and passes
         # over empty splits
@@ -161,7 +164,7 @@ class Mi355AttnBackend(AttentionBackend):
     def init_forward_metadata(self, forward_batch):
         ops = get_ops()
         bs = forward_batch.batch_size
-        if self.is_latent_window or self.is_layered:
+        if self.walks_positions:
             self.forward_metadata = ForwardMetadata()
             self.forward_metadata.latent_blocks = {}
             return
@@ -207,7 +210,7 @@ class Mi355AttnBackend(AttentionBackend):
 
     # ---- HIP-graph capture / replay (static shapes; nothing to refresh per replay) ----
     def init_cuda_graph_state(self, max_bs: int, max_num_tokens: int):
-        if self.is_layered:
+        if self.walks_positions:
             return          # these kernels plan their own key ranges and bring their own scratch
         self._scratch(max_bs, MAX_KV_SPLITS)
         if self.sliding_window_size:
@@ -218,8 +221,8 @@ class Mi355AttnBackend(AttentionBackend):
     def init_forward_metadata_capture_cuda_graph(self, bs, num_tokens, req_pool_indices, seq_lens,
                                                  encoder_lens, forward_mode, spec_info):
         assert forward_mode.is_decode_or_idle(), "only decode is captured"
-        if self.is_layered:
-            self.forward_metadata = ForwardMetadata()
+        if self.walks_positions:
+            self.forward_metadata = ForwardMetadata(longest=self.max_context_len)
             self.forward_metadata.latent_blocks = {}
             return
         # one graph serves every step: split for the longest context the model can reach
@@ -240,7 +243,7 @@ class Mi355AttnBackend(AttentionBackend):
 
     def init_forward_metadata_replay_cuda_graph(self, bs, req_pool_indices, seq_lens, seq_lens_sum,
                                                 encoder_lens, forward_mode, spec_info, seq_lens_cpu):
-        if self.is_layered:
+        if self.walks_positions:
             return
         # the captured kernels read req_to_token / seq_lens from the static buffers directly; only the
         # window gather of sliding-window models is refreshed (into the buffers the graph captured)
@@ -332,6 +335,15 @@ class Mi355AttnBackend(AttentionBackend):
             cache[bq] = host.contiguous().to(self.device, non_blocking=True)
         return cache[bq]
 
+    def _longest(self, forward_batch) -> Optional[int]:
+        """The longest sequence of a decode step as far as the host knows it, in a captured step the most that the model can reach (key
+        ranges that a shorter batch leaves empty cost their launch's fixed part alone); None in an extend."""
+        if not forward_batch.forward_mode.is_decode():
+            return None
+        if forward_batch.seq_lens_cpu is not None:
+            return int(forward_batch.seq_lens_cpu.max())
+        return self.forward_metadata.longest
+
     def forward_latent_window(self, qa, qr, gate, layer, forward_batch, out, cache_layer=None):
         """qa [T, H, rank] absorbed queries, qr [T, H, rope] unrotated, gate [T, H] logits or None -> out [T, H, rank], over
         the rows of cache_layer (the layer's own by default), its last layer.window tokens or (0) every earlier one.
@@ -342,11 +354,10 @@ class Mi355AttnBackend(AttentionBackend):
         if bq <= 0:
             raise NotImplementedError(f"latent window attention: rank {layer.kv_rank} + rope {layer.rope_dim} is not served")
         cache = forward_batch.token_to_kv_pool.get_key_buffer(layer.layer_id if cache_layer is None else cache_layer)
-        splits = 1
-        if forward_batch.forward_mode.is_decode() and forward_batch.seq_lens_cpu is not None:
+        splits, longest = 1, self._longest(forward_batch)
+        if longest is not None:
             # a decode step has few workgroups: long windows are cut into key ranges that a second launch merges
-            splits = ops.latent_window_attention_splits(qa.shape[0], layer.tp_q_head_num, layer.kv_rank, layer.window,
-                                                        int(forward_batch.seq_lens_cpu.max()) - 1, qa.dtype)
+            splits = ops.latent_window_attention_splits(qa.shape[0], layer.tp_q_head_num, layer.kv_rank, layer.window, longest - 1, qa.dtype)
         return ops.latent_window_attention(
             qa, qr, cache, out, forward_batch.req_to_token_pool.req_to_token, forward_batch.req_pool_indices,
             forward_batch.positions, layer.sink.data if layer.sink is not None else None, layer.inv_freq, layer.rot_dims, layer.window,
@@ -431,10 +442,9 @@ class Mi355AttnBackend(AttentionBackend):
         bq = ops.window_attention_block_tokens(layer.tp_q_head_num, layer.tp_k_head_num, layer.qk_head_dim, layer.v_head_dim, q.dtype)
         if q.stride(0) % 8 or q.stride(1) % 8:
             q = q.contiguous()      # a column block of a wider row that does not start every head on 16 bytes
-        splits = 1
-        if forward_batch.forward_mode.is_decode() and forward_batch.seq_lens_cpu is not None:
-            splits = ops.window_attention_splits(q.shape[0], layer.tp_q_head_num, layer.tp_k_head_num,
-                                                 int(forward_batch.seq_lens_cpu.max()), layer.window, q.dtype,
+        splits, longest = 1, self._longest(forward_batch)
+        if longest is not None:
+            splits = ops.window_attention_splits(q.shape[0], layer.tp_q_head_num, layer.tp_k_head_num, longest, layer.window, q.dtype,
                                                  **({"pool": layer.pool} if extra.get("pool") else {}))
         return ops.window_attention(
             q, k_cache, v_cache, out, forward_batch.req_to_token_pool.req_to_token, forward_batch.req_pool_indices,

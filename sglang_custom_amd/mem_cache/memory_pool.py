@@ -22,7 +22,11 @@ class ReqToTokenPool:
         self.size = size
         self.max_context_len = max_context_len
         self.device = device
-        self.req_to_token = torch.zeros((size, max_context_len), dtype=torch.int32, device=device)
+        # One more row than requests lies behind the table, for kernels that are given its number: the padded rows of a captured step.  It is
+        # never handed out, so its tokens stay at slot 0 (the sink row of the caches) and its state at slot 0 of the state pool.
+        self.table = torch.zeros((size + 1, max_context_len), dtype=torch.int32, device=device)
+        self.req_to_token = self.table[:size]
+        self.pad_row = size
         self.free_slots = list(range(size))
         # models whose sequences carry state from step to step: the pool of state rows (SequenceStatePool) and the
         # device map row of this table -> state slot, written when a request's row is (re)allocated
@@ -31,7 +35,7 @@ class ReqToTokenPool:
 
     def attach_state_pool(self, state_pool: "SequenceStatePool") -> None:
         self.state_pool = state_pool
-        self.req_to_state = torch.zeros(self.size, dtype=torch.int32, device=self.device)
+        self.req_to_state = torch.zeros(self.size + 1, dtype=torch.int32, device=self.device)[: self.size]      # (pad_row's: slot 0)
 
     def take_state(self, reqs) -> None:
         """Give every request of a new prefill batch that has none yet a state slot, and point the requests' rows of
@@ -210,7 +214,7 @@ class SequenceStatePool:
     [slots, taps - 1, channels], row taps - 2 the most recent; the keys are the model's own).
     A request holds one slot from its first prefill portion until it finishes or is retracted; what a freed slot
     holds is never read again, because a sequence's first token (position 0) takes no state.  Slot 0 is never
-    handed out."""
+    handed out: padded rows of a captured step write it."""
 
     def __init__(self, size: int, layer_num: int, hidden: int, device: str, matrices: Optional[dict] = None,
                  convs: Optional[dict] = None, vectors: Optional[dict] = None):

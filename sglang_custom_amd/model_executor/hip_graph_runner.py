@@ -2,7 +2,7 @@
 static input buffers -- the role of the reference's CudaGraphRunner
 (python/sglang/srt/model_executor/cuda_graph_runner.py: can_run :342, capture_one_batch_size
 :456, replay_prepare :626-700, replay :702-730).  ~330 kernel launches per step collapse into
-one graph launch; padded rows use seq_len fill value 1 and KV slot 0 (the sink row)."""
+one graph launch; padded rows use seq_len fill value 1, KV slot 0 (the sink row) and the request table's row for padding."""
 import bisect
 import contextlib
 import gc
@@ -48,7 +48,8 @@ class HipGraphRunner:
         self.seq_len_fill_value = model_runner.attn_backend.get_cuda_graph_seq_len_fill_value()
         # static inputs (cuda_graph_runner.py:270-290)
         self.input_ids = torch.zeros(self.max_bs, dtype=torch.int64, device=dev)
-        self.req_pool_indices = torch.zeros(self.max_bs, dtype=torch.int64, device=dev)
+        self.pad_row = model_runner.req_to_token_pool.pad_row
+        self.req_pool_indices = torch.full((self.max_bs,), self.pad_row, dtype=torch.int64, device=dev)
         self.seq_lens = torch.full((self.max_bs,), self.seq_len_fill_value, dtype=torch.int64, device=dev)
         self.out_cache_loc = torch.zeros(self.max_bs, dtype=torch.int64, device=dev)
         self.positions = torch.zeros(self.max_bs, dtype=torch.int64, device=dev)
@@ -64,12 +65,14 @@ class HipGraphRunner:
 
     def _static_batch(self, bs: int) -> ForwardBatch:
         mr = self.model_runner
-        return ForwardBatch(
+        fb = ForwardBatch(
             forward_mode=ForwardMode.DECODE, batch_size=bs, input_ids=self.input_ids[:bs],
             req_pool_indices=self.req_pool_indices[:bs], seq_lens=self.seq_lens[:bs],
             out_cache_loc=self.out_cache_loc[:bs], seq_lens_sum=bs * self.seq_len_fill_value,
             positions=self.positions[:bs], req_to_token_pool=mr.req_to_token_pool,
             token_to_kv_pool=mr.token_to_kv_pool, attn_backend=mr.attn_backend)
+        fb._init_seq_state(mr)
+        return fb
 
     def capture(self):
         from ..distributed.parallel_state import check_collectives, tp_barrier
@@ -109,7 +112,9 @@ class HipGraphRunner:
         if bs != raw_bs:
             self.seq_lens.fill_(self.seq_len_fill_value)
             self.out_cache_loc.zero_()
-            self.req_pool_indices.zero_()
+            self.req_pool_indices.fill_(self.pad_row)
+            if getattr(self.model_runner.attn_backend, "walks_positions", False):
+                self.positions.zero_()
         dsts = [self.input_ids, self.req_pool_indices, self.seq_lens, self.out_cache_loc, self.positions]
         srcs = [forward_batch.input_ids, forward_batch.req_pool_indices, forward_batch.seq_lens,
                 forward_batch.out_cache_loc, forward_batch.positions]

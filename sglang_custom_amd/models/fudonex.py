@@ -222,7 +222,7 @@ class FudonexModel(nn.Module):
 
 
 class FudonexForCausalLM(nn.Module):
-    supports_hip_graph = False    # a captured decode step pads the batch with row 0 of the request table, whose state slot it would overwrite
+    supports_hip_graph = True     # padded rows of a captured step write the state pool's slot 0 and the caches' sink slot
 
     def __init__(self, config, dtype=torch.bfloat16, device="cuda", quant_method_factory=None):
         super().__init__()

@@ -197,8 +197,6 @@ class SilatarModel(nn.Module):
 
 
 class SilatarForCausalLM(nn.Module):
-    supports_hip_graph = False    # a captured decode step pads the batch with row 0 of the request table, whose state slot it would overwrite
-
     def __init__(self, config, dtype=torch.bfloat16, device="cuda", quant_method_factory=None):
         super().__init__()
         if quant_method_factory is not None:
@@ -208,6 +206,7 @@ class SilatarForCausalLM(nn.Module):
         self.config = config
         self.dtype = dtype
         self.needs_sequence_state = bool(config.needs_sequence_state)
+        self.supports_hip_graph = not self.needs_sequence_state     # (matrix memories have not been run in a captured step)
         self.model = SilatarModel(config, dtype, device)
         self.lm_head = ParallelLMHead(config.vocab_size, config.hidden_size, dtype, device)
         self.logits_processor = LogitsProcessor(config)

@@ -1,0 +1,49 @@
+"""Captured decode steps of the families that keep state per sequence (Fudonex) or latent rows (Silatar without matrix memories), against
+the whole-sequence oracles: eager prompts between the replays, padded batches, requests that end and begin again in their rows, and a
+request at row 0 of the request table that waits while padded batches of others run (its state is its own)."""
+import pytest
+
+import fudonex_util as fu
+import silatar_util as su
+from oracle import fudonex_ref, silatar_ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(autouse=True)
+def _product_ops():
+    from sglang_custom_amd import ops_backend
+    from sglang_custom_amd.distributed import parallel_state
+
+    ops_backend.set_ops_backend(None)      # the HIP library (get_ops() loads it and raises if it is missing)
+    parallel_state.init_distributed_environment(1, 0)
+    yield
+
+
+# the families' own engine tests take the same limits
+@pytest.mark.parametrize("family,dtype,tol", [("fudonex", "float32", 3e-5), ("fudonex", "bfloat16", 6e-2), ("silatar", "float32", 3e-5),
+                                              ("silatar", "bfloat16", 6e-2)])
+def test_replays_against_the_oracle(family, dtype, tol):
+    if family == "fudonex":
+        u, ref, cfg = fu, fudonex_ref, fu.make_config()
+    else:
+        u, ref, cfg = su, silatar_ref, su.make_config(layers=[(su.latent(), su.dense(96)), (su.latent(kv_rank=24), su.dense(64)), (su.latent(), None)], width=96,
+                                                      loop=(0, 2, 2))
+    w = u.make_weights(cfg, seed=4)
+    prompts = u.random_prompts(cfg, [40, 25, 18, 22, 9], seed=6)
+    want = {k: ref.forward(cfg, w, p) for k, p in prompts.items()}
+    mr = u.build_runner(cfg, w, dtype=dtype, device=DEV, max_total_tokens=160, max_running_requests=5, cuda_graph_bs=[1, 4])
+    assert mr.graph_runner is not None
+    sched = [[("r0", 20), ("r1", 5)], [("r2", 3), ("r3", 7)]]                  # r0 holds row 0
+    sched += [[("r1", 1), ("r2", 1), ("r3", 1)]] * 6                           # three in a graph of four while r0 waits
+    sched += [[("r0", 1)]] * 5 + [[("r0", 1), ("r1", 1)]] * 4                  # alone, and two of four
+    sched += [[("r0", 4), ("r4", 2)]]                                          # a portion between the replays
+    sched += [[("r0", 1), ("r1", 1), ("r2", 1), ("r3", 1)]] * 7                # whole
+    sched += [[("r1", 1), ("r2", 1), ("r4", 1)], [("r1", 2), ("r2", 1), ("r3", 2), ("r4", 6)]]
+    assert {k: sum(n for s in sched for r, n in s if r == k) for k in prompts} == {k: len(p) for k, p in prompts.items()}
+    for _ in range(2):       # the second time over used slots and rows
+        u.replay_and_compare(mr, cfg, w, prompts, sched, tol, want_all=want)
+        assert mr.req_to_token_pool.available_size() == mr.req_to_token_pool.size
+        assert mr.token_to_kv_pool_allocator.available_size() == mr.max_total_num_tokens
+        assert not mr.req_to_token_pool.table[mr.req_to_token_pool.pad_row].any()

@@ -515,6 +515,13 @@ int mi355_fused_add_rmsnorm_partials(void* x, void* residual, const void* weight
                                      int nsplit, int64_t rows, int64_t hidden, float eps, int dtype,
                                      void* stream);
 
+/* mi355_fused_add_rmsnorm_partials (at most 8 splits) and the packed projection behind it in one launch, for 1 or 2 rows: x = rmsnorm(sum of part [nsplit, M, K]
+ * + residual) with that call's rounding points, residual_out [M, K] = the new residual (NOT residual's memory), and either (y)
+ * y [M, N / 2] = SiluAndMul(x @ W^T) over a gate / up packed weight, or (out_part) the projection's partials [splits, M, N].
+ * mi355_norm_linear_packed_splits: how many splits that are; 0: the shape is not served. */
+int mi355_norm_linear_packed_splits(int64_t m, int64_t n, int64_t k, int silu_mul);
+int mi355_norm_linear_packed(void* y, float* out_part, void* residual_out, const float* part, int nsplit, const void* residual,
+                             const void* norm_weight, float eps, const void* w_packed, int64_t m, int64_t n, int64_t k, int dtype, void* stream);
 /* gate_up projection with SiLU-and-mul fused into the epilogue: y[m, j] = T(silu(g_j)) * u_j with
  * g = x W_gate^T, u = x W_up^T each rounded to T first (the rounding points of the unfused ops).
  * w_packed = mi355_pack_weight of the [2d, K] matrix whose 16-row tile t holds gate rows

@@ -85,6 +85,8 @@ _SIGNATURES = {
     "mi355_fp8_packed_partials": (I, [P, P, P, L, L, L, P]),
     "mi355_rmsnorm_ex": (I, [P, P, P, P, P, I, P, P, P, P, L, L, F, I, P]),
     "mi355_silu_and_mul_quant_fp8": (I, [P, P, P, L, L, L, I, P]),
+    "mi355_norm_linear_packed_splits": (I, [L, L, L, I]),
+    "mi355_norm_linear_packed": (I, [P, P, P, P, I, P, P, F, P, L, L, L, I, P]),
     "mi355_linear_packed_splits": (I, [L, L, L]),
     "mi355_linear_packed_partials": (I, [P, P, P, L, L, L, L, I, P]),
     "mi355_ar_region_bytes": (L, [L]),

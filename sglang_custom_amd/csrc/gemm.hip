@@ -713,6 +713,173 @@ static bool skinny_ok(int64_t m, int64_t n, int64_t k, int64_t x_stride, const v
 
 static bool use_ring(int64_t k) { return k % SK_BK == 0 && g_gemm_variant == 0; }
 
+// ---- a norm and the projection behind it, one or two rows ----------------------------------------
+// y = rmsnorm(sum of the partials + residual) @ W^T: every workgroup forms the normalised rows by itself, in LDS, while its first weight
+// requests are under way (4 or 8 splits of 8 or 16 KB a row, from L2), and then streams its weights without a barrier.  The first workgroup alone
+// writes the new residual, to memory that the others do not read.  A norm of its own is a launch between two projections.  us, norm and
+// projection -> here (the projection alone), bf16, rotating weights: 1 row, K 2048, 2 x 8192 columns with SiLU 16.0 -> 13.3 (13.3),
+// 3072 7.4 -> 4.95 (4.4), 2 rows 15.3 -> 12.8 and 7.6 -> 5.5; 1 row, K 4096, 2 x 14336 41.6 -> 38.7 (38.4), 6144 14.5 -> 11.5 (10.8).
+// Its requests must not wait for the weights behind them, so all splits go out at once and in straight code (with a loop over them
+// 2 x 14336 columns took 45 us); more rows than two are more bytes from L2 in every workgroup than the launch costs (3 rows, K 2048: 15.3 -> 21).
+// Same rounding points as rmsnorm_vec_kernel: the partials' sum to T, the sum with the residual unrounded into the norm and
+// rounded into the residual; the squares are added in another order.
+// CH: groups of eight elements that a lane has of its row (a row is `waves / rows` waves'), U: splits at most.  ACT: weights packed with gate and up
+// rows interleaved, SiLU-and-mul on the result, else this split's fp32 partials for the consumer.
+struct NormLinearParams {
+  const float* part;      // [nsplit][M][K]
+  const void* residual;   // [M][K]
+  void* residual_out;
+  const void* norm_w;
+  const void* w;          // packed
+  void* y;                // ACT: [M][N / 2]
+  float* out_part;        // [splits][M][N]
+  int nsplit, M, N, K, k_per_split;
+  float eps;
+};
+constexpr int NL_ROWS = 2, NL_SPLITS = 8, NL_PAD = 32;   // LDS rows lie 64 bytes further than their length: two rows' fragments in other banks
+template <typename T, bool ACT, int CH, int U>
+__global__ __launch_bounds__(512) void norm_linear_kernel(NormLinearParams p) {
+  using frag = typename Mfma<T>::frag;
+  constexpr int S = 8;     // fragment steps of a 256-deep chunk
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  T* const xs = reinterpret_cast<T*>(smem_raw);       // [M][K + NL_PAD]
+  __shared__ float sums[8];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int r16 = lane & 15, q = lane >> 4, row_len = p.K + NL_PAD;
+  const int tile = min((int)blockIdx.x * waves + wave, ((p.N + 63) >> 6) * 4 - 1);
+  const int ks = blockIdx.y * p.k_per_split, nchunks = (min(p.K, ks + p.k_per_split) - ks) / 256;
+  const T* const wrow = (const T*)p.w + (((int64_t)(tile >> 2) * (p.K / 32) * 4 + (tile & 3)) * 64 + lane) * 8 + (int64_t)ks * 64;
+  frag w0[S], w1[S], w2[S];
+  auto load_w = [&](frag (&dst)[S], int chunk) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      dst[s] = __builtin_nontemporal_load(reinterpret_cast<const frag*>(wrow + (int64_t)(chunk * 256 + s * 32) * 64));
+  };
+
+  // ---- the rows: requests first, so that nothing waits for the weights behind them ----
+  const int per = waves / p.M, m = min(wave / per, p.M - 1);       // waves of a row; a wave without one repeats the last row's end
+  const int at = (wave - m * per) * 64 + lane, nvec = p.K >> 3;
+  const bool mine = wave < per * p.M;
+  Vec<T, 8> res[CH], nw[CH];
+  float sum[CH][8];
+  int vi[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    vi[c] = at + c * per * 64;
+    const int64_t vo = (int64_t)min(vi[c], nvec - 1) * 8;
+    res[c] = ldvec<T, 8>((const T*)p.residual + (int64_t)m * p.K + vo);
+    nw[c] = ldvec<T, 8>((const T*)p.norm_w + vo);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum[c][j] = 0.f;
+  }
+  // (all of them at once, in straight code: a loop's waits would be for the weights too)
+  float4 f[U][CH][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const float* src = p.part + ((int64_t)min(u, p.nsplit - 1) * p.M + m) * p.K + min(vi[c], nvec - 1) * 8;
+      f[u][c][0] = *reinterpret_cast<const float4*>(src);
+      f[u][c][1] = *reinterpret_cast<const float4*>(src + 4);
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  load_w(w0, 0);
+  if constexpr (CH * U <= 8) load_w(w1, nchunks > 1 ? 1 : 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const bool there = u < p.nsplit;
+      sum[c][0] += there ? f[u][c][0].x : 0.f; sum[c][1] += there ? f[u][c][0].y : 0.f;
+      sum[c][2] += there ? f[u][c][0].z : 0.f; sum[c][3] += there ? f[u][c][0].w : 0.f;
+      sum[c][4] += there ? f[u][c][1].x : 0.f; sum[c][5] += there ? f[u][c][1].y : 0.f;
+      sum[c][6] += there ? f[u][c][1].z : 0.f; sum[c][7] += there ? f[u][c][1].w : 0.f;
+    }
+  if constexpr (CH * U > 8) load_w(w1, nchunks > 1 ? 1 : 0);
+  float ss = 0.f;
+  const bool writer = blockIdx.x == 0 && blockIdx.y == 0 && mine;
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (mine && vi[c] < nvec) {
+      Vec<T, 8> r;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        sum[c][j] = to_f32(from_f32<T>(sum[c][j])) + to_f32(res[c].v[j]);
+        r.v[j] = from_f32<T>(sum[c][j]);
+        ss += sum[c][j] * sum[c][j];
+      }
+      if (writer) stvec<T, 8>((T*)p.residual_out + (int64_t)m * p.K + vi[c] * 8, r);
+    }
+  ss = wave_sum(ss);
+  if (lane == 0) sums[wave] = ss;
+  __syncthreads();
+  ss = 0.f;
+  for (int i = 0; i < per; ++i) ss += sums[m * per + i];
+  const float inv = 1.0f / sqrtf(ss / (float)p.K + p.eps);
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (mine && vi[c] < nvec) {
+      Vec<T, 8> o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o.v[j] = from_f32<T>((sum[c][j] * inv) * to_f32(nw[c].v[j]));
+      stvec<T, 8>(xs + m * row_len + vi[c] * 8, o);
+    }
+  __syncthreads();
+
+  // ---- the product: fragment rows past the last repeat it (their results are not stored) ----
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  const T* const xt = xs + min(r16, p.M - 1) * row_len + ks + q * 8;
+  auto compute = [&](const frag (&wc)[S], int chunk) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc = Mfma<T>::run(wc[s], *reinterpret_cast<const frag*>(xt + chunk * 256 + s * 32), acc);
+  };
+  int c = 0;
+  for (; c + 2 < nchunks; ++c) {
+    load_w(w2, c + 2);
+    compute(w0, c);
+#pragma unroll
+    for (int s = 0; s < S; ++s) { w0[s] = w1[s]; w1[s] = w2[s]; }
+  }
+  compute(w0, c);
+  if (c + 1 < nchunks) compute(w1, c + 1);
+
+  const int real_tile = (int)blockIdx.x * waves + wave;
+  if constexpr (ACT) {
+    // lanes q < 2 hold gate features 8 tile + 4 q + r of row r16, those 32 lanes higher the up features
+    float up[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      acc[r] = round_to<T>(acc[r]);
+      up[r] = __shfl_xor(acc[r], 32, 64);
+    }
+    const int n0 = real_tile * 8 + 4 * q, half = p.N >> 1;
+    if (q < 2 && r16 < p.M && n0 < half) {
+      Vec<T, 4> o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o.v[r] = silu_mul_one<T>(from_f32<T>(acc[r]), from_f32<T>(up[r]));
+      stvec<T, 4>((T*)p.y + (int64_t)r16 * half + n0, o);
+    }
+  } else {
+    const int n0 = real_tile * 16 + 4 * q;
+    if (r16 < p.M && n0 < p.N) *reinterpret_cast<f32x4*>(p.out_part + ((int64_t)blockIdx.y * p.M + r16) * p.N + n0) = acc;
+  }
+}
+
+template <typename T>
+static int launch_norm_linear(const NormLinearParams& p, const SkinnyPlan& plan, bool act, hipStream_t st) {
+  const bool two = p.K > 512 * (plan.waves / p.M), many = p.nsplit > 4;
+  const size_t lds = (size_t)p.M * (p.K + NL_PAD) * sizeof(T);
+#define MI355_NL(ACT) \
+  (two ? (many ? norm_linear_kernel<T, ACT, 2, 8> : norm_linear_kernel<T, ACT, 2, 4>) : (many ? norm_linear_kernel<T, ACT, 1, 8> : norm_linear_kernel<T, ACT, 1, 4>))
+  void (*kern)(NormLinearParams) = act ? MI355_NL(true) : MI355_NL(false);
+#undef MI355_NL
+  if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(kern, dim3((unsigned)plan.nblocks, (unsigned)plan.splits), dim3(64 * plan.waves), lds, st, p);
+  MI355_CHECK_LAUNCH("norm_linear_packed");
+  return MI355_OK;
+}
+
 template <typename T, int MT, int NT, typename OUT, bool PACKED, int WAVES, bool ACT = false>
 static void launch_ring(const T* x, const T* w, const void* bias, OUT* y, float* slab, unsigned* counters,
                         int M, int N, int K, int64_t x_stride, const SkinnyPlan& p, hipStream_t st,
@@ -1087,6 +1254,30 @@ int mi355_linear_packed_silu_mul(void* y, const void* x, const void* w_packed, i
     launch_skinny<f16_t, f16_t, true, true>((const f16_t*)x, (const f16_t*)w_packed, nullptr, (f16_t*)y, workspace, (int)m, (int)n, (int)k, x_stride, st);
   MI355_CHECK_LAUNCH("linear_packed_silu_mul");
   return MI355_OK;
+}
+
+int mi355_norm_linear_packed_splits(int64_t m, int64_t n, int64_t k, int silu_mul) {
+  if (m < 1 || m > NL_ROWS || n < 16 || n % 16 != 0 || n >= 64 * 1024 || k < SK_BK || k % SK_BK != 0 || g_gemm_variant != 0) return 0;
+  const SkinnyPlan p = plan_skinny(m, n, k, true);
+  if (p.nt != 1 || (silu_mul && p.splits != 1) || k > 1024 * (p.waves / m) || m * (k + NL_PAD) * 2 > 96 * 1024) return 0;
+  return p.splits;
+}
+
+int mi355_norm_linear_packed(void* y, float* out_part, void* residual_out, const float* part, int nsplit, const void* residual,
+                             const void* norm_weight, float eps, const void* w_packed, int64_t m, int64_t n, int64_t k, int dtype, void* stream) {
+  const bool act = y != nullptr;
+  MI355_REQUIRE((y != nullptr) != (out_part != nullptr) && residual_out && part && residual && norm_weight && w_packed && nsplit >= 1 && nsplit <= NL_SPLITS,
+                MI355_ERR_INVALID, "norm_linear_packed: null pointer, not exactly one result, or more than %d splits", NL_SPLITS);
+  MI355_REQUIRE(mi355_norm_linear_packed_splits(m, n, k, act) > 0 && (dtype == MI355_BF16 || dtype == MI355_F16), MI355_ERR_UNSUPPORTED,
+                "norm_linear_packed: needs 1 to %d rows, K %% 256 == 0, N %% 16 == 0, N < 65536, a 16-bit dtype (m=%lld n=%lld k=%lld)", NL_ROWS,
+                (long long)m, (long long)n, (long long)k);
+  MI355_REQUIRE(residual_out != residual, MI355_ERR_INVALID, "norm_linear_packed: the residual is read while the new one is written");
+  MI355_REQUIRE(aligned16(part) && aligned16(residual) && aligned16(residual_out) && aligned16(norm_weight) && aligned16(w_packed) &&
+                    (act ? aligned16(y) : aligned16(out_part)), MI355_ERR_INVALID, "norm_linear_packed: misaligned pointer");
+  NormLinearParams p = {part, residual, residual_out, norm_weight, w_packed, y, out_part, nsplit, (int)m, (int)n, (int)k, 0, eps};
+  const SkinnyPlan plan = plan_skinny(m, n, k, true);
+  p.k_per_split = plan.k_per_split;
+  return dtype == MI355_BF16 ? launch_norm_linear<bf16_t>(p, plan, act, (hipStream_t)stream) : launch_norm_linear<f16_t>(p, plan, act, (hipStream_t)stream);
 }
 
 int mi355_linear(void* y, const void* x, const void* w, const void* bias, int64_t m, int64_t n,

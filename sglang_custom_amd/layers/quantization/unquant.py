@@ -177,6 +177,14 @@ def decode_linear_deferred(layer, x, needs_all_reduce: bool = True):
     return None if part is None else SplitKPartials(part)
 
 
+def takes_norm_in_front(layer, packed, hidden, norm, silu_mul: bool = False) -> bool:
+    """Whether `layer` (16-bit, its packed weight given) forms the rows of the norm in front of it by itself (ops.norm_linear_packed): few rows of
+    a decode step whose projection has left its sum to that norm."""
+    return (DECODE_FUSION and isinstance(hidden, SplitKPartials) and hidden.x_scale is None and packed is not None and packed.is_cuda
+            and isinstance(layer.quant_method, UnquantizedLinearMethod) and packed.dtype == norm.weight.dtype and getattr(layer, "bias", None) is None
+            and hidden.part.shape[0] <= 8 and get_ops().norm_linear_packed_splits(hidden.shape[0], layer.weight.shape[0], hidden.shape[1], silu_mul) > 0)
+
+
 def prefill_linear(x2: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """16-bit rows [M, K] (M > SKINNY_MAX_M) against a plain weight [N, K]."""
     if x2.is_cuda and PREFILL_GEMM == "tiled":

@@ -22,11 +22,13 @@ from ..layers.logits_processor import LogitsProcessor
 from ..layers.quantization.unquant import (
     QuantizedAct,
     SKINNY_MAX_M,
+    SplitKPartials,
     UnquantizedLinearMethod,
     decode_linear_deferred,
     gate_up_silu_mul,
     pack_for_decode,
     pack_gate_up_for_decode,
+    takes_norm_in_front,
 )
 from ..layers.quantization.w8a8_fp8 import W8A8Fp8LinearMethod, prefill_takes_quantised_rows
 from ..layers.quantization.w8a8_fp8 import gate_up_silu_mul_prefill as gate_up_silu_mul_prefill_fp8
@@ -50,8 +52,11 @@ class LlamaMLP(nn.Module):
         self.down_proj = RowParallelLinear(intermediate_size, hidden_size, dtype, device, qm())
         self.act_fn = SiluAndMul()
 
-    def forward(self, x):
-        if isinstance(self.gate_up_proj.quant_method, UnquantizedLinearMethod):
+    def forward(self, x, activated: bool = False):
+        """activated: x is act_fn(gate_up_proj(..)) already."""
+        if activated:
+            pass
+        elif isinstance(self.gate_up_proj.quant_method, UnquantizedLinearMethod):
             x = gate_up_silu_mul(self.gate_up_proj, self.act_fn, x)
         elif (fused := gate_up_silu_mul_prefill_fp8(self.gate_up_proj, x)) is not None:
             x = fused   # prefill: fp8 GEMM with the scales and SiLU-and-mul in its epilogue
@@ -110,22 +115,26 @@ class LlamaAttention(nn.Module):
         self.attn = RadixAttention(self.num_heads, self.head_dim, self.scaling,
                                    num_kv_heads=self.num_kv_heads, layer_id=layer_id)
 
+    def fused_decode_ok(self, dtype, forward_batch) -> bool:
+        pool = forward_batch.token_to_kv_pool
+        return (forward_batch.forward_mode.is_decode()
+                and getattr(pool, "dtype", None) in (dtype, torch.float8_e4m3fn)
+                and (pool.dtype == dtype or self.head_dim == 128)    # one-byte rows at other head sizes: a kernel of their own
+                and forward_batch.attn_backend.supports_fused_qkv(self.attn, self.rotary_emb, dtype))
+
     def _fused_decode(self, positions, hidden_states, forward_batch):
         """Decode fast path: the qkv GEMM leaves its split-K partials and ONE attention launch does
         the reduction, RoPE, the KV-cache write and the attention.  None when it does not apply."""
-        backend = forward_batch.attn_backend
-        pool = forward_batch.token_to_kv_pool
-        if (not forward_batch.forward_mode.is_decode()
-                or getattr(pool, "dtype", None) not in (hidden_states.dtype, torch.float8_e4m3fn)
-                or (pool.dtype != hidden_states.dtype and self.head_dim != 128)    # one-byte rows at other head sizes: a kernel of their own
-                or not backend.supports_fused_qkv(self.attn, self.rotary_emb, hidden_states.dtype)):
+        if not self.fused_decode_ok(hidden_states.dtype, forward_batch):
             return None
         part = decode_linear_deferred(self.qkv_proj, hidden_states, needs_all_reduce=False)
         if part is None:
             return None
-        return backend.forward_decode_fused_qkv(part.part, positions, self.rotary_emb.cos_sin_cache, self.attn,
-                                                forward_batch, part.x_scale, part.w_scale,
-                                                out_dtype=hidden_states.dtype)
+        return self._attend_partials(positions, part, hidden_states.dtype, forward_batch)
+
+    def _attend_partials(self, positions, part, dtype, forward_batch):
+        return forward_batch.attn_backend.forward_decode_fused_qkv(part.part, positions, self.rotary_emb.cos_sin_cache, self.attn,
+                                                                   forward_batch, part.x_scale, part.w_scale, out_dtype=dtype)
 
     def _fused_prefill_qkv(self, positions, hidden_states, forward_batch):
         """Prefill fast path: ONE launch computes the qkv projection, rotates q and k and writes the new
@@ -163,8 +172,13 @@ class LlamaAttention(nn.Module):
                                        rope.cos_sin_cache, rope.is_neox_style, kb, vb, forward_batch.out_cache_loc,
                                        x_scale=xs, w_scale=ws, out_dtype=dtype, split_tail=True)
 
-    def forward(self, positions, hidden_states, forward_batch):
-        attn_output = self._fused_decode(positions, hidden_states, forward_batch)
+    def forward(self, positions, hidden_states, forward_batch, qkv_part=None, dtype=None):
+        """qkv_part: the qkv projection's partials where the caller has them (fused_decode_ok; dtype: the activations'), hidden_states
+        is then not read."""
+        if qkv_part is not None:
+            attn_output = self._attend_partials(positions, qkv_part, dtype, forward_batch)
+        else:
+            attn_output = self._fused_decode(positions, hidden_states, forward_batch)
         if attn_output is not None:
             deferred = decode_linear_deferred(self.o_proj, attn_output)
             if deferred is not None:
@@ -212,6 +226,14 @@ class LlamaDecoderLayer(nn.Module):
             q_in = prefill_takes_quantised_rows(self.self_attn.qkv_proj, m, dtype)
             q_mlp = prefill_takes_quantised_rows(self.mlp.gate_up_proj, m, dtype)
             dense = False
+        at = self.self_attn
+        norm_in = self.input_layernorm
+        if (takes_norm_in_front(at.qkv_proj, getattr(at.qkv_proj, "weight_packed", None), hidden_states, norm_in)
+                and at.fused_decode_ok(norm_in.weight.dtype, forward_batch)):
+            part, residual = get_ops().norm_linear_packed(hidden_states.part, residual, norm_in.weight.data, norm_in.variance_epsilon,
+                                                    at.qkv_proj.weight_packed, at.qkv_proj.weight.shape[0])
+            hidden_states = at(positions, None, forward_batch, SplitKPartials(part), norm_in.weight.dtype)
+            return self._after_attention(hidden_states, residual, q_mlp, dense)
         if residual is None:
             residual = hidden_states
             hidden_states = (self.input_layernorm(hidden_states, quant_fp8=True, dense=dense) if q_in
@@ -221,6 +243,15 @@ class LlamaDecoderLayer(nn.Module):
         else:
             hidden_states, residual = self.input_layernorm(hidden_states, residual)
         hidden_states = self.self_attn(positions, hidden_states, forward_batch)
+        return self._after_attention(hidden_states, residual, q_mlp, dense)
+
+    def _after_attention(self, hidden_states, residual, q_mlp: bool, dense: bool):
+        norm, gate_up = self.post_attention_layernorm, self.mlp.gate_up_proj
+        packed = getattr(gate_up, "weight_packed_gate_up", None)
+        if takes_norm_in_front(gate_up, packed, hidden_states, norm, silu_mul=True):
+            act, residual = get_ops().norm_linear_packed(hidden_states.part, residual, norm.weight.data, norm.variance_epsilon, packed,
+                                                         gate_up.weight.shape[0], silu_mul=True)
+            return self.mlp(act, activated=True), residual
         if q_mlp:
             hidden_states, residual = self.post_attention_layernorm(hidden_states, residual, quant_fp8=True, dense=dense)
         else:

@@ -958,6 +958,31 @@ def fused_add_rmsnorm_partials(part: torch.Tensor, residual: torch.Tensor, weigh
     return x
 
 
+def norm_linear_packed_splits(m: int, n: int, k: int, silu_mul: bool = False) -> int:
+    """The splits of norm_linear_packed's partials; 0 where it does not serve the shape."""
+    return _lib_().mi355_norm_linear_packed_splits(m, n, k, 1 if silu_mul else 0)
+
+
+def norm_linear_packed(part: torch.Tensor, residual: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight_packed: torch.Tensor,
+                       n: int, silu_mul: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+    """fused_add_rmsnorm_partials and the packed projection of its rows in one launch (few rows): returns (split-K partials, or with
+    silu_mul the activated rows, the new residual).  residual itself stays as it is: other workgroups still read it."""
+    _gpu(part, residual, norm_weight, weight_packed)
+    assert part.dim() == 3 and part.is_contiguous() and part.dtype == torch.float32
+    assert residual.is_contiguous() and residual.shape == part.shape[1:] and residual.dtype == norm_weight.dtype == weight_packed.dtype
+    assert norm_weight.is_contiguous() and norm_weight.numel() == part.shape[2]
+    s, m, k = part.shape
+    splits = norm_linear_packed_splits(m, n, k, silu_mul)
+    assert splits > 0 and s <= 8 and weight_packed.numel() == _lib_().mi355_packed_weight_elems(n, k)
+    out = (torch.empty((m, n // 2), dtype=residual.dtype, device=part.device) if silu_mul
+           else torch.empty((splits, m, n), dtype=torch.float32, device=part.device))
+    new = torch.empty_like(residual)
+    check(_lib_().mi355_norm_linear_packed(out.data_ptr() if silu_mul else None, None if silu_mul else out.data_ptr(), new.data_ptr(),
+                                           part.data_ptr(), s, residual.data_ptr(), norm_weight.data_ptr(), float(eps), weight_packed.data_ptr(),
+                                           m, n, k, _dt(residual), _stream(part)), "norm_linear_packed")
+    return out, new
+
+
 def fp8_packed_partials(xq: torch.Tensor, wq_packed: torch.Tensor, n: int) -> Optional[torch.Tensor]:
     """fp8 x fp8 GEMM of fp8_scaled_mm_packed left as raw fp32 split-K partials [splits, M, N]; the
     consumer applies (sum * x_scale[m]) * w_scale[n].  None when the shape is not served."""

@@ -327,9 +327,21 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     const int st = (li >> 5) * 8 + (b & 7), within = li & 31;
     if (st >= p.nsuper) return;
     const int sup_m = st / p.snt, sup_n = st - sup_m * p.snt;
-    tm = sup_m * 8 + (within & 7);
-    tn = sup_n * 4 + (within >> 3);
-    if (tm >= p.mt || tn >= p.nt) return;
+    // An expert's last tile is the one with padding.  The block's others go first, so that the short ones fill up where long ones end: 32
+    // experts of 2048 x 2048, 4 per token, 1000 tokens 279 -> 263 us the layer (3000 313 either way), of 4096 x 4096, 1871 tokens 695 -> 667.
+    const int used = min(*p.tiles_used, p.mt), rank = within >> 2;
+    unsigned last = 0;     // of the block's eight tiles
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int t = sup_m * 8 + i;
+      last |= (t + 1 >= used || p.tile_expert[max(min(t, used - 1), 0)] != p.tile_expert[max(min(t + 1, used - 1), 0)]) ? 1u << i : 0u;
+    }
+    const int whole = 8 - __popc(last);
+    unsigned of = rank < whole ? ~last & 255u : last;
+    for (int i = rank < whole ? rank : rank - whole; i > 0; --i) of &= of - 1;
+    tm = sup_m * 8 + __builtin_ctz(of);
+    tn = sup_n * 4 + (within & 3);
+    if (tm >= used || tn >= p.nt) return;
   } else if (p.splits == 0 || b < p.full) {
     const int at = (b & 7) * (p.splits == 0 ? (int)(gridDim.x >> 3) : p.full >> 3) + li;
     if (at >= p.mt * p.nt) return;
@@ -350,7 +362,6 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   // 88 us with padding worked on, 55 without (268 MB of weights); 1024 tokens: 85 and 72; 3000 tokens: 148 and 145.
   int live = 256;
   if constexpr (EPI == 3) {
-    if (tm >= *p.tiles_used) return;
     if (p.row_map != nullptr) {
       live = 0;
 #pragma unroll

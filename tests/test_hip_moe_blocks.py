@@ -138,3 +138,34 @@ def test_every_expert_walks_all_of_k(ops, K):
     for e in range(E):
         part = slice(256 * e, 256 * e + 256)
         assert torch.equal(y[part], (x.float()[rows[part].long()] @ w[e].float().T).to(torch.bfloat16)), e
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gelu_of_the_tiles(ops, dtype):
+    """The activation in the epilogue through products that copy their input: -20 .. 20 against float64, within half an ulp of the result's
+    type, 2^-20 for the polynomial and z^2 2^-24 for the exponent's two roundings (exp(-z^2 / 2) at -12: 4e-6), and 2^-121 where the
+    exponential is no normal number; infinity stays, minus infinity and NaN give NaN as z * (1 + erf) does."""
+    x = torch.zeros(256, 128, dtype=dtype)
+    x[:, :63] = torch.linspace(-20, 20, 256 * 63).view(256, 63).to(dtype)
+    big = 3e38 if dtype == torch.bfloat16 else 6e4
+    x[:3, 63] = torch.tensor([big, -big, float("nan")])
+    w = torch.zeros(1, 64, 128, dtype=dtype)
+    w[0, :, :64] = torch.eye(64)
+    w[0, 63, 63] = 4.0 if dtype == torch.bfloat16 else 6e4
+    w[0, 63, 64:] = 0.0
+    x[0, 64:] = 0.0
+    rows, te, used = torch.arange(256, dtype=torch.int32, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV), torch.ones(1, dtype=torch.int32, device=DEV)
+    y, xd, wd = torch.empty(256, 64, dtype=dtype, device=DEV), x.to(DEV), w.to(DEV)
+    ops.check(ops._lib_().mi355_moe_grouped_linear_tiled(y.data_ptr(), xd.data_ptr(), 128, wd.data_ptr(), rows.data_ptr(), te.data_ptr(), used.data_ptr(),
+                                                         1, 256, 64, 128, ops._dt(xd), ops._stream(xd)), "tiled")
+    torch.cuda.synchronize()
+    z = x[3:, :63].double()
+    want = 0.5 * z * torch.erfc(-z / 2 ** 0.5)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    least = 2.0 ** -121 if dtype == torch.bfloat16 else 2.0 ** -25      # (half the spacing of fp16's smallest numbers)
+    assert ((y[3:, :63].cpu().double() - want).abs() <= (ulp + 2.0 ** -20 + z ** 2 * 2.0 ** -24) * want.abs() + least).all()
+    if dtype == torch.bfloat16:
+        assert y[0, 63] == float("inf") and y[1, 63].isnan()
+    else:
+        assert y[0, 63] == float("inf")     # (3.6e9 rounds to infinity; its negative to zero)
+    assert y[2].isnan().any()

@@ -531,6 +531,10 @@ int mi355_norm_linear_packed(void* y, float* out_part, void* residual_out, const
 int mi355_linear_packed_silu_mul(void* y, const void* x, const void* w_packed, int64_t m, int64_t n,
                                  int64_t k, int64_t x_stride, void* workspace,
                                  int64_t workspace_bytes, int dtype, void* stream);
+/* The same with the activation chosen: 0 SiLU (rounded before the product, as above), 1 tanh-GELU (its product with up rounded once, as
+ * mi355_gelu_tanh_and_mul). */
+int mi355_linear_packed_act_mul(void* y, const void* x, const void* w_packed, int64_t m, int64_t n, int64_t k, int64_t x_stride,
+                                void* workspace, int64_t workspace_bytes, int act, int dtype, void* stream);
 
 /* Large-M (prefill) projection: y = x @ W^T with 16-bit operands, fp32 accumulation on the matrix
  * cores, one rounding to the output dtype (= dtype).  x [M, K] (row stride x_stride, a multiple

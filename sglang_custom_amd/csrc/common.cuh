@@ -314,6 +314,10 @@ template <typename T> __device__ __forceinline__ T silu_mul_one(T a, T b) {
   return from_f32<T>(s * to_f32(b));
 }
 
+__device__ __forceinline__ float gelu_tanh_f(float z) {
+  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+
 // round_to<T> on two values at once.  For bf16 this is one v_cvt_pk_bf16_f32 (round to nearest even, the
 // rounding round_to<bf16_t> does on the bits) and two bit operations; going through the integer view keeps
 // the compiler from treating the round trip as a no-op.

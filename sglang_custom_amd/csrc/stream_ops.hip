@@ -431,9 +431,6 @@ __global__ __launch_bounds__(256) void commit_state_kernel(
   }
 }
 
-__device__ __forceinline__ float gelu_tanh_f(float z) {
-  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-}
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 // out[t][i] = gelu_tanh(gate[t][i]) * up[t][i], 16 bytes of each operand per thread (d and the row stride multiples of the

@@ -1064,9 +1064,12 @@ def pack_weight_gate_up(weight: torch.Tensor) -> torch.Tensor:
     return pack_weight(inter.reshape(n2, K).contiguous())
 
 
-def linear_packed_silu_mul(x: torch.Tensor, weight_packed: torch.Tensor, n: int) -> torch.Tensor:
+_GATE_ACTS = {"silu": 0, "gelu_tanh": 1}
+
+
+def linear_packed_silu_mul(x: torch.Tensor, weight_packed: torch.Tensor, n: int, act: str = "silu") -> torch.Tensor:
     """SiluAndMul(x @ W_gate_up^T) in one kernel (models/llama.py:94-98) for M <= 64 rows;
-    weight_packed from pack_weight_gate_up, n = 2d rows, returns [M, d]."""
+    weight_packed from pack_weight_gate_up, n = 2d rows, returns [M, d].  act "gelu_tanh": gelu_tanh_and_mul instead."""
     _gpu(x, weight_packed)
     assert x.dim() == 2 and x.stride(1) == 1 and weight_packed.dtype == x.dtype
     M, K = x.shape
@@ -1077,9 +1080,9 @@ def linear_packed_silu_mul(x: torch.Tensor, weight_packed: torch.Tensor, n: int)
     assert weight_packed.numel() == lib.mi355_packed_weight_elems(n, K)
     need = lib.mi355_linear_workspace_bytes(M, n, K)
     ws = _workspace(x.device, need) if need > 0 else None
-    check(lib.mi355_linear_packed_silu_mul(y.data_ptr(), x.data_ptr(), weight_packed.data_ptr(), M, n, K,
-                                           x.stride(0), _p(ws), ws.numel() if ws is not None else 0,
-                                           _dt(x), _stream(x)), "linear_packed_silu_mul")
+    check(lib.mi355_linear_packed_act_mul(y.data_ptr(), x.data_ptr(), weight_packed.data_ptr(), M, n, K,
+                                          x.stride(0), _p(ws), ws.numel() if ws is not None else 0, _GATE_ACTS[act],
+                                          _dt(x), _stream(x)), "linear_packed_act_mul")
     return y
 
 

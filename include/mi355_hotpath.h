@@ -985,7 +985,9 @@ int mi355_window_attention(void* out, const void* q, const void* k_cache, const 
  * mi355_linear_recurrence_ssm_sized, mi355_gated_delta_rule_sized: the same for a caller that knows the step's tokens in all and its
  *   longest segment (0, 0: it does not).  With one decay per head and token, segments and key_dim <= 64, a launch that
  *   mi355_recurrence_takes_chunks says so for then takes 64 tokens at a time: other sums in the same precision, several times
- *   faster on few long segments, slower on many short ones. */
+ *   faster on few long segments, slower on many short ones.
+ * ..._ws: the same with a workspace of mi355_recurrence_workspace_bytes (16-byte aligned, no contents expected; 0: none wanted, null or
+ *   smaller: done without), in which a first launch leaves what the chunks' products take from their own tokens alone.  Same bits. */
 int mi355_rmsnorm_residual_add_scaled(float* x, void* h_out, const void* y, int64_t y_stride, const void* weight,
                                       const void* layer_scale, float offset, float mult, int64_t tokens, int64_t hidden, float eps,
                                       int dtype, void* stream);
@@ -1037,6 +1039,23 @@ int mi355_gated_delta_rule_sized(float* out, float* state, const void* q, const 
                               int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
                               int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
                               int64_t tokens, int64_t longest, void* stream);
+int mi355_linear_recurrence_ssm_ws(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
+                                const void* gate_bias, const float* head_decay, const float* dt_logits, int64_t dt_token_stride,
+                                const float* dt_bias, const float* rate_log, const float* skip, const int32_t* req_to_state,
+                                const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                                const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                                int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t gate_token_stride,
+                                float q_scale, float tau, int qk_dtype, int v_dtype, int64_t tokens, int64_t longest, void* workspace,
+                              int64_t workspace_bytes, void* stream);
+int mi355_gated_delta_rule_ws(float* out, float* state, const void* q, const void* k, const void* v, const void* beta_logits,
+                              const float* gate_logits, const float* rate_bias, const float* rate_log, const int32_t* req_to_state,
+                              const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                              const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                              int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
+                              int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
+                              int64_t tokens, int64_t longest, void* workspace,
+                              int64_t workspace_bytes, void* stream);
+int64_t mi355_recurrence_workspace_bytes(int delta, int64_t batch, int heads, int key_dim, int value_dim, int64_t tokens, int64_t longest);
 int mi355_recurrence_takes_chunks(int delta, int64_t batch, int heads, int key_dim, int value_dim, int64_t tokens, int64_t longest);
 
 /* ---- window attention with averaged blocks before the window and a gate per head -------------------------

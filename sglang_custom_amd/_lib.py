@@ -162,6 +162,9 @@ _SIGNATURES = {
     "mi355_gated_delta_rule_ex": (I, [P, P, P, P, P, P, P, P, P, P, P, P, P, P, L, I, I, I, I, L, L, L, L, L, F, I, I, I, I, P]),
     "mi355_linear_recurrence_ssm_sized": (I, [P, P, P, P, P, P, P, P, P, L, P, P, P, P, P, P, P, P, L, I, I, I, I, L, L, L, L, F, F, I, I, L, L, P]),
     "mi355_gated_delta_rule_sized": (I, [P, P, P, P, P, P, P, P, P, P, P, P, P, P, L, I, I, I, I, L, L, L, L, L, F, I, I, I, I, L, L, P]),
+    "mi355_linear_recurrence_ssm_ws": (I, [P, P, P, P, P, P, P, P, P, L, P, P, P, P, P, P, P, P, L, I, I, I, I, L, L, L, L, F, F, I, I, L, L, P, L, P]),
+    "mi355_gated_delta_rule_ws": (I, [P, P, P, P, P, P, P, P, P, P, P, P, P, P, L, I, I, I, I, L, L, L, L, L, F, I, I, I, I, L, L, P, L, P]),
+    "mi355_recurrence_workspace_bytes": (L, [I, L, I, I, I, L, L]),
     "mi355_recurrence_takes_chunks": (I, [I, L, I, I, I, L, L]),
     "mi355_pool_kv_blocks": (I, [P, P, P, P, P, P, P, P, L, L, I, I, I, I, I, I, P]),
     "mi355_window_attention_pooled": (I, [P, P, P, P, P, P, P, P, P, P, P, L, P, P, L, L, L, L, L, L, I, I, I, I, I, I, I, F, I, P, L, I, I, P]),

@@ -141,10 +141,12 @@ __global__ __launch_bounds__(256) void linear_recurrence_kernel(
 // blocks of 16 tokens with their inverses.  L is summed in double and
 // kept as two floats, so that differences of long sums lose nothing.  Exponents are never positive.
 // One workgroup of 8 waves per (sequence, head, 32 value columns), chunk after chunk; the next chunk's rows are on their way
-// while one is multiplied.  A token by token launch is a chain of LDS reads, multiply-adds and lane exchanges of 1000 (plain) and
-// 1400 (delta) cycles a token, on one wave per SIMD: 4 x 1900 tokens, 16 heads of 64 x 128 took 800 and 1105 us; this takes
-// 214 and 342 (161 and 265 with every product in fp32, whose errors were 1.4 and 1.7 times the token by token form's at
-// strong decays; now they are 0.6 to 1.0 times), bound by the matrix instructions' issue and five to eight barriers a chunk.
+// while one is multiplied, and where it pays what needs no state comes from a launch in front.  A token by token launch is a chain of LDS reads, multiply-adds and lane exchanges of 1000 (plain) and
+// 1400 (delta) cycles a token, on one wave per SIMD: 4 x 1900 tokens, 16 heads of 64 x 128 took 800 and 1105 us; this took
+// 214 and 342 in one launch (161 and 265 with every product in fp32, whose errors were 1.4 and 1.7 times the token by token form's at
+// strong decays; now they are 0.6 to 1.0 times), takes 195 and 317 with the system solved in registers and the state in two buffers, and 148
+// and 206 with the launch in front.  A chunk then takes its workgroup 4.0 and 5.2 us: 1.4 of them double products, 1.1 the outputs' products,
+// the rest the rows' way through LDS and one or three barriers.
 // What a later token of a chunk holds is multiplied by zero for an earlier one, which an infinity or a NaN survives.  They stay in
 // the state, to the end: a sequence that ends with one in its state is done again token by token, so that non-finite
 // inputs reach their own token's outputs and later ones only.  (The second run's code costs the delta rule's chunks 3 % through
@@ -260,22 +262,175 @@ __device__ __forceinline__ void token_recurrence(ChunkArgsInMemory& p) {
     if (d0 + r < p.dk && in_v) sp[(int64_t)r * p.dv] = S[r];
 }
 
+// What a chunk's products take from its own tokens alone, in front of the serial launch: one record per (chunk, head), fragments as the
+// lanes of a product hold them.  Floats: e^(L_t) [64], the state's weights e^(L_end - L_s) w_s [64], beta [64], 64 unused, ten tiles of M,
+// and for the delta rule the system's six tiles under the diagonal ones and those ones' four inverses, tiles of [64 lanes][4].
+constexpr int CK_M = 4 * CK, CK_A = CK_M + 10 * 256, CK_INV = CK_A + 6 * 256;
+constexpr int chunk_record(bool delta) { return delta ? CK_INV + 4 * 256 : CK_A; }
+
+// 64 tokens' decays, by one wave, a token a lane: L in two floats (null: not kept), e^L, the weights in the state, w
+template <bool DELTA>
+__device__ __forceinline__ void chunk_decays(float z, float beta_logit, float rate, float bias, int m, int lane, float* L0, float* L1, float* EL,
+                                             float* WS, float* W) {
+  const float sp_ = softplus_f(z + bias);
+  float la = -rate * sp_;
+  la = la < -1e4f ? -1e4f : la;      // e^-10000 is zero as well, and differences of sums stay finite
+  if (lane >= m) la = 0.f;
+  double sum = (double)la;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double up = __shfl_up(sum, o, 64);
+    if (lane >= o) sum += up;
+  }
+  const double end = __shfl(sum, 63, 64);
+  const float hi = (float)sum;
+  L0[lane] = hi;
+  L1[lane] = (float)(sum - (double)hi);
+  EL[lane] = expf(hi);
+  const float w = DELTA ? 1.0f / (1.0f + expf(-beta_logit)) : sp_;
+  W[lane] = lane < m ? w : 0.f;
+  WS[lane] = expf((float)(end - sum)) * (DELTA ? 1.f : lane < m ? w : 0.f);
+}
+
+// tile (ts, tt) of the weights, on or under the diagonal; lane holds s = 16 ts + 4 lg + r of token t = 16 tt + li: of u_s in out_t and
+// (delta) of the system, its diagonal left out
+template <bool DELTA>
+__device__ __forceinline__ void chunk_weights(const float* Q, const float* K, const float* L0, const float* L1, const float* W, int tt, int ts, int li,
+                                              int lg, f32x4& o, f32x4& sys) {
+  const int t = tt * 16 + li, s = ts * 16 + 4 * lg;
+  const f32x4 qk = tile_mma_exact(K + ts * 16 * CLD, Q + t * CLD, li, lg);
+  const f32x4 l0 = f4(L0 + s), l1 = f4(L1 + s), w = f4(W + s);
+  const float lt0 = L0[t], lt1 = L1[t];
+  f32x4 a;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    a[r] = expf(fminf((lt0 - l0[r]) + (lt1 - l1[r]), 0.f));
+    o[r] = s + r <= t ? qk[r] * a[r] * (DELTA ? 1.f : w[r]) : 0.f;
+  }
+  if constexpr (DELTA) {
+    const f32x4 kk = tile_mma_exact(K + ts * 16 * CLD, K + t * CLD, li, lg);
+    const float beta = W[t];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sys[r] = s + r < t ? kk[r] * a[r] * beta : 0.f;
+  }
+}
+
+// the inverse of a unit lower triangular block of 16, a [16][ld] its strictly lower part: lane j < 16 has column j; to inv [16][20]
+__device__ __forceinline__ void block_inverse(const float* a, int ld, float* inv, int lane) {
+  float x[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    float acc = lane == t ? 1.f : 0.f;
+#pragma unroll
+    for (int s4 = 0; s4 < t; s4 += 4) {
+      const f32x4 av = f4(a + t * ld + s4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (s4 + r < t) acc = fmaf(-av[r], x[s4 + r], acc);
+    }
+    x[t] = acc;
+    inv[t * 20 + lane] = acc;
+  }
+}
+
+__device__ __forceinline__ int chunks_of(int n) { return n > 0 ? (n + CK - 1) / CK : 0; }
+
+// The records, a workgroup each, in no order: a column block's own workgroups of the serial launch each did this again, chunk after chunk.
+// 1952 of them (4 x 1900 tokens, 16 heads, fp32 q and k) take 28 us, with the delta rule's system 47: 84 and 104 MB, and 10 (20) tiles of
+// double products.
+constexpr int CW_THREADS = 256;
 template <typename QT, typename VT, bool DELTA>
-__global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_recurrence_kernel(ChunkArgs p) {
+__global__ __launch_bounds__(CW_THREADS) void chunk_weights_kernel(ChunkArgs p, float* records, int batch) {
+  __shared__ __attribute__((aligned(16))) float Q[CK * CLD], K[CK * CLD], L0[CK], L1[CK], HEAD[3 * CK];
+  __shared__ __attribute__((aligned(16))) float AD[DELTA ? 4 * 16 * 20 : 4], INV[DELTA ? 4 * 16 * 20 : 4];
+  const int h = blockIdx.y, hq = h / (p.heads / p.qk_heads);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+  // the sequence that this chunk of the step belongs to: chunks are numbered through the sequences
+  int64_t chunk = blockIdx.x;
+  int b = -1, n = 0;
+  for (int i0 = 0; i0 < batch; i0 += 64) {
+    const int len = i0 + lane < batch ? p.seg_len[i0 + lane] : 0;
+    int end = chunks_of(len);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(end, o, 64);
+      if (lane >= o) end += up;
+    }
+    const unsigned long long behind = __ballot((int64_t)end > chunk);
+    if (behind != 0) {
+      const int first = __ffsll(behind) - 1;
+      b = i0 + first;
+      n = __shfl(len, first, 64);
+      chunk -= __shfl(end, first, 64) - chunks_of(n);
+      break;
+    }
+    chunk -= __shfl(end, 63, 64);
+  }
+  if (b < 0) return;
+  const int64_t t0 = p.seg_start[b] + chunk * CK;
+  const int m = (int)min((int64_t)CK, n - chunk * CK);
+  float* const rec = records + ((int64_t)blockIdx.x * p.heads + h) * chunk_record(DELTA);
+  const QT* const qg = (const QT*)p.q;
+  const QT* const kg = (const QT*)p.k;
+  QT qr[16], kr[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int e = tid + CW_THREADS * u, t = min(e >> 6, m - 1), i = min(e & 63, p.dk - 1);
+    qr[u] = qg[(t0 + t) * p.q_stride + (int64_t)hq * p.dk + i];
+    kr[u] = kg[(t0 + t) * p.k_stride + (int64_t)hq * p.dk + i];
+  }
+  if (wave == 0) {
+    const int64_t t = t0 + min(lane, m - 1);
+    const float z = p.logits[t * p.logit_stride + h];
+    float beta = 0.f;
+    if (DELTA)
+      beta = p.beta_f32 ? static_cast<const float*>(p.beta_logits)[t * p.beta_stride + h]
+                        : to_f32(static_cast<const VT*>(p.beta_logits)[t * p.beta_stride + h]);
+    chunk_decays<DELTA>(z, beta, expf(p.rate_log[h]), p.bias[h], m, lane, L0, L1, HEAD, HEAD + CK, HEAD + 2 * CK);
+  }
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int e = tid + CW_THREADS * u, t = e >> 6, i = e & 63;
+    const bool in = t < m && i < p.dk;
+    Q[t * CLD + i] = in ? to_f32(qr[u]) * p.q_scale : 0.f;
+    K[t * CLD + i] = in ? to_f32(kr[u]) : 0.f;
+  }
+  __syncthreads();
+  if (tid < 3 * CK) rec[tid] = HEAD[tid];
+  for (int x = wave; x < 10; x += CW_THREADS / 64) {
+    const int tt = x < 1 ? 0 : x < 3 ? 1 : x < 6 ? 2 : 3, ts = x - tt * (tt + 1) / 2;
+    f32x4 o, sys;
+    chunk_weights<DELTA>(Q, K, L0, L1, HEAD + 2 * CK, tt, ts, li, lg, o, sys);
+    *reinterpret_cast<f32x4*>(rec + CK_M + x * 256 + 4 * lane) = o;
+    if constexpr (DELTA) {
+      if (tt == ts) *reinterpret_cast<f32x4*>(AD + (tt * 16 + li) * 20 + 4 * lg) = sys;
+      else *reinterpret_cast<f32x4*>(rec + CK_A + (tt * (tt - 1) / 2 + ts) * 256 + 4 * lane) = sys;
+    }
+  }
+  if constexpr (DELTA) {
+    __syncthreads();
+    if (lane < 16) block_inverse(AD + wave * 16 * 20, 20, INV + wave * 16 * 20, lane);
+    __syncthreads();
+    *reinterpret_cast<f32x4*>(rec + CK_INV + wave * 256 + 4 * lane) = f4(INV + (wave * 16 + li) * 20 + 4 * lg);
+  }
+}
+
+// PREP: with chunk_weights_kernel's records for `chunks` of the step's chunks (a sequence that has more goes token by token)
+template <typename QT, typename VT, bool DELTA, bool PREP>
+__global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_recurrence_kernel(ChunkArgs p, const float* records, int64_t chunks) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* const Q = lds;                       // [t][d]
-  float* const K = Q + CK * CLD;              // [t][d]
-  float* const KT = K + CK * CLD;             // [d][t]
-  float* const M = KT + CK * CLD;             // [t][s] weights of u_s in out_t
-  float* const ST = M + CK * CLD;             // [c][d] state
-  float* const U = ST + RC_COLS * CLD;        // [c][t] v, then the right-hand side, then u
-  float* const L0 = U + RC_COLS * CLD;        // [t] L, upper part
-  float* const L1 = L0 + CK;                  // [t] lower part
-  float* const EL = L1 + CK;                  // [t] e^(L_t)
-  float* const WS = EL + CK;                  // [s] e^(L_end - L_s) w_s
-  float* const W = WS + CK;                   // [s] w_s (plain) or beta_t (delta)
-  float* const A = W + CK;                    // delta: [t][s] strictly lower part of the system
-  float* const INV = A + CK * CLD;            // delta: [4][16][20] inverses of its diagonal blocks
+  constexpr int REC = chunk_record(DELTA), RV = (REC / 4 + CK_THREADS - 1) / CK_THREADS;
+  constexpr int BUF = 2 * CK * CLD + RC_COLS * CLD + REC;                 // PREP: a chunk's rows and record, twice
+  float* const ST = lds;                                                  // [2][c][d] state
+  float* Q = ST + 2 * RC_COLS * CLD;                                      // [t][d]
+  float* K = Q + CK * CLD;                                                // [t][d]
+  float* U = K + CK * CLD;                                                // [c][t] v, then the right-hand side, then u
+  float* R = U + RC_COLS * CLD;                                           // PREP: the record, else its first three rows
+  float* const L0 = R + 3 * CK;                                           // [t] L, upper part
+  float* const L1 = L0 + CK;                                              // [t] lower part
+  float* const M = L1 + CK;                                               // [t][s] weights of u_s in out_t
+  float* const A = M + CK * CLD;                                          // delta: [t][s] strictly lower part of the system
+  float* const INV = A + CK * CLD;                                        // delta: [4][16][20] inverses of its diagonal blocks
   __shared__ int not_finite;
   const int b = blockIdx.z, h = blockIdx.y, c0 = blockIdx.x * RC_COLS;
   const int hq = h / (p.heads / p.qk_heads);
@@ -283,6 +438,16 @@ __global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
   const int64_t t0 = p.seg_start[b];
   const int n = p.seg_len[b];
   if (n <= 0) return;
+  const float* rec = nullptr;
+  bool served = true;
+  if constexpr (PREP) {
+    int before = 0;
+    for (int i = lane; i < b; i += 64) before += chunks_of(p.seg_len[i]);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) before += __shfl_xor(before, o, 64);
+    served = (int64_t)before + chunks_of(n) <= chunks;
+    rec = records + ((int64_t)before * p.heads + h) * REC;
+  }
   const int64_t slot = p.req_to_state[p.req_pool_indices[b]];
   float* const sp = p.state + ((slot * p.heads + h) * (int64_t)p.dk) * p.dv;
   const bool fresh = p.positions[t0] == 0;
@@ -297,28 +462,33 @@ __global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
     ST[c * CLD + i] = (!fresh && i < p.dk && c0 + c < p.dv) ? sp[(int64_t)i * p.dv + c0 + c] : 0.f;
   }
-  if (tid == 0) not_finite = 0;
+  if (tid == 0) not_finite = !served;
   // this wave's tile of the state: d = 16 (wave >> 1) + 4 lg + r, column 16 (wave & 1) + li
   const int sd = (wave >> 1) * 16, sc = (wave & 1) * 16;
 
-  // the next chunk's elements: 8 of q and of k (element tid + 512 u is token e >> 6, channel e & 63), 4 of v, one logit (or two)
+  // the next chunk's elements: tokens 8 wave + u of q and of k, channel lane; 4 of v, tokens 4 (tid >> 5) + u; one logit (or two)
   QT qr[8], kr[8];
   VT vr[4];
   float zr = 0.f, br = 0.f;
+  f32x4 rr[RV];
   auto request = [&](int base) {
     const int m = n - base;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int e = tid + CK_THREADS * u, t = min(e >> 6, m - 1), i = min(e & 63, p.dk - 1);
+      const int t = min(8 * wave + u, m - 1), i = min(lane, p.dk - 1);
       qr[u] = qg[(t0 + base + t) * p.q_stride + (int64_t)hq * p.dk + i];
       kr[u] = kg[(t0 + base + t) * p.k_stride + (int64_t)hq * p.dk + i];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int e = tid + CK_THREADS * u, t = min(e >> 5, m - 1), c = min(c0 + (e & 31), p.dv - 1);
+      const int t = min(4 * (tid >> 5) + u, m - 1), c = min(c0 + (tid & 31), p.dv - 1);
       vr[u] = vg[(t0 + base + t) * p.v_stride + (int64_t)h * p.dv + c];
     }
-    if (tid < 64) {
+    if constexpr (PREP) {
+      const float* const src = rec + (int64_t)(base / CK) * p.heads * REC;
+#pragma unroll
+      for (int u = 0; u < RV; ++u) rr[u] = f4(src + 4 * min(tid + CK_THREADS * u, REC / 4 - 1));
+    } else if (tid < 64) {
       const int64_t t = t0 + base + min(tid, m - 1);
       zr = p.logits[t * p.logit_stride + h];
       if (DELTA)
@@ -326,74 +496,63 @@ __global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                         : to_f32(static_cast<const VT*>(p.beta_logits)[t * p.beta_stride + h]);
     }
   };
-  request(0);
-
-  for (int base = 0; base < n; base += CK) {
-    const int m = min(CK, n - base);
-    __syncthreads();                     // the last chunk is done with, the state is in LDS
+  auto stage = [&](int base) {
+    const int m = n - base;
+    f32x4 v4;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int e = tid + CK_THREADS * u, t = e >> 6, i = e & 63;
-      const bool in = t < m && i < p.dk;
-      const float kv = in ? to_f32(kr[u]) : 0.f;
-      Q[t * CLD + i] = in ? to_f32(qr[u]) * p.q_scale : 0.f;
-      K[t * CLD + i] = kv;
-      KT[i * CLD + t] = kv;
+      const int t = 8 * wave + u;
+      const bool in = t < m && lane < p.dk;
+      Q[t * CLD + lane] = in ? to_f32(qr[u]) * p.q_scale : 0.f;
+      K[t * CLD + lane] = in ? to_f32(kr[u]) : 0.f;
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + CK_THREADS * u, t = e >> 5, c = e & 31;
-      U[c * CLD + t] = t < m && c0 + c < p.dv ? to_f32(vr[u]) : 0.f;
-    }
-    if (tid < 64) {
-      const float sp_ = softplus_f(zr + bias);
-      float la = -rate * sp_;
-      la = la < -1e4f ? -1e4f : la;      // e^-10000 is zero as well, and differences of sums stay finite
-      if (lane >= m) la = 0.f;
-      double sum = (double)la;
+    for (int u = 0; u < 4; ++u) v4[u] = 4 * (tid >> 5) + u < m && c0 + (tid & 31) < p.dv ? to_f32(vr[u]) : 0.f;
+    *reinterpret_cast<f32x4*>(U + (tid & 31) * CLD + 4 * (tid >> 5)) = v4;
+    if constexpr (PREP) {
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const double up = __shfl_up(sum, o, 64);
-        if (lane >= o) sum += up;
-      }
-      const double end = __shfl(sum, 63, 64);
-      const float hi = (float)sum;
-      L0[lane] = hi;
-      L1[lane] = (float)(sum - (double)hi);
-      EL[lane] = expf(hi);
-      const float w = DELTA ? 1.0f / (1.0f + expf(-br)) : sp_;
-      W[lane] = lane < m ? w : 0.f;
-      WS[lane] = expf((float)(end - sum)) * (DELTA ? 1.f : lane < m ? w : 0.f);
+      for (int u = 0; u < RV; ++u)
+        if (tid + CK_THREADS * u < REC / 4) *reinterpret_cast<f32x4*>(R + 4 * (tid + CK_THREADS * u)) = rr[u];
+    } else if (tid < 64) {
+      chunk_decays<DELTA>(zr, br, rate, bias, m, lane, L0, L1, R, R + CK, R + 2 * CK);
     }
-    __syncthreads();
-    if (base + CK < n) request(base + CK);
+  };
+  auto other_buffer = [&](int cur) { Q += cur ? -BUF : BUF, K += cur ? -BUF : BUF, U += cur ? -BUF : BUF, R += cur ? -BUF : BUF; };
+  const int last_base = (n - 1) / CK * CK;
+  if (served) {
+    request(0);
+    stage(0);
+    request(min(CK, last_base));
+  }
+  __syncthreads();
+
+  int cur = 0;
+  for (int base = 0; served && base < n; base += CK, cur ^= 1) {
+    const int m = min(CK, n - base);
+    const float* const EL = R;                    // [t] e^(L_t)
+    const float* const WS = EL + CK;              // [s] e^(L_end - L_s) w_s
+    const float* const W = WS + CK;               // [s] w_s (plain) or beta_t (delta)
+    const float* const S0 = ST + cur * RC_COLS * CLD;
     const float el_end = EL[CK - 1];
 
-    // weights: tiles (s, t) on and under the diagonal; lane holds s = 16 ts + 4 lg + r of token t = 16 tt + li
-    for (int x = wave; x < 10; x += 8) {
-      const int tt = x < 1 ? 0 : x < 3 ? 1 : x < 6 ? 2 : 3, ts = x - tt * (tt + 1) / 2;
-      const int t = tt * 16 + li, s = ts * 16 + 4 * lg;
-      const f32x4 qk = tile_mma_exact(K + ts * 16 * CLD, Q + t * CLD, li, lg);
-      const f32x4 l0 = f4(L0 + s), l1 = f4(L1 + s), w = f4(W + s);
-      const float lt0 = L0[t], lt1 = L1[t];
-      f32x4 o, a;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        a[r] = expf(fminf((lt0 - l0[r]) + (lt1 - l1[r]), 0.f));
-        o[r] = s + r <= t ? qk[r] * a[r] * (DELTA ? 1.f : w[r]) : 0.f;
-      }
-      *reinterpret_cast<f32x4*>(M + t * CLD + s) = o;
-      if constexpr (DELTA) {
-        const f32x4 kk = tile_mma_exact(K + ts * 16 * CLD, K + t * CLD, li, lg);
-        const float beta = W[t];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = s + r < t ? kk[r] * a[r] * beta : 0.f;
-        *reinterpret_cast<f32x4*>(A + t * CLD + s) = o;
+    if constexpr (!PREP) {
+      for (int x = wave; x < 10; x += 8) {
+        const int tt = x < 1 ? 0 : x < 3 ? 1 : x < 6 ? 2 : 3, ts = x - tt * (tt + 1) / 2;
+        f32x4 o, sys;
+        chunk_weights<DELTA>(Q, K, L0, L1, W, tt, ts, li, lg, o, sys);
+        *reinterpret_cast<f32x4*>(M + (tt * 16 + li) * CLD + ts * 16 + 4 * lg) = o;
+        if constexpr (DELTA) *reinterpret_cast<f32x4*>(A + (tt * 16 + li) * CLD + ts * 16 + 4 * lg) = sys;
       }
     }
+    auto weights = [&](int tt, int s) { return PREP ? f4(R + CK_M + (tt * (tt + 1) / 2 + s) * 256 + 4 * lane) : f4(M + (tt * 16 + li) * CLD + s * 16 + 4 * lg); };
+    // what the state's start has in the outputs: wave takes column tile wave & 1 of token tile wave >> 1; lane holds columns 4 lg + r of
+    // token li of the tile.  (The six waves that solve nothing take it while the other two do.)
+    f32x4 from_state;
+    auto start_of_out = [&] { from_state = tile_mma(S0 + (sc + li) * CLD + 4 * lg, Q + (sd + li) * CLD + 4 * lg) * EL[sd + li]; };
+    if (!DELTA || wave < 2) start_of_out();
     if constexpr (DELTA) {
       // right-hand side: lane holds tokens t = 16 (wave >> 1) + 4 lg + r of column 16 (wave & 1) + li
-      const f32x4 y = tile_mma(K + (sd + li) * CLD + 4 * lg, ST + (sc + li) * CLD + 4 * lg);
+      const f32x4 y = tile_mma(K + (sd + li) * CLD + 4 * lg, S0 + (sc + li) * CLD + 4 * lg);
       float* const up = U + (sc + li) * CLD + sd + 4 * lg;
       const f32x4 vv = f4(up), el = f4(EL + sd + 4 * lg), be = f4(W + sd + 4 * lg);
       f32x4 o;
@@ -401,90 +560,120 @@ __global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
       for (int r = 0; r < 4; ++r) o[r] = be[r] * (vv[r] - el[r] * y[r]);
       *reinterpret_cast<f32x4*>(up) = o;
       __syncthreads();
-      // inverses of the four diagonal blocks: wave w, lane j < 16 has column j of block w
-      if (wave < 4 && lane < 16) {
-        float x[16];
-        const float* a = A + (wave * 16) * CLD + wave * 16;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-          float acc = lane == t ? 1.f : 0.f;
-#pragma unroll
-          for (int s4 = 0; s4 < t; s4 += 4) {
-            const f32x4 av = f4(a + t * CLD + s4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (s4 + r < t) acc = fmaf(-av[r], x[s4 + r], acc);
-          }
-          x[t] = acc;
-          INV[(wave * 16 + t) * 20 + lane] = acc;
-        }
+      if constexpr (!PREP) {
+        // inverses of the four diagonal blocks
+        if (wave < 4 && lane < 16) block_inverse(A + (wave * 16) * CLD + wave * 16, CLD, INV + wave * 16 * 20, lane);
+        __syncthreads();
       }
-      __syncthreads();
-      // two waves, 16 columns each: block by block, what the earlier blocks take off and the diagonal block's inverse
+      // two waves, 16 columns each: block by block, what the earlier blocks take off and the diagonal block's inverse.  lane: tokens
+      // 16 blk + 4 lg + r of column li, which is also a B row's k, so that a solved block goes on from the registers
       if (wave < 2) {
-        float* const uc = U + (wave * 16 + li) * CLD;
+        float* const uc = U + (wave * 16 + li) * CLD + 4 * lg;
+        f32x4 off[4], rhs[4], inv[4], a[6];
 #pragma unroll
         for (int blk = 0; blk < 4; ++blk) {
-          f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-          for (int s = 0; s < blk; ++s) mma4(acc, f4(A + (blk * 16 + li) * CLD + s * 16 + 4 * lg), f4(uc + s * 16 + 4 * lg));
-          f32x4 rhs = f4(uc + blk * 16 + 4 * lg) - acc;     // lane: tokens 16 blk + 4 lg + r of column li, which is also a B row's k
+          off[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+          rhs[blk] = f4(uc + blk * 16);
+          inv[blk] = PREP ? f4(R + CK_INV + blk * 256 + 4 * lane) : f4(INV + (blk * 16 + li) * 20 + 4 * lg);
+#pragma unroll
+          for (int s = 0; s < blk; ++s)
+            a[blk * (blk - 1) / 2 + s] = PREP ? f4(R + CK_A + (blk * (blk - 1) / 2 + s) * 256 + 4 * lane) : f4(A + (blk * 16 + li) * CLD + s * 16 + 4 * lg);
+        }
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) {
           f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
-          mma4(x, f4(INV + (blk * 16 + li) * 20 + 4 * lg), rhs);
-          *reinterpret_cast<f32x4*>(uc + blk * 16 + 4 * lg) = x;
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          mma4(x, inv[blk], rhs[blk] - off[blk]);
+          *reinterpret_cast<f32x4*>(uc + blk * 16) = x;
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int to = blk + 1; to < 4; ++to)
+              off[to] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[to * (to - 1) / 2 + blk][j], x[j], off[to], 0, 0, 0);
         }
+      } else {
+        start_of_out();
       }
     }
-    __syncthreads();
-    // outputs: wave takes column tile wave & 1 of token tile wave >> 1; lane holds columns 4 lg + r of token li of the tile
-    {
-      const int t = sd + li;
-      f32x4 acc = tile_mma(ST + (sc + li) * CLD + 4 * lg, Q + t * CLD + 4 * lg) * EL[t];
-      for (int s = 0; s <= wave >> 1; ++s) {
-        f32x4 part = f32x4{0.f, 0.f, 0.f, 0.f};
-        mma4(part, f4(U + (sc + li) * CLD + s * 16 + 4 * lg), f4(M + t * CLD + s * 16 + 4 * lg));
-        acc += part;
-      }
-      if (t < m) {
-        float* const o = p.out + ((t0 + base + t) * p.heads + h) * (int64_t)p.dv + c0 + sc + 4 * lg;
+    if (DELTA || !PREP) __syncthreads();
+    f32x4 us[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (!DELTA) acc[r] = fmaf(skip, U[(sc + 4 * lg + r) * CLD + t], acc[r]);
-        if (p.dv % 4 == 0 && c0 + sc + 4 * lg + 4 <= p.dv) {
-          *reinterpret_cast<f32x4*>(o) = acc;
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (c0 + sc + 4 * lg + r < p.dv) o[r] = acc[r];
-        }
-      }
-    }
+    for (int s = 0; s < 4; ++s) us[s] = f4(U + (sc + li) * CLD + s * 16 + 4 * lg);
     // state, in double like the weights: the sum over 64 tokens rounds once
     f64x4 p64 = f64x4{0., 0., 0., 0.}, q64 = p64;
-    const float* const kt = KT + (sd + 4 * (li & 3) + (li >> 2)) * CLD + 4 * lg;
+    const float* const kt = K + 4 * lg * CLD + sd + 4 * (li & 3) + (li >> 2);
 #pragma unroll
     for (int s = 0; s < 4; s += 2) {
-      const f32x4 k0 = f4(kt + s * 16), k1 = f4(kt + s * 16 + 16);
-      const f32x4 u0 = f4(U + (sc + li) * CLD + s * 16 + 4 * lg), u1 = f4(U + (sc + li) * CLD + s * 16 + 16 + 4 * lg);
+      f32x4 k0, k1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) k0[j] = kt[(s * 16 + j) * CLD], k1[j] = kt[(s * 16 + 16 + j) * CLD];
       const f32x4 w0 = f4(WS + s * 16 + 4 * lg), w1 = f4(WS + s * 16 + 16 + 4 * lg);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        p64 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k0[j], (double)u0[j] * (double)w0[j], p64, 0, 0, 0);
-        q64 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k1[j], (double)u1[j] * (double)w1[j], q64, 0, 0, 0);
+        p64 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k0[j], (double)us[s][j] * (double)w0[j], p64, 0, 0, 0);
+        q64 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k1[j], (double)us[s + 1][j] * (double)w1[j], q64, 0, 0, 0);
       }
     }
-    f32x4 S = f4(ST + (sc + li) * CLD + sd + 4 * lg);
+    f32x4 S = f4(S0 + (sc + li) * CLD + sd + 4 * lg);
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[r] = (float)((double)S[r] * (double)el_end + (p64[r] + q64[r]));
-    __syncthreads();                     // every wave has read the old state
-    *reinterpret_cast<f32x4*>(ST + (sc + li) * CLD + sd + 4 * lg) = S;
+    *reinterpret_cast<f32x4*>(ST + (cur ^ 1) * RC_COLS * CLD + (sc + li) * CLD + sd + 4 * lg) = S;
+    // outputs
+    const int t = sd + li;
+    f32x4 acc = from_state;
+    auto add = [&](auto tiles) {
+      constexpr int N = decltype(tiles)::value;
+      f32x4 part[N], ws[N];
+#pragma unroll
+      for (int s = 0; s < N; ++s) {
+        part[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+        ws[s] = weights(N - 1, s);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int s = 0; s < N; ++s) part[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(us[s][j], ws[s][j], part[s], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < N; ++s) acc += part[s];
+    };
+    switch (wave >> 1) {
+      case 0: add(std::integral_constant<int, 1>{}); break;
+      case 1: add(std::integral_constant<int, 2>{}); break;
+      case 2: add(std::integral_constant<int, 3>{}); break;
+      default: add(std::integral_constant<int, 4>{});
+    }
+    if constexpr (!DELTA) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = fmaf(skip, U[(sc + 4 * lg + r) * CLD + t], acc[r]);
+    }
+    if constexpr (PREP) {
+      // the next chunk's rows into the other buffer, the ones behind it from memory (at the end the last ones again: no branch).  In front of
+      // the stores, for whose end a use of those rows would wait as well
+      other_buffer(cur);
+      stage(base + CK);
+      request(min(base + 2 * CK, last_base));
+    }
+    if (t < m) {
+      float* const o = p.out + ((t0 + base + t) * p.heads + h) * (int64_t)p.dv + c0 + sc + 4 * lg;
+      if (p.dv % 4 == 0 && c0 + sc + 4 * lg + 4 <= p.dv) {
+        *reinterpret_cast<f32x4*>(o) = acc;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c0 + sc + 4 * lg + r < p.dv) o[r] = acc[r];
+      }
+    }
+    if (!PREP && base + CK < n) {
+      __syncthreads();
+      stage(base + CK);
+      request(min(base + 2 * CK, last_base));
+    }
+    __syncthreads();
   }
-  __syncthreads();
   float last[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int e = tid + CK_THREADS * u, i = e >> 5, c = e & 31;
-    last[u] = ST[c * CLD + i];
+    last[u] = ST[cur * RC_COLS * CLD + c * CLD + i];
     if (!isfinite(last[u])) not_finite = 1;
   }
   __syncthreads();
@@ -530,12 +719,35 @@ inline bool chunks_serve(bool delta, int64_t batch, int heads, int dk, int dv, i
   return seg_len != nullptr && (dv % 4 != 0 || aligned16(out)) && chunks_pay(delta, batch, heads, dk, dv, tokens, longest);
 }
 
+// Which of them have records made in front: a chunk behind that costs its workgroup 2.6 us less (delta 5.2), the launch and the first record
+// 8 (10), and 1000 records 14 (24).  Measured, without / with (16 heads of 64 x 128):
+//   plain  1 x 130  23 / 24   1 x 256  30 / 28   4 x 256  32 / 34   1 x 1000  104 / 74   4 x 1900  195 / 148
+//   delta  1 x 130  37 / 32   4 x 130  37 / 35   4 x 256  49 / 46   1 x 1000  174 / 97   4 x 1900  317 / 206
+inline int64_t chunk_records_bytes(bool delta, int64_t batch, int heads, int dk, int dv, int64_t tokens, int64_t longest) {
+  if (!chunks_pay(delta, batch, heads, dk, dv, tokens, longest)) return 0;
+  const double most = (double)cdiv(longest, CK), chunks = std::min(batch * most, tokens / (double)CK + batch);
+  const double rounds = std::ceil(batch * (double)heads * cdiv(dv, RC_COLS) / 256);
+  if ((delta ? 5.2 : 2.6) * std::max(most, rounds * chunks / batch) < (delta ? 10 : 8) + (delta ? 0.024 : 0.014) * chunks * heads) return 0;
+  const int64_t bytes = (tokens / CK + batch) * heads * (int64_t)sizeof(float) * chunk_record(delta);
+  return bytes <= ((int64_t)1 << 30) ? bytes : 0;
+}
+
 template <typename QT, typename VT, bool DELTA>
-int launch_chunks(const ChunkArgs& p, int64_t batch, hipStream_t st) {
-  constexpr size_t bytes = sizeof(float) * (4 * CK * CLD + 2 * RC_COLS * CLD + 5 * CK + (DELTA ? CK * CLD + 4 * 16 * 20 : 0));
-  auto kern = chunk_recurrence_kernel<QT, VT, DELTA>;
-  (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(p.dv, RC_COLS), (unsigned)p.heads, (unsigned)batch), dim3(CK_THREADS), bytes, st, p);
+int launch_chunks(const ChunkArgs& p, int64_t batch, int64_t tokens, int64_t longest, float* records, int64_t bytes, hipStream_t st) {
+  const dim3 grid((unsigned)cdiv(p.dv, RC_COLS), (unsigned)p.heads, (unsigned)batch);
+  const int64_t need = chunk_records_bytes(DELTA, batch, p.heads, p.dk, p.dv, tokens, longest), chunks = tokens / CK + batch;
+  if (records != nullptr && need > 0 && bytes >= need && aligned16(records)) {
+    constexpr size_t lds = sizeof(float) * (2 * RC_COLS * CLD + 2 * (2 * CK * CLD + RC_COLS * CLD + chunk_record(DELTA)));
+    auto kern = chunk_recurrence_kernel<QT, VT, DELTA, true>;
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((chunk_weights_kernel<QT, VT, DELTA>), dim3((unsigned)chunks, (unsigned)p.heads), dim3(CW_THREADS), 0, st, p, records, (int)batch);
+    hipLaunchKernelGGL(kern, grid, dim3(CK_THREADS), lds, st, p, records, chunks);
+    return MI355_OK;
+  }
+  constexpr size_t lds = sizeof(float) * (3 * RC_COLS * CLD + 3 * CK * CLD + 5 * CK + (DELTA ? CK * CLD + 4 * 16 * 20 : 0));
+  auto kern = chunk_recurrence_kernel<QT, VT, DELTA, false>;
+  (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(kern, grid, dim3(CK_THREADS), lds, st, p, (const float*)nullptr, (int64_t)0);
   return MI355_OK;
 }
 
@@ -545,11 +757,11 @@ int launch_recurrence(float* out, float* state, const void* q, const void* k, co
                       const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions, int64_t batch, int heads, int dk,
                       int dv, int64_t qs, int64_t ks, int64_t vs, int64_t gs, float q_scale, float tau, int qk_heads, const float* dt_logits,
                       int64_t dts, const float* dt_bias, const float* rate_log, const float* skip, int64_t tokens, int64_t longest,
-                      hipStream_t stream) {
+                      float* records, int64_t record_bytes, hipStream_t stream) {
   if (dt_logits != nullptr && chunks_serve(false, batch, heads, dk, dv, tokens, longest, seg_len, out)) {
     const ChunkArgs p{out, state, q, k, v, dt_logits, dt_bias, rate_log, skip, nullptr, req_to_state, req_pool_indices, seg_start, seg_len,
                       positions, qs, ks, vs, dts, 0, heads, qk_heads, dk, dv, 0, q_scale};
-    return launch_chunks<QT, VT, false>(p, batch, stream);
+    return launch_chunks<QT, VT, false>(p, batch, tokens, longest, records, record_bytes, stream);
   }
   const dim3 grid((unsigned)cdiv(dv, RC_COLS), (unsigned)heads, (unsigned)batch);
 #define MI355_RC_LAUNCH(R)                                                                                                     \
@@ -679,11 +891,12 @@ int launch_delta(float* out, float* state, const void* q, const void* k, const v
                  const float* gate_logits, const float* rate_bias, const float* rate_log, const int32_t* req_to_state,
                  const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len, const int64_t* positions,
                  int64_t batch, int heads, int qk_heads, int dk, int dv, int64_t qs, int64_t ks, int64_t vs, int64_t bs, int64_t gs,
-                 float q_scale, int gate_per_head, int beta_f32, int64_t tokens, int64_t longest, hipStream_t stream) {
+                 float q_scale, int gate_per_head, int beta_f32, int64_t tokens, int64_t longest, float* records, int64_t record_bytes,
+                 hipStream_t stream) {
   if (gate_per_head && chunks_serve(true, batch, heads, dk, dv, tokens, longest, seg_len, out)) {
     const ChunkArgs p{out, state, q, k, v, gate_logits, rate_bias, rate_log, nullptr, beta_logits, req_to_state, req_pool_indices, seg_start,
                       seg_len, positions, qs, ks, vs, gs, bs, heads, qk_heads, dk, dv, beta_f32, q_scale};
-    return launch_chunks<QT, VT, true>(p, batch, stream);
+    return launch_chunks<QT, VT, true>(p, batch, tokens, longest, records, record_bytes, stream);
   }
   const dim3 grid((unsigned)cdiv(dv, RC_COLS), (unsigned)heads, (unsigned)batch);
 #define MI355_GD_LAUNCH(R)                                                                                                     \
@@ -871,6 +1084,10 @@ int mi355_recurrence_takes_chunks(int delta, int64_t batch, int heads, int key_d
   return heads > 0 && key_dim > 0 && value_dim > 0 && chunks_pay(delta != 0, batch, heads, key_dim, value_dim, tokens, longest);
 }
 
+int64_t mi355_recurrence_workspace_bytes(int delta, int64_t batch, int heads, int key_dim, int value_dim, int64_t tokens, int64_t longest) {
+  return heads > 0 && key_dim > 0 && value_dim > 0 ? chunk_records_bytes(delta != 0, batch, heads, key_dim, value_dim, tokens, longest) : 0;
+}
+
 int mi355_linear_recurrence(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
                             const void* gate_bias, const float* head_decay, const int32_t* req_to_state,
                             const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
@@ -905,6 +1122,20 @@ int mi355_linear_recurrence_ssm_sized(float* out, float* state, const void* q, c
                                 const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
                                 int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t gate_token_stride,
                                 float q_scale, float tau, int qk_dtype, int v_dtype, int64_t tokens, int64_t longest, void* stream) {
+  return mi355_linear_recurrence_ssm_ws(out, state, q, k, v, gate_logits, gate_bias, head_decay, dt_logits, dt_token_stride, dt_bias, rate_log, skip,
+                                        req_to_state, req_pool_indices, seg_start, seg_len, positions, batch, heads, qk_heads, key_dim,
+                                        value_dim, q_token_stride, k_token_stride, v_token_stride, gate_token_stride, q_scale, tau,
+                                        qk_dtype, v_dtype, tokens, longest, nullptr, 0, stream);
+}
+
+int mi355_linear_recurrence_ssm_ws(float* out, float* state, const void* q, const void* k, const void* v, const float* gate_logits,
+                                const void* gate_bias, const float* head_decay, const float* dt_logits, int64_t dt_token_stride,
+                                const float* dt_bias, const float* rate_log, const float* skip, const int32_t* req_to_state,
+                                const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                                const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                                int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t gate_token_stride,
+                                float q_scale, float tau, int qk_dtype, int v_dtype, int64_t tokens, int64_t longest, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
   MI355_REQUIRE(out && state && q && k && v && req_to_state && req_pool_indices && positions, MI355_ERR_INVALID,
                 "linear_recurrence: null pointer");
   MI355_REQUIRE((gate_logits != nullptr) + (head_decay != nullptr) + (dt_logits != nullptr) == 1, MI355_ERR_INVALID,
@@ -925,12 +1156,12 @@ int mi355_linear_recurrence_ssm_sized(float* out, float* state, const void* q, c
       rc = launch_recurrence<T, T>(out, state, q, k, v, gate_logits, gate_bias, head_decay, req_to_state, req_pool_indices,
                                    seg_start, seg_len, positions, batch, heads, key_dim, value_dim, q_token_stride, k_token_stride,
                                    v_token_stride, gate_token_stride, q_scale, tau, qk_heads, dt_logits, dt_token_stride, dt_bias,
-                                   rate_log, skip, tokens, longest, (hipStream_t)stream);
+                                   rate_log, skip, tokens, longest, (float*)workspace, workspace_bytes, (hipStream_t)stream);
     else
       rc = launch_recurrence<float, T>(out, state, q, k, v, gate_logits, gate_bias, head_decay, req_to_state, req_pool_indices,
                                        seg_start, seg_len, positions, batch, heads, key_dim, value_dim, q_token_stride,
                                        k_token_stride, v_token_stride, gate_token_stride, q_scale, tau, qk_heads, dt_logits,
-                                       dt_token_stride, dt_bias, rate_log, skip, tokens, longest, (hipStream_t)stream);
+                                       dt_token_stride, dt_bias, rate_log, skip, tokens, longest, (float*)workspace, workspace_bytes, (hipStream_t)stream);
   });
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("linear_recurrence");
@@ -969,6 +1200,20 @@ int mi355_gated_delta_rule_sized(float* out, float* state, const void* q, const 
                               int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
                               int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
                               int64_t tokens, int64_t longest, void* stream) {
+  return mi355_gated_delta_rule_ws(out, state, q, k, v, beta_logits, gate_logits, rate_bias, rate_log, req_to_state, req_pool_indices, seg_start,
+                                   seg_len, positions, batch, heads, qk_heads, key_dim, value_dim, q_token_stride, k_token_stride,
+                                   v_token_stride, beta_token_stride, gate_token_stride, q_scale, gate_per_head, beta_f32, qk_dtype,
+                                   v_dtype, tokens, longest, nullptr, 0, stream);
+}
+
+int mi355_gated_delta_rule_ws(float* out, float* state, const void* q, const void* k, const void* v, const void* beta_logits,
+                              const float* gate_logits, const float* rate_bias, const float* rate_log, const int32_t* req_to_state,
+                              const int64_t* req_pool_indices, const int32_t* seg_start, const int32_t* seg_len,
+                              const int64_t* positions, int64_t batch, int heads, int qk_heads, int key_dim, int value_dim,
+                              int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride, int64_t beta_token_stride,
+                              int64_t gate_token_stride, float q_scale, int gate_per_head, int beta_f32, int qk_dtype, int v_dtype,
+                              int64_t tokens, int64_t longest, void* workspace,
+                              int64_t workspace_bytes, void* stream) {
   MI355_REQUIRE(out && state && q && k && v && beta_logits && gate_logits && rate_bias && rate_log && req_to_state &&
                     req_pool_indices && positions, MI355_ERR_INVALID, "gated_delta_rule: null pointer");
   MI355_REQUIRE((seg_start == nullptr) == (seg_len == nullptr), MI355_ERR_INVALID,
@@ -985,12 +1230,12 @@ int mi355_gated_delta_rule_sized(float* out, float* state, const void* q, const 
       rc = launch_delta<T, T>(out, state, q, k, v, beta_logits, gate_logits, rate_bias, rate_log, req_to_state, req_pool_indices,
                               seg_start, seg_len, positions, batch, heads, qk_heads, key_dim, value_dim, q_token_stride,
                               k_token_stride, v_token_stride, beta_token_stride, gate_token_stride, q_scale, gate_per_head, beta_f32,
-                              tokens, longest, (hipStream_t)stream);
+                              tokens, longest, (float*)workspace, workspace_bytes, (hipStream_t)stream);
     else
       rc = launch_delta<float, T>(out, state, q, k, v, beta_logits, gate_logits, rate_bias, rate_log, req_to_state,
                                   req_pool_indices, seg_start, seg_len, positions, batch, heads, qk_heads, key_dim, value_dim,
                                   q_token_stride, k_token_stride, v_token_stride, beta_token_stride, gate_token_stride, q_scale,
-                                  gate_per_head, beta_f32, tokens, longest, (hipStream_t)stream);
+                                  gate_per_head, beta_f32, tokens, longest, (float*)workspace, workspace_bytes, (hipStream_t)stream);
   });
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("gated_delta_rule");

@@ -1601,6 +1601,12 @@ def _longest(longest: Optional[int], tokens: int, batch: int) -> int:
     return int(longest) if longest is not None else -(-tokens // max(batch, 1))
 
 
+def _chunk_records(delta: bool, batch: int, heads: int, dk: int, dv: int, tokens: int, longest: int, device):
+    """Scratch memory for a recurrence that takes many tokens at a time, its bytes (0: none wanted)."""
+    need = _lib_().mi355_recurrence_workspace_bytes(int(delta), batch, heads, dk, dv, tokens, longest)
+    return (torch.empty(need, dtype=torch.uint8, device=device) if need else None), need
+
+
 def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, state: torch.Tensor,
                       req_to_state: torch.Tensor, req_pool_indices: torch.Tensor, positions: torch.Tensor, q_scale: float,
                       gate_logits: Optional[torch.Tensor] = None, gate_bias: Optional[torch.Tensor] = None, tau: float = 1.0,
@@ -1639,13 +1645,15 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: to
     _, ss, sl = _seg(tok_req, seg_start, seg_len)
     B = req_pool_indices.numel()
     assert seg_start is not None or B == T, "without segments every token is a sequence of its own"
-    check(_lib_().mi355_linear_recurrence_ssm_sized(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+    longest = _longest(longest, T, B)
+    ws, need = _chunk_records(False, B, H, dk, dv, T, longest, v.device) if dt_logits is not None and ss is not None else (None, 0)
+    check(_lib_().mi355_linear_recurrence_ssm_ws(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                               _p(gate_logits), _p(gate_bias), _p(head_decay), _p(dt_logits),
                                               dt_logits.stride(0) if dt_logits is not None else 0, _p(dt_bias), _p(rate_log), _p(skip),
                                               req_to_state.data_ptr(), req_pool_indices.data_ptr(), ss, sl, positions.data_ptr(), B,
                                               H, G, dk, dv, q.stride(0), k.stride(0), v.stride(0),
                                               gate_logits.stride(0) if gate_logits is not None else 0, float(q_scale), float(tau),
-                                              _dt(q), _dt(v), T, _longest(longest, T, B), _stream(q)), "linear_recurrence")
+                                              _dt(q), _dt(v), T, longest, _p(ws), need, _stream(q)), "linear_recurrence")
     return out
 
 
@@ -1912,12 +1920,14 @@ def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta_log
     _, ss, sl = _seg(tok_req, seg_start, seg_len)
     B = req_pool_indices.numel()
     assert seg_start is not None or B == T, "without segments every token is a sequence of its own"
-    check(_lib_().mi355_gated_delta_rule_sized(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+    longest = _longest(longest, T, B)
+    ws, need = _chunk_records(True, B, H, dk, dv, T, longest, v.device) if per_head and ss is not None else (None, 0)
+    check(_lib_().mi355_gated_delta_rule_ws(out.data_ptr(), state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                                             beta_logits.data_ptr(), gate_logits.data_ptr(), rate_bias.data_ptr(), rate_log.data_ptr(),
                                             req_to_state.data_ptr(), req_pool_indices.data_ptr(), ss, sl, positions.data_ptr(), B, H, G,
                                             dk, dv, q.stride(0), k.stride(0), v.stride(0), beta_logits.stride(0), gate_logits.stride(0),
                                             float(q_scale), int(per_head), int(beta_logits.dtype == torch.float32 and v.dtype != torch.float32),
-                                            _dt(q), _dt(v), T, _longest(longest, T, B), _stream(q)), "gated_delta_rule")
+                                            _dt(q), _dt(v), T, longest, _p(ws), need, _stream(q)), "gated_delta_rule")
     return out
 
 

@@ -135,3 +135,36 @@ def test_non_finite_inputs_reach_no_earlier_token(what, delta):
         ok = ref.isfinite()
         assert torch.equal(got.isfinite(), ok)
         assert (got - ref)[ok].norm() <= 1e-5 * ref[ok].norm()
+
+
+@pytest.mark.parametrize("lens", [(449,), (200, 0, 64, 331, 1), tuple(900 if i == 69 else 130 if i % 9 == 1 else 0 for i in range(70)), (2000, 65)])
+@pytest.mark.parametrize("H,G,dk,dv,qk,vt", [(4, 2, 64, 128, torch.float32, torch.bfloat16), (2, 1, 40, 33, torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("delta", [False, True])
+def test_records_in_front_change_no_bits(lens, H, G, dk, dv, qk, vt, delta, monkeypatch):
+    """What depends on no state from a launch of its own: the same operations, so the same bits, for sequences of none to many chunks
+    whose segments lie in any order."""
+    from sglang_custom_amd import ops
+
+    c = _case(lens, H, G, dk, dv, qk, vt, len(lens) + dk, -1.0)
+    T, B = sum(lens), len(lens)
+    order = torch.randperm(B, generator=torch.Generator().manual_seed(7))      # the sequences' order, not their segments'
+    n = torch.tensor(lens, dtype=torch.int32)[order]
+    start = torch.where(n > 0, c["start"][order], 0).to(torch.int32)
+    d = {k: t.to(DEV) for k, t in c.items()}
+    seg = dict(tok_req=torch.zeros(T, dtype=torch.int32, device=DEV), seg_start=start.to(DEV), seg_len=n.to(DEV), longest=max(lens))
+    args = (d["slots"].int()[order.to(DEV)], torch.arange(B, device=DEV), d["pos"], 0.25)
+    q, k = d["q"][:, : G * dk].view(T, G, dk), d["k"].view(T, G, dk)
+    wanted = ops._chunk_records
+
+    def run(records):
+        monkeypatch.setattr(ops, "_chunk_records", records)
+        out, state = torch.full((T, H, dv), float("nan"), device=DEV), d["state"].clone()
+        if delta:
+            ops.gated_delta_rule(q, k, d["v"], d["beta"], d["z"], d["bias"], d["rate"], out, state, *args, **seg)
+        else:
+            ops.linear_recurrence(q, k, d["v"], out, state, *args, dt_logits=d["z"], dt_bias=d["bias"], rate_log=d["rate"], skip=d["skip"], **seg)
+        return out, state
+
+    assert wanted(delta, B, H, dk, dv, T, max(lens), DEV)[1] > 0, "the case is for the chunks"
+    got, want = run(wanted), run(lambda *a: (None, 0))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and got[0].isfinite().all()

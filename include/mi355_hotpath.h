@@ -535,6 +535,9 @@ int mi355_linear_packed_silu_mul(void* y, const void* x, const void* w_packed, i
  * mi355_gelu_tanh_and_mul). */
 int mi355_linear_packed_act_mul(void* y, const void* x, const void* w_packed, int64_t m, int64_t n, int64_t k, int64_t x_stride,
                                 void* workspace, int64_t workspace_bytes, int act, int dtype, void* stream);
+/* mi355_linear_packed to fp32, the results (rounded to dtype, as there) times scale: logits with a factor.  K % 256 == 0. */
+int mi355_linear_packed_scaled(float* y, const void* x, const void* w_packed, float scale, int64_t m, int64_t n, int64_t k, int64_t x_stride,
+                               void* workspace, int64_t workspace_bytes, int dtype, void* stream);
 
 /* Large-M (prefill) projection: y = x @ W^T with 16-bit operands, fp32 accumulation on the matrix
  * cores, one rounding to the output dtype (= dtype).  x [M, K] (row stride x_stride, a multiple

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const void* __restrict__ bias_,
     OUT* __restrict__ y, float* __restrict__ slab, unsigned* __restrict__ counters, int M, int N,
     int K, int64_t x_stride, int k_per_split, const float* __restrict__ x_scale,
-    const float* __restrict__ w_scale) {
+    const float* __restrict__ w_scale, float out_scale) {   // out_scale: of fp32 results, after their rounding to T
   using frag = typename Mfma<T>::frag;
   constexpr bool FP8 = std::is_same<T, fp8_t>::value;
   constexpr int VE = 16 / sizeof(T);          // elements per 16-byte fragment (8, or 16 for fp8)
@@ -414,6 +414,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_ring_kernel(
         } else {
           const T* bias = static_cast<const T*>(bias_);
           o4[r] = finish<T, OUT>(v[r], bias ? to_f32(bias[n]) : 0.f);
+          if constexpr (std::is_same<OUT, float>::value) o4[r] *= out_scale;
         }
       }
       store4(y + (int64_t)m * N, n0, N, o4);
@@ -891,20 +892,20 @@ static int launch_norm_linear(const NormLinearParams& p, const SkinnyPlan& plan,
 template <typename T, int MT, int NT, typename OUT, bool PACKED, int WAVES, int ACT = ACT_NONE>
 static void launch_ring(const T* x, const T* w, const void* bias, OUT* y, float* slab, unsigned* counters,
                         int M, int N, int K, int64_t x_stride, const SkinnyPlan& p, hipStream_t st,
-                        const float* x_scale = nullptr, const float* w_scale = nullptr) {
+                        const float* x_scale = nullptr, const float* w_scale = nullptr, float out_scale = 1.f) {
   const dim3 grid((unsigned)p.nblocks, (unsigned)p.splits);
   const size_t lds = 2 * (16 * MT) * (512 / NT + 32);   // bytes: same tile geometry for 16-bit and fp8
   auto kern = gemm_ring_kernel<T, MT, NT, OUT, PACKED, WAVES, ACT>;
   if (lds > 48 * 1024)
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), lds, st, x, w, bias, y, slab, counters, M, N, K,
-                     x_stride, p.k_per_split, x_scale, w_scale);
+                     x_stride, p.k_per_split, x_scale, w_scale, out_scale);
 }
 
 template <typename T, int MT, int NT, typename OUT, bool PACKED, int ACT = ACT_NONE>
 static void launch_skinny_cfg(const T* x, const T* w, const T* bias, OUT* y, char* ws, int M,
                               int N, int K, int64_t x_stride, const SkinnyPlan& p,
-                              hipStream_t st, float* part = nullptr) {
+                              hipStream_t st, float* part = nullptr, float out_scale = 1.f) {
   unsigned* counters = p.splits > 1 ? reinterpret_cast<unsigned*>(ws) : nullptr;
   float* slab = p.splits > 1 ? reinterpret_cast<float*>(ws + p.counter_bytes) : nullptr;
   if (part) {   // deferred reduction (ring kernel only; the caller checked): y == nullptr selects it
@@ -914,15 +915,15 @@ static void launch_skinny_cfg(const T* x, const T* w, const T* bias, OUT* y, cha
   }
   if (use_ring(K) || ACT) {
     if constexpr (PACKED && NT == 1) {
-      if (p.waves == 8) return launch_ring<T, MT, NT, OUT, PACKED, 8, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st);
-      if (p.waves == 7) return launch_ring<T, MT, NT, OUT, PACKED, 7, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st);
-      if (p.waves == 6) return launch_ring<T, MT, NT, OUT, PACKED, 6, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st);
-      return launch_ring<T, MT, NT, OUT, PACKED, 4, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st);
+      if (p.waves == 8) return launch_ring<T, MT, NT, OUT, PACKED, 8, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st, nullptr, nullptr, out_scale);
+      if (p.waves == 7) return launch_ring<T, MT, NT, OUT, PACKED, 7, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st, nullptr, nullptr, out_scale);
+      if (p.waves == 6) return launch_ring<T, MT, NT, OUT, PACKED, 6, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st, nullptr, nullptr, out_scale);
+      return launch_ring<T, MT, NT, OUT, PACKED, 4, ACT>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st, nullptr, nullptr, out_scale);
     }
     if constexpr (!ACT && PACKED && NT == 2)
-      if (p.waves == 8) return launch_ring<T, MT, NT, OUT, PACKED, 8>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st);
+      if (p.waves == 8) return launch_ring<T, MT, NT, OUT, PACKED, 8>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st, nullptr, nullptr, out_scale);
     if constexpr (!ACT)
-      return launch_ring<T, MT, NT, OUT, PACKED, 4>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st);
+      return launch_ring<T, MT, NT, OUT, PACKED, 4>(x, w, bias, y, slab, counters, M, N, K, x_stride, p, st, nullptr, nullptr, out_scale);
   }
   if constexpr (ACT) return;   // callers check the preconditions (ring kernel, one tile per wave)
   else {
@@ -940,10 +941,10 @@ static void launch_skinny_cfg(const T* x, const T* w, const T* bias, OUT* y, cha
 
 template <typename T, typename OUT, bool PACKED = false, int ACT = ACT_NONE>
 static void launch_skinny(const T* x, const T* w, const T* bias, OUT* y, void* ws, int M, int N,
-                          int K, int64_t x_stride, hipStream_t st, float* part = nullptr) {
+                          int K, int64_t x_stride, hipStream_t st, float* part = nullptr, float out_scale = 1.f) {
   const SkinnyPlan p = plan_skinny(M, N, K, use_ring(K) && PACKED);
   const int mt = (M + 15) / 16;
-#define SK(MT_, NT_) launch_skinny_cfg<T, MT_, NT_, OUT, PACKED, ACT>(x, w, bias, y, (char*)ws, M, N, K, x_stride, p, st, part)
+#define SK(MT_, NT_) launch_skinny_cfg<T, MT_, NT_, OUT, PACKED, ACT>(x, w, bias, y, (char*)ws, M, N, K, x_stride, p, st, part, out_scale)
   if constexpr (ACT) {
     if (mt <= 1) SK(1, 1); else if (mt <= 2) SK(2, 1); else SK(4, 1);
   } else if (p.nt == 2) {
@@ -1204,6 +1205,26 @@ int mi355_linear_packed(void* y, const void* x, const void* w_packed, const void
     else launch_skinny<f16_t, f16_t, true>((const f16_t*)x, (const f16_t*)w_packed, (const f16_t*)bias, (f16_t*)y, workspace, (int)m, (int)n, (int)k, x_stride, st);
   }
   MI355_CHECK_LAUNCH("linear_packed");
+  return MI355_OK;
+}
+
+int mi355_linear_packed_scaled(float* y, const void* x, const void* w_packed, float scale, int64_t m, int64_t n, int64_t k, int64_t x_stride,
+                               void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
+  MI355_REQUIRE(y && x && w_packed, MI355_ERR_INVALID, "linear_packed_scaled: null pointer");
+  MI355_REQUIRE(m >= 0 && m <= 64 && n > 0 && k > 0 && x_stride >= k && x_stride % 8 == 0, MI355_ERR_INVALID,
+                "linear_packed_scaled: needs 0 <= M <= 64 (m=%lld n=%lld k=%lld)", (long long)m, (long long)n, (long long)k);
+  MI355_REQUIRE(use_ring(k) && (dtype == MI355_BF16 || dtype == MI355_F16), MI355_ERR_UNSUPPORTED,
+                "linear_packed_scaled: 16-bit operands and K %% 256 == 0 (k=%lld)", (long long)k);
+  MI355_REQUIRE(aligned16(x) && aligned16(w_packed), MI355_ERR_INVALID, "linear_packed_scaled: misaligned pointer");
+  if (m == 0) return MI355_OK;
+  const int64_t need = mi355_linear_workspace_bytes(m, n, k);
+  MI355_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)), MI355_ERR_INVALID,
+                "linear_packed_scaled: workspace of %lld bytes (16-B aligned) required, got %lld", (long long)need, (long long)workspace_bytes);
+  if (dtype == MI355_BF16)
+    launch_skinny<bf16_t, float, true>((const bf16_t*)x, (const bf16_t*)w_packed, nullptr, y, workspace, (int)m, (int)n, (int)k, x_stride, (hipStream_t)stream, nullptr, scale);
+  else
+    launch_skinny<f16_t, float, true>((const f16_t*)x, (const f16_t*)w_packed, nullptr, y, workspace, (int)m, (int)n, (int)k, x_stride, (hipStream_t)stream, nullptr, scale);
+  MI355_CHECK_LAUNCH("linear_packed_scaled");
   return MI355_OK;
 }
 

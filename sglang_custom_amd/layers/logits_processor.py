@@ -118,11 +118,11 @@ class LogitsProcessor(nn.Module):
 
     def _get_logits(self, hidden_states: torch.Tensor, lm_head) -> torch.Tensor:
         w = lm_head.weight
-        single = not self.do_tensor_parallel_all_gather and self.logit_scale is None
+        single = not self.do_tensor_parallel_all_gather
         x = hidden_states.to(w.dtype)
         if single and (x.shape[0] <= 64 or x.dtype == torch.float32 or not x.is_cuda):
-            # T-rounded logits widened to fp32 in the GEMM epilogue (= matmul(...).float())
-            logits = decode_linear(lm_head, x, None, out_dtype=torch.float32)
+            # T-rounded logits widened to fp32 in the GEMM epilogue (= matmul(...).float()), and scaled there: one rounding, not two
+            logits = decode_linear(lm_head, x, None, out_dtype=torch.float32, scale=self.logit_scale)
             return logits[:, : self.config.vocab_size]
         if x.shape[0] <= 64 or x.dtype == torch.float32 or not x.is_cuda:
             logits = decode_linear(lm_head, x, None)

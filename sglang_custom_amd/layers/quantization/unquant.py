@@ -54,20 +54,23 @@ def pack_for_decode(layer) -> None:
     """Keep a second copy of a 16-bit weight in the decode GEMM's streaming order (MFMA-fragment
     blocks, ops.pack_weight).  The row-major copy stays: prefill GEMMs, the embedding gather and
     checkpoint loading use it.  2x weight bytes is the price of reading decode weights as whole
-    contiguous lines; at 288 GB of HBM per GPU it is not the binding constraint."""
+    contiguous lines; at 288 GB of HBM per GPU it is not the binding constraint.  (Output heads at 64 rows, plain / packed:
+    32768 x 4096 63 / 46 us, 32768 x 2048 34 / 25.)"""
     w = layer.weight
     layer.weight_packed = None
     if w.is_cuda and w.dtype in (torch.bfloat16, torch.float16) and w.shape[1] % 32 == 0:
         layer.weight_packed = get_ops().pack_weight(w.data)
 
 
-def decode_linear(layer, x2: torch.Tensor, bias: Optional[torch.Tensor], out_dtype=None) -> torch.Tensor:
-    """M <= 64 rows (or fp32): the hand-written kernels, on the packed copy when there is one."""
+def decode_linear(layer, x2: torch.Tensor, bias: Optional[torch.Tensor], out_dtype=None, scale: Optional[float] = None) -> torch.Tensor:
+    """M <= 64 rows (or fp32): the hand-written kernels, on the packed copy when there is one.  scale: of an fp32 result, applied to the
+    widened values."""
     ops = get_ops()
     wp = getattr(layer, "weight_packed", None)
     if wp is not None and x2.shape[0] <= SKINNY_MAX_M and x2.stride(0) % 8 == 0:
-        return ops.linear_packed(x2, wp, layer.weight.shape[0], bias, out_dtype=out_dtype)
-    return ops.linear(x2, layer.weight, bias, out_dtype=out_dtype)
+        return ops.linear_packed(x2, wp, layer.weight.shape[0], bias, out_dtype=out_dtype, scale=1.0 if scale is None else scale)
+    y = ops.linear(x2, layer.weight, bias, out_dtype=out_dtype)
+    return y if scale is None else y.mul_(scale)
 
 
 def pack_gate_up_for_decode(layer) -> None:

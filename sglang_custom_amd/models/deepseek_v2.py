@@ -33,6 +33,7 @@ from ..layers.quantization.unquant import (
     QuantizedAct,
     UnquantizedLinearMethod,
     decode_linear_deferred,
+    pack_for_decode,
     pack_gate_up_for_decode,
 )
 from ..layers.radix_attention import RadixAttention
@@ -423,6 +424,7 @@ class DeepseekV2ForCausalLM(nn.Module):
             if isinstance(gu.quant_method, UnquantizedLinearMethod):
                 pack_gate_up_for_decode(gu)     # gate and up rows interleaved: SiLU-and-mul in the decode GEMM's epilogue
             layer.self_attn.post_load_weights()
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

@@ -53,7 +53,7 @@ from ..layers.linear_recurrence import (
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.post_norm import NormedResidualAdd
 from ..layers.pre_norm import OffsetRMSNorm
-from ..layers.quantization.unquant import gate_up_silu_mul, pack_gate_up_for_decode
+from ..layers.quantization.unquant import gate_up_silu_mul, pack_for_decode, pack_gate_up_for_decode
 from ..layers.rotary_embedding import scaled_pair_inv_freq
 from ..layers.short_conv import ShortCausalConv
 from ..layers.vocab_parallel_embedding import ParallelLMHead
@@ -326,6 +326,7 @@ class FudonexForCausalLM(nn.Module):
         for layer in self.model.layers:
             if layer.mlp is not None:
                 pack_gate_up_for_decode(layer.mlp.gate_up)   # gate and up rows interleaved: silu * up in the decode GEMM's epilogue
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

@@ -38,6 +38,7 @@ from ..layers.logits_processor import LogitsProcessor
 from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.pre_norm import BranchResidualAdd, OffsetRMSNorm
 from ..layers.short_conv import ShortCausalConv
+from ..layers.quantization.unquant import pack_for_decode
 from ..layers.vocab_parallel_embedding import ParallelLMHead
 from ..layers.window_attention import WindowSinkAttention
 from ..ops_backend import get_ops
@@ -340,6 +341,7 @@ class GataraxForCausalLM(nn.Module):
     def process_weights_after_loading(self) -> None:
         for lin in self._linears():
             lin.quant_method.process_weights_after_loading(lin)
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

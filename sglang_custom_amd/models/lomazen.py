@@ -40,7 +40,7 @@ from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import PassEntry, RMSNormResidualAdd
 from ..layers.pre_norm import OffsetRMSNorm
 from ..layers.rotary_embedding import banded_pair_inv_freq
-from ..layers.quantization.unquant import SKINNY_MAX_M, pack_gate_up_for_decode
+from ..layers.quantization.unquant import SKINNY_MAX_M, pack_for_decode, pack_gate_up_for_decode
 from ..layers.vocab_parallel_embedding import ParallelLMHead
 from ..ops_backend import get_ops
 
@@ -245,6 +245,7 @@ class LomazenForCausalLM(nn.Module):
         for module in self.modules():
             if isinstance(module, LomazenMLP):
                 pack_gate_up_for_decode(module.gate_up)     # gate and up rows interleaved: GELU * up in the decode GEMM's epilogue
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

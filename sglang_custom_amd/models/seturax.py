@@ -30,6 +30,7 @@ from ..layers.latent_window_attention import LatentWindowAttention
 from ..layers.linear import ReplicatedLinear
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.token_shift import BigramHashEmbedding, GatedResidual, ShiftedLayerNorm
+from ..layers.quantization.unquant import pack_for_decode
 from ..layers.vocab_parallel_embedding import ParallelLMHead
 from ..ops_backend import get_ops
 
@@ -187,6 +188,7 @@ class SeturaxForCausalLM(nn.Module):
     def process_weights_after_loading(self) -> None:
         for lin in self._linears():
             lin.quant_method.process_weights_after_loading(lin)
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

@@ -43,7 +43,7 @@ from ..layers.linear_recurrence import HeadNormGate, MatrixMemory
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import LayerNormResidualAdd
-from ..layers.quantization.unquant import prefill_linear
+from ..layers.quantization.unquant import pack_for_decode, prefill_linear
 from ..layers.rotary_embedding import scaled_pair_inv_freq
 from ..layers.token_shift import ShiftedLayerNorm
 from ..layers.vocab_parallel_embedding import ParallelLMHead
@@ -284,6 +284,7 @@ class SilatarForCausalLM(nn.Module):
                 module.quant_method.process_weights_after_loading(module)
             elif isinstance(module, (PerHeadLinear, SilatarLatentAttention)):
                 module.process_weights_after_loading()
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

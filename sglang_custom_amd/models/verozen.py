@@ -31,6 +31,7 @@ from ..layers.logits_processor import LogitsProcessor
 from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import GroupRMSNorm, NormedResidualAdd
 from ..layers.sigmoid_attention import SigmoidAttention
+from ..layers.quantization.unquant import pack_for_decode
 from ..layers.vocab_parallel_embedding import ParallelLMHead
 from ..ops_backend import get_ops
 
@@ -302,6 +303,7 @@ class VerozenForCausalLM(nn.Module):
     def process_weights_after_loading(self) -> None:
         for lin in self._linears():
             lin.quant_method.process_weights_after_loading(lin)
+        pack_for_decode(self.lm_head)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0, std: float = 0.02) -> None:

@@ -907,8 +907,9 @@ def pack_weight(weight: torch.Tensor) -> torch.Tensor:
 
 
 def linear_packed(x: torch.Tensor, weight_packed: torch.Tensor, n: int, bias: Optional[torch.Tensor] = None,
-                  out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """linear() for M <= 64 on a weight produced by pack_weight (n = number of output features)."""
+                  out_dtype: Optional[torch.dtype] = None, scale: float = 1.0) -> torch.Tensor:
+    """linear() for M <= 64 on a weight produced by pack_weight (n = number of output features).  scale: of an fp32 result, after its
+    rounding to x's type."""
     _gpu(x, weight_packed, bias)
     assert x.dim() == 2 and x.stride(1) == 1 and weight_packed.dtype == x.dtype
     M, K = x.shape
@@ -920,6 +921,13 @@ def linear_packed(x: torch.Tensor, weight_packed: torch.Tensor, n: int, bias: Op
     assert weight_packed.numel() == lib.mi355_packed_weight_elems(n, K)
     need = lib.mi355_linear_workspace_bytes(M, n, K)
     ws = _workspace(x.device, need) if need > 0 else None
+    if scale != 1.0:
+        assert out_dtype == torch.float32 and bias is None
+        if K % 256:
+            return linear_packed(x, weight_packed, n, None, out_dtype).mul_(scale)
+        check(lib.mi355_linear_packed_scaled(y.data_ptr(), x.data_ptr(), weight_packed.data_ptr(), float(scale), M, n, K, x.stride(0),
+                                             _p(ws), ws.numel() if ws is not None else 0, _dt(x), _stream(x)), "linear_packed_scaled")
+        return y
     check(lib.mi355_linear_packed(y.data_ptr(), x.data_ptr(), weight_packed.data_ptr(), _p(bias), M, n, K,
                                   x.stride(0), _p(ws), ws.numel() if ws is not None else 0, _dt(x),
                                   _DT[out_dtype], _stream(x)), "linear_packed")

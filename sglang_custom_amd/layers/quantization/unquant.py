@@ -20,6 +20,7 @@ import torch.nn.functional as F
 from ...ops_backend import get_ops
 
 SKINNY_MAX_M = 64
+FEW_MAX_M = 256         # rows up to which mi355_linear_few may be ahead: asking it costs the host 3 us, which steps of 400 rows feel
 # Deferred split-K reduction / fused decode step (bit-identical to the unfused kernels; the switch
 # exists so that tests and profiles can run both).
 DECODE_FUSION = True
@@ -96,7 +97,7 @@ def gate_up_silu_mul(layer, act_fn, x: torch.Tensor) -> torch.Tensor:
         return y.view(*x.shape[:-1], y.shape[-1])
     w = layer.weight
     plain = x2.is_cuda and isinstance(layer.quant_method, UnquantizedLinearMethod) and getattr(layer, "bias", None) is None
-    if plain and x2.shape[0] > SKINNY_MAX_M and PREFILL_GEMM != "library":
+    if plain and SKINNY_MAX_M < x2.shape[0] <= FEW_MAX_M and PREFILL_GEMM != "library":
         y = get_ops().linear_few(x2, w, None, silu_mul=True)
         if y is not None:
             return y.view(*x.shape[:-1], y.shape[-1])
@@ -190,7 +191,7 @@ def takes_norm_in_front(layer, packed, hidden, norm, silu_mul: bool = False) -> 
 
 def prefill_linear(x2: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """16-bit rows [M, K] (M > SKINNY_MAX_M) against a plain weight [N, K]."""
-    if x2.is_cuda and PREFILL_GEMM == "tiled":
+    if x2.shape[0] <= FEW_MAX_M and x2.is_cuda and PREFILL_GEMM == "tiled":
         y = get_ops().linear_few(x2, weight, bias)
         if y is not None:
             return y

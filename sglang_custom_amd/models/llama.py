@@ -226,9 +226,9 @@ class LlamaDecoderLayer(nn.Module):
             q_in = prefill_takes_quantised_rows(self.self_attn.qkv_proj, m, dtype)
             q_mlp = prefill_takes_quantised_rows(self.mlp.gate_up_proj, m, dtype)
             dense = False
-        at = self.self_attn
-        norm_in = self.input_layernorm
-        if (takes_norm_in_front(at.qkv_proj, getattr(at.qkv_proj, "weight_packed", None), hidden_states, norm_in)
+        if (isinstance(hidden_states, SplitKPartials)
+                and takes_norm_in_front((at := self.self_attn).qkv_proj, getattr(at.qkv_proj, "weight_packed", None), hidden_states,
+                                        norm_in := self.input_layernorm)
                 and at.fused_decode_ok(norm_in.weight.dtype, forward_batch)):
             part, residual = get_ops().norm_linear_packed(hidden_states.part, residual, norm_in.weight.data, norm_in.variance_epsilon,
                                                     at.qkv_proj.weight_packed, at.qkv_proj.weight.shape[0])
@@ -246,9 +246,9 @@ class LlamaDecoderLayer(nn.Module):
         return self._after_attention(hidden_states, residual, q_mlp, dense)
 
     def _after_attention(self, hidden_states, residual, q_mlp: bool, dense: bool):
-        norm, gate_up = self.post_attention_layernorm, self.mlp.gate_up_proj
-        packed = getattr(gate_up, "weight_packed_gate_up", None)
-        if takes_norm_in_front(gate_up, packed, hidden_states, norm, silu_mul=True):
+        if (isinstance(hidden_states, SplitKPartials)
+                and takes_norm_in_front(gate_up := self.mlp.gate_up_proj, packed := getattr(gate_up, "weight_packed_gate_up", None), hidden_states,
+                                        norm := self.post_attention_layernorm, silu_mul=True)):
             act, residual = get_ops().norm_linear_packed(hidden_states.part, residual, norm.weight.data, norm.variance_epsilon, packed,
                                                          gate_up.weight.shape[0], silu_mul=True)
             return self.mlp(act, activated=True), residual

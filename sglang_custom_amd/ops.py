@@ -58,12 +58,13 @@ def _kv_layout(buf: torch.Tensor) -> int:
     [heads, slots, 2, d] one seen the same way; anything else is refused."""
     if buf.is_contiguous():
         return 0
-    assert buf.dim() == 3 and buf.stride(2) == 1, f"KV cache tensor with strides {buf.stride()}"
+    strides = buf.stride()
+    assert len(strides) == 3 and strides[2] == 1, f"KV cache tensor with strides {strides}"
     s, _, d = buf.shape
-    if buf.stride() == (d, s * d, 1):
+    if strides == (d, s * d, 1):
         return KV_HEAD_MAJOR
-    assert buf.stride() == (2 * d, 2 * s * d, 1), \
-        f"KV cache tensor is neither [slots, heads, d] contiguous nor a head-major view: strides {buf.stride()}"
+    assert strides == (2 * d, 2 * s * d, 1), \
+        f"KV cache tensor is neither [slots, heads, d] contiguous nor a head-major view: strides {strides}"
     return KV_HEAD_MAJOR | KV_INTERLEAVED
 
 
@@ -718,8 +719,10 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
     bs = qo_indptr.numel() - 1
     lib, dt = _lib_(), _kvdt(q_extend, k_buffer, v_buffer)
     # few blocks of queries over many keys: workgroups share a block's keys (kv_indices holds the cached tokens' slots)
-    splits = lib.mi355_extend_attention_splits(T, bs, int(max_len_extend), kv_indices.numel(), 1 if custom_mask is not None else 0, Hq, D, Dv,
-                                               float(sm_scale), float(logit_cap), int(sliding_window_size), dt)
+    splits, cached = 1, kv_indices.numel()
+    if cached >= 512:
+        splits = lib.mi355_extend_attention_splits(T, bs, int(max_len_extend), cached, 1 if custom_mask is not None else 0, Hq, D, Dv,
+                                                   float(sm_scale), float(logit_cap), int(sliding_window_size), dt)
     need = lib.mi355_extend_attention_workspace_bytes(T, Hq, Dv, splits) if splits > 1 else 0
     ws = torch.empty(need, dtype=torch.uint8, device=q_extend.device) if need else None
     check(lib.mi355_extend_attention_ws(
@@ -812,9 +815,12 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return y
 
 
+FEW_MAX_M, FEW_MAX_M_FP8 = 256, 512     # rows up to which mi355_linear_few may be ahead: asking it costs the host 3 us
+
+
 def linear_few_supported(m: int, n: int, k: int, out_dtype: torch.dtype, silu_mul: bool = False, fp8: bool = False) -> bool:
     """Whether linear_few serves the shape."""
-    return out_dtype in (torch.bfloat16, torch.float16) and bool(
+    return m <= (FEW_MAX_M_FP8 if fp8 else FEW_MAX_M) and out_dtype in (torch.bfloat16, torch.float16) and bool(
         _lib_().mi355_linear_few_supported(m, n, k, 1 if fp8 else 0, _DT[out_dtype], 1 if silu_mul else 0))
 
 
@@ -825,10 +831,12 @@ def linear_few(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     fill the chip with them; None where another kernel is ahead (more rows, more columns than one round of workgroups) or the operands are
     none that it takes (16-byte rows)."""
     m, k = x.shape
-    n = weight.shape[0]
     fp8 = x_scale is not None
+    if not 0 < m <= (FEW_MAX_M_FP8 if fp8 else FEW_MAX_M):
+        return None
+    n = weight.shape[0]
     out_dtype = out_dtype or x.dtype
-    if (not 0 < m <= 512 or not x.is_cuda or out_dtype not in (torch.bfloat16, torch.float16) or (x.stride(0) != k if fp8 else x.stride(0) % 8 != 0)
+    if (not x.is_cuda or out_dtype not in (torch.bfloat16, torch.float16) or (x.stride(0) != k if fp8 else x.stride(0) % 8 != 0)
             or x.stride(1) != 1 or not weight.is_contiguous() or weight.dtype != x.dtype or weight.shape[1] != k
             or (bias is not None and (silu_mul or bias.dtype != out_dtype or not bias.is_contiguous() or bias.data_ptr() % 16 != 0))
             or x.data_ptr() % 16 != 0 or weight.data_ptr() % 16 != 0):

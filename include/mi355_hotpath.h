@@ -1173,6 +1173,10 @@ int mi355_qkv_rotate_write(void* q_out, void* k_cache, void* v_cache, const void
 int mi355_rmsnorm_residual_add_next(float* x, void* h, const void* y, int64_t y_stride, const int32_t* rows, const float* coef, int n_rows,
                                     const void* w_out, const void* w_next, int64_t tokens, int64_t hidden, float eps, int dtype,
                                     void* stream);
+/* mi355_rmsnorm_residual_add_next (rms) or mi355_layernorm_residual_add with b[t] = the sum over splits of part [splits][tokens][hidden], in
+ * their order, rounded to dtype (mi355_linear_packed_partials).  hidden % 8 == 0, <= 8192. */
+int mi355_norm_residual_add_partials(float* x, void* h, const float* part, int splits, const void* w_out, const void* w_next, int64_t tokens,
+                                     int64_t hidden, float eps, int rms, int dtype, void* stream);
 int mi355_pass_entry(float* x, void* h, const void* y, int64_t y_stride, const float* table, const int64_t* ids, int64_t vocab,
                      const float* step, const void* w_next, int64_t tokens, int64_t hidden, float eps, int dtype, void* stream);
 

@@ -134,6 +134,10 @@ __global__ __launch_bounds__(256) void layernorm_shift_kernel(
 // b = sum_j coef[t][j] * y[rows[t][j]] (coef null: 1; rows null: y[t]) + sigmoid(gate[t]) * y2[t] (y2 null: nothing); N the layer
 // norm, or (RMS) the division by the root mean square.  KEEP > 0: the row stays in
 // registers, KEEP groups of eight features per thread (D <= 2048 KEEP, 16-byte accesses); KEEP 0: any D, the row in LDS.
+// part (KEEP > 0; with neither rows nor y2): y[t] are the sums over a decode product's splits [split][t][D], rounded to T.  Rows of up to
+// 4096 features have the stream and both weights on their way with y: a step of few tokens waits for memory once instead of three times.
+// (64 rows of 2048, eight splits: product 12.7 us with the sums in it and norm 4.7 before, 8.7 and 5.0 now; four splits 8.0 and 4.7, now 6.1
+// and 5.0.  More splits than a norm's rows can hide do not occur: a product has at most 16.)
 struct LnAddParams {
   float* x;
   void* h;
@@ -144,8 +148,9 @@ struct LnAddParams {
   const float* gate;
   const void* w_out;
   const void* w_next;
+  const float* part;
   int64_t y_stride, y2_stride, gate_stride, D;
-  int n_rows;
+  int n_rows, splits;
   float eps;
 };
 
@@ -246,14 +251,38 @@ __global__ __launch_bounds__(256) void layernorm_residual_add_kernel(const LnAdd
   T* h = static_cast<T*>(p.h) + t * D;
   const float sg = y2 != nullptr ? 1.0f / (1.0f + expf(-p.gate[t * p.gate_stride])) : 0.f;
   if constexpr (KEEP > 0) {
-    float v[KEEP][8];
+    constexpr int EARLY = KEEP <= 2 ? KEEP : 0;
+    float v[KEEP][8], xs[EARLY + 1][8], wo[EARLY + 1][8], wn[EARLY + 1][8];
+#pragma unroll
+    for (int g = 0; g < EARLY; ++g) {
+      const int64_t i = 8 * ((int64_t)threadIdx.x + 256 * g);
+      if (i >= D) continue;
+      ld8f<float>(xr + i, xs[g]);
+      ld8f<T>(w_out + i, wo[g]);
+      if (w_next != nullptr) ld8f<T>(w_next + i, wn[g]);
+    }
 #pragma unroll
     for (int g = 0; g < KEEP; ++g) {
       const int64_t i = 8 * ((int64_t)threadIdx.x + 256 * g);
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[g][k] = 0.f;
       if (i >= D) continue;
-      if (p.rows == nullptr) {
+      if (p.part != nullptr) {
+        const float* const src = p.part + t * D + i;
+        const int64_t split = (int64_t)gridDim.x * D;
+        for (int s0 = 0; s0 < p.splits; s0 += 8) {       // eight splits' loads in flight, the last one's again where there are fewer
+          float e[8][8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) ld8f<float>(src + min(s0 + u, p.splits - 1) * split, e[u]);
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (s0 + u < p.splits) v[g][k] += e[u][k];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[g][k] = round_to<T>(v[g][k]);
+      } else if (p.rows == nullptr) {
         ld8f<T>(y + t * p.y_stride + i, v[g]);
       } else {
         for (int j = 0; j < p.n_rows; ++j) {      // fixed order: the sum does not depend on where the rows lie
@@ -277,10 +306,12 @@ __global__ __launch_bounds__(256) void layernorm_residual_add_kernel(const LnAdd
       const int64_t i = 8 * ((int64_t)threadIdx.x + 256 * g);
       if (i >= D) continue;
       float w[8], r[8];
-      ld8f<T>(w_out + i, w);
-      ld8f<float>(xr + i, r);
+      if (EARLY == 0) {
+        ld8f<T>(w_out + i, w);
+        ld8f<float>(xr + i, r);
+      }
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[g][k] = r[k] + v[g][k] * w[k];
+      for (int k = 0; k < 8; ++k) v[g][k] = EARLY ? xs[g < EARLY ? g : 0][k] + v[g][k] * wo[g < EARLY ? g : 0][k] : r[k] + v[g][k] * w[k];
       st8f<float>(xr + i, v[g]);
       if (w_next == nullptr && p.h != nullptr) st8f<T>(h + i, v[g]);
     }
@@ -291,9 +322,9 @@ __global__ __launch_bounds__(256) void layernorm_residual_add_kernel(const LnAdd
       const int64_t i = 8 * ((int64_t)threadIdx.x + 256 * g);
       if (i >= D) continue;
       float w[8];
-      ld8f<T>(w_next + i, w);
+      if (EARLY == 0) ld8f<T>(w_next + i, w);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) w[k] *= v[g][k];
+      for (int k = 0; k < 8; ++k) w[k] = (EARLY ? wn[g < EARLY ? g : 0][k] : w[k]) * v[g][k];
       st8f<T>(h + i, w);
     }
   } else {
@@ -578,15 +609,16 @@ int mi355_gated_residual_add(float* x, const void* g1, const void* b1, const voi
 
 static int norm_residual_add(LnAddParams& p, int64_t tokens, int rms, int dtype, void* stream) {
   const int64_t hidden = p.D;
-  MI355_REQUIRE(p.x && p.y && p.w_out && (p.h != nullptr || p.w_next == nullptr), MI355_ERR_INVALID, "norm_residual_add: null pointer");
+  MI355_REQUIRE(p.x && (p.y || p.part) && p.w_out && (p.h != nullptr || p.w_next == nullptr), MI355_ERR_INVALID, "norm_residual_add: null pointer");
   MI355_REQUIRE((p.y2 == nullptr) == (p.gate == nullptr) && (p.rows == nullptr || p.n_rows > 0) && (p.coef == nullptr || p.rows != nullptr),
                 MI355_ERR_INVALID, "norm_residual_add: the second branch comes with its gate, picked rows with their count, factors with rows");
   MI355_REQUIRE(tokens >= 0 && tokens < (1ll << 31) && hidden > 0 && hidden <= 32768 && p.y_stride >= hidden &&
                     (p.y2 == nullptr || p.y2_stride >= hidden), MI355_ERR_INVALID, "norm_residual_add: bad shape");
   if (tokens == 0) return MI355_OK;
-  const bool vec = hidden % 8 == 0 && hidden <= 8192 && p.y_stride % 8 == 0 && aligned16(p.x) && aligned16(p.y) && aligned16(p.w_out) &&
+  const bool vec = hidden % 8 == 0 && hidden <= 8192 && p.y_stride % 8 == 0 && aligned16(p.x) && aligned16(p.y) && aligned16(p.part) && aligned16(p.w_out) &&
                    (p.h == nullptr || aligned16(p.h)) && (p.w_next == nullptr || aligned16(p.w_next)) &&
                    (p.y2 == nullptr || (aligned16(p.y2) && p.y2_stride % 8 == 0));
+  MI355_REQUIRE(p.part == nullptr || (vec && p.splits > 0), MI355_ERR_UNSUPPORTED, "norm_residual_add: split sums of rows of whole 16-byte pieces up to 8192");
   const dim3 grid((unsigned)tokens), block(256);
   const int keep = !vec ? 0 : hidden <= 2048 ? 1 : hidden <= 4096 ? 2 : 4;
   const size_t lds = keep == 0 ? (size_t)hidden * sizeof(float) : 0;
@@ -613,6 +645,7 @@ int mi355_layernorm_residual_add(float* x, void* h, const void* y, int64_t y_str
   LnAddParams p;
   p.x = x; p.h = h; p.y = y; p.rows = rows; p.coef = nullptr; p.y2 = y2; p.gate = y2_gate; p.w_out = w_out; p.w_next = w_next;
   p.y_stride = y_stride; p.y2_stride = y2_stride; p.gate_stride = gate_stride; p.D = hidden; p.n_rows = n_rows; p.eps = eps;
+  p.part = nullptr; p.splits = 0;
   return norm_residual_add(p, tokens, 0, dtype, stream);
 }
 
@@ -622,7 +655,18 @@ int mi355_rmsnorm_residual_add_next(float* x, void* h, const void* y, int64_t y_
   LnAddParams p;
   p.x = x; p.h = h; p.y = y; p.rows = rows; p.coef = coef; p.y2 = nullptr; p.gate = nullptr; p.w_out = w_out; p.w_next = w_next;
   p.y_stride = y_stride; p.y2_stride = 0; p.gate_stride = 0; p.D = hidden; p.n_rows = n_rows; p.eps = eps;
+  p.part = nullptr; p.splits = 0;
   return norm_residual_add(p, tokens, 1, dtype, stream);
+}
+
+int mi355_norm_residual_add_partials(float* x, void* h, const float* part, int splits, const void* w_out, const void* w_next, int64_t tokens,
+                                     int64_t hidden, float eps, int rms, int dtype, void* stream) {
+  MI355_REQUIRE(part != nullptr && splits > 0, MI355_ERR_INVALID, "norm_residual_add_partials: no split sums");
+  LnAddParams p;
+  p.x = x; p.h = h; p.y = nullptr; p.rows = nullptr; p.coef = nullptr; p.y2 = nullptr; p.gate = nullptr; p.w_out = w_out; p.w_next = w_next;
+  p.y_stride = hidden; p.y2_stride = 0; p.gate_stride = 0; p.D = hidden; p.n_rows = 0; p.eps = eps;
+  p.part = part; p.splits = splits;
+  return norm_residual_add(p, tokens, rms, dtype, stream);
 }
 
 int mi355_pass_entry(float* x, void* h, const void* y, int64_t y_stride, const float* table, const int64_t* ids, int64_t vocab,

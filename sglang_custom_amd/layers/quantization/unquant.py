@@ -152,6 +152,12 @@ class PendingAllReduce:
         return self.partial.dtype
 
 
+def linear_for_norm(layer, x: torch.Tensor):
+    """layer(x) for a post-norm that sums a decode product's splits itself (SplitKPartials), the tensor where there are none."""
+    y = decode_linear_deferred(layer, x) if layer.weight.shape[0] % 8 == 0 and layer.weight.shape[0] <= 8192 else None
+    return layer(x)[0] if y is None else y
+
+
 def decode_linear_deferred(layer, x, needs_all_reduce: bool = True):
     """layer(x) on the decode path, leaving the split-K reduction to the kernel that consumes it; None
     when the layer, the shape or the ops backend does not support it.  A row-parallel layer

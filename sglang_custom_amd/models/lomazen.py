@@ -40,7 +40,7 @@ from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import PassEntry, RMSNormResidualAdd
 from ..layers.pre_norm import OffsetRMSNorm
 from ..layers.rotary_embedding import banded_pair_inv_freq
-from ..layers.quantization.unquant import SKINNY_MAX_M, pack_for_decode, pack_gate_up_for_decode
+from ..layers.quantization.unquant import SKINNY_MAX_M, linear_for_norm, pack_for_decode, pack_gate_up_for_decode
 from ..layers.vocab_parallel_embedding import ParallelLMHead
 from ..ops_backend import get_ops
 
@@ -78,7 +78,7 @@ class LomazenAttention(nn.Module):
         q = self.attn.rotate_and_write(p[:, :nq], p[:, nq: nq + nk], p[:, nq + nk: nq + nk + nv], positions, forward_batch, run)
         o = torch.empty((T, self.H, self.dv), dtype=h.dtype, device=h.device)
         self.attn(q, forward_batch, o, run, gate=p[:, nq + nk + nv: nq + nk + nv + ng])
-        return self.o_proj(o.view(T, self.H * self.dv))[0]
+        return linear_for_norm(self.o_proj, o.view(T, self.H * self.dv))
 
 
 class LomazenMLP(nn.Module):
@@ -94,7 +94,7 @@ class LomazenMLP(nn.Module):
         wp = getattr(self.gate_up, "weight_packed_gate_up", None)
         if wp is not None and h.shape[0] <= SKINNY_MAX_M and h.stride(0) % 8 == 0:
             # a decode step: the unit in the product's epilogue (the dense layers of 64 rows 452 -> 443 us a step: a launch and 2 passes over [rows, ff] each)
-            return dict(y=self.down(get_ops().linear_packed_silu_mul(h, wp, 2 * self.ff, act="gelu_tanh"))[0])
+            return dict(y=linear_for_norm(self.down, get_ops().linear_packed_silu_mul(h, wp, 2 * self.ff, act="gelu_tanh")))
         gu = self.gate_up(h)[0]
         return dict(y=self.down(self.act(gu[:, : self.ff], gu[:, self.ff:]))[0])
 

@@ -43,7 +43,7 @@ from ..layers.linear_recurrence import HeadNormGate, MatrixMemory
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import LayerNormResidualAdd
-from ..layers.quantization.unquant import pack_for_decode, prefill_linear
+from ..layers.quantization.unquant import linear_for_norm, pack_for_decode, prefill_linear
 from ..layers.rotary_embedding import scaled_pair_inv_freq
 from ..layers.token_shift import ShiftedLayerNorm
 from ..layers.vocab_parallel_embedding import ParallelLMHead
@@ -77,11 +77,11 @@ class SilatarLatentAttention(nn.Module):
             # nothing cached: keys and values per head cost less than scores and sums in the latent space
             expand = lambda c: prefill_linear(c, self.kv_expand).view(T, H, self.dn + self.dv)
             o = forward_batch.attn_backend.forward_latent_prefill(q, expand, self.attn, forward_batch, cache_layer=run)
-            return self.o_proj(o.view(T, H * self.dv))[0]
+            return linear_for_norm(self.o_proj, o.view(T, H * self.dv))
         qa = self.uk(q[..., : self.dn])
         o_lat = torch.empty((H, T, self.rank), dtype=h.dtype, device=h.device).transpose(0, 1)
         self.attn(qa, q[..., self.dn:], None, forward_batch, o_lat, cache_layer=run)
-        return self.o_proj(self.uv(o_lat).reshape(T, H * self.dv))[0]
+        return linear_for_norm(self.o_proj, self.uv(o_lat).reshape(T, H * self.dv))
 
 
     def process_weights_after_loading(self) -> None:
@@ -107,7 +107,7 @@ class SilatarMatrixMemory(nn.Module):
         q, k = p[:, : H * d].view(T, H, d), p[:, H * d: 2 * H * d].view(T, H, d)
         v = p[:, 2 * H * d: 2 * H * d + H * dv].view(T, H, dv)
         o = self.memory(q, k, v, gates, forward_batch, cache_layer=run)
-        return self.o_proj(self.norm_gate(o, p[:, 2 * H * d + H * dv:]))[0]
+        return linear_for_norm(self.o_proj, self.norm_gate(o, p[:, 2 * H * d + H * dv:]))
 
 
 class SilatarMLP(nn.Module):
@@ -119,7 +119,7 @@ class SilatarMLP(nn.Module):
 
     def forward(self, h):
         """-> what LayerNormResidualAdd takes besides the stream and the next norm."""
-        return dict(y=self.down(self.act(self.up(h)[0]))[0])
+        return dict(y=linear_for_norm(self.down, self.act(self.up(h)[0])))
 
 
 class SilatarMoE(nn.Module):

@@ -2233,6 +2233,21 @@ def rmsnorm_residual_add_next(x: torch.Tensor, y: torch.Tensor, w_out: torch.Ten
     return h
 
 
+def norm_residual_add_partials(x: torch.Tensor, part: torch.Tensor, w_out: torch.Tensor, w_next: Optional[torch.Tensor], eps: float,
+                               rms: bool) -> Optional[torch.Tensor]:
+    """rmsnorm_residual_add_next with copy (rms) or layernorm_residual_add with y = the sum of a decode product's splits, part fp32
+    [splits, T, D], rounded to the weights' dtype: the same bits as of the summed product."""
+    _gpu(x, part, w_out, w_next)
+    T, D = x.shape
+    assert x.dtype == torch.float32 and x.is_contiguous() and part.dtype == torch.float32 and part.is_contiguous() and part.shape[1:] == (T, D)
+    for w in (w_out, w_next):
+        assert w is None or (w.dtype == w_out.dtype and w.numel() == D and w.is_contiguous())
+    h = torch.empty((T, D), dtype=w_out.dtype, device=x.device) if (w_next is not None or rms) else None
+    check(_lib_().mi355_norm_residual_add_partials(x.data_ptr(), _p(h), part.data_ptr(), part.shape[0], w_out.data_ptr(), _p(w_next), T, D,
+                                                   float(eps), int(rms), _dt(w_out), _stream(x)), "norm_residual_add_partials")
+    return h
+
+
 def pass_entry(x: torch.Tensor, y: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, step: torch.Tensor, w_next: torch.Tensor,
                eps: float) -> torch.Tensor:
     """x = y + table[ids] + step in place of what the fp32 rows held; returns x over its root mean square times w_next."""

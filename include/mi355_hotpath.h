@@ -503,6 +503,11 @@ int mi355_linear_packed(void* y, const void* x, const void* w_packed, const void
 int mi355_fp8_packed_splits(int64_t m, int64_t n, int64_t k);
 int mi355_fp8_packed_partials(float* part, const uint8_t* xq, const uint8_t* wq_packed, int64_t m, int64_t n,
                               int64_t k, void* stream);
+/* mi355_per_token_quant_fp8 and mi355_fp8_packed_partials in one launch, for x [m, k] in 16 bits (rows x_stride apart): partials
+ * [mi355_fp8_quant_packed_splits][m][n] and scales [m], the same bits.  _splits 0: not served. */
+int mi355_fp8_quant_packed_splits(int64_t m, int64_t n, int64_t k);
+int mi355_fp8_quant_packed_partials(float* part, float* scales, const void* x, int64_t x_stride, const uint8_t* wq_packed, int64_t m, int64_t n,
+                                    int64_t k, int dtype, void* stream);
 int mi355_rmsnorm_ex(void* out, const void* x, void* residual, const void* weight, const float* part,
                      int nsplit, const float* part_x_scale, const float* part_w_scale, uint8_t* q_out,
                      float* q_scale, int64_t rows, int64_t hidden, float eps, int dtype, void* stream);

@@ -60,6 +60,8 @@ _SIGNATURES = {
     "mi355_mla_prefill_assemble": (I, [P, P, P, P, P, L, P, L, P, P, I, I, P, P, L, I, I, I, I, I, L, L, I, P]),
     "mi355_linear_packed": (I, [P, P, P, P, L, L, L, L, P, L, I, I, P]),
     "mi355_linear_packed_silu_mul": (I, [P, P, P, L, L, L, L, P, L, I, P]),
+    "mi355_fp8_quant_packed_splits": (I, [L, L, L]),
+    "mi355_fp8_quant_packed_partials": (I, [P, P, P, L, P, L, L, L, I, P]),
     "mi355_linear_packed_scaled": (I, [P, P, P, F, L, L, L, L, P, L, I, P]),
     "mi355_linear_packed_act_mul": (I, [P, P, P, L, L, L, L, P, L, I, I, P]),
     "mi355_linear_tiled_supported": (I, [L, L, L, I, I]),

@@ -1105,6 +1105,104 @@ static SkinnyPlan plan_fp8(int64_t m, int64_t n, int64_t k) {
   return p;
 }
 
+// The quantisation of few 16-bit rows (at most 8 of at most 4096) inside the product behind it: every workgroup reads all of them, whose largest
+// values are a row's scale, and keeps its own range of K as fp8 in LDS while its first weights are on their way.  us,
+// quantisation and product | this: 4096 x 4096 with 1 row 6.9 | 4.6, 4 7.0 | 4.7, 8 7.2 | 5.6, 12 7.5 | 7.3, 16 7.4 | 7.4 (128 KB of rows a workgroup; four
+// more waves for the rows: 7.3, and a microsecond more at few rows); 8192 x 4096 with 1 10.6 | 8.0, 8 10.8 | 8.5; 4096 x 2048 7.7 | 5.2, 7.9 | 5.9.
+struct QuantLinearParams {
+  const void* x;          // [M][K], rows x_stride apart
+  const uint8_t* w;       // packed
+  float* part;            // [splits][M][N]
+  float* scales;          // [M]
+  int64_t x_stride;
+  int M, N, K, k_per_split;
+};
+template <typename T, int RPW, int CH>
+__global__ __launch_bounds__(512) void quant_linear_kernel(QuantLinearParams p) {
+  using frag = typename Mfma<fp8_t>::frag;
+  constexpr int S = 8, BK = 512;     // fragment steps of a chunk of K
+  constexpr float FP8_MAX = 448.0f;
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];       // [M][k_per_split + 32]: rows' fragments in other banks
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int r16 = lane & 15, q = lane >> 4, row_len = p.k_per_split + 32, nvec = p.K >> 3;
+  const int real_tile = (int)blockIdx.x * waves + wave, tile = min(real_tile, ((p.N + 63) >> 6) * 4 - 1);
+  const int ks = blockIdx.y * p.k_per_split, ke = min(p.K, ks + p.k_per_split), nchunks = (ke - ks) / BK;
+  const uint8_t* const wrow = p.w + (((int64_t)(tile >> 2) * (p.K / 64) * 4 + (tile & 3)) * 64 + lane) * 16 + (int64_t)ks * 64;
+  frag w0[S], w1[S], w2[S];
+  auto load_w = [&](frag (&dst)[S], int chunk) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      dst[s] = __builtin_nontemporal_load(reinterpret_cast<const frag*>(wrow + (int64_t)(chunk * BK + s * 64) * 64));
+  };
+  // wave w has rows RPW w and on (past the last: the last again, the same bytes to the same place)
+  Vec<T, 8> v[RPW][CH];
+#pragma unroll
+  for (int r = 0; r < RPW; ++r)
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      v[r][j] = ldvec<T, 8>((const T*)p.x + (int64_t)min(wave * RPW + r, p.M - 1) * p.x_stride + (int64_t)min(lane + 64 * j, nvec - 1) * 8);
+  __builtin_amdgcn_sched_barrier(0);
+  load_w(w0, 0);
+  load_w(w1, nchunks > 1 ? 1 : 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < RPW; ++r) {
+    const int row = min(wave * RPW + r, p.M - 1);
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(to_f32(v[r][j].v[k])));
+    const float sc = fmaxf(wave_max(amax), 1e-10f) / FP8_MAX, inv = 1.0f / sc;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && lane == 0) p.scales[row] = sc;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k0 = (lane + 64 * j) * 8;
+      if (k0 < ks || k0 >= ke) continue;
+      unsigned out[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float f[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f[k] = fminf(fmaxf(to_f32(v[r][j].v[4 * h + k]) * inv, -FP8_MAX), FP8_MAX);
+        int pk = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+        pk = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], pk, true);
+        out[h] = (unsigned)pk;
+      }
+      *reinterpret_cast<uint2*>(smem_raw + row * row_len + k0 - ks) = uint2{out[0], out[1]};
+    }
+  }
+  __syncthreads();
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  const char* const xt = smem_raw + min(r16, p.M - 1) * row_len + q * 16;     // (fragment rows past the last: their results are not stored)
+  auto compute = [&](const frag (&wc)[S], int chunk) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc = Mfma<fp8_t>::run(wc[s], *reinterpret_cast<const frag*>(xt + chunk * BK + s * 64), acc);
+  };
+  int c = 0;
+  for (; c + 2 < nchunks; ++c) {
+    load_w(w2, c + 2);
+    compute(w0, c);
+#pragma unroll
+    for (int s = 0; s < S; ++s) { w0[s] = w1[s]; w1[s] = w2[s]; }
+  }
+  compute(w0, c);
+  if (c + 1 < nchunks) compute(w1, c + 1);
+  const int n0 = real_tile * 16 + 4 * q;
+  if (r16 < p.M && n0 < p.N) *reinterpret_cast<f32x4*>(p.part + ((int64_t)blockIdx.y * p.M + r16) * p.N + n0) = acc;
+}
+
+template <typename T>
+static void launch_quant_linear(const QuantLinearParams& p, const SkinnyPlan& plan, hipStream_t st) {
+  const int rpw = (p.M + plan.waves - 1) / plan.waves;
+  const bool wide = p.K > 2048;
+  void (*kern)(QuantLinearParams) = rpw <= 1 ? (wide ? quant_linear_kernel<T, 1, 8> : quant_linear_kernel<T, 1, 4>)
+                                             : (wide ? quant_linear_kernel<T, 2, 8> : quant_linear_kernel<T, 2, 4>);
+  const size_t lds = (size_t)p.M * (p.k_per_split + 32);
+  if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(kern, dim3((unsigned)plan.nblocks, (unsigned)plan.splits), dim3(64 * plan.waves), lds, st, p);
+}
+
 template <typename OUT, int MT>
 static void launch_fp8_mt(const fp8_t* x, const fp8_t* w, const void* bias, OUT* y, char* ws, int M, int N,
                           int K, const SkinnyPlan& p, const float* xs, const float* wsc, hipStream_t st,
@@ -1410,6 +1508,27 @@ int mi355_fp8_scaled_mm_packed(void* y, const uint8_t* xq, const uint8_t* wq_pac
 int mi355_fp8_packed_splits(int64_t m, int64_t n, int64_t k) {
   if (m < 1 || m > 64 || n < 1 || n >= 64 * 1024 || k < 512 || k % 512 != 0 || g_gemm_variant != 0) return 0;
   return plan_fp8(m, n, k).splits;
+}
+
+int mi355_fp8_quant_packed_splits(int64_t m, int64_t n, int64_t k) {
+  if (m < 1 || m > 8 || n % 4 != 0 || k > 4096) return 0;
+  return mi355_fp8_packed_splits(m, n, k);
+}
+
+int mi355_fp8_quant_packed_partials(float* part, float* scales, const void* x, int64_t x_stride, const uint8_t* wq_packed, int64_t m, int64_t n,
+                                    int64_t k, int dtype, void* stream) {
+  MI355_REQUIRE(part && scales && x && wq_packed, MI355_ERR_INVALID, "fp8_quant_packed_partials: null pointer");
+  MI355_REQUIRE(mi355_fp8_quant_packed_splits(m, n, k) > 0 && (dtype == MI355_BF16 || dtype == MI355_F16), MI355_ERR_UNSUPPORTED,
+                "fp8_quant_packed_partials: 16-bit rows, 1 <= M <= 8, N %% 4 == 0, K %% 512 == 0, K <= 4096 (m=%lld n=%lld k=%lld)",
+                (long long)m, (long long)n, (long long)k);
+  MI355_REQUIRE(x_stride >= k && x_stride % 8 == 0 && aligned16(x) && aligned16(wq_packed) && aligned16(part), MI355_ERR_INVALID,
+                "fp8_quant_packed_partials: misaligned pointer");
+  const SkinnyPlan plan = plan_fp8(m, n, k);
+  const QuantLinearParams p{x, wq_packed, part, scales, x_stride, (int)m, (int)n, (int)k, (int)plan.k_per_split};
+  if (dtype == MI355_BF16) launch_quant_linear<bf16_t>(p, plan, (hipStream_t)stream);
+  else launch_quant_linear<f16_t>(p, plan, (hipStream_t)stream);
+  MI355_CHECK_LAUNCH("fp8_quant_packed_partials");
+  return MI355_OK;
 }
 
 int mi355_fp8_packed_partials(float* part, const uint8_t* xq, const uint8_t* wq_packed, int64_t m, int64_t n,

@@ -175,6 +175,8 @@ def decode_linear_deferred(layer, x, needs_all_reduce: bool = True):
         if isinstance(x, QuantizedAct):
             xq, xs = x.xq, x.x_scale
         else:
+            if layer.k_padded == x.shape[1] and (fused := ops.fp8_quant_packed_partials(x, wp, n)) is not None:
+                return SplitKPartials(fused[0], fused[1], layer.weight_scale.data)
             xq, xs = ops.per_token_quant_fp8(x, pad_to=layer.k_padded)
         if xq.shape[1] != layer.k_padded:
             return None

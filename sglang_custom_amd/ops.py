@@ -1015,6 +1015,20 @@ def fp8_packed_partials(xq: torch.Tensor, wq_packed: torch.Tensor, n: int) -> Op
     return part
 
 
+def fp8_quant_packed_partials(x: torch.Tensor, wq_packed: torch.Tensor, n: int) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """per_token_quant_fp8 and fp8_packed_partials in one launch for few 16-bit rows: (partials, scales [M, 1]); None when not served."""
+    _gpu(x, wq_packed)
+    m, k = x.shape
+    splits = _lib_().mi355_fp8_quant_packed_splits(m, n, k) if x.dtype in (torch.bfloat16, torch.float16) else 0
+    if splits <= 0 or x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0:
+        return None
+    part = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+    scales = torch.empty((m, 1), dtype=torch.float32, device=x.device)
+    check(_lib_().mi355_fp8_quant_packed_partials(part.data_ptr(), scales.data_ptr(), x.data_ptr(), x.stride(0), wq_packed.data_ptr(), m, n, k,
+                                                  _dt(x), _stream(x)), "fp8_quant_packed_partials")
+    return part, scales
+
+
 def rmsnorm_ex(weight: torch.Tensor, eps: float, x: Optional[torch.Tensor] = None,
                residual: Optional[torch.Tensor] = None, part: Optional[torch.Tensor] = None,
                part_x_scale: Optional[torch.Tensor] = None, part_w_scale: Optional[torch.Tensor] = None,

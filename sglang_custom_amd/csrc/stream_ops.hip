@@ -134,8 +134,10 @@ __global__ __launch_bounds__(256) void layernorm_shift_kernel(
 // b = sum_j coef[t][j] * y[rows[t][j]] (coef null: 1; rows null: y[t]) + sigmoid(gate[t]) * y2[t] (y2 null: nothing); N the layer
 // norm, or (RMS) the division by the root mean square.  KEEP > 0: the row stays in
 // registers, KEEP groups of eight features per thread (D <= 2048 KEEP, 16-byte accesses); KEEP 0: any D, the row in LDS.
-// part (KEEP > 0; with neither rows nor y2): y[t] are the sums over a decode product's splits [split][t][D], rounded to T.  Rows of up to
+// PART (KEEP > 0; with neither rows nor y2): y[t] are the sums over a decode product's splits [split][t][D], rounded to T.  Rows of up to
 // 4096 features have the stream and both weights on their way with y: a step of few tokens waits for memory once instead of three times.
+// Its registers stay out of the other form, whose thousands of rows hide the waits by their number (a prompt of 7400 rows of 2048 lost 3 us a
+// norm with them).
 // (64 rows of 2048, eight splits: product 12.7 us with the sums in it and norm 4.7 before, 8.7 and 5.0 now; four splits 8.0 and 4.7, now 6.1
 // and 5.0.  More splits than a norm's rows can hide do not occur: a product has at most 16.)
 struct LnAddParams {
@@ -239,7 +241,7 @@ __device__ __forceinline__ void ln_lds(float* buf, int64_t D, float eps, float* 
   for (int64_t i = threadIdx.x; i < D; i += 256) buf[i] = (buf[i] - mean) * inv;
 }
 
-template <typename T, int KEEP, bool RMS>
+template <typename T, int KEEP, bool RMS, bool PART>
 __global__ __launch_bounds__(256) void layernorm_residual_add_kernel(const LnAddParams p) {
   __shared__ float red[16];
   const int64_t t = blockIdx.x, D = p.D;
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(256) void layernorm_residual_add_kernel(const LnAdd
   T* h = static_cast<T*>(p.h) + t * D;
   const float sg = y2 != nullptr ? 1.0f / (1.0f + expf(-p.gate[t * p.gate_stride])) : 0.f;
   if constexpr (KEEP > 0) {
-    constexpr int EARLY = KEEP <= 2 ? KEEP : 0;
+    constexpr int EARLY = PART && KEEP <= 2 ? KEEP : 0;
     float v[KEEP][8], xs[EARLY + 1][8], wo[EARLY + 1][8], wn[EARLY + 1][8];
 #pragma unroll
     for (int g = 0; g < EARLY; ++g) {
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(256) void layernorm_residual_add_kernel(const LnAdd
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[g][k] = 0.f;
       if (i >= D) continue;
-      if (p.part != nullptr) {
+      if constexpr (PART) {
         const float* const src = p.part + t * D + i;
         const int64_t split = (int64_t)gridDim.x * D;
         for (int s0 = 0; s0 < p.splits; s0 += 8) {       // eight splits' loads in flight, the last one's again where there are fewer
@@ -622,18 +624,20 @@ static int norm_residual_add(LnAddParams& p, int64_t tokens, int rms, int dtype,
   const dim3 grid((unsigned)tokens), block(256);
   const int keep = !vec ? 0 : hidden <= 2048 ? 1 : hidden <= 4096 ? 2 : 4;
   const size_t lds = keep == 0 ? (size_t)hidden * sizeof(float) : 0;
+#define LN_ADD(KEEP, PART) go(rms ? layernorm_residual_add_kernel<T, KEEP, true, PART> : layernorm_residual_add_kernel<T, KEEP, false, PART>)
   MI355_DISPATCH_DTYPE(dtype, "norm_residual_add", {
     auto go = [&](auto kern) {
       if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       hipLaunchKernelGGL(kern, grid, block, lds, (hipStream_t)stream, p);
     };
     switch (keep) {
-      case 1: go(rms ? layernorm_residual_add_kernel<T, 1, true> : layernorm_residual_add_kernel<T, 1, false>); break;
-      case 2: go(rms ? layernorm_residual_add_kernel<T, 2, true> : layernorm_residual_add_kernel<T, 2, false>); break;
-      case 4: go(rms ? layernorm_residual_add_kernel<T, 4, true> : layernorm_residual_add_kernel<T, 4, false>); break;
-      default: go(rms ? layernorm_residual_add_kernel<T, 0, true> : layernorm_residual_add_kernel<T, 0, false>); break;
+      case 1: if (p.part) LN_ADD(1, true); else LN_ADD(1, false); break;
+      case 2: if (p.part) LN_ADD(2, true); else LN_ADD(2, false); break;
+      case 4: if (p.part) LN_ADD(4, true); else LN_ADD(4, false); break;
+      default: LN_ADD(0, false); break;
     }
   });
+#undef LN_ADD
   MI355_CHECK_LAUNCH("norm_residual_add");
   return MI355_OK;
 }

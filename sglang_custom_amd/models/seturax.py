@@ -120,7 +120,7 @@ class SeturaxModel(nn.Module):
 
 class SeturaxForCausalLM(nn.Module):
     needs_sequence_state = True
-    supports_hip_graph = False    # a captured decode step pads the batch with row 0 of the request table, whose state slot it would overwrite
+    supports_hip_graph = False    # (its steps have not been run captured)
 
     def __init__(self, config, dtype=torch.bfloat16, device="cuda", quant_method_factory=None):
         super().__init__()

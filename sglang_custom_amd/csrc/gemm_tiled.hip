@@ -97,7 +97,7 @@ template <bool FP8> __device__ __forceinline__ int gt_swz(int r) {
 
 // T: output dtype and, for 16-bit GEMMs, the operand dtype.  FP8: operands are OCP e4m3fn bytes.
 // EPI 0: y = T(acc (+ bias)); EPI 1: W = [gate; up] (N = 2 I rows), y[m, j] = silu_mul(T(gate_j), T(up_j));
-// fp8: acc is first scaled, (acc * x_scale[m]) * w_scale[n].
+// EPI 4: y = T(gelu_erf(T(acc))); EPI 5: as EPI 1 with y[m, j] = T(gelu_tanh(T(gate_j)) T(up_j)).  fp8: acc is first scaled, (acc * x_scale[m]) * w_scale[n].
 // Epilogue of the qkv projection (EPI 2): neox RoPE over the whole 128-wide head on the q and k heads with
 // the rounding points of mi355_rope_inplace (cos / sin -> T; every product and sum rounds to T on its own, so
 // no contraction here); rotated q / k and plain v go to y, the k and v rows also to the KV cache.
@@ -221,7 +221,8 @@ __device__ __forceinline__ void tile_of(const GemmTiledParams& p, int at, int& t
 // nearest to exp(x^2) erfc(x) / 2 over x in [0, 14] (fitted here to the least relative error, 1.1e-7); above zero z - z Phi(-z).  In fp32 its largest error
 // is half of 0.5 z (1 + erff(z / sqrt 2))'s over [-8, 8] (2.4e-7; below -3, where 1 + erf cancels, it stays at 3e-6 of the result),
 // rounded to 16 bits they have the same error to six digits.  Fifteen instructions and two of a quarter rate for erff's forty, which nothing
-// covers in an epilogue: 32 experts' first product of 3000 x 4 rows, 2048 x 2048, 140 -> 131 us (113 without it).
+// covers in an epilogue: 32 experts' first product of 3000 x 4 rows, 2048 x 2048, 140 -> 131 us (113 without it); a dense one of 7725 x 8192
+// columns, K 2048, about 45 us longer with it, for a launch of 61 to 67 of its own (4 TB/s).
 __device__ __forceinline__ float gelu_erf(float z) {
   const float u = fabsf(z), t = __builtin_amdgcn_rcpf(fmaf(0.29698484809834996f, u, 1.0f));
   float p = 3.71014210e-02f;
@@ -237,13 +238,22 @@ __device__ __forceinline__ float gelu_erf(float z) {
   return z > 0.f ? fmaf(-fminf(z, 30.f), h, z) : z * h;     // (infinity: itself; minus infinity and NaN: NaN, as by the formula)
 }
 
+// z / 2 (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))) as z / (1 + e^(-2 ..)): nothing cancels below zero, and two instructions of a quarter rate for
+// tanhf's thirty.  In the product's epilogue for a launch and two passes over the columns: a prompt of 4 x 1800 tokens through four layers of
+// 2 x 5632 columns 3625 -> 3455 us in all, 3 x 360 1065 -> 991.
+__device__ __forceinline__ float gelu_tanh_logistic(float z) {
+  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.3022081985f * fmaf(0.044715f * z * z, z, z)));
+}
+
+constexpr bool gt_pairs(int epi) { return epi == 1 || epi == 5; }   // W = [gate; up]
+
 // The results of NM groups of 16 rows (row mbase + 16 mi + r16 is lane (q4, r16)'s in group mi; mbase: the first group's first row).
 // acc[mi][ni][r]: W slot 16 ni + 4 q4 + r of the wave's 64, which the load mapping made output column 16 q4 + 4 ni + r (plain) or
 // gate / up column 8 q4 + 4 (ni & 1) + r.  EPI 3: `live` rows of the tile are no padding.
 template <typename T, int EPI, bool FP8, int NM>
 __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], int m0, int tm, int tn, int wc, int q4, int r16,
                                               int live) {
-  const int ncols = EPI == 1 ? (p.N >> 1) : p.N;   // output columns
+  const int ncols = gt_pairs(EPI) ? (p.N >> 1) : p.N;   // output columns
   const int mbase = m0 + r16;
   T* yg = (T*)p.y;
   const T* bias = (const T*)p.bias;
@@ -256,7 +266,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
   if constexpr (EPI == 2) {
     if (p.cs_f32) qkv_rope_epilogue<T, FP8, true, NM>(p, acc, sxm, mbase, tn, wc, q4);
     else qkv_rope_epilogue<T, FP8, false, NM>(p, acc, sxm, mbase, tn, wc, q4);
-  } else if (EPI == 1) {
+  } else if (gt_pairs(EPI)) {
     const int j0 = tn * 128 + wc * 32 + q4 * 8;
     if (j0 < ncols) {
       float sg[8], su[8];
@@ -275,7 +285,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
           for (int r = 0; r < 4; ++r) {
             float gv = acc[mi][h][r], uv = acc[mi][2 + h][r];
             if (FP8) { gv = (gv * sxm[mi]) * sg[h * 4 + r]; uv = (uv * sxm[mi]) * su[h * 4 + r]; }
-            o.v[h * 4 + r] = silu_mul_one<T>(from_f32<T>(gv), from_f32<T>(uv));
+            o.v[h * 4 + r] = EPI == 5 ? from_f32<T>(gelu_tanh_logistic(round_to<T>(gv)) * round_to<T>(uv)) : silu_mul_one<T>(from_f32<T>(gv), from_f32<T>(uv));
           }
         if (m < p.M) stvec<T, 8>(yg + (int64_t)m * p.ldy + j0, o);
       }
@@ -302,6 +312,10 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
           for (int r = 0; r < 4; ++r) {
             float v0 = acc[mi][ni][r], v1 = acc[mi][2 + ni][r];
             if (FP8) { v0 = (v0 * sxm[mi]) * sw[ni * 4 + r]; v1 = (v1 * sxm[mi]) * sw[8 + ni * 4 + r]; }
+            if constexpr (EPI == 4) {
+              v0 = gelu_erf(round_to<T>(v0));
+              v1 = gelu_erf(round_to<T>(v1));
+            }
             if constexpr (EPI == 3) {
               if (p.act == 1) {
                 v0 = gelu_erf(v0);
@@ -398,7 +412,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const char* xg = (const char*)p.x;
   const char* wg = (const char*)p.w;
   if constexpr (EPI == 3) wg += (int64_t)p.tile_expert[tm] * p.w_expert_stride * ES;
-  const int ncols = EPI == 1 ? (p.N >> 1) : p.N;   // output columns
+  const int ncols = gt_pairs(EPI) ? (p.N >> 1) : p.N;   // output columns
 
   // ---- per-lane source pointers of the eight load instructions a wave issues per K tile -----
   // A wave requests data only in its READ slot (a load-to-LDS holds the issuing wave ~40 cycles: in
@@ -430,7 +444,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
       xs[h] = xg + ((int64_t)m * p.ldx) * ES + c * 16;
       const int rb = h * 128 + rr, wcb = rb >> 6, sl = rb & 63, ni = sl >> 4, ii = sl & 15;
       int n;
-      if (EPI == 1) {
+      if (gt_pairs(EPI)) {
         int j = tn * 128 + wcb * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3);
         j = j < ncols ? j : ncols - 1;
         n = j + (ni >> 1) * ncols;
@@ -618,15 +632,17 @@ int launch_gemm_tiled(const GemmTiledParams& p, hipStream_t st) {
   return MI355_OK;
 }
 
+bool pairs(int epilogue) { return epilogue == 1 || epilogue == 3; }   // of an entry point: W = [gate; up]
+
 void fill_tiles(GemmTiledParams& p, int64_t m, int64_t n, int epilogue) {
   p.positions = nullptr; p.cos_sin = nullptr; p.cs_f32 = 0; p.hq = p.hkv = 0;
   p.k_buffer = p.v_buffer = nullptr; p.loc = nullptr; p.loc_i32 = 0; p.kv_slot = p.kv_head = 0;
   p.row_map = p.tile_expert = p.tiles_used = nullptr; p.gather = 0; p.w_expert_stride = 0; p.act = 0;
   p.full = p.tail = p.splits = 0; p.part = nullptr;
-  const int ncols = epilogue == 1 ? (int)(n / 2) : (int)n;
+  const int ncols = pairs(epilogue) ? (int)(n / 2) : (int)n;
   p.ldy = ncols;
   p.mt = cdiv(m, 256);
-  p.nt = epilogue == 1 ? cdiv(ncols, 128) : cdiv(ncols, 256);
+  p.nt = pairs(epilogue) ? cdiv(ncols, 128) : cdiv(ncols, 256);
   p.snt = cdiv(p.nt, 4);
   p.nsuper = cdiv(p.mt, 8) * p.snt;
 }
@@ -637,7 +653,7 @@ void fill_tiles(GemmTiledParams& p, int64_t m, int64_t n, int epilogue) {
 // 2 x 14336 columns, K 4096, 520 rows (80, 3) 168 -> 147, 1134 (48, 4) 262 -> 236, 1962 (128, 2) 373 -> 366.  Past half a round
 // (1353 rows of the last: 160 tiles) there is nobody to share with; 128 tiles of K 2048 gain less than the sums cost (101 either way).
 int plan_tail(int64_t m, int64_t n, int64_t kbytes, int epilogue) {
-  const int64_t tiles = cdiv(m, 256) * (epilogue == 1 ? cdiv(n / 2, 128) : cdiv(n, 256));
+  const int64_t tiles = cdiv(m, 256) * (pairs(epilogue) ? cdiv(n / 2, 128) : cdiv(n, 256));
   const int64_t kt = kbytes >> 7, tail = tiles % 256;
   if (tail == 0) return 0;
   int best = 0;
@@ -883,14 +899,14 @@ extern "C" int mi355_tiled_tail_splits(int64_t m, int64_t n, int64_t k, int fp8,
 }
 
 extern "C" int64_t mi355_tiled_tail_workspace_bytes(int64_t m, int64_t n, int64_t k, int fp8, int epilogue) {
-  const int64_t tail = (cdiv(m, 256) * (epilogue == 1 ? cdiv(n / 2, 128) : cdiv(n, 256))) % 256;
+  const int64_t tail = (cdiv(m, 256) * (pairs(epilogue) ? cdiv(n / 2, 128) : cdiv(n, 256))) % 256;
   return mi355_tiled_tail_splits(m, n, k, fp8, epilogue) * tail * 65536 * 4;
 }
 
 extern "C" int mi355_linear_tiled_supported(int64_t m, int64_t n, int64_t k, int dtype, int epilogue) {
   if (dtype != MI355_BF16 && dtype != MI355_F16) return 0;
   if (m < 1 || n < 16 || k < 128 || (k & 63) != 0 || m > (1 << 24) || n > (1 << 24)) return 0;
-  return ((epilogue == 0 || epilogue == 1) && n % 16 == 0) ? 1 : 0;   // silu-mul: 8 gate + 8 up columns per lane
+  return (epilogue >= 0 && epilogue <= 3 && n % 16 == 0) ? 1 : 0;   // silu-mul: 8 gate + 8 up columns per lane
 }
 
 extern "C" int mi355_linear_tiled(void* y, const void* x, const void* w, const void* bias, int64_t m,
@@ -911,7 +927,7 @@ extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, cons
   MI355_REQUIRE(aligned16(x) && aligned16(w) && aligned16(y) && (bias == nullptr || aligned16(bias)),
                 MI355_ERR_INVALID, "mi355_linear_tiled: pointers must be 16-byte aligned");
   MI355_REQUIRE(epilogue == 0 || bias == nullptr, MI355_ERR_UNSUPPORTED,
-                "mi355_linear_tiled: no bias with the SiLU-and-mul epilogue");
+                "mi355_linear_tiled: no bias with an activation in the epilogue");
   GemmTiledParams p;
   p.x = x; p.w = w; p.bias = bias; p.y = y;
   p.x_scale = nullptr; p.w_scale = nullptr;
@@ -920,6 +936,8 @@ extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, cons
   fill_tiles(p, m, n, epilogue);
   if (const int rc = set_tail(p, plan_tail(m, n, k * 2, epilogue), workspace, workspace_bytes, "mi355_linear_tiled_ws")) return rc;
   hipStream_t st = (hipStream_t)stream;
+  if (epilogue == 3) return dtype == MI355_BF16 ? launch_gemm_tiled<bf16_t, 5, false>(p, st) : launch_gemm_tiled<f16_t, 5, false>(p, st);
+  if (epilogue == 2) return dtype == MI355_BF16 ? launch_gemm_tiled<bf16_t, 4, false>(p, st) : launch_gemm_tiled<f16_t, 4, false>(p, st);
   if (dtype == MI355_BF16)
     return epilogue == 1 ? launch_gemm_tiled<bf16_t, 1, false>(p, st) : launch_gemm_tiled<bf16_t, 0, false>(p, st);
   return epilogue == 1 ? launch_gemm_tiled<f16_t, 1, false>(p, st) : launch_gemm_tiled<f16_t, 0, false>(p, st);
@@ -928,7 +946,7 @@ extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, cons
 extern "C" int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out_dtype, int epilogue);
 
 extern "C" int mi355_linear_few_supported(int64_t m, int64_t n, int64_t k, int fp8, int out_dtype, int epilogue) {
-  if (!(fp8 ? mi355_fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, epilogue) : mi355_linear_tiled_supported(m, n, k, out_dtype, epilogue))) return 0;
+  if (epilogue > 1 || !(fp8 ? mi355_fp8_scaled_mm_tiled_supported(m, n, k, out_dtype, epilogue) : mi355_linear_tiled_supported(m, n, k, out_dtype, epilogue))) return 0;
   return plan_few(m, n, k, fp8 != 0).shape >= 0 ? 1 : 0;
 }
 

@@ -154,7 +154,7 @@ class PendingAllReduce:
 
 def linear_for_norm(layer, x: torch.Tensor):
     """layer(x) for a post-norm that sums a decode product's splits itself (SplitKPartials), the tensor where there are none."""
-    y = decode_linear_deferred(layer, x) if layer.weight.shape[0] % 8 == 0 and layer.weight.shape[0] <= 8192 else None
+    y = decode_linear_deferred(layer, x) if x.shape[0] <= SKINNY_MAX_M and layer.weight.shape[0] % 8 == 0 and layer.weight.shape[0] <= 8192 else None
     return layer(x)[0] if y is None else y
 
 
@@ -195,6 +195,17 @@ def takes_norm_in_front(layer, packed, hidden, norm, silu_mul: bool = False) -> 
     return (DECODE_FUSION and isinstance(hidden, SplitKPartials) and hidden.x_scale is None and packed is not None and packed.is_cuda
             and isinstance(layer.quant_method, UnquantizedLinearMethod) and packed.dtype == norm.weight.dtype and getattr(layer, "bias", None) is None
             and hidden.part.shape[0] <= 8 and get_ops().norm_linear_packed_splits(hidden.shape[0], layer.weight.shape[0], hidden.shape[1], silu_mul) > 0)
+
+
+def prefill_linear_act(layer, x: torch.Tensor, act: str) -> Optional[torch.Tensor]:
+    """The unit act ("gelu_erf", or "gelu_tanh_mul" over [gate; up]) of layer(x) for 2-d rows and a layer without a bias, in the product's epilogue;
+    None where the 256 x 256 tiles do not serve the product."""
+    w = layer.weight
+    if not (x.shape[0] > FEW_MAX_M and x.is_cuda and _use_tiled(x.shape[0], w.shape[0], w.shape[0], w.shape[1], x.dtype, act == "gelu_tanh_mul")
+            and isinstance(layer.quant_method, UnquantizedLinearMethod) and getattr(layer, "bias", None) is None
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()):
+        return None
+    return get_ops().linear_tiled(x, w, None, split_tail=True, act=act)
 
 
 def prefill_linear(x2: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:

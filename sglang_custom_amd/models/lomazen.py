@@ -40,7 +40,7 @@ from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import PassEntry, RMSNormResidualAdd
 from ..layers.pre_norm import OffsetRMSNorm
 from ..layers.rotary_embedding import banded_pair_inv_freq
-from ..layers.quantization.unquant import SKINNY_MAX_M, linear_for_norm, pack_for_decode, pack_gate_up_for_decode
+from ..layers.quantization.unquant import SKINNY_MAX_M, linear_for_norm, pack_for_decode, pack_gate_up_for_decode, prefill_linear_act
 from ..layers.vocab_parallel_embedding import ParallelLMHead
 from ..ops_backend import get_ops
 
@@ -95,6 +95,9 @@ class LomazenMLP(nn.Module):
         if wp is not None and h.shape[0] <= SKINNY_MAX_M and h.stride(0) % 8 == 0:
             # a decode step: the unit in the product's epilogue (the dense layers of 64 rows 452 -> 443 us a step: a launch and 2 passes over [rows, ff] each)
             return dict(y=linear_for_norm(self.down, get_ops().linear_packed_silu_mul(h, wp, 2 * self.ff, act="gelu_tanh")))
+        a = prefill_linear_act(self.gate_up, h, "gelu_tanh_mul")
+        if a is not None:
+            return dict(y=self.down(a)[0])
         gu = self.gate_up(h)[0]
         return dict(y=self.down(self.act(gu[:, : self.ff], gu[:, self.ff:]))[0])
 
@@ -168,7 +171,7 @@ class LomazenModel(nn.Module):
 
 
 class LomazenForCausalLM(nn.Module):
-    supports_hip_graph = True     # padded rows of a captured step attend to the request table's row 0 and write the sink slot
+    supports_hip_graph = True     # padded rows of a captured step attend to and write the sink slot
 
     def __init__(self, config, dtype=torch.bfloat16, device="cuda", quant_method_factory=None):
         super().__init__()

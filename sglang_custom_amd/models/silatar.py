@@ -43,7 +43,7 @@ from ..layers.linear_recurrence import HeadNormGate, MatrixMemory
 from ..layers.logits_processor import LogitsProcessor
 from ..layers.moe import GroupedExperts, GroupedTopKRouter
 from ..layers.post_norm import LayerNormResidualAdd
-from ..layers.quantization.unquant import linear_for_norm, pack_for_decode, prefill_linear
+from ..layers.quantization.unquant import linear_for_norm, pack_for_decode, prefill_linear, prefill_linear_act
 from ..layers.rotary_embedding import scaled_pair_inv_freq
 from ..layers.token_shift import ShiftedLayerNorm
 from ..layers.vocab_parallel_embedding import ParallelLMHead
@@ -119,7 +119,8 @@ class SilatarMLP(nn.Module):
 
     def forward(self, h):
         """-> what LayerNormResidualAdd takes besides the stream and the next norm."""
-        return dict(y=linear_for_norm(self.down, self.act(self.up(h)[0])))
+        a = prefill_linear_act(self.up, h, "gelu_erf")
+        return dict(y=linear_for_norm(self.down, self.act(self.up(h)[0]) if a is None else a))
 
 
 class SilatarMoE(nn.Module):

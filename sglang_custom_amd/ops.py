@@ -795,23 +795,30 @@ def _tail_workspace(split_tail: bool, m: int, n: int, k: int, fp8: bool, silu_mu
     return (torch.empty(need, dtype=torch.uint8, device=device), need) if need else (None, 0)
 
 
+_TILED_ACTS = {None: 0, "silu_mul": 1, "gelu_erf": 2, "gelu_tanh_mul": 3}
+
+
 def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
-                 silu_mul: bool = False, split_tail: bool = False) -> torch.Tensor:
+                 silu_mul: bool = False, split_tail: bool = False, act: Optional[str] = None) -> torch.Tensor:
     """Prefill-sized F.linear(x, weight, bias) (layers/quantization/unquant.py:110-122) on the
     256 x 256-tile matrix-core kernel; silu_mul=True applies SiluAndMul (layers/activation.py:55-65)
-    to the [gate; up] output in the epilogue and returns [M, N / 2].  split_tail: tiles beyond whole rounds of
+    to the [gate; up] output in the epilogue and returns [M, N / 2], act "gelu_tanh_mul" gelu_tanh_and_mul, "gelu_erf" that
+    unit to the rounded output.  split_tail: tiles beyond whole rounds of
     the chip may share K (tiled_tail_splits); their sums are then added in another order than the others'."""
+    assert not (silu_mul and act)
+    epilogue = _TILED_ACTS["silu_mul" if silu_mul else act]
     _gpu(x, weight, bias)
     assert x.dim() == 2 and x.stride(1) == 1 and weight.is_contiguous() and weight.dtype == x.dtype
     M, K = x.shape
     N = weight.shape[0]
     assert weight.shape[1] == K
-    y = torch.empty((M, N // 2 if silu_mul else N), dtype=x.dtype, device=x.device)
+    pairs = epilogue in (1, 3)
+    y = torch.empty((M, N // 2 if pairs else N), dtype=x.dtype, device=x.device)
     if M == 0:
         return y
-    ws, nbytes = _tail_workspace(split_tail, M, N, K, False, silu_mul, x.device)
+    ws, nbytes = _tail_workspace(split_tail, M, N, K, False, pairs, x.device)
     check(_lib_().mi355_linear_tiled_ws(y.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(bias), M, N, K, x.stride(0), _dt(x),
-                                        1 if silu_mul else 0, _p(ws), nbytes, _stream(x)), "linear_tiled")
+                                        epilogue, _p(ws), nbytes, _stream(x)), "linear_tiled")
     return y
 
 

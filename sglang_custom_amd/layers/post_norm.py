@@ -70,8 +70,10 @@ class LayerNormResidualAdd(nn.Module):
 
     def forward(self, x: torch.Tensor, y: torch.Tensor, next_weight: Optional[torch.Tensor], rows: Optional[torch.Tensor] = None,
                 y2: Optional[torch.Tensor] = None, y2_gate: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-        """x fp32 [T, D], updated in place; returns LN(x) * next_weight in the weight's dtype.  y: also a decode product's SplitKPartials."""
+        """x fp32 [T, D], updated in place; returns LN(x) * next_weight in the weight's dtype.  y: also a decode product's SplitKPartials
+        (of 16-bit weights, alone: no picked rows, no second branch)."""
         if isinstance(y, SplitKPartials):
+            assert rows is None and y2 is None and y2_gate is None and y.x_scale is None and y.w_scale is None
             return get_ops().norm_residual_add_partials(x, y.part, self.weight.data, next_weight, self.eps, rms=False)
         return get_ops().layernorm_residual_add(x, y, self.weight.data, next_weight, self.eps, rows=rows, y2=y2, y2_gate=y2_gate)
 
@@ -85,8 +87,9 @@ class RMSNormResidualAdd(nn.Module):
     def forward(self, x: torch.Tensor, y: torch.Tensor, next_weight: Optional[torch.Tensor], rows: Optional[torch.Tensor] = None,
                 coef: Optional[torch.Tensor] = None) -> torch.Tensor:
         """x fp32 [T, D], updated in place; returns N(x) * next_weight, or x (next_weight None), in the weight's dtype.  y: also a decode
-        product's SplitKPartials."""
+        product's SplitKPartials (of 16-bit weights, without picked rows)."""
         if isinstance(y, SplitKPartials):
+            assert rows is None and coef is None and y.x_scale is None and y.w_scale is None
             return get_ops().norm_residual_add_partials(x, y.part, self.weight.data, next_weight, self.eps, rms=True)
         return get_ops().rmsnorm_residual_add_next(x, y, self.weight.data, next_weight, self.eps, rows=rows, coef=coef, copy=True)
 

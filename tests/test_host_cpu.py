@@ -831,3 +831,30 @@ def test_expert_block_class(pairs, experts, columns, block):
     assert ops.moe_block_class(pairs, experts, True, True, columns) == block
     assert ops.moe_block_class(pairs, experts, True, False, columns) == (1 if pairs >= 256 * experts else 0)
     assert ops.moe_block_class(pairs, experts, False, False, columns) == 0
+
+
+@pytest.mark.parametrize("rms,extra", [(False, ("rows",)), (False, ("y2",)), (False, ("y2_gate",)), (True, ("rows",)), (True, ("coef",)),
+                                       (False, ("x_scale",)), (True, ("x_scale", "w_scale")), (True, ())])
+def test_split_sums_come_to_a_post_norm_alone(rms, extra):
+    """The norm that sums a product's splits takes neither picked rows nor a second branch nor scales: what it would leave out is refused."""
+    from types import SimpleNamespace
+
+    from sglang_custom_amd import ops_backend
+    from sglang_custom_amd.layers.post_norm import LayerNormResidualAdd, RMSNormResidualAdd
+    from sglang_custom_amd.layers.quantization.unquant import SplitKPartials
+
+    calls = []
+    ops_backend.set_ops_backend(SimpleNamespace(norm_residual_add_partials=lambda *a, **kw: calls.append(kw)))
+    try:
+        norm = (RMSNormResidualAdd if rms else LayerNormResidualAdd)(8, 1e-5, torch.bfloat16, "cpu")
+        there = torch.ones(2, 8)
+        y = SplitKPartials(torch.zeros(3, 2, 8), **{k: there for k in extra if k.endswith("scale")})
+        kw = {k: there for k in extra if not k.endswith("scale")}
+        if extra:
+            with pytest.raises(AssertionError):
+                norm(torch.zeros(2, 8), y, None, **kw)
+        else:
+            norm(torch.zeros(2, 8), y, None, **kw)
+        assert calls == ([] if extra else [dict(rms=rms)])
+    finally:
+        ops_backend.set_ops_backend(None)

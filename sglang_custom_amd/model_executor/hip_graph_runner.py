@@ -55,6 +55,9 @@ class HipGraphRunner:
         self.positions = torch.zeros(self.max_bs, dtype=torch.int64, device=dev)
         self.graphs: Dict[int, torch.cuda.CUDAGraph] = {}
         self.outputs: Dict[int, torch.Tensor] = {}
+        # what a captured step was recorded over: its tensors (a state pool's h_last among them) are allocated outside the graphs' memory
+        # pool, and the recorded kernels read and write them by their addresses
+        self.batches: Dict[int, ForwardBatch] = {}
         self.pool = None
         model_runner.attn_backend.init_cuda_graph_state(self.max_bs, self.max_bs)
         with collector_paused():
@@ -100,6 +103,7 @@ class HipGraphRunner:
                 self.pool = self.pool or g.pool()
                 self.graphs[bs] = g
                 self.outputs[bs] = out
+                self.batches[bs] = fb
         torch.cuda.current_stream().wait_stream(stream)
         torch.cuda.synchronize()
         # ranks capture at different speeds: a collective of the warm-up runs that gave up waiting

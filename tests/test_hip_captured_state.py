@@ -1,6 +1,9 @@
 """Captured decode steps of the families that keep state per sequence (Fudonex) or latent rows (Silatar without matrix memories), against
 the whole-sequence oracles: eager prompts between the replays, padded batches, requests that end and begin again in their rows, and a
 request at row 0 of the request table that waits while padded batches of others run (its state is its own)."""
+import gc
+import weakref
+
 import pytest
 
 import fudonex_util as fu
@@ -47,3 +50,20 @@ def test_replays_against_the_oracle(family, dtype, tol):
         assert mr.req_to_token_pool.available_size() == mr.req_to_token_pool.size
         assert mr.token_to_kv_pool_allocator.available_size() == mr.max_total_num_tokens
         assert not mr.req_to_token_pool.table[mr.req_to_token_pool.pad_row].any()
+
+
+def test_what_a_graph_was_recorded_over_stays(monkeypatch):
+    """A captured step's kernels keep the addresses of its batch's tensors, which the graphs' memory pool does not hold."""
+    from sglang_custom_amd.model_executor.forward_batch_info import ForwardBatch
+
+    made, init = [], ForwardBatch._init_seq_state
+
+    def recording(self, runner):
+        init(self, runner)
+        made.append(weakref.ref(self.seq_state.h_last))
+
+    monkeypatch.setattr(ForwardBatch, "_init_seq_state", recording)
+    cfg = fu.make_config()
+    mr = fu.build_runner(cfg, fu.make_weights(cfg, seed=4), dtype="bfloat16", device=DEV, max_total_tokens=160, cuda_graph_bs=[1, 4])
+    gc.collect()
+    assert mr.graph_runner is not None and len(made) == 2 and all(t() is not None for t in made)

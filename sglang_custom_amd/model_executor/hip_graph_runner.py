@@ -64,7 +64,9 @@ class HipGraphRunner:
             self.capture()
 
     def can_run(self, forward_batch: ForwardBatch) -> bool:
-        return forward_batch.forward_mode.is_decode() and forward_batch.batch_size <= self.max_bs
+        # (a model that is asked for its residual streams runs eager: the graphs were recorded without the copies)
+        return (forward_batch.forward_mode.is_decode() and forward_batch.batch_size <= self.max_bs
+                and getattr(getattr(self.model_runner.model, "model", None), "capture_streams", None) is None)
 
     def _static_batch(self, bs: int) -> ForwardBatch:
         mr = self.model_runner

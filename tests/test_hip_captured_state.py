@@ -7,8 +7,10 @@ import weakref
 import pytest
 
 import fudonex_util as fu
+import lomazen_util as lu
 import silatar_util as su
 from oracle import fudonex_ref, silatar_ref
+from sglang_custom_amd.managers.trace_replay import TraceReplayer
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -67,3 +69,21 @@ def test_what_a_graph_was_recorded_over_stays(monkeypatch):
     mr = fu.build_runner(cfg, fu.make_weights(cfg, seed=4), dtype="bfloat16", device=DEV, max_total_tokens=160, cuda_graph_bs=[1, 4])
     gc.collect()
     assert mr.graph_runner is not None and len(made) == 2 and all(t() is not None for t in made)
+
+
+@pytest.mark.parametrize("family", ["fudonex", "silatar", "lomazen"])
+def test_streams_of_a_decode_step(family):
+    """A list in capture_streams receives the residual behind every layer of a decode step too, though the model's steps are captured."""
+    u = {"fudonex": fu, "silatar": su, "lomazen": lu}[family]
+    cfg = su.make_config(layers=[(su.latent(), su.dense())] * 2, loop=None) if family == "silatar" else u.make_config()
+    mr = u.build_runner(cfg, u.make_weights(cfg, seed=4), dtype="bfloat16", device=DEV, max_total_tokens=160, cuda_graph_bs=[1])
+    rp, tokens = TraceReplayer(mr), u.random_prompts(cfg, [4], seed=6)["r0"]
+    step = lambda t: rp.step([dict(id="r0", tokens=t, want=[0])])
+    step(tokens[:2])
+    mr.model.model.capture_streams = got = []
+    step(tokens[2:3])
+    n = len(mr.model_config.layer_runs) if family != "fudonex" else len(cfg["layers"])
+    assert mr.graph_runner is not None and [tuple(x.shape) for x in got] == [(1, cfg["width"])] * n
+    mr.model.model.capture_streams = None
+    step(tokens[3:])
+    assert len(got) == n

@@ -51,6 +51,7 @@ class ForwardMetadata:
     window_kv_indices: Optional[torch.Tensor] = None
     window_num_kv_splits: int = 1
     latent_blocks: Optional[dict] = None   # run length -> int32 [n, 2] token runs (forward_latent_window)
+    extend_shared: Optional[dict] = None   # what the layers of an extend over cached tokens share (ops.extend_attention_fwd)
 
 
 class Mi355AttnBackend(AttentionBackend):
@@ -202,7 +203,8 @@ class Mi355AttnBackend(AttentionBackend):
         else:
             kv_indices = self._dummy_idx
         md = ForwardMetadata(qo_indptr=qo_indptr, kv_indptr=kv_indptr, kv_indices=kv_indices,
-                             max_extend_len=max(forward_batch.extend_seq_lens_cpu))
+                             max_extend_len=max(forward_batch.extend_seq_lens_cpu),
+                             extend_shared={} if prefix_sum > 0 and kv_indices.is_cuda else None)
         if self.sliding_window_size:
             md.window_kv_indptr, md.window_kv_indices = self._window(
                 forward_batch.extend_prefix_lens, forward_batch.extend_prefix_lens_cpu, forward_batch.req_pool_indices, bs)
@@ -606,5 +608,6 @@ class Mi355AttnBackend(AttentionBackend):
             kbuf, vbuf,
             md.qo_indptr, md.window_kv_indptr if windowed else md.kv_indptr,
             md.window_kv_indices if windowed else md.kv_indices, None, True, None, md.max_extend_len,
-            layer.scaling, layer.logit_cap, sliding_window_size=layer.sliding_window_size if windowed else -1)
+            layer.scaling, layer.logit_cap, sliding_window_size=layer.sliding_window_size if windowed else -1,
+            **({"shared": md.extend_shared} if md.extend_shared is not None else {}))
         return o

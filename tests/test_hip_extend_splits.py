@@ -69,3 +69,58 @@ def test_rule(ops, rows, bs, longest, prefix, hq, d, want):
     assert f(rows, bs, longest, prefix, 0, hq, d, d, 0.1, 0.0, -1, 1) == want
     assert f(rows, bs, longest, prefix, 0, hq, d, d, 0.1, 30.0, -1, 1) == 1 and f(rows, bs, longest, prefix, 0, hq, d, d, 0.1, 0.0, 64, 1) == 1
     assert f(rows, bs, longest, prefix, 0, hq, d, d, 0.1, 0.0, -1, 0) == 1          # fp32 has no matrix-core kernel
+
+
+def test_layers_of_a_step_share_the_rule_and_its_memory(ops, monkeypatch):
+    """The second launch of a step asks nothing and gives the same bits; another shape under the same dict has an entry of its own."""
+    lib, asked = ops._lib_(), []
+    rule = lib.mi355_extend_attention_splits
+
+    class Counting:
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def mi355_extend_attention_splits(self, *a):
+            asked.append(rule(*a))
+            return asked[-1]
+
+    monkeypatch.setattr(ops, "_lib_", lambda: Counting())
+    g, d, hkv, pre = torch.Generator().manual_seed(5), 64, 2, 1000
+    r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    kb, vb = r(pre + 9, hkv, d), r(pre + 9, hkv, d)
+    slots = (torch.randperm(pre + 8, generator=g)[:pre] + 1).to(torch.int32).to(DEV)
+    kv, shared = torch.tensor([0, pre], dtype=torch.int32, device=DEV), {}
+    for ext, hq in ((70, 4), (70, 8), (200, 4)):
+        q, k, v = r(ext, hq, d), r(ext, hkv, d), r(ext, hkv, d)
+        qo, out = torch.tensor([0, ext], dtype=torch.int32, device=DEV), []
+        for kw in ({}, {"shared": shared}, {"shared": shared}):
+            o = torch.empty_like(q)
+            ops.extend_attention_fwd(q, k, v, o, kb, vb, qo, kv, slots, None, True, None, ext, d ** -0.5, **kw)
+            out.append(o)
+        assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    assert len(asked) == 6 and asked[0] > 1 and len(shared) == 3
+
+
+def test_a_model_step_asks_once(monkeypatch):
+    """An extend over cached tokens through a model: one entry for all of its layers, none without a prefix."""
+    from sglang_custom_amd import bench_one_batch as bob, ops_backend
+    from sglang_custom_amd.configs.model_config import ModelConfig
+    from sglang_custom_amd.distributed import parallel_state
+    from sglang_custom_amd.managers.schedule_batch import Req
+    from sglang_custom_amd.model_executor.model_runner import ModelRunner
+    from sglang_custom_amd.model_loader.synthetic import hf_config_dict, make_synthetic_llama_weights
+    from sglang_custom_amd.server_args import ServerArgs
+
+    ops_backend.set_ops_backend(None)
+    parallel_state.init_distributed_environment(1, 0)
+    cfg = hf_config_dict("tiny-llama-d64", "bfloat16")
+    w = make_synthetic_llama_weights(cfg, seed=1, dtype=torch.bfloat16)
+    mr = ModelRunner(ModelConfig(cfg, dtype="bfloat16"), ServerArgs(dtype="bfloat16", max_total_tokens=1024, max_running_requests=2, disable_cuda_graph=True),
+                     weights={k: v.to(DEV) for k, v in w.items()})
+    tokens = torch.randint(0, cfg["vocab_size"], (600,), generator=torch.Generator().manual_seed(2)).tolist()
+    _, _, batch = bob.extend([Req(0, tokens[:520])], mr)
+    assert mr.attn_backend.forward_metadata.extend_shared is None
+    req = Req(1, tokens)
+    req.init_next_round_input(mr.req_to_token_pool.req_to_token[int(batch.req_pool_indices[0]), :520].clone())
+    bob.extend([req], mr)
+    assert len(mr.attn_backend.forward_metadata.extend_shared) == 1

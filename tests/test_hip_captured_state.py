@@ -54,6 +54,37 @@ def test_replays_against_the_oracle(family, dtype, tol):
         assert not mr.req_to_token_pool.table[mr.req_to_token_pool.pad_row].any()
 
 
+@pytest.mark.parametrize("family,dtype,tol", [("fudonex", "float32", 3e-5), ("fudonex", "bfloat16", 6e-2), ("silatar", "bfloat16", 6e-2)])
+def test_replays_with_many_key_ranges(family, dtype, tol, monkeypatch):
+    """A captured step has its key ranges from the model's context length: at 8192 tokens ten and sixteen (windows and averaged blocks) and 64 (latent rows),
+    of which sequences of up to 78 tokens leave all but one to three without a key and padded rows all but one.  Silatar's with mixtures."""
+    from sglang_custom_amd import ops
+    from sglang_custom_amd.configs.model_config import ModelConfig
+    from sglang_custom_amd.model_executor.model_runner import ModelRunner
+    from sglang_custom_amd.server_args import ServerArgs
+
+    ranges = []
+    for name in ("window_attention_splits", "latent_window_attention_splits"):
+        monkeypatch.setattr(ops, name, lambda *a, rule=getattr(ops, name), **kw: (ranges.append(rule(*a, **kw)), ranges[-1])[1])
+    if family == "fudonex":
+        u, ref, cfg = fu, fudonex_ref, fu.make_config()
+    else:
+        moe = [su.moe(experts=3, top=3, ff=40, shared=(24, 1.1)), su.moe(experts=2, top=2, ff=32, shared=None)]
+        u, ref, cfg = su, silatar_ref, su.make_config(layers=[(su.latent(), moe[0]), (su.latent(kv_rank=24), su.dense(64)), (su.latent(), moe[1])], width=96,
+                                                      loop=(0, 2, 2))
+    w = u.make_weights(cfg, seed=4)
+    prompts = u.random_prompts(cfg, [78, 25, 12], seed=6)
+    want = {k: ref.forward(cfg, w, p) for k, p in prompts.items()}
+    mr = ModelRunner(ModelConfig(cfg, dtype=dtype, context_length=8192),
+                     ServerArgs(dtype=dtype, device=DEV, max_total_tokens=160, max_running_requests=4, context_length=8192, cuda_graph_bs=[1, 4]),
+                     weights={k: v.to(DEV) for k, v in w.items()})
+    assert mr.graph_runner is not None and set(ranges) == ({10, 16} if family == "fudonex" else {64})
+    sched = [[("r0", 60), ("r1", 5)]] + [[("r0", 1)]] * 4 + [[("r2", 2)]] + [[("r0", 1), ("r1", 1), ("r2", 1)]] * 10 + [[("r0", 1), ("r1", 1)]] * 4
+    sched += [[("r1", 1)]] * 6
+    for _ in range(2):
+        u.replay_and_compare(mr, cfg, w, prompts, sched, tol, want_all=want)
+
+
 def test_what_a_graph_was_recorded_over_stays(monkeypatch):
     """A captured step's kernels keep the addresses of its batch's tensors, which the graphs' memory pool does not hold."""
     from sglang_custom_amd.model_executor.forward_batch_info import ForwardBatch

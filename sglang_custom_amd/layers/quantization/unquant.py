@@ -17,10 +17,10 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
+from ...ops import FEW_MAX_M
 from ...ops_backend import get_ops
 
 SKINNY_MAX_M = 64
-FEW_MAX_M = 256         # rows up to which mi355_linear_few may be ahead: asking it costs the host 3 us, which steps of 400 rows feel
 # Deferred split-K reduction / fused decode step (bit-identical to the unfused kernels; the switch
 # exists so that tests and profiles can run both).
 DECODE_FUSION = True

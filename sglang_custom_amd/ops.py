@@ -831,7 +831,8 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return y
 
 
-FEW_MAX_M, FEW_MAX_M_FP8 = 256, 512     # rows up to which mi355_linear_few may be ahead: asking it costs the host 3 us
+# Rows up to which mi355_linear_few may be ahead (its own rule refuses more): asking it costs the host 3 us, which steps of 400 rows feel.
+FEW_MAX_M, FEW_MAX_M_FP8 = 256, 512
 
 
 def linear_few_supported(m: int, n: int, k: int, out_dtype: torch.dtype, silu_mul: bool = False, fp8: bool = False) -> bool:

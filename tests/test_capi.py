@@ -116,3 +116,12 @@ def test_split_plan_of_captured_launches(lib, bs, hkv, keys, most, fp8, splits, 
     assert lib.mi355_decode_split_plan(bs, hkv, keys, most, fp8, ctypes.byref(f), ctypes.byref(k)) == splits
     assert (f.value, k.value) == (fewest, split_keys)
     assert splits == (lib.mi355_decode_num_splits_fp8 if fp8 else lib.mi355_decode_num_splits)(bs, hkv, keys, most)
+
+
+def test_few_rows_limits_agree(lib):
+    """The front end asks mi355_linear_few's rule up to FEW_MAX_M rows (one-byte operands FEW_MAX_M_FP8): where the rule itself ends."""
+    from sglang_custom_amd import _lib, ops
+
+    for fp8, most in ((0, ops.FEW_MAX_M), (1, ops.FEW_MAX_M_FP8)):
+        assert lib.mi355_linear_few_supported(most, 2048, 2048, fp8, _lib.BF16, 0) == 1
+        assert lib.mi355_linear_few_supported(most + 1, 2048, 2048, fp8, _lib.BF16, 0) == 0

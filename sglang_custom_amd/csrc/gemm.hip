@@ -878,12 +878,11 @@ __global__ __launch_bounds__(512) void norm_linear_kernel(NormLinearParams p) {
 template <typename T>
 static int launch_norm_linear(const NormLinearParams& p, const SkinnyPlan& plan, bool act, hipStream_t st) {
   const bool two = p.K > 512 * (plan.waves / p.M), many = p.nsplit > 4;
-  const size_t lds = (size_t)p.M * (p.K + NL_PAD) * sizeof(T);
+  const size_t lds = (size_t)p.M * (p.K + NL_PAD) * sizeof(T);     // (at most 16.5 KB: K <= 1024 waves / M)
 #define MI355_NL(ACT) \
   (two ? (many ? norm_linear_kernel<T, ACT, 2, 8> : norm_linear_kernel<T, ACT, 2, 4>) : (many ? norm_linear_kernel<T, ACT, 1, 8> : norm_linear_kernel<T, ACT, 1, 4>))
   void (*kern)(NormLinearParams) = act ? MI355_NL(true) : MI355_NL(false);
 #undef MI355_NL
-  if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL(kern, dim3((unsigned)plan.nblocks, (unsigned)plan.splits), dim3(64 * plan.waves), lds, st, p);
   MI355_CHECK_LAUNCH("norm_linear_packed");
   return MI355_OK;
@@ -1198,8 +1197,7 @@ static void launch_quant_linear(const QuantLinearParams& p, const SkinnyPlan& pl
   const bool wide = p.K > 2048;
   void (*kern)(QuantLinearParams) = rpw <= 1 ? (wide ? quant_linear_kernel<T, 1, 8> : quant_linear_kernel<T, 1, 4>)
                                              : (wide ? quant_linear_kernel<T, 2, 8> : quant_linear_kernel<T, 2, 4>);
-  const size_t lds = (size_t)p.M * (p.k_per_split + 32);
-  if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const size_t lds = (size_t)p.M * (p.k_per_split + 32);     // (at most 33 KB)
   hipLaunchKernelGGL(kern, dim3((unsigned)plan.nblocks, (unsigned)plan.splits), dim3(64 * plan.waves), lds, st, p);
 }
 
@@ -1397,7 +1395,7 @@ int mi355_linear_packed_act_mul(void* y, const void* x, const void* w_packed, in
 int mi355_norm_linear_packed_splits(int64_t m, int64_t n, int64_t k, int silu_mul) {
   if (m < 1 || m > NL_ROWS || n < 16 || n % 16 != 0 || n >= 64 * 1024 || k < SK_BK || k % SK_BK != 0 || g_gemm_variant != 0) return 0;
   const SkinnyPlan p = plan_skinny(m, n, k, true);
-  if (p.nt != 1 || (silu_mul && p.splits != 1) || k > 1024 * (p.waves / m) || m * (k + NL_PAD) * 2 > 96 * 1024) return 0;
+  if (p.nt != 1 || (silu_mul && p.splits != 1) || k > 1024 * (p.waves / m)) return 0;
   return p.splits;
 }
 

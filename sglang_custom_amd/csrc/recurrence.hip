@@ -698,7 +698,10 @@ __global__ __launch_bounds__(CK_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 // sequences have segments, of known lengths (tokens in all, the longest one), and less time by the two forms' models, which fit what
 // was measured within 15 % (16 heads of 64 x 128, in us).  A token of the token-by-token form takes a chain of 0.40 (delta 0.55)
 // or, from some 1000 workgroups on, its share of the chip, 0.43 (0.60) per 1000 of them; a chunk takes its workgroup 6.7 (10.6), one
-// workgroup to a CU, and about 3 more before the first.  Measured, token by token / chunks:
+// workgroup to a CU, and about 3 more before the first.  That is the price of chunks in one launch as they first were: with the state in two
+// buffers they take a tenth less, behind records 4.0 (5.2), so where the rule takes chunks they are ahead by more, and many middling prompts
+// that it leaves token by token (64 x 500) may be faster in chunks behind records; the lines have not been measured again.  Measured, token
+// by token / chunks in that first form:
 //   plain  1 x 16   9.8 / 10.4   1 x 64   27 / 11     8 x 65   32 / 35    16 x 64    42 / 42    64 x 4    27 / 149   64 x 500   813 / 905
 //   delta  1 x 16  12.4 / 14.9   1 x 64   38 / 16     8 x 65   43 / 51    16 x 64    54 / 58    64 x 4    27 / 213   64 x 500  1096 / 1409
 //   plain  4 x 2000   827 / 223   16 x 1000   464 / 440   16 x 2000   1010 / 865;   delta   1130 / 348   667 / 691   1369 / 1372

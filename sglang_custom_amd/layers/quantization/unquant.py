@@ -21,8 +21,8 @@ from ...ops import FEW_MAX_M
 from ...ops_backend import get_ops
 
 SKINNY_MAX_M = 64
-# Deferred split-K reduction / fused decode step (bit-identical to the unfused kernels; the switch
-# exists so that tests and profiles can run both).
+# Deferred split-K reduction / fused decode step (bit-identical to the unfused kernels but for the norm inside a projection of one or two
+# rows, ops.norm_linear_packed, which adds the squares in another order; the switch exists so that tests and profiles can run both).
 DECODE_FUSION = True
 # "tiled" | "auto" | "library" for 16-bit GEMMs with more than SKINNY_MAX_M rows (see the module docstring)
 PREFILL_GEMM = os.environ.get("MI355_PREFILL_GEMM", "tiled")

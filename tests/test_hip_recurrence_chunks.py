@@ -168,3 +168,37 @@ def test_records_in_front_change_no_bits(lens, H, G, dk, dv, qk, vt, delta, monk
     assert wanted(delta, B, H, dk, dv, T, max(lens), DEV)[1] > 0, "the case is for the chunks"
     got, want = run(wanted), run(lambda *a: (None, 0))
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and got[0].isfinite().all()
+
+
+@pytest.mark.parametrize("what,delta", [(w, d) for w in ("v", "k", "q", "z", "beta", "state") for d in (False, True) if d or w != "beta"])
+def test_records_with_values_that_are_no_numbers(what, delta, monkeypatch):
+    """An infinity and a NaN in a middle chunk: with records in front every output and state is what it is without them, and the tokens before are
+    finite."""
+    from sglang_custom_amd import ops
+
+    lens, H, G, dk, dv = (449, 330), 2, 1, 40, 33
+    c = _case(lens, H, G, dk, dv, torch.float32, torch.float32, 12, -1.0)
+    bad = {"v": (c["v"][200, 1, 5:6], c["v"][449 + 127, 0, 32:]), "k": (c["k"][200, 7:8], c["k"][449 + 127, 39:]), "q": (c["q"][200, 7:8], c["q"][449 + 127, 39:40]),
+           "z": (c["z"][200, :1], c["z"][449 + 127, 1:]), "beta": (c["beta"][200, :1], c["beta"][449 + 127, 1:]),
+           "state": (c["state"][int(c["slots"][1]), 0, 3, :1], c["state"][int(c["slots"][1]), 1, 5, 32:])}[what]
+    bad[0].fill_(float("inf") if what in ("v", "k", "state") else float("nan"))
+    bad[1].fill_(float("nan"))
+    d, T = {k: t.to(DEV) for k, t in c.items()}, sum(lens)
+    seg = dict(tok_req=torch.zeros(T, dtype=torch.int32, device=DEV), seg_start=d["start"], seg_len=torch.tensor(lens, dtype=torch.int32, device=DEV), longest=max(lens))
+    args = (d["slots"].int(), torch.arange(2, device=DEV), d["pos"], 0.25)
+    q, k = d["q"][:, : G * dk].view(T, G, dk), d["k"].view(T, G, dk)
+    wanted, results = ops._chunk_records, []
+    assert wanted(delta, 2, H, dk, dv, T, max(lens), DEV)[1] > 0, "the case is for the records"
+    for records in (wanted, lambda *a: (None, 0)):
+        monkeypatch.setattr(ops, "_chunk_records", records)
+        out, state = torch.zeros(T, H, dv, device=DEV), d["state"].clone()
+        if delta:
+            ops.gated_delta_rule(q, k, d["v"], d["beta"], d["z"], d["bias"], d["rate"], out, state, *args, **seg)
+        else:
+            ops.linear_recurrence(q, k, d["v"], out, state, *args, dt_logits=d["z"], dt_bias=d["bias"], rate_log=d["rate"], skip=d["skip"], **seg)
+        results.append((out, state))
+    for a, b in zip(*results):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+    out = results[0][0]
+    assert out[:200].isfinite().all() and not out.isfinite().all()
+    assert what == "state" or out[449: 449 + 127].isfinite().all()

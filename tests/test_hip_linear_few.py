@@ -75,3 +75,25 @@ def test_what_is_left_to_others(ops):
     assert ops.linear_few(torch.zeros(128 * 1024 + 1, dtype=torch.bfloat16, device=DEV)[1:].view(128, 1024), w) is None    # 2-byte aligned
     assert ops.linear_few(x, w, torch.zeros(2048, device=DEV)) is None                                          # a bias of another type
     assert ops.linear_few(x.float(), w.float()) is None
+
+
+# one split and several (their sums' memory is the graph's own), both epilogues
+@pytest.mark.parametrize("m,n,k,fp8,silu", [(96, 2048, 2048, False, False), (128, 2048, 8192, False, False), (96, 4096, 1024, False, True), (96, 4096, 4096, True, False)])
+def test_captured(ops, m, n, k, fp8, silu):
+    """Decode steps of more than 64 rows are captured too where they are asked for: replays over new rows give the eager call's bits."""
+    g = torch.Generator().manual_seed(m + n)
+    cast = lambda t: t.to(torch.float8_e4m3fn if fp8 else torch.bfloat16).to(DEV)
+    x, w = cast(torch.randn(m, k, generator=g)), cast(torch.randn(n, k, generator=g))
+    scales = (torch.rand(m, 1, generator=g).to(DEV), torch.rand(n, generator=g).to(DEV), torch.bfloat16) if fp8 else ()
+    run = lambda: ops.linear_few(x, w, None, silu, *scales)
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = run()
+    for _ in range(4):
+        x.copy_(cast(torch.randn(m, k, generator=g)))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = y.clone()
+        assert torch.equal(got, run())

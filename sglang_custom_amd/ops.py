@@ -72,11 +72,12 @@ def _kvdt(t: torch.Tensor, cache: torch.Tensor, v_cache: Optional[torch.Tensor] 
     """dtype code of the 16-bit tensors, flagged when `cache` is an fp8 KV buffer and when it is head-major."""
     lay = _kv_layout(cache)
     if v_cache is not None:
-        assert _kv_layout(v_cache) == lay and v_cache.shape[0] == cache.shape[0], "k and v cache layouts differ"
-        if lay & KV_INTERLEAVED:
-            assert (v_cache.shape == cache.shape
+        if lay & KV_INTERLEAVED:     # (the key rows' shape and strides have the key rows' layout: it is not looked up again)
+            assert (v_cache.shape == cache.shape and v_cache.stride() == cache.stride()
                     and v_cache.data_ptr() == cache.data_ptr() + cache.shape[2] * cache.element_size()), \
                 "an interleaved cache holds a token's value row right behind its key row"
+        else:
+            assert _kv_layout(v_cache) == lay and v_cache.shape[0] == cache.shape[0], "k and v cache layouts differ"
     return _dt(t) | (KV_FP8 if cache.dtype == torch.float8_e4m3fn else 0) | lay
 
 
@@ -181,7 +182,7 @@ def rope_inplace(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, head
     check(_lib_().mi355_rope_inplace(
         q2.data_ptr(), k2.data_ptr(), _p(v) if fused else None, positions.data_ptr(),
         cos_sin_cache.data_ptr(), cache_dt, T, hq, hkv, head_size, rotary_dim, q2.stride(0),
-        k2.stride(0), v.view(T, -1).stride(0) if fused else 0, 1 if is_neox else 0,
+        k2.stride(0), v2.stride(0) if fused else 0, 1 if is_neox else 0,
         _p(k_buffer) if fused else None, _p(v_buffer) if fused else None,
         _p(loc) if fused else None, _IT[loc.dtype] if fused else I64,
         k_buffer.shape[0] if fused else 0, _kvdt(q, k_buffer, v_buffer) if fused else _dt(q), _stream(q)), "rope_inplace")
@@ -703,7 +704,8 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
     """extend_attention_fwd(...) (triton_ops/extend_attention.py:306-438), same argument order.  shared: a dict that the layers of one step
     pass, launches that follow each other on one stream: the first asks the split rule and allocates the partial sums' memory, the others
     use both.  (Host time, which an eager step of few tokens is bound by: 2.6 us a layer beside the merge launch's 3.4.  4 x 97 tokens on
-    1465 cached, 16 layers of head_dim 64: 3.26 ms unsplit, 3.46 with every layer asking, 3.36 so.)"""
+    1465 cached, 16 layers of head_dim 64: 3.26 ms unsplit, 3.46 with every layer asking, 3.36 so; what the layout checks and views of
+    rotation and attention no longer do twice is as much again: four runs in turn 3.26 to 3.50 ms unsplit, 3.19 to 3.36 now.)"""
     _gpu(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices)
     T, Hq, D = q_extend.shape
     Hkv, Dv = v_extend.shape[1], v_extend.shape[2]

@@ -858,3 +858,37 @@ def test_split_sums_come_to_a_post_norm_alone(rms, extra):
         assert calls == ([] if extra else [dict(rms=rms)])
     finally:
         ops_backend.set_ops_backend(None)
+
+
+@pytest.mark.parametrize("slots,heads,d", [(5, 2, 8), (5, 1, 8), (1, 2, 8), (1, 1, 8)])
+def test_kv_layout_codes(slots, heads, d):
+    """Pairs of cache tensors in every layout that the code knows and some that it does not: accepted where both have the same one (an interleaved
+    pair the value row right behind the key row), with the code of its own rule."""
+    from sglang_custom_amd import ops
+
+    plain = lambda: torch.zeros(slots, heads, d, dtype=torch.bfloat16)
+    major = lambda: torch.zeros(heads, slots, d, dtype=torch.bfloat16).permute(1, 0, 2)
+    both = torch.zeros(heads, slots, 2, d, dtype=torch.bfloat16)
+    wide = torch.zeros(heads, slots, 3, d, dtype=torch.bfloat16)
+    tensors = [plain(), major(), both[:, :, 0].permute(1, 0, 2), both[:, :, 1].permute(1, 0, 2), torch.zeros(heads, slots, 2, d, dtype=torch.bfloat16)[:, :, 1].permute(1, 0, 2),
+               wide[:, :, 0].permute(1, 0, 2), both[:, :, 0].permute(1, 0, 2)[..., : d // 2], torch.zeros(slots, heads, 2 * d, dtype=torch.bfloat16)[..., d:],
+               torch.zeros(slots + 1, heads, d, dtype=torch.bfloat16)]
+
+    def layout(t):
+        try:
+            return ops._kv_layout(t)
+        except AssertionError:
+            return None
+
+    q = torch.zeros(1, dtype=torch.bfloat16)
+    for k in tensors:
+        for v in tensors:
+            want = layout(k)
+            if want is not None and (layout(v) != want or v.shape[0] != k.shape[0]
+                                     or (want & ops.KV_INTERLEAVED and (v.shape != k.shape or v.data_ptr() != k.data_ptr() + 2 * d))):
+                want = None
+            if want is None:
+                with pytest.raises(AssertionError):
+                    ops._kvdt(q, k, v)
+            else:
+                assert ops._kvdt(q, k, v) == ops._dt(q) | want

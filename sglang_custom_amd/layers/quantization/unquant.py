@@ -163,12 +163,13 @@ def decode_linear_deferred(layer, x, needs_all_reduce: bool = True):
     when the layer, the shape or the ops backend does not support it.  A row-parallel layer
     (needs_all_reduce) qualifies only at TP=1: its output would have to cross ranks first.  x is a
     [M, K] tensor or, for an fp8 layer, a QuantizedAct."""
+    if not DECODE_FUSION or len(x.shape) != 2 or not 1 <= x.shape[0] <= SKINNY_MAX_M:     # (first: prompts ask twice a layer, 2 us less each)
+        return None
     from .w8a8_fp8 import W8A8Fp8LinearMethod
 
     ops = get_ops()
     wp = getattr(layer, "weight_packed", None)
-    if (not DECODE_FUSION or wp is None or (needs_all_reduce and getattr(layer, "tp_size", 1) != 1)
-            or len(x.shape) != 2 or not 1 <= x.shape[0] <= SKINNY_MAX_M):
+    if wp is None or (needs_all_reduce and getattr(layer, "tp_size", 1) != 1):
         return None
     n = layer.weight.shape[0]
     if isinstance(layer.quant_method, W8A8Fp8LinearMethod):

@@ -704,8 +704,7 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
     """extend_attention_fwd(...) (triton_ops/extend_attention.py:306-438), same argument order.  shared: a dict that the layers of one step
     pass, launches that follow each other on one stream: the first asks the split rule and allocates the partial sums' memory, the others
     use both.  (Host time, which an eager step of few tokens is bound by: 2.6 us a layer beside the merge launch's 3.4.  4 x 97 tokens on
-    1465 cached, 16 layers of head_dim 64: 3.26 ms unsplit, 3.46 with every layer asking, 3.36 so; what the layout checks and views of
-    rotation and attention no longer do twice is as much again: four runs in turn 3.26 to 3.50 ms unsplit, 3.19 to 3.36 now.)"""
+    1465 cached, 16 layers of head_dim 64: 3.24 ms unsplit, 3.46 with every layer asking, 3.36 so, 3.27 since such steps check less elsewhere.)"""
     _gpu(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices)
     T, Hq, D = q_extend.shape
     Hkv, Dv = v_extend.shape[1], v_extend.shape[2]

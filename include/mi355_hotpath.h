@@ -550,8 +550,8 @@ int mi355_linear_packed_scaled(float* y, const void* x, const void* w_packed, fl
  * epilogue 1 (W = [gate; up], N = 2 I): y [M, I], y[m, j] = T(silu(T(g_j))) * T(u_j) with the rounding
  * points of the unfused GEMM + SiluAndMul pair; epilogue 2: y [M, N] = T(gelu(T(acc))), gelu(z) = z / 2 (1 + erf(z / sqrt 2)),
  * without bias; epilogue 3: as 1 with y[m, j] = T(gelu_tanh(T(g_j)) T(u_j)), gelu_tanh(z) = z / 2 (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))).
- * Needs K % 64 == 0, K >= 128, N % 16 == 0
- * (mi355_linear_tiled_supported returns 1); no workspace, nothing allocated.
+ * Needs K % 64 == 0, 128 <= K < 2^23, N % 16 == 0, x_stride < 2^23
+ * (mi355_linear_tiled_supported returns 1 for the shape); no workspace, nothing allocated.
  * replaces: UnquantizedLinearMethod.apply / F.linear at prefill sizes
  *           (layers/quantization/unquant.py:110-122) and, with epilogue 1, LlamaMLP.forward's
  *           gate_up_proj + act_fn (models/llama.py:94-98, layers/activation.py:55-65). */

@@ -26,12 +26,21 @@
 //   * LDS rows are 128 bytes; the 16-byte chunk index is XOR-ed with a function of the row on the
 //     SOURCE address of the load (the load unit writes lane-linear) and again on the fragment read:
 //     conflict-free ds_read_b128 for 16-byte (16-bit) and 32-byte (fp8) fragments.
-//   * W rows are assigned to MFMA row slots so that a lane ends up with 16 consecutive output
-//     columns (or, for SiLU-and-mul, 8 gate columns and the 8 matching up columns): the epilogue
-//     writes whole 128-byte lines with 16-byte stores and needs no cross-lane traffic.
+//   * W rows are assigned to MFMA row slots so that a lane ends up with two runs of 8 consecutive output
+//     columns, 32 apart (or, for SiLU-and-mul, 8 gate columns and the 8 matching up columns): a 16-byte store
+//     of a wave writes 64 bytes in a row of each of its 16 rows, and needs no cross-lane traffic (16 columns in a row for a
+//     lane leave every second 16 bytes of a line to the next store: 4096 x 4096, K 2048, one tile a CU, 56.2 us instead of 53.2);
 //   * workgroup -> tile: consecutive workgroups round-robin over the 8 XCDs, so workgroups b and
 //     b + 8 share an L2; each XCD works through 8 x 4 blocks of tiles (32 CUs = one block);
+//   * a workgroup stays on its CU and takes tile after tile: the K tiles of all its output tiles are one stream of requests, so
+//     the next tile's operands are on their way while the last one's results are written (a group writes its results in front of
+//     its first READ slot of the next tile, next to the other group's last MATRIX slot);
 //   * tiles beyond whole rounds of 256 may be split over K, their sums added by a second launch that also runs the epilogue.
+// A tile that ends costs what its K tiles do not: with a workgroup per tile 10.6 us (7725 x 8192 columns, K 2048: 200 us of which the K
+// tiles take 160), as it is 6.5.  us, a workgroup per tile -> now: 7725 x 8192 x K 2048 200.2 -> 187.5, K 4096 361 -> 346; 4605 x 6144 x K
+// 4096 169 -> 163; 2 x 14336 x K 4096 with SiLU-and-mul 771 -> 751; 4096 x K 14336 511 -> 500.  (Waiting for the next tile's requests and
+// not for the stores behind them gained nothing more; four waves of 128 x 128, a third fewer LDS reads, 2 to 9 % slower: K tiles of
+// 2470 cycles instead of 2260, for nothing covers a wave's own LDS reads and requests but its MFMAs.)
 // What bounds it: the card's power.  The MFMAs of a K tile take 2048 of its 2320 cycles (88 %), but with random operands the
 // clock falls to 1.7 GHz (4096 x 4096 x 4096: 98 us; with x = 0 2.17 GHz and 77).  So the order of a matrix slot's MFMAs counts: W fragments
 // go forth in one row of x fragments and back in the next, one operand of every MFMA the last one's (a loop of MFMAs alone 2045 ->
@@ -45,6 +54,7 @@ namespace {
 constexpr int GT_HALF = 128 * 128;      // bytes of one half-tile
 constexpr int GT_STAGE = 4 * GT_HALF;   // one K tile: x (2 halves) + W (2 halves)
 constexpr int GT_LDS = 2 * GT_STAGE;    // 131072
+constexpr int64_t GT_MAX_STRIDE = (1 << 23) - 8;   // elements between rows of x and W: 128 rows are addressed with 31 bits
 
 struct GemmTiledParams {
   const void* x;
@@ -248,15 +258,15 @@ __device__ __forceinline__ float gelu_tanh_logistic(float z) {
 constexpr bool gt_pairs(int epi) { return epi == 1 || epi == 5; }   // W = [gate; up]
 
 // The results of NM groups of 16 rows (row mbase + 16 mi + r16 is lane (q4, r16)'s in group mi; mbase: the first group's first row).
-// acc[mi][ni][r]: W slot 16 ni + 4 q4 + r of the wave's 64, which the load mapping made output column 16 q4 + 4 ni + r (plain) or
-// gate / up column 8 q4 + 4 (ni & 1) + r.  EPI 3: `live` rows of the tile are no padding.
-template <typename T, int EPI, bool FP8, int NM>
+// acc[mi][ni][r]: W slot 16 ni + 4 q4 + r of the wave's 64, which the load mapping made output column 32 (ni >> 1) + 8 q4 + 4 (ni & 1) + r
+// (plain) or column 8 q4 + 4 (ni & 1) + r of gate (ni < 2) or up.  EPI 3: `live` rows of the tile are no padding.
+template <typename T, int EPI, bool FP8, int NM, bool BIAS>
 __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], int m0, int tm, int tn, int wc, int q4, int r16,
                                               int live) {
   const int ncols = gt_pairs(EPI) ? (p.N >> 1) : p.N;   // output columns
   const int mbase = m0 + r16;
   T* yg = (T*)p.y;
-  const T* bias = (const T*)p.bias;
+  [[maybe_unused]] const T* bias = (const T*)p.bias;
   float sxm[NM];
 #pragma unroll
   for (int mi = 0; mi < NM; ++mi) {
@@ -291,13 +301,16 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
       }
     }
   } else {
-    const int n0 = tn * 256 + wc * 64 + q4 * 16;
+    const int n0 = tn * 256 + wc * 64 + q4 * 8, n1 = n0 + 32;
     if (n0 < p.N) {
       float bv[16], sw[16];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) { bv[j] = 0.f; sw[j] = FP8 ? p.w_scale[n0 + j] : 1.f; }
-      if (bias != nullptr) {
-        const Vec<T, 8> b0 = ldvec<T, 8>(bias + n0), b1 = ldvec<T, 8>(bias + n0 + 8);
+      for (int j = 0; j < 8; ++j) {
+        sw[j] = FP8 ? p.w_scale[n0 + j] : 1.f;
+        sw[8 + j] = FP8 ? p.w_scale[min(n1, p.N - 8) + j] : 1.f;
+      }
+      if constexpr (BIAS) {
+        const Vec<T, 8> b0 = ldvec<T, 8>(bias + n0), b1 = ldvec<T, 8>(bias + min(n1, p.N - 8));
 #pragma unroll
         for (int j = 0; j < 8; ++j) { bv[j] = to_f32(b0.v[j]); bv[8 + j] = to_f32(b1.v[j]); }
       }
@@ -325,23 +338,74 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
                 v1 = fmaxf(v1, 0.f); v1 *= v1;
               }
             }
-            o0.v[ni * 4 + r] = from_f32<T>(v0 + bv[ni * 4 + r]);
-            o1.v[ni * 4 + r] = from_f32<T>(v1 + bv[8 + ni * 4 + r]);
+            if constexpr (BIAS) {
+              v0 += bv[ni * 4 + r];
+              v1 += bv[8 + ni * 4 + r];
+            }
+            o0.v[ni * 4 + r] = from_f32<T>(v0);
+            o1.v[ni * 4 + r] = from_f32<T>(v1);
           }
         if (EPI == 3 ? m - tm * 256 < live : m < p.M) {
           stvec<T, 8>(yg + (int64_t)m * p.ldy + n0, o0);
-          stvec<T, 8>(yg + (int64_t)m * p.ldy + n0 + 8, o1);
+          if (n1 < p.N) stvec<T, 8>(yg + (int64_t)m * p.ldy + n1, o1);
         }
       }
     }
   }
 }
 
-// MIXED (EPI 3): tiles without padding are as likely as tiles with; a wave whose rows are all there then takes a loop without the
-// conditions that leave padding out.  Those cost a full tile 5 %, the second loop a mostly empty one 3 to 6 (32 experts of 2048 x
-// 2048, 4 per token, both products: 8192 tokens 663 -> 624 us with it, 3000 297 -> 288, 1024 193 -> 197; 256 of 2048 x 512, 8 per
-// token, 64 tokens 304 -> 322).
-template <typename T, int EPI, bool FP8, bool MIXED>
+// The buffer that holds half h of a group's operand in tile (tm, tn), from its first row on: W for group 0 (waves of pairs: their gate or up
+// rows), x for group 1.  Rows past the matrix read as zeros (of a gate, they are up rows); their results are not stored.
+template <int EPI, int ES>
+__device__ __forceinline__ auto gt_half(const GemmTiledParams& p, int tm, int tn, int g, int wc, int h) {
+  constexpr int NR = gt_pairs(EPI) ? 64 : 128;
+  const int64_t row = g == 0 ? (int64_t)tn * (2 * NR) + h * NR + (gt_pairs(EPI) && (wc & 1) ? p.N >> 1 : 0) : (int64_t)tm * 256 + h * 128;
+  const int64_t rows = g == 0 ? p.N : p.M, ld = (g == 0 ? (int64_t)p.K : p.ldx) * ES;
+  const int64_t bytes = row < rows ? min((rows - 1 - row) * ld + (int64_t)p.K * ES, (int64_t)0x7fffffff) : 0;
+  return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)(g == 0 ? p.w : p.x) + row * ld), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ void blds16(__amdgpu_buffer_rsrc_t r, char* l, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)l, 16, voff, soff, 0, 0);
+}
+
+// What a workgroup works on: an output tile, or a split of a tail tile (K tiles t0 .. t0 + T - 1, sums to `part`).
+struct GtItem { int tm, tn, t0, T; float* part; bool valid; };
+
+// Item i of this workgroup.  Consecutive workgroups go to the eight XCDs in turn, and every XCD gets an equal run of the tiles in block
+// order (bands of 8 rows, blocks of 4 columns inside): whole blocks in turn left some XCDs a round more than others where the last band is
+// short -- 18 x 24 tiles: 72 on two XCDs and 40 on four, of 32 CUs each.  M = 4605, K = 4096: N = 6144 267 -> 190 us, N = 28672 846 -> 792;
+// 7381 x 2048 -> 2 x 5632 302 -> 280.  Splits of tail tiles come last (whole tiles are a multiple of 256 then, an equal number for
+// every workgroup); every XCD takes neighbouring ones, one stretch of K of all the tail's operands.
+__device__ __forceinline__ GtItem gt_item(const GemmTiledParams& p, int i, int kt) {
+  GtItem it{0, 0, 0, kt, nullptr, false};
+  const int xcd = blockIdx.x & 7, li = blockIdx.x >> 3, wide = gridDim.x >> 3;
+  const int whole = p.splits == 0 ? p.mt * p.nt : p.full, per = (whole + 7) >> 3, j = li + i * wide;
+  if (j < per) {
+    const int at = xcd * per + j;
+    it.valid = at < whole;
+    if (it.valid) tile_of(p, at, it.tm, it.tn);
+  } else if (p.splits != 0 && j - per < wide) {
+    const int tper = (p.tail * p.splits + 7) >> 3, u = xcd * tper + li;
+    it.valid = li < tper && u < p.tail * p.splits;
+    if (it.valid) {
+      const int k = u / p.tail, t = u - k * p.tail;
+      tile_of(p, p.full + t, it.tm, it.tn);
+      it.part = p.part + ((int64_t)k * p.tail + t) * 65536;
+      it.t0 = kt * k / p.splits;
+      it.T = kt * (k + 1) / p.splits - it.t0;
+    }
+  }
+  return it;
+}
+
+#define GT_SLOT_END()                                                                        \
+  do {                                                                                       \
+    __builtin_amdgcn_sched_barrier(0);                                                       \
+    __builtin_amdgcn_s_barrier();                                                            \
+    __builtin_amdgcn_sched_barrier(0);                                                       \
+  } while (0)
+
+template <typename T, int EPI, bool FP8>
 __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   extern __shared__ __attribute__((aligned(16))) char sm[];
   using frag = typename Mfma<T>::frag;
@@ -349,16 +413,193 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = wave >> 2, wc = wave & 3;
+  const int kt = (p.K * ES) >> 7;   // K tiles of 128 bytes per row
+
+  GtItem cur = gt_item(p, 0, kt);
+  if (!cur.valid) return;
+
+  // ---- the eight load instructions a wave issues per K tile -----------------------------------
+  // A wave requests data only in its READ slot (a load-to-LDS holds the issuing wave ~40 cycles: in
+  // front of or between the MFMAs of a matrix slot that time is lost to the matrix pipe, next to the
+  // LDS reads of a READ slot it is covered by the other group's MFMAs).  Group 0 (READ slot 2t) requests
+  // W of tile t + 1, both halves; group 1 (READ slot 2t + 1) requests x rows 128..255 of tile t + 1 and
+  // x rows 0..127 of tile t + 2: each is free when requested (its last reader finished a slot earlier)
+  // and is waited for -- by the waves that requested it, at the end of their MATRIX slot -- before
+  // the barrier in front of the first slot that reads it.  A half-tile is 16 pieces of 8 rows x 128
+  // bytes; wave wc of the group requests pieces 4 wc .. 4 wc + 3 of its group's two half-tiles:
+  //   ldA: group 0 W rows 0..127 (tile t + 1), group 1 x rows 128..255 (tile t + 1)
+  //   ldB: group 0 W rows 128..255 (tile t + 1), group 1 x rows 0..127 (tile t + 2)
+  // A lane's offsets inside a half-tile's buffer are the same for every tile.
+  int voff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int rr = (wc * 4 + i) * 8 + (lane >> 3);             // row inside the half-tile
+    const int c = (lane & 7) ^ gt_swz<FP8>(rr);                // logical 16-byte chunk this lane fetches
+    const int ni = (rr & 63) >> 4, ii = rr & 15, at8 = (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3);
+    // EPI 2: a tile is two heads; wave wcb serves head 2 tn + (wcb >> 1), rotation pairs d and d + 64 with
+    // d = 32 (wcb & 1) + at8: a lane ends with 8 d's and their partners.  Pairs: gt_half knows gate (ni < 2) from up.
+    const int n = gt_pairs(EPI) ? (rr >> 6) * 32 + at8 : EPI == 2 ? (rr >> 6) * 32 + at8 + (ni >> 1) * 64 : (rr >> 6) * 64 + at8 + (ni >> 1) * 32;
+    voff[i] = (g == 0 ? n * p.K : rr * (int)p.ldx) * ES + c * 16;
+  }
+  const int hA = g == 0 ? 0 : 1, hB = g == 0 ? 1 : 0;
+  auto rA = gt_half<EPI, ES>(p, cur.tm, cur.tn, g, wc, hA), rB = gt_half<EPI, ES>(p, cur.tm, cur.tn, g, wc, hB);
+  // LDS image of a K tile: x rows 0..255 (two halves), then W rows 0..255 (two halves)
+  constexpr int LX0 = 0, LX1 = GT_HALF, LW0 = 2 * GT_HALF, LW1 = 3 * GT_HALF;
+  char* const lds_w = sm + wc * 4096;   // this wave's four 1-KiB pieces inside a half-tile
+  const int ldA_l = g == 0 ? LW0 : LX1, ldB_l = g == 0 ? LW1 : LX0;
+  const int ldB_d = g == 0 ? 1 : 2;     // tile distance of the second request (the first is always t + 1)
+// four 1-KiB pieces of one half-tile: bytes `koff` .. of the rows of buffer r, to stage `stage` (a running number's parity)
+#define GT_REQUEST(r, koff, stage, ldso)                                                     \
+  _Pragma("unroll") for (int i = 0; i < 4; ++i)                                              \
+      blds16(r, lds_w + (((stage) & 1) ? GT_STAGE : 0) + (ldso) + i * 1024, voff[i], koff)
+
+  // ---- prologue: all of tile 0 and x rows 0..127 of tile 1 ------------------------------------
+  int koff = cur.t0 * 128;    // of K tile t
+  GT_REQUEST(rA, koff, 0, ldA_l);            // W0(0) | x1(0)
+  GT_REQUEST(rB, koff, 0, ldB_l);            // W1(0) | x0(0)
+  if (g == 1) GT_REQUEST(rB, koff + 128, 1, ldB_l);   // x0(1)
+
+  // ---- fragment read addresses ----------------------------------------------------------------
+  // 16-bit: fragment of k-step kk = chunk 4 kk + q4 (k-step 1 is rd0 ^ 64); fp8: the fragment of the
+  // whole 128-deep tile = chunks 2 q4 and 2 q4 + 1 (rd0 and rd0 ^ 16)
+  const int r16 = lane & 15, q4 = lane >> 4;
+  const int rd0 = r16 * 128 + (((FP8 ? 2 * q4 : q4) ^ gt_swz<FP8>(r16)) << 4);
+  const int a_off = g * GT_HALF, b_off = 2 * GT_HALF + wc * 8192;
+
+  f32x4 acc[8][4];
+  // two 16-byte registers per fragment slot: k-steps 0 / 1 (16-bit) or the two halves of the 32-byte
+  // fp8 fragment
+  i32x4 af[2][8], bf[2][4];
+  int s = 0;                  // running number of the K tile: which stage it lies in
+#define GT_TILE(FIRST, REQUESTS)                                                             \
+  do {                                                                                       \
+    const int cur_ = (s & 1) ? GT_STAGE : 0;                                                 \
+    /* READ slot: request the group's two half-tiles, read the fragments of the whole K tile */ \
+    REQUESTS                                                                                 \
+    _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) {                                       \
+      const int ro_ = rd0 ^ (FP8 ? (kk << 4) : (kk << 6));                                   \
+      const char* ab_ = sm + cur_ + a_off + ro_;                                             \
+      const char* bb_ = sm + cur_ + b_off + ro_;                                             \
+      _Pragma("unroll") for (int ni = 0; ni < 4; ++ni)                                       \
+          bf[kk][ni] = *reinterpret_cast<const i32x4*>(bb_ + ni * 2048);                     \
+      _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                       \
+          af[kk][mi] = *reinterpret_cast<const i32x4*>(ab_ + mi * 2048);                     \
+    }                                                                                        \
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                       \
+    GT_SLOT_END();                                                                           \
+    /* MATRIX slot: nothing but MFMAs, then the wave's requests of its READ slot must have landed */ \
+    __builtin_amdgcn_s_setprio(1);                                                           \
+    if constexpr (FP8) {                                                                     \
+      _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                       \
+        _Pragma("unroll") for (int nj = 0; nj < 4; ++nj) {                                   \
+          const int ni = (mi & 1) ? 3 - nj : nj;                                             \
+          const i32x8 a8_ = __builtin_shufflevector(bf[0][ni], bf[1][ni], 0, 1, 2, 3, 4, 5, 6, 7);\
+          const i32x8 b8_ = __builtin_shufflevector(af[0][mi], af[1][mi], 0, 1, 2, 3, 4, 5, 6, 7);\
+          acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(                    \
+              a8_, b8_, (FIRST) ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[mi][ni], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f); \
+        }                                                                                    \
+    } else {                                                                                 \
+      _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                       \
+        _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                     \
+          _Pragma("unroll") for (int nj = 0; nj < 4; ++nj) {                                 \
+              const int ni = (mi & 1) ? 3 - nj : nj;                                         \
+              acc[mi][ni] = Mfma<T>::run(__builtin_bit_cast(frag, bf[kk][ni]), __builtin_bit_cast(frag, af[kk][mi]), \
+                                         (FIRST) && kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[mi][ni]); \
+          }                                                                                  \
+    }                                                                                        \
+    __builtin_amdgcn_s_setprio(0);                                                           \
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                         \
+    GT_SLOT_END();                                                                           \
+    ++s; koff += 128;                                                                        \
+  } while (0)
+#define GT_REQUESTS_INSIDE { GT_REQUEST(rA, koff + 128, s + 1, ldA_l); GT_REQUEST(rB, koff + 128 * ldB_d, s + ldB_d, ldB_l); }
+
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile 0 (and x rows 0..127 of tile 1) have landed
+  GT_SLOT_END();
+  if (g == 1) GT_SLOT_END();   // the second group runs one slot behind the first
+  for (int item = 1;; ++item) {
+    const GtItem nxt = gt_item(p, item, kt);
+    const auto nA = gt_half<EPI, ES>(p, nxt.tm, nxt.tn, g, wc, hA), nB = gt_half<EPI, ES>(p, nxt.tm, nxt.tn, g, wc, hB);
+    const int nk = nxt.t0 * 128;
+    int t = 0;
+    if (!FP8 && cur.T > 2) {   // (sums that start in the MFMAs)
+      GT_TILE(true, GT_REQUESTS_INSIDE);
+      t = 1;
+    } else {
+#pragma unroll
+      for (int mi = 0; mi < 8; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (; t + 2 < cur.T; ++t) GT_TILE(false, GT_REQUESTS_INSIDE);
+    // The last two K tiles: x rows 0..127 and then everything is the next item's.  fp8 in a loop: as straight code the compiler moves
+    // those MFMAs behind the barriers, into the epilogue, with 480 bytes of spilled registers.
+    if constexpr (FP8) {
+#pragma unroll 1
+      for (; t < cur.T; ++t) {
+        const bool last = t + 1 == cur.T;
+        GT_TILE(false, {
+          if (!last) { GT_REQUEST(rA, koff + 128, s + 1, ldA_l); }
+          else if (nxt.valid) { GT_REQUEST(nA, nk, s + 1, ldA_l); }
+          if (!last && g == 0) { GT_REQUEST(rB, koff + 128, s + 1, ldB_l); }
+          else if (nxt.valid) { GT_REQUEST(nB, last && g == 1 ? nk + 128 : nk, last ? s + ldB_d : s, ldB_l); }
+        });
+      }
+    } else {
+      GT_TILE(false, {
+        GT_REQUEST(rA, koff + 128, s + 1, ldA_l);
+        if (g == 0) { GT_REQUEST(rB, koff + 128, s + 1, ldB_l); }
+        else if (nxt.valid) { GT_REQUEST(nB, nk, s, ldB_l); }
+      });
+      GT_TILE(false, {
+        if (nxt.valid) {
+          GT_REQUEST(nA, nk, s + 1, ldA_l);
+          GT_REQUEST(nB, nk + 128 * (ldB_d - 1), s + ldB_d, ldB_l);
+        }
+      });
+    }
+    if (!nxt.valid && g == 0) __builtin_amdgcn_s_barrier();   // (the other group is one slot behind)
+    if (cur.part != nullptr) {   // a split of a tail tile: its sums as they lie in the registers
+#pragma unroll
+      for (int mi = 0; mi < 8; ++mi)
+        if (cur.tm * 256 + g * 128 + mi * 16 < p.M)
+#pragma unroll
+          for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(cur.part + ((wave * 8 + mi) * 4 + ni) * 256 + lane * 4) = acc[mi][ni];
+    } else if (EPI == 0 && p.bias != nullptr) {
+      tile_epilogue<T, EPI, FP8, 8, true>(p, acc, cur.tm * 256 + g * 128, cur.tm, cur.tn, wc, q4, r16, 256);
+    } else {
+      tile_epilogue<T, EPI, FP8, 8, false>(p, acc, cur.tm * 256 + g * 128, cur.tm, cur.tn, wc, q4, r16, 256);
+    }
+    if (!nxt.valid) break;
+    cur = nxt;
+    rA = nA;
+    rB = nB;
+    koff = nk;
+  }
+#undef GT_REQUEST
+#undef GT_REQUESTS_INSIDE
+#undef GT_TILE
+}
+
+// The grouped products: a workgroup per tile, in blocks of 8 x 4 tiles (only the device knows how many tiles there are).
+// MIXED: tiles without padding are as likely as tiles with; a wave whose rows are all there then takes a loop without the
+// conditions that leave padding out.  Those cost a full tile 5 %, the second loop a mostly empty one 3 to 6 (32 experts of 2048 x
+// 2048, 4 per token, both products: 8192 tokens 663 -> 624 us with it, 3000 297 -> 288, 1024 193 -> 197; 256 of 2048 x 512, 8 per
+// token, 64 tokens 304 -> 322).
+template <typename T, bool MIXED>
+__global__ __launch_bounds__(512) void gemm_grouped_kernel(GemmTiledParams p) {
+  extern __shared__ __attribute__((aligned(16))) char sm[];
+  using frag = typename Mfma<T>::frag;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = wave >> 2, wc = wave & 3;
 
   // ---- workgroup -> output tile ------------------------------------------------------------
-  // Consecutive workgroups go to the eight XCDs in turn.  EPI 3, whose tile count only the device knows: blocks of 8 x 4 tiles
-  // in turn.  Otherwise every XCD gets an equal run of the tiles in block order (bands of 8 rows, blocks of 4 columns inside):
-  // whole blocks in turn left some XCDs a round more than others where the last band is short -- 18 x 24 tiles: 72 on two
-  // XCDs and 40 on four, of 32 CUs each.  M = 4605, K = 4096: N = 6144 267 -> 190 us, N = 28672 846 -> 792; 7381 x 2048 -> 2 x 5632 302 -> 280.
+  // Consecutive workgroups go to the eight XCDs in turn: blocks of 8 x 4 tiles in turn.
   const int b = blockIdx.x, li = b >> 3;
-  int tm, tn, T_ = (p.K * ES) >> 7, t0 = 0;   // K tiles of 128 bytes per row, and the first one of a split
-  float* part = nullptr;
-  if constexpr (EPI == 3) {
+  int tm, tn;
+  const int T_ = p.K >> 6;     // K tiles of 128 bytes per row
+  {
     const int st = (li >> 5) * 8 + (b & 7), within = li & 31;
     if (st >= p.nsuper) return;
     const int sup_m = st / p.snt, sup_n = st - sup_m * p.snt;
@@ -377,42 +618,24 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     tm = sup_m * 8 + __builtin_ctz(of);
     tn = sup_n * 4 + (within & 3);
     if (tm >= used || tn >= p.nt) return;
-  } else if (p.splits == 0 || b < p.full) {
-    const int at = (b & 7) * (p.splits == 0 ? (int)(gridDim.x >> 3) : p.full >> 3) + li;
-    if (at >= p.mt * p.nt) return;
-    tile_of(p, at, tm, tn);
-  } else {
-    // a split of a tail tile; every XCD takes neighbouring splits, one stretch of K of all the tail's operands
-    const int u = b - p.full, at = (u & 7) * (int)((gridDim.x - p.full) >> 3) + (u >> 3);
-    if (at >= p.tail * p.splits) return;
-    const int k = at / p.tail, t = at - k * p.tail;
-    tile_of(p, p.full + t, tm, tn);
-    part = p.part + ((int64_t)k * p.tail + t) * 65536;
-    const int all = T_;
-    t0 = all * k / p.splits;
-    T_ = all * (k + 1) / p.splits - t0;
   }
-  // EPI 3: rows of the tile up to the last one that is no padding (a plan's padding lies behind them; between them it reads row 0).
+  // Rows of the tile up to the last one that is no padding (a plan's padding lies behind them; between them it reads row 0).
   // Padding rows are neither loaded, multiplied nor stored, 8, 16 and 1 at a time: an expert's last tile is as long as its rows.  64 tokens x 4 of 32 experts (2048 x 2048):
   // 88 us with padding worked on, 55 without (268 MB of weights); 1024 tokens: 85 and 72; 3000 tokens: 148 and 145.
   int live = 256;
-  if constexpr (EPI == 3) {
-    if (p.row_map != nullptr) {
-      live = 0;
+  if (p.row_map != nullptr) {
+    live = 0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const unsigned long long there = __ballot(p.row_map[tm * 256 + i * 64 + lane] >= 0);
-        live = there != 0 ? 64 * i + 64 - __clzll(there) : live;
-      }
-      live = __builtin_amdgcn_readfirstlane(live);
+    for (int i = 0; i < 4; ++i) {
+      const unsigned long long there = __ballot(p.row_map[tm * 256 + i * 64 + lane] >= 0);
+      live = there != 0 ? 64 * i + 64 - __clzll(there) : live;
     }
+    live = __builtin_amdgcn_readfirstlane(live);
   }
-  const int live_mi = EPI == 3 ? min(max((live - g * 128 + 15) >> 4, 0), 8) : 8;
+  const int live_mi = min(max((live - g * 128 + 15) >> 4, 0), 8);
 
   const char* xg = (const char*)p.x;
-  const char* wg = (const char*)p.w;
-  if constexpr (EPI == 3) wg += (int64_t)p.tile_expert[tm] * p.w_expert_stride * ES;
-  const int ncols = gt_pairs(EPI) ? (p.N >> 1) : p.N;   // output columns
+  const char* wg = (const char*)p.w + (int64_t)p.tile_expert[tm] * p.w_expert_stride * 2;
 
   // ---- per-lane source pointers of the eight load instructions a wave issues per K tile -----
   // A wave requests data only in its READ slot (a load-to-LDS holds the issuing wave ~40 cycles: in
@@ -430,36 +653,23 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int rr = (wc * 4 + i) * 8 + (lane >> 3);             // row inside the half-tile
-    const int c = (lane & 7) ^ gt_swz<FP8>(rr);                // logical 16-byte chunk this lane fetches
+    const int c = (lane & 7) ^ gt_swz<false>(rr);                // logical 16-byte chunk this lane fetches
     const char* xs[2];
     const char* ws[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       int m = tm * 256 + h * 128 + rr;
       m = m < p.M ? m : p.M - 1;
-      if constexpr (EPI == 3) {
-        // gathered rows; a padding row reads row 0 (its products are not stored)
-        if (p.gather) m = max(p.row_map[m], 0);
-      }
-      xs[h] = xg + ((int64_t)m * p.ldx) * ES + c * 16;
+      // gathered rows; a padding row reads row 0 (its products are not stored)
+      if (p.gather) m = max(p.row_map[m], 0);
+      xs[h] = xg + ((int64_t)m * p.ldx) * 2 + c * 16;
       const int rb = h * 128 + rr, wcb = rb >> 6, sl = rb & 63, ni = sl >> 4, ii = sl & 15;
-      int n;
-      if (gt_pairs(EPI)) {
-        int j = tn * 128 + wcb * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3);
-        j = j < ncols ? j : ncols - 1;
-        n = j + (ni >> 1) * ncols;
-      } else if (EPI == 2) {
-        // a tile is two heads; wave wcb serves head 2 tn + (wcb >> 1), rotation pairs d and d + 64 with
-        // d = 32 (wcb & 1) + 8 (ii >> 2) + 4 (ni & 1) + (ii & 3): a lane ends with 8 d's and their partners
-        n = (2 * tn + (wcb >> 1)) * 128 + (wcb & 1) * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3) + (ni >> 1) * 64;
-      } else {
-        n = tn * 256 + wcb * 64 + (ii >> 2) * 16 + ni * 4 + (ii & 3);
-        n = n < p.N ? n : p.N - 1;
-      }
-      ws[h] = wg + ((int64_t)n * p.K) * ES + c * 16;
+      int n = tn * 256 + wcb * 64 + (ni >> 1) * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3);
+      n = n < p.N ? n : p.N - 1;
+      ws[h] = wg + ((int64_t)n * p.K) * 2 + c * 16;
     }
-    ldA[i] = (g == 0 ? ws[0] : xs[1]) + (int64_t)t0 * 128;
-    ldB[i] = (g == 0 ? ws[1] : xs[0]) + (int64_t)t0 * 128;
+    ldA[i] = g == 0 ? ws[0] : xs[1];
+    ldB[i] = g == 0 ? ws[1] : xs[0];
   }
   // LDS image of a K tile: x rows 0..255 (two halves), then W rows 0..255 (two halves)
   constexpr int LX0 = 0, LX1 = GT_HALF, LW0 = 2 * GT_HALF, LW1 = 3 * GT_HALF;
@@ -467,13 +677,13 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const int ldA_l = g == 0 ? LW0 : LX1, ldB_l = g == 0 ? LW1 : LX0;
   const int ldB_d = g == 0 ? 1 : 2;     // tile distance of the second request (the first is always t + 1)
 
-  // EPI 3: every expert's K is walked from another tile on and round the end.  Rows of operands lie 4 KB or more apart, so workgroups in
+  // Every expert's K is walked from another tile on and round the end.  Rows of operands lie 4 KB or more apart, so workgroups in
   // step ask for the same 128-byte column of all the weights and with it for few memory channels.  A layer of 32 experts of 2048 x 2048, 4
   // per token, us with K from its start -> staggered: 16 tokens 154 -> 131, 131 tokens 187 -> 144 (one product 75 -> 53: 268 MB at 5.1 TB/s),
   // 1000 309 -> 279, 3000 325 -> 310; by column of tiles as well 147 at 131, by that alone 167.  A dense product's rows and columns have one order
   // of K each, whichever tile they are in and whatever is fused behind it.
-  const int rot = EPI == 3 ? p.tile_expert[tm] % T_ : 0;
-#define GT_AT(tl) ((int64_t)(EPI == 3 && (tl) + rot >= T_ ? (tl) + rot - T_ : (tl) + rot) * 128)
+  const int rot = p.tile_expert[tm] % T_;
+#define GT_AT(tl) ((int64_t)((tl) + rot >= T_ ? (tl) + rot - T_ : (tl) + rot) * 128)
 
   // ---- prologue: all of tile 0 and x rows 0..127 of tile 1 ------------------------------------
 #pragma unroll
@@ -486,10 +696,9 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   }
 
   // ---- fragment read addresses ----------------------------------------------------------------
-  // 16-bit: fragment of k-step kk = chunk 4 kk + q4 (k-step 1 is rd0 ^ 64); fp8: the fragment of the
-  // whole 128-deep tile = chunks 2 q4 and 2 q4 + 1 (rd0 and rd0 ^ 16)
+  // fragment of k-step kk = chunk 4 kk + q4 (k-step 1 is rd0 ^ 64)
   const int r16 = lane & 15, q4 = lane >> 4;
-  const int rd0 = r16 * 128 + (((FP8 ? 2 * q4 : q4) ^ gt_swz<FP8>(r16)) << 4);
+  const int rd0 = r16 * 128 + ((q4 ^ gt_swz<false>(r16)) << 4);
   const int a_off = g * GT_HALF, b_off = 2 * GT_HALF + wc * 8192;
 
   f32x4 acc[8][4];
@@ -497,13 +706,11 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   for (int mi = 0; mi < 8; ++mi)
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // two 16-byte registers per fragment slot: k-steps 0 / 1 (16-bit) or the two halves of the 32-byte
-  // fp8 fragment
   i32x4 af[2][8], bf[2][4];
 
   // how many of the wave's four pieces of x rows 128..255 (ldA of group 1) and 0..127 (ldB) hold rows that are no padding
-  const int nA = EPI == 3 && g == 1 ? min(max((live - 128 - wc * 32 + 7) >> 3, 0), 4) : 4;
-  const int nB = EPI == 3 && g == 1 ? min(max((live - wc * 32 + 7) >> 3, 0), 4) : 4;
+  const int nA = g == 1 ? min(max((live - 128 - wc * 32 + 7) >> 3, 0), 4) : 4;
+  const int nB = g == 1 ? min(max((live - wc * 32 + 7) >> 3, 0), 4) : 4;
 // four 1-KiB pieces of one half-tile of tile `tl`; TAIL: nothing past the last tile
 #define GT_LOAD4(ptr, ldso, tl, TAIL, PART, COUNT)                                           \
   do {                                                                                       \
@@ -513,12 +720,6 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
           if (!(PART) || i < (COUNT)) glds16(ptr[i] + GT_AT(tl), d_ + i * 1024);   \
     }                                                                                        \
   } while (0)
-#define GT_SLOT_END()                                                                        \
-  do {                                                                                       \
-    __builtin_amdgcn_sched_barrier(0);                                                       \
-    __builtin_amdgcn_s_barrier();                                                            \
-    __builtin_amdgcn_sched_barrier(0);                                                       \
-  } while (0)
 #define GT_TILE(t, TAIL, PART)                                                               \
   do {                                                                                       \
     const int cur_ = ((t) & 1) ? GT_STAGE : 0;                                               \
@@ -526,7 +727,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     GT_LOAD4(ldA, ldA_l, (t) + 1, TAIL, PART, nA);                                           \
     GT_LOAD4(ldB, ldB_l, (t) + ldB_d, TAIL, PART, nB);                                       \
     _Pragma("unroll") for (int kk = 0; kk < 2; ++kk) {                                       \
-      const int ro_ = rd0 ^ (FP8 ? (kk << 4) : (kk << 6));                                   \
+      const int ro_ = rd0 ^ (kk << 6);                                                        \
       const char* ab_ = sm + cur_ + a_off + ro_;                                             \
       const char* bb_ = sm + cur_ + b_off + ro_;                                             \
       _Pragma("unroll") for (int ni = 0; ni < 4; ++ni)                                       \
@@ -538,25 +739,14 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     GT_SLOT_END();                                                                           \
     /* MATRIX slot: nothing but MFMAs, then the wave's requests of its READ slot must have landed */ \
     __builtin_amdgcn_s_setprio(1);                                                           \
-    if constexpr (FP8) {                                                                     \
+    _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                         \
       _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                       \
+        if (!(PART) || mi < live_mi)                                                         \
         _Pragma("unroll") for (int nj = 0; nj < 4; ++nj) {                                   \
-          const int ni = (mi & 1) ? 3 - nj : nj;                                             \
-          const i32x8 a8_ = __builtin_shufflevector(bf[0][ni], bf[1][ni], 0, 1, 2, 3, 4, 5, 6, 7);\
-          const i32x8 b8_ = __builtin_shufflevector(af[0][mi], af[1][mi], 0, 1, 2, 3, 4, 5, 6, 7);\
-          acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(                    \
-              a8_, b8_, acc[mi][ni], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);                    \
+            const int ni = (mi & 1) ? 3 - nj : nj;                                           \
+            acc[mi][ni] = Mfma<T>::run(__builtin_bit_cast(frag, bf[kk][ni]),                 \
+                                       __builtin_bit_cast(frag, af[kk][mi]), acc[mi][ni]);   \
         }                                                                                    \
-    } else {                                                                                 \
-      _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                       \
-        _Pragma("unroll") for (int mi = 0; mi < 8; ++mi)                                     \
-          if (!(PART) || mi < live_mi)                                                       \
-          _Pragma("unroll") for (int nj = 0; nj < 4; ++nj) {                                 \
-              const int ni = (mi & 1) ? 3 - nj : nj;                                         \
-              acc[mi][ni] = Mfma<T>::run(__builtin_bit_cast(frag, bf[kk][ni]),               \
-                                         __builtin_bit_cast(frag, af[kk][mi]), acc[mi][ni]); \
-          }                                                                                  \
-    }                                                                                        \
     __builtin_amdgcn_s_setprio(0);                                                           \
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                         \
     GT_SLOT_END();                                                                           \
@@ -566,7 +756,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   GT_SLOT_END();
   if (g == 1) GT_SLOT_END();   // the second group runs one slot behind the first
   int t = 0;
-  if (EPI == 3 && (!MIXED || live_mi < 8 || nA < 4 || nB < 4)) {   // (per wave; the barriers are as many either way)
+  if (!MIXED || live_mi < 8 || nA < 4 || nB < 4) {   // (per wave; the barriers are as many either way)
     for (; t + 2 < T_; ++t) GT_TILE(t, false, true);
     for (; t < T_; ++t) GT_TILE(t, true, true);
   } else {
@@ -575,23 +765,12 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   }
   if (g == 0) __builtin_amdgcn_s_barrier();
 #undef GT_LOAD4
-#undef GT_SLOT_END
 #undef GT_TILE
 #undef GT_AT
 
-  // ---- epilogue ---------------------------------------------------------------------------------
-  if constexpr (EPI != 3) {
-    if (part != nullptr) {   // a split of a tail tile: its sums as they lie in the registers
-#pragma unroll
-      for (int mi = 0; mi < 8; ++mi)
-        if (tm * 256 + g * 128 + mi * 16 < p.M)
-#pragma unroll
-          for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(part + ((wave * 8 + mi) * 4 + ni) * 256 + lane * 4) = acc[mi][ni];
-      return;
-    }
-  }
-  tile_epilogue<T, EPI, FP8, 8>(p, acc, tm * 256 + g * 128, tm, tn, wc, q4, r16, live);
+  tile_epilogue<T, 3, false, 8, false>(p, acc, tm * 256 + g * 128, tm, tn, wc, q4, r16, live);
 }
+#undef GT_SLOT_END
 
 // Sums the splits of the tail tiles in their order and finishes the tiles: a wave takes one 16-row group of one of the tile's waves,
 // its lanes' values in the order in which they were left (whole 1-KiB lines).
@@ -613,22 +792,28 @@ __global__ __launch_bounds__(256) void gemm_tiled_tail_kernel(GemmTiledParams p)
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) acc[0][ni] += *reinterpret_cast<const f32x4*>(src + (int64_t)k * p.tail * 65536 + ni * 256);
   }
-  tile_epilogue<T, EPI, FP8, 1>(p, acc, m0, tm, tn, wc, q4, r16, 256);
+  if (EPI == 0 && p.bias != nullptr) tile_epilogue<T, EPI, FP8, 1, true>(p, acc, m0, tm, tn, wc, q4, r16, 256);
+  else tile_epilogue<T, EPI, FP8, 1, false>(p, acc, m0, tm, tn, wc, q4, r16, 256);
 }
 
-template <typename T, int EPI, bool FP8, bool MIXED = false>
+template <typename T, int EPI, bool FP8>
 int launch_gemm_tiled(const GemmTiledParams& p, hipStream_t st) {
-  auto kern = gemm_tiled_kernel<T, EPI, FP8, MIXED>;
+  auto kern = gemm_tiled_kernel<T, EPI, FP8>;
   (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS);
-  // 8 x 4 blocks, or tiles, in equal numbers for every XCD
-  const int per = EPI == 3 ? (p.nsuper + 7) / 8 * 32 : p.splits == 0 ? (int)cdiv((int64_t)p.mt * p.nt, 8)
-                                                     : p.full / 8 + (int)cdiv((int64_t)p.tail * p.splits, 8);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(per * 8)), dim3(512), GT_LDS, st, p);
-  if constexpr (EPI != 3) {
-    if (p.splits != 0) hipLaunchKernelGGL((gemm_tiled_tail_kernel<T, EPI, FP8>), dim3((unsigned)p.tail * 16), dim3(256), 0, st, p);
-  }
-  MI355_CHECK_LAUNCH(EPI == 3 ? "mi355_moe_grouped_linear_tiled" : EPI == 2 ? "mi355_qkv_proj_rope_tiled"
-                     : FP8 ? "mi355_fp8_scaled_mm_tiled" : "mi355_linear_tiled");
+  // workgroups that stay: as many as there are CUs, in equal numbers for every XCD (with whole tiles in front of a tail: all of them)
+  const int per = p.splits == 0 ? (int)cdiv((int64_t)p.mt * p.nt, 8) : std::max(p.full / 8, (int)cdiv((int64_t)p.tail * p.splits, 8));
+  hipLaunchKernelGGL(kern, dim3((unsigned)(std::min(per, 32) * 8)), dim3(512), GT_LDS, st, p);
+  if (p.splits != 0) hipLaunchKernelGGL((gemm_tiled_tail_kernel<T, EPI, FP8>), dim3((unsigned)p.tail * 16), dim3(256), 0, st, p);
+  MI355_CHECK_LAUNCH(EPI == 2 ? "mi355_qkv_proj_rope_tiled" : FP8 ? "mi355_fp8_scaled_mm_tiled" : "mi355_linear_tiled");
+  return MI355_OK;
+}
+
+template <typename T, bool MIXED>
+int launch_gemm_grouped(const GemmTiledParams& p, hipStream_t st) {
+  auto kern = gemm_grouped_kernel<T, MIXED>;
+  (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((p.nsuper + 7) / 8 * 32 * 8)), dim3(512), GT_LDS, st, p);   // 8 x 4 blocks in equal numbers for every XCD
+  MI355_CHECK_LAUNCH("mi355_moe_grouped_linear_tiled");
   return MI355_OK;
 }
 
@@ -711,7 +896,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_few_kernel(GemmTiledPa
       const int r = row - BM, G = tn * WN + (r >> 6), ni = (r & 63) >> 4, ii = r & 15;   // the wave's 64 columns, as tile_epilogue has them
       int n;
       if (EPI == 1) n = min(G * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3), ncols - 1) + (ni >> 1) * ncols;
-      else n = min(G * 64 + (ii >> 2) * 16 + ni * 4 + (ii & 3), p.N - 1);
+      else n = min(G * 64 + (ni >> 1) * 32 + (ii >> 2) * 8 + (ni & 1) * 4 + (ii & 3), p.N - 1);
       src[i] = (const char*)p.w + (int64_t)n * p.K * ES + c * 16;
     }
     src[i] += (int64_t)t0 * 128;
@@ -809,7 +994,8 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_few_kernel(GemmTiledPa
         for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(part + mi * 1024 + ni * 256) = acc[mi][ni];
     return;
   }
-  tile_epilogue<T, EPI, FP8, NM>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+  if (EPI == 0 && p.bias != nullptr) tile_epilogue<T, EPI, FP8, NM, true>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+  else tile_epilogue<T, EPI, FP8, NM, false>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
 }
 
 // A wave adds the splits' sums of 16 rows x 64 columns (W rows) in their order and finishes them.
@@ -828,7 +1014,8 @@ __global__ __launch_bounds__(256) void gemm_few_tail_kernel(GemmTiledParams p, i
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) acc[0][ni] += *reinterpret_cast<const f32x4*>(src + (int64_t)k * groups * rows16 * 1024 + ni * 256);
   }
-  tile_epilogue<T, EPI, FP8, 1>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+  if (EPI == 0 && p.bias != nullptr) tile_epilogue<T, EPI, FP8, 1, true>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+  else tile_epilogue<T, EPI, FP8, 1, false>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
 }
 
 template <typename T, int EPI, bool FP8, int NM, int WM, int WN, int KS, int NS>
@@ -905,7 +1092,7 @@ extern "C" int64_t mi355_tiled_tail_workspace_bytes(int64_t m, int64_t n, int64_
 
 extern "C" int mi355_linear_tiled_supported(int64_t m, int64_t n, int64_t k, int dtype, int epilogue) {
   if (dtype != MI355_BF16 && dtype != MI355_F16) return 0;
-  if (m < 1 || n < 16 || k < 128 || (k & 63) != 0 || m > (1 << 24) || n > (1 << 24)) return 0;
+  if (m < 1 || n < 16 || k < 128 || (k & 63) != 0 || m > (1 << 24) || n > (1 << 24) || k > GT_MAX_STRIDE) return 0;
   return (epilogue >= 0 && epilogue <= 3 && n % 16 == 0) ? 1 : 0;   // silu-mul: 8 gate + 8 up columns per lane
 }
 
@@ -922,8 +1109,8 @@ extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, cons
   MI355_REQUIRE(mi355_linear_tiled_supported(m, n, k, dtype, epilogue), MI355_ERR_UNSUPPORTED,
                 "mi355_linear_tiled: needs a 16-bit dtype, K %% 64 == 0, K >= 128, N %% 16 == 0 (m=%ld n=%ld k=%ld "
                 "dtype=%d epilogue=%d)", (long)m, (long)n, (long)k, dtype, epilogue);
-  MI355_REQUIRE(x_stride >= k && x_stride % 8 == 0, MI355_ERR_INVALID,
-                "mi355_linear_tiled: x_stride must be >= K and a multiple of 8 elements");
+  MI355_REQUIRE(x_stride >= k && x_stride % 8 == 0 && x_stride <= GT_MAX_STRIDE, MI355_ERR_INVALID,
+                "mi355_linear_tiled: x_stride must be >= K, a multiple of 8 elements and below 2^23");
   MI355_REQUIRE(aligned16(x) && aligned16(w) && aligned16(y) && (bias == nullptr || aligned16(bias)),
                 MI355_ERR_INVALID, "mi355_linear_tiled: pointers must be 16-byte aligned");
   MI355_REQUIRE(epilogue == 0 || bias == nullptr, MI355_ERR_UNSUPPORTED,
@@ -1007,8 +1194,8 @@ int moe_grouped_linear_tiled(void* y, const void* x, int64_t x_stride, const voi
   fill_tiles(p, rows, n, 0);
   p.row_map = row_map; p.gather = gather; p.tile_expert = tile_expert; p.tiles_used = tiles_used; p.w_expert_stride = n * k; p.act = act;
   hipStream_t st = (hipStream_t)stream;
-  if (mixed) return dtype == MI355_BF16 ? launch_gemm_tiled<bf16_t, 3, false, true>(p, st) : launch_gemm_tiled<f16_t, 3, false, true>(p, st);
-  return dtype == MI355_BF16 ? launch_gemm_tiled<bf16_t, 3, false>(p, st) : launch_gemm_tiled<f16_t, 3, false>(p, st);
+  if (mixed) return dtype == MI355_BF16 ? launch_gemm_grouped<bf16_t, true>(p, st) : launch_gemm_grouped<f16_t, true>(p, st);
+  return dtype == MI355_BF16 ? launch_gemm_grouped<bf16_t, false>(p, st) : launch_gemm_grouped<f16_t, false>(p, st);
 }
 }  // namespace mi355
 
@@ -1021,7 +1208,7 @@ extern "C" int mi355_moe_grouped_linear_tiled(void* y, const void* x, int64_t x_
 
 extern "C" int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out_dtype, int epilogue) {
   if (out_dtype != MI355_BF16 && out_dtype != MI355_F16) return 0;
-  if (m < 1 || n < 16 || k < 256 || (k & 127) != 0 || m > (1 << 24) || n > (1 << 24)) return 0;
+  if (m < 1 || n < 16 || k < 256 || (k & 127) != 0 || m > (1 << 24) || n > (1 << 24) || k > GT_MAX_STRIDE) return 0;
   return ((epilogue == 0 || epilogue == 1) && n % 16 == 0) ? 1 : 0;
 }
 
@@ -1060,7 +1247,7 @@ extern "C" int mi355_qkv_proj_rope_tiled_supported(int64_t m, int64_t k, int hq,
                                                    int rotary_dim, int is_neox, int dtype, int fp8) {
   if (dtype != MI355_BF16 && dtype != MI355_F16) return 0;
   if (head_dim != 128 || rotary_dim != 128 || !is_neox || hq < 1 || hkv < 1 || ((hq + 2 * hkv) & 1)) return 0;
-  if (m < 1 || m > (1 << 24)) return 0;
+  if (m < 1 || m > (1 << 24) || k > GT_MAX_STRIDE) return 0;
   return fp8 ? (k >= 256 && (k & 127) == 0) : (k >= 128 && (k & 63) == 0);
 }
 
@@ -1097,7 +1284,7 @@ extern "C" int mi355_qkv_proj_rope_tiled_ws(void* qkv, const void* x, const void
                 "mi355_qkv_proj_rope_tiled: cos_sin_cache must be fp32 or the tensor dtype");
   MI355_REQUIRE(loc_itype == MI355_I32 || loc_itype == MI355_I64, MI355_ERR_INVALID,
                 "mi355_qkv_proj_rope_tiled: loc must be int32 or int64");
-  MI355_REQUIRE(fp8 ? x_stride == k : (x_stride >= k && x_stride % 8 == 0), MI355_ERR_INVALID,
+  MI355_REQUIRE(fp8 ? x_stride == k : (x_stride >= k && x_stride % 8 == 0 && x_stride <= GT_MAX_STRIDE), MI355_ERR_INVALID,
                 "mi355_qkv_proj_rope_tiled: bad x_stride");
   MI355_REQUIRE(aligned16(x) && aligned16(w) && aligned16(qkv) && aligned16(cos_sin_cache) && aligned16(k_buffer) &&
                     aligned16(v_buffer) && num_slots > 0 && num_slots < (1ll << 31),

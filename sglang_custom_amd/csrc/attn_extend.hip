@@ -583,9 +583,23 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // careful (D = 64): value rows may hold infinities and NaN, which no product with a weight of zero may meet (keys that the query does not
 // see) nor with a weight's lower terms.  The images then hold the rows without them, and beside them, in the half that is free, the rows
 // as they are, from which they are added for the queries that see their key.  Returns (the same in all threads) whether a result is no number.
+// DIRECT: the load unit writes the K/V images itself (buffer loads to LDS), the next tile's into a second stage while this one is worked on: one
+// barrier a tile, and no registers, addresses of 64 bits or LDS stores for it.  A quarter of a launch was the tile's way through
+// registers (1 x 4000 tokens, 32 / 8 heads: 168 us, 127 without any loads after the first tile; 4 x 490 on 1750 cached 90 and 63).  Rows of a tile are
+// addressed with 32 bits: from the head's first cached row, or from the tile's own first row of this launch.  (global_load_lds would do without
+// that, but the compiler takes it for a flat access and then waits for every LDS read behind it to the last one: 173 us.)
+// us a launch, 16-bit rows: registers | DIRECT | and the weights of a k-step made beside the MFMAs of the one before, MFMAs at a raised wave
+// priority: 5 x 1100 ragged 49.5 | 45.5 | 43.5; 4 x 515 on 1999 ragged 93.7 | 81.4 | 79.0; 192-wide latents of 4 x 2048
+// tokens, 32 heads 238 | 213 | 204, 16 heads 131 | 114 | 108; 1 x 4000 179 | 163 | 155.
 // SPLIT: gridDim.y workgroups share the block's key tiles, in runs of at least SPLIT_TILES; extend_split_merge_kernel adds their sums.
 constexpr int SPLIT_TILES = 4;
-template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128, bool MASK = false, bool SPLIT = false>
+template <int DQ> constexpr int direct_stage_bytes() { return 2 * 64 * 256 + (DQ > 128 ? 64 * 128 : 0); }
+// A buffer of 4 GiB from p on, and 16 bytes a lane of it to LDS (l and the lanes behind it)
+__device__ __forceinline__ auto wide_rsrc(const void* p) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, -1, 0x00020000); }
+__device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t r, char* l, unsigned off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)l, 16, (int)off, 0, 0, 0);
+}
+template <typename T, bool KV8, int DQ, bool LATENT = false, int D = 128, bool MASK = false, bool SPLIT = false, bool DIRECT = false>
 __device__ __forceinline__ bool extend_attn_mfma32_body(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, const ExtendParams& p, int nqb, int npairs, bool careful = false) {
@@ -597,9 +611,13 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
   constexpr int ND = D / 32;      // 32-feature tiles of the output
   static_assert((D == 128 && (DQ == 128 || (DQ == 192 && !KV8))) || (D == 64 && DQ == 64), "64, 128, or 192 + 128 over a 16-bit cache");
   using frag = typename Mfma32<T>::frag;
-  __shared__ __attribute__((aligned(16))) char ks[64 * 256];
-  __shared__ __attribute__((aligned(16))) char ks2[WIDE ? 64 * 256 : 16];
-  __shared__ __attribute__((aligned(16))) char vs[64 * 256];
+  static_assert(!DIRECT || (D == 128 && !KV8 && (DQ == 128 || LATENT)), "16-bit rows, from the cache or of this launch");
+  constexpr int STAGE = direct_stage_bytes<DQ>();
+  extern __shared__ __attribute__((aligned(16))) char sm_direct[];
+  __shared__ __attribute__((aligned(16))) char sm_images[DIRECT ? 16 : (WIDE ? 3 : 2) * 64 * 256 + 16];
+  char* const ks = DIRECT ? sm_direct : sm_images;
+  char* const vs = ks + 64 * 256;
+  char* const ks2 = vs + 64 * 256;
 
   int tid = (int)threadIdx.x;
   if (careful) asm volatile("" : "+v"(tid));    // (addresses of its own: the first pass's would be kept for it in scratch memory)
@@ -686,6 +704,7 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
   const int my_limit = causal ? prefix + qrow_c : prefix + ext - 1;   // last visible key of this lane's query
   const int wave_min_limit = causal ? prefix + min(r0 + wave * 32, ext - 1) : prefix + ext - 1;
   const int wave_max_limit = causal ? prefix + min(r0 + wave * 32 + 31, ext - 1) : prefix + ext - 1;
+  const bool no_rows = r0 + __builtin_amdgcn_readfirstlane(wave) * 32 >= ext;
   const uint8_t* mask_row = MASK ? p.custom_mask + p.mask_indptr[b] + (int64_t)qrow_c * (prefix + ext) : nullptr;
 
   // tile staging: thread -> rows tid / CH + SR i, 16-B chunk tid % CH
@@ -786,6 +805,49 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     }
   };
 
+  // DIRECT: rows srow + 16 i of a tile go to the image's rows 4 wave + 16 i .. + 3 (1 KiB a wave, in the lanes' order); lane sch of a row fetches the
+  // chunk that belongs there.  Rows of this launch: the tile's first row is the buffer's base; cached ones: the head's first.
+  [[maybe_unused]] const unsigned gch = (sch ^ (((srow & 3) << 2) | ((srow >> 2) & 3))) * 16u, gch2 = (sch2 ^ ((srow2 >> 1) & 7)) * 16u;
+  [[maybe_unused]] const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
+  [[maybe_unused]] auto direct_tile = [&](int kt, int stage) {
+    char* const dst = sm_direct + stage * STAGE + 1024 * wave_u;
+    const int64_t tok = (int64_t)q_start - prefix + kt * 64;
+    const int left = total - kt * 64;      // rows of the tile that exist
+    if (LATENT || kt * 64 >= prefix) {
+      const auto rk = wide_rsrc(k_ext + tok * p.k_stride + (int64_t)kvh * (LATENT ? p.kv_head : DQ));
+      const auto rv = wide_rsrc(v_ext + tok * p.v_stride + (int64_t)kvh * (LATENT ? p.kv_head : D));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = min(srow + 16 * i, left - 1);
+        buffer_to_lds16(rk, dst + 4096 * i, row * (unsigned)p.k_stride * 2 + gch);
+        buffer_to_lds16(rv, dst + 16384 + 4096 * i, row * (unsigned)p.v_stride * 2 + gch);
+      }
+      if constexpr (LATENT) {
+        const auto rr = wide_rsrc((const T*)p.k_rope + tok * p.k_rope_stride);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) buffer_to_lds16(rr, dst + 32768 + 4096 * j, min(srow2 + 32 * j, left - 1) * (unsigned)p.k_rope_stride * 2 + gch2);
+      }
+    } else if (kt * 64 + 64 <= prefix) {
+      const auto rk = wide_rsrc(kbuf + kvh * p.kb_head), rv = wide_rsrc(vbuf + kvh * p.vb_head);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        buffer_to_lds16(rk, dst + 4096 * i, next_slot[i] * (unsigned)(p.kb_slot * 2) + gch);
+        buffer_to_lds16(rv, dst + 16384 + 4096 * i, next_slot[i] * (unsigned)(p.vb_slot * 2) + gch);
+      }
+    } else {   // the tile that holds the prefix's last rows and the first new ones: through registers
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = min(kt * 64 + srow + 16 * i, total - 1);
+        const bool old = key < prefix;
+        const T* kp = old ? kbuf + (int64_t)next_slot[i] * p.kb_slot + kvh * p.kb_head : k_ext + (int64_t)(q_start + key - prefix) * p.k_stride + (int64_t)kvh * DQ;
+        const T* vp = old ? vbuf + (int64_t)next_slot[i] * p.vb_slot + kvh * p.vb_head : v_ext + (int64_t)(q_start + key - prefix) * p.v_stride + (int64_t)kvh * D;
+        const Vec<T, 8> kx = ldvec<T, 8>(kp + gch / 2), vx = ldvec<T, 8>(vp + gch / 2);
+        *reinterpret_cast<Vec<T, 8>*>(dst + 4096 * i + 16 * lane) = kx;
+        *reinterpret_cast<Vec<T, 8>*>(dst + 16384 + 4096 * i + 16 * lane) = vx;
+      }
+    }
+  };
+
   f32x16 ot[ND];
 #pragma unroll
   for (int dt = 0; dt < ND; ++dt)
@@ -797,10 +859,12 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
   // (row & 15) only, i.e. on the lane: chunk ^ fx = (2 s) ^ (h ^ fx).
   const int fx = ((j32 & 3) << 2) | ((j32 >> 2) & 3);
   const int kcx = hh ^ fx;
+  int cur = 0;                                              // DIRECT: the tile's stage
   const char* k_rd = ks + 256 * j32;                        // + 8192 hf + 16 * ((2 s) ^ kcx)
-  const char* k_rd2 = ks2 + 256 * j32;                      // steps 8 .. : chunk 2 (s - 8) + h of the second image
+  const char* k_rd2 = ks2 + (DIRECT ? 128 : 256) * j32;     // steps 8 .. : chunk 2 (s - 8) + h of the second image
   auto k_frag = [&](int s_, int hf) -> frag {
-    const char* base = (WIDE && s_ >= 8) ? k_rd2 : k_rd;
+    if (DIRECT && WIDE && s_ >= 8) return *reinterpret_cast<const frag*>(k_rd2 + cur + 4096 * hf + 16 * ((2 * (s_ & 7)) ^ (hh ^ ((j32 >> 1) & 7))));
+    const char* base = ((WIDE && s_ >= 8) ? k_rd2 : k_rd) + cur;
     return *reinterpret_cast<const frag*>(base + 8192 * hf + 16 * ((2 * (s_ & 7)) ^ kcx));
   };
   // V^T fragment of (d tile dt, 16-key step u): lane group (l >> 4) = 2 h + dhalf serves features
@@ -837,24 +901,40 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     }
   };
 
-  if (!careful) {
+  if constexpr (DIRECT) {
+    if (!LATENT) load_slots(first_tile);
+    direct_tile(first_tile, 0);
+    if (!LATENT) load_slots(first_tile + 1);
+  } else if (!careful) {
     if (!LATENT) load_slots(first_tile);
     load_tile(first_tile);
     if (!LATENT) load_slots(first_tile + 1);
   }
   for (int kt = first_tile; kt < n_tiles; ++kt) {
-    __syncthreads();            // previous tile fully consumed
-    if (careful) {              // (nothing ahead: no registers spilled for a rare path)
-      load_slots(kt);
-      load_tile(kt);
-    }
-    store_tile();
-    __syncthreads();
-    if (!careful) {
-      if (kt + 1 < n_tiles) load_tile(kt + 1);
+    if constexpr (DIRECT) {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): this wave's part of the tile and the next one's slots are there
+      __builtin_amdgcn_s_barrier();         // everybody's part is, and the other stage has been read
+      __builtin_amdgcn_sched_barrier(0);
+      const int stage = (kt - first_tile) & 1;
+      cur = stage * STAGE;
+      if (kt + 1 < n_tiles) direct_tile(kt + 1, stage ^ 1);
       if (!LATENT) load_slots(kt + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      __syncthreads();            // previous tile fully consumed
+      if (careful) {              // (nothing ahead: no registers spilled for a rare path)
+        load_slots(kt);
+        load_tile(kt);
+      }
+      store_tile();
+      __syncthreads();
+      if (!careful) {
+        if (kt + 1 < n_tiles) load_tile(kt + 1);
+        if (!LATENT) load_slots(kt + 2);
+      }
     }
-    if (kt * 64 > wave_max_limit) continue;   // every key of the tile is masked for every query of this wave (wave-uniform)
+    if (kt * 64 > wave_max_limit || no_rows) continue;   // nothing of the tile counts for any query of this wave (wave-uniform)
 
     f32x16 st[2];
 #pragma unroll
@@ -875,10 +955,11 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     auto v_read = [&](int i, int slot_) {
       const int u = i / ND, dt = i % ND;
       const int ch = 4 * dt + vch;
-      vlo[slot_] = TrRead<T>::run(reinterpret_cast<const T*>(v_rd + 256 * (16 * u) + 16 * (ch ^ vf_lo)));
-      vhi[slot_] = TrRead<T>::run(reinterpret_cast<const T*>(v_rd + 256 * (16 * u + 8) + 16 * (ch ^ vf_hi)));
+      vlo[slot_] = TrRead<T>::run(reinterpret_cast<const T*>(v_rd + cur + 256 * (16 * u) + 16 * (ch ^ vf_lo)));
+      vhi[slot_] = TrRead<T>::run(reinterpret_cast<const T*>(v_rd + cur + 256 * (16 * u + 8) + 16 * (ch ^ vf_hi)));
     };
     __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       if (s + 2 < NS) {
@@ -896,6 +977,7 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
       st[1] = Mfma32<T>::run(kr[s % 3][1], qf[s], st[1]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    __builtin_amdgcn_s_setprio(0);
     // Softmax on the raw scores: the scale (sm_scale * log2 e > 0, checked by the launcher) commutes with
     // the maximum and folds into the exponent's multiply-add.  Only tiles that cross the wave's diagonal
     // pay for masking (two instructions per score: the key offsets within a tile are compile-time
@@ -941,15 +1023,18 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
     m = mnew;
     float psum = 0.f;
     frag pb[TERMS ? 3 : 4];
+    // the lane's weights 2 j and 2 j + 1 of k-step u
+    [[maybe_unused]] auto weights2 = [&](int u, int j) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float pe = raw_exp2(__builtin_fmaf(st[u >> 1][8 * (u & 1) + 2 * j + e], qmul, -ms));
+        psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V
+        pb[u][2 * j + e] = (T)pe;
+      }
+    };
     if constexpr (!TERMS) {
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float pe = raw_exp2(__builtin_fmaf(st[hf][i], qmul, -ms));
-          psum += pe;                          // fp32 weights in the denominator, T-rounded weights in P.V
-          pb[2 * hf + (i >> 3)][i & 7] = (T)pe;
-        }
+      for (int j = 0; j < 4; ++j) weights2(0, j);
     }
     // TERMS: the lane's eight weights of k-step u.  Those below 2^-126 count: exp2f, in a tile that may have one (wave-uniform); the bare
     // instruction makes them zero.
@@ -982,12 +1067,12 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
 #pragma unroll
       for (int t = 0; t < 3; ++t) pb[t] = __builtin_bit_cast(frag, w[t]);
     };
-    if constexpr (!TERMS) lsum = lsum * alpha + psum;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt) ot[dt] *= alpha;
     }
     __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int i = 0; i < 4 * ND; ++i) {   // (u, dt) = (i / ND, i % ND); fragment i + 4 is requested right behind MFMA i
       frag va;
@@ -1008,7 +1093,15 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
         v_read(i + 4, i & 3);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (!TERMS) {
+        if (i / ND < 3) {
+          weights2(i / ND + 1, i % ND);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
     }
+    __builtin_amdgcn_s_setprio(0);
+    if constexpr (!TERMS) lsum = lsum * alpha + psum;
     if constexpr (TERMS) {
       lsum = lsum * alpha + psum;
       if (careful) add_odd_values(kt);
@@ -1060,11 +1153,11 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
 // ~270 registers and runs one workgroup per CU instead of spilling (measured at 4 x 4096 tokens x 16 heads: 470 TFLOP/s
 // against 412 with 24 spilled registers at two workgroups per CU; issuing the next tile's loads behind the score phase
 // spills more).
-template <typename T, bool KV8, bool SPLIT>
+template <typename T, bool KV8, bool SPLIT, bool DIRECT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_mfma32_kernel(
     const T* __restrict__ q_ext, const T* __restrict__ k_ext, const T* __restrict__ v_ext, T* __restrict__ o_ext,
     const T* __restrict__ kbuf, const T* __restrict__ vbuf, ExtendParams p, int nqb, int npairs) {
-  extend_attn_mfma32_body<T, KV8, 128, false, 128, false, SPLIT>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
+  extend_attn_mfma32_body<T, KV8, 128, false, 128, false, SPLIT, DIRECT>(q_ext, k_ext, v_ext, o_ext, kbuf, vbuf, p, nqb, npairs);
 }
 // Head dimension 64 needs 190 registers: two workgroups per CU (three, with a few registers in scratch memory, took longer: 4 x 340 tokens on 1180
 // cached 80 us).  Bound by the softmax's instructions (about fifteen per score, five of them the weights' three terms, beside an MFMA
@@ -1138,7 +1231,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_latent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o, ExtendParams p, int nqb, int npairs) {
-  extend_attn_mfma32_body<T, false, 192, true>(q, k, v, o, nullptr, nullptr, p, nqb, npairs);
+  extend_attn_mfma32_body<T, false, 192, true, 128, false, false, true>(q, k, v, o, nullptr, nullptr, p, nqb, npairs);
 }
 
 template <typename T, int DP, int BN>
@@ -1183,9 +1276,10 @@ static bool mfma32_serves(int D, int Dv, bool kv8, bool mask, int sliding_window
 
 template <typename T, int D>
 static int launch_mfma32(const void* q, const void* k, const void* v, void* o, const void* kb, const void* vb, const ExtendParams& p,
-                         int64_t bs, int nqb, int64_t npairs, int64_t wgs, int splits, bool kv8, hipStream_t st) {
+                         int64_t bs, int nqb, int64_t npairs, int64_t wgs, int splits, bool kv8, int64_t num_slots, hipStream_t st) {
   using Kernel = void (*)(const T*, const T*, const T*, T*, const T*, const T*, ExtendParams, int, int);
   Kernel kernel;
+  int lds = 0;
   if constexpr (D == 64) {
     if (splits > 1)
       kernel = p.custom_mask ? (kv8 ? extend_attn_mfma32_d64_kernel<T, true, true, true> : extend_attn_mfma32_d64_kernel<T, false, true, true>)
@@ -1194,10 +1288,16 @@ static int launch_mfma32(const void* q, const void* k, const void* v, void* o, c
       kernel = p.custom_mask ? (kv8 ? extend_attn_mfma32_d64_kernel<T, true, true, false> : extend_attn_mfma32_d64_kernel<T, false, true, false>)
                              : (kv8 ? extend_attn_mfma32_d64_kernel<T, true, false, false> : extend_attn_mfma32_d64_kernel<T, false, false, false>);
   } else {
-    if (splits > 1) kernel = kv8 ? extend_attn_mfma32_kernel<T, true, true> : extend_attn_mfma32_kernel<T, false, true>;
-    else kernel = kv8 ? extend_attn_mfma32_kernel<T, true, false> : extend_attn_mfma32_kernel<T, false, false>;
+    // (32-bit offsets: the cache of 4 GiB a layer and side, new rows of 16 MiB)
+    const bool direct = !kv8 && num_slots > 0 && num_slots < (1ll << 31) && num_slots * std::max(p.kb_slot, p.vb_slot) * 2 <= 0xffff0000ll &&
+                        p.k_stride < (1 << 23) && p.v_stride < (1 << 23);
+    if (direct) kernel = splits > 1 ? extend_attn_mfma32_kernel<T, false, true, true> : extend_attn_mfma32_kernel<T, false, false, true>;
+    else if (kv8) kernel = splits > 1 ? extend_attn_mfma32_kernel<T, true, true, false> : extend_attn_mfma32_kernel<T, true, false, false>;
+    else kernel = splits > 1 ? extend_attn_mfma32_kernel<T, false, true, false> : extend_attn_mfma32_kernel<T, false, false, false>;
+    if (direct) lds = 2 * direct_stage_bytes<128>();
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)wgs, (unsigned)splits), dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, (T*)o, (const T*)kb,
+  if (lds != 0) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)wgs, (unsigned)splits), dim3(256), lds, st, (const T*)q, (const T*)k, (const T*)v, (T*)o, (const T*)kb,
                      (const T*)vb, p, nqb, (int)npairs);
   if (splits > 1) {
     const int64_t items = p.rows * p.hq;
@@ -1210,7 +1310,7 @@ static int launch_mfma32(const void* q, const void* k, const void* v, void* o, c
 template <typename T>
 static int launch_extend(const void* q, const void* k, const void* v, void* o, const void* kb,
                          const void* vb, const ExtendParams& p, int64_t bs, int64_t max_len_extend,
-                         bool kv8, int splits, hipStream_t st) {   // kv8: the KV cache holds e4m3fn bytes
+                         bool kv8, int splits, int64_t num_slots, hipStream_t st) {   // kv8: the KV cache holds e4m3fn bytes
   constexpr int VE = V16<T>::n;
   const int dmax = p.D > p.Dv ? p.D : p.Dv;
   const bool vec = p.D % VE == 0 && p.Dv % VE == 0 && p.q_stride % VE == 0 &&
@@ -1223,8 +1323,8 @@ static int launch_extend(const void* q, const void* k, const void* v, void* o, c
       const int64_t npairs = bs * p.hkv;
       const int64_t wgs = 8 * ((npairs + 7) / 8) * (p.hq / p.hkv) * nqb;
       if (wgs < (int64_t)1 << 31) {
-        if (p.D == 64) return launch_mfma32<T, 64>(q, k, v, o, kb, vb, p, bs, nqb, npairs, wgs, splits, kv8, st);
-        if (p.D == 128) return launch_mfma32<T, 128>(q, k, v, o, kb, vb, p, bs, nqb, npairs, wgs, splits, kv8, st);
+        if (p.D == 64) return launch_mfma32<T, 64>(q, k, v, o, kb, vb, p, bs, nqb, npairs, wgs, splits, kv8, num_slots, st);
+        if (p.D == 128) return launch_mfma32<T, 128>(q, k, v, o, kb, vb, p, bs, nqb, npairs, wgs, splits, kv8, num_slots, st);
         hipLaunchKernelGGL((extend_attn_mfma32_wide_kernel<T>), dim3((unsigned)wgs), dim3(256), 0, st, (const T*)q, (const T*)k,
                            (const T*)v, (T*)o, (const T*)kb, (const T*)vb, p, nqb, (int)npairs);
         return MI355_OK;
@@ -1360,7 +1460,7 @@ int mi355_extend_attention_ws(const void* q_extend, const void* k_extend, const 
   }
   MI355_DISPATCH_DTYPE(dtype, "extend_attention",
                        rc = launch_extend<T>(q_extend, k_extend, v_extend, o_extend, k_buffer,
-                                             v_buffer, p, bs, max_len_extend, kv8, splits > 1 ? splits : 1, (hipStream_t)stream));
+                                             v_buffer, p, bs, max_len_extend, kv8, splits > 1 ? splits : 1, num_slots, (hipStream_t)stream));
   if (rc != MI355_OK) return rc;
   MI355_CHECK_LAUNCH("extend_attention");
   return MI355_OK;
@@ -1382,8 +1482,8 @@ int mi355_latent_prefill_attention(void* out, const void* q, int64_t q_stride, c
                 nope_dim, rope_dim, v_dim, rot_dims, dtype);
   MI355_REQUIRE(bs >= 0 && max_len >= 0 && heads > 0 && scale > 0.f, MI355_ERR_INVALID, "latent_prefill_attention: bad shape");
   MI355_REQUIRE(q_stride >= (int64_t)heads * 192 && q_stride % 8 == 0 && kv_stride >= (int64_t)heads * 256 && kv_stride % 8 == 0 &&
-                    k_rope_stride >= 64 && k_rope_stride % 8 == 0 && aligned16(q) && aligned16(kv) && aligned16(k_rope) && aligned16(out),
-                MI355_ERR_INVALID, "latent_prefill_attention: rows must be 16-byte aligned and hold every head");
+                    k_rope_stride >= 64 && k_rope_stride % 8 == 0 && kv_stride < (1 << 23) && k_rope_stride < (1 << 23) && aligned16(q) && aligned16(kv) && aligned16(k_rope) && aligned16(out),
+                MI355_ERR_INVALID, "latent_prefill_attention: rows must be 16-byte aligned, hold every head and lie less than 2^23 elements apart");
   if (bs == 0 || max_len == 0) return MI355_OK;
   ExtendParams p = {};
   p.seg_start = seg_start; p.seg_len = seg_len; p.positions = positions; p.inv_freq = inv_freq;
@@ -1394,11 +1494,13 @@ int mi355_latent_prefill_attention(void* out, const void* q, int64_t q_stride, c
   const int nqb = (int)((max_len + 127) / 128);
   const int64_t npairs = bs * heads, wgs = 8 * ((npairs + 7) / 8) * nqb;
   MI355_REQUIRE(wgs < (int64_t)1 << 31, MI355_ERR_UNSUPPORTED, "latent_prefill_attention: too many query blocks");
+  constexpr int lds = 2 * direct_stage_bytes<192>();     // 80 KiB: two workgroups a CU
 #define MI355_LP(T)                                                                                                            \
-  hipLaunchKernelGGL((extend_attn_latent_kernel<T>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, (const T*)q,       \
+  (void)hipFuncSetAttribute((const void*)extend_attn_latent_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);       \
+  hipLaunchKernelGGL((extend_attn_latent_kernel<T>), dim3((unsigned)wgs), dim3(256), lds, (hipStream_t)stream, (const T*)q,       \
                      (const T*)kv, (const T*)kv + 128, (T*)out, p, nqb, (int)npairs)
-  if (dtype == MI355_BF16) MI355_LP(bf16_t);
-  else MI355_LP(f16_t);
+  if (dtype == MI355_BF16) { MI355_LP(bf16_t); }
+  else { MI355_LP(f16_t); }
 #undef MI355_LP
   MI355_CHECK_LAUNCH("latent_prefill_attention");
   return MI355_OK;

@@ -237,19 +237,22 @@ __global__ __launch_bounds__(256) void window_attention_merge_kernel(T* __restri
 // exchanges over registers, and its weights are, rounded to T, the B operand of O^T += V^T P^T as they stand (one MFMA
 // 16x16x32 per 16 result columns, V read transposed).  Nothing travels between waves; the tiles of K and V take turns in two
 // LDS buffers, one barrier each, the next tile's rows on their way from memory meanwhile.
-// What bounds it: the vector ALU (about 90 operations per lane and tile beside 16 MFMAs at d = dv = 128).  7381 prefill tokens
-// of 16 heads over 4, d = 128, window 512 and averaged blocks of 64 (37 GFLOP): 116 us; 273 with S = Q K^T, where a row's
-// scores lay in 16 lanes, its weights and factor went through LDS and the waves shared the result columns (three barriers).
+// What bounds it: the vector ALU (about 90 operations per lane and tile beside 16 MFMAs at d = dv = 128; half of them in a tile
+// that every row of the run sees whole, which has no masks).  FULL: d and dv are 64 CK and 64 CT, so that no condition stands
+// between a tile's reads and MFMAs and the compiler requests the reads ahead; the other widths keep the general loops.  7381
+// prefill tokens of 16 heads over 4, d = 128, window 512 and averaged blocks of 64 (37 GFLOP), a launch inside a prefill step: 137 us
+// with masks on every tile and the general loops, 116 now.  A form with S = Q K^T, where a row's scores lay in 16 lanes, its
+// weights and factor went through LDS and the waves shared the result columns (three barriers), took 2.35 times the time.
 // Single tokens of 4 heads a key head are one live wave, whose chain is shorter too: 1 / 64 / 256 tokens x 2000 keys, same heads and
 // window, 22 / 31 / 66 us against 31 / 41 / 131.
 // sm: 2 x (Ks [32][d + 8] | Vs [32][dv + 8])   (all T)
 constexpr int WAM_ROWS = 64;
 constexpr int WAM_MAX = 256;     // d and dv
 
-template <typename T, int CT, int CK>
+template <typename T, int CT, int CK, bool FULL>
 __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smraw[];
-  const int d = a.d, dv = a.dv;
+  const int d = FULL ? 64 * CK : a.d, dv = FULL ? 64 * CT : a.dv;
   const int qld = d + 8, vld = dv + 8;
   const int buf_elems = WA_KT * (qld + vld);     // one tile's keys and values; two tiles in turn
   const int rep = a.heads / a.kv_heads;
@@ -362,27 +365,36 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
       }
     }
     // the lane holds eight scores of its row: keys 4 lg + x of both halves of the tile
-    bool seen[8];
-    float x8[8], mx = run_m;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int j = j0 + 16 * (i >> 2) + 4 * lg + (i & 3);
-      seen[i] = ptile ? (rp >= 0 && j * a.pool + a.pool - 1 <= rp - a.window) : (j <= rp && (a.window <= 0 || rp - j < a.window));
-      x8[i] = seen[i] ? s[i >> 2][i & 3] * a.scale : WA_NEG;
-      mx = fmaxf(mx, x8[i]);
-    }
-    mx = max_xor<16>(mx);
-    mx = max_xor<32>(mx);
-    const float alpha = __expf(run_m - mx);
-    run_m = mx;
+    float alpha, sum = 0.f;
     Vec<T, 8> p8;      // key slots 8 lg + i of the product with V: the keys above, in that order
-    float sum = 0.f;
+    auto weigh = [&](auto whole) {
+      bool seen[8];
+      float x8[8], mx = run_m;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float pe = seen[i] ? __expf(x8[i] - mx) : 0.f;
-      sum += pe;
-      p8.v[i] = from_f32<T>(pe);
-    }
+      for (int i = 0; i < 8; ++i) {
+        const int j = j0 + 16 * (i >> 2) + 4 * lg + (i & 3);
+        seen[i] = whole.value || (ptile ? (rp >= 0 && j * a.pool + a.pool - 1 <= rp - a.window)
+                                        : (j <= rp && (a.window <= 0 || rp - j < a.window)));
+        x8[i] = seen[i] ? s[i >> 2][i & 3] * a.scale : WA_NEG;
+        mx = fmaxf(mx, x8[i]);
+      }
+      mx = max_xor<16>(mx);
+      mx = max_xor<32>(mx);
+      alpha = __expf(run_m - mx);
+      run_m = mx;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float pe = seen[i] ? __expf(x8[i] - mx) : 0.f;
+        sum += pe;
+        p8.v[i] = from_f32<T>(pe);
+      }
+    };
+    // every row of the run sees every key of the tile (rows without a token compute what nobody stores)
+    if (ptile ? (j0 + WA_KT) * a.pool - 1 <= first - a.window
+              : j0 + WA_KT - 1 <= first && (a.window <= 0 || last - j0 < a.window))
+      weigh(std::true_type());
+    else
+      weigh(std::false_type());
     run_l = run_l * alpha + sum;
     if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
@@ -510,22 +522,24 @@ template <typename T> int launch_window(const WaArgs& a, dim3 grid, bool mfma, h
   if constexpr (!std::is_same<T, float>::value) {
     if (mfma) {
       const size_t lds = 2 * (size_t)WA_KT * (a.d + 8 + a.dv + 8) * sizeof(T);
-#define MI355_WA_LAUNCH(CT, CK)                                                                                                \
+#define MI355_WA_LAUNCH(CT, CK, FULL)                                                                                          \
   do {                                                                                                                         \
     if (lds > 64 * 1024) {                                                                                                     \
-      hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel<T, CT, CK>,                                 \
+      hipError_t e = hipFuncSetAttribute((const void*)window_attention_mfma_kernel<T, CT, CK, FULL>,                           \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                                \
       MI355_REQUIRE(e == hipSuccess, MI355_ERR_LAUNCH, "window_attention: %zu bytes of LDS refused", lds);                     \
     }                                                                                                                          \
-    hipLaunchKernelGGL((window_attention_mfma_kernel<T, CT, CK>), grid, dim3(256), lds, stream, a);                            \
+    hipLaunchKernelGGL((window_attention_mfma_kernel<T, CT, CK, FULL>), grid, dim3(256), lds, stream, a);                      \
   } while (0)
 #define MI355_WA_KEYS(CT)                                                                                                      \
   do {                                                                                                                         \
-    if (a.d <= 64) MI355_WA_LAUNCH(CT, 1);                                                                                     \
-    else if (a.d <= 128) MI355_WA_LAUNCH(CT, 2);                                                                               \
-    else MI355_WA_LAUNCH(CT, 4);                                                                                               \
+    if (a.d <= 64) MI355_WA_LAUNCH(CT, 1, false);                                                                              \
+    else if (a.d <= 128) MI355_WA_LAUNCH(CT, 2, false);                                                                        \
+    else MI355_WA_LAUNCH(CT, 4, false);                                                                                        \
   } while (0)
-      if (a.dv <= 64) MI355_WA_KEYS(1);
+      if (a.d == 64 && a.dv == 64) MI355_WA_LAUNCH(1, 1, true);
+      else if (a.d == 128 && a.dv == 128) MI355_WA_LAUNCH(2, 2, true);
+      else if (a.dv <= 64) MI355_WA_KEYS(1);
       else if (a.dv <= 128) MI355_WA_KEYS(2);
       else MI355_WA_KEYS(4);
 #undef MI355_WA_KEYS

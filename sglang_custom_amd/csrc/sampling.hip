@@ -192,7 +192,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_temperature_kernel(
 // every chunk normalises itself with what all of them left.  (A chunk without a number in it has no maximum to take off: its
 // -inf entries count zero and a NaN makes its sum NaN, and with it the row, as one pass over the row has it.)  One workgroup per
 // row reads its 0.5 MB three times with 4 bytes a lane in flight and has one CU's exponentials: 64 rows of 128256 took 146 us (64 CUs at work); this takes
-// 13 + 14 us (33 MB read twice, the second time from L2, then read and written; 16 + 16 with a precise division per entry in
+// 11 + 10 us (33 MB read twice, the second time from L2, then read and written; 16 + 16 with a precise division per entry in
 // both), bound by the exponentials and by the latency of a chunk's one round of loads.
 constexpr int MAX_CHUNKS = 16;
 struct ChunkSpan {
@@ -239,13 +239,19 @@ __device__ __forceinline__ void span_each(const float* __restrict__ row, int64_t
 // How a row's exponents are formed.  A temperature that is an ordinary positive number divides once: (x - max x) * (1 / t), where x / t
 // takes a precise division per entry in both launches, and no further from float64 (the difference is exact near the maximum, where the mass is).
 // Any other temperature (zero, negative, NaN, past 1e30 either way) keeps x / t - max(x / t).
-struct RowScale {
+// Which of the two is decided once for a launch's row, in front of its loops: as a choice inside them it had both sides computed for every
+// entry, and the division's dozen instructions were a third of what there was (64 rows x 128256: 13.4 and 21.6 us so, 11.5 and 19.2
+// this way; 200 rows, whose chunks are not held, 53 and 52 against 38 and 50).
+template <bool PLAIN> struct RowScale {
   float t, inv;
-  bool plain;
-  __device__ __forceinline__ explicit RowScale(float t_) : t(t_), inv(1.0f / t_), plain(t_ >= 1e-30f && t_ <= 1e30f) {}
-  __device__ __forceinline__ float key(float x) const { return plain ? x : x / t; }                 // what the maximum is taken of
-  __device__ __forceinline__ float power(float k, float mx) const { return expf(plain ? (k - mx) * inv : k - mx); }
+  __device__ __forceinline__ explicit RowScale(float t_) : t(t_), inv(1.0f / t_) {}
+  __device__ __forceinline__ float key(float x) const { return PLAIN ? x : x / t; }                 // what the maximum is taken of
+  __device__ __forceinline__ float power(float k, float mx) const { return expf(PLAIN ? (k - mx) * inv : k - mx); }
 };
+template <typename F> __device__ __forceinline__ void with_row_scale(float t, F&& f) {
+  if (t >= 1e-30f && t <= 1e30f) f(RowScale<true>(t));
+  else f(RowScale<false>(t));
+}
 
 constexpr int KEEP = 8;   // 16-byte pieces of a chunk that a thread holds: chunks up to 32 K entries, every vocabulary up to 512 K at few rows
 
@@ -266,53 +272,60 @@ __global__ __launch_bounds__(SAMP_THREADS) void softmax_partials_kernel(
   const float* row = logits + (int64_t)r * row_stride;
   const bool vec = (row_stride % 4 == 0) && aligned16(logits);
   const ChunkSpan sp = chunk_span(vocab, c, chunks);
-  const RowScale rs(temperatures[r]);
+  const float t = temperatures[r];
   float mx = -INFINITY, sum = 0.f;
   // More rows have fewer and longer chunks (row_chunks), which go through span_each twice: both launches at 128256 entries, 64 rows
-  // (4 chunks) 41 us, 86 (3) 73, 200 (2) 116; a whole row a workgroup 157, 163, 182.
+  // (4 chunks) 41 us, 86 (3) 73, 200 (2) 116; a whole row a workgroup 157, 163, 182 (all with a division per entry: 200 rows are 82 without).
   if (vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS && sp.v0 < sp.v1) {
     // The chunk is read once, into registers.
     Vec<float, 4> v[KEEP];
     chunk_load(v, row, sp);
     const int64_t k = vocab / 4 * 4 + threadIdx.x;
     const bool one = sp.tail && k < vocab;
-    const float last = one ? rs.key(row[k]) : -INFINITY;
+    float last = one ? row[k] : -INFINITY;
+    with_row_scale(t, [&](auto rs) {
+      if (one) last = rs.key(last);
 #pragma unroll
-    for (int u = 0; u < KEEP; ++u)
+      for (int u = 0; u < KEEP; ++u)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[u].v[j] = rs.key(v[u].v[j]);
-        mx = fmaxf(mx, v[u].v[j]);   // (a piece past the end repeats the last one: the maximum does not mind)
-      }
-    mx = block_reduce_max(fmaxf(mx, last), red);
-    const float ref = mx == -INFINITY ? 0.f : mx;
+        for (int j = 0; j < 4; ++j) {
+          v[u].v[j] = rs.key(v[u].v[j]);
+          mx = fmaxf(mx, v[u].v[j]);   // (a piece past the end repeats the last one: the maximum does not mind)
+        }
+      mx = block_reduce_max(fmaxf(mx, last), red);
+      const float ref = mx == -INFINITY ? 0.f : mx;
 #pragma unroll
-    for (int u = 0; u < KEEP; ++u)
-      if (sp.v0 + threadIdx.x + u * SAMP_THREADS < sp.v1)
+      for (int u = 0; u < KEEP; ++u)
+        if (sp.v0 + threadIdx.x + u * SAMP_THREADS < sp.v1)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sum += rs.power(v[u].v[j], ref);
-    if (one) sum += rs.power(last, ref);
+          for (int j = 0; j < 4; ++j) sum += rs.power(v[u].v[j], ref);
+      if (one) sum += rs.power(last, ref);
+    });
   } else {
-    span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, rs.key(x)); });
-    mx = block_reduce_max(mx, red);
-    const float ref = mx == -INFINITY ? 0.f : mx;
-    span_each(row, vocab, sp, vec, [&](float x) { sum += rs.power(rs.key(x), ref); });
+    with_row_scale(t, [&](auto rs) {
+      span_each(row, vocab, sp, vec, [&](float x) { mx = fmaxf(mx, rs.key(x)); });
+      mx = block_reduce_max(mx, red);
+      const float ref = mx == -INFINITY ? 0.f : mx;
+      span_each(row, vocab, sp, vec, [&](float x) { sum += rs.power(rs.key(x), ref); });
+    });
   }
   sum = block_reduce_sum(sum, red);
   if (threadIdx.x == 0) partials[(int64_t)r * chunks + c] = float2{mx, sum};
 }
 
-// The row's maximum and sum from what its chunks left, and the entries' probabilities.
-struct RowNorm {
-  RowScale rs;
+// The row's maximum and sum from what its chunks left, and the entries' probabilities.  p: the lane's chunk (a lane per chunk).
+__device__ __forceinline__ float2 chunk_partial(const float2* __restrict__ partials, int chunks) {
+  const int i = threadIdx.x & (MAX_CHUNKS - 1);
+  return i < chunks ? partials[i] : float2{-INFINITY, 0.f};
+}
+template <typename SCALE> struct RowNorm {
+  SCALE rs;
   float mx, sum, inv_sum;
-  __device__ __forceinline__ RowNorm(const float2* __restrict__ partials, int chunks, float t) : rs(t) {
-    const int i = threadIdx.x & (MAX_CHUNKS - 1);
-    const float2 p = i < chunks ? partials[i] : float2{-INFINITY, 0.f};     // a lane per chunk
+  __device__ __forceinline__ RowNorm(SCALE rs_, float2 p, int chunks) : rs(rs_) {
     mx = p.x;
 #pragma unroll
     for (int o = MAX_CHUNKS / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    sum = i < chunks ? p.y * rs.power(p.x, mx) : 0.f;
+    sum = (int)(threadIdx.x & (MAX_CHUNKS - 1)) < chunks ? p.y * rs.power(p.x, mx) : 0.f;
 #pragma unroll
     for (int o = MAX_CHUNKS / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
     inv_sum = 1.0f / sum;
@@ -503,7 +516,7 @@ __global__ __launch_bounds__(SAMP_THREADS) void topk_topp_minp_sample_kernel(
 // (no probability does) takes sample_whole_row.
 // The one-workgroup routine meets each of its four levels' 128256 entries in 256 bins of two binades, a handful of which
 // take nearly all of them: 64 rows of 128256 with top_k 50, top_p 0.9 took 451 us, bound by those LDS atomics.  Launch 1 beside the
-// softmax takes 20 us for that (apart 14 + 13), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 12 from the
+// softmax takes 19 us for that (apart 10 + 14), bound by LDS atomics, exponentials and 66 MB read and written; launch 2 takes 12 from the
 // lists, a chain of some twenty barriers (28 from the row, one CU's pass over 0.5 MB; 58 when thousands are kept).
 constexpr int SB_BINS = 2048, SB_SHIFT = 19, SB_LIST = 8192, SB_SHORT = 512, SB_TILE = 256, SB_MAX_TILES = 4096;
 constexpr int SB_SUM_BITS = 40;
@@ -628,7 +641,7 @@ __device__ __forceinline__ void chunk_list(const Vec<float, 4> (&v)[KEEP], float
 }
 
 // NORM: `data` holds logits, which become probabilities on the way (launch 2 of softmax_temperature); BINS: bins and lists of the
-// probabilities.  Both at once: 64 rows x 128256 20 us, apart 14 + 13.
+// probabilities.  Both at once: 64 rows x 128256 19 us, apart 10 + 14.
 template <bool NORM, bool BINS>
 __global__ __launch_bounds__(SAMP_THREADS) void sample_chunk_kernel(float* __restrict__ data, const float2* __restrict__ partials,
                                                                     const float* __restrict__ temperatures, const int32_t* __restrict__ top_ks,
@@ -644,80 +657,104 @@ __global__ __launch_bounds__(SAMP_THREADS) void sample_chunk_kernel(float* __res
   const int want = BINS && top_ks != nullptr ? max(top_ks[r], 0) : 0x7fffffff;
   const bool listed = BINS && (want <= SB_TOP || (top_ps != nullptr && top_ps[r] < 1.0f));
   const bool held = (NORM || listed) && vec && sp.v1 - sp.v0 <= KEEP * SAMP_THREADS && sp.v0 < sp.v1;
-  Vec<float, 4> v[KEEP];
-  if (held) chunk_load(v, row, sp);
-  const RowNorm norm(partials + (NORM ? (int64_t)r * chunks : 0), NORM ? chunks : 0, NORM ? temperatures[r] : 1.0f);
-  if constexpr (BINS) {
-    for (int i = tid; i < SB_BINS; i += SAMP_THREADS) sm.hist[i] = 0;
-    __syncthreads();
-  }
+  const float temperature = NORM ? temperatures[r] : 1.0f;
+  const float2 partial = NORM ? chunk_partial(partials + (int64_t)r * chunks, chunks) : float2{0.f, 0.f};
   const int64_t k = vocab / 4 * 4 + tid;
   const bool one = sp.tail && k < vocab;
-  float mx = 0.f, last = 0.f;
+  float mx = 0.f, last = one ? row[k] : 0.f;
   int count = -1, lowest = SB_BINS;
-  if (one) {
-    last = NORM ? norm.prob(row[k]) : row[k];
-    if (NORM) row[k] = last;
-    mx = fmaxf(mx, last);
-    if (BINS) sb_count(sm.hist, last);
-  }
-  if (held) {
-#pragma unroll
-    for (int u = 0; u < KEEP; ++u) {
-      const int64_t i = sp.v0 + tid + u * SAMP_THREADS;
-      if (i < sp.v1) {
-        if constexpr (NORM) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[u].v[j] = norm.prob(v[u].v[j]);
-          stvec<float, 4>(row + i * 4, v[u]);
-        }
-        if constexpr (BINS)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            mx = fmaxf(mx, v[u].v[j]);
-            sb_count(sm.hist, v[u].v[j]);
-          }
-      }
+  auto clear = [&] {
+    if constexpr (BINS) {
+      for (int i = tid; i < SB_BINS; i += SAMP_THREADS) sm.hist[i] = 0;
+      __syncthreads();
     }
+  };
+  // f(prob), prob: of a logit, or the probability that it is already; the row's tail entry is taken here
+  auto with_prob = [&](auto&& f) {
+    auto go = [&](auto prob) {
+      if (one) {
+        last = prob(last);
+        if (NORM) row[k] = last;
+        mx = fmaxf(mx, last);
+        if (BINS) sb_count(sm.hist, last);
+      }
+      f(prob);
+    };
+    if constexpr (NORM)
+      with_row_scale(temperature, [&](auto rs) {
+        const RowNorm<decltype(rs)> norm(rs, partial, chunks);
+        go([&](float x) { return norm.prob(x); });
+      });
+    else
+      go([](float x) { return x; });
+  };
+  if (held) {
+    Vec<float, 4> v[KEEP];
+    chunk_load(v, row, sp);
+    clear();
+    with_prob([&](auto prob) {
+#pragma unroll
+      for (int u = 0; u < KEEP; ++u) {
+        const int64_t i = sp.v0 + tid + u * SAMP_THREADS;
+        if (i < sp.v1) {
+          if constexpr (NORM) {
+            Vec<float, 4> w;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w.v[j] = prob(v[u].v[j]);
+            stvec<float, 4>(row + i * 4, w);
+            if (BINS) v[u] = w;
+          }
+          if constexpr (BINS)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              mx = fmaxf(mx, v[u].v[j]);
+              sb_count(sm.hist, v[u].v[j]);
+            }
+        }
+      }
+    });
     if constexpr (BINS) {
       __syncthreads();
       const int most = SB_TOP / chunks;
       if (listed) chunk_list(v, last, sp, vocab, most, want, sm, lists + (int64_t)r * SB_TOP + c * most, count, lowest);
     }
   } else {
-    auto load = [&](int64_t i) {
-      Vec<float, 4> w;
-      if (vec) w = ldvec<float, 4>(row + i * 4);
-      else
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w.v[j] = row[i * 4 + j];
-      return w;
-    };
-    auto take = [&](Vec<float, 4> w, int64_t i) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (NORM) w.v[j] = norm.prob(w.v[j]);
-        mx = fmaxf(mx, w.v[j]);
-        if (BINS) sb_count(sm.hist, w.v[j]);
-      }
-      if (NORM) {
-        if (vec) stvec<float, 4>(row + i * 4, w);
+    clear();
+    with_prob([&](auto prob) {
+      auto load = [&](int64_t i) {
+        Vec<float, 4> w;
+        if (vec) w = ldvec<float, 4>(row + i * 4);
         else
 #pragma unroll
-          for (int j = 0; j < 4; ++j) row[i * 4 + j] = w.v[j];
-      }
-    };
-    int64_t i = sp.v0 + tid;
-    if constexpr (!NORM) {     // four loads in flight (beside the exponentials they gain nothing: 200 rows x 128256 166 us the batch, 173 so)
-      for (; i + 3 * SAMP_THREADS < sp.v1; i += 4 * SAMP_THREADS) {
-        Vec<float, 4> w[4];
+          for (int j = 0; j < 4; ++j) w.v[j] = row[i * 4 + j];
+        return w;
+      };
+      auto take = [&](Vec<float, 4> w, int64_t i) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) w[u] = load(i + u * SAMP_THREADS);
+        for (int j = 0; j < 4; ++j) {
+          if (NORM) w.v[j] = prob(w.v[j]);
+          mx = fmaxf(mx, w.v[j]);
+          if (BINS) sb_count(sm.hist, w.v[j]);
+        }
+        if (NORM) {
+          if (vec) stvec<float, 4>(row + i * 4, w);
+          else
 #pragma unroll
-        for (int u = 0; u < 4; ++u) take(w[u], i + u * SAMP_THREADS);
+            for (int j = 0; j < 4; ++j) row[i * 4 + j] = w.v[j];
+        }
+      };
+      int64_t i = sp.v0 + tid;
+      if constexpr (!NORM) {     // four loads in flight (beside the exponentials they gain nothing: 200 rows x 128256 166 us the batch, 173 so)
+        for (; i + 3 * SAMP_THREADS < sp.v1; i += 4 * SAMP_THREADS) {
+          Vec<float, 4> w[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) w[u] = load(i + u * SAMP_THREADS);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) take(w[u], i + u * SAMP_THREADS);
+        }
       }
-    }
-    for (; i < sp.v1; i += SAMP_THREADS) take(load(i), i);
+      for (; i < sp.v1; i += SAMP_THREADS) take(load(i), i);
+    });
   }
   if constexpr (BINS) {
     mx = block_reduce_max(mx, sm.red);

@@ -10,8 +10,8 @@
 //   * K is walked in tiles of 128 BYTES per row (64 16-bit or 128 fp8 elements); a tile's operands
 //     live in LDS as four HALF-TILES of 128 rows x 128 bytes (x rows 0..127, x rows 128..255, W rows
 //     0..127, W rows 128..255), two tiles resident;
-//   * the load unit writes LDS itself (global_load_lds_dwordx4, 8 rows x 128 B per wave-instruction:
-//     whole cache lines);
+//   * the load unit writes LDS itself (16 bytes a lane, 8 rows x 128 B per wave-instruction: whole cache
+//     lines; buffer loads, in the grouped kernel global ones);
 //   * the eight waves form two groups of four (group = row half of the tile, wave-in-group = 64
 //     output columns).  A wave alternates a READ slot (its 8 load requests, then 24 ds_read_b128: its A
 //     and B fragments of a whole K tile) with a MATRIX slot (nothing but 64 x v_mfma_f32_16x16x32 on

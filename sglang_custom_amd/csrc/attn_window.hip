@@ -367,7 +367,9 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
     // the lane holds eight scores of its row: keys 4 lg + x of both halves of the tile
     float alpha, sum = 0.f;
     Vec<T, 8> p8;      // key slots 8 lg + i of the product with V: the keys above, in that order
+    // A score is rounded where it is scaled, in both forms: a row's weights do not depend on which rows share its tiles.
     auto weigh = [&](auto whole) {
+#pragma clang fp contract(off)
       bool seen[8];
       float x8[8], mx = run_m;
 #pragma unroll

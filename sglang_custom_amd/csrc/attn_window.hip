@@ -239,18 +239,22 @@ __global__ __launch_bounds__(256) void window_attention_merge_kernel(T* __restri
 // LDS buffers, one barrier each, the next tile's rows on their way from memory meanwhile.
 // What bounds it: the vector ALU (about 90 operations per lane and tile beside 16 MFMAs at d = dv = 128; half of them in a tile
 // that every row of the run sees whole, which has no masks).  FULL: d and dv are 64 CK and 64 CT, so that no condition stands
-// between a tile's reads and MFMAs and the compiler requests the reads ahead; the other widths keep the general loops.  7381
-// prefill tokens of 16 heads over 4, d = 128, window 512 and averaged blocks of 64 (37 GFLOP), a launch inside a prefill step: 137 us
-// with masks on every tile and the general loops, 116 now.  A form with S = Q K^T, where a row's scores lay in 16 lanes, its
-// weights and factor went through LDS and the waves shared the result columns (three barriers), took 2.35 times the time.
+// between a tile's reads and MFMAs and the compiler requests the reads ahead; the other widths keep the general loops.  us a launch over
+// 7381 prefill tokens of 16 heads over 4, masks on every tile and the general loops | now, at window 512 with averaged blocks of 64, window
+// 64, window 16 (no tile is whole) and no window: d = dv = 128 122 | 104, 52.3 | 51.6, 45.0 | 44.9, 220 | 170; 64 72 | 57, 26.8 | 26.8, 23.1 | 23.2,
+// 151 | 104; 96 100 | 90, 41.3 | 41.4, 34.0 | 34.8, 203 | 170; 192 and 128 151 | 136, 62.4 | 62.0, 48.0 | 48.6, 287 | 245; 64 and 256 170 | 154,
+// 74.9 | 74.8, 62.0 | 62.6, 306 | 263; 256 263 | 241, 99.0 | 99.7, 77.7 | 79.4, 485 | 425.  A form with S = Q K^T, where a row's scores lay in
+// 16 lanes, its weights and factor went through LDS and the waves shared the result columns (three barriers), took 2.35 times the time.
 // Single tokens of 4 heads a key head are one live wave, whose chain is shorter too: 1 / 64 / 256 tokens x 2000 keys, same heads and
 // window, 22 / 31 / 66 us against 31 / 41 / 131.
+// Widths in (64, 128] by the general loops are held to 128 registers, four waves a SIMD (three spilled in front of the loop): at 131 and three
+// waves 96 wide took 103, 44.6, 36.4 and 182 us of the above.
 // sm: 2 x (Ks [32][d + 8] | Vs [32][dv + 8])   (all T)
 constexpr int WAM_ROWS = 64;
 constexpr int WAM_MAX = 256;     // d and dv
 
 template <typename T, int CT, int CK, bool FULL>
-__global__ __launch_bounds__(256) void window_attention_mfma_kernel(WaArgs a) {
+__global__ __launch_bounds__(256, CT == 2 && CK == 2 && !FULL ? 4 : 1) void window_attention_mfma_kernel(WaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smraw[];
   const int d = FULL ? 64 * CK : a.d, dv = FULL ? 64 * CT : a.dv;
   const int qld = d + 8, vld = dv + 8;

@@ -550,8 +550,8 @@ int mi355_linear_packed_scaled(float* y, const void* x, const void* w_packed, fl
  * epilogue 1 (W = [gate; up], N = 2 I): y [M, I], y[m, j] = T(silu(T(g_j))) * T(u_j) with the rounding
  * points of the unfused GEMM + SiluAndMul pair; epilogue 2: y [M, N] = T(gelu(T(acc))), gelu(z) = z / 2 (1 + erf(z / sqrt 2)),
  * without bias; epilogue 3: as 1 with y[m, j] = T(gelu_tanh(T(g_j)) T(u_j)), gelu_tanh(z) = z / 2 (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))).
- * Needs K % 64 == 0, 128 <= K < 2^23, N % 16 == 0, x_stride < 2^23
- * (mi355_linear_tiled_supported returns 1 for the shape); no workspace, nothing allocated.
+ * Needs K % 64 == 0, K >= 128, N % 16 == 0, rows of x and W below 2^31 bytes (mi355_linear_tiled_supported returns 1); any x_stride;
+ * no workspace, nothing allocated.
  * replaces: UnquantizedLinearMethod.apply / F.linear at prefill sizes
  *           (layers/quantization/unquant.py:110-122) and, with epilogue 1, LlamaMLP.forward's
  *           gate_up_proj + act_fn (models/llama.py:94-98, layers/activation.py:55-65). */
@@ -603,7 +603,7 @@ int mi355_linear_few(void* y, const void* x, const void* w, const float* x_scale
  * per-token / per-channel scales applied to the fp32 accumulator as (acc * x_scale[m]) * w_scale[n],
  * then bias, one rounding to out_dtype; epilogue 1 = SiLU-and-mul over wq = [gate; up] as in
  * mi355_linear_tiled.  xq [M, K] and wq [N, K] contiguous e4m3fn bytes.  Needs K % 128 == 0, K >= 256,
- * N % 16 == 0 (mi355_fp8_scaled_mm_tiled_supported returns 1); no workspace.
+ * N % 16 == 0, K < 2^31 (mi355_fp8_scaled_mm_tiled_supported returns 1); no workspace.
  * replaces: apply_fp8_linear's torch._scaled_mm / fp8_scaled_mm call at prefill sizes
  *           (layers/quantization/fp8_utils.py:676-749, sgl-kernel/csrc/gemm/fp8_gemm_kernel.cu). */
 int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out_dtype, int epilogue);
@@ -623,7 +623,7 @@ int mi355_fp8_scaled_mm_tiled_ws(void* y, const uint8_t* xq, const uint8_t* wq, 
  * x_scale != NULL selects the fp8 form: x, w are e4m3fn bytes with per-token x_scale[M] and per-channel
  * w_scale[N] applied as in mi355_fp8_scaled_mm_tiled (x_stride must then equal k).
  * Needs head_dim = rotary_dim = 128, is_neox, an even hq + 2 hkv, a 16-bit dtype, K % 64 == 0 and K >= 128
- * (fp8: K % 128 == 0, K >= 256), no bias; cos_sin_cache [max_pos, 128] fp32 or the dtype; loc int32 / int64.
+ * (fp8: K % 128 == 0, K >= 256), rows of x and w below 2^31 bytes, no bias; cos_sin_cache [max_pos, 128] fp32 or the dtype; loc int32 / int64.
  * replaces: LlamaAttention.forward's qkv_proj -> rotary_emb -> set_kv_buffer sequence at prefill
  *           (models/llama.py:187-199, layers/rotary_embedding.py:222-246, mem_cache/memory_pool.py:425-458). */
 int mi355_qkv_proj_rope_tiled_supported(int64_t m, int64_t k, int hq, int hkv, int head_dim, int rotary_dim,

@@ -54,7 +54,8 @@ namespace {
 constexpr int GT_HALF = 128 * 128;      // bytes of one half-tile
 constexpr int GT_STAGE = 4 * GT_HALF;   // one K tile: x (2 halves) + W (2 halves)
 constexpr int GT_LDS = 2 * GT_STAGE;    // 131072
-constexpr int64_t GT_MAX_STRIDE = (1 << 23) - 8;   // elements between rows of x and W: 128 rows are addressed with 31 bits
+constexpr int64_t GT_MAX_STRIDE = (1 << 23) - 8;   // elements between rows of x and W up to which 128 rows are addressed with 31 bits
+constexpr int64_t GT_MAX_ROW = (1ll << 31) - 128;  // bytes of a row, counted with 31 bits
 
 struct GemmTiledParams {
   const void* x;
@@ -356,16 +357,27 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
 
 // The buffer that holds half h of a group's operand in tile (tm, tn), from its first row on: W for group 0 (waves of pairs: their gate or up
 // rows), x for group 1.  Rows past the matrix read as zeros (of a gate, they are up rows); their results are not stored.
-template <int EPI, int ES>
+// WIDE: rows that lie further apart than a buffer's offsets reach: their address, and how many there are from it on (none: less than
+// one; row `left` - 1 is the matrix's last one whatever its sign, and stands for those past it).
+struct GtRows { const char* p; int64_t ld; int left; };
+template <int EPI, int ES, bool WIDE>
 __device__ __forceinline__ auto gt_half(const GemmTiledParams& p, int tm, int tn, int g, int wc, int h) {
   constexpr int NR = gt_pairs(EPI) ? 64 : 128;
   const int64_t row = g == 0 ? (int64_t)tn * (2 * NR) + h * NR + (gt_pairs(EPI) && (wc & 1) ? p.N >> 1 : 0) : (int64_t)tm * 256 + h * 128;
   const int64_t rows = g == 0 ? p.N : p.M, ld = (g == 0 ? (int64_t)p.K : p.ldx) * ES;
-  const int64_t bytes = row < rows ? min((rows - 1 - row) * ld + (int64_t)p.K * ES, (int64_t)0x7fffffff) : 0;
-  return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)(g == 0 ? p.w : p.x) + row * ld), 0, (int)bytes, 0x00020000);
+  if constexpr (WIDE) {
+    return GtRows{(const char*)(g == 0 ? p.w : p.x) + row * ld, ld, (int)(rows - row)};
+  } else {
+    const int64_t bytes = row < rows ? min((rows - 1 - row) * ld + (int64_t)p.K * ES, (int64_t)0x7fffffff) : 0;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)(g == 0 ? p.w : p.x) + row * ld), 0, (int)bytes, 0x00020000);
+  }
 }
-__device__ __forceinline__ void blds16(__amdgpu_buffer_rsrc_t r, char* l, int voff, int soff) {
+// 16 bytes a lane to LDS.  voff: bytes behind the half's first row (WIDE: 128 times the row, plus bytes), soff: bytes along the rows
+__device__ __forceinline__ void gt_load(__amdgpu_buffer_rsrc_t r, char* l, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)l, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ void gt_load(const GtRows& r, char* l, int voff, int soff) {
+  glds16(r.p + min(voff >> 7, r.left - 1) * r.ld + (voff & 127) + soff, l);
 }
 
 // What a workgroup works on: an output tile, or a split of a tail tile (K tiles t0 .. t0 + T - 1, sums to `part`).
@@ -405,7 +417,7 @@ __device__ __forceinline__ GtItem gt_item(const GemmTiledParams& p, int i, int k
     __builtin_amdgcn_sched_barrier(0);                                                       \
   } while (0)
 
-template <typename T, int EPI, bool FP8>
+template <typename T, int EPI, bool FP8, bool WIDE>
 __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   extern __shared__ __attribute__((aligned(16))) char sm[];
   using frag = typename Mfma<T>::frag;
@@ -439,10 +451,10 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
     // EPI 2: a tile is two heads; wave wcb serves head 2 tn + (wcb >> 1), rotation pairs d and d + 64 with
     // d = 32 (wcb & 1) + at8: a lane ends with 8 d's and their partners.  Pairs: gt_half knows gate (ni < 2) from up.
     const int n = gt_pairs(EPI) ? (rr >> 6) * 32 + at8 : EPI == 2 ? (rr >> 6) * 32 + at8 + (ni >> 1) * 64 : (rr >> 6) * 64 + at8 + (ni >> 1) * 32;
-    voff[i] = (g == 0 ? n * p.K : rr * (int)p.ldx) * ES + c * 16;
+    voff[i] = (WIDE ? (g == 0 ? n : rr) * 128 : (g == 0 ? n * p.K : rr * (int)p.ldx) * ES) + c * 16;
   }
   const int hA = g == 0 ? 0 : 1, hB = g == 0 ? 1 : 0;
-  auto rA = gt_half<EPI, ES>(p, cur.tm, cur.tn, g, wc, hA), rB = gt_half<EPI, ES>(p, cur.tm, cur.tn, g, wc, hB);
+  auto rA = gt_half<EPI, ES, WIDE>(p, cur.tm, cur.tn, g, wc, hA), rB = gt_half<EPI, ES, WIDE>(p, cur.tm, cur.tn, g, wc, hB);
   // LDS image of a K tile: x rows 0..255 (two halves), then W rows 0..255 (two halves)
   constexpr int LX0 = 0, LX1 = GT_HALF, LW0 = 2 * GT_HALF, LW1 = 3 * GT_HALF;
   char* const lds_w = sm + wc * 4096;   // this wave's four 1-KiB pieces inside a half-tile
@@ -451,7 +463,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
 // four 1-KiB pieces of one half-tile: bytes `koff` .. of the rows of buffer r, to stage `stage` (a running number's parity)
 #define GT_REQUEST(r, koff, stage, ldso)                                                     \
   _Pragma("unroll") for (int i = 0; i < 4; ++i)                                              \
-      blds16(r, lds_w + (((stage) & 1) ? GT_STAGE : 0) + (ldso) + i * 1024, voff[i], koff)
+      gt_load(r, lds_w + (((stage) & 1) ? GT_STAGE : 0) + (ldso) + i * 1024, voff[i], koff)
 
   // ---- prologue: all of tile 0 and x rows 0..127 of tile 1 ------------------------------------
   int koff = cur.t0 * 128;    // of K tile t
@@ -519,7 +531,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   if (g == 1) GT_SLOT_END();   // the second group runs one slot behind the first
   for (int item = 1;; ++item) {
     const GtItem nxt = gt_item(p, item, kt);
-    const auto nA = gt_half<EPI, ES>(p, nxt.tm, nxt.tn, g, wc, hA), nB = gt_half<EPI, ES>(p, nxt.tm, nxt.tn, g, wc, hB);
+    const auto nA = gt_half<EPI, ES, WIDE>(p, nxt.tm, nxt.tn, g, wc, hA), nB = gt_half<EPI, ES, WIDE>(p, nxt.tm, nxt.tn, g, wc, hB);
     const int nk = nxt.t0 * 128;
     int t = 0;
     if (!FP8 && cur.T > 2) {   // (sums that start in the MFMAs)
@@ -798,7 +810,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_tail_kernel(GemmTiledParams p)
 
 template <typename T, int EPI, bool FP8>
 int launch_gemm_tiled(const GemmTiledParams& p, hipStream_t st) {
-  auto kern = gemm_tiled_kernel<T, EPI, FP8>;
+  auto kern = std::max<int64_t>(p.ldx, p.K) > GT_MAX_STRIDE ? gemm_tiled_kernel<T, EPI, FP8, true> : gemm_tiled_kernel<T, EPI, FP8, false>;
   (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS);
   // workgroups that stay: as many as there are CUs, in equal numbers for every XCD (with whole tiles in front of a tail: all of them)
   const int per = p.splits == 0 ? (int)cdiv((int64_t)p.mt * p.nt, 8) : std::max(p.full / 8, (int)cdiv((int64_t)p.tail * p.splits, 8));
@@ -1092,7 +1104,7 @@ extern "C" int64_t mi355_tiled_tail_workspace_bytes(int64_t m, int64_t n, int64_
 
 extern "C" int mi355_linear_tiled_supported(int64_t m, int64_t n, int64_t k, int dtype, int epilogue) {
   if (dtype != MI355_BF16 && dtype != MI355_F16) return 0;
-  if (m < 1 || n < 16 || k < 128 || (k & 63) != 0 || m > (1 << 24) || n > (1 << 24) || k > GT_MAX_STRIDE) return 0;
+  if (m < 1 || n < 16 || k < 128 || (k & 63) != 0 || m > (1 << 24) || n > (1 << 24) || k * 2 > GT_MAX_ROW) return 0;
   return (epilogue >= 0 && epilogue <= 3 && n % 16 == 0) ? 1 : 0;   // silu-mul: 8 gate + 8 up columns per lane
 }
 
@@ -1109,8 +1121,8 @@ extern "C" int mi355_linear_tiled_ws(void* y, const void* x, const void* w, cons
   MI355_REQUIRE(mi355_linear_tiled_supported(m, n, k, dtype, epilogue), MI355_ERR_UNSUPPORTED,
                 "mi355_linear_tiled: needs a 16-bit dtype, K %% 64 == 0, K >= 128, N %% 16 == 0 (m=%ld n=%ld k=%ld "
                 "dtype=%d epilogue=%d)", (long)m, (long)n, (long)k, dtype, epilogue);
-  MI355_REQUIRE(x_stride >= k && x_stride % 8 == 0 && x_stride <= GT_MAX_STRIDE, MI355_ERR_INVALID,
-                "mi355_linear_tiled: x_stride must be >= K, a multiple of 8 elements and below 2^23");
+  MI355_REQUIRE(x_stride >= k && x_stride % 8 == 0, MI355_ERR_INVALID,
+                "mi355_linear_tiled: x_stride must be >= K and a multiple of 8 elements");
   MI355_REQUIRE(aligned16(x) && aligned16(w) && aligned16(y) && (bias == nullptr || aligned16(bias)),
                 MI355_ERR_INVALID, "mi355_linear_tiled: pointers must be 16-byte aligned");
   MI355_REQUIRE(epilogue == 0 || bias == nullptr, MI355_ERR_UNSUPPORTED,
@@ -1208,7 +1220,7 @@ extern "C" int mi355_moe_grouped_linear_tiled(void* y, const void* x, int64_t x_
 
 extern "C" int mi355_fp8_scaled_mm_tiled_supported(int64_t m, int64_t n, int64_t k, int out_dtype, int epilogue) {
   if (out_dtype != MI355_BF16 && out_dtype != MI355_F16) return 0;
-  if (m < 1 || n < 16 || k < 256 || (k & 127) != 0 || m > (1 << 24) || n > (1 << 24) || k > GT_MAX_STRIDE) return 0;
+  if (m < 1 || n < 16 || k < 256 || (k & 127) != 0 || m > (1 << 24) || n > (1 << 24) || k > GT_MAX_ROW) return 0;
   return ((epilogue == 0 || epilogue == 1) && n % 16 == 0) ? 1 : 0;
 }
 
@@ -1247,7 +1259,7 @@ extern "C" int mi355_qkv_proj_rope_tiled_supported(int64_t m, int64_t k, int hq,
                                                    int rotary_dim, int is_neox, int dtype, int fp8) {
   if (dtype != MI355_BF16 && dtype != MI355_F16) return 0;
   if (head_dim != 128 || rotary_dim != 128 || !is_neox || hq < 1 || hkv < 1 || ((hq + 2 * hkv) & 1)) return 0;
-  if (m < 1 || m > (1 << 24) || k > GT_MAX_STRIDE) return 0;
+  if (m < 1 || m > (1 << 24) || (fp8 ? k : k * 2) > GT_MAX_ROW) return 0;
   return fp8 ? (k >= 256 && (k & 127) == 0) : (k >= 128 && (k & 63) == 0);
 }
 
@@ -1284,7 +1296,7 @@ extern "C" int mi355_qkv_proj_rope_tiled_ws(void* qkv, const void* x, const void
                 "mi355_qkv_proj_rope_tiled: cos_sin_cache must be fp32 or the tensor dtype");
   MI355_REQUIRE(loc_itype == MI355_I32 || loc_itype == MI355_I64, MI355_ERR_INVALID,
                 "mi355_qkv_proj_rope_tiled: loc must be int32 or int64");
-  MI355_REQUIRE(fp8 ? x_stride == k : (x_stride >= k && x_stride % 8 == 0 && x_stride <= GT_MAX_STRIDE), MI355_ERR_INVALID,
+  MI355_REQUIRE(fp8 ? x_stride == k : (x_stride >= k && x_stride % 8 == 0), MI355_ERR_INVALID,
                 "mi355_qkv_proj_rope_tiled: bad x_stride");
   MI355_REQUIRE(aligned16(x) && aligned16(w) && aligned16(qkv) && aligned16(cos_sin_cache) && aligned16(k_buffer) &&
                     aligned16(v_buffer) && num_slots > 0 && num_slots < (1ll << 31),

@@ -805,7 +805,6 @@ def _tail_workspace(split_tail: bool, m: int, n: int, k: int, fp8: bool, silu_mu
     return (torch.empty(need, dtype=torch.uint8, device=device), need) if need else (None, 0)
 
 
-_TILED_MAX_STRIDE = 1 << 23   # elements: the kernel addresses 128 rows with 31 bits
 _TILED_ACTS = {None: 0, "silu_mul": 1, "gelu_erf": 2, "gelu_tanh_mul": 3}
 
 
@@ -827,8 +826,6 @@ def linear_tiled(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     y = torch.empty((M, N // 2 if pairs else N), dtype=x.dtype, device=x.device)
     if M == 0:
         return y
-    if x.stride(0) >= _TILED_MAX_STRIDE:
-        x = x.contiguous()
     ws, nbytes = _tail_workspace(split_tail, M, N, K, False, pairs, x.device)
     check(_lib_().mi355_linear_tiled_ws(y.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(bias), M, N, K, x.stride(0), _dt(x),
                                         epilogue, _p(ws), nbytes, _stream(x)), "linear_tiled")
@@ -913,8 +910,6 @@ def qkv_proj_rope_tiled(x: torch.Tensor, weight: torch.Tensor, hq: int, hkv: int
     qkv = torch.empty((M, N), dtype=dtype, device=x.device)
     if M == 0:
         return qkv
-    if x.stride(0) >= _TILED_MAX_STRIDE:
-        x = x.contiguous()
     ws, nbytes = _tail_workspace(split_tail, M, N, K, fp8, False, x.device)
     check(_lib_().mi355_qkv_proj_rope_tiled_ws(
         qkv.data_ptr(), x.data_ptr(), weight.data_ptr(), _p(x_scale), _p(w_scale), M, K, x.stride(0), hq, hkv,

@@ -1227,11 +1227,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // tokens x 16 heads: 154 us, and about 70 for that projection; the absorbed launch with its two per-head products took 1570 us).
 // Without a prefix to address, and with the rope part's rows dealt to all threads (two pieces each instead of four to half of
 // them), the body fits 256 registers: two workgroups per CU, one's softmax beside the other's MFMAs.  At one per CU: 226 us; 32
-// heads 404 -> 238.
-template <typename T>
+// heads 404 -> 238.  DIRECT: for rows that 32-bit offsets reach.
+template <typename T, bool DIRECT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void extend_attn_latent_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ o, ExtendParams p, int nqb, int npairs) {
-  extend_attn_mfma32_body<T, false, 192, true, 128, false, false, true>(q, k, v, o, nullptr, nullptr, p, nqb, npairs);
+  extend_attn_mfma32_body<T, false, 192, true, 128, false, false, DIRECT>(q, k, v, o, nullptr, nullptr, p, nqb, npairs);
 }
 
 template <typename T, int DP, int BN>
@@ -1482,8 +1482,8 @@ int mi355_latent_prefill_attention(void* out, const void* q, int64_t q_stride, c
                 nope_dim, rope_dim, v_dim, rot_dims, dtype);
   MI355_REQUIRE(bs >= 0 && max_len >= 0 && heads > 0 && scale > 0.f, MI355_ERR_INVALID, "latent_prefill_attention: bad shape");
   MI355_REQUIRE(q_stride >= (int64_t)heads * 192 && q_stride % 8 == 0 && kv_stride >= (int64_t)heads * 256 && kv_stride % 8 == 0 &&
-                    k_rope_stride >= 64 && k_rope_stride % 8 == 0 && kv_stride < (1 << 23) && k_rope_stride < (1 << 23) && aligned16(q) && aligned16(kv) && aligned16(k_rope) && aligned16(out),
-                MI355_ERR_INVALID, "latent_prefill_attention: rows must be 16-byte aligned, hold every head and lie less than 2^23 elements apart");
+                    k_rope_stride >= 64 && k_rope_stride % 8 == 0 && aligned16(q) && aligned16(kv) && aligned16(k_rope) && aligned16(out),
+                MI355_ERR_INVALID, "latent_prefill_attention: rows must be 16-byte aligned and hold every head");
   if (bs == 0 || max_len == 0) return MI355_OK;
   ExtendParams p = {};
   p.seg_start = seg_start; p.seg_len = seg_len; p.positions = positions; p.inv_freq = inv_freq;
@@ -1494,11 +1494,14 @@ int mi355_latent_prefill_attention(void* out, const void* q, int64_t q_stride, c
   const int nqb = (int)((max_len + 127) / 128);
   const int64_t npairs = bs * heads, wgs = 8 * ((npairs + 7) / 8) * nqb;
   MI355_REQUIRE(wgs < (int64_t)1 << 31, MI355_ERR_UNSUPPORTED, "latent_prefill_attention: too many query blocks");
-  constexpr int lds = 2 * direct_stage_bytes<192>();     // 80 KiB: two workgroups a CU
+  // 80 KiB: two workgroups a CU (rows of 2^23 elements and more apart: through registers, as before there were buffer loads)
+  const bool direct = kv_stride < (1 << 23) && k_rope_stride < (1 << 23);
+  const int lds = direct ? 2 * direct_stage_bytes<192>() : 0;
 #define MI355_LP(T)                                                                                                            \
-  (void)hipFuncSetAttribute((const void*)extend_attn_latent_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);       \
-  hipLaunchKernelGGL((extend_attn_latent_kernel<T>), dim3((unsigned)wgs), dim3(256), lds, (hipStream_t)stream, (const T*)q,       \
-                     (const T*)kv, (const T*)kv + 128, (T*)out, p, nqb, (int)npairs)
+  auto kernel = direct ? extend_attn_latent_kernel<T, true> : extend_attn_latent_kernel<T, false>;                             \
+  if (lds != 0) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);               \
+  hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), lds, (hipStream_t)stream, (const T*)q, (const T*)kv, (const T*)kv + 128, (T*)out, p, \
+                     nqb, (int)npairs)
   if (dtype == MI355_BF16) { MI355_LP(bf16_t); }
   else { MI355_LP(f16_t); }
 #undef MI355_LP

@@ -1506,8 +1506,6 @@ def latent_prefill_attention(q: torch.Tensor, kv: torch.Tensor, k_rope: torch.Te
     assert kv.shape[:2] == (T, H) and k_rope.shape[0] == T and positions.numel() == T
     assert q.dtype == kv.dtype == k_rope.dtype and seg_start.dtype == seg_len.dtype == torch.int32 and positions.dtype == torch.int64
     assert rot_dims == 0 or (inv_freq.dtype == torch.float32 and 2 * inv_freq.numel() >= rot_dims)
-    if max(kv.stride(0), k_rope.stride(0)) >= 1 << 23:     # (the kernel addresses 64 rows with 31 bits)
-        kv, k_rope = kv.contiguous(), k_rope.contiguous()
     out = torch.empty((T, H, v), dtype=q.dtype, device=q.device)
     check(_lib_().mi355_latent_prefill_attention(out.data_ptr(), q.data_ptr(), q.stride(0), kv.data_ptr(), kv.stride(0), k_rope.data_ptr(),
                                                  k_rope.stride(0), seg_start.data_ptr(), seg_len.data_ptr(), positions.data_ptr(),

@@ -60,3 +60,28 @@ def test_refusals():
     assert not ops.latent_prefill_attention_supported(128, 64, 128, 32, False, torch.bfloat16)     # pairs across lanes
     assert not ops.latent_prefill_attention_supported(64, 64, 128, 64, True, torch.bfloat16)
     assert not ops.latent_prefill_attention_supported(128, 64, 128, 64, True, torch.float32)
+
+
+@pytest.mark.parametrize("lens", [[1], [70, 1, 129]])
+@pytest.mark.parametrize("kv_far,rope_far", [(True, False), (False, True), (True, True)])
+def test_rows_far_apart(lens, kv_far, rope_far):
+    """Rows 2^23 elements apart, further than 32-bit offsets reach, one row (whose stride torch does not take for one) and several: the bits
+    of the same rows close together."""
+    from sglang_custom_amd import ops
+
+    T, H, stride = sum(lens), 2, 1 << 23
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q, kv, rope = (torch.randn(T, w, device=DEV, generator=g).bfloat16() for w in (H * 192, H * 256, 64))
+    start = torch.tensor([sum(lens[:i]) for i in range(len(lens))], dtype=torch.int32, device=DEV)
+    n, pos = torch.tensor(lens, dtype=torch.int32, device=DEV), torch.arange(T, device=DEV)
+
+    def far(x):
+        rows = torch.empty((T - 1) * stride + x.shape[1], dtype=x.dtype, device=DEV).as_strided(x.shape, (stride, 1))
+        return rows.copy_(x)
+
+    def run(kv, rope):
+        assert kv.stride(0) in (H * 256, stride)
+        return ops.latent_prefill_attention(q.view(T, H, 192), kv.as_strided((T, H, 256), (kv.stride(0), 256, 1)), rope, start, n, pos, None, 0,
+                                            max(lens), 0.1)
+
+    assert torch.equal(run(far(kv) if kv_far else kv, far(rope) if rope_far else rope), run(kv, rope))

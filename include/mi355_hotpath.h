@@ -251,7 +251,8 @@ int mi355_decode_split_plan(int64_t bs, int hkv, int64_t max_seq_len, int max_sp
  * k_buffer[kv_indices[kv_indptr[b]..kv_indptr[b+1]]].  Phase 1 attends the prefix (no mask),
  * phase 2 the new tokens (causal if is_causal).  custom_mask (uint8, may be NULL) follows the
  * reference layout: mask_indptr[b] + row * (prefix+extend) + col, applied to phase 2 always
- * and to phase 1 unless skip_prefix_custom_mask.  sliding_window_size < 0 = off.
+ * and to phase 1 unless skip_prefix_custom_mask.  sliding_window_size < 0 = off.  num_slots: of the cache; in the [slots, Hkv, D] layout
+ * it only chooses between two forms of the kernel that give the same bits (up to 4 GiB of rows a buffer, and beyond).
  * replaces: extend_attention_fwd (layers/attention/triton_ops/extend_attention.py:306-438),
  *           extend_attention_cpu (sgl-kernel/csrc/cpu/extend.cpp:579-722),
  *           TorchNativeAttnBackend._run_sdpa_forward_extend (torch_native_backend.py:27-110). */

@@ -29,6 +29,7 @@ struct ExtendParams {
   float sm_scale, logit_cap;
   // the cache buffers: elements between consecutive slots / consecutive kv heads ([slots, hkv, d] or head-major)
   int64_t kb_slot, kb_head, vb_slot, vb_head;
+  uint32_t near_slots;   // DIRECT: slots below this one lie within the 32-bit offsets of a buffer
   int kv8;   // the cache holds e4m3fn bytes behind the element pointers (strides count bytes); read by the VALU kernel
   // latent form (extend_attn_latent_kernel): whole sequences, tokens seg_start[b] .. + seg_len[b]
   const int32_t* seg_start;
@@ -806,7 +807,8 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
   };
 
   // DIRECT: rows srow + 16 i of a tile go to the image's rows 4 wave + 16 i .. + 3 (1 KiB a wave, in the lanes' order); lane sch of a row fetches the
-  // chunk that belongs there.  Rows of this launch: the tile's first row is the buffer's base; cached ones: the head's first.
+  // chunk that belongs there.  Rows of this launch: the tile's first row is the buffer's base; cached ones: the head's first.  A wave that has a
+  // slot further away than the offsets reach (the launcher goes by the slots that the caller says there are) takes its rows through registers.
   [[maybe_unused]] const unsigned gch = (sch ^ (((srow & 3) << 2) | ((srow >> 2) & 3))) * 16u, gch2 = (sch2 ^ ((srow2 >> 1) & 7)) * 16u;
   [[maybe_unused]] const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
   [[maybe_unused]] auto direct_tile = [&](int kt, int stage) {
@@ -827,14 +829,16 @@ __device__ __forceinline__ bool extend_attn_mfma32_body(
 #pragma unroll
         for (int j = 0; j < 2; ++j) buffer_to_lds16(rr, dst + 32768 + 4096 * j, min(srow2 + 32 * j, left - 1) * (unsigned)p.k_rope_stride * 2 + gch2);
       }
-    } else if (kt * 64 + 64 <= prefix) {
+    } else if (kt * 64 + 64 <= prefix &&
+               __builtin_amdgcn_ballot_w64(max(max((uint32_t)next_slot[0], (uint32_t)next_slot[1]), max((uint32_t)next_slot[2], (uint32_t)next_slot[3])) >=
+                                           p.near_slots) == 0) {
       const auto rk = wide_rsrc(kbuf + kvh * p.kb_head), rv = wide_rsrc(vbuf + kvh * p.vb_head);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         buffer_to_lds16(rk, dst + 4096 * i, next_slot[i] * (unsigned)(p.kb_slot * 2) + gch);
         buffer_to_lds16(rv, dst + 16384 + 4096 * i, next_slot[i] * (unsigned)(p.vb_slot * 2) + gch);
       }
-    } else {   // the tile that holds the prefix's last rows and the first new ones: through registers
+    } else {   // the tile that holds the prefix's last rows and the first new ones, or rows far away: through registers
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = min(kt * 64 + srow + 16 * i, total - 1);
@@ -1275,7 +1279,7 @@ static bool mfma32_serves(int D, int Dv, bool kv8, bool mask, int sliding_window
 }
 
 template <typename T, int D>
-static int launch_mfma32(const void* q, const void* k, const void* v, void* o, const void* kb, const void* vb, const ExtendParams& p,
+static int launch_mfma32(const void* q, const void* k, const void* v, void* o, const void* kb, const void* vb, ExtendParams p,
                          int64_t bs, int nqb, int64_t npairs, int64_t wgs, int splits, bool kv8, int64_t num_slots, hipStream_t st) {
   using Kernel = void (*)(const T*, const T*, const T*, T*, const T*, const T*, ExtendParams, int, int);
   Kernel kernel;
@@ -1289,8 +1293,9 @@ static int launch_mfma32(const void* q, const void* k, const void* v, void* o, c
                              : (kv8 ? extend_attn_mfma32_d64_kernel<T, true, false, false> : extend_attn_mfma32_d64_kernel<T, false, false, false>);
   } else {
     // (32-bit offsets: the cache of 4 GiB a layer and side, new rows of 16 MiB)
-    const bool direct = !kv8 && num_slots > 0 && num_slots < (1ll << 31) && num_slots * std::max(p.kb_slot, p.vb_slot) * 2 <= 0xffff0000ll &&
-                        p.k_stride < (1 << 23) && p.v_stride < (1 << 23);
+    const int64_t near = 0xffff0000ll / (2 * std::max(p.kb_slot, p.vb_slot));
+    const bool direct = !kv8 && num_slots > 0 && num_slots <= near && p.k_stride < (1 << 23) && p.v_stride < (1 << 23);
+    p.near_slots = (uint32_t)near;
     if (direct) kernel = splits > 1 ? extend_attn_mfma32_kernel<T, false, true, true> : extend_attn_mfma32_kernel<T, false, false, true>;
     else if (kv8) kernel = splits > 1 ? extend_attn_mfma32_kernel<T, true, true, false> : extend_attn_mfma32_kernel<T, true, false, false>;
     else kernel = splits > 1 ? extend_attn_mfma32_kernel<T, false, true, false> : extend_attn_mfma32_kernel<T, false, false, false>;

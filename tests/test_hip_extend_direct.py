@@ -67,7 +67,7 @@ def test_cached_offsets_past_two_gib():
 
     hq, hkv, D, slots, P, T = 8, 8, 128, 1_900_000, 100, 40
     if torch.cuda.get_device_properties(0).total_memory < 32 << 30:
-        pytest.skip("16 GiB of cache")
+        pytest.skip("8 GiB of cache")
     g = torch.Generator(device=DEV).manual_seed(3)
     kb, vb = (torch.zeros(slots, hkv, D, device=DEV, dtype=torch.bfloat16) for _ in range(2))
     rows = [torch.randn(P, hkv, D, device=DEV, generator=g).bfloat16() for _ in range(2)]
@@ -81,3 +81,40 @@ def test_cached_offsets_past_two_gib():
         ops.extend_attention_fwd(q, k, v, o, kb, vb, qo, kvp, at.int(), None, True, None, T, D ** -0.5)
         out.append(o)
     assert torch.equal(out[0], out[1]) and bool((out[0] != 0).any())
+
+
+@pytest.mark.parametrize("num_slots", [1, 0, 2_200_000])
+def test_slots_past_four_gib(num_slots):
+    """A cache of more than 4 GiB, its rows near, far and mixed within a tile, whatever count of slots the caller gives ([slots, heads, D] does
+    not need it): the bits of a small cache with the same rows."""
+    from sglang_custom_amd import _lib, ops
+
+    lib = _lib.load()
+    hq, hkv, D, slots, P, T = 8, 8, 128, 2_200_000, 300, 40
+    if torch.cuda.get_device_properties(0).total_memory < 32 << 30:
+        pytest.skip("9 GiB of cache")
+    g = torch.Generator(device=DEV).manual_seed(4)
+    rows = [torch.randn(P, hkv, D, device=DEV, generator=g).bfloat16() for _ in range(2)]
+    q, k, v = (torch.randn(T, h, D, device=DEV, generator=g).bfloat16() for h in (hq, hkv, hkv))
+    qo, kvp = (torch.tensor([0, n], dtype=torch.int32, device=DEV) for n in (T, P))
+
+    def run(kb, vb, at, count, splits):
+        o = torch.full((T, hq, D), float("nan"), device=DEV, dtype=torch.bfloat16)
+        need = lib.mi355_extend_attention_workspace_bytes(T, hq, D, splits) if splits > 1 else 0
+        ws, kvi = torch.empty(max(need, 16), dtype=torch.uint8, device=DEV), at.int()
+        assert lib.mi355_extend_attention_ws(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), kb.data_ptr(), vb.data_ptr(), qo.data_ptr(), kvp.data_ptr(), kvi.data_ptr(), None,
+            None, 1, 1, 1, T, hq, hkv, D, D, hq * D, hkv * D, hkv * D, count, D ** -0.5, 0.0, 0, ops._kvdt(q, kb, vb), T, splits, ws.data_ptr(), need,
+            torch.cuda.current_stream().cuda_stream) == 0
+        return o
+
+    near = torch.arange(5, 5 + P, device=DEV)
+    far = torch.arange(slots - 5 - P, slots - 5, device=DEV)
+    edge = 0xFFFF0000 // (2 * hkv * D) - 100 + torch.arange(P, device=DEV)          # the first tiles within reach, the last ones not
+    mixed = torch.where(torch.arange(P, device=DEV) % 7 == 3, far, near)
+    kb, vb = (torch.full((slots, hkv, D), float("nan"), device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    want = [run(rows[0], rows[1], torch.arange(P, device=DEV), P, splits) for splits in (1, 2)]
+    for at in (near, far, edge, mixed):
+        kb[at], vb[at] = rows
+        for splits in (1, 2):
+            assert torch.equal(run(kb, vb, at, num_slots, splits), want[splits - 1])

@@ -113,12 +113,14 @@ template <bool FP8> __device__ __forceinline__ int gt_swz(int r) {
 // the rounding points of mi355_rope_inplace (cos / sin -> T; every product and sum rounds to T on its own, so
 // no contraction here); rotated q / k and plain v go to y, the k and v rows also to the KV cache.
 // The lane holds, for each of its 8 rows, columns d0 .. d0 + 7 of one head (acc[mi][0..1]) and their rotation
-// partners d0 + 64 .. d0 + 71 (acc[mi][2..3]).  Every load (positions, cache slots, cos / sin rows) is
-// requested before the arithmetic of the rows it belongs to: nothing else runs on the CU during an epilogue,
-// so a chain of dependent loads per row would be paid in full.
+// partners d0 + 64 .. d0 + 71 (acc[mi][2..3]).  Bound by the latency of its loads (positions, and the cos / sin rows that they name): all
+// positions are requested first, cos / sin, cache slots and scales two or three rows ahead of the row that is worked on, and both groups of waves are
+// here at once (TOGETHER in the kernel), or the second's chain would begin where the first's ends.  6144 columns, K 4096, us at 4605, 7725
+// and 16384 rows of bf16: the groups one behind the other, two rows' loads at a time and 14 registers in scratch memory 192.6, 297, 609; no register
+// there (see the kernel) 191, 297, 605; the groups together 188.6, 290, 590; rows ahead 185, 289, 583 (a workgroup per tile 191.7, 297, 598).
+// fp8 at 4605 and 7725: 111, 170; 108, 166; 106, 161; 105, 159 (105.6, 165).
 template <typename T, bool FP8, bool CSF32, int NM>
-__device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], const float (&sxm)[NM],
-                                                  int mbase, int tn, int wc, int q4) {
+__device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], int mbase, int tn, int wc, int q4) {
 #pragma clang fp contract(off)
   T* yg = (T*)p.y;
   const int head = 2 * tn + (wc >> 1), d0 = (wc & 1) * 32 + q4 * 8;
@@ -133,88 +135,66 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x
     slo[j] = FP8 ? p.w_scale[col0 + j] : 1.f;
     shi[j] = FP8 ? p.w_scale[col0 + 64 + j] : 1.f;
   }
-  int posv[NM], slotv[NM];   // positions and slot numbers fit 31 bits (the host checks the slot count)
+  // R - 1 rows' cos / sin, slots and scales are on their way in front of the row that is worked on (register budget)
+  constexpr int R = CSF32 ? 3 : 4;
+  auto row_of = [&](int mi) { return min(mbase + mi * 16, p.M - 1); };
+  int posv[NM], slotv[R];   // positions and slot numbers fit 31 bits (the host checks the slot count)
+  using CS = std::conditional_t<CSF32, float, T>;
+  Vec<CS, 8> c[R], sn[R];
+  float sxm[R];
+#pragma unroll
+  for (int mi = 0; mi < NM; ++mi) posv[mi] = (int)p.positions[row_of(mi)];
+  auto request = [&](int mi) {   // (v heads read cos / sin too and ignore them: the branch below is wave-uniform)
+    const int i = mi % R, m = row_of(mi);
+    const int64_t pos = posv[mi];
+    const CS* cs = (const CS*)p.cos_sin + pos * 128 + d0;
+#pragma unroll
+    for (int at = 0; at < 8; at += V16<CS>::n) {
+      const auto cv = ldvec<CS, V16<CS>::n>(cs + at), sv = ldvec<CS, V16<CS>::n>(cs + 64 + at);
+#pragma unroll
+      for (int j = 0; j < V16<CS>::n; ++j) { c[i].v[at + j] = cv.v[j]; sn[i].v[at + j] = sv.v[j]; }
+    }
+    slotv[i] = cache_dst == nullptr ? 0 : p.loc_i32 ? ((const int32_t*)p.loc)[m] : (int)((const int64_t*)p.loc)[m];
+    sxm[i] = FP8 ? p.x_scale[m] : 1.f;
+  };
+#pragma unroll
+  for (int mi = 0; mi < min(R - 1, NM); ++mi) request(mi);
 #pragma unroll
   for (int mi = 0; mi < NM; ++mi) {
-    const int m = mbase + mi * 16;
-    posv[mi] = (int)p.positions[m < p.M ? m : p.M - 1];
-    slotv[mi] = 0;
-  }
-  if (cache_dst != nullptr) {
-    if (p.loc_i32) {
+    if (mi + R - 1 < NM) request(mi + R - 1);
+    const int i = mi % R, m = mbase + mi * 16;
+    float x1[8], x2[8];
 #pragma unroll
-      for (int mi = 0; mi < NM; ++mi) {
-        const int m = mbase + mi * 16;
-        slotv[mi] = ((const int32_t*)p.loc)[m < p.M ? m : p.M - 1];
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float lo = acc[mi][h][r], hi = acc[mi][2 + h][r];
+        if (FP8) { lo = (lo * sxm[i]) * slo[h * 4 + r]; hi = (hi * sxm[i]) * shi[h * 4 + r]; }
+        round2_to<T>(lo, hi, x1[h * 4 + r], x2[h * 4 + r]);   // the projection's own result, rounded to T
+      }
+    Vec<T, 8> o1, o2;
+    if (rot) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float cj = to_f32(c[i].v[j]), sj = to_f32(sn[i].v[j]);
+        if constexpr (CSF32) round2_to<T>(cj, sj, cj, sj);   // a table of dtype T holds rounded values already
+        float a1, a2, b1, b2;
+        round2_to<T>(x1[j] * cj, x2[j] * sj, a1, a2);
+        round2_to<T>(x2[j] * cj, x1[j] * sj, b1, b2);
+        o1.v[j] = from_f32<T>(a1 - a2);
+        o2.v[j] = from_f32<T>(b1 + b2);
       }
     } else {
 #pragma unroll
-      for (int mi = 0; mi < NM; ++mi) {
-        const int m = mbase + mi * 16;
-        slotv[mi] = (int)((const int64_t*)p.loc)[m < p.M ? m : p.M - 1];
-      }
+      for (int j = 0; j < 8; ++j) { o1.v[j] = from_f32<T>(x1[j]); o2.v[j] = from_f32<T>(x2[j]); }
     }
-  }
-  constexpr int G = NM < 4 ? NM : (CSF32 || FP8) ? 2 : 4;   // rows whose cos / sin are in flight together (register budget)
-#pragma unroll
-  for (int half = 0; half < NM / G; ++half) {
-    // cos / sin of G rows (v heads read them too and ignore them: the branch below is wave-uniform)
-    float c[G][8], sn[G][8];
-#pragma unroll
-    for (int i = 0; i < G; ++i) {
-      const int64_t pos = posv[half * G + i];
-      if constexpr (CSF32) {
-        const float* cs = (const float*)p.cos_sin + pos * 128 + d0;
-        const float4 c0 = *reinterpret_cast<const float4*>(cs), c1 = *reinterpret_cast<const float4*>(cs + 4);
-        const float4 s0 = *reinterpret_cast<const float4*>(cs + 64), s1 = *reinterpret_cast<const float4*>(cs + 68);
-        c[i][0] = c0.x; c[i][1] = c0.y; c[i][2] = c0.z; c[i][3] = c0.w;
-        c[i][4] = c1.x; c[i][5] = c1.y; c[i][6] = c1.z; c[i][7] = c1.w;
-        sn[i][0] = s0.x; sn[i][1] = s0.y; sn[i][2] = s0.z; sn[i][3] = s0.w;
-        sn[i][4] = s1.x; sn[i][5] = s1.y; sn[i][6] = s1.z; sn[i][7] = s1.w;
-      } else {
-        const T* cs = (const T*)p.cos_sin + pos * 128 + d0;
-        const Vec<T, 8> cv = ldvec<T, 8>(cs), sv = ldvec<T, 8>(cs + 64);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { c[i][j] = to_f32(cv.v[j]); sn[i][j] = to_f32(sv.v[j]); }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < G; ++i) {
-      const int mi = half * G + i;
-      const int m = mbase + mi * 16;
-      float x1[8], x2[8];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float lo = acc[mi][h][r], hi = acc[mi][2 + h][r];
-          if (FP8) { lo = (lo * sxm[mi]) * slo[h * 4 + r]; hi = (hi * sxm[mi]) * shi[h * 4 + r]; }
-          round2_to<T>(lo, hi, x1[h * 4 + r], x2[h * 4 + r]);   // the projection's own result, rounded to T
-        }
-      Vec<T, 8> o1, o2;
-      if (rot) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float cj = c[i][j], sj = sn[i][j];
-          if constexpr (CSF32) round2_to<T>(cj, sj, cj, sj);   // a table of dtype T holds rounded values already
-          float a1, a2, b1, b2;
-          round2_to<T>(x1[j] * cj, x2[j] * sj, a1, a2);
-          round2_to<T>(x2[j] * cj, x1[j] * sj, b1, b2);
-          o1.v[j] = from_f32<T>(a1 - a2);
-          o2.v[j] = from_f32<T>(b1 + b2);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { o1.v[j] = from_f32<T>(x1[j]); o2.v[j] = from_f32<T>(x2[j]); }
-      }
-      if (m < p.M) {
-        stvec<T, 8>(yg + (int64_t)m * p.ldy + col0, o1);
-        stvec<T, 8>(yg + (int64_t)m * p.ldy + col0 + 64, o2);
-        if (cache_dst != nullptr) {
-          T* dst = cache_dst + (int64_t)slotv[mi] * p.kv_slot;
-          stvec<T, 8>(dst, o1);
-          stvec<T, 8>(dst + 64, o2);
-        }
+    if (m < p.M) {
+      stvec<T, 8>(yg + (int64_t)m * p.ldy + col0, o1);
+      stvec<T, 8>(yg + (int64_t)m * p.ldy + col0 + 64, o2);
+      if (cache_dst != nullptr) {
+        T* dst = cache_dst + (int64_t)slotv[i] * p.kv_slot;
+        stvec<T, 8>(dst, o1);
+        stvec<T, 8>(dst + 64, o2);
       }
     }
   }
@@ -268,15 +248,15 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
   const int mbase = m0 + r16;
   T* yg = (T*)p.y;
   [[maybe_unused]] const T* bias = (const T*)p.bias;
-  float sxm[NM];
+  [[maybe_unused]] float sxm[NM];
 #pragma unroll
   for (int mi = 0; mi < NM; ++mi) {
     const int m = mbase + mi * 16;
-    sxm[mi] = FP8 ? p.x_scale[m < p.M ? m : p.M - 1] : 1.f;
+    sxm[mi] = FP8 && EPI != 2 ? p.x_scale[m < p.M ? m : p.M - 1] : 1.f;
   }
   if constexpr (EPI == 2) {
-    if (p.cs_f32) qkv_rope_epilogue<T, FP8, true, NM>(p, acc, sxm, mbase, tn, wc, q4);
-    else qkv_rope_epilogue<T, FP8, false, NM>(p, acc, sxm, mbase, tn, wc, q4);
+    if (p.cs_f32) qkv_rope_epilogue<T, FP8, true, NM>(p, acc, mbase, tn, wc, q4);
+    else qkv_rope_epilogue<T, FP8, false, NM>(p, acc, mbase, tn, wc, q4);
   } else if (gt_pairs(EPI)) {
     const int j0 = tn * 128 + wc * 32 + q4 * 8;
     if (j0 < ncols) {
@@ -397,8 +377,10 @@ __device__ __forceinline__ GtItem gt_item(const GemmTiledParams& p, int i, int k
     it.valid = at < whole;
     if (it.valid) tile_of(p, at, it.tm, it.tn);
   } else if (p.splits != 0 && j - per < wide) {
-    const int tper = (p.tail * p.splits + 7) >> 3, u = xcd * tper + li;
-    it.valid = li < tper && u < p.tail * p.splits;
+    int mine = li;
+    asm volatile("" : "+s"(mine));    // (else the split is worked out in front of the tiles, and kept for all of them)
+    const int tper = (p.tail * p.splits + 7) >> 3, u = xcd * tper + mine;
+    it.valid = mine < tper && u < p.tail * p.splits;
     if (it.valid) {
       const int k = u / p.tail, t = u - k * p.tail;
       tile_of(p, p.full + t, it.tm, it.tn);
@@ -478,6 +460,8 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
   const int rd0 = r16 * 128 + (((FP8 ? 2 * q4 : q4) ^ gt_swz<FP8>(r16)) << 4);
   const int a_off = g * GT_HALF, b_off = 2 * GT_HALF + wc * 8192;
 
+  // EPI 2 waits for loads: both groups at once
+  constexpr bool TOGETHER = EPI == 2;
   f32x4 acc[8][4];
   // two 16-byte registers per fragment slot: k-steps 0 / 1 (16-bit) or the two halves of the 32-byte
   // fp8 fragment
@@ -570,19 +554,29 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
         }
       });
     }
-    if (!nxt.valid && g == 0) __builtin_amdgcn_s_barrier();   // (the other group is one slot behind)
+    if ((TOGETHER || !nxt.valid) && g == 0) __builtin_amdgcn_s_barrier();   // (the other group is one slot behind)
+    // The lane's number and the arguments again: otherwise the compiler works out the epilogue's addresses in front of all tiles and keeps
+    // them, with every argument, in scratch memory and in lanes of a register.  2 x 14336 columns with SiLU-and-mul, 65536 rows: 10.70 ms so,
+    // 10.22 this way (a workgroup per tile 10.45).
+    int zero = 0;
+    asm volatile("" : "+v"(zero));
+    const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+    auto args = (const __attribute__((address_space(4))) GemmTiledParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const GemmTiledParams& pe = *(const GemmTiledParams*)args;
     if (cur.part != nullptr) {   // a split of a tail tile: its sums as they lie in the registers
 #pragma unroll
       for (int mi = 0; mi < 8; ++mi)
-        if (cur.tm * 256 + g * 128 + mi * 16 < p.M)
+        if (cur.tm * 256 + g * 128 + mi * 16 < pe.M)
 #pragma unroll
-          for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(cur.part + ((wave * 8 + mi) * 4 + ni) * 256 + lane * 4) = acc[mi][ni];
-    } else if (EPI == 0 && p.bias != nullptr) {
-      tile_epilogue<T, EPI, FP8, 8, true>(p, acc, cur.tm * 256 + g * 128, cur.tm, cur.tn, wc, q4, r16, 256);
+          for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(cur.part + ((wave * 8 + mi) * 4 + ni) * 256 + el * 4) = acc[mi][ni];
+    } else if (EPI == 0 && pe.bias != nullptr) {
+      tile_epilogue<T, EPI, FP8, 8, true>(pe, acc, cur.tm * 256 + g * 128, cur.tm, cur.tn, wc, el >> 4, el & 15, 256);
     } else {
-      tile_epilogue<T, EPI, FP8, 8, false>(p, acc, cur.tm * 256 + g * 128, cur.tm, cur.tn, wc, q4, r16, 256);
+      tile_epilogue<T, EPI, FP8, 8, false>(pe, acc, cur.tm * 256 + g * 128, cur.tm, cur.tn, wc, el >> 4, el & 15, 256);
     }
     if (!nxt.valid) break;
+    if (TOGETHER && g == 1) GT_SLOT_END();   // and is again
     cur = nxt;
     rA = nA;
     rB = nB;

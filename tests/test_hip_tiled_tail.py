@@ -73,6 +73,38 @@ def test_split_tiles_rotate_and_write_the_cache(ops, m, k, hq, hkv):
         assert torch.equal(a, b)
 
 
+# more tiles than CUs, so that workgroups take a second one: whole (408 tiles: their rest shares nothing), with K tiles that are two, odd and
+# many; and behind whole ones, a rest of 32 tiles that shares K.  Ragged last rows
+@pytest.mark.parametrize("m,k,hq,hkv", [(4100, 128, 30, 9), (4100, 320, 30, 9), (4090, 1024, 38, 5), (2820, 1088, 30, 9)])
+@pytest.mark.parametrize("form", ["bf16", "f16", "fp8", "fp8 f16"])
+@pytest.mark.parametrize("cs_f32", [True, False])
+def test_qkv_rope_over_several_tiles_a_workgroup(ops, m, k, hq, hkv, form, cs_f32):
+    """The projection as torch has it (exact: whole numbers), then the rotation and cache write of their own kernel."""
+    g = torch.Generator().manual_seed(m + k)
+    dt, fp8 = torch.float16 if "f16" in form.replace("bf16", "") else torch.bfloat16, "fp8" in form
+    if fp8:
+        k *= 2
+    n = (hq + 2 * hkv) * 128
+    assert -(-m // 256) * n // 256 > 256 and (ops.tiled_tail_splits(m, n, k, fp8) > 1) == (m == 2820)
+    x, w = ints(g, m, k), ints(g, n, k)
+    pos = torch.randint(0, 500, (m,), generator=g).to(DEV)
+    angle = torch.rand(500, 64, generator=g) * 6
+    cs = torch.cat([angle.cos(), angle.sin()], 1).to(DEV, torch.float32 if cs_f32 else dt)
+    loc = torch.randperm(m + 9, generator=g)[:m].to(DEV, torch.int32 if m % 4 else torch.int64)
+    xs, ws = (2.0 ** torch.randint(-3, 2, (r,), generator=g).float().to(DEV) if fp8 else torch.ones(r, device=DEV) for r in (m, n))
+    ref = ((x @ w.T) * xs[:, None] * ws).to(dt)
+    kb, vb, kr, vr = (torch.zeros(m + 9, hkv, 128, dtype=dt, device=DEV) for _ in range(4))
+    q, kk, v = ref.split([hq * 128, hkv * 128, hkv * 128], dim=-1)
+    ops.rope_inplace(pos, q, kk, 128, cs, True, v=v, k_buffer=kr, v_buffer=vr, loc=loc)
+    for split in (False, True):
+        if fp8:
+            f8 = torch.float8_e4m3fn
+            got = ops.qkv_proj_rope_tiled(x.to(f8), w.to(f8), hq, hkv, 128, pos, cs, True, kb, vb, loc, xs, ws, dt, split_tail=split)
+        else:
+            got = ops.qkv_proj_rope_tiled(x.to(dt), w.to(dt), hq, hkv, 128, pos, cs, True, kb, vb, loc, split_tail=split)
+        assert torch.equal(got, ref) and torch.equal(kb, kr) and torch.equal(vb, vr)
+
+
 def test_a_workspace_that_is_too_small_is_refused(ops):
     lib = ops._lib_()
     m, n, k = 300, 4096, 14336

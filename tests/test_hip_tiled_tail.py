@@ -6,8 +6,8 @@ import torch
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 # rows, columns, K: no whole round (one tile; one live row in the second; sixteen splits), tails of 16 and 128 tiles behind a whole
-# round, K tiles that do not divide by the splits
-SHAPES = [(65, 240, 2048), (257, 2048, 8192), (4100, 4080, 1088), (2048, 12288, 2624), (300, 4096, 14336)]
+# round, K tiles that do not divide by the splits, tails of 50 and 41 (33 and 8 of pairs) with ragged last rows and columns
+SHAPES = [(65, 240, 2048), (257, 2048, 8192), (4100, 4080, 1088), (2048, 12288, 2624), (300, 4096, 14336), (4103, 4368, 1152), (8200, 2064, 2048)]
 
 
 @pytest.fixture(scope="module")

@@ -591,7 +591,8 @@ __device__ __forceinline__ int xor_image_off(int row, int ch) {   // bytes; ch =
 // that, but the compiler takes it for a flat access and then waits for every LDS read behind it to the last one: 173 us.)
 // us a launch, 16-bit rows: registers | DIRECT | and the weights of a k-step made beside the MFMAs of the one before, MFMAs at a raised wave
 // priority: 5 x 1100 ragged 49.5 | 45.5 | 43.5; 4 x 515 on 1999 ragged 93.7 | 81.4 | 79.0; 192-wide latents of 4 x 2048
-// tokens, 32 heads 238 | 213 | 204, 16 heads 131 | 114 | 108; 1 x 4000 179 | 163 | 155.
+// tokens, 32 heads 238 | 213 | 204, 16 heads 131 | 114 | 108; 1 x 4000 179 | 163 | 155 (a slower card than the one of the figures above; on a third one
+// 1 x 4000 167 | 146, 4 x 490 on 1750 95 | 82, 8 x 200 on 3000 134 | 109, registers | now).
 // SPLIT: gridDim.y workgroups share the block's key tiles, in runs of at least SPLIT_TILES; extend_split_merge_kernel adds their sums.
 constexpr int SPLIT_TILES = 4;
 template <int DQ> constexpr int direct_stage_bytes() { return 2 * 64 * 256 + (DQ > 128 ? 64 * 128 : 0); }

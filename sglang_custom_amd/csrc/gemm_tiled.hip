@@ -34,13 +34,15 @@
 //     b + 8 share an L2; each XCD works through 8 x 4 blocks of tiles (32 CUs = one block);
 //   * a workgroup stays on its CU and takes tile after tile: the K tiles of all its output tiles are one stream of requests, so
 //     the next tile's operands are on their way while the last one's results are written (a group writes its results in front of
-//     its first READ slot of the next tile, next to the other group's last MATRIX slot);
+//     its first READ slot of the next tile, next to the other group's last MATRIX slot; with RoPE both write at once, see there);
 //   * tiles beyond whole rounds of 256 may be split over K, their sums added by a second launch that also runs the epilogue.
 // A tile that ends costs what its K tiles do not: with a workgroup per tile 10.6 us (7725 x 8192 columns, K 2048: 200 us of which the K
 // tiles take 160), as it is 6.5.  us, a workgroup per tile -> now: 7725 x 8192 x K 2048 200.2 -> 187.5, K 4096 361 -> 346; 4605 x 6144 x K
 // 4096 169 -> 163; 2 x 14336 x K 4096 with SiLU-and-mul 771 -> 751; 4096 x K 14336 511 -> 500.  (Waiting for the next tile's requests and
-// not for the stores behind them gained nothing more; four waves of 128 x 128, a third fewer LDS reads, 2 to 9 % slower: K tiles of
-// 2470 cycles instead of 2260, for nothing covers a wave's own LDS reads and requests but its MFMAs.)
+// not for the stores behind them gained nothing more; four waves of 128 x 128, a third fewer LDS reads, 2 to 9 % slower: a K tile with x = 0
+// takes 1.03 us instead of 0.945, for nothing covers a wave's own LDS reads and requests but its MFMAs.)  That the walk through the tiles is fixed
+// costs nothing over many rounds: 65536 rows, a workgroup per tile -> now, ms, 2 x 14336 columns 10.56 -> 10.29, 4096 x K 14336 5.19 -> 5.06, 4096
+// x K 4096 1.50 -> 1.43; the first token of 64 x 1024 682 -> 661.
 // What bounds it: the card's power.  The MFMAs of a K tile take 2048 of its 2320 cycles (88 %), but with random operands the
 // clock falls to 1.7 GHz (4096 x 4096 x 4096: 98 us; with x = 0 2.17 GHz and 77).  So the order of a matrix slot's MFMAs counts: W fragments
 // go forth in one row of x fragments and back in the next, one operand of every MFMA the last one's (a loop of MFMAs alone 2045 ->
@@ -839,10 +841,10 @@ void fill_tiles(GemmTiledParams& p, int64_t m, int64_t n, int epilogue) {
 }
 
 // One workgroup is one CU, so tiles beyond whole rounds of 256 keep few CUs busy for as long as a round takes: those are split over K
-// where that pays.  Measured costs, in us: a K tile 1.2, a split of a tile (256 KiB of sums, written and read again) 0.075, the launch
-// that sums them 3.  bf16, us, whole tiles -> split: 4605 x 4096 x K 4096 (32 tail tiles, 5 splits) 168 -> 126, K 14336 (8) 538 -> 380;
-// 2 x 14336 columns, K 4096, 520 rows (80, 3) 168 -> 147, 1134 (48, 4) 262 -> 236, 1962 (128, 2) 373 -> 366.  Past half a round
-// (1353 rows of the last: 160 tiles) there is nobody to share with; 128 tiles of K 2048 gain less than the sums cost (101 either way).
+// where that pays.  Measured costs, in us: a K tile 1.2 (1.14 since workgroups stay), a split of a tile (256 KiB of sums, written and read again)
+// 0.075, the launch that sums them 3.  bf16, us, whole tiles -> split: 4605 x 4096 x K 4096 (32 tail tiles, 5 splits) 157 -> 123, K 14336 (8) 523 -> 372;
+// 2 x 14336 columns, K 4096, 520 rows (80, 3) 158 -> 128, 1134 (48, 5) 255 -> 219, 1962 (128, 2) 360 -> 351.  Past half a round
+// (1353 rows of the last: 160 tiles) there is nobody to share with; 128 tiles of K 2048 (42 us whole) gain less than the sums cost.
 int plan_tail(int64_t m, int64_t n, int64_t kbytes, int epilogue) {
   const int64_t tiles = cdiv(m, 256) * (pairs(epilogue) ? cdiv(n / 2, 128) : cdiv(n, 256));
   const int64_t kt = kbytes >> 7, tail = tiles % 256;
@@ -872,7 +874,7 @@ int set_tail(GemmTiledParams& p, int splits, void* workspace, int64_t workspace_
 // tiles of 16 NM x 64 outputs a wave.  KS groups of waves take K tiles in turn, each with a ring of its own, and add their sums
 // through LDS: two groups are two times as many bytes in flight where there are fewer tiles than CUs.  Tiles may be split over K further,
 // with sums in `part` as they lie in the registers (gemm_few_tail_kernel adds them).  K starts at another tile in every
-// column of tiles and goes round the end (see gemm_tiled_kernel on why): a row's result depends on its own values alone.
+// column of tiles and goes round the end (see gemm_grouped_kernel on why): a row's result depends on its own values alone.
 template <typename T, int EPI, bool FP8, int NM, int WM, int WN, int KS, int NS>
 __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_few_kernel(GemmTiledParams p) {
   extern __shared__ __attribute__((aligned(16))) char sm[];

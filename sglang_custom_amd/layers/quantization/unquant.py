@@ -26,15 +26,17 @@ SKINNY_MAX_M = 64
 DECODE_FUSION = True
 # "tiled" | "auto" | "library" for 16-bit GEMMs with more than SKINNY_MAX_M rows (see the module docstring)
 PREFILL_GEMM = os.environ.get("MI355_PREFILL_GEMM", "tiled")
-# below this many 256 x 256 output tiles the one-tile-per-workgroup kernel leaves most CUs idle
+# below this many 256 x 256 output tiles the kernel leaves too many CUs idle (us, library | tiled: 6144 x 4096 with 1300 rows, 144 tiles, 70 | 82,
+# 1700, 168, 74 | 81, 1962, 192, 83 | 83, 2300, 216, 86 | 86; 4096 x 4096 with 2300, 144, 67 | 75, 2800, 176, 76 | 79, 3100, 208, 81 | 82; 8192 x
+# 2048 with 1300, 192, 42 | 45, 1700, 224, 49 | 48)
 TILED_MIN_TILES = 192
 # ... unless the tiles share long reductions: with K split over the idle CUs the kernel is ahead of the library from K = 8192 on, but
-# for the few rows whose sums cost as much as the product (us, library | split: 4096 x 14336 with 126 rows 52 | 40, 330 75 | 58, 646
-# 106 | 84, 1134 140 | 125; 4096 x 11264 with 80 rows 36 | 37, 128 61 | 39, 700 84 | 72; 2048 x 8192 with 128 rows 22 | 25, 200
-# 30 | 27, 1000 52 | 48, 1353 53 | 56, 2100 83 | 74; 2048 x 5632 with 400 rows 26 | 29, 1000 40 | 40, 1500 45 | 48).  Products of less
-# than 2.1 billion multiply-adds are launches and sums more than anything else (library / split: 512 x 8192 with 300 rows 0.78, 128 x 16384 with
-# 256 0.64, 1024 x 14336 with 128 0.97, 150 1.23; 1280 x 8192 with 200 1.08), and columns of 16384 leave at most four workgroups a
-# tile (x 8192 with 150 to 300 rows 0.77 to 0.93, x 16384 0.85 to 1.25; 8192 x 8192 0.88 to 1.36, x 14336 1.01 to 1.77)
+# for the few rows whose sums cost as much as the product (us, library | split: 4096 x 14336 with 126 rows 41 | 35, 330 65 | 53, 646
+# 88 | 78, 1134 130 | 114; 4096 x 11264 with 80 rows 32 | 30, 128 47 | 31, 700 73 | 68; 2048 x 8192 with 128 rows 20 | 22, 200
+# 28 | 24, 1000 48 | 47, 1353 53 | 56, 2100 73 | 73; 2048 x 5632 with 400 rows 22 | 27, 1000 36 | 39, 1500 40 | 48).  Products of less
+# than 2.1 billion multiply-adds are launches and sums more than anything else (library / split: 512 x 8192 with 300 rows 0.83, 128 x 16384 with
+# 256 0.64, 1024 x 14336 with 128 0.97, 150 1.23; 1280 x 8192 with 200 1.03), and columns of 16384 leave at most four workgroups a
+# tile (x 8192 with 150 to 300 rows 0.77 to 1.01, x 16384 0.85 to 1.25; 8192 x 8192 0.88 to 1.36, x 14336 1.01 to 1.77)
 SPLIT_MIN_K = 8192
 SPLIT_MIN_MK = 1200000
 SPLIT_MIN_MACS = 2.1e9

@@ -34,14 +34,14 @@ SKINNY_MAX_M = 64
 # (hipBLASLt) on the plain projections and 1.23x on gate_up, whose scales and SiLU-and-mul run in its
 # epilogue -- and few rows (to 512) on the smaller tiles of mi355_linear_few; "library" = torch._scaled_mm everywhere.
 PREFILL_GEMM = os.environ.get("MI355_PREFILL_FP8_GEMM", "auto")
-# Below this many 256 x 256 output tiles too many CUs idle (us, library | tiled: 4096 x 4096 with 1600 rows, 112 tiles, 34 | 42, 6144 x 4096
-# with 1100, 120, 36 | 43; 4096 x 4096 with 2300 rows, 144, 57 | 44, 6144 x 4096 with 1600, 168, 57 | 45; 4096 x 14336 with 2300, 144,
-# 171 | 128) ...
+# Below this many 256 x 256 output tiles too many CUs idle (us, library | tiled: 4096 x 4096 with 1600 rows, 112 tiles, 36 | 43, 6144 x 4096
+# with 1100, 120, 34 | 41; 4096 x 4096 with 2300 rows, 144, 51 | 42, 6144 x 4096 with 1600, 168, 50 | 42; 4096 x 14336 with 2300, 144,
+# 138 | 112) ...
 TILED_MIN_TILES = 144
-# ... unless they share long reductions (4096 x 14336 with 80 rows 26 | 31, 150 35 | 33, 300 49 | 39, 646 70 | 52, 1100 90 | 71), the shorter
-# the more rows and columns it takes (library / split: 2048 x 14336 with 256 rows 0.92, 300 1.07; 4096 x 11264 with 256 0.88, 300
-# 1.08; x 8192 with 300 0.90, 520 1.12; 2048 x 8192 with 800 0.83, 1100 1.17), and 128 rows (8192 x 14336 with 90 0.90, 128
-# 1.06) and at most 8192 columns (16384 x 8192 0.91, x 16384 0.7 to 0.95)
+# ... unless they share long reductions (4096 x 14336 with 80 rows 24 | 25, 150 28 | 28, 300 39 | 35, 646 58 | 49, 1100 86 | 67), the shorter
+# the more rows and columns it takes (library / split: 2048 x 14336 with 256 rows 0.95, 300 0.97; 4096 x 11264 with 256 0.83, 300
+# 1.01; x 8192 with 300 0.90, 520 1.03; 2048 x 8192 with 800 0.84, 1100 1.04), and 128 rows (8192 x 14336 with 90 0.89, 128
+# 1.11) and at most 8192 columns (16384 x 8192 0.91, x 16384 0.7 to 0.95)
 SPLIT_MIN_K = 8192
 SPLIT_MIN_M = 128
 SPLIT_MIN_MNKK = 1.2e14

@@ -200,6 +200,9 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmTiledParams& p, f32x
       }
     }
   }
+  // (an end of its own for each kind of table: else the compiler joins the two forms' last stores and cuts one of them into pieces of 2 to 8 bytes)
+  if constexpr (CSF32) asm volatile("; table in fp32" ::: "memory");
+  else asm volatile("; table in the results' type" ::: "memory");
 }
 
 // Tile number `at` of the tile order: bands of 8 rows of tiles, blocks of 4 columns inside.
@@ -242,7 +245,9 @@ constexpr bool gt_pairs(int epi) { return epi == 1 || epi == 5; }   // W = [gate
 
 // The results of NM groups of 16 rows (row mbase + 16 mi + r16 is lane (q4, r16)'s in group mi; mbase: the first group's first row).
 // acc[mi][ni][r]: W slot 16 ni + 4 q4 + r of the wave's 64, which the load mapping made output column 32 (ni >> 1) + 8 q4 + 4 (ni & 1) + r
-// (plain) or column 8 q4 + 4 (ni & 1) + r of gate (ni < 2) or up.  EPI 3: `live` rows of the tile are no padding.
+// (plain) or column 8 q4 + 4 (ni & 1) + r of gate (ni < 2) or up.  EPI 3: `live` rows of the tile are no padding.  BIAS: if there is one.  (With
+// a form for each case in a small kernel the compiler joins their last stores, and cuts them into pieces of 2 to 8 bytes: the sums of 128 tail tiles
+// 13.5 -> 16.0 us.)
 template <typename T, int EPI, bool FP8, int NM, bool BIAS>
 __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&acc)[NM][4], int m0, int tm, int tn, int wc, int q4, int r16,
                                               int live) {
@@ -293,9 +298,13 @@ __device__ __forceinline__ void tile_epilogue(const GemmTiledParams& p, f32x4 (&
         sw[8 + j] = FP8 ? p.w_scale[min(n1, p.N - 8) + j] : 1.f;
       }
       if constexpr (BIAS) {
-        const Vec<T, 8> b0 = ldvec<T, 8>(bias + n0), b1 = ldvec<T, 8>(bias + min(n1, p.N - 8));
 #pragma unroll
-        for (int j = 0; j < 8; ++j) { bv[j] = to_f32(b0.v[j]); bv[8 + j] = to_f32(b1.v[j]); }
+        for (int j = 0; j < 16; ++j) bv[j] = 0.f;
+        if (bias != nullptr) {
+          const Vec<T, 8> b0 = ldvec<T, 8>(bias + n0), b1 = ldvec<T, 8>(bias + min(n1, p.N - 8));
+#pragma unroll
+          for (int j = 0; j < 8; ++j) { bv[j] = to_f32(b0.v[j]); bv[8 + j] = to_f32(b1.v[j]); }
+        }
       }
 #pragma unroll
       for (int mi = 0; mi < NM; ++mi) {
@@ -557,7 +566,7 @@ __global__ __launch_bounds__(512) void gemm_tiled_kernel(GemmTiledParams p) {
       });
     }
     if ((TOGETHER || !nxt.valid) && g == 0) __builtin_amdgcn_s_barrier();   // (the other group is one slot behind)
-    // The lane's number and the arguments again: otherwise the compiler works out the epilogue's addresses in front of all tiles and keeps
+    // The lane's number and the arguments (the kernel's only one, so that they lie first) again: otherwise the compiler works out the epilogue's addresses in front of all tiles and keeps
     // them, with every argument, in scratch memory and in lanes of a register.  2 x 14336 columns with SiLU-and-mul, 65536 rows: 10.70 ms so,
     // 10.22 this way (a workgroup per tile 10.45).
     int zero = 0;
@@ -800,8 +809,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_tail_kernel(GemmTiledParams p)
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) acc[0][ni] += *reinterpret_cast<const f32x4*>(src + (int64_t)k * p.tail * 65536 + ni * 256);
   }
-  if (EPI == 0 && p.bias != nullptr) tile_epilogue<T, EPI, FP8, 1, true>(p, acc, m0, tm, tn, wc, q4, r16, 256);
-  else tile_epilogue<T, EPI, FP8, 1, false>(p, acc, m0, tm, tn, wc, q4, r16, 256);
+  tile_epilogue<T, EPI, FP8, 1, EPI == 0>(p, acc, m0, tm, tn, wc, q4, r16, 256);
 }
 
 template <typename T, int EPI, bool FP8>
@@ -1002,8 +1010,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void gemm_few_kernel(GemmTiledPa
         for (int ni = 0; ni < 4; ++ni) *reinterpret_cast<f32x4*>(part + mi * 1024 + ni * 256) = acc[mi][ni];
     return;
   }
-  if (EPI == 0 && p.bias != nullptr) tile_epilogue<T, EPI, FP8, NM, true>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
-  else tile_epilogue<T, EPI, FP8, NM, false>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+  tile_epilogue<T, EPI, FP8, NM, EPI == 0>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
 }
 
 // A wave adds the splits' sums of 16 rows x 64 columns (W rows) in their order and finishes them.
@@ -1022,8 +1029,7 @@ __global__ __launch_bounds__(256) void gemm_few_tail_kernel(GemmTiledParams p, i
 #pragma unroll
     for (int ni = 0; ni < 4; ++ni) acc[0][ni] += *reinterpret_cast<const f32x4*>(src + (int64_t)k * groups * rows16 * 1024 + ni * 256);
   }
-  if (EPI == 0 && p.bias != nullptr) tile_epilogue<T, EPI, FP8, 1, true>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
-  else tile_epilogue<T, EPI, FP8, 1, false>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
+  tile_epilogue<T, EPI, FP8, 1, EPI == 0>(p, acc, m0, 0, G >> 2, G & 3, q4, r16, 256);
 }
 
 template <typename T, int EPI, bool FP8, int NM, int WM, int WN, int KS, int NS>
